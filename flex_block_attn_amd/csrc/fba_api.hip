@@ -61,7 +61,8 @@ int check_ptrs(std::initializer_list<std::pair<const char*, const void*>> ps) {
 hipError_t launch_dkdv_variant(fba::BwdParams& p, hipStream_t stream) {
   const char* env = getenv("FBA_DKDV_KEYS_PER_WAVE");
   const int keys = env ? atoi(env) : 64;
-  if (!p.tiled && keys == 64) return fba::launch_bwd_dkdv64(p, stream);
+  if (p.tiled) return fba::launch_bwd_dkdv_slab(p, stream);
+  if (keys == 64) return fba::launch_bwd_dkdv64(p, stream);
   return fba::launch_bwd_dkdv(p, stream);
 }
 
@@ -459,7 +460,7 @@ int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, cons
   p.ds_ws = (__bf16*)ds_ws; p.pair_base = pair_base; p.k_slot = kt_slot; p.q_slot = slot_table;
   p.ws_pairs = ds_ws_bytes / (128 * 128 * 2);
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = fba::launch_bwd_dkdv(p, (hipStream_t)hip_stream);
+  hipError_t e = fba::launch_bwd_dkdv_slab(p, (hipStream_t)hip_stream);
   if (e != hipSuccess) return hip_fail(e, "dkdv (tile lists, hand-over) launch");
   e = fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (from dS, tile lists) launch");

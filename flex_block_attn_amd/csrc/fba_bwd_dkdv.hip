@@ -41,12 +41,11 @@ using IC = std::integral_constant<int, N>;
 
 }  // namespace
 
-// kTiled = false: q_block and k_block are multiples of 128; list entries are query blocks, expanded to q_block/32 slabs.
-// kTiled = true: tile lists; list entries are 32-row query slabs with a predicate per (key group, 16-row half-slab).
+// Block lists only (q_block and k_block multiples of 128; list entries are query blocks, expanded to q_block/32 slabs); tile
+// lists have a kernel of their own (fba_bwd_dkdv_slab.hip).
 // kHandOver: every wave also stores the bf16 dS it forms to p.ds_ws (layout: fba_common.h), so that dQ = dS K can be
-// formed later without recomputing S and dP.  With tile lists the workspace is divided into (128-row query tile, 128-key
-// tile) pairs and a wave that leaves a slab out stores nothing for it.
-template <bool kTiled, bool kHandOver>
+// formed later without recomputing S and dP.
+template <bool kHandOver>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void dkdv_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int TK = 128;
@@ -85,11 +84,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   const int kblk = (kt * TK) / p.k_block;
   const int64_t krow0 = (int64_t)bhk * p.Skv + (int64_t)kt * TK;
 
-  const int nsub = kTiled ? 1 : p.q_block / kSlab;
-  const int row_len = kTiled ? p.Sq / kSlab : p.nQ;  // entries per list row
+  const int nsub = p.q_block / kSlab;
+  const int row_len = p.nQ;  // entries per list row
   auto list_row = [&](int g) -> int64_t {
     const int64_t bh = (int64_t)b * p.Hq + hkv * group + g;
-    return (p.mask_bh == 1 ? 0 : bh) * (kTiled ? tiles_per_head : p.nK) + (kTiled ? kt : kblk);
+    return (p.mask_bh == 1 ? 0 : bh) * p.nK + kblk;
   };
   const ConstIdx k_cnt = const_idx(p.k_cnt);
   int slabs_all = 0;
@@ -97,8 +96,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   slabs_all *= nsub;
   // this work-group's range of listed slabs: all of them, or part `part` of `parts` (boundaries on multiples of four slabs)
   const int s_begin = parts == 1 ? 0 : 4 * (int)(((int64_t)(slabs_all / 4) * part) / parts);
-  // (the last part takes what is left over: with tile lists the number of listed slabs need not be a multiple of four)
-  const int nslabs = (part + 1 == parts ? slabs_all : 4 * (int)(((int64_t)(slabs_all / 4) * (part + 1)) / parts)) - s_begin;
+  const int nslabs = (parts == 1 ? slabs_all : 4 * (int)(((int64_t)(slabs_all / 4) * (part + 1)) / parts)) - s_begin;
   // (query head of the group, list entry, slab inside the query block) of slab s_begin
   int g_begin = 0, e_begin = 0, sub_begin = 0;
   if (parts > 1) {
@@ -156,7 +154,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         head_row0 = ((int64_t)b * p.Hq + hkv * group + g_cur) * p.Sq;
         e_cur = 0;
       }
-      row_next = head_row0 + (kTiled ? (int64_t)(idx_cur[e_cur] >> 8) * kSlab : (int64_t)idx_cur[e_cur] * p.q_block);
+      row_next = head_row0 + (int64_t)idx_cur[e_cur] * p.q_block;
       rem = nsub;
     };
     auto advance = [&]() {
@@ -188,50 +186,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
       idx_cur = const_idx(p.k_idx + lr * row_len);
       head_row0 = ((int64_t)b * p.Hq + hkv * group + g_cur) * p.Sq;
       e_cur = e_begin;
-      row_next = head_row0 + (kTiled ? (int64_t)(idx_cur[e_cur] >> 8) * kSlab : (int64_t)idx_cur[e_cur] * p.q_block + sub_begin * kSlab);
+      row_next = head_row0 + (int64_t)idx_cur[e_cur] * p.q_block + sub_begin * kSlab;
       rem = nsub - sub_begin;
     }
     request_pair(0);
     request_pair(1);
 
-    // tile lists: predicate bits of this wave's slab, from a second walk over the same lists (two entries per step)
-    // (with the hand-over also the entry's tile-pair number and its slab inside the query tile)
-    int g_cmp = -1, e_cmp = -1, cnt_cmp = 0, bits_cmp = 0, sub_cmp = 0;
-    int64_t slot_cmp = 0, head_slot0 = 0;
-    ConstIdx idx_cmp = nullptr, slot_idx_cmp = nullptr;
-    auto enter_cmp_head = [&]() {  // list row of query head g_cmp of the group
-      const int64_t lr = list_row(g_cmp);
-      cnt_cmp = k_cnt[lr];
-      idx_cmp = const_idx(p.k_idx + lr * row_len);
-      if constexpr (kHandOver) {
-        slot_idx_cmp = const_idx(p.k_slot + lr * row_len);
-        const int64_t bh = (int64_t)b * p.Hq + hkv * group + g_cmp;
-        head_slot0 = p.mask_bh == 1 ? bh * const_idx(p.pair_base)[tiles_per_head] : 0;
-      }
-    };
-    auto next_bits = [&]() {
-      ++e_cmp;
-      while (e_cmp >= cnt_cmp) {
-        if (++g_cmp >= group) { bits_cmp = 0; return; }
-        enter_cmp_head();
-        e_cmp = 0;
-      }
-      const int ent = idx_cmp[e_cmp];
-      bits_cmp = ent & 255;
-      if constexpr (kHandOver) {
-        sub_cmp = (ent >> 8) & 3;
-        slot_cmp = head_slot0 + slot_idx_cmp[e_cmp];
-      }
-    };
-    if constexpr (kTiled) {
-      if (parts > 1) {  // start in the middle of the lists, as the cursor of the copies does
-        g_cmp = g_begin;
-        enter_cmp_head();
-        e_cmp = e_begin - 1;
-      }
-      next_bits();
-      if (par) next_bits();
-    }
     // dS hand-over: (query head of the group, list entry, slab inside the query block) of the slab this wave computes
     // next, and the pair number of entry 0 of that head's list row
     int h_g = -1, h_e = -1, h_s = 0, h_cnt = 0;
@@ -259,7 +219,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         ho_next_entry();
       }
     };
-    if constexpr (kHandOver && !kTiled) {
+    if constexpr (kHandOver) {
       if (parts == 1) {
         ho_next_entry();
       } else {
@@ -310,16 +270,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         s = mfma32(lds_read_b128(q_ptr[ks] + so), lds_read_b128(k_ptr[ks]), s);
         dp = mfma32(lds_read_b128(q_ptr[ks] + so + kSlabBytes), lds_read_b128(k_ptr[ks] + kTileBytes), dp);
       }
-      // does this wave's key block select the first / second 16 query rows of the slab?
-      const bool on0 = !kTiled || ((bits_cmp >> (2 * kg)) & 1) != 0;
-      const bool on1 = !kTiled || ((bits_cmp >> (2 * kg + 1)) & 1) != 0;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x4 l4 = lds_read_f32x4(st_ptr + so + 32 * g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           float pv = fast_exp2(__builtin_fmaf(s[4 * g + e], c, -l4[e]));
-          if constexpr (kTiled) pv = (g < 2 ? on0 : on1) ? pv : 0.f;  // a select: inf or NaN of a masked row is discarded
           s[4 * g + e] = pv;
           dp[4 * g + e] = pv * dp[4 * g + e];
         }
@@ -331,11 +287,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         dsk[j] = pack8(dp[8 * j + 0], dp[8 * j + 1], dp[8 * j + 2], dp[8 * j + 3], dp[8 * j + 4], dp[8 * j + 5], dp[8 * j + 6], dp[8 * j + 7]);
       }
       if constexpr (kHandOver) {
-        char* unit = reinterpret_cast<char*>(p.ds_ws);
-        if constexpr (kTiled)  // 16 units per tile pair, ordered (32-key slab, 32-row slab)
-          unit += slot_cmp * (16 * kDsUnitBytes) + (kg * 4 + sub_cmp) * kDsUnitBytes;
-        else
-          unit += (h_slot0 + h_e) * pair_bytes + ((int64_t)((h_s >> 2) * nsub_k + t_key) * 4 + (h_s & 3)) * kDsUnitBytes;
+        char* unit = reinterpret_cast<char*>(p.ds_ws) + (h_slot0 + h_e) * pair_bytes + ((int64_t)((h_s >> 2) * nsub_k + t_key) * 4 + (h_s & 3)) * kDsUnitBytes;
         // written once, read once by another kernel much later: streaming stores, so that they do not push the Q / dO
         // slabs that other work-groups are about to fetch out of L2
         store16_stream(unit, ho_off0, dsk[0]);
@@ -355,11 +307,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
 
     const int npairs = (nslabs + 1) >> 1;
     auto step = [&](auto half_c, int s2) {
-      // tile lists: a wave whose 32 keys are selected by neither half of the slab leaves the slab out (wave-uniform)
-      const bool worked = 2 * s2 + par < nslabs && (!kTiled || ((bits_cmp >> (2 * kg)) & 3) != 0);
+      const bool worked = 2 * s2 + par < nslabs;
       if (worked) compute(half_c);
-      if constexpr (kTiled) { next_bits(); next_bits(); }
-      if constexpr (kHandOver && !kTiled) ho_advance(2);
+      if constexpr (kHandOver) ho_advance(2);
       // this wave's copies of the next pair, requested one step ago, must have landed.  The two dS stores of this step, if
       // the wave made any, are younger and may still be on their way (the counter covers loads and stores alike and runs
       // down in issue order).
@@ -431,8 +381,7 @@ hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream) {
   plan_xcd_mapping(p.B * p.Hkv, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   const bool hand_over = p.ds_ws != nullptr;
-  void (*fn)(const BwdParams) = p.tiled ? (hand_over ? &dkdv_kernel<true, true> : &dkdv_kernel<true, false>)
-                                        : (hand_over ? &dkdv_kernel<false, true> : &dkdv_kernel<false, false>);
+  void (*fn)(const BwdParams) = hand_over ? &dkdv_kernel<true> : &dkdv_kernel<false>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
   if (e != hipSuccess) return e;
   // large launches let the work-groups claim their grid indices, with some work-groups more than indices (claim_work)
@@ -447,10 +396,8 @@ hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream) {
   }
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes + 16, stream, p);
   if (split_items > 0) {
-    const int64_t row0 = (int64_t)p.split.first * 128;
-    e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, p.dv, row0, split_items, 1.f, stream);
-    if (e != hipSuccess) return e;
-    e = launch_partial_sum(p.split.ws + 128 * kHeadDim, p.split.parts, 2 * 128 * kHeadDim, p.dk, row0, split_items, p.scale, stream);
+    const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
+    e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, 128, outs, 2, (int64_t)p.split.first * 128, split_items, stream);
     if (e != hipSuccess) return e;
   }
   if (hand_over) {

@@ -50,7 +50,6 @@ FBA_DEVICE void drain_matrix_pipe() { asm volatile("s_nop 15\n\ts_nop 15\n\ts_no
 // formed later without recomputing S and dP.
 template <bool kHandOver>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1))) void dkdv64_kernel(const BwdParams p) {
-  constexpr bool kTiled = false;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int TK = 128;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
@@ -84,11 +83,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int kblk = (kt * TK) / p.k_block;
   const int64_t krow0 = (int64_t)bhk * p.Skv + (int64_t)kt * TK;
 
-  const int nsub = kTiled ? 1 : p.q_block / kSlab;
-  const int row_len = kTiled ? p.Sq / kSlab : p.nQ;  // entries per list row
+  const int nsub = p.q_block / kSlab;
+  const int row_len = p.nQ;  // entries per list row
   auto list_row = [&](int g) -> int64_t {
     const int64_t bh = (int64_t)b * p.Hq + hkv * group + g;
-    return (p.mask_bh == 1 ? 0 : bh) * (kTiled ? tiles_per_head : p.nK) + (kTiled ? kt : kblk);
+    return (p.mask_bh == 1 ? 0 : bh) * p.nK + kblk;
   };
   const ConstIdx k_cnt = const_idx(p.k_cnt);
   int slabs_all = 0;
@@ -613,10 +612,8 @@ hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
   }
   hipLaunchKernelGGL(fn, dim3(grid), dim3(256), kSmemBytes + 16, stream, p);
   if (split_items > 0) {
-    const int64_t row0 = (int64_t)p.split.first * 128;
-    e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, p.dv, row0, split_items, 1.f, stream);
-    if (e != hipSuccess) return e;
-    e = launch_partial_sum(p.split.ws + 128 * kHeadDim, p.split.parts, 2 * 128 * kHeadDim, p.dk, row0, split_items, p.scale, stream);
+    const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
+    e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, 128, outs, 2, (int64_t)p.split.first * 128, split_items, stream);
     if (e != hipSuccess) return e;
   }
   if (p.ds_ws != nullptr) {

@@ -1,0 +1,419 @@
+// Backward, dK and dV on tile lists: gfx950, head_dim 128, bf16 in / fp32 accumulate / bf16 out, no atomics.
+//
+// Same mathematics as the kernels on block lists (fba_bwd_dkdv.hip).  Block sizes that are not multiples of 128 give the
+// two 64-key halves of a 128-key tile query slabs of their own (with independent random 64-token blocks at 40 % density the
+// tile's list is 64 % long and a half needs 62 % of its entries), so here a work-group owns 64 keys, which always lie in one
+// key block, and walks exactly the slabs that select them.
+//
+// Work-group = 64 key rows of one (batch, kv head), eight waves, two per SIMD.  Wave w works on keys 32 (w % 2) .. +31 and on
+// every fourth 32-query slab (w / 2 = position in a group of four), lane = key:
+//   S = Q K^T, dP = dO V^T             A = Q / dO slab rows from LDS, B = K rows in registers / V rows from LDS
+//   P = exp2(c S - lse2[q]),  dS = P o (dP - delta[q])
+//   dV^T += dO^T P,  dK^T += Q^T dS    A = dO / Q slab through transposing LDS fetches, B = P / dS packed to bf16
+// The list is first compacted into LDS: the entries of the 128-key tile whose predicate bits name this half, up to kChapter
+// at a time (a longer list is worked off in several such chapters), so that a step costs one LDS read instead of a walk.
+// The four waves of a key group hold partial sums over their slabs, which meet in LDS at the end.
+// LDS: ring of two steps x four (Q slab | dO slab | lse2 | -delta) buffers, the V rows (16 KiB), the compacted list.
+//
+// Bound by the matrix pipe and the arithmetic between its instructions (two waves per SIMD take turns), like the 32-key
+// kernel on block lists.  Two waves share a slab instead of four, so a quarter more bytes travel L2 -> LDS than with
+// 128-key work-groups that walk the union of their halves' lists with the idle half skipping, but every wave works in every
+// step: B1 H24 S30720, independent 64 x 64 blocks, 40 % kept, dK/dV + dQ 19.2 -> 16.0 ms.  Where all halves of a tile
+// agree (k_block a multiple of 128) the same kernel is as fast as 128-key work-groups were (15.6 -> 15.9 ms with 64-row
+// query blocks, 14.9 either way when the rows agree as well).
+#include <type_traits>
+
+#include "fba_common.h"
+#include "fba_kernels.h"
+
+namespace fba {
+
+namespace {
+
+constexpr int kSlab = 32;
+constexpr int kSlabBytes = kSlab * kRowBytes;       // 8 KiB
+constexpr int kStatBytes = 2 * kSlab * 4;           // lse2[32] | -delta[32]
+constexpr int kStageBytes = 2 * kSlabBytes + kStatBytes;
+constexpr int kPar = 4;                             // slabs per step
+constexpr int kTK = 64;                             // keys per work-group
+constexpr int kTileBase = 2 * kPar * kStageBytes;   // V rows, behind the ring (two buffers per position in a step)
+constexpr int kListBase = kTileBase + kTK * kRowBytes;
+constexpr int kRound = 512;                         // list entries scanned at a time: 64 per wave
+constexpr int kChapter = 2 * kRound;                // entries the LDS list holds, 8 bytes each
+constexpr int kCountBase = kListBase + kChapter * 8;  // two sets of eight counts, one per wave
+constexpr int kClaimBase = kCountBase + 64;
+constexpr int kSmemBytes = kClaimBase + 16;
+constexpr int kSlotFloats = 2 * kTK * kHeadDim;     // partial result of one part of a split item: dV rows, then dK rows
+
+template <int N>
+using IC = std::integral_constant<int, N>;
+
+}  // namespace
+
+// kHandOver: every wave also stores the bf16 dS it forms to p.ds_ws (tile pairs of 16 units, see fba_common.h).
+// kHalves: q_block is an odd multiple of 16, so a 32-row slab may be selected by one of its 16-row halves only.
+template <bool kHandOver, bool kHalves>
+__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void dkdv_slab_kernel(const BwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = wave & 1, par = wave >> 1;  // 32-key group, position in a step
+  // the grid index this work-group works on: its own, or one it claims (a launch with claim counters)
+  int grid_index = (int)blockIdx.x;
+  if (p.queue != nullptr) {
+    volatile int* claimed = reinterpret_cast<volatile int*>(smem + kClaimBase);
+    if (tid == 0) *claimed = claim_work(p.queue, xcd_id(), p.total_work);
+    __syncthreads();
+    grid_index = __builtin_amdgcn_readfirstlane(*claimed);
+    if (grid_index < 0) return;
+  }
+  // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
+  int item, part = 0, parts = 1;
+  if (grid_index < p.split.main_wgs) {
+    item = xcd_remap(grid_index, p.items_per_xcd);
+    if (item >= p.split.first) return;
+  } else {
+    const int s = grid_index - p.split.main_wgs;
+    item = p.split.first + s / p.split.parts;
+    part = s - (item - p.split.first) * p.split.parts;
+    parts = p.split.parts;
+  }
+  const int tiles_per_head = p.Skv / kTK;
+  const int bhk = item / tiles_per_head;
+  const int kt = item - bhk * tiles_per_head;
+  const int half = kt & 1;  // of the 128-key tile whose lists these are
+  const int b = bhk / p.Hkv, hkv = bhk - b * p.Hkv;
+  const int group = p.Hq / p.Hkv;
+  const int64_t krow0 = (int64_t)bhk * p.Skv + (int64_t)kt * kTK;
+  const int row_len = p.Sq / kSlab;  // entries per list row
+  const int lists_per_head = p.Skv / 128;
+  // lists that number more pairs than the workspace holds: no slab is touched, and the outputs become NaN
+  bool fits = true;
+  if constexpr (kHandOver) fits = workspace_holds_lists(p);
+
+  const uint32_t lds0 = lds_addr(smem);
+  // the two waves of a position bring in its slab together, 16 rows (four wave-level copies) each
+  uint32_t dma_off[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int row = 16 * kg + 4 * g + (lane >> 4);
+    dma_off[g] = (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4));
+  }
+  {  // V rows: wave w brings in rows 8 w .. 8 w + 7 (two copies)
+    const char* src = reinterpret_cast<const char*>(p.v) + (krow0 + 8 * wave) * kRowBytes;
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const int row = 8 * wave + 4 * g + (lane >> 4);
+      dma16(lds0 + kTileBase + (8 * wave + 4 * g) * kRowBytes, src, (uint32_t)((4 * g + (lane >> 4)) * kRowBytes + (((lane & 15) ^ swz(row)) << 4)));
+    }
+  }
+  // K rows of the wave as B operands, in registers for the whole list: lane holds key l32, d = 16 ks + 8 h .. +7
+  bf16x8 kreg[8];
+  {
+    const __bf16* kp = p.k + (krow0 + 32 * kg + l32) * kHeadDim + 8 * h;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) kreg[ks] = *reinterpret_cast<const bf16x8*>(kp + 16 * ks);
+  }
+
+  // Compaction of the tile's lists (one per query head of the group) into LDS, a round of 512 entries at a time: every wave
+  // tests 64 of them and the waves' counts give each its place.  The scan position is scalar state, the same in all waves.
+  // An LDS entry is {slab number over all heads << 2 | bits of its two 16-row halves, tile-pair number}.
+  int scan_g = fits ? 0 : group, scan_e = 0, seen = 0, flip_count = 0;
+  int2* const list = reinterpret_cast<int2*>(smem + kListBase);
+  // Places the entries of this half numbered [lo, hi) that follow the scan position, as many rounds as fit; returns how many.
+  auto fill = [&](int lo, int hi) -> int {
+    int n = 0;
+    while (scan_g < group) {
+      const int64_t bh = (int64_t)b * p.Hq + hkv * group + scan_g;
+      const int64_t lr = (p.mask_bh == 1 ? 0 : bh) * lists_per_head + (kt >> 1);
+      const int cnt = const_idx(p.k_cnt)[lr];
+      while (scan_e < cnt) {
+        if (n > kChapter - kRound || seen >= hi) return n;
+        const int e = scan_e + tid;
+        const int ent = e < cnt ? p.k_idx[lr * row_len + e] : 0;
+        int pair = 0;
+        if constexpr (kHandOver) {
+          pair = e < cnt ? p.k_slot[lr * row_len + e] : 0;
+          if (p.mask_bh == 1) pair += (int)(bh * const_idx(p.pair_base)[lists_per_head]);
+        }
+        const int bits = (ent >> (4 * half)) & 3;
+        const unsigned long long on = __ballot(bits != 0);
+        int* counts = reinterpret_cast<int*>(smem + kCountBase) + 8 * flip_count;
+        flip_count ^= 1;
+        if (lane == 0) counts[wave] = __popcll(on);
+        __syncthreads();
+        int before = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+          const int c = __builtin_amdgcn_readfirstlane(counts[w]);
+          before += w < wave ? c : 0;
+          all += c;
+        }
+        const int first = seen > lo ? seen : lo, last = seen + all < hi ? seen + all : hi;
+        const int at = seen + before + __popcll(on & ((1ull << lane) - 1ull));
+        if (bits != 0 && at >= first && at < last) {
+          int2 v;
+          v.x = (((int)(bh * row_len) + (ent >> 8)) << 2) | bits;
+          v.y = pair;
+          list[n + at - first] = v;
+        }
+        n += last > first ? last - first : 0;
+        seen += all;
+        scan_e += kRound;
+      }
+      scan_e = 0;
+      ++scan_g;
+    }
+    return n;
+  };
+  int lo = 0, hi = 0x7fffffff;
+  if (parts > 1) {  // this work-group's share of the slabs that select these keys
+    while (scan_g < group) fill(0, 0x7fffffff);
+    const int total = seen;
+    scan_g = fits ? 0 : group;
+    scan_e = seen = 0;
+    lo = (int)((int64_t)total * part / parts);
+    hi = (int)((int64_t)total * (part + 1) / parts);
+    __syncthreads();  // what the counting scan left in the list is not mixed with what follows
+  }
+
+  f32x16 acc_k[4], acc_v[4];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { acc_k[mb][r] = 0.f; acc_v[mb][r] = 0.f; }
+
+  RowMajorOffsets rm;
+  rm.init(lane);
+  TransposedOffsets tr;
+  tr.init(lane);
+  const char* const qbase = reinterpret_cast<const char*>(p.q);
+  const char* const dobase = reinterpret_cast<const char*>(p.d_o);
+  const char* const stbase = reinterpret_cast<const char*>(p.stats);
+  const int64_t rows_total = (int64_t)p.B * p.Hq * p.Sq;
+  // statistics copy: lanes 0..31 fetch lse2[row0 + l], lanes 32..63 fetch -delta[row0 + l - 32]
+  const uint32_t stat_off = (uint32_t)((lane >> 5) * rows_total * 4 + (lane & 31) * 4);
+  const uint32_t ho_off0 = (uint32_t)ds_unit_store_off(0, lane);
+  const float c = p.scale_log2e;
+  // ring buffer of position `par`, step parity s: byte (2 par + s) * kStageBytes
+  const uint32_t ring_dst = lds0 + 2 * par * kStageBytes;
+  // per-lane fetch addresses with the wave's share folded in; what remains is a compile-time displacement
+  const LdsPtr lds = lds_ptr(smem);
+  LdsPtr q_ptr[8], v_ptr[8], t_ptr[4][2];
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) {
+    q_ptr[ks] = lds + rm.rd[ks] + 2 * par * kStageBytes;
+    v_ptr[ks] = lds + rm.rd[ks] + kTileBase + kg * kSlabBytes;
+  }
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    t_ptr[mb][0] = lds + tr.rd[mb][0] + 2 * par * kStageBytes;
+    t_ptr[mb][1] = lds + tr.rd[mb][1] + 2 * par * kStageBytes;
+  }
+  const LdsPtr st_ptr = lds + 2 * par * kStageBytes + 2 * kSlabBytes + 16 * h;
+
+  // Copy i (0..8) of the nine that a wave owes for its slab of a step: Q rows, dO rows, statistics.
+  auto copy_part = [&](int i, uint32_t dst, int slab) {
+    const int64_t row = (int64_t)slab * kSlab;
+    if (i < 4) dma16(dst + (16 * kg + 4 * i) * kRowBytes, qbase + row * kRowBytes, dma_off[i]);
+    else if (i < 8) dma16(dst + kSlabBytes + (16 * kg + 4 * (i - 4)) * kRowBytes, dobase + row * kRowBytes, dma_off[i - 4]);
+    else dma4(dst + 2 * kSlabBytes, stbase + row * 4, stat_off);  // both waves copy the same 256 bytes
+  };
+
+  // One slab against this wave's 32 keys.  The copies of the next step's slab are issued in between the matrix
+  // instructions of S and dP.
+  auto compute = [&](auto buf_c, int x, int y, int x_next) {
+    constexpr int so = decltype(buf_c)::value * kStageBytes;
+    constexpr int no = kStageBytes - so;
+    f32x16 s, dp;
+    // accumulator element 4g + e of half-wave h is query row 8g + 4h + e of the slab; dP starts from -delta of its row
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 d4 = lds_read_f32x4(st_ptr + so + 4 * kSlab + 32 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { s[4 * g + e] = 0.f; dp[4 * g + e] = d4[e]; }
+    }
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      s = mfma32(lds_read_b128(q_ptr[ks] + so), kreg[ks], s);
+      dp = mfma32(lds_read_b128(q_ptr[ks] + so + kSlabBytes), lds_read_b128(v_ptr[ks]), dp);
+      copy_part(ks, ring_dst + no, x_next >> 2);
+    }
+    copy_part(8, ring_dst + no, x_next >> 2);
+    const bool on0 = !kHalves || (x & 1) != 0, on1 = !kHalves || (x & 2) != 0;  // are the two 16-row halves selected?
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x4 l4 = lds_read_f32x4(st_ptr + so + 32 * g);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float pv = fast_exp2(__builtin_fmaf(s[4 * g + e], c, -l4[e]));
+        if constexpr (kHalves) pv = (g < 2 ? on0 : on1) ? pv : 0.f;  // a select: inf or NaN of a masked row is discarded
+        s[4 * g + e] = pv;
+        dp[4 * g + e] = pv * dp[4 * g + e];
+      }
+    }
+    bf16x8 pk[2], dsk[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      pk[j] = pack8(s[8 * j + 0], s[8 * j + 1], s[8 * j + 2], s[8 * j + 3], s[8 * j + 4], s[8 * j + 5], s[8 * j + 6], s[8 * j + 7]);
+      dsk[j] = pack8(dp[8 * j + 0], dp[8 * j + 1], dp[8 * j + 2], dp[8 * j + 3], dp[8 * j + 4], dp[8 * j + 5], dp[8 * j + 6], dp[8 * j + 7]);
+    }
+    if constexpr (kHandOver) {
+      // 16 units per tile pair, ordered (32-key slab, 32-row slab); streaming stores: written once, read once much later
+      char* unit = reinterpret_cast<char*>(p.ds_ws) + (int64_t)y * (16 * kDsUnitBytes) + ((2 * half + kg) * 4 + ((x >> 2) & 3)) * kDsUnitBytes;
+      store16_stream(unit, ho_off0, dsk[0]);
+      store16_stream_second(unit, ho_off0, dsk[1]);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        const int roff = so + 16 * j * kRowBytes;
+        const bf16x8 adv = cat(lds_read_tr(t_ptr[mb][0] + kSlabBytes + roff), lds_read_tr(t_ptr[mb][1] + kSlabBytes + roff));
+        acc_v[mb] = mfma32(adv, pk[j], acc_v[mb]);
+        const bf16x8 adk = cat(lds_read_tr(t_ptr[mb][0] + roff), lds_read_tr(t_ptr[mb][1] + roff));
+        acc_k[mb] = mfma32(adk, dsk[j], acc_k[mb]);
+      }
+  };
+
+  // Every chapter of the list: entry 4 i + par is this wave's slab of step i (past the end: the last entry, copied into a
+  // buffer nobody reads, so that every wave has the same number of copies in flight at every wait).
+  for (;;) {
+    const int n = fill(lo, hi);
+    if (n == 0) break;
+    __syncthreads();  // the list is complete
+    const int nsteps = (n + kPar - 1) / kPar;
+    auto entry_of = [&](int step) -> int2 {
+      const int at = kPar * step + par;
+      return list[at < n ? at : n - 1];
+    };
+    auto uniform = [](int2 v) -> int2 { return make_int2(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y)); };
+    int2 cur = uniform(entry_of(0)), nxt = uniform(entry_of(1));
+#pragma unroll
+    for (int i = 0; i < 9; ++i) copy_part(i, ring_dst, cur.x >> 2);
+    wait_vmem<0>();
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) pin(kreg[ks]);
+    auto step = [&](auto buf_c, int i) {
+      const int2 after = entry_of(i + 2);  // read ahead, used behind the barrier
+      const bool worked = kPar * i + par < n;
+      if (worked) {
+        compute(buf_c, cur.x, cur.y, nxt.x);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 9; ++j) copy_part(j, ring_dst + kStageBytes - decltype(buf_c)::value * kStageBytes, nxt.x >> 2);
+      }
+      // the copies of the next step's slab must have landed; the two dS stores, if any, are younger and may still fly (the
+      // counter covers loads and stores alike and runs down in issue order)
+      if (kHandOver && worked) wait_vmem<2>(); else wait_vmem<0>();
+      __syncthreads();  // everybody is done with this step's buffers and everybody's copies for the next have landed
+      cur = nxt;
+      nxt = uniform(after);
+    };
+    for (int i = 0; i < nsteps; i += 2) {
+      step(IC<0>{}, i);
+      if (i + 1 < nsteps) step(IC<1>{}, i + 1);
+    }
+    wait_vmem<0>();
+    __syncthreads();  // no copy is writing LDS any more, and nobody reads the list
+  }
+  wait_vmem<0>();
+  __syncthreads();
+
+  // The four waves of a key group add up their partial sums through LDS: positions 2 and 3 hand theirs to 0 and 1, then 1
+  // hands its dV part to 0 and 0 its dK part to 1 (32 KiB and 16 KiB per wave).
+  auto put = [&](const f32x16 (&a)[4], int base) {
+    f32x4* dst = reinterpret_cast<f32x4*>(smem + base) + lane;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) dst[(mb * 4 + g) * 64] = (f32x4){a[mb][4 * g + 0], a[mb][4 * g + 1], a[mb][4 * g + 2], a[mb][4 * g + 3]};
+  };
+  auto take = [&](f32x16 (&a)[4], int base) {
+    const f32x4* src = reinterpret_cast<const f32x4*>(smem + base) + lane;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x4 r = src[(mb * 4 + g) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[mb][4 * g + e] += r[e];
+      }
+  };
+  const int slot32 = ((par & 1) * 2 + kg) * 32768;
+  if (par >= 2) {
+    put(acc_v, slot32);
+    put(acc_k, slot32 + 16384);
+  }
+  __syncthreads();
+  if (par < 2) {
+    take(acc_v, slot32);
+    take(acc_k, slot32 + 16384);
+  }
+  __syncthreads();
+  if (par == 0) put(acc_k, kg * 16384);
+  if (par == 1) put(acc_v, 32768 + kg * 16384);
+  __syncthreads();
+  if (par >= 2) return;
+  if (par == 0) take(acc_v, 32768 + kg * 16384);
+  else take(acc_k, kg * 16384);
+
+  const float poison = fits ? 1.f : __builtin_nanf("");
+  if (parts > 1) {
+    // part of a split item: unscaled fp32 partial sums go to the workspace, dV rows (position 0), then dK rows (position 1)
+    float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * kSlotFloats + par * (kTK * kHeadDim) + (kg * 32 + l32) * kHeadDim;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& a = par ? acc_k[mb] : acc_v[mb];
+        *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) =
+            (f32x4){a[4 * g + 0] * poison, a[4 * g + 1] * poison, a[4 * g + 2] * poison, a[4 * g + 3] * poison};
+      }
+    return;
+  }
+  // position 0 writes dV, position 1 writes dK (both zero when no query block selects these keys)
+  __bf16* orow = (par ? p.dk : p.dv) + (krow0 + kg * 32 + l32) * kHeadDim;
+  const float oscale = (par ? p.scale : 1.f) * poison;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const f32x16& a = par ? acc_k[mb] : acc_v[mb];
+      *reinterpret_cast<bf16x4*>(orow + 32 * mb + 8 * g + 4 * h) =
+          pack4(a[4 * g + 0] * oscale, a[4 * g + 1] * oscale, a[4 * g + 2] * oscale, a[4 * g + 3] * oscale);
+    }
+}
+
+hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
+  p.num_items = p.B * p.Hkv * (p.Skv / kTK);
+  // tail splitting (one work-group per compute unit)
+  void* const caller_ws = p.split.ws;  // whether or not anything is split
+  p.split = plan_split(p.num_items, 1, kSlotFloats * 4, p.split.ws, p.split_ws_bytes);
+  plan_xcd_mapping(p.B * p.Hkv, p.split.first, p.items_per_xcd, p.split.main_wgs);
+  const int split_items = p.num_items - p.split.first;
+  const bool hand_over = p.ds_ws != nullptr, halves = p.q_block % 32 != 0;
+  void (*fn)(const BwdParams) = hand_over ? (halves ? &dkdv_slab_kernel<true, true> : &dkdv_slab_kernel<true, false>)
+                                          : (halves ? &dkdv_slab_kernel<false, true> : &dkdv_slab_kernel<false, false>);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes);
+  if (e != hipSuccess) return e;
+  // large launches let the work-groups claim their grid indices, with some work-groups more than indices (claim_work)
+  p.total_work = p.split.main_wgs + split_items * p.split.parts;
+  int grid = p.total_work;
+  p.queue = nullptr;
+  if (claims_wanted(p.items_per_xcd, p.total_work, 1))
+    p.queue = work_queue_in(caller_ws, p.split_ws_bytes, (int64_t)split_items * p.split.parts * kSlotFloats * 4);
+  if (p.queue != nullptr) {
+    if ((e = launch_queue_reset(p.queue, stream)) != hipSuccess) return e;
+    grid += surplus_work_groups(p.total_work);
+  }
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes, stream, p);
+  if (split_items > 0) {
+    const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, kTK * kHeadDim}};
+    return launch_partial_sum(p.split.ws, p.split.parts, kSlotFloats, kTK, outs, 2, (int64_t)p.split.first * kTK, split_items, stream);
+  }
+  return hipGetLastError();
+}
+
+}  // namespace fba

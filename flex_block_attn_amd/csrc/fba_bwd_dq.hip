@@ -252,8 +252,10 @@ hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kSmem, stream, p);
-  if (split_items > 0)
-    return launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, p.dq, (int64_t)p.split.first * 128, split_items, p.scale, stream);
+  if (split_items > 0) {
+    const PartialOut out{p.dq, p.scale, 0};
+    return launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, (int64_t)p.split.first * 128, split_items, stream);
+  }
   return hipGetLastError();
 }
 

@@ -246,24 +246,28 @@ hipError_t zero_unit_address(const char** out) {
 
 }  // namespace
 
-// Sums the fp32 partial tiles of the split items in part order: out = scale * sum_p partial_p, as bf16.  One thread per
-// four columns; `rows_per_slot` rows of 128 columns per part, `sections` consecutive outputs per slot (dK/dV: two).
+// Sums the fp32 partial rows of the split items in part order: out = scale * sum_p partial_p, as bf16.  One thread per four
+// columns; an item has `rows` rows of 128 columns; blockIdx.y picks the output (dK/dV: two per slot, one launch for both).
+struct PartialOuts {
+  PartialOut out[2];
+};
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_sum_kernel(const float* ws, int parts, int64_t slot_floats,
-                                                                                          __bf16* out, int64_t out_row0, float scale) {
+                                                                                          int rows, PartialOuts outs, int64_t out_row0) {
   const int tid = threadIdx.x;
-  const int64_t row = (int64_t)blockIdx.x * 8 + (tid >> 5);  // row among 128 * (split items) rows
+  const PartialOut& o = outs.out[blockIdx.y];
+  const int row = blockIdx.x * 8 + (tid >> 5);  // among the rows of all split items
   const int c4 = (tid & 31) * 4;
-  const int64_t it = row >> 7;
-  const int r = (int)(row & 127);
-  const float* src = ws + it * parts * slot_floats + r * kHeadDim + c4;
+  const int it = row / rows, r = row - it * rows;
+  const float* src = ws + (int64_t)it * parts * slot_floats + o.offset + r * kHeadDim + c4;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int q = 0; q < parts; ++q) acc += *reinterpret_cast<const f32x4*>(src + q * slot_floats);
-  *reinterpret_cast<bf16x4*>(out + (out_row0 + row) * kHeadDim + c4) = pack4(acc[0] * scale, acc[1] * scale, acc[2] * scale, acc[3] * scale);
+  *reinterpret_cast<bf16x4*>(o.out + (out_row0 + row) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
 }
 
-hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, __bf16* out, int64_t out_row0, int n_items, float scale,
-                              hipStream_t stream) {
-  hipLaunchKernelGGL(partial_sum_kernel, dim3(n_items * 16), dim3(256), 0, stream, ws, parts, slot_floats, out, out_row0, scale);
+hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int64_t out_row0,
+                              int n_items, hipStream_t stream) {
+  PartialOuts o{{outs[0], outs[n_outs - 1]}};
+  hipLaunchKernelGGL(partial_sum_kernel, dim3(n_items * (rows / 8), n_outs), dim3(256), 0, stream, ws, parts, slot_floats, rows, o, out_row0);
   return hipGetLastError();
 }
 
@@ -298,7 +302,8 @@ hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kSmem, stream, p);
   if (split_items > 0) {
-    e = launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, p.dq, (int64_t)p.split.first * 128, split_items, p.scale, stream);
+    const PartialOut out{p.dq, p.scale, 0};
+    e = launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, (int64_t)p.split.first * 128, split_items, stream);
     if (e != hipSuccess) return e;
   }
   return launch_poison_unless_fit(p, p.dq, nullptr, (int64_t)p.B * p.Hq * p.Sq * kHeadDim, stream);

@@ -125,6 +125,7 @@ hipError_t launch_bwd_stats(const __bf16* o, const __bf16* d_o, const float* lse
 hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream);  // block lists only: 64 keys per wave, one wave per SIMD
+hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream);  // tile lists only: 64 keys per work-group
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream);
 // The lists of a hand-over call live in device memory, so only kernels can tell whether the pairs they number fit the
 // workspace.  Every kernel that stores or fetches dS tests it first (workspace_holds_lists, fba_common.h) and returns at
@@ -141,8 +142,14 @@ bool claims_wanted(int items_per_xcd, int total_work, int wgs_per_cu);
 inline int surplus_work_groups(int total_work) { return (total_work / 8 + 7) / 8 * 8; }
 hipError_t launch_queue_reset(int* queue, hipStream_t stream);
 int device_compute_units();
-hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, __bf16* out, int64_t out_row0, int n_items, float scale,
-                              hipStream_t stream);
+// One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats).
+struct PartialOut {
+  __bf16* out;
+  float scale;
+  int64_t offset;
+};
+hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int64_t out_row0,
+                              int n_items, hipStream_t stream);
 hipError_t launch_probe_mfma(const float* src, float* sink, int work_groups, int iters, hipStream_t stream);
 hipError_t launch_probe_read(const void* src, int64_t bytes, uint32_t* sink, int work_groups, hipStream_t stream);
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
