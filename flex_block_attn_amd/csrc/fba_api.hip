@@ -111,6 +111,16 @@ int check_lists(const Shape& s, bool tiled, const char* what) {
   return FBA_OK;
 }
 
+int check_tile_list_shape(int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block) {
+  if (q_block <= 0 || q_block % 16 != 0) return fail(FBA_ERR_INVALID, "q_block (%d) must be a positive multiple of 16", q_block);
+  if (k_block <= 0 || k_block % 64 != 0) return fail(FBA_ERR_INVALID, "k_block (%d) must be a positive multiple of 64", k_block);
+  const int64_t Sq = (int64_t)nQ * q_block, Skv = (int64_t)nK * k_block;
+  if (Sq % 128 != 0 || Skv % 128 != 0)
+    return fail(FBA_ERR_UNSUPPORTED, "tile lists need Sq (%lld) and Skv (%lld) to be multiples of 128", (long long)Sq, (long long)Skv);
+  if (Sq / 32 >= (1 << 23) || nK >= (1 << 23)) return fail(FBA_ERR_INVALID, "sequence too long for 24-bit list entries");
+  return FBA_OK;
+}
+
 int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, const int32_t* q_cnt, const int32_t* q_idx,
              int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
              int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream, bool tiled) {
@@ -199,12 +209,8 @@ int32_t fba_tile_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t
                        int32_t* qt_cnt, int32_t* qt_ent, int32_t* kt_cnt, int32_t* kt_ent, void* hip_stream) {
   if (mask_bh <= 0 || nQ <= 0 || nK <= 0)
     return fail(FBA_ERR_INVALID, "mask_bh, nQ, nK must be positive (got %lld %d %d)", (long long)mask_bh, nQ, nK);
-  if (q_block <= 0 || q_block % 16 != 0) return fail(FBA_ERR_INVALID, "q_block (%d) must be a positive multiple of 16", q_block);
-  if (k_block <= 0 || k_block % 64 != 0) return fail(FBA_ERR_INVALID, "k_block (%d) must be a positive multiple of 64", k_block);
+  if (int rc = check_tile_list_shape(nQ, nK, q_block, k_block)) return rc;
   const int64_t Sq = (int64_t)nQ * q_block, Skv = (int64_t)nK * k_block;
-  if (Sq % 128 != 0 || Skv % 128 != 0)
-    return fail(FBA_ERR_UNSUPPORTED, "tile lists need Sq (%lld) and Skv (%lld) to be multiples of 128", (long long)Sq, (long long)Skv);
-  if (Sq / 32 >= (1 << 23) || nK >= (1 << 23)) return fail(FBA_ERR_INVALID, "sequence too long for 24-bit list entries");
   if (!mask || !qt_cnt || !qt_ent || !kt_cnt || !kt_ent) return fail(FBA_ERR_INVALID, "null pointer argument");
   hipError_t e = fba::launch_tile_lists(mask, mask_bh, nQ, nK, q_block, k_block, (int)(Sq / 128), (int)(Skv / 128), (int)(Sq / 32),
                                         qt_cnt, qt_ent, kt_cnt, kt_ent, (hipStream_t)hip_stream);
@@ -501,6 +507,65 @@ int scratch_address(float** out) {
 }  // namespace
 
 extern "C" {
+
+int32_t fba_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block, int32_t* q_cnt,
+                  int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream) {
+  const bool both = k_cnt != nullptr && k_idx != nullptr;
+  if (!both && (k_cnt != nullptr || k_idx != nullptr)) return fail(FBA_ERR_INVALID, "k_cnt and k_idx must both be given or both be null");
+  if (both) {
+    return q_block % 128 == 0 && k_block % 128 == 0 ? fba_mask_compact(mask, mask_bh, nQ, nK, q_cnt, q_idx, k_cnt, k_idx, hip_stream)
+                                                    : fba_tile_lists(mask, mask_bh, nQ, nK, q_block, k_block, q_cnt, q_idx, k_cnt, k_idx, hip_stream);
+  }
+  if (mask_bh <= 0 || nQ <= 0 || nK <= 0)
+    return fail(FBA_ERR_INVALID, "mask_bh, nQ, nK must be positive (got %lld %d %d)", (long long)mask_bh, nQ, nK);
+  if (!mask || !q_cnt || !q_idx) return fail(FBA_ERR_INVALID, "null pointer argument");
+  hipError_t e;
+  if (q_block % 128 == 0 && k_block % 128 == 0) {
+    e = fba::launch_mask_compact(mask, mask_bh, nQ, nK, q_cnt, q_idx, nullptr, nullptr, (hipStream_t)hip_stream);
+  } else {
+    if (int rc = check_tile_list_shape(nQ, nK, q_block, k_block)) return rc;
+    e = fba::launch_tile_lists(mask, mask_bh, nQ, nK, q_block, k_block, (int)((int64_t)nQ * q_block / 128), 0, 0, q_cnt, q_idx, nullptr,
+                               nullptr, (hipStream_t)hip_stream);
+  }
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "list launch");
+}
+
+// For problems that take less time than it costs to number their pairs and to wait for the count: B1 H2 S1536, 384-token
+// blocks, forward + backward 304 -> 224 us against numbered pairs (four launches, a pinned copy and a wait less); B2 H8/2
+// S3136 q16 k64 430 -> 332 us.  The price is a workspace of all pairs instead of the selected ones, so the caller draws the
+// line where its memory limit does.
+int32_t fba_bwd_dense(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,
+                      void* ds_ws, int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* q_cnt, const int32_t* q_idx,
+                      const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq,
+                      int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
+                      void* hip_stream) {
+  const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
+  if (int rc = check_shape(s)) return rc;
+  const bool tiled = q_block % 128 != 0 || k_block % 128 != 0;
+  if (int rc = check_lists(s, tiled, "backward")) return rc;
+  if (int rc = check_split_ws(split_ws, split_ws_bytes)) return rc;
+  // everything is validated before the first launch, so that a rejected call leaves nothing on the stream
+  if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}, {"ds_ws", ds_ws}})) return rc;
+  if (!lse || !stats || !q_cnt || !q_idx || !k_cnt || !k_idx) return fail(FBA_ERR_INVALID, "null pointer argument");
+  if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
+  const int64_t need = (int64_t)B * Hq * Sq * Skv * 2;
+  if (ds_ws_bytes < need)
+    return fail(FBA_ERR_INVALID, "backward: ds_ws holds %lld bytes, all pairs of %d heads, %d x %d, need %lld", (long long)ds_ws_bytes, B * Hq, Sq,
+                Skv, (long long)need);
+  if (int rc = fba_bwd_stats(o, d_o, lse, stats, (int64_t)B * Hq * Sq, head_dim, hip_stream)) return rc;
+  fba::BwdParams p{};
+  fill_bwd(p, s);
+  p.tiled = tiled ? 1 : 0;
+  p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
+  p.stats = stats; p.dq = (__bf16*)dq; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv;
+  p.q_cnt = q_cnt; p.q_idx = q_idx; p.k_cnt = k_cnt; p.k_idx = k_idx;
+  p.ds_ws = (__bf16*)ds_ws;  // pair_base stays null: dense numbering
+  p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
+  hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream);
+  if (e != hipSuccess) return hip_fail(e, "dkdv (dense hand-over) launch");
+  e = fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (from dS, dense) launch");
+}
 
 int32_t fba_bwd_noalloc(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
                         void* dq, void* dk, void* dv, const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt,

@@ -49,10 +49,6 @@ template <bool kHandOver>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void dkdv_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int TK = 128;
-  if constexpr (kHandOver) {
-    if (!workspace_holds_lists(p)) return;  // the launcher's last launch reports it
-  }
-
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kg = wave & 3, par = wave >> 2;
@@ -94,6 +90,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   int slabs_all = 0;
   for (int g = 0; g < group; ++g) slabs_all += k_cnt[list_row(g)];
   slabs_all *= nsub;
+  if constexpr (kHandOver) {
+    if (!workspace_holds_lists(p)) slabs_all = 0;  // no slab is touched, and the outputs become NaN at the end
+  }
   // this work-group's range of listed slabs: all of them, or part `part` of `parts` (boundaries on multiples of four slabs)
   const int s_begin = parts == 1 ? 0 : 4 * (int)(((int64_t)(slabs_all / 4) * part) / parts);
   const int nslabs = (parts == 1 ? slabs_all : 4 * (int)(((int64_t)(slabs_all / 4) * (part + 1)) / parts)) - s_begin;
@@ -200,6 +199,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     const int nsub_k = p.k_block / kSlab;
     const int t_key = 4 * ((kt * TK - kblk * p.k_block) / TK) + kg;  // this wave's 32-key slab inside the key block
     const uint32_t ho_off0 = (uint32_t)ds_unit_store_off(0, lane), ho_off1 = (uint32_t)ds_unit_store_off(1, lane);
+    const bool dense = p.pair_base == nullptr;  // pairs numbered by position instead of in list order
     auto ho_next_entry = [&]() {
       ++h_e;
       while (h_e >= h_cnt) {
@@ -208,7 +208,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         h_cnt = k_cnt[lr];
         const ConstIdx pb = const_idx(p.pair_base);
         const int64_t bh = (int64_t)b * p.Hq + hkv * group + h_g;
-        h_slot0 = pb[lr] + (p.mask_bh == 1 ? bh * pb[p.nK] : 0);
+        h_slot0 = dense ? (bh * p.nK + kblk) * p.nQ : pb[lr] + (p.mask_bh == 1 ? bh * pb[p.nK] : 0);
         h_e = 0;
       }
     };
@@ -228,7 +228,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         h_cnt = k_cnt[lr];
         const ConstIdx pb = const_idx(p.pair_base);
         const int64_t bh = (int64_t)b * p.Hq + hkv * group + h_g;
-        h_slot0 = pb[lr] + (p.mask_bh == 1 ? bh * pb[p.nK] : 0);
+        h_slot0 = dense ? (bh * p.nK + kblk) * p.nQ : pb[lr] + (p.mask_bh == 1 ? bh * pb[p.nK] : 0);
         h_e = e_begin;
         h_s = sub_begin;
       }
@@ -287,7 +287,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         dsk[j] = pack8(dp[8 * j + 0], dp[8 * j + 1], dp[8 * j + 2], dp[8 * j + 3], dp[8 * j + 4], dp[8 * j + 5], dp[8 * j + 6], dp[8 * j + 7]);
       }
       if constexpr (kHandOver) {
-        char* unit = reinterpret_cast<char*>(p.ds_ws) + (h_slot0 + h_e) * pair_bytes + ((int64_t)((h_s >> 2) * nsub_k + t_key) * 4 + (h_s & 3)) * kDsUnitBytes;
+        const int pair = dense ? const_idx(p.k_idx + list_row(h_g) * row_len)[h_e] : h_e;
+        char* unit = reinterpret_cast<char*>(p.ds_ws) + (h_slot0 + pair) * pair_bytes + ((int64_t)((h_s >> 2) * nsub_k + t_key) * 4 + (h_s & 3)) * kDsUnitBytes;
         // written once, read once by another kernel much later: streaming stores, so that they do not push the Q / dO
         // slabs that other work-groups are about to fetch out of L2
         store16_stream(unit, ho_off0, dsk[0]);
@@ -347,6 +348,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
       }
   }
 
+  float poison = 1.f;
+  if constexpr (kHandOver) poison = poison_unless_fit(p);
   if (parts > 1) {
     // part of a split item: unscaled fp32 partial sums go to the workspace, dV tile (parity 0), then dK tile (parity 1)
     float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (2 * TK * kHeadDim) + par * (TK * kHeadDim) +
@@ -356,13 +359,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const f32x16& a = par ? acc_k[mb] : acc_v[mb];
-        *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) = (f32x4){a[4 * g + 0], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+        *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) = 
+            (f32x4){a[4 * g + 0] * poison, a[4 * g + 1] * poison, a[4 * g + 2] * poison, a[4 * g + 3] * poison};
       }
     return;
   }
   // parity 0 writes dV, parity 1 writes dK (both zero when no query block selects this key tile)
   __bf16* orow = (par ? p.dk : p.dv) + (krow0 + kg * 32 + l32) * kHeadDim;
-  const float oscale = par ? p.scale : 1.f;
+  const float oscale = (par ? p.scale : 1.f) * poison;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -399,9 +403,6 @@ hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
     e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, 128, outs, 2, (int64_t)p.split.first * 128, split_items, stream);
     if (e != hipSuccess) return e;
-  }
-  if (hand_over) {
-    return launch_poison_unless_fit(p, p.dk, p.dv, (int64_t)p.B * p.Hkv * p.Skv * kHeadDim, stream);
   }
   return hipGetLastError();
 }

@@ -46,10 +46,11 @@ FBA_DEVICE void drain_matrix_pipe() { asm volatile("s_nop 15\n\ts_nop 15\n\ts_no
 }  // namespace
 
 // Block lists only (q_block and k_block multiples of 128; list entries are query blocks, expanded to q_block/32 slabs).
-// kHandOver: every wave also stores the bf16 dS it forms to p.ds_ws (layout: fba_common.h), so that dQ = dS K can be
-// formed later without recomputing S and dP.
-template <bool kHandOver>
+// kMode (kNumbered, kDense): every wave also stores the bf16 dS it forms to p.ds_ws (layout: fba_common.h), so that dQ = dS K
+// can be formed later without recomputing S and dP.
+template <int kMode>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1))) void dkdv64_kernel(const BwdParams p) {
+  constexpr bool kHandOver = kMode != kRecompute;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int TK = 128;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
@@ -93,10 +94,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   int slabs_all = 0;
   for (int g = 0; g < group; ++g) slabs_all += k_cnt[list_row(g)];
   slabs_all *= nsub;
-  if constexpr (kHandOver) {
+  if constexpr (kMode == kNumbered) {
     // lists that number more pairs than the workspace holds: no slab is touched, nothing is stored into the workspace
-    // (the launcher's last launch then reports it)
-    if (!workspace_holds_lists(p)) slabs_all = 0;
+    // and the outputs become NaN at the end.  The factor that does it waits in LDS, behind the claim: formed again at the
+    // end, or held in a register, it costs the slab loop scalar registers it does not have.
+    const float poison = poison_unless_fit(p);
+    if (!(poison == 1.f)) slabs_all = 0;
+    if (tid == 0) *reinterpret_cast<volatile float*>(smem + kSmemBytes + 4) = poison;
   }
   // this work-group's range of listed slabs: all of them, or part `part` of `parts` (boundaries on multiples of four slabs;
   // block lists only)
@@ -199,14 +203,19 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       const int64_t bh = (int64_t)b * p.Hq + hkv * group + g;
       head_row0 = bh * p.Sq;
       if constexpr (kHandOver) {
-        const ConstIdx pb = const_idx(p.pair_base);
-        slot0_cur = pb[lr] + (p.mask_bh == 1 ? bh * pb[p.nK] : 0);
+        if constexpr (kMode == kDense) {
+          slot0_cur = (bh * p.nK + kblk) * p.nQ;
+        } else {
+          const ConstIdx pb = const_idx(p.pair_base);
+          slot0_cur = pb[lr] + (p.mask_bh == 1 ? bh * pb[p.nK] : 0);
+        }
       }
     };
     auto enter_block = [&](int first_sub) {  // entry e_cur of the current head, starting at slab first_sub (a multiple of 4)
-      row_next = head_row0 + (int64_t)idx_cur[e_cur] * p.q_block + first_sub * kSlab;
+      const int q_blk = idx_cur[e_cur];
+      row_next = head_row0 + (int64_t)q_blk * p.q_block + first_sub * kSlab;
       if constexpr (kHandOver)
-        unit_next = (slot0_cur + e_cur) * pair_bytes + ((int64_t)((first_sub >> 2) * nsub_k + t_key) * 4) * kDsUnitBytes;
+        unit_next = (slot0_cur + (kMode == kDense ? q_blk : e_cur)) * pair_bytes + ((int64_t)((first_sub >> 2) * nsub_k + t_key) * 4) * kDsUnitBytes;
       sub = first_sub;
       rem = (nsub - first_sub) >> 1;
     };
@@ -559,6 +568,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         }
   }
 
+  float poison = 1.f;
+  if constexpr (kMode == kNumbered) {
+    __syncthreads();
+    poison = *reinterpret_cast<volatile float*>(smem + kSmemBytes + 4);
+  }
   if (parts > 1) {
     // part of a split item: unscaled fp32 partial sums go to the workspace, dV tile (parity 0), then dK tile (parity 1)
     float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (2 * TK * kHeadDim) + par * (TK * kHeadDim) +
@@ -570,13 +584,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const f32x16& a = par ? acc_k[grp][mb] : acc_v[grp][mb];
-          *reinterpret_cast<f32x4*>(prow + grp * 32 * kHeadDim + 32 * mb + 8 * g + 4 * h) = (f32x4){a[4 * g + 0], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+          *reinterpret_cast<f32x4*>(prow + grp * 32 * kHeadDim + 32 * mb + 8 * g + 4 * h) =
+              (f32x4){a[4 * g + 0] * poison, a[4 * g + 1] * poison, a[4 * g + 2] * poison, a[4 * g + 3] * poison};
         }
     return;
   }
   // parity 0 writes dV, parity 1 writes dK (both zero when no query block selects this key tile)
   __bf16* orow = (par ? p.dk : p.dv) + (krow0 + kg * 64 + l32) * kHeadDim;
-  const float oscale = par ? p.scale : 1.f;
+  const float oscale = (par ? p.scale : 1.f) * poison;
 #pragma unroll
   for (int grp = 0; grp < 2; ++grp)
 #pragma unroll
@@ -596,7 +611,7 @@ hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
   p.split = plan_split(p.num_items, 1, 2 * 128 * kHeadDim * 4, p.split.ws, p.split_ws_bytes);
   plan_xcd_mapping(p.B * p.Hkv, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
-  void (*fn)(const BwdParams) = p.ds_ws != nullptr ? &dkdv64_kernel<true> : &dkdv64_kernel<false>;
+  void (*fn)(const BwdParams) = p.ds_ws == nullptr ? &dkdv64_kernel<kRecompute> : p.pair_base == nullptr ? &dkdv64_kernel<kDense> : &dkdv64_kernel<kNumbered>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
   if (e != hipSuccess) return e;
   // Launches of several rounds with contiguous spans per XCD let the work-groups claim their grid indices, with some more
@@ -615,9 +630,6 @@ hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
     e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, 128, outs, 2, (int64_t)p.split.first * 128, split_items, stream);
     if (e != hipSuccess) return e;
-  }
-  if (p.ds_ws != nullptr) {
-    return launch_poison_unless_fit(p, p.dk, p.dv, (int64_t)p.B * p.Hkv * p.Skv * kHeadDim, stream);
   }
   return hipGetLastError();
 }

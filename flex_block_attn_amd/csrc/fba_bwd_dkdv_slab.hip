@@ -133,8 +133,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         const int ent = e < cnt ? p.k_idx[lr * row_len + e] : 0;
         int pair = 0;
         if constexpr (kHandOver) {
-          pair = e < cnt ? p.k_slot[lr * row_len + e] : 0;
-          if (p.mask_bh == 1) pair += (int)(bh * const_idx(p.pair_base)[lists_per_head]);
+          if (p.pair_base == nullptr) {  // dense numbering
+            pair = (int)((bh * lists_per_head + (kt >> 1)) * (p.Sq / 128)) + (ent >> 10);
+          } else {
+            pair = e < cnt ? p.k_slot[lr * row_len + e] : 0;
+            if (p.mask_bh == 1) pair += (int)(bh * const_idx(p.pair_base)[lists_per_head]);
+          }
         }
         const int bits = (ent >> (4 * half)) & 3;
         const unsigned long long on = __ballot(bits != 0);
@@ -359,7 +363,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   if (par == 0) take(acc_v, 32768 + kg * 16384);
   else take(acc_k, kg * 16384);
 
-  const float poison = fits ? 1.f : __builtin_nanf("");
+  float poison = 1.f;
+  if constexpr (kHandOver) poison = poison_unless_fit(p);
   if (parts > 1) {
     // part of a split item: unscaled fp32 partial sums go to the workspace, dV rows (position 0), then dK rows (position 1)
     float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * kSlotFloats + par * (kTK * kHeadDim) + (kg * 32 + l32) * kHeadDim;

@@ -37,12 +37,11 @@ using IC = std::integral_constant<int, N>;
 
 }  // namespace
 
-template <bool kTiled>
+template <bool kTiled, int kMode>  // kMode: kNumbered or kDense
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void dq_from_ds_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // ring [4] of (K slab | dS units)
   constexpr int TQ = 128;
 
-  if (!workspace_holds_lists(p)) return;  // the launcher's last launch reports it
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
@@ -69,10 +68,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int tq = kTiled ? 0 : (qt * TQ - qblk * p.q_block) / TQ;  // this tile's position inside its query block
   const int n_kt = p.Skv / 128;
   const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (kTiled ? tiles_per_head : p.nQ) + (kTiled ? qt : qblk);
-  const int cnt = p.q_cnt[mrow];
+  constexpr bool dense = kMode == kDense;
+  // lists that number more pairs than the workspace holds: nothing is fetched, and the output becomes NaN
+  const int cnt = dense || workspace_holds_lists(p) ? p.q_cnt[mrow] : 0;
   const ConstIdx idx = const_idx(p.q_idx + mrow * p.nK);
   // block lists: pair number per list entry; tile lists: pair number per key tile, for this query tile
-  const ConstIdx slot = const_idx(p.q_slot + mrow * (kTiled ? n_kt : p.nK));
+  const ConstIdx slots = const_idx(dense ? nullptr : p.q_slot + mrow * (kTiled ? n_kt : p.nK));
+  auto slot = [&](int e) -> int64_t {
+    if constexpr (!dense) return slots[e];
+    else return kTiled ? ((int64_t)bh * n_kt + e) * tiles_per_head + qt : ((int64_t)bh * p.nK + idx[e]) * p.nQ + qblk;
+  };
   const int nsub = p.k_block / kSlab;
   // this work-group's range of 32-key steps of the list: all of it, or part `part` of `parts` (boundaries on whole rings)
   const int steps_all = cnt * nsub;
@@ -83,7 +88,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int64_t pair_bytes = kTiled ? 16 * kDsUnitBytes : (int64_t)p.q_block * p.k_block * 2;
   // dS of this wave's 32 rows: pair base + (tq * nsub + t) * 4 units + wave, t = 32-key slab inside the key block (inside
   // the key tile with tile lists)
-  const int64_t head_pairs = p.mask_bh == 1 ? (int64_t)bh * const_idx(p.pair_base)[kTiled ? n_kt : p.nK] : 0;
+  const int64_t head_pairs = p.mask_bh == 1 && !dense ? (int64_t)bh * const_idx(p.pair_base)[kTiled ? n_kt : p.nK] : 0;
   const char* ds_base = reinterpret_cast<const char*>(p.ds_ws) + head_pairs * pair_bytes + ((int64_t)tq * nsub * 4 + wave) * kDsUnitBytes;
   auto key_block = [&](int e) -> int { return kTiled ? idx[e] >> 8 : idx[e]; };
   const int wave_bits = 3 << (2 * wave);  // predicate bits of this wave's two 16-row groups in a tile-list entry
@@ -115,14 +120,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int64_t block_bytes = (int64_t)p.k_block * kRowBytes;
   int e_next = e_begin + 1, rem = nsub - sub_begin;
   int64_t k_off = nsteps > 0 ? key_block(e_begin) * block_bytes + (int64_t)sub_begin * kSlabBytes : 0;
-  int64_t ds_off_g = nsteps > 0 && !kTiled ? slot[e_begin] * pair_bytes + (int64_t)sub_begin * (4 * kDsUnitBytes) : 0;
+  int64_t ds_off_g = nsteps > 0 && !kTiled ? slot(e_begin) * pair_bytes + (int64_t)sub_begin * (4 * kDsUnitBytes) : 0;
   int blk_next = e_next < cnt ? key_block(e_next) : 0;
-  int slot_next = e_next < cnt && !kTiled ? slot[e_next] : 0;
+  int64_t slot_next = e_next < cnt && !kTiled ? slot(e_next) : 0;
   // tile lists: predicate bits of the entry being requested and of the next one; pair number of the key tile that the
   // next stage's slab lies in, read one stage ahead
   int bits_req = kTiled && cnt > 0 ? idx[0] & 255 : 0;
   int bits_req_next = kTiled && cnt > 1 ? idx[1] & 255 : 0;
-  int tile_slot = kTiled && cnt > 0 ? slot[(int)(k_off >> 15)] : 0;  // 32 KiB of K rows per key tile
+  int64_t tile_slot = kTiled && cnt > 0 ? slot((int)(k_off >> 15)) : 0;  // 32 KiB of K rows per key tile
   const uint32_t lane16 = (uint32_t)lane * 16;
   auto copy_next = [&](int ring) {
     const uint32_t dst = ring_dst + ring * kStageBytes;
@@ -130,7 +135,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     const char* src = ds_base + ds_off_g;
     if constexpr (kTiled) {
       const int t = (int)(k_off >> 13) & 3;  // 32-key slab inside its key tile
-      src = (bits_req & wave_bits) != 0 ? ds_base + (int64_t)tile_slot * pair_bytes + t * (4 * kDsUnitBytes) : p.zero_unit;
+      src = (bits_req & wave_bits) != 0 ? ds_base + tile_slot * pair_bytes + t * (4 * kDsUnitBytes) : p.zero_unit;
     }
     dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes, src, lane16);
     dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes + 1024, src, lane16 + 1024);
@@ -142,12 +147,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       ++e_next;
       blk_next = e_next < cnt ? key_block(e_next) : 0;
       if constexpr (kTiled) bits_req_next = e_next < cnt ? idx[e_next] & 255 : 0;
-      else slot_next = e_next < cnt ? slot[e_next] : 0;
+      else slot_next = e_next < cnt ? slot(e_next) : 0;
     } else {
       k_off += kSlabBytes;
       ds_off_g += 4 * kDsUnitBytes;
     }
-    if constexpr (kTiled) tile_slot = slot[(int)(k_off >> 15)];  // past the last stage: some listed tile's number, unused
+    if constexpr (kTiled) tile_slot = slot((int)(k_off >> 15));  // past the last stage: some listed tile's number, unused
   };
 
   if (nsteps > 0) {
@@ -199,22 +204,25 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     }
   }
 
+  const float poison = dense ? 1.f : poison_unless_fit(p);
   if (parts > 1) {  // part of a split item: unscaled fp32 partial sums go to the workspace
     float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) = (f32x4){acc[mb][4 * g + 0], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]};
+        *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) = 
+            (f32x4){acc[mb][4 * g + 0] * poison, acc[mb][4 * g + 1] * poison, acc[mb][4 * g + 2] * poison, acc[mb][4 * g + 3] * poison};
     return;
   }
   __bf16* orow = p.dq + (qrow0 + l32) * kHeadDim;
+  const float oscale = p.scale * poison;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const bf16x4 ov = pack4(acc[mb][4 * g + 0] * p.scale, acc[mb][4 * g + 1] * p.scale, acc[mb][4 * g + 2] * p.scale,
-                              acc[mb][4 * g + 3] * p.scale);
+      const bf16x4 ov = pack4(acc[mb][4 * g + 0] * oscale, acc[mb][4 * g + 1] * oscale, acc[mb][4 * g + 2] * oscale,
+                              acc[mb][4 * g + 3] * oscale);
       *reinterpret_cast<bf16x4*>(orow + 32 * mb + 8 * g + 4 * h) = ov;
     }
 }
@@ -271,22 +279,6 @@ hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, i
   return hipGetLastError();
 }
 
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void poison_unless_fit_kernel(const BwdParams p, __bf16* __restrict__ out_a, __bf16* __restrict__ out_b, int64_t n) {
-  if (workspace_holds_lists(p)) return;
-  const __bf16 nan = (__bf16)__builtin_nanf("");
-  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
-    out_a[t] = nan;
-    if (out_b) out_b[t] = nan;
-  }
-}
-
-hipError_t launch_poison_unless_fit(const BwdParams& p, __bf16* out_a, __bf16* out_b, int64_t n, hipStream_t stream) {
-  if (n <= 0) return hipSuccess;
-  const int64_t blocks = (n + 255) / 256;
-  hipLaunchKernelGGL(poison_unless_fit_kernel, dim3((unsigned)(blocks < 64 ? blocks : 64)), dim3(256), 0, stream, p, out_a, out_b, n);
-  return hipGetLastError();
-}
-
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
   constexpr int kSmem = kRing * kStageBytes;
   if (p.ds_ws == nullptr) return hipErrorInvalidValue;
@@ -295,7 +287,9 @@ hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
   p.split = plan_split(p.num_items, 2, 128 * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
-  void (*fn)(const BwdParams) = p.tiled ? &dq_from_ds_kernel<true> : &dq_from_ds_kernel<false>;
+  void (*fn)(const BwdParams) = p.pair_base == nullptr
+      ? (p.tiled ? &dq_from_ds_kernel<true, kDense> : &dq_from_ds_kernel<false, kDense>)
+      : (p.tiled ? &dq_from_ds_kernel<true, kNumbered> : &dq_from_ds_kernel<false, kNumbered>);
   hipError_t e = hipSuccess;
   if (p.tiled && (e = zero_unit_address(&p.zero_unit)) != hipSuccess) return e;
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
@@ -306,7 +300,7 @@ hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
     e = launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, (int64_t)p.split.first * 128, split_items, stream);
     if (e != hipSuccess) return e;
   }
-  return launch_poison_unless_fit(p, p.dq, nullptr, (int64_t)p.B * p.Hq * p.Sq * kHeadDim, stream);
+  return hipGetLastError();
 }
 
 }  // namespace fba

@@ -374,10 +374,16 @@ constexpr int kDsUnitBytes = 2048;
 // touches the pairs from pair_base[0] up to pair_base[rows], once per (batch, head) when all share one mask.
 template <typename P>
 FBA_DEVICE bool workspace_holds_lists(const P& p) {
+  if (p.pair_base == nullptr) return true;  // dense numbering: the host has compared the sizes
   const ConstIdx pb = const_idx(p.pair_base);
   const int64_t rows = p.mask_bh * (p.tiled ? p.Skv / 128 : p.nK);
   const int64_t listed = (int64_t)(pb[rows] - pb[0]) * (p.mask_bh == 1 ? (int64_t)p.B * p.Hq : 1);
   return listed <= p.ws_pairs;
 }
+
+// 1, or NaN where the lists do not fit: every kernel of a hand-over call multiplies its (then empty) results by it, so that
+// the call fails loudly instead of writing out of bounds.
+template <typename P>
+FBA_DEVICE float poison_unless_fit(const P& p) { return workspace_holds_lists(p) ? 1.f : __builtin_nanf(""); }
 
 }  // namespace fba

@@ -96,6 +96,8 @@ struct BwdParams {
   //   k_slot    [mask_bh, Skv/128, Sq/32]:      pair number of every kt_ent entry
   //   q_slot    [mask_bh, Sq/128, Skv/128]:     pair number of (query tile, key tile), -1 where nothing is listed
   //   zero_unit: 2 KiB of zeros in device memory, read in place of a dS unit that no wave stored
+  // pair_base null: dense numbering, a place for every pair whether selected or not, (bh * nK + J) * nQ + I (tile lists:
+  // (bh * Skv/128 + U) * Sq/128 + T) with bh over all heads; q_slot and k_slot are not read
   __bf16* ds_ws;
   int64_t ws_pairs;  // pairs ds_ws has room for
   const int32_t* pair_base;
@@ -109,6 +111,10 @@ struct BwdParams {
   int total_work;
   int64_t split_ws_bytes;  // size of split.ws as handed in by the caller
 };
+
+// How a backward call hands dS over: not at all (dQ recomputes), through pairs numbered in list order, or through a place
+// for every pair (dense numbering, see BwdParams).
+constexpr int kRecompute = 0, kNumbered = 1, kDense = 2;
 
 hipError_t launch_mask_compact(const uint8_t* mask, int64_t mask_bh, int nQ, int nK, int32_t* q_cnt, int32_t* q_idx,
                                int32_t* k_cnt, int32_t* k_idx, hipStream_t stream);
@@ -127,11 +133,6 @@ hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream);  // block lists only: 64 keys per wave, one wave per SIMD
 hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream);  // tile lists only: 64 keys per work-group
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream);
-// The lists of a hand-over call live in device memory, so only kernels can tell whether the pairs they number fit the
-// workspace.  Every kernel that stores or fetches dS tests it first (workspace_holds_lists, fba_common.h) and returns at
-// once when they do not; this launch then fills `n` bf16 values at `out_a` (and at `out_b` unless null) with NaN, so that
-// the call fails loudly instead of writing out of bounds.
-hipError_t launch_poison_unless_fit(const BwdParams& p, __bf16* out_a, __bf16* out_b, int64_t n, hipStream_t stream);
 // Room for the claim counters behind `partial_bytes` of partial results in a tail-splitting workspace (null if there is
 // none), and the launch that zeroes them.
 int* work_queue_in(void* ws, int64_t ws_bytes, int64_t partial_bytes);

@@ -17,7 +17,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void mask_comp
     int32_t* __restrict__ q_idx, int32_t* __restrict__ k_cnt, int32_t* __restrict__ k_idx) {
   const int lane = threadIdx.x & 63;
   const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int64_t n_qrows = mask_bh * nQ, n_krows = mask_bh * nK;
+  const int64_t n_qrows = mask_bh * nQ, n_krows = k_cnt != nullptr ? mask_bh * nK : 0;  // forward alone needs no key-major lists
   if (w >= n_qrows + n_krows) return;
 
   const bool row_pass = w < n_qrows;
@@ -45,7 +45,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void mask_comp
 
 hipError_t launch_mask_compact(const uint8_t* mask, int64_t mask_bh, int nQ, int nK, int32_t* q_cnt, int32_t* q_idx,
                                int32_t* k_cnt, int32_t* k_idx, hipStream_t stream) {
-  const int64_t waves = mask_bh * ((int64_t)nQ + nK);
+  const int64_t waves = mask_bh * ((int64_t)nQ + (k_cnt != nullptr ? nK : 0));
   const int64_t blocks = (waves + 3) / 4;
   if (blocks <= 0) return hipSuccess;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;

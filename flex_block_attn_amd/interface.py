@@ -313,6 +313,18 @@ def ds_workspace_bytes(lists, B, Hq, q_block_size, kv_block_size):
     return pairs, pairs * (128 * 128 if lists.tiled else q_block_size * kv_block_size) * 2
 
 
+def dense_ds_bytes(q, k):
+    """Bytes of a dS workspace with a place for every (query row, key) pair of every head (fba_bwd_dense)."""
+    return q.shape[0] * q.shape[1] * q.shape[2] * k.shape[2] * 2
+
+
+def dense_ds_fits(q, k):
+    """Whether backward can hand dS over without numbering the selected pairs: true for small problems, where the numbering
+    launches and the wait for the pair count would be a good part of the time (sequences up to about 6900 tokens with the
+    default limits)."""
+    return dense_ds_bytes(q, k) <= ds_workspace_limit(q, k)
+
+
 XCDS = 8  # a launch that gives every XCD whole heads of its own runs faster per head than one that makes XCDs share heads
 
 
@@ -353,7 +365,8 @@ def backward_with_lists(q, k, v, o, lse, do, q_block_size, kv_block_size, lists,
 
     hand_over=None (default): the key-major kernel stores dS once and dQ is formed from it (ten products per block
     pair instead of fourteen), in chunks of heads through a workspace of at most `ds_workspace_limit(q, k)` bytes; if not
-    even one kv head fits, as False.  True: the same with one workspace for all heads, whatever its size (fba_bwd_handover /
+    even one kv head fits, as False.  Small problems whose pairs are not numbered yet use a workspace with a place for every
+    pair (fba_bwd_dense).  True: the same with one workspace for all heads, whatever its size (fba_bwd_handover /
     fba_bwd_tiled_handover in one call).  False: dQ recomputes S and dP (fba_bwd or fba_bwd_tiled, no workspace)."""
     B, Hq, Hkv, Sq, Skv = _check_qkv(q, k, v)
     _check_lists(lists, q, B, Hq, Sq, Skv, q_block_size, kv_block_size)
@@ -371,7 +384,13 @@ def backward_with_lists(q, k, v, o, lse, do, q_block_size, kv_block_size, lists,
     dv = torch.empty_like(v)
     pair_bytes = (128 * 128 if lists.tiled else q_block_size * kv_block_size) * 2
     chunks = ds_ws = None
-    if hand_over or hand_over is None:
+    dense = hand_over is None and lists.pair_base is None and dense_ds_fits(q, k)
+    if dense:
+        try:
+            ds_ws = torch.empty((dense_ds_bytes(q, k),), dtype=torch.uint8, device=q.device)
+        except torch.OutOfMemoryError:
+            dense = False
+    elif hand_over or hand_over is None:
         unit_pairs, bounds = _unit_pairs(lists, B, Hq, Hkv)
         if sum(unit_pairs) > 0:
             chunks = [(0, B * Hkv, sum(unit_pairs))] if hand_over else plan_head_chunks(unit_pairs, pair_bytes, ds_workspace_limit(q, k))
@@ -391,7 +410,9 @@ def backward_with_lists(q, k, v, o, lse, do, q_block_size, kv_block_size, lists,
             common = (_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(stats), _ptr(dq), _ptr(dk), _ptr(dv),
                       _ptr(lists.q_cnt), _ptr(lists.q_idx), _ptr(lists.k_cnt), _ptr(lists.k_idx), M,
                       B, Hq, Hkv, Sq, Skv, HEAD_DIM, q_block_size, kv_block_size)
-            if lists.tiled:
+            if dense:
+                _lib.call("fba_bwd_dense", *common[:7], _ptr(ds_ws), ds_ws.numel(), *common[7:], sp_ptr, sp_bytes, _stream())
+            elif lists.tiled:
                 _lib.call("fba_bwd_tiled", *common, sp_ptr, sp_bytes, _stream())
             else:
                 _lib.call("fba_bwd", *common, sp_ptr, sp_bytes, _stream())
@@ -456,7 +477,7 @@ class FlexBlockAttnFunc(torch.autograd.Function):
     def forward(ctx, q, k, v, q_block_size, kv_block_size, block_mask, is_grad_enabled):
         _check_blocks(q, k, q_block_size, kv_block_size, block_mask)
         is_grad = is_grad_enabled and any(x.requires_grad for x in [q, k, v])
-        lists = lists_for(block_mask, q_block_size, kv_block_size, with_pair_numbers=is_grad)
+        lists = lists_for(block_mask, q_block_size, kv_block_size, with_pair_numbers=is_grad and not dense_ds_fits(q, k))
         o, lse = forward_with_lists(q, k, v, q_block_size, kv_block_size, lists)
         if is_grad:
             ctx.save_for_backward(q, k, v, o, lse)

@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2003
+#define FBA_VERSION 2004
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -151,6 +151,25 @@ int32_t fba_bwd_dq_from_ds(const void* k, const void* ds_ws, int64_t ds_ws_bytes
                            const int32_t* q_slot, const int32_t* pair_base, int64_t n_pairs, int64_t mask_bh, int32_t B, int32_t Hq,
                            int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block,
                            void* split_ws, int64_t split_ws_bytes, void* hip_stream);
+
+/*
+ * The lists of one mask in the flavour its block sizes need (fba_mask_compact's or fba_tile_lists', same shapes), with the
+ * key-major half left out when k_cnt and k_idx are null: forward reads the query-major lists only.
+ */
+int32_t fba_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block, int32_t* q_cnt,
+                  int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream);
+
+/*
+ * Backward with dS handed over in a workspace that has a place for every (query block, key block) pair, selected or not:
+ * B * Hq * Sq * Skv bf16.  Nothing has to be numbered and no pair count has to reach the host, which is what small problems
+ * spend their time on.  Takes block lists or tile lists, whichever the block sizes need; results are bit for bit those of
+ * fba_bwd_handover / fba_bwd_tiled_handover.
+ */
+int32_t fba_bwd_dense(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,
+                      void* ds_ws, int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* q_cnt, const int32_t* q_idx,
+                      const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq,
+                      int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
+                      void* hip_stream);
 
 /*
  * fba_bwd without the `stats` argument, for callers that cannot allocate device memory (tight serving loops, harnesses
