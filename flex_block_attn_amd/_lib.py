@@ -1,13 +1,18 @@
-"""ctypes binding of libfba_gfx950.so (the C ABI declared in include/fba.h).
+"""Bindings of libfba_gfx950.so (the C ABI declared in include/fba.h): ctypes for single entry points, and the host module
+fba_torch (csrc/fba_torch.cpp), which runs whole operator calls.
 
-There is no CPU or PyTorch fallback: if the library has not been built, or a call fails, an exception is raised.
+There is no CPU or PyTorch fallback: if either has not been built, or a call fails, an exception is raised.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # FBA_LIBRARY points the loader at another build of the same ABI (an instrumented or experimental one)
 LIB_PATH = os.environ.get("FBA_LIBRARY") or os.path.join(_HERE, "csrc", "libfba_gfx950.so")
+
+HOST_MODULE_PATH = os.path.join(_HERE, "csrc", "fba_torch.so")
 
 FBA_OK = 0
 FBA_ERR_INVALID = 1
@@ -52,6 +57,7 @@ SIGNATURES = {
 ABI_VERSION = 2004
 
 _lib = None
+_host = None
 
 
 class FbaError(RuntimeError):
@@ -97,3 +103,18 @@ def check(code):
 def call(name, *args):
     """Call an entry point and raise FbaError on a non-zero return."""
     check(getattr(load(), name)(*args))
+
+
+def host():
+    """The host module, bound to the library (once).  Raises if either is missing."""
+    global _host
+    if _host is None:
+        load()  # checks the library's version
+        if not os.path.exists(HOST_MODULE_PATH):
+            raise ImportError(f"{HOST_MODULE_PATH} is missing: build it with `python -m flex_block_attn_amd.build`. There is no fallback path.")
+        loader = importlib.machinery.ExtensionFileLoader("fba_torch", HOST_MODULE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("fba_torch", loader))
+        loader.exec_module(module)
+        module.bind(LIB_PATH)
+        _host = module
+    return _host

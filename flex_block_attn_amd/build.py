@@ -1,6 +1,6 @@
-"""Build recipe for the gfx950 shared library (hipcc cross-compiles without a GPU).
+"""Build recipe for the gfx950 shared library (hipcc cross-compiles without a GPU) and the host module beside it.
 
-    python -m flex_block_attn_amd.build            # compile csrc/*.hip -> csrc/libfba_gfx950.so
+    python -m flex_block_attn_amd.build            # csrc/*.hip -> csrc/libfba_gfx950.so, csrc/fba_torch.cpp -> csrc/fba_torch.so
     python -m flex_block_attn_amd.build --verbose  # also print per-kernel register / LDS usage
 
 The library is built in-tree so that it travels with the source tree to the machine that has the GPU.
@@ -11,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_NAME = "libfba_gfx950.so"
@@ -114,12 +115,35 @@ def check_asm_mfma_hazards():
             raise RuntimeError(f"{src}: a vector instruction writes an operand of an inline-asm matrix instruction right in front of it:\n{lines}")
 
 
+HOST_MODULE_PATH = os.path.join(CSRC, "fba_torch.so")
+
+
+def build_host_module():
+    """Compile csrc/fba_torch.cpp (host code only, against the installed torch) into the extension module fba_torch."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
+    tmp = HOST_MODULE_PATH + ".tmp"
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-DTORCH_EXTENSION_NAME=fba_torch",
+           "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *["-I" + i for i in inc],
+           os.path.join(CSRC, "fba_torch.cpp"), "-o", tmp, "-L" + os.path.join(root, "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compiling fba_torch.cpp failed:\n{r.stdout}{r.stderr}")
+    os.replace(tmp, HOST_MODULE_PATH)
+    return HOST_MODULE_PATH
+
+
 def build_library(verbose=False):
-    """Compile every HIP source and link libfba_gfx950.so. Returns the library path."""
-    with concurrent.futures.ThreadPoolExecutor(max_workers=4) as ex:
+    """Compile every HIP source and link libfba_gfx950.so, and build the host module. Returns the library path."""
+    with concurrent.futures.ThreadPoolExecutor(max_workers=5) as ex:
+        host = ex.submit(build_host_module)
         check = ex.submit(check_asm_mfma_hazards)
         results = list(ex.map(lambda s: _compile_one(s, verbose), SOURCES))
         check.result()
+        host.result()
     if verbose:
         for _, log in results:
             if log:

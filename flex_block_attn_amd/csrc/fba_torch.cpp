@@ -1,0 +1,414 @@
+// Host side of the operator in native code: what runs between a call of flex_block_attn_func and the kernels of
+// libfba_gfx950.so, and the autograd node that carries it.  Everything here is host work around the C ABI of include/fba.h:
+// checks, allocations from torch's caching allocator, the plan of the backward pass, launches.
+//
+// Why native: on small problems the kernels take a few tens of microseconds, and the same steps in Python took several times
+// that.  Per call, Python / native: B1 H1 S768, 128-token blocks, forward 45 / 16 us; B1 H2 S1536, 384-token blocks, forward +
+// backward 224 / 88 us; large problems the same.
+//
+// The library is not linked but bound by path (bind), so that FBA_LIBRARY can name another build of it.
+#include <dlfcn.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/core/Event.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/custom_class.h>
+#include <torch/extension.h>
+
+#include "../../include/fba.h"
+
+namespace {
+
+constexpr int64_t kHeadDim = 128;
+constexpr int64_t kXcds = 8;
+
+// ---------------------------------------------------------------------------------------------------------------------
+// the C ABI, bound at run time
+// ---------------------------------------------------------------------------------------------------------------------
+#define FBA_FUNCTIONS(X)                                                                                                      \
+  X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots) X(fba_tile_slots) X(fba_fwd) X(fba_fwd_tiled) \
+      X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense)
+
+struct Library {
+#define DECLARE(f) decltype(&::f) f = nullptr;
+  FBA_FUNCTIONS(DECLARE)
+#undef DECLARE
+} lib;
+
+void bind(const std::string& path) {
+  void* handle = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+  TORCH_CHECK(handle != nullptr, "cannot load ", path, ": ", dlerror());
+#define RESOLVE(f)                                                    \
+  lib.f = reinterpret_cast<decltype(&::f)>(dlsym(handle, #f));        \
+  TORCH_CHECK(lib.f != nullptr, path, " does not export ", #f);
+  FBA_FUNCTIONS(RESOLVE)
+#undef RESOLVE
+}
+
+// Failure of a C ABI call; becomes _lib.FbaError where it reaches Python (see the translator below).
+struct CallError : std::runtime_error {
+  int code;
+  explicit CallError(int c) : std::runtime_error(std::string("libfba_gfx950 error ") + std::to_string(c) + ": " + lib.fba_last_error()), code(c) {}
+};
+void check(int code) {
+  if (code != FBA_OK) throw CallError(code);
+}
+
+void* current_stream(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// ---------------------------------------------------------------------------------------------------------------------
+// shapes and lists
+// ---------------------------------------------------------------------------------------------------------------------
+struct Problem {
+  int64_t B, Hq, Hkv, Sq, Skv, q_block, k_block, mask_bh;
+  bool tiled() const { return q_block % 128 != 0 || k_block % 128 != 0; }
+  int64_t nQ() const { return Sq / q_block; }
+  int64_t nK() const { return Skv / k_block; }
+  int64_t pair_bytes() const { return (tiled() ? 128 * 128 : q_block * k_block) * 2; }
+  int64_t dense_bytes() const { return B * Hq * Sq * Skv * 2; }
+};
+
+// What the kernels read: query-major and key-major lists (block lists or tile lists) and, once the pairs are numbered, their
+// numbers (see include/fba.h).
+struct Lists {
+  int32_t *q_cnt = nullptr, *q_idx = nullptr, *k_cnt = nullptr, *k_idx = nullptr;
+  int32_t *pair_base = nullptr, *q_slot = nullptr, *k_slot = nullptr;
+  int64_t q_rows, q_len, k_rows, k_len, slot_len;  // per head of the mask
+  explicit Lists(const Problem& p) {
+    q_rows = p.tiled() ? p.Sq / 128 : p.nQ();
+    q_len = p.nK();
+    k_rows = p.tiled() ? p.Skv / 128 : p.nK();
+    k_len = p.tiled() ? p.Sq / 32 : p.nQ();
+    slot_len = p.tiled() ? p.Skv / 128 : p.nK();  // entries of a q_slot row
+  }
+};
+
+// Largest dS workspace backward allocates on its own: at most `limit` bytes, and at most `factor` times the bytes of the
+// call's own tensors (q, o, dO, dq and k, v, dk, dv in bf16).
+int64_t ds_limit(const at::Tensor& q, const at::Tensor& k, double limit, double factor) {
+  const double own = 2.0 * (5.0 * q.numel() + 4.0 * k.numel());
+  return (int64_t)std::min(limit, factor * own);
+}
+
+using Chunk = std::tuple<int64_t, int64_t, int64_t>;  // first unit, end unit, pairs
+
+// Cuts the (batch, kv head) units into consecutive chunks of equal length whose dS fits `limit` bytes: as few chunks as the
+// total needs, shortened while some chunk is still too large, and then, if a chunk holds more than one unit per XCD,
+// shortened to a multiple of the XCD count (twelve heads per chunk cost dK/dV 3 % against eight).  Nothing when a single
+// unit does not fit.
+c10::optional<std::vector<Chunk>> plan_head_chunks(const std::vector<int64_t>& unit_pairs, int64_t pair_bytes, int64_t limit) {
+  const int64_t n = (int64_t)unit_pairs.size();
+  int64_t total = 0;
+  for (int64_t u : unit_pairs) total += u;
+  total *= pair_bytes;
+  if (total == 0) return std::vector<Chunk>{{0, n, 0}};
+  auto cut = [&](int64_t per) {
+    std::vector<Chunk> chunks;
+    for (int64_t u = 0; u < n; u += per) {
+      int64_t pairs = 0;
+      for (int64_t i = u; i < std::min(n, u + per); ++i) pairs += unit_pairs[i];
+      chunks.emplace_back(u, std::min(n, u + per), pairs);
+    }
+    return chunks;
+  };
+  auto fits = [&](int64_t per) {
+    for (const Chunk& c : cut(per))
+      if (std::get<2>(c) * pair_bytes > limit) return false;
+    return true;
+  };
+  if (limit <= 0) return c10::nullopt;
+  const int64_t want = (total + limit - 1) / limit;
+  int64_t per = (n + want - 1) / want;
+  while (per >= 1 && !fits(per)) --per;
+  if (per < 1) return c10::nullopt;
+  if (per < n && per > kXcds && per % kXcds != 0 && fits(per - per % kXcds)) per -= per % kXcds;
+  return cut(per);
+}
+
+struct SplitWorkspace {  // see "Tail splitting" in include/fba.h
+  at::Tensor buffer;
+  int64_t bytes;
+  SplitWorkspace(const at::Tensor& like, int64_t n) : bytes(n) {
+    if (n > 0) buffer = at::empty({n}, like.options().dtype(at::kByte));
+  }
+  void* ptr() const { return bytes > 0 ? buffer.data_ptr() : nullptr; }
+};
+
+// ---------------------------------------------------------------------------------------------------------------------
+// forward and backward on lists
+// ---------------------------------------------------------------------------------------------------------------------
+std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const Lists& l,
+                                              int64_t split_bytes) {
+  at::Tensor o = at::empty_like(q);
+  at::Tensor lse = at::empty({p.B, p.Hq, p.Sq, 1}, q.options().dtype(at::kFloat));
+  SplitWorkspace split(q, split_bytes);
+  check((p.tiled() ? lib.fba_fwd_tiled : lib.fba_fwd)(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), l.q_cnt, l.q_idx,
+                                                      p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(),
+                                                      split.bytes, current_stream(q)));
+  return {o, lse};
+}
+
+enum class HandOver { kNever, kAuto, kWhole };  // dQ recomputes; as the limits allow; all heads at once whatever the size
+
+// bounds: pair numbers at the head boundaries of the mask (mask_bh + 1 of them); empty: pairs not numbered.
+std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o,
+                                     const at::Tensor& lse, const at::Tensor& d_o, const Lists& l, const std::vector<int64_t>& bounds, HandOver mode,
+                                     bool dense, int64_t limit, int64_t split_bytes) {
+  at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+  void* const stream = current_stream(q);
+  const int64_t group = p.Hq / p.Hkv, units = p.B * p.Hkv;
+  auto workspace = [&](int64_t bytes) {
+    at::Tensor ws;
+    try {
+      ws = at::empty({bytes}, q.options().dtype(at::kByte));
+    } catch (const c10::OutOfMemoryError&) {
+      if (mode == HandOver::kWhole) throw;
+    }
+    return ws;
+  };
+  at::Tensor ds;
+  c10::optional<std::vector<Chunk>> chunks;
+  if (dense) {
+    ds = workspace(p.dense_bytes());
+  } else if (mode != HandOver::kNever && !bounds.empty()) {
+    std::vector<int64_t> unit_pairs(units);
+    int64_t total = 0, most = 0;
+    for (int64_t u = 0; u < units; ++u) {  // the heads of a GQA group share their kv head's launch
+      unit_pairs[u] = p.mask_bh == 1 ? bounds.back() * group : bounds[(u + 1) * group] - bounds[u * group];
+      total += unit_pairs[u];
+    }
+    if (total > 0) {
+      if (mode == HandOver::kWhole) chunks = std::vector<Chunk>{{0, units, total}};
+      else chunks = plan_head_chunks(unit_pairs, p.pair_bytes(), limit);
+    }
+    if (chunks) {
+      for (const Chunk& c : *chunks) most = std::max(most, std::get<2>(c));
+      ds = workspace(most * p.pair_bytes());
+    }
+  }
+  SplitWorkspace split(q, split_bytes);
+  const auto f32 = q.options().dtype(at::kFloat);
+  if (!ds.defined() || dense) {
+    at::Tensor stats = at::empty({2, p.B, p.Hq, p.Sq}, f32);
+    if (ds.defined())
+      check(lib.fba_bwd_dense(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(), stats.data_ptr<float>(),
+                              ds.data_ptr(), ds.numel(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, p.mask_bh,
+                              p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes, stream));
+    else
+      check((p.tiled() ? lib.fba_bwd_tiled : lib.fba_bwd)(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(),
+                                                          stats.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), l.q_cnt, l.q_idx,
+                                                          l.k_cnt, l.k_idx, p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block,
+                                                          p.k_block, split.ptr(), split.bytes, stream));
+    return {dq, dk, dv};
+  }
+  // One launch sequence per chunk of kv heads [u0, u1): every pointer moves to the chunk's first head, the chunk is described
+  // as a batch of one, and the workspace pointer is moved back by the pairs of the heads in front of the chunk, so that the
+  // absolute pair numbers of the lists land inside the workspace.
+  int64_t longest = 0;
+  for (const Chunk& c : *chunks) longest = std::max(longest, std::get<1>(c) - std::get<0>(c));
+  at::Tensor stats = at::empty({2, longest * group * p.Sq}, f32);
+  auto bf16_at = [](const at::Tensor& t, int64_t elements) { return static_cast<char*>(t.data_ptr()) + 2 * elements; };
+  for (const auto& [u0, u1, pairs] : *chunks) {
+    const int64_t h0 = u0 * group, nh = (u1 - u0) * group, nu = u1 - u0;
+    const int64_t m0 = p.mask_bh > 1 ? h0 : 0;  // first head of the list tensors
+    const int64_t qo = h0 * p.Sq * kHeadDim, ko = u0 * p.Skv * kHeadDim;
+    char* const ws = static_cast<char*>(ds.data_ptr()) - (p.mask_bh > 1 ? bounds[h0] * p.pair_bytes() : 0);
+    const int64_t mask_bh = p.mask_bh > 1 ? nh : 1;
+    const float* lse0 = lse.data_ptr<float>() + h0 * p.Sq;
+    const int32_t *q_cnt = l.q_cnt + m0 * l.q_rows, *q_idx = l.q_idx + m0 * l.q_rows * l.q_len;
+    const int32_t *k_cnt = l.k_cnt + m0 * l.k_rows, *k_idx = l.k_idx + m0 * l.k_rows * l.k_len;
+    const int32_t *base = l.pair_base + m0 * l.k_rows, *q_slot = l.q_slot + m0 * l.q_rows * l.slot_len;
+    if (p.tiled())
+      check(lib.fba_bwd_tiled_handover(bf16_at(q, qo), bf16_at(k, ko), bf16_at(v, ko), bf16_at(o, qo), bf16_at(d_o, qo), lse0, stats.data_ptr<float>(), ws,
+                                       pairs * p.pair_bytes(), bf16_at(dq, qo), bf16_at(dk, ko), bf16_at(dv, ko), q_cnt, q_idx, k_cnt, k_idx, base,
+                                       l.k_slot + m0 * l.k_rows * l.k_len, q_slot, pairs, mask_bh, 1, nh, nu, p.Sq, p.Skv, kHeadDim, p.q_block,
+                                       p.k_block, split.ptr(), split.bytes, stream));
+    else
+      check(lib.fba_bwd_handover(bf16_at(q, qo), bf16_at(k, ko), bf16_at(v, ko), bf16_at(o, qo), bf16_at(d_o, qo), lse0, stats.data_ptr<float>(), ws,
+                                 pairs * p.pair_bytes(), bf16_at(dq, qo), bf16_at(dk, ko), bf16_at(dv, ko), q_cnt, q_idx, k_cnt, k_idx, base, q_slot,
+                                 pairs, mask_bh, 1, nh, nu, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes, stream));
+  }
+  return {dq, dk, dv};
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// the whole operator
+// ---------------------------------------------------------------------------------------------------------------------
+// What backward needs besides tensors autograd saves: the lists (one allocation), the host copy of the pair numbers at the
+// head boundaries when the pairs are numbered, and the settings of the call.
+struct Saved : torch::CustomClassHolder {
+  Problem p;
+  Lists lists;
+  at::Tensor list_buffer, host_bounds;
+  c10::Event copied{c10::DeviceType::CUDA};
+  bool dense;
+  int64_t limit, split_bytes;
+  explicit Saved(const Problem& problem) : p(problem), lists(problem) {}
+};
+
+// The lists of `mask` in one buffer; key-major half and (numbered) pair numbers only where backward will read them.
+void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered) {
+  const Problem& p = s.p;
+  Lists& l = s.lists;
+  const int64_t M = p.mask_bh;
+  int64_t used = 0;
+  auto take = [&](int64_t n) {
+    const int64_t at = used;
+    used += (n + 63) / 64 * 64;
+    return at;
+  };
+  const int64_t q_cnt = take(M * l.q_rows), q_idx = take(M * l.q_rows * l.q_len);
+  int64_t k_cnt = 0, k_idx = 0, base = 0, q_slot = 0, k_slot = 0;
+  if (backward) {
+    k_cnt = take(M * l.k_rows);
+    k_idx = take(M * l.k_rows * l.k_len);
+  }
+  if (numbered) {
+    base = take(M * l.k_rows + 1);
+    q_slot = take(M * l.q_rows * l.slot_len);
+    if (p.tiled()) k_slot = take(M * l.k_rows * l.k_len);
+  }
+  s.list_buffer = at::empty({used}, mask.options().dtype(at::kInt));
+  int32_t* const b = s.list_buffer.data_ptr<int32_t>();
+  void* const stream = current_stream(mask);
+  l.q_cnt = b + q_cnt;
+  l.q_idx = b + q_idx;
+  if (backward) {
+    l.k_cnt = b + k_cnt;
+    l.k_idx = b + k_idx;
+  }
+  check(lib.fba_lists(static_cast<const uint8_t*>(mask.data_ptr()), M, p.nQ(), p.nK(), p.q_block, p.k_block, l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, stream));
+  if (!numbered) return;
+  l.pair_base = b + base;
+  l.q_slot = b + q_slot;
+  if (p.tiled()) {
+    l.k_slot = b + k_slot;
+    check(lib.fba_tile_slots(l.k_cnt, l.k_idx, M, l.q_rows, l.k_rows, l.pair_base, l.k_slot, l.q_slot, stream));
+  } else {
+    check(lib.fba_pair_slots(l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, M, p.nQ(), p.nK(), l.pair_base, l.q_slot, stream));
+  }
+  // The copy is ordered before whatever the caller enqueues next: backward waits for it alone, not for the forward kernel.
+  s.host_bounds = at::empty({M + 1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  s.host_bounds.copy_(s.list_buffer.narrow(0, base, M * l.k_rows + 1).slice(0, 0, c10::nullopt, l.k_rows), /*non_blocking=*/true);
+  s.copied.record(c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(mask.device()));
+}
+
+struct Attention : torch::autograd::Function<Attention> {
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask,
+                            c10::intrusive_ptr<Saved> s) {
+    build_lists(*s, mask, /*backward=*/true, /*numbered=*/!s->dense);
+    auto [o, lse] = run_forward(s->p, q, k, v, s->lists, s->split_bytes);
+    ctx->save_for_backward({q, k, v, o, lse});
+    ctx->saved_data["s"] = c10::IValue::make_capsule(std::move(s));
+    return o;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
+    const auto t = ctx->get_saved_variables();
+    const auto capsule = ctx->saved_data["s"].toCapsule();
+    Saved& s = *static_cast<Saved*>(capsule.get());
+    const c10::DeviceGuard guard(t[0].device());
+    const at::Tensor d_o = grads[0].to(at::kBFloat16).contiguous();
+    std::vector<int64_t> bounds;
+    if (!s.dense) {
+      s.copied.synchronize();
+      const int32_t* h = s.host_bounds.data_ptr<int32_t>();
+      bounds.assign(h, h + s.p.mask_bh + 1);
+    }
+    auto g = run_backward(s.p, t[0], t[1], t[2], t[3], t[4], d_o, s.lists, bounds, HandOver::kAuto, s.dense, s.limit, s.split_bytes);
+    return {g[0], g[1], g[2], at::Tensor(), at::Tensor()};
+  }
+};
+
+// flex_block_attn_func for arguments that need no preparation; nothing for all others (wrong types or shapes, lengths that
+// have to be padded), which Python then reports or prepares.
+c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t q_block, int64_t k_block, const at::Tensor& mask,
+                                    double limit, double factor, int64_t split_bytes) {
+  for (const at::Tensor* t : {&q, &k, &v})
+    if (!t->is_cuda() || t->scalar_type() != at::kBFloat16 || t->dim() != 4 || !t->is_contiguous() || t->size(3) != kHeadDim ||
+        t->device() != q.device() || (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) != 0)
+      return c10::nullopt;
+  if (mask.device() != q.device() || mask.scalar_type() != at::kBool || (mask.dim() != 2 && mask.dim() != 4) || !mask.is_contiguous()) return c10::nullopt;
+  Problem p{q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), q_block, k_block, mask.dim() == 2 ? 1 : q.size(0) * q.size(1)};
+  const int64_t md = mask.dim();
+  if (q.numel() == 0 || k.numel() == 0 || k.size(0) != p.B || v.sizes() != k.sizes() || p.Hq % p.Hkv != 0) return c10::nullopt;
+  if (q_block <= 0 || k_block <= 0 || q_block % 16 != 0 || k_block % 64 != 0 || (k_block % q_block != 0 && q_block % k_block != 0)) return c10::nullopt;
+  if (p.Sq % q_block != 0 || p.Skv % k_block != 0 || mask.size(md - 2) != p.nQ() || mask.size(md - 1) != p.nK()) return c10::nullopt;
+  if (md == 4 && (mask.size(0) != p.B || mask.size(1) != p.Hq)) return c10::nullopt;
+  if (p.tiled() && (p.Sq % 128 != 0 || p.Skv % 128 != 0)) return c10::nullopt;
+  if (p.B * p.Hq * p.Sq >= (1LL << 30) || p.B * p.Hkv * p.Skv >= (1LL << 30) || p.mask_bh * p.nQ() * p.nK() > 0x7fffffffLL ||
+      p.mask_bh * (p.Sq / 32 + 1) * (p.Skv / 128 + 1) > 0x7fffffffLL)
+    return c10::nullopt;
+  const c10::DeviceGuard guard(q.device());
+  if (split_bytes < 0) split_bytes = lib.fba_split_workspace_bytes();
+  auto s = c10::make_intrusive<Saved>(p);
+  s->split_bytes = split_bytes;
+  const bool backward = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+  if (!backward) {
+    build_lists(*s, mask, false, false);
+    return run_forward(p, q, k, v, s->lists, split_bytes).first;
+  }
+  s->limit = ds_limit(q, k, limit, factor);
+  s->dense = p.dense_bytes() <= s->limit;
+  return Attention::apply(q, k, v, mask, std::move(s));
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// entry points on lists (checked by the caller)
+// ---------------------------------------------------------------------------------------------------------------------
+int32_t* ints(const c10::optional<at::Tensor>& t) { return t ? t->data_ptr<int32_t>() : nullptr; }
+
+Problem problem_of(const at::Tensor& q, const at::Tensor& k, int64_t q_block, int64_t k_block, int64_t mask_bh) {
+  return {q.size(0), q.size(1), k.size(1), q.size(2), k.size(2), q_block, k_block, mask_bh};
+}
+
+std::pair<at::Tensor, at::Tensor> forward_on_lists(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t q_block, int64_t k_block,
+                                                   int64_t mask_bh, const at::Tensor& q_cnt, const at::Tensor& q_idx, int64_t split_bytes) {
+  const c10::DeviceGuard guard(q.device());
+  const Problem p = problem_of(q, k, q_block, k_block, mask_bh);
+  Lists l(p);
+  l.q_cnt = q_cnt.data_ptr<int32_t>();
+  l.q_idx = q_idx.data_ptr<int32_t>();
+  return run_forward(p, q, k, v, l, split_bytes);
+}
+
+std::vector<at::Tensor> backward_on_lists(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& lse,
+                                          const at::Tensor& d_o, int64_t q_block, int64_t k_block, int64_t mask_bh, const at::Tensor& q_cnt,
+                                          const at::Tensor& q_idx, const at::Tensor& k_cnt, const at::Tensor& k_idx,
+                                          const c10::optional<at::Tensor>& pair_base, const c10::optional<at::Tensor>& q_slot,
+                                          const c10::optional<at::Tensor>& k_slot, const std::vector<int64_t>& bounds, c10::optional<bool> hand_over,
+                                          bool dense, int64_t limit, int64_t split_bytes) {
+  const c10::DeviceGuard guard(q.device());
+  const Problem p = problem_of(q, k, q_block, k_block, mask_bh);
+  Lists l(p);
+  l.q_cnt = q_cnt.data_ptr<int32_t>();
+  l.q_idx = q_idx.data_ptr<int32_t>();
+  l.k_cnt = k_cnt.data_ptr<int32_t>();
+  l.k_idx = k_idx.data_ptr<int32_t>();
+  l.pair_base = ints(pair_base);
+  l.q_slot = ints(q_slot);
+  l.k_slot = ints(k_slot);
+  const HandOver mode = !hand_over ? HandOver::kAuto : *hand_over ? HandOver::kWhole : HandOver::kNever;
+  return run_backward(p, q, k, v, o, lse, d_o, l, bounds, mode, dense, limit, split_bytes);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  namespace py = pybind11;
+  py::register_exception_translator([](std::exception_ptr e) {
+    try {
+      if (e) std::rethrow_exception(e);
+    } catch (const CallError& err) {
+      py::object cls = py::module_::import("flex_block_attn_amd._lib").attr("FbaError");
+      PyErr_SetObject(cls.ptr(), cls(err.code, lib.fba_last_error()).ptr());
+    }
+  });
+  m.def("bind", &bind);
+  m.def("plan_head_chunks", &plan_head_chunks);
+  m.def("attention", &attention, py::call_guard<py::gil_scoped_release>());
+  m.def("forward", &forward_on_lists, py::call_guard<py::gil_scoped_release>());
+  m.def("backward", &backward_on_lists, py::call_guard<py::gil_scoped_release>());
+}

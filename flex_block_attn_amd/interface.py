@@ -2,8 +2,9 @@
 
 Same names, argument order and return arity as the reference's flex_block_attn/flex_block_attn_interface.py
 (`flex_block_attn_func` :91-106, `FlexBlockAttnFunc` :14-89, `_flex_block_attn_forward` :6-8,
-`_flex_block_attn_backward` :10-12).  The compiled half is libfba_gfx950.so, reached through ctypes with raw device
-pointers and the current HIP stream; PyTorch only provides device memory and autograd plumbing.
+`_flex_block_attn_backward` :10-12).  The kernels live in libfba_gfx950.so; the host work around them (allocations, the plan
+of the backward pass, launches, the autograd node) is native code in the module fba_torch.  This file holds the checks and
+their messages, and the calls on precompacted lists.
 
 What differs from the reference, deliberately:
   * the bool block mask is turned into index lists once, on the GPU (`compact_block_mask`), at its true
@@ -225,9 +226,13 @@ def _check_lists(lists, q, B, Hq, Sq, Skv, q_block_size, kv_block_size):
 SPLIT_WORKSPACE_MIB = os.environ.get("FBA_SPLIT_WORKSPACE_MIB")
 
 
+def _split_bytes():
+    return _lib.load().fba_split_workspace_bytes() if SPLIT_WORKSPACE_MIB is None else int(float(SPLIT_WORKSPACE_MIB) * 2 ** 20)
+
+
 def _split_workspace(device):
     """(tensor or None, pointer, bytes) of a fresh tail-splitting workspace on `device`."""
-    n = _lib.load().fba_split_workspace_bytes() if SPLIT_WORKSPACE_MIB is None else int(float(SPLIT_WORKSPACE_MIB) * 2 ** 20)
+    n = _split_bytes()
     if n <= 0:
         return None, None, 0
     ws = torch.empty((n,), dtype=torch.uint8, device=device)
@@ -238,14 +243,7 @@ def forward_with_lists(q, k, v, q_block_size, kv_block_size, lists):
     """Forward on compacted lists -> (o [B,H,Sq,128] bf16, lse [B,H,Sq,1] fp32)."""
     B, Hq, Hkv, Sq, Skv = _check_qkv(q, k, v)
     _check_lists(lists, q, B, Hq, Sq, Skv, q_block_size, kv_block_size)
-    o = torch.empty_like(q)
-    lse = torch.empty((B, Hq, Sq, 1), dtype=torch.float32, device=q.device)
-    args = (_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(lists.q_cnt), _ptr(lists.q_idx), lists.mask_bh,
-            B, Hq, Hkv, Sq, Skv, HEAD_DIM, q_block_size, kv_block_size)
-    with torch.cuda.device(q.device):
-        _ws, ws_ptr, ws_bytes = _split_workspace(q.device)
-        _lib.call("fba_fwd_tiled" if lists.tiled else "fba_fwd", *args, ws_ptr, ws_bytes, _stream())
-    return o, lse
+    return _lib.host().forward(q, k, v, q_block_size, kv_block_size, lists.mask_bh, lists.q_cnt, lists.q_idx, _split_bytes())
 
 
 def number_pairs(lists):
@@ -325,39 +323,12 @@ def dense_ds_fits(q, k):
     return dense_ds_bytes(q, k) <= ds_workspace_limit(q, k)
 
 
-XCDS = 8  # a launch that gives every XCD whole heads of its own runs faster per head than one that makes XCDs share heads
-
-
 def plan_head_chunks(unit_pairs, pair_bytes, limit_bytes):
     """Cuts the (batch, kv head) units into consecutive chunks of equal length whose dS fits `limit_bytes`: as few chunks
     as the total needs, shortened while some chunk is still too large, and then, if a chunk holds more than one unit per
     XCD, shortened to a multiple of the XCD count (twelve heads per chunk cost dK/dV 3 % against eight).  Returns
     [(first unit, end unit, pairs)], or None when a single unit does not fit."""
-    n = len(unit_pairs)
-    total = sum(unit_pairs) * pair_bytes
-    if total == 0:
-        return [(0, n, 0)]
-
-    def cut(per):
-        return [(u, min(n, u + per), sum(unit_pairs[u: u + per])) for u in range(0, n, per)]
-
-    def fits(chunks):
-        return all(c[2] * pair_bytes <= limit_bytes for c in chunks)
-
-    limit_bytes = int(limit_bytes)
-    per = -(-n // max(1, -(-total // max(1, limit_bytes)))) if limit_bytes > 0 else 0
-    while per >= 1 and not fits(cut(per)):
-        per -= 1
-    if per < 1:
-        return None
-    if per < n and per > XCDS and per % XCDS and fits(cut(per - per % XCDS)):
-        per -= per % XCDS
-    return cut(per)
-
-
-def _offset(t, elements):
-    """Device pointer `elements` elements into tensor t (may point below t for the shifted dS workspace)."""
-    return ctypes.c_void_p(t.data_ptr() + elements * t.element_size())
+    return _lib.host().plan_head_chunks(list(unit_pairs), pair_bytes, int(limit_bytes))
 
 
 def backward_with_lists(q, k, v, o, lse, do, q_block_size, kv_block_size, lists, hand_over=None):
@@ -379,72 +350,10 @@ def backward_with_lists(q, k, v, o, lse, do, q_block_size, kv_block_size, lists,
     if lse.dtype != torch.float32 or lse.numel() != B * Hq * Sq:
         raise ValueError("lse must be float32 with B*H*Sq elements")
     lse = lse.contiguous()
-    dq = torch.empty_like(q)
-    dk = torch.empty_like(k)
-    dv = torch.empty_like(v)
-    pair_bytes = (128 * 128 if lists.tiled else q_block_size * kv_block_size) * 2
-    chunks = ds_ws = None
     dense = hand_over is None and lists.pair_base is None and dense_ds_fits(q, k)
-    if dense:
-        try:
-            ds_ws = torch.empty((dense_ds_bytes(q, k),), dtype=torch.uint8, device=q.device)
-        except torch.OutOfMemoryError:
-            dense = False
-    elif hand_over or hand_over is None:
-        unit_pairs, bounds = _unit_pairs(lists, B, Hq, Hkv)
-        if sum(unit_pairs) > 0:
-            chunks = [(0, B * Hkv, sum(unit_pairs))] if hand_over else plan_head_chunks(unit_pairs, pair_bytes, ds_workspace_limit(q, k))
-        if chunks is not None:
-            try:
-                ds_ws = torch.empty((max(c[2] for c in chunks) * pair_bytes,), dtype=torch.uint8, device=q.device)
-            except torch.OutOfMemoryError:
-                if hand_over:
-                    raise
-                chunks = None
-    group = Hq // Hkv
-    M = lists.mask_bh
-    with torch.cuda.device(q.device):
-        _ws, sp_ptr, sp_bytes = _split_workspace(q.device)
-        if chunks is None:
-            stats = torch.empty((2, B, Hq, Sq), dtype=torch.float32, device=q.device)
-            common = (_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(stats), _ptr(dq), _ptr(dk), _ptr(dv),
-                      _ptr(lists.q_cnt), _ptr(lists.q_idx), _ptr(lists.k_cnt), _ptr(lists.k_idx), M,
-                      B, Hq, Hkv, Sq, Skv, HEAD_DIM, q_block_size, kv_block_size)
-            if dense:
-                _lib.call("fba_bwd_dense", *common[:7], _ptr(ds_ws), ds_ws.numel(), *common[7:], sp_ptr, sp_bytes, _stream())
-            elif lists.tiled:
-                _lib.call("fba_bwd_tiled", *common, sp_ptr, sp_bytes, _stream())
-            else:
-                _lib.call("fba_bwd", *common, sp_ptr, sp_bytes, _stream())
-            return dq, dk, dv
-        # one launch sequence per chunk of kv heads [u0, u1): every pointer moves to the chunk's first head, the chunk is
-        # described as a batch of one, and the workspace pointer is moved back by the pairs of the heads in front of the
-        # chunk, so that the absolute pair numbers of the lists land inside the workspace
-        stats = torch.empty((2, max(c[1] - c[0] for c in chunks) * group * Sq), dtype=torch.float32, device=q.device)
-        n_qt, n_kt = Sq // 128, Skv // 128
-        for u0, u1, pairs in chunks:
-            h0, nh, nu = u0 * group, (u1 - u0) * group, u1 - u0
-            m0 = h0 if M > 1 else 0  # first row of the per-head list tensors
-            qo, ko = h0 * Sq * HEAD_DIM, u0 * Skv * HEAD_DIM
-            ws_ptr = ctypes.c_void_p(ds_ws.data_ptr() - (bounds[h0] * pair_bytes if M > 1 else 0))
-            shape = (nh if M > 1 else 1, 1, nh, nu, Sq, Skv, HEAD_DIM, q_block_size, kv_block_size)
-            if lists.tiled:
-                _lib.call(
-                    "fba_bwd_tiled_handover", _offset(q, qo), _offset(k, ko), _offset(v, ko), _offset(o, qo), _offset(do, qo), _offset(lse, h0 * Sq),
-                    _ptr(stats), ws_ptr, pairs * pair_bytes, _offset(dq, qo), _offset(dk, ko), _offset(dv, ko),
-                    _offset(lists.q_cnt, m0 * n_qt), _offset(lists.q_idx, m0 * n_qt * lists.nK), _offset(lists.k_cnt, m0 * n_kt),
-                    _offset(lists.k_idx, m0 * n_kt * 4 * n_qt), _offset(lists.pair_base, m0 * n_kt), _offset(lists.k_slot, m0 * n_kt * 4 * n_qt),
-                    _offset(lists.q_slot, m0 * n_qt * n_kt), pairs, *shape, sp_ptr, sp_bytes, _stream(),
-                )
-            else:
-                nQ, nK = lists.nQ, lists.nK
-                _lib.call(
-                    "fba_bwd_handover", _offset(q, qo), _offset(k, ko), _offset(v, ko), _offset(o, qo), _offset(do, qo), _offset(lse, h0 * Sq),
-                    _ptr(stats), ws_ptr, pairs * pair_bytes, _offset(dq, qo), _offset(dk, ko), _offset(dv, ko),
-                    _offset(lists.q_cnt, m0 * nQ), _offset(lists.q_idx, m0 * nQ * nK), _offset(lists.k_cnt, m0 * nK), _offset(lists.k_idx, m0 * nK * nQ),
-                    _offset(lists.pair_base, m0 * nK), _offset(lists.q_slot, m0 * nQ * nK), pairs, *shape, sp_ptr, sp_bytes, _stream(),
-                )
-    return dq, dk, dv
+    bounds = [] if dense or hand_over is False else number_pairs(lists).pair_bounds()
+    return tuple(_lib.host().backward(q, k, v, o, lse, do, q_block_size, kv_block_size, lists.mask_bh, lists.q_cnt, lists.q_idx, lists.k_cnt, lists.k_idx,
+                                      lists.pair_base, lists.q_slot, lists.k_slot, bounds, hand_over, dense, ds_workspace_limit(q, k), _split_bytes()))
 
 
 def _flex_block_attn_forward(q, k, v, q_block_size, kv_block_size, block_mask, small_block_mask, use_small_block_mode):
@@ -500,6 +409,13 @@ def flex_block_attn_func(q, k, v, q_block_size, kv_block_size, block_mask):
     q: (batch, heads, q_seq_len, 128) bf16; k, v: (batch, kv_heads, kv_seq_len, 128) bf16; block_mask: bool
     [q_seq_len / q_block_size, kv_seq_len / kv_block_size] or [batch, heads, ...]. Returns o shaped like q.
     """
+    if type(q_block_size) is int and type(kv_block_size) is int:
+        split = -1 if SPLIT_WORKSPACE_MIB is None else _split_bytes()
+        o = _lib.host().attention(q, k, v, q_block_size, kv_block_size, block_mask, DS_WORKSPACE_LIMIT_GIB * 2 ** 30, DS_WORKSPACE_FACTOR, split)
+        if o is not None:
+            return o
+    # arguments that need preparation (lengths that are no whole tiles, a mask that is not contiguous), and everything that
+    # is going to be reported
     pad_q = _pad_rows(q.shape[2], q_block_size, kv_block_size)
     pad_k = _pad_rows(k.shape[2], kv_block_size, q_block_size)
     if pad_q == 0 and pad_k == 0:

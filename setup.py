@@ -1,6 +1,6 @@
-"""pip install . / python setup.py build_ext --inplace: builds flex_block_attn_amd/csrc/libfba_gfx950.so with hipcc (the
-recipe lives in flex_block_attn_amd/build.py) and installs the two packages, flex_block_attn_amd and its import-name
-alias flex_block_attn.  No torch extension machinery is involved: the library is a plain C-ABI shared object."""
+"""pip install . / python setup.py build_ext --inplace: builds flex_block_attn_amd/csrc/libfba_gfx950.so with hipcc and the
+host module csrc/fba_torch.so against the installed torch (the recipe lives in flex_block_attn_amd/build.py) and installs
+the two packages, flex_block_attn_amd and its import-name alias flex_block_attn."""
 import os
 import sys
 
@@ -41,7 +41,7 @@ setup(
     version="1.0.0",
     description="Block-sparse attention for AMD MI355X (gfx950) with the flex-block-attn operator API",
     packages=find_packages(include=["flex_block_attn_amd", "flex_block_attn"]),
-    package_data={"flex_block_attn_amd": ["csrc/*.so", "csrc/*.hip", "csrc/*.h"]},
+    package_data={"flex_block_attn_amd": ["csrc/*.so", "csrc/*.hip", "csrc/*.cpp", "csrc/*.h"]},
     python_requires=">=3.9",
     cmdclass={"build_ext": BuildLibrary, "build_py": BuildPyWithLibrary},
 )
