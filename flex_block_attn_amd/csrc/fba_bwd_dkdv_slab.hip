@@ -18,9 +18,8 @@
 // Bound by the matrix pipe and the arithmetic between its instructions (two waves per SIMD take turns), like the 32-key
 // kernel on block lists.  Two waves share a slab instead of four, so a quarter more bytes travel L2 -> LDS than with
 // 128-key work-groups that walk the union of their halves' lists with the idle half skipping, but every wave works in every
-// step: B1 H24 S30720, independent 64 x 64 blocks, 40 % kept, dK/dV + dQ 19.2 -> 16.0 ms.  Where all halves of a tile
-// agree (k_block a multiple of 128) the same kernel is as fast as 128-key work-groups were (15.6 -> 15.9 ms with 64-row
-// query blocks, 14.9 either way when the rows agree as well).
+// step: B1 H24 S30720, independent 64 x 64 blocks, 40 % kept, dK/dV + dQ 19.2 -> 14.5 ms.  It wins where all halves of a tile
+// agree as well (15.7 -> 14.4 ms with 64-row query blocks and 128-key blocks, 14.8 -> 13.4 when the rows agree too).
 #include <type_traits>
 
 #include "fba_common.h"
@@ -181,6 +180,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     __syncthreads();  // what the counting scan left in the list is not mixed with what follows
   }
 
+  int n = fill(lo, hi);
   f32x16 acc_k[4], acc_v[4];
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
@@ -282,9 +282,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
 
   // Every chapter of the list: entry 4 i + par is this wave's slab of step i (past the end: the last entry, copied into a
   // buffer nobody reads, so that every wave has the same number of copies in flight at every wait).
-  for (;;) {
-    const int n = fill(lo, hi);
-    if (n == 0) break;
+  while (n > 0) {
     __syncthreads();  // the list is complete
     const int nsteps = (n + kPar - 1) / kPar;
     auto entry_of = [&](int step) -> int2 {
@@ -321,6 +319,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     }
     wait_vmem<0>();
     __syncthreads();  // no copy is writing LDS any more, and nobody reads the list
+    // Most lists are one chapter.  Whatever is live across a further scan goes to scratch on the way, so that scan sits here
+    // and not at the top of the loop, where every work-group would pass it: there it spilled 165 registers per lane in front
+    // of the first chapter, and B2 H22 S3584, q64 k128, 57 % kept took 883 us instead of 498.
+    n = __builtin_expect(scan_g < group && seen < hi, 0) ? fill(lo, hi) : 0;
   }
   wait_vmem<0>();
   __syncthreads();
