@@ -397,7 +397,7 @@ hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
   p.num_items = p.B * p.Hkv * (p.Skv / kTK);
   // tail splitting (one work-group per compute unit)
   void* const caller_ws = p.split.ws;  // whether or not anything is split
-  p.split = plan_split(p.num_items, 1, kSlotFloats * 4, p.split.ws, p.split_ws_bytes);
+  p.split = plan_split(p.num_items, 1, p.Hq / p.Hkv * (p.Sq / 32), 9, kSlotFloats * 4, p.split.ws, p.split_ws_bytes);
   plan_xcd_mapping(p.B * p.Hkv, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   const bool hand_over = p.ds_ws != nullptr, halves = p.q_block % 32 != 0;

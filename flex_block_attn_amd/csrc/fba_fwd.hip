@@ -389,7 +389,7 @@ hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   const int rows = wide ? 384 : 128;
   p.num_items = p.B * p.Hq * (p.Sq / rows);
   // tail splitting for the 128-row kernels (two work-groups per compute unit)
-  p.split = plan_split(p.num_items, 2, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes);
+  p.split = plan_split(p.num_items, 2, p.Skv / 32, 9, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_wgs = (p.num_items - p.split.first) * p.split.parts;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);

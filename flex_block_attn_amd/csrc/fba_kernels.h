@@ -23,8 +23,10 @@ struct SplitPlan {
 };
 
 // Items and work-group slots of a launch -> plan (first = num_items, parts = 1 when nothing is split).  `slot_bytes` is
-// what one part stores; the workspace must hold (num_items - first) * parts of them.  main_wgs is left to the launcher.
-SplitPlan plan_split(int num_items, int wgs_per_cu, int64_t slot_bytes, void* ws, int64_t ws_bytes);
+// what one part stores; the workspace must hold (num_items - first) * parts of them.  `max_steps` is the longest possible list
+// of an item in steps, `step_cost` what a step takes in units of what one part's results cost (see fba_split.hip).  main_wgs
+// is left to the launcher.
+SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, double step_cost, int64_t slot_bytes, void* ws, int64_t ws_bytes);
 
 // How the whole items of a launch are dealt to the XCDs (see xcd_remap): contiguous spans when the launch has at least
 // one (batch, head) per XCD, work-group order otherwise.  Sets items_per_xcd and the number of work-groups that come

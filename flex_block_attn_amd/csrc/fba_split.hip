@@ -52,10 +52,18 @@ hipError_t launch_queue_reset(int* queue, hipStream_t stream) {
 }
 
 // The hardware hands work-groups to free slots in index order.  With n items on s slots the last n % s items form a
-// partial round; when that round would fill at most half of the slots, each of its items is cut into floor(s / (n % s))
+// partial round; when that round would fill at most half of the slots, each of its items is cut into up to floor(s / (n % s))
 // parts (at most 8), so that the parts fill the slots once and take 1 / parts of a round.  Launches smaller than the
 // machine (n < s) are split the same way.
-SplitPlan plan_split(int num_items, int wgs_per_cu, int64_t slot_bytes, void* ws, int64_t ws_bytes) {
+//
+// How many parts pay: every part writes its partial results, and the merge reads them back, so with m items of at most
+// max_steps steps each the round takes about  max_steps step_cost / parts + m parts  in units of what one part's results
+// cost, least at parts = sqrt(max_steps step_cost / m).  The lists are on the device: step_cost assumes that 40 % of the
+// longest possible list is there.  One part's 64 KiB cost 27 ns at what the stores and the merge sustain (2.4 TB/s) and a
+// forward step of such a round 0.65 us, so forward has step_cost 9.  Measured, forward / backward in us (always as many
+// parts as slots allow, against this rule): B1 H8 S768, 128-token blocks, half kept 22.0 / 54.9 -> 15.8 / 43.0; H4 S1536
+// 23.9 / 58.5 -> 19.8 / 54.7; H8 S4096, a quarter kept 43.2 / 104.8 -> 37.0 / 92.9.
+SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, double step_cost, int64_t slot_bytes, void* ws, int64_t ws_bytes) {
   SplitPlan plan{nullptr, num_items, 1, 0};
   if (ws == nullptr || num_items <= 0) return plan;
   int slots = compute_units() * wgs_per_cu;
@@ -64,8 +72,10 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int64_t slot_bytes, void* ws
   if (rest == 0 || 2 * rest > slots) return plan;
   int parts = slots / rest;
   if (parts > 8) parts = 8;
+  const double whole = max_steps * step_cost;
+  while (parts >= 2 && (double)parts * parts * rest > whole) --parts;
   while (parts >= 2 && (int64_t)rest * parts * slot_bytes > ws_bytes) --parts;
-  if (parts < 2) return plan;
+  if (parts < 2 || whole / parts + (double)rest * parts > 0.9 * whole) return plan;
   plan.ws = static_cast<float*>(ws);
   plan.first = num_items - rest;
   plan.parts = parts;
