@@ -67,15 +67,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   }
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
   int item, part = 0, parts = 1;
-  if (grid_index < p.split.main_wgs) {
-    item = xcd_remap(grid_index, p.items_per_xcd);
+  const int slot = grid_index - p.split.main_wgs;  // where a part's results go
+  if (slot < 0) {
+    item = p.order != nullptr ? grid_index : xcd_remap(grid_index, p.items_per_xcd);
     if (item >= p.split.first) return;
   } else {
-    const int s = grid_index - p.split.main_wgs;
-    item = p.split.first + s / p.split.parts;
-    part = s - (item - p.split.first) * p.split.parts;
     parts = p.split.parts;
+    item = p.split.first + slot / parts;
+    part = slot % parts;
   }
+  if (p.order != nullptr) item = const_idx(p.order)[item];
   const int tiles_per_head = p.Skv / TK;
   const int bhk = item / tiles_per_head;
   const int kt = item - bhk * tiles_per_head;
@@ -575,7 +576,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   }
   if (parts > 1) {
     // part of a split item: unscaled fp32 partial sums go to the workspace, dV tile (parity 0), then dK tile (parity 1)
-    float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (2 * TK * kHeadDim) + par * (TK * kHeadDim) +
+    float* prow = p.split.ws + (int64_t)slot * (2 * TK * kHeadDim) + par * (TK * kHeadDim) +
                   (kg * 64 + l32) * kHeadDim;
 #pragma unroll
     for (int grp = 0; grp < 2; ++grp)
@@ -605,30 +606,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 }
 
 hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
-  p.num_items = p.B * p.Hkv * (p.Skv / 128);
-  // tail splitting (one work-group per compute unit); a part stores two 128 x 128 fp32 tiles
-  void* const caller_ws = p.split.ws;  // whether or not anything is split
-  p.split = plan_split(p.num_items, 1, p.Hq / p.Hkv * (p.Sq / 32), 6, 2 * 128 * kHeadDim * 4, p.split.ws, p.split_ws_bytes);
-  plan_xcd_mapping(p.B * p.Hkv, p.split.first, p.items_per_xcd, p.split.main_wgs);
-  const int split_items = p.num_items - p.split.first;
   void (*fn)(const BwdParams) = p.ds_ws == nullptr ? &dkdv64_kernel<kRecompute> : p.pair_base == nullptr ? &dkdv64_kernel<kDense> : &dkdv64_kernel<kNumbered>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
   if (e != hipSuccess) return e;
-  // Launches of several rounds with contiguous spans per XCD let the work-groups claim their grid indices, with some more
-  // work-groups than indices, so that an XCD that is through early takes over from the others (claim_work).
-  p.total_work = p.split.main_wgs + split_items * p.split.parts;
-  int grid = p.total_work;
-  p.queue = nullptr;
-  if (claims_wanted(p.items_per_xcd, p.total_work, 1))
-    p.queue = work_queue_in(caller_ws, p.split_ws_bytes, (int64_t)split_items * p.split.parts * 2 * 128 * kHeadDim * 4);
-  if (p.queue != nullptr) {
-    if ((e = launch_queue_reset(p.queue, stream)) != hipSuccess) return e;
-    grid += surplus_work_groups(p.total_work);
-  }
+  int grid;
+  if ((e = plan_key_tiles(p, 128, 6, 2 * 128 * kHeadDim * 4, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(256), kSmemBytes + 16, stream, p);
+  const int split_items = p.num_items - p.split.first;
   if (split_items > 0) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
-    e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, 128, outs, 2, (int64_t)p.split.first * 128, split_items, stream);
+    e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, 128, outs, 2, p.split.first, split_items, p.order, stream);
     if (e != hipSuccess) return e;
   }
   return hipGetLastError();

@@ -394,31 +394,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
 }
 
 hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
-  p.num_items = p.B * p.Hkv * (p.Skv / kTK);
-  // tail splitting (one work-group per compute unit)
-  void* const caller_ws = p.split.ws;  // whether or not anything is split
-  p.split = plan_split(p.num_items, 1, p.Hq / p.Hkv * (p.Sq / 32), 9, kSlotFloats * 4, p.split.ws, p.split_ws_bytes);
-  plan_xcd_mapping(p.B * p.Hkv, p.split.first, p.items_per_xcd, p.split.main_wgs);
-  const int split_items = p.num_items - p.split.first;
   const bool hand_over = p.ds_ws != nullptr, halves = p.q_block % 32 != 0;
   void (*fn)(const BwdParams) = hand_over ? (halves ? &dkdv_slab_kernel<true, true> : &dkdv_slab_kernel<true, false>)
                                           : (halves ? &dkdv_slab_kernel<false, true> : &dkdv_slab_kernel<false, false>);
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes);
   if (e != hipSuccess) return e;
-  // large launches let the work-groups claim their grid indices, with some work-groups more than indices (claim_work)
-  p.total_work = p.split.main_wgs + split_items * p.split.parts;
-  int grid = p.total_work;
-  p.queue = nullptr;
-  if (claims_wanted(p.items_per_xcd, p.total_work, 1))
-    p.queue = work_queue_in(caller_ws, p.split_ws_bytes, (int64_t)split_items * p.split.parts * kSlotFloats * 4);
-  if (p.queue != nullptr) {
-    if ((e = launch_queue_reset(p.queue, stream)) != hipSuccess) return e;
-    grid += surplus_work_groups(p.total_work);
-  }
+  int grid;
+  if ((e = plan_key_tiles(p, kTK, 9, kSlotFloats * 4, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes, stream, p);
+  const int split_items = p.num_items - p.split.first;
   if (split_items > 0) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, kTK * kHeadDim}};
-    return launch_partial_sum(p.split.ws, p.split.parts, kSlotFloats, kTK, outs, 2, (int64_t)p.split.first * kTK, split_items, stream);
+    return launch_partial_sum(p.split.ws, p.split.parts, kSlotFloats, kTK, outs, 2, p.split.first, split_items, p.order, stream);
   }
   return hipGetLastError();
 }

@@ -254,7 +254,7 @@ hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kSmem, stream, p);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0};
-    return launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, (int64_t)p.split.first * 128, split_items, stream);
+    return launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, p.split.first, split_items, nullptr, stream);
   }
   return hipGetLastError();
 }

@@ -260,22 +260,23 @@ struct PartialOuts {
   PartialOut out[2];
 };
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_sum_kernel(const float* ws, int parts, int64_t slot_floats,
-                                                                                          int rows, PartialOuts outs, int64_t out_row0) {
+                                                                                          int rows, PartialOuts outs, int first, const int32_t* order) {
   const int tid = threadIdx.x;
   const PartialOut& o = outs.out[blockIdx.y];
   const int row = blockIdx.x * 8 + (tid >> 5);  // among the rows of all split items
   const int c4 = (tid & 31) * 4;
   const int it = row / rows, r = row - it * rows;
+  const int64_t item = order != nullptr ? order[first + it] : first + it;
   const float* src = ws + (int64_t)it * parts * slot_floats + o.offset + r * kHeadDim + c4;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int q = 0; q < parts; ++q) acc += *reinterpret_cast<const f32x4*>(src + q * slot_floats);
-  *reinterpret_cast<bf16x4*>(o.out + (out_row0 + row) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
+  *reinterpret_cast<bf16x4*>(o.out + (item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
 }
 
-hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int64_t out_row0,
-                              int n_items, hipStream_t stream) {
+hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int first, int n_items,
+                              const int32_t* order, hipStream_t stream) {
   PartialOuts o{{outs[0], outs[n_outs - 1]}};
-  hipLaunchKernelGGL(partial_sum_kernel, dim3(n_items * (rows / 8), n_outs), dim3(256), 0, stream, ws, parts, slot_floats, rows, o, out_row0);
+  hipLaunchKernelGGL(partial_sum_kernel, dim3(n_items * (rows / 8), n_outs), dim3(256), 0, stream, ws, parts, slot_floats, rows, o, first, order);
   return hipGetLastError();
 }
 
@@ -297,7 +298,7 @@ hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kSmem, stream, p);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0};
-    e = launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, (int64_t)p.split.first * 128, split_items, stream);
+    e = launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, p.split.first, split_items, nullptr, stream);
     if (e != hipSuccess) return e;
   }
   return hipGetLastError();

@@ -111,6 +111,9 @@ struct BwdParams {
   // index i), and the number of grid indices there are to claim (see claim_work)
   int* queue;
   int total_work;
+  // dkdv64_kernel, dkdv_kernel on block lists: the item of every grid index, long lists first (null: items in xcd_remap's
+  // order; see order_items_kernel)
+  const int32_t* order;
   int64_t split_ws_bytes;  // size of split.ws as handed in by the caller
 };
 
@@ -135,15 +138,9 @@ hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream);  // block lists only: 64 keys per wave, one wave per SIMD
 hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream);  // tile lists only: 64 keys per work-group
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream);
-// Room for the claim counters behind `partial_bytes` of partial results in a tail-splitting workspace (null if there is
-// none), and the launch that zeroes them.
-int* work_queue_in(void* ws, int64_t ws_bytes, int64_t partial_bytes);
-// Is a launch of `total_work` grid indices at `wgs_per_cu` work-groups per compute unit worth claiming?  (At least four
-// rounds; FBA_CLAIM_WORK=0 in the environment switches claiming off, for measurements.)
-bool claims_wanted(int items_per_xcd, int total_work, int wgs_per_cu);
-// Work-groups launched on top of the grid indices of a claiming launch: an eighth more, a whole number per XCD.
-inline int surplus_work_groups(int total_work) { return (total_work / 8 + 7) / 8 * 8; }
-hipError_t launch_queue_reset(int* queue, hipStream_t stream);
+// Shape of a dK/dV launch over key tiles of `tile_rows` rows, whose parts store `slot_bytes` each: sets p.num_items, split,
+// items_per_xcd, order, queue and total_work and the number of work-groups, and launches what has to run in front.
+hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t slot_bytes, int& grid, hipStream_t stream);
 int device_compute_units();
 // One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats).
 struct PartialOut {
@@ -151,8 +148,9 @@ struct PartialOut {
   float scale;
   int64_t offset;
 };
-hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int64_t out_row0,
-                              int n_items, hipStream_t stream);
+// Items [first, first + n_items) were split; order: null, or the item of every grid index.
+hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int first, int n_items,
+                              const int32_t* order, hipStream_t stream);
 hipError_t launch_probe_mfma(const float* src, float* sink, int work_groups, int iters, hipStream_t stream);
 hipError_t launch_probe_read(const void* src, int64_t bytes, uint32_t* sink, int work_groups, hipStream_t stream);
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,

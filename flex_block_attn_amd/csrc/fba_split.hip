@@ -27,30 +27,6 @@ int compute_units() {
 
 int device_compute_units() { return compute_units(); }
 
-namespace {
-constexpr int kQueueBytes = 256;
-__global__ void queue_reset_kernel(int* queue) { queue[threadIdx.x] = 0; }
-}  // namespace
-
-bool claims_wanted(int items_per_xcd, int total_work, int wgs_per_cu) {
-  const char* e = getenv("FBA_CLAIM_WORK");
-  const bool off = e != nullptr && e[0] == '0';
-  (void)items_per_xcd;  // either mapping deals grid index i to XCD i % 8, which is all a claim relies on
-  return !off && total_work >= 4 * compute_units() * wgs_per_cu;
-}
-
-int* work_queue_in(void* ws, int64_t ws_bytes, int64_t partial_bytes) {
-  if (ws == nullptr) return nullptr;
-  const int64_t off = (ws_bytes - kQueueBytes) & ~(int64_t)15;
-  if (off < partial_bytes) return nullptr;
-  return reinterpret_cast<int*>(static_cast<char*>(ws) + off);
-}
-
-hipError_t launch_queue_reset(int* queue, hipStream_t stream) {
-  hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(kQueueBytes / 4), 0, stream, queue);
-  return hipGetLastError();
-}
-
 // The hardware hands work-groups to free slots in index order.  With n items on s slots the last n % s items form a
 // partial round; when that round would fill at most half of the slots, each of its items is cut into up to floor(s / (n % s))
 // parts (at most 8), so that the parts fill the slots once and take 1 / parts of a round.  Launches smaller than the
@@ -80,6 +56,110 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, double step_c
   plan.first = num_items - rest;
   plan.parts = parts;
   return plan;
+}
+
+namespace {
+
+constexpr int kQueueBytes = 256;
+constexpr int kRankBlock = 256;
+
+__global__ void queue_reset_kernel(int* queue) { queue[threadIdx.x] = 0; }
+
+// Which item every grid index of a dK/dV launch works on: long lists first.  The lists of a random mask differ by 10-20 %
+// in length, so with items in index order the last round of work-groups ends with the longest list that happened to start
+// last; in falling order of length the last ones to start are the short ones.  An item's key is the number of listed
+// query blocks over the query heads of its group.
+//
+// The items are dealt to `spans` runs (one per XCD, whose work-groups get the grid indices XCD, XCD + 8, ..., or a single one),
+// every run is cut into segments of `segment` items counted from its end, and each segment is sorted by counting, for every
+// item, the items of the segment in front of it (longer, or as long with a lower number): no atomics, one result.  Segments
+// keep the heads of a large launch one after the other, so that work-groups that run together still share Q and dO in L2.
+// Grid: spans * ceil(longest run / 256) blocks.
+__global__ __attribute__((amdgpu_flat_work_group_size(kRankBlock, kRankBlock))) void order_items_kernel(const BwdParams p, int spans, int segment, int32_t* order) {
+  __shared__ int lens[kRankBlock];
+  const int tid = threadIdx.x;
+  if (p.queue != nullptr && blockIdx.x == 0 && tid < kQueueBytes / 4) p.queue[tid] = 0;
+  const int span = blockIdx.x % spans, i0 = blockIdx.x / spans * kRankBlock;
+  const int start = span * (p.num_items / spans) + min(span, p.num_items % spans);
+  const int count = p.num_items / spans + (span < p.num_items % spans);
+  if (i0 >= count) return;
+  const int tiles_per_head = p.Skv / 128, group = p.Hq / p.Hkv;
+  auto length = [&](int i) {  // of item i of the run
+    const int item = start + i;
+    const int bhk = item / tiles_per_head, kblk = (item - bhk * tiles_per_head) * 128 / p.k_block;
+    if (p.mask_bh == 1) return p.k_cnt[kblk];
+    const int64_t row = (int64_t)bhk * group * p.nK + kblk;  // query heads of a kv head are consecutive
+    int n = 0;
+    for (int g = 0; g < group; ++g) n += p.k_cnt[row + (int64_t)g * p.nK];
+    return n;
+  };
+  auto segment_end = [&](int i) { return count - (count - 1 - i) / segment * segment; };
+  const int i = min(i0 + tid, count - 1);
+  const int own = length(i), hi = segment_end(i), lo = max(0, hi - segment);
+  const int from = max(0, segment_end(i0) - segment), to = segment_end(min(i0 + kRankBlock, count) - 1);  // of all items of the block
+  int rank = lo;
+  for (int j0 = from; j0 < to; j0 += kRankBlock) {
+    __syncthreads();
+    lens[tid] = length(min(j0 + tid, count - 1));
+    __syncthreads();
+    const int first = max(lo, j0), last = min(hi, j0 + kRankBlock);
+    for (int j = first; j < last; ++j) {
+      const int other = lens[j - j0];
+      rank += other > own || (other == own && j < i);
+    }
+  }
+  if (i0 + tid < count) order[(int64_t)rank * spans + span] = start + i;
+}
+
+}  // namespace
+
+hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t slot_bytes, int& grid, hipStream_t stream) {
+  const int slots = compute_units();  // one work-group per compute unit
+  const int heads = p.B * p.Hkv;
+  char* const ws = reinterpret_cast<char*>(p.split.ws);  // whether or not anything is split
+  p.num_items = heads * (p.Skv / tile_rows);
+  p.split = plan_split(p.num_items, 1, p.Hq / p.Hkv * (p.Sq / 32), step_cost, slot_bytes, ws, p.split_ws_bytes);
+  plan_xcd_mapping(heads, p.split.first, p.items_per_xcd, p.split.main_wgs);
+  const int parts = (p.num_items - p.split.first) * p.split.parts;
+  p.queue = nullptr;
+  p.order = nullptr;
+
+  // What else lives in the workspace, from its end: the claim counters, then the order of the items.
+  int64_t top = ws == nullptr ? 0 : (p.split_ws_bytes - kQueueBytes) & ~(int64_t)15;
+  const int64_t bottom = parts * slot_bytes;
+  int* const queue = ws != nullptr && top >= bottom ? reinterpret_cast<int*>(ws + top) : nullptr;
+  top = (top - (int64_t)p.num_items * 4) & ~(int64_t)15;
+  // Items are ordered where they start in more than one round and in at most eight, and the longest possible list has at
+  // least 128 slabs.  One round starts everything at once; over many rounds the spread of the last one no longer counts, while
+  // tiles in index order share more of their lists in L2 (structured masks): measured, steps with items in index order /
+  // ordered, B2 H16/4 S8192 (2 rounds) 1113 / 1062 us, B1 H24 S30720 random (7.5 rounds per chunk) 16.53 / 16.04 ms, H24
+  // S69120 top-k (17 rounds) 25.3 / 25.2 ms, H24 S115200 sliding window (28 rounds) 52.1 / 52.9 ms.  With shorter lists the
+  // spread is worth less than the launch (3 us).
+  const bool ordered = !p.tiled && queue != nullptr && top >= bottom && p.num_items > slots && p.num_items <= 8 * slots && p.Hq / p.Hkv * (p.Sq / 32) >= 128;
+  if (ordered) p.split.main_wgs = p.split.first;
+
+  // Launches of four rounds and more let the work-groups claim their grid indices, with some more work-groups than indices,
+  // so that an XCD that is through early takes over from the others (claim_work; either mapping deals grid index i to XCD
+  // i % 8, which is all a claim relies on).  FBA_CLAIM_WORK=0 switches claiming off, for measurements.
+  p.total_work = p.split.main_wgs + parts;
+  grid = p.total_work;
+  const char* claim = getenv("FBA_CLAIM_WORK");
+  if (queue != nullptr && !(claim != nullptr && claim[0] == '0') && p.total_work >= 4 * slots) {
+    p.queue = queue;
+    grid += (p.total_work / 8 + 7) / 8 * 8;  // an eighth more work-groups, a whole number per XCD
+  }
+  if (ordered) {
+    const int spans = heads >= 8 ? 8 : 1;
+    const int tiles_per_head = p.Skv / tile_rows, two_rounds = 2 * slots / spans;
+    const int segment = (two_rounds + tiles_per_head - 1) / tiles_per_head * tiles_per_head;
+    const int blocks = spans * (((p.num_items + spans - 1) / spans + kRankBlock - 1) / kRankBlock);
+    int32_t* const order = reinterpret_cast<int32_t*>(ws + top);
+    hipLaunchKernelGGL(order_items_kernel, dim3(blocks), dim3(kRankBlock), 0, stream, p, spans, segment, order);
+    p.order = order;
+  } else if (p.queue != nullptr) {
+    hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(kQueueBytes / 4), 0, stream, p.queue);
+  }
+  return hipGetLastError();
 }
 
 }  // namespace fba
