@@ -15,6 +15,7 @@
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/custom_class.h>
 #include <torch/extension.h>
 
@@ -326,6 +327,11 @@ struct Attention : torch::autograd::Function<Attention> {
 // have to be padded), which Python then reports or prepares.
 c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t q_block, int64_t k_block, const at::Tensor& mask,
                                     double limit, double factor, int64_t split_bytes) {
+  // a traced call has to appear in the trace, and forward-mode differentiation has to be refused: both go through the Python
+  // autograd function, which does that
+  if (torch::jit::tracer::isTracing()) return c10::nullopt;
+  for (const at::Tensor* t : {&q, &k, &v})
+    if (t->_fw_grad(0).defined()) return c10::nullopt;
   for (const at::Tensor* t : {&q, &k, &v})
     if (!t->is_cuda() || t->scalar_type() != at::kBFloat16 || t->dim() != 4 || !t->is_contiguous() || t->size(3) != kHeadDim ||
         t->device() != q.device() || (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) != 0)
