@@ -355,34 +355,349 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     }
 }
 
+// Forward on tile lists whose tiles are not of one mind: q_block no multiple of 128, so the two 64-row halves of a 128-row
+// tile select key blocks of their own.
+//
+// Work-group = 64 query rows, four waves, two work-groups per CU.  The unit of work is a chunk of 64 keys; wave w owns rows
+// 32 (w % 2) .. +31 against keys 32 (w / 2) .. +31 of every chunk, with the same pipeline as fwd_kernel (P_{t-1} V_{t-1} |
+// softmax of S_t | S_{t+1}).  The two waves of a row group keep softmax statistics and O of their own, which meet in LDS at
+// the end.  Rings of three K chunks and two V chunks (80 KiB, half of a CU's LDS): step t requests V_t and K_{t+3}.
+// The list is that of the 128-row tile; every wave keeps 64 of its entries in a register, one per lane, with a scalar mask of
+// those that name this half, and takes them in order: no list in LDS, no scalar loads to wait for, only selected chunks.
+//
+// Bound like fwd_kernel by the matrix pipe, the softmax between its instructions and the clock these allow.  A chunk feeds half
+// as many matrix instructions per byte copied as there, but with 128-row work-groups a chunk that one half selects kept the
+// waves of the other waiting: B1 H24 S30720, independent 64 x 64 blocks, 40 % kept, a tile's list holds 64 % of the blocks and
+// the step took 21.98 ms, now 19.30; B2 H8/2 S3136 q16 k64, a quarter kept, 301 -> 289 us.
+//
+// kRows: q_block is no multiple of 64, so the four 16-row groups of a half differ as well: a wave leaves out the matrix work
+// of chunks that neither of its groups selects, rows switched off inside an active wave are dealt with by selects.
+constexpr int kChunkBytes = 2 * kSlabBytes;  // 64 keys
+constexpr int kHalfRows = 64;
+constexpr int kHalfSlotBytes = (kHalfRows * kHeadDim + 2 * kHalfRows) * 4;  // partial result of one part of a split item
+constexpr int kHalfSmem = 5 * kChunkBytes;
+
+// The entries of a tile list that name one 64-row half, in order.  All lanes of a wave call everything together.
+struct HalfList {
+  const int32_t* list;
+  int cnt, half_mask, lane;
+  int base;                  // position of `entries` in the list
+  int entries, ahead;        // this lane's entry among the 64 at `base` and the 64 behind them
+  unsigned long long left;   // lanes whose entry names the half and has not been taken
+
+  FBA_DEVICE int load(int at) const { return at + lane < cnt ? list[at + lane] : 0; }
+  FBA_DEVICE unsigned long long named(int e) const { return __builtin_amdgcn_ballot_w64((e & half_mask) != 0); }
+  FBA_DEVICE int total() const {
+    int n = 0;
+    for (int at = 0; at < cnt; at += 256) {  // four loads in flight
+      const int e0 = load(at), e1 = load(at + 64), e2 = load(at + 128), e3 = load(at + 192);
+      n += __popcll(named(e0)) + __popcll(named(e1)) + __popcll(named(e2)) + __popcll(named(e3));
+    }
+    return n;
+  }
+  // next() gives entry number `skip` of those that name the half
+  FBA_DEVICE void start(int skip) {
+    base = 0;
+    entries = load(0);
+    ahead = load(64);
+    left = named(entries);
+    while (__popcll(left) <= skip && base + 64 < cnt) {
+      skip -= __popcll(left);
+      refill();
+    }
+    for (; skip > 0; --skip) left &= left - 1;
+  }
+  FBA_DEVICE void refill() {
+    base += 64;
+    entries = ahead;
+    ahead = load(base + 64);
+    left = named(entries);
+  }
+  FBA_DEVICE bool next(int& entry) {
+    while (left == 0) {
+      if (base + 64 >= cnt) return false;
+      refill();
+    }
+    entry = __builtin_amdgcn_readlane(entries, __builtin_ctzll(left));
+    left &= left - 1;
+    return true;
+  }
+};
+
+template <bool kRows>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void fwd_half_kernel(const FwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // K ring [3][16 KiB] | V ring [2][16 KiB]
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rg = wave & 1, par = wave >> 1;  // row group, 32-key slab of a chunk
+  int item, part = 0, parts = 1;
+  if ((int)blockIdx.x < p.split.main_wgs) {
+    item = xcd_remap(blockIdx.x, p.items_per_xcd);
+    if (item >= p.split.first) return;
+  } else {
+    const int s = blockIdx.x - p.split.main_wgs;
+    item = p.split.first + s / p.split.parts;
+    part = s - (item - p.split.first) * p.split.parts;
+    parts = p.split.parts;
+  }
+  const int tiles_per_head = p.Sq / kHalfRows;
+  const int bh = item / tiles_per_head;
+  const int qt = item - bh * tiles_per_head;
+  const int half = qt & 1;  // of the 128-row tile whose list this is
+  const int b = bh / p.Hq, hq = bh - b * p.Hq;
+  const int hkv = hq / (p.Hq / p.Hkv);
+  const int64_t qrow0 = (int64_t)bh * p.Sq + (int64_t)qt * kHalfRows + rg * 32;
+  const __bf16* qp = p.q + qrow0 * kHeadDim;
+  const char* kp = reinterpret_cast<const char*>(p.k + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
+  const char* vp = reinterpret_cast<const char*>(p.v + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
+
+  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (p.Sq / 128) + (qt >> 1);
+  HalfList cursor;
+  cursor.list = p.q_idx + mrow * p.nK;
+  cursor.cnt = const_idx(p.q_cnt)[mrow];
+  cursor.half_mask = 15 << (4 * half);
+  cursor.lane = lane;
+
+  FwdState st;
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) st.qreg[ks] = *reinterpret_cast<const bf16x8*>(qp + (int64_t)l32 * kHeadDim + 16 * ks + 8 * h);
+  const int per_block = p.k_block / 64;
+  const int chunks = cursor.total() * per_block;
+  const int t_begin = (int)((int64_t)chunks * part / parts), t_end = (int)((int64_t)chunks * (part + 1) / parts);
+  const int nsteps = t_end - t_begin;
+
+  st.rm.init(lane);
+  st.tr.init(lane);
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) st.rm.rd[ks] += par * kSlabBytes;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb) {
+    st.tr.rd[mb][0] += par * kSlabBytes;
+    st.tr.rd[mb][1] += par * kSlabBytes;
+  }
+  st.c = p.scale_log2e;
+  st.m_run = kRows ? -1e30f : -INFINITY;  // finite where whole slabs can be masked out, so that exp2 never sees inf - inf
+  st.l_run = 0.f;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st.acc_o[mb][r] = 0.f;
+
+  char* const k_lds = smem;
+  char* const v_lds = smem + 3 * kChunkBytes;
+  // wave w brings in rows 16 w .. 16 w + 15 of every chunk, four copies each of K and V
+  uint32_t dma_off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 16 * wave + 4 * i + (lane >> 4);
+    dma_off[i] = (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4));
+  }
+  const uint32_t k_dst = lds_addr(k_lds) + 16 * wave * kRowBytes, v_dst = lds_addr(v_lds) + 16 * wave * kRowBytes;
+
+  if (nsteps > 0) {
+    // a chunk: number of its first key / 64, predicate bits of the half's four row groups in the low bits
+    cursor.start(t_begin / per_block);
+    int entry = 0;
+    cursor.next(entry);
+    int chunk = (((entry >> 8) * per_block + t_begin % per_block) << 4) | ((entry >> (4 * half)) & 15);
+    int rem = per_block - t_begin % per_block;
+    auto next_chunk = [&]() -> int {  // past the end: the last one again
+      const int now = chunk;
+      if (--rem > 0) {
+        chunk += 16;
+      } else if (cursor.next(entry)) {
+        rem = per_block;
+        chunk = ((entry >> 8) * per_block << 4) | ((entry >> (4 * half)) & 15);
+      } else {
+        rem = 1;
+      }
+      return now;
+    };
+    auto source = [](const char* base, int c) { return base + (int64_t)(c >> 4) * kChunkBytes; };
+    auto copy_piece = [&](int i, uint32_t dst, const char* src) { dma16(dst + 4 * i * kRowBytes, src, dma_off[i]); };
+    int c0 = next_chunk(), c1 = next_chunk(), c2 = next_chunk();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) copy_piece(i, k_dst, source(kp, c0));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) copy_piece(i, k_dst + kChunkBytes, source(kp, c1));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) copy_piece(i, k_dst + 2 * kChunkBytes, source(kp, c2));
+    int c3 = next_chunk();
+    wait_vmem<4>();  // K_0 and K_1
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) pin(st.qreg[ks]);
+    f32x16 s_cur = qk_half(st, k_lds);
+    pin(s_cur);
+    __syncthreads();  // K_3 goes where K_0 was
+
+    bf16x8 p_prev[2];
+    const int wave_bits = 3 << (2 * rg), group_bit = 1 << (2 * rg + (l32 >> 4));
+    bool w_prev = false;  // did this wave form P for the previous chunk?
+    // step t, RK = t % 3, RV = t % 2
+    auto step = [&](auto rk_c, auto rv_c, auto first_c) {
+      constexpr int RK = decltype(rk_c)::value, RV = decltype(rv_c)::value;
+      constexpr bool kFirst = decltype(first_c)::value;
+      const bool w_cur = !kRows || (c0 & wave_bits) != 0, w_nxt = !kRows || (c1 & wave_bits) != 0;
+      const char* const k_src = source(kp, c3);
+      const char* const v_src = source(vp, c0);
+      auto copies = [&](int i) {
+        if (i < 4) copy_piece(i, v_dst + RV * kChunkBytes, v_src);
+        else copy_piece(i - 4, k_dst + RK * kChunkBytes, k_src);
+      };
+      if (!kFirst && (!kRows || w_prev)) {
+        pv_half(st, v_lds + (1 - RV) * kChunkBytes, p_prev, copies);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) copies(i);
+      }
+      const bool active = !kRows || (c0 & group_bit) != 0;
+      if (w_cur) softmax_reference(st, s_cur, active);
+      f32x16 s_nxt;
+      if (w_nxt) s_nxt = qk_half(st, k_lds + ((RK + 1) % 3) * kChunkBytes);  // past the last chunk: stale data, unused
+      else s_nxt = s_cur;
+      if (w_cur) softmax_exp<kRows>(st, s_cur, p_prev, active);
+      w_prev = w_cur;
+      pin(p_prev[0]);
+      pin(p_prev[1]);
+      s_cur = s_nxt;
+      c0 = c1;
+      c1 = c2;
+      c2 = c3;
+      c3 = next_chunk();
+      // V_t and K_{t+2} must have landed; the four copies of K_{t+3} may still fly.  (A list load among them only makes the
+      // wait stricter.)
+      wait_vmem<4>();
+      __syncthreads();
+    };
+    step(IC<0>{}, IC<0>{}, std::true_type{});
+    for (int t = 1; t < nsteps; t += 6) {
+      step(IC<1>{}, IC<1>{}, std::false_type{});
+      if (t + 1 >= nsteps) break;
+      step(IC<2>{}, IC<0>{}, std::false_type{});
+      if (t + 2 >= nsteps) break;
+      step(IC<0>{}, IC<1>{}, std::false_type{});
+      if (t + 3 >= nsteps) break;
+      step(IC<1>{}, IC<0>{}, std::false_type{});
+      if (t + 4 >= nsteps) break;
+      step(IC<2>{}, IC<1>{}, std::false_type{});
+      if (t + 5 >= nsteps) break;
+      step(IC<0>{}, IC<0>{}, std::false_type{});
+    }
+    if (!kRows || w_prev) pv_half(st, v_lds + ((nsteps - 1) & 1) * kChunkBytes, p_prev);
+  }
+  wait_vmem<0>();  // no copy is writing LDS any more
+  __syncthreads();
+
+  // The two waves of a row group: each hands the other half of its O^T (64 of the 128 columns) and its statistics
+  const int keep = 2 * par;  // this wave ends up with accumulators keep, keep + 1
+  {
+    f32x4* dst = reinterpret_cast<f32x4*>(smem + wave * kSlabBytes) + lane;
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& a = par ? st.acc_o[mb] : st.acc_o[mb + 2];
+        dst[(mb * 4 + g) * 64] = (f32x4){a[4 * g + 0], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+      }
+    float* stat = reinterpret_cast<float*>(smem + 4 * kSlabBytes) + wave * 128;
+    stat[lane] = st.m_run;
+    stat[64 + lane] = st.l_run;
+  }
+  __syncthreads();
+  const int other = wave ^ 2;
+  const float* stat = reinterpret_cast<const float*>(smem + 4 * kSlabBytes) + other * 128;
+  const float m_other = stat[lane];
+  const float m = fmaxf(st.m_run, m_other);
+  const float w_own = st.m_run == -INFINITY ? 0.f : fast_exp2((st.m_run - m) * st.c);
+  const float w_other = m_other == -INFINITY ? 0.f : fast_exp2((m_other - m) * st.c);
+  const float l = sum_halves(w_own * st.l_run + w_other * stat[64 + lane]);
+  f32x4 out[2][4];
+  {
+    const f32x4* src = reinterpret_cast<const f32x4*>(smem + other * kSlabBytes) + lane;
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& a = par ? st.acc_o[mb + 2] : st.acc_o[mb];
+        const f32x4 o = src[(mb * 4 + g) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[mb][g][e] = w_own * a[4 * g + e] + w_other * o[e];
+      }
+  }
+  if (parts > 1) {  // as in fwd_kernel
+    float* slot = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (kHalfSlotBytes / 4);
+    float* prow = slot + (rg * 32 + l32) * kHeadDim;
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(prow + 32 * (keep + mb) + 8 * g + 4 * h) = out[mb][g];
+    if (h == 0 && par == 0) {
+      slot[kHalfRows * kHeadDim + rg * 32 + l32] = m * st.c;
+      slot[kHalfRows * kHeadDim + kHalfRows + rg * 32 + l32] = l;
+    }
+    return;
+  }
+  __bf16* orow = p.o + (qrow0 + l32) * kHeadDim;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (h == 0 && par == 0) p.lse[qrow0 + l32] = l > 0.f ? (m * st.c + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<bf16x4*>(orow + 32 * (keep + mb) + 8 * g + 4 * h) =
+          pack4(out[mb][g][0] * inv, out[mb][g][1] * inv, out[mb][g][2] * inv, out[mb][g][3] * inv);
+}
+
 // Combines the parts of the split items: O = sum_p 2^(m_p - m) O_p / sum_p 2^(m_p - m) l_p with m = max_p m_p, in part
 // order.  One thread per (query row, four head-dim columns).
+template <int kTileRows>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge_kernel(const FwdParams p) {
   const int tid = threadIdx.x;
-  const int row = blockIdx.x * 8 + (tid >> 5), c4 = (tid & 31) * 4;  // row among the 128 * (split items) rows
-  const int it = row >> 7, r = row & 127;
+  constexpr int kSlotFloats = kTileRows * kHeadDim + 2 * kTileRows;
+  const int row = blockIdx.x * 8 + (tid >> 5), c4 = (tid & 31) * 4;  // row among the kTileRows * (split items) rows
+  const int it = row / kTileRows, r = row % kTileRows;
   const int item = p.split.first + it;
   const int parts = p.split.parts;
-  const float* slot0 = p.split.ws + (int64_t)it * parts * (kFwdSlotBytes / 4);
+  const float* slot0 = p.split.ws + (int64_t)it * parts * kSlotFloats;
   float m = -INFINITY;
-  for (int q = 0; q < parts; ++q) m = fmaxf(m, slot0[(int64_t)q * (kFwdSlotBytes / 4) + 128 * kHeadDim + r]);
+  for (int q = 0; q < parts; ++q) m = fmaxf(m, slot0[(int64_t)q * kSlotFloats + kTileRows * kHeadDim + r]);
   float l = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int q = 0; q < parts; ++q) {
-    const float* slot = slot0 + (int64_t)q * (kFwdSlotBytes / 4);
-    const float mq = slot[128 * kHeadDim + r];
+    const float* slot = slot0 + (int64_t)q * kSlotFloats;
+    const float mq = slot[kTileRows * kHeadDim + r];
     const float w = mq == -INFINITY ? 0.f : fast_exp2(mq - m);
-    l += w * slot[128 * kHeadDim + 128 + r];
+    l += w * slot[kTileRows * kHeadDim + kTileRows + r];
     const f32x4 o4 = *reinterpret_cast<const f32x4*>(slot + r * kHeadDim + c4);
     acc += w * o4;
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  const int64_t orow = (int64_t)item * 128 + r;  // items are consecutive 128-row tiles of [B, Hq, Sq]
+  const int64_t orow = (int64_t)item * kTileRows + r;  // items are consecutive tiles of [B, Hq, Sq]
   *reinterpret_cast<bf16x4*>(p.o + orow * kHeadDim + c4) = pack4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
   if (c4 == 0) p.lse[orow] = l > 0.f ? (m + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
 }
 
+namespace {
+
+hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
+  void (*fn)(const FwdParams) = p.q_block % 64 != 0 ? &fwd_half_kernel<true> : &fwd_half_kernel<false>;
+  p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
+  // two work-groups per compute unit; a step is as long as one of fwd_kernel, a part's results are half as large
+  p.split = plan_split(p.num_items, 2, p.Skv / 64, 18, kHalfSlotBytes, p.split.ws, p.split_ws_bytes);
+  plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
+  const int split_items = p.num_items - p.split.first;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kHalfSmem);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kHalfSmem, stream, p);
+  if (split_items > 0) hipLaunchKernelGGL(fwd_merge_kernel<kHalfRows>, dim3(split_items * kHalfRows / 8), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
+  if (p.tiled && p.q_block % 128 != 0) return launch_fwd_halves(p, stream);
   constexpr int kSmem = 2 * kRing * kSlabBytes;
   const bool wide = !p.tiled && p.q_block % 384 == 0 && p.variant != 1;
   void (*fn)(const FwdParams) = p.tiled ? &fwd_kernel<true, 4> : wide ? &fwd_kernel<false, 12> : &fwd_kernel<false, 4>;
@@ -395,7 +710,7 @@ hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs), dim3(rows * 2), kSmem, stream, p);
-  if (split_wgs > 0) hipLaunchKernelGGL(fwd_merge_kernel, dim3((p.num_items - p.split.first) * 16), dim3(256), 0, stream, p);
+  if (split_wgs > 0) hipLaunchKernelGGL(fwd_merge_kernel<128>, dim3((p.num_items - p.split.first) * 16), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
