@@ -76,7 +76,7 @@ FBA_DEVICE void pv_half(FwdState& st, const char* v_half, const bf16x8 (&pk)[2])
 
 // Raise the softmax reference if some row of the wave would otherwise see exponents above kLazy.  Until then
 // P = exp2(c (S - m)) may exceed 1, which fp32 sums and bf16 P both carry.
-// `active` is false for a query row whose own mask block does not select the current key block (tile lists only).
+// `active` is false for a query row whose own mask block does not select the current key block (q_block no multiple of 64 only).
 FBA_DEVICE void softmax_reference(FwdState& st, const f32x16& s, bool active) {
   float mx = s[0];
 #pragma unroll
@@ -96,13 +96,13 @@ FBA_DEVICE void softmax_reference(FwdState& st, const f32x16& s, bool active) {
 }
 
 // P^T = exp2(c S^T - c m), packed to bf16 as the B operand of the two 16-key MFMA steps.
-template <bool kTiled>
+template <bool kRows>
 FBA_DEVICE void softmax_exp(FwdState& st, f32x16& s, bf16x8 (&pk)[2], bool active) {
   const float mc = st.m_run * st.c;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     s[r] = fast_exp2(__builtin_fmaf(s[r], st.c, -mc));
-    if constexpr (kTiled) s[r] = active ? s[r] : 0.f;
+    if constexpr (kRows) s[r] = active ? s[r] : 0.f;
   }
 #pragma unroll
   for (int j = 0; j < 2; ++j)
@@ -118,17 +118,15 @@ FBA_DEVICE void softmax_exp(FwdState& st, f32x16& s, bf16x8 (&pk)[2], bool activ
 
 }  // namespace
 
-// kTiled = false: q_block is a multiple of 128, the list of a work-group is the block list of its query block.
-// kTiled = true: tile lists with a predicate per 16-row group (any q_block that is a multiple of 16).
-// kWaves = 4: 128 query rows per work-group, two work-groups per CU.  kWaves = 12 (q_block a multiple of 384, block
-// lists): 384 rows, one work-group per CU with three waves per SIMD; every K / V slab brought into LDS then feeds three
+// Block lists: q_block and k_block are multiples of 128, the list of a work-group is that of its query block.
+// kWaves = 4: 128 query rows per work-group, two work-groups per CU.  kWaves = 12 (q_block a multiple of 384):
+// 384 rows, one work-group per CU with three waves per SIMD; every K / V slab brought into LDS then feeds three
 // times as many matrix instructions (the reference shares its K / V tiles between three consumer groups for the same
 // reason, flex_block_attn_h100.cu:912-928).
-template <bool kTiled, int kWaves>
+template <int kWaves>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(kWaves == 12 ? 3 : 2, kWaves == 12 ? 3 : 2))) void fwd_kernel(const FwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // K ring [4][8 KiB] | V ring [4][8 KiB]
   constexpr int TQ = 32 * kWaves;
-  static_assert(!kTiled || kWaves == 4, "tile lists describe 128-row tiles");
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -154,12 +152,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const char* kp = reinterpret_cast<const char*>(p.k + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
   const char* vp = reinterpret_cast<const char*>(p.v + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
 
-  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (kTiled ? tiles_per_head : p.nQ) + (kTiled ? qt : (qt * TQ) / p.q_block);
+  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * p.nQ + (qt * TQ) / p.q_block;
   const int cnt = p.q_cnt[mrow];
   const ConstIdx idx = const_idx(p.q_idx + mrow * p.nK);
-  auto key_block = [&](int e) -> int { return kTiled ? idx[e] >> 8 : idx[e]; };
-  // predicate bit of this lane's 16-row group in a tile-list entry
-  const int group_bit = 1 << (2 * wave + (l32 >> 4));
   const int nsub = p.k_block / kSlab;
   // this work-group's range of 32-key steps of the list: all of it, or part `part` of `parts` (even boundaries)
   const int steps_all = cnt * nsub;
@@ -175,7 +170,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   st.rm.init(lane);
   st.tr.init(lane);
   st.c = p.scale_log2e;
-  st.m_run = kTiled ? -1e30f : -INFINITY;  // finite where whole slabs can be masked out, so that exp2 never sees inf - inf
+  st.m_run = -INFINITY;
   st.l_run = 0.f;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
@@ -193,15 +188,15 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   // the scalar load is off the critical path.  V requests trail K requests by two slabs and reuse their offsets.
   const int64_t block_bytes = (int64_t)p.k_block * kRowBytes;
   int e_next = e_begin + 1, rem = nsub - sub_begin;
-  int64_t src_off = nsteps > 0 ? key_block(e_begin) * block_bytes + (int64_t)sub_begin * kSlabBytes : 0;
-  int blk_next = e_next < cnt ? key_block(e_next) : 0;
+  int64_t src_off = nsteps > 0 ? idx[e_begin] * block_bytes + (int64_t)sub_begin * kSlabBytes : 0;
+  int blk_next = e_next < cnt ? idx[e_next] : 0;
   auto next_off = [&]() -> int64_t {
     const int64_t off = src_off;
     if (--rem == 0) {
       rem = nsub;
       src_off = blk_next * block_bytes;
       ++e_next;
-      blk_next = e_next < cnt ? key_block(e_next) : 0;
+      blk_next = e_next < cnt ? idx[e_next] : 0;
     } else {
       src_off += kSlabBytes;
     }
@@ -237,31 +232,21 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     int64_t hist0 = off[4], hist1 = off[3];  // offsets of the two youngest K requests
 
     bf16x8 p_prev[2];
-    // predicate of the slab whose softmax is next (tile lists): all 16-row groups share the entry, each lane tests its bit
-    int e_cmp = e_begin, rem_cmp = nsub - sub_begin;
-    int bits_cmp = kTiled ? idx[e_begin] & 255 : 255;
-    int bits_ahead = kTiled && e_begin + 1 < cnt ? idx[e_begin + 1] & 255 : 0;  // predicate bits of the following list entry
-    // A wave whose two 16-row groups are both switched off for a slab leaves that slab's matrix work out altogether
-    // (wave-uniform branches); rows switched off inside an active wave are dealt with by selects.
-    const int wave_bits = 3 << (2 * wave);
-    bool w_prev = false;  // did this wave form P for the previous slab?
     // The copies a step requests (K_{t+5} into the buffer of K_{t+1}, V_{t+3} into that of V_{t-1}, both free behind the
     // step's barrier) are issued by the following step, in between its first matrix instructions where the work-group
-    // has block lists and four waves: a copy takes a wave tens of cycles to issue, which the matrix pipe then covers.
+    // has four waves: a copy takes a wave tens of cycles to issue, which the matrix pipe then covers.
     // Every step requests both, so that the counter of copies in flight means the same thing at every wait; past the end
     // of the list they repeat a listed slab into a buffer that nobody reads any more.
     uint32_t owed_k_dst = 0, owed_v_dst = 0;
     const char* owed_k_src = kp;
     const char* owed_v_src = vp;
     bool owed = false;
-    constexpr bool kSpread = !kTiled && kWaves == 4;
+    constexpr bool kSpread = kWaves == 4;
 
     // step t (t % 4 == R): O += P_{t-1} V_{t-1} | softmax(S_t) | S_{t+1} = K_{t+1} Q^T
     auto step = [&](auto ring_c, auto first_c, int t) {
       constexpr int R = decltype(ring_c)::value;
       constexpr bool kFirst = decltype(first_c)::value;
-      const bool w_cur = !kTiled || (bits_cmp & wave_bits) != 0;
-      const bool w_nxt = !kTiled || ((rem_cmp > 1 ? bits_cmp : bits_ahead) & wave_bits) != 0;
       // P_{t-1} was formed against the reference m of step t-1, so it must reach O before step t may raise m
       if constexpr (kSpread && !kFirst) {
         pv_half(st, v_lds + ((R + 3) & 3) * kSlabBytes, p_prev, [&](int i) {
@@ -275,25 +260,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
           copy_k(owed_k_dst, owed_k_src);
           copy_v(owed_v_dst, owed_v_src);
         }
-        if constexpr (!kFirst) {
-          if (w_prev) pv_half(st, v_lds + ((R + 3) & 3) * kSlabBytes, p_prev);
-        }
+        if constexpr (!kFirst) pv_half(st, v_lds + ((R + 3) & 3) * kSlabBytes, p_prev);
       }
-      const bool active = !kTiled || (bits_cmp & group_bit) != 0;
-      if (w_cur) softmax_reference(st, s_cur, active);
-      f32x16 s_nxt;
-      if (w_nxt) s_nxt = qk_half(st, k_lds + ((R + 1) & 3) * kSlabBytes);  // past the last slab: stale data, unused
-      else s_nxt = s_cur;
-      if (w_cur) softmax_exp<kTiled>(st, s_cur, p_prev, active);  // p_prev := P_t
-      w_prev = w_cur;
-      if constexpr (kTiled) {
-        if (--rem_cmp == 0) {
-          rem_cmp = nsub;
-          ++e_cmp;
-          bits_cmp = bits_ahead;
-          bits_ahead = e_cmp + 1 < cnt ? idx[e_cmp + 1] & 255 : 0;
-        }
-      }
+      softmax_reference(st, s_cur, true);
+      f32x16 s_nxt = qk_half(st, k_lds + ((R + 1) & 3) * kSlabBytes);  // past the last slab: stale data, unused
+      softmax_exp<false>(st, s_cur, p_prev, true);  // p_prev := P_t
       // P_t is only consumed after the barrier; without the pins its arithmetic sinks there, away from the MFMAs it is
       // meant to overlap with
       pin(p_prev[0]);
@@ -320,7 +291,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
       step(IC<1>{}, std::false_type{}, t + 3);
     }
     // O += P_{n-1} V_{n-1}
-    if (w_prev) pv_half(st, v_lds + ((nsteps - 1) & 3) * kSlabBytes, p_prev);
+    pv_half(st, v_lds + ((nsteps - 1) & 3) * kSlabBytes, p_prev);
     wait_vmem<0>();  // no copy may still be writing LDS when the work-group gives it back
   }
 
@@ -355,8 +326,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     }
 }
 
-// Forward on tile lists whose tiles are not of one mind: q_block no multiple of 128, so the two 64-row halves of a 128-row
-// tile select key blocks of their own.
+// Forward on tile lists (q_block or k_block no multiple of 128).
 //
 // Work-group = 64 query rows, four waves, two work-groups per CU.  The unit of work is a chunk of 64 keys; wave w owns rows
 // 32 (w % 2) .. +31 against keys 32 (w / 2) .. +31 of every chunk, with the same pipeline as fwd_kernel (P_{t-1} V_{t-1} |
@@ -368,7 +338,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
 // Bound like fwd_kernel by the matrix pipe, the softmax between its instructions and the clock these allow.  A chunk feeds half
 // as many matrix instructions per byte copied as there, but with 128-row work-groups a chunk that one half selects kept the
 // waves of the other waiting: B1 H24 S30720, independent 64 x 64 blocks, 40 % kept, a tile's list holds 64 % of the blocks and
-// the step took 21.98 ms, now 19.30; B2 H8/2 S3136 q16 k64, a quarter kept, 301 -> 289 us.
+// the step took 21.98 ms, now 19.30; B2 H8/2 S3136 q16 k64, a quarter kept, 301 -> 289 us.  Where the halves agree it is ahead as
+// well, of a 128-row kernel that reads its tile list entry by entry: forward, 128-row query blocks and 64-key blocks, H24 S30720
+// 5.18 -> 4.83 ms, H8 S4096 48 -> 37 us.
 //
 // kRows: q_block is no multiple of 64, so the four 16-row groups of a half differ as well: a wave leaves out the matrix work
 // of chunks that neither of its groups selects, rows switched off inside an active wave are dealt with by selects.
@@ -697,10 +669,10 @@ hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
 }  // namespace
 
 hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
-  if (p.tiled && p.q_block % 128 != 0) return launch_fwd_halves(p, stream);
+  if (p.tiled) return launch_fwd_halves(p, stream);
   constexpr int kSmem = 2 * kRing * kSlabBytes;
-  const bool wide = !p.tiled && p.q_block % 384 == 0 && p.variant != 1;
-  void (*fn)(const FwdParams) = p.tiled ? &fwd_kernel<true, 4> : wide ? &fwd_kernel<false, 12> : &fwd_kernel<false, 4>;
+  const bool wide = p.q_block % 384 == 0 && p.variant != 1;
+  void (*fn)(const FwdParams) = wide ? &fwd_kernel<12> : &fwd_kernel<4>;
   const int rows = wide ? 384 : 128;
   p.num_items = p.B * p.Hq * (p.Sq / rows);
   // tail splitting for the 128-row kernels (two work-groups per compute unit)

@@ -1,5 +1,5 @@
-"""Forward on tile lists whose 128-row tiles are not of one mind (q_block no multiple of 128): work-groups of 64 rows that take
-the entries naming their half from a register of 64 at a time.  List lengths around 64 and its multiples, halves that select
+"""Forward on tile lists: work-groups of 64 rows that take the entries naming their half of a 128-row tile from a register of 64
+at a time.  List lengths around 64 and its multiples, halves that select
 nothing, the first or only the last entries, one chunk in all, key blocks of one and of several chunks, 16-row groups, grouped
 heads, shared and separate masks, split launches.  Against the oracle's explicit dense formula (fp32) with the operator's parity
 bar for N(0,1) inputs; O, LSE bit-equal on a repeat, and rows without keys exactly 0 and -inf."""
@@ -38,6 +38,8 @@ def _mask(kind, shape, g):
     (1, 3, 3, 768, 1152, 48, 192, 4, "random"),   # row groups that straddle halves, three chunks to a block
     (1, 2, 2, 1152, 1152, 192, 384, 2, "random"),
     (1, 1, 1, 640, 640, 320, 64, 4, "one"),
+    (1, 3, 1, 384, 1152, 128, 64, 4, "random"),   # halves that agree
+    (1, 2, 2, 768, 1152, 384, 192, 2, "ends"),
     (2, 24, 24, 1536, 1536, 64, 64, 4, "random"),  # more items than slots
     (1, 30, 30, 1152, 768, 16, 64, 4, "random"),   # the last round of 28 items is split
 ])
