@@ -530,6 +530,29 @@ int32_t fba_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, 
   return e == hipSuccess ? FBA_OK : hip_fail(e, "list launch");
 }
 
+int32_t fba_resize_rows(int32_t n, const void* const* src, void* const* dst, const int64_t* n_seq, const int32_t* src_len, const int32_t* dst_len,
+                        void* hip_stream) {
+  if (n < 1 || n > 3) return fail(FBA_ERR_INVALID, "resize_rows takes one to three tensors (got %d)", n);
+  if (!src || !dst || !n_seq || !src_len || !dst_len) return fail(FBA_ERR_INVALID, "null pointer argument");
+  for (int j = 0; j < n; ++j) {
+    if (int rc = check_ptrs({{"src", src[j]}, {"dst", dst[j]}})) return rc;
+    if (n_seq[j] <= 0 || src_len[j] <= 0 || dst_len[j] <= 0)
+      return fail(FBA_ERR_INVALID, "sequences and lengths must be positive (got %lld %d %d)", (long long)n_seq[j], src_len[j], dst_len[j]);
+    if (n_seq[j] >= (1LL << 31)) return fail(FBA_ERR_INVALID, "too many sequences (%lld)", (long long)n_seq[j]);
+  }
+  hipError_t e = fba::launch_resize_rows(n, src, dst, n_seq, src_len, dst_len, (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "resize_rows launch");
+}
+
+int32_t fba_resize_mask(const uint8_t* src, uint8_t* dst, int64_t mask_bh, int32_t src_q, int32_t src_k, int32_t dst_q, int32_t dst_k, void* hip_stream) {
+  if (mask_bh <= 0 || src_q <= 0 || src_k <= 0 || dst_q <= 0 || dst_k <= 0)
+    return fail(FBA_ERR_INVALID, "mask_bh and the numbers of blocks must be positive (got %lld %d %d %d %d)", (long long)mask_bh, src_q, src_k, dst_q, dst_k);
+  if (mask_bh >= (1LL << 31)) return fail(FBA_ERR_INVALID, "too many masks (%lld)", (long long)mask_bh);
+  if (!src || !dst) return fail(FBA_ERR_INVALID, "null pointer argument");
+  hipError_t e = fba::launch_resize_mask(src, dst, mask_bh, src_q, src_k, dst_q, dst_k, (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "resize_mask launch");
+}
+
 // For problems that take less time than it costs to number their pairs and to wait for the count: B1 H2 S1536, 384-token
 // blocks, forward + backward 304 -> 224 us against numbered pairs (four launches, a pinned copy and a wait less); B2 H8/2
 // S3136 q16 k64 430 -> 332 us.  The price is a workspace of all pairs instead of the selected ones, so the caller draws the

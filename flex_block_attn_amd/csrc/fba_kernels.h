@@ -131,6 +131,9 @@ hipError_t launch_ssta_mask(const float* q_mean, const float* k_mean, const uint
                             int nK, int q_block, int k_block, int topk, int band, int sink, hipStream_t stream);
 hipError_t launch_tile_permute(const void* x, void* out, int64_t n_seq, int T, int H, int W, int tT, int tH, int tW,
                                int to_tiles, hipStream_t stream);
+hipError_t launch_resize_rows(int n, const void* const* src, void* const* dst, const int64_t* n_seq, const int32_t* src_len, const int32_t* dst_len,
+                              hipStream_t stream);
+hipError_t launch_resize_mask(const uint8_t* src, uint8_t* dst, int64_t M, int src_q, int src_k, int dst_q, int dst_k, hipStream_t stream);
 hipError_t launch_fwd(FwdParams p, hipStream_t stream);
 hipError_t launch_bwd_stats(const __bf16* o, const __bf16* d_o, const float* lse, float* stats, int64_t rows, hipStream_t stream);
 hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream);

@@ -9,6 +9,8 @@
 // The library is not linked but bound by path (bind), so that FBA_LIBRARY can name another build of it.
 #include <dlfcn.h>
 
+#include <numeric>
+
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/Event.h>
@@ -31,7 +33,7 @@ constexpr int64_t kXcds = 8;
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                      \
   X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots) X(fba_tile_slots) X(fba_fwd) X(fba_fwd_tiled) \
-      X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense)
+      X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
 #define DECLARE(f) decltype(&::f) f = nullptr;
@@ -89,8 +91,8 @@ struct Lists {
 
 // Largest dS workspace backward allocates on its own: at most `limit` bytes, and at most `factor` times the bytes of the
 // call's own tensors (q, o, dO, dq and k, v, dk, dv in bf16).
-int64_t ds_limit(const at::Tensor& q, const at::Tensor& k, double limit, double factor) {
-  const double own = 2.0 * (5.0 * q.numel() + 4.0 * k.numel());
+int64_t ds_limit(const Problem& p, double limit, double factor) {
+  const double own = 2.0 * kHeadDim * (5.0 * p.B * p.Hq * p.Sq + 4.0 * p.B * p.Hkv * p.Skv);
   return (int64_t)std::min(limit, factor * own);
 }
 
@@ -247,6 +249,8 @@ struct Saved : torch::CustomClassHolder {
   c10::Event copied{c10::DeviceType::CUDA};
   bool dense;
   int64_t limit, split_bytes;
+  int64_t q_len, kv_len;  // of the caller's tensors; p describes the padded ones
+  bool padded() const { return q_len != p.Sq || kv_len != p.Skv; }
   explicit Saved(const Problem& problem) : p(problem), lists(problem) {}
 };
 
@@ -297,12 +301,50 @@ void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered)
   s.copied.record(c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(mask.device()));
 }
 
+// Sequences that are no whole number of 128-row tiles: copies cut or padded with zeros to `len` rows, all in one launch.  A
+// tensor that has the length already is returned as it is.
+std::vector<at::Tensor> resized(const std::vector<std::pair<at::Tensor, int64_t>>& tensors) {
+  std::vector<at::Tensor> out;
+  const void* src[3];
+  void* dst[3];
+  int64_t n_seq[3];
+  int32_t src_len[3], dst_len[3], n = 0;
+  for (const auto& [t, len] : tensors) {
+    out.push_back(t.size(2) == len ? t : at::empty({t.size(0), t.size(1), len, kHeadDim}, t.options()));
+    if (t.size(2) == len) continue;
+    src[n] = t.data_ptr();
+    dst[n] = out.back().data_ptr();
+    n_seq[n] = t.size(0) * t.size(1);
+    src_len[n] = t.size(2);
+    dst_len[n++] = len;
+  }
+  if (n > 0) check(lib.fba_resize_rows(n, src, dst, n_seq, src_len, dst_len, current_stream(tensors[0].first)));
+  return out;
+}
+
+// Inputs of a call as the kernels take them.  No block selects the rows that are appended.
+struct Inputs {
+  at::Tensor q, k, v, mask;
+  Inputs(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_, const at::Tensor& mask_, const Saved& s) : q(q_), k(k_), v(v_), mask(mask_) {
+    if (!s.padded()) return;
+    const Problem& p = s.p;
+    auto r = resized({{q, p.Sq}, {k, p.Skv}, {v, p.Skv}});
+    q = r[0];
+    k = r[1];
+    v = r[2];
+    mask = at::empty({p.mask_bh, p.nQ(), p.nK()}, mask_.options());
+    check(lib.fba_resize_mask(static_cast<const uint8_t*>(mask_.data_ptr()), static_cast<uint8_t*>(mask.data_ptr()), p.mask_bh, s.q_len / p.q_block,
+                              s.kv_len / p.k_block, p.nQ(), p.nK(), current_stream(q)));
+  }
+};
+
 struct Attention : torch::autograd::Function<Attention> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask,
                             c10::intrusive_ptr<Saved> s) {
-    build_lists(*s, mask, /*backward=*/true, /*numbered=*/!s->dense);
-    auto [o, lse] = run_forward(s->p, q, k, v, s->lists, s->split_bytes);
-    ctx->save_for_backward({q, k, v, o, lse});
+    const Inputs in(q, k, v, mask, *s);
+    build_lists(*s, in.mask, /*backward=*/true, /*numbered=*/!s->dense);
+    auto [o, lse] = run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
+    ctx->save_for_backward({in.q, in.k, in.v, o, lse});
     ctx->saved_data["s"] = c10::IValue::make_capsule(std::move(s));
     return o;
   }
@@ -319,12 +361,13 @@ struct Attention : torch::autograd::Function<Attention> {
       bounds.assign(h, h + s.p.mask_bh + 1);
     }
     auto g = run_backward(s.p, t[0], t[1], t[2], t[3], t[4], d_o, s.lists, bounds, HandOver::kAuto, s.dense, s.limit, s.split_bytes);
+    if (s.padded()) g = resized({{g[0], s.q_len}, {g[1], s.kv_len}, {g[2], s.kv_len}});
     return {g[0], g[1], g[2], at::Tensor(), at::Tensor()};
   }
 };
 
-// flex_block_attn_func for arguments that need no preparation; nothing for all others (wrong types or shapes, lengths that
-// have to be padded), which Python then reports or prepares.
+// flex_block_attn_func for arguments that need no preparation but padding to whole tiles; nothing for all others (wrong types or
+// shapes, strided tensors), which Python then reports or prepares.
 c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t q_block, int64_t k_block, const at::Tensor& mask,
                                     double limit, double factor, int64_t split_bytes) {
   // a traced call has to appear in the trace, and forward-mode differentiation has to be refused: both go through the Python
@@ -343,7 +386,12 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   if (q_block <= 0 || k_block <= 0 || q_block % 16 != 0 || k_block % 64 != 0 || (k_block % q_block != 0 && q_block % k_block != 0)) return c10::nullopt;
   if (p.Sq % q_block != 0 || p.Skv % k_block != 0 || mask.size(md - 2) != p.nQ() || mask.size(md - 1) != p.nK()) return c10::nullopt;
   if (md == 4 && (mask.size(0) != p.B || mask.size(1) != p.Hq)) return c10::nullopt;
-  if (p.tiled() && (p.Sq % 128 != 0 || p.Skv % 128 != 0)) return c10::nullopt;
+  const int64_t q_len = p.Sq, kv_len = p.Skv;
+  if (p.tiled()) {  // whole blocks are appended until the tiles are whole as well
+    auto whole = [](int64_t len, int64_t block) { return len % 128 == 0 ? len : (len + std::lcm(block, 128L) - 1) / std::lcm(block, 128L) * std::lcm(block, 128L); };
+    p.Sq = whole(q_len, q_block);
+    p.Skv = whole(kv_len, k_block);
+  }
   if (p.B * p.Hq * p.Sq >= (1LL << 30) || p.B * p.Hkv * p.Skv >= (1LL << 30) || p.mask_bh * p.nQ() * p.nK() > 0x7fffffffLL ||
       p.mask_bh * (p.Sq / 32 + 1) * (p.Skv / 128 + 1) > 0x7fffffffLL)
     return c10::nullopt;
@@ -351,14 +399,20 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   if (split_bytes < 0) split_bytes = lib.fba_split_workspace_bytes();
   auto s = c10::make_intrusive<Saved>(p);
   s->split_bytes = split_bytes;
+  s->q_len = q_len;
+  s->kv_len = kv_len;
   const bool backward = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
   if (!backward) {
-    build_lists(*s, mask, false, false);
-    return run_forward(p, q, k, v, s->lists, split_bytes).first;
+    const Inputs in(q, k, v, mask, *s);
+    build_lists(*s, in.mask, false, false);
+    const at::Tensor o = run_forward(p, in.q, in.k, in.v, s->lists, split_bytes).first;
+    return s->padded() ? o.narrow(2, 0, q_len) : o;
   }
-  s->limit = ds_limit(q, k, limit, factor);
+  s->limit = ds_limit(p, limit, factor);
   s->dense = p.dense_bytes() <= s->limit;
-  return Attention::apply(q, k, v, mask, std::move(s));
+  const bool cut = q_len != p.Sq;
+  const at::Tensor o = Attention::apply(q, k, v, mask, std::move(s));
+  return cut ? o.narrow(2, 0, q_len) : o;
 }
 
 // ---------------------------------------------------------------------------------------------------------------------

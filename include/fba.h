@@ -65,7 +65,7 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  *                   the call's work on the stream; its contents before and after are meaningless
  *   split_ws_bytes  its size; fba_split_workspace_bytes() is what the planner can use at most (a smaller buffer limits
  *                   the number of ranges, never correctness)
- * On tile lists forward and the dK/dV kernel split; the dQ kernels do not.
+ * On tile lists forward (64-row tiles) and the dK/dV kernel split; the dQ kernels do not.
  * The same workspace lends its last 256 bytes (when they lie behind the partial results) to the dK/dV kernels of launches of
  * four rounds and more: eight counters, zeroed by a one-wave launch in front, from which the work-groups claim the tile they
  * work on, with an eighth more work-groups launched than there are tiles.  The hardware deals work-groups to the eight
@@ -158,6 +158,17 @@ int32_t fba_bwd_dq_from_ds(const void* k, const void* ds_ws, int64_t ds_ws_bytes
  */
 int32_t fba_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block, int32_t* q_cnt,
                   int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream);
+
+/*
+ * Sequences that are no whole number of 128-row tiles (possible with tile lists only) are worked on in padded copies.
+ * fba_resize_rows: dst[s, r, :] = src[s, r, :] for r < min(src_len, dst_len), zeros for the rows dst has more, for n (1 to 3)
+ * tensors of n_seq[j] sequences of 256-byte rows, 16-byte aligned; the arrays are read before the call returns.
+ * fba_resize_mask: the same for a block mask [mask_bh, src_q, src_k] -> [mask_bh, dst_q, dst_k].
+ */
+int32_t fba_resize_rows(int32_t n, const void* const* src, void* const* dst, const int64_t* n_seq, const int32_t* src_len,
+                        const int32_t* dst_len, void* hip_stream);
+int32_t fba_resize_mask(const uint8_t* src, uint8_t* dst, int64_t mask_bh, int32_t src_q, int32_t src_k, int32_t dst_q, int32_t dst_k,
+                        void* hip_stream);
 
 /*
  * Backward with dS handed over in a workspace that has a place for every (query block, key block) pair, selected or not:
