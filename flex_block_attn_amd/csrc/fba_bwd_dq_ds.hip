@@ -6,12 +6,13 @@
 // once, and this query-major kernel reads it back: two products per pair instead of the six of dq_kernel, which
 // recomputes S and dP.  Every dQ element is still written exactly once, by the work-group that owns its row.
 //
-// Work-group = 128 query rows, wave = 32 rows, lane = query row:
+// Work-group = kWaves waves of 32 query rows, lane = query row (128 rows, two work-groups per CU; 256 or 384 rows, one per CU):
 //   dQ^T += K^T dS^T                   A = K slab through transposing LDS fetches, B = dS^T through transposing LDS
 //                                      fetches of the wave's own dS unit (layout: fba_common.h)
-// The kernel does 8 MFMAs per 16 KiB it reads, so it runs at the speed of memory: K slabs (8 KiB, shared by the four
-// waves, mostly L2 hits) and dS units (2 KiB per wave, each read exactly once from HBM) travel global -> LDS directly
-// into a ring of four stages; stage t+4 is requested when stage t is dead.
+// A wave does 8 MFMAs per 2 KiB of dS and its share of a K slab, so the kernel runs at the speed of memory: K slabs (8 KiB, shared
+// by the waves, mostly L2 hits) and dS units (2 KiB per wave, each read exactly once from HBM) travel global -> LDS directly
+// into a ring of four stages; stage t+4 is requested when stage t is dead.  More rows per work-group share a K slab among more
+// waves: half (256 rows) or a third (384) of the K bytes, and with 384 rows half as much dS again in flight per CU.
 //
 // kTiled: tile lists.  The workspace is divided into (128-row query tile, 128-key tile) pairs of 16 units; the list of the
 // work-group's query tile names key blocks with a predicate per 16 rows.  A wave whose rows do not select a key block has
@@ -29,7 +30,7 @@ namespace {
 
 constexpr int kSlab = 32;
 constexpr int kSlabBytes = kSlab * kRowBytes;        // 8 KiB: one K slab, or the four dS units of a step
-constexpr int kStageBytes = 2 * kSlabBytes;          // K slab | dS units
+constexpr int stage_bytes(int waves) { return kSlabBytes + waves * kDsUnitBytes; }  // K slab | dS units
 constexpr int kRing = 4;
 
 template <int N>
@@ -37,10 +38,13 @@ using IC = std::integral_constant<int, N>;
 
 }  // namespace
 
-template <bool kTiled, int kMode>  // kMode: kNumbered or kDense
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void dq_from_ds_kernel(const BwdParams p) {
+template <bool kTiled, int kMode, int kWaves>  // kMode: kNumbered or kDense
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(kWaves == 12 ? 3 : 2, kWaves == 12 ? 3 : 2))) void dq_from_ds_kernel(
+    const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // ring [4] of (K slab | dS units)
-  constexpr int TQ = 128;
+  constexpr int TQ = 32 * kWaves;
+  constexpr int kStageBytes = stage_bytes(kWaves);
+  static_assert(!kTiled || kWaves == 4, "tile lists describe 128-row tiles");
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -65,7 +69,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const char* kp = reinterpret_cast<const char*>(p.k + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
 
   const int qblk = (qt * TQ) / p.q_block;
-  const int tq = kTiled ? 0 : (qt * TQ - qblk * p.q_block) / TQ;  // this tile's position inside its query block
+  // the 128-row tile of the query block that this wave's rows lie in
+  const int tq = kTiled ? 0 : (qt * TQ - qblk * p.q_block) / 128 + (wave >> 2);
   const int n_kt = p.Skv / 128;
   const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (kTiled ? tiles_per_head : p.nQ) + (kTiled ? qt : qblk);
   constexpr bool dense = kMode == kDense;
@@ -89,14 +94,28 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   // dS of this wave's 32 rows: pair base + (tq * nsub + t) * 4 units + wave, t = 32-key slab inside the key block (inside
   // the key tile with tile lists)
   const int64_t head_pairs = p.mask_bh == 1 && !dense ? (int64_t)bh * const_idx(p.pair_base)[kTiled ? n_kt : p.nK] : 0;
-  const char* ds_base = reinterpret_cast<const char*>(p.ds_ws) + head_pairs * pair_bytes + ((int64_t)tq * nsub * 4 + wave) * kDsUnitBytes;
+  const char* ds_base = reinterpret_cast<const char*>(p.ds_ws) + head_pairs * pair_bytes + ((int64_t)tq * nsub * 4 + (wave & 3)) * kDsUnitBytes;
   auto key_block = [&](int e) -> int { return kTiled ? idx[e] >> 8 : idx[e]; };
   const int wave_bits = 3 << (2 * wave);  // predicate bits of this wave's two 16-row groups in a tile-list entry
 
   TransposedOffsets tr;
   tr.init(lane);
-  SlabDma dma;
-  dma.init(wave, lane);
+  // K slab: two copies of four rows by each of four waves, or one by each of the first eight
+  const bool copies_k = kWaves <= 8 || wave < 8;
+  uint32_t k_off_lane[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int row = 4 * (kWaves == 4 ? 2 * wave + g : wave & 7) + (lane >> 4);
+    k_off_lane[g] = (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4));
+  }
+  const uint32_t k_dst_wave = (uint32_t)((kWaves == 4 ? 2 * wave : wave & 7) * 4 * kRowBytes);
+  // until the copies of all but the `n` youngest stages have landed
+  auto wait_stages = [&](auto n_c) {
+    constexpr int n = decltype(n_c)::value;
+    if constexpr (kWaves == 4) wait_vmem<4 * n>();
+    else if (copies_k) wait_vmem<3 * n>();
+    else wait_vmem<2 * n>();
+  };
   const uint32_t ring_dst = lds_addr(smem);
   // Transposing fetches of the B operand from the wave's unit.  Group G = lane / 16 of the wave serves query rows
   // 16 (G % 2) .. +15 and the key half 4 (G / 2) .. +3 of each 8 keys; source lane s = lane % 16 addresses the slot of
@@ -131,7 +150,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const uint32_t lane16 = (uint32_t)lane * 16;
   auto copy_next = [&](int ring) {
     const uint32_t dst = ring_dst + ring * kStageBytes;
-    dma.copy(dst, kp + k_off);
+    if constexpr (kWaves == 4) {
+      dma16(dst + k_dst_wave, kp + k_off, k_off_lane[0]);
+      dma16(dst + k_dst_wave + 4 * kRowBytes, kp + k_off, k_off_lane[1]);
+    } else {
+      if (copies_k) dma16(dst + k_dst_wave, kp + k_off, k_off_lane[0]);
+    }
     const char* src = ds_base + ds_off_g;
     if constexpr (kTiled) {
       const int t = (int)(k_off >> 13) & 3;  // 32-key slab inside its key tile
@@ -191,8 +215,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
           bits_ahead = e_cmp + 1 < cnt ? idx[e_cmp + 1] & 255 : 0;
         }
       }
-      // stage t+1 must have landed (first read in step t+1); the copies of stages t+2 and t+3 (4 each) may still fly
-      if (t + 3 < nsteps) wait_vmem<8>(); else if (t + 2 < nsteps) wait_vmem<4>(); else wait_vmem<0>();
+      // stage t+1 must have landed (first read in step t+1); the copies of stages t+2 and t+3 may still fly
+      if (t + 3 < nsteps) wait_stages(IC<2>{}); else if (t + 2 < nsteps) wait_stages(IC<1>{}); else wait_stages(IC<0>{});
       __syncthreads();
       if (t + 4 < nsteps) copy_next(R);
     };
@@ -280,28 +304,47 @@ hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, i
   return hipGetLastError();
 }
 
-hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
-  constexpr int kSmem = kRing * kStageBytes;
-  if (p.ds_ws == nullptr) return hipErrorInvalidValue;
-  p.num_items = p.B * p.Hq * (p.Sq / 128);
-  // tail splitting on block lists (two work-groups per compute unit); a part stores a 128 x 128 fp32 tile
-  p.split = plan_split(p.num_items, 2, p.Skv / 32, 4, 128 * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes);
+namespace {
+
+template <int kWaves>
+hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
+  constexpr int kRows = 32 * kWaves, kSmem = kRing * stage_bytes(kWaves);
+  p.num_items = p.B * p.Hq * (p.Sq / kRows);
+  // tail splitting on block lists (two work-groups of four waves per compute unit, one of more); a part stores a tile of fp32 sums
+  p.split = plan_split(p.num_items, kWaves == 4 ? 2 : 1, p.Skv / 32, 4, kRows * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
-  void (*fn)(const BwdParams) = p.pair_base == nullptr
-      ? (p.tiled ? &dq_from_ds_kernel<true, kDense> : &dq_from_ds_kernel<false, kDense>)
-      : (p.tiled ? &dq_from_ds_kernel<true, kNumbered> : &dq_from_ds_kernel<false, kNumbered>);
+  const bool dense = p.pair_base == nullptr;
+  void (*fn)(const BwdParams) = dense ? &dq_from_ds_kernel<false, kDense, kWaves> : &dq_from_ds_kernel<false, kNumbered, kWaves>;
   hipError_t e = hipSuccess;
-  if (p.tiled && (e = zero_unit_address(&p.zero_unit)) != hipSuccess) return e;
+  if constexpr (kWaves == 4) {
+    if (p.tiled) {
+      fn = dense ? &dq_from_ds_kernel<true, kDense, kWaves> : &dq_from_ds_kernel<true, kNumbered, kWaves>;
+      if ((e = zero_unit_address(&p.zero_unit)) != hipSuccess) return e;
+    }
+  }
   e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kSmem, stream, p);
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(64 * kWaves), kSmem, stream, p);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0};
-    e = launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, p.split.first, split_items, nullptr, stream);
+    e = launch_partial_sum(p.split.ws, p.split.parts, kRows * kHeadDim, kRows, &out, 1, p.split.first, split_items, nullptr, stream);
     if (e != hipSuccess) return e;
   }
   return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
+  if (p.ds_ws == nullptr) return hipErrorInvalidValue;
+  // Wide work-groups where the query blocks allow them and the launch has two rounds of them: smaller launches fill the chip
+  // better with 128 rows.  Backward, 128 rows everywhere / wide, 40 % kept: H24 S30720, 384-token blocks 12.49 -> 12.31 ms (dQ
+  // 3.36 -> 3.18 ms), 256-token blocks 12.49 -> 12.25 ms; H24 S115200 sliding window, step 51.5 -> 50.9 ms.
+  const int64_t rows = (int64_t)p.B * p.Hq * p.Sq, enough = 2LL * device_compute_units();  // work-groups
+  if (!p.tiled && p.q_block % 384 == 0 && rows / 384 >= enough) return launch_dq_rows<12>(p, stream);
+  if (!p.tiled && p.q_block % 256 == 0 && rows / 256 >= enough) return launch_dq_rows<8>(p, stream);
+  return launch_dq_rows<4>(p, stream);
 }
 
 }  // namespace fba
