@@ -134,7 +134,7 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
   // tiles in index order share more of their lists in L2 (structured masks): measured, steps with items in index order /
   // ordered, B2 H16/4 S8192 (2 rounds) 1113 / 1062 us, B1 H24 S30720 random (7.5 rounds per chunk) 16.53 / 16.04 ms, H24
   // S69120 top-k (17 rounds) 25.3 / 25.2 ms, H24 S115200 sliding window (28 rounds) 52.1 / 52.9 ms.  With shorter lists the
-  // spread is worth less than the launch (3 us).
+  // spread is worth less than the launch (21 us for 640 items, rocprofv3).
   const bool ordered = !p.tiled && queue != nullptr && top >= bottom && p.num_items > slots && p.num_items <= 8 * slots && p.Hq / p.Hkv * (p.Sq / 32) >= 128;
   if (ordered) p.split.main_wgs = p.split.first;
 
