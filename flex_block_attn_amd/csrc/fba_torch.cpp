@@ -338,6 +338,16 @@ struct Inputs {
   }
 };
 
+// What autograd hands back in backward is whatever a saved-tensor hook made of it (another type, shape or layout), and the
+// kernels read it by raw pointer: the same contract as for the inputs of a call.  `o` and `lse` may be strided, q, k, v not.
+at::Tensor unpacked(const Saved& s, const char* name, const at::Tensor& t, at::IntArrayRef shape, at::ScalarType type, bool strided) {
+  TORCH_CHECK_VALUE(t.defined() && t.device() == s.list_buffer.device(), "saved ", name, " must come back as a tensor on ", s.list_buffer.device());
+  TORCH_CHECK_TYPE(t.scalar_type() == type, "saved ", name, " must come back as ", type, ", got ", t.scalar_type());
+  TORCH_CHECK_VALUE(t.sizes() == shape, "saved ", name, " must come back with shape ", shape, ", got ", t.sizes());
+  TORCH_CHECK_VALUE(strided || t.is_contiguous(), "saved ", name, " must come back contiguous");
+  return t.contiguous();
+}
+
 struct Attention : torch::autograd::Function<Attention> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask,
                             c10::intrusive_ptr<Saved> s) {
@@ -349,18 +359,23 @@ struct Attention : torch::autograd::Function<Attention> {
     return o;
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
-    const auto t = ctx->get_saved_variables();
+    const auto saved = ctx->get_saved_variables();
     const auto capsule = ctx->saved_data["s"].toCapsule();
     Saved& s = *static_cast<Saved*>(capsule.get());
-    const c10::DeviceGuard guard(t[0].device());
+    const c10::DeviceGuard guard(s.list_buffer.device());
+    const Problem& p = s.p;
+    const int64_t q_shape[4] = {p.B, p.Hq, p.Sq, kHeadDim}, kv_shape[4] = {p.B, p.Hkv, p.Skv, kHeadDim}, lse_shape[4] = {p.B, p.Hq, p.Sq, 1};
+    const at::Tensor q = unpacked(s, "q", saved[0], q_shape, at::kBFloat16, false), k = unpacked(s, "k", saved[1], kv_shape, at::kBFloat16, false),
+                     v = unpacked(s, "v", saved[2], kv_shape, at::kBFloat16, false), o = unpacked(s, "o", saved[3], q_shape, at::kBFloat16, true),
+                     lse = unpacked(s, "lse", saved[4], lse_shape, at::kFloat, true);
     const at::Tensor d_o = grads[0].to(at::kBFloat16).contiguous();
     std::vector<int64_t> bounds;
     if (!s.dense) {
       s.copied.synchronize();
       const int32_t* h = s.host_bounds.data_ptr<int32_t>();
-      bounds.assign(h, h + s.p.mask_bh + 1);
+      bounds.assign(h, h + p.mask_bh + 1);
     }
-    auto g = run_backward(s.p, t[0], t[1], t[2], t[3], t[4], d_o, s.lists, bounds, HandOver::kAuto, s.dense, s.limit, s.split_bytes);
+    auto g = run_backward(p, q, k, v, o, lse, d_o, s.lists, bounds, HandOver::kAuto, s.dense, s.limit, s.split_bytes);
     if (s.padded()) g = resized({{g[0], s.q_len}, {g[1], s.kv_len}, {g[2], s.kv_len}});
     return {g[0], g[1], g[2], at::Tensor(), at::Tensor()};
   }

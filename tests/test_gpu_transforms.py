@@ -56,3 +56,53 @@ def test_saved_tensor_hooks_see_the_inputs(gpu):
     assert len(packed) == 5  # q, k, v, o, lse
     want = torch.autograd.grad(fba.flex_block_attn_func(q, k, v, 128, 128, mask), (q, k, v), torch.ones_like(o))
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+# what a saved-tensor hook may not turn a tensor into, by its place among (q, k, v, o, lse): the kernels read by raw pointer
+BAD = {
+    "fewer rows": (0, lambda t: t[:, :, :128].contiguous(), ValueError),
+    "no batch": (1, lambda t: t[0], ValueError),
+    "another type": (2, lambda t: t.float(), TypeError),
+    "another type of o": (3, lambda t: t.half(), TypeError),
+    "left on the host": (1, lambda t: t.cpu(), ValueError),
+    "strided": (0, lambda t: t.transpose(2, 3).contiguous().transpose(2, 3), ValueError),
+    "lse in half precision": (4, lambda t: t.half(), TypeError),
+    "lse cut short": (4, lambda t: t[:, :, :-1], ValueError),
+}
+
+
+@pytest.mark.parametrize("what", BAD)
+def test_unpacked_tensors_are_checked(gpu, what):
+    import flex_block_attn_amd as fba
+
+    place, change, error = BAD[what]
+    q, k, v = (t.requires_grad_(True) for t in _inputs(gpu, 5))
+    mask = torch.ones((2, 2), dtype=torch.bool, device=gpu)
+    order = []
+
+    def unpack(packed):
+        number, t = packed
+        return change(t) if number == place else t
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: order.append(0) or (len(order) - 1, t), unpack):
+        o = fba.flex_block_attn_func(q, k, v, 128, 128, mask)
+    with pytest.raises(error, match="saved"):
+        torch.autograd.grad(o, (q, k, v), torch.ones_like(o))
+
+
+def test_unpacked_output_may_be_strided(gpu):
+    import flex_block_attn_amd as fba
+
+    q, k, v = (t.requires_grad_(True) for t in _inputs(gpu, 6))
+    mask = torch.ones((2, 2), dtype=torch.bool, device=gpu)
+    order = []
+
+    def unpack(packed):
+        number, t = packed
+        return t.transpose(2, 3).contiguous().transpose(2, 3) if number >= 3 else t
+
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: order.append(0) or (len(order) - 1, t), unpack):
+        o = fba.flex_block_attn_func(q, k, v, 128, 128, mask)
+    got = torch.autograd.grad(o, (q, k, v), torch.ones_like(o))
+    want = torch.autograd.grad(fba.flex_block_attn_func(q, k, v, 128, 128, mask), (q, k, v), torch.ones_like(o))
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
