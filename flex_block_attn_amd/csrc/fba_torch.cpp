@@ -16,6 +16,7 @@
 #include <c10/core/Event.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/custom_class.h>
@@ -51,13 +52,20 @@ void bind(const std::string& path) {
 #undef RESOLVE
 }
 
-// Failure of a C ABI call; becomes _lib.FbaError where it reaches Python (see the translator below).
-struct CallError : std::runtime_error {
-  int code;
-  explicit CallError(int c) : std::runtime_error(std::string("libfba_gfx950 error ") + std::to_string(c) + ": " + lib.fba_last_error()), code(c) {}
-};
+// A failed C ABI call raises _lib.FbaError.  It is set as a Python error here, and not translated where a call returns to
+// Python, because a failure in backward travels through the autograd engine, which hands on Python errors as they are and
+// makes a plain RuntimeError of any other exception.
+[[noreturn]] void raise_call_error(int code) {
+  const std::string message = lib.fba_last_error();  // of this thread
+  pybind11::gil_scoped_acquire gil;
+  const pybind11::object type = pybind11::module_::import("flex_block_attn_amd._lib").attr("FbaError");
+  PyErr_SetObject(type.ptr(), type(code, message).ptr());
+  python_error error;
+  error.persist();
+  throw error;
+}
 void check(int code) {
-  if (code != FBA_OK) throw CallError(code);
+  if (code != FBA_OK) raise_call_error(code);
 }
 
 void* current_stream(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -472,18 +480,9 @@ std::vector<at::Tensor> backward_on_lists(const at::Tensor& q, const at::Tensor&
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  namespace py = pybind11;
-  py::register_exception_translator([](std::exception_ptr e) {
-    try {
-      if (e) std::rethrow_exception(e);
-    } catch (const CallError& err) {
-      py::object cls = py::module_::import("flex_block_attn_amd._lib").attr("FbaError");
-      PyErr_SetObject(cls.ptr(), cls(err.code, lib.fba_last_error()).ptr());
-    }
-  });
   m.def("bind", &bind);
   m.def("plan_head_chunks", &plan_head_chunks);
-  m.def("attention", &attention, py::call_guard<py::gil_scoped_release>());
-  m.def("forward", &forward_on_lists, py::call_guard<py::gil_scoped_release>());
-  m.def("backward", &backward_on_lists, py::call_guard<py::gil_scoped_release>());
+  m.def("attention", &attention, pybind11::call_guard<pybind11::gil_scoped_release>());
+  m.def("forward", &forward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
+  m.def("backward", &backward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
 }
