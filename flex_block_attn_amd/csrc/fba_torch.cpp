@@ -32,9 +32,10 @@ constexpr int64_t kXcds = 8;
 // ---------------------------------------------------------------------------------------------------------------------
 // the C ABI, bound at run time
 // ---------------------------------------------------------------------------------------------------------------------
-#define FBA_FUNCTIONS(X)                                                                                                      \
-  X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots) X(fba_tile_slots) X(fba_fwd) X(fba_fwd_tiled) \
-      X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) X(fba_resize_rows) X(fba_resize_mask)
+#define FBA_FUNCTIONS(X)                                                                                                \
+  X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots) X(fba_tile_slots)        \
+  X(fba_fwd) X(fba_fwd_tiled) X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) \
+  X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
 #define DECLARE(f) decltype(&::f) f = nullptr;
@@ -42,14 +43,21 @@ struct Library {
 #undef DECLARE
 } lib;
 
+// Everything is resolved before anything is replaced: a library that is refused leaves the one in use bound.
 void bind(const std::string& path) {
   void* handle = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
   TORCH_CHECK(handle != nullptr, "cannot load ", path, ": ", dlerror());
+  Library found;
 #define RESOLVE(f)                                                    \
-  lib.f = reinterpret_cast<decltype(&::f)>(dlsym(handle, #f));        \
-  TORCH_CHECK(lib.f != nullptr, path, " does not export ", #f);
+  found.f = reinterpret_cast<decltype(&::f)>(dlsym(handle, #f));      \
+  TORCH_CHECK(found.f != nullptr, path, " does not export ", #f);
   FBA_FUNCTIONS(RESOLVE)
 #undef RESOLVE
+  // the argument lists of this module are those of the header it was compiled with
+  if (found.fba_version() != FBA_VERSION)
+    throw pybind11::import_error(path + " reports version " + std::to_string(found.fba_version()) + ", the host module was built for version " +
+                                 std::to_string(FBA_VERSION) + ": rebuild both with `python -m flex_block_attn_amd.build`");
+  lib = found;
 }
 
 // A failed C ABI call raises _lib.FbaError.  It is set as a Python error here, and not translated where a call returns to

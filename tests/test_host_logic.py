@@ -344,3 +344,17 @@ def test_build_check_finds_a_write_in_front_of_an_asm_matrix_instruction():
     assert find_asm_mfma_hazards(far) == []
     assert len(find_asm_mfma_hazards("\n".join(["v_mov_b32_e32 v50, 0", ".LBB0_7:", mfma]))) == 1
     assert find_asm_mfma_hazards("\n".join(["v_mov_b32_e32 v50, 0", "v_mfma_f32_32x32x16_bf16 v[0:15], v[54:57], v[50:53], v[0:15]"])) == []
+
+
+def test_host_module_refuses_a_library_of_another_version(lib, tmp_path):
+    """The host module calls the library with the argument lists of the header it was compiled with."""
+    import subprocess
+
+    source = tmp_path / "other.c"
+    names = [n for n in lib.SIGNATURES if n != "fba_version"]
+    source.write_text("int fba_version(void) { return 1; }\n" + "".join(f"int {n}(void) {{ return 0; }}\n" for n in names))
+    other = str(tmp_path / "libother.so")
+    subprocess.run([os.environ.get("CC", "gcc"), "-shared", "-fPIC", str(source), "-o", other], check=True)
+    with pytest.raises(ImportError, match=f"version 1, .* version {lib.ABI_VERSION}"):
+        lib.host().bind(other)
+    lib.host().bind(lib.LIB_PATH)
