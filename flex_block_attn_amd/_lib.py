@@ -8,6 +8,8 @@ import importlib.machinery
 import importlib.util
 import os
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # FBA_LIBRARY points the loader at another build of the same ABI (an instrumented or experimental one)
 LIB_PATH = os.environ.get("FBA_LIBRARY") or os.path.join(_HERE, "csrc", "libfba_gfx950.so")
@@ -114,6 +116,9 @@ def host():
         load()  # checks the library's version
         if not os.path.exists(HOST_MODULE_PATH):
             raise ImportError(f"{HOST_MODULE_PATH} is missing: build it with `python -m flex_block_attn_amd.build`. There is no fallback path.")
+        with open(HOST_MODULE_PATH, "rb") as f:
+            if f"fba_torch built for torch {torch.__version__};".encode() not in f.read():
+                raise ImportError(f"{HOST_MODULE_PATH} was built for another torch than {torch.__version__}: rebuild it with `python -m flex_block_attn_amd.build`.")
         loader = importlib.machinery.ExtensionFileLoader("fba_torch", HOST_MODULE_PATH)
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("fba_torch", loader))
         loader.exec_module(module)

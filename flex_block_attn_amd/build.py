@@ -127,7 +127,7 @@ def build_host_module():
            os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), sysconfig.get_paths()["include"]]
     tmp = HOST_MODULE_PATH + ".tmp"
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM", "-DTORCH_EXTENSION_NAME=fba_torch",
-           "-DTORCH_API_INCLUDE_EXTENSION_H", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *["-I" + i for i in inc],
+           "-DTORCH_API_INCLUDE_EXTENSION_H", f'-DFBA_TORCH_BUILD="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *["-I" + i for i in inc],
            os.path.join(CSRC, "fba_torch.cpp"), "-o", tmp, "-L" + os.path.join(root, "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

@@ -24,6 +24,10 @@
 
 #include "../../include/fba.h"
 
+// Which torch this was compiled against.  The loader looks for this text in the file before it loads it (another torch's ABI may
+// differ without a symbol that does not resolve), so it has to stay in the image.
+extern "C" __attribute__((used, visibility("default"))) const char fba_torch_built_for[] = "fba_torch built for torch " FBA_TORCH_BUILD ";";
+
 namespace {
 
 constexpr int64_t kHeadDim = 128;

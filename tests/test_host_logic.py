@@ -358,3 +358,15 @@ def test_host_module_refuses_a_library_of_another_version(lib, tmp_path):
     with pytest.raises(ImportError, match=f"version 1, .* version {lib.ABI_VERSION}"):
         lib.host().bind(other)
     lib.host().bind(lib.LIB_PATH)
+
+
+def test_host_module_of_another_torch_is_not_loaded(lib, tmp_path, monkeypatch):
+    built_for = f"fba_torch built for torch {torch.__version__};".encode()
+    data = open(lib.HOST_MODULE_PATH, "rb").read()
+    assert built_for in data
+    other = tmp_path / "fba_torch.so"
+    other.write_bytes(data.replace(built_for, built_for.replace(b"for torch ", b"for TORCH ")))
+    monkeypatch.setattr(lib, "HOST_MODULE_PATH", str(other))
+    monkeypatch.setattr(lib, "_host", None)
+    with pytest.raises(ImportError, match="built for another torch"):
+        lib.host()
