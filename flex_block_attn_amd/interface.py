@@ -221,13 +221,13 @@ def _check_lists(lists, q, B, Hq, Sq, Skv, q_block_size, kv_block_size):
                              f"got {tuple(t.shape)} {t.dtype} on {t.device}")
 
 
-# Workspace for tail splitting (see include/fba.h), allocated per call from torch's caching allocator; MiB, 0 switches
+# Workspace for tail splitting (see include/fba.h), allocated per call from torch's caching allocator; MiB, 0 or less switches
 # splitting off, unset: what the library's planner can use at most.
 SPLIT_WORKSPACE_MIB = os.environ.get("FBA_SPLIT_WORKSPACE_MIB")
 
 
 def _split_bytes():
-    return _lib.load().fba_split_workspace_bytes() if SPLIT_WORKSPACE_MIB is None else int(float(SPLIT_WORKSPACE_MIB) * 2 ** 20)
+    return _lib.load().fba_split_workspace_bytes() if SPLIT_WORKSPACE_MIB is None else max(0, int(float(SPLIT_WORKSPACE_MIB) * 2 ** 20))
 
 
 def _split_workspace(device):

@@ -370,3 +370,12 @@ def test_host_module_of_another_torch_is_not_loaded(lib, tmp_path, monkeypatch):
     monkeypatch.setattr(lib, "_host", None)
     with pytest.raises(ImportError, match="built for another torch"):
         lib.host()
+
+
+@pytest.mark.parametrize("mib,expected", [("-1", 0), ("0", 0), ("0.5", 2 ** 19), ("3", 3 * 2 ** 20)])
+def test_split_workspace_setting(monkeypatch, mib, expected):
+    """A negative size means no workspace; the native call takes a negative one for "the default"."""
+    from flex_block_attn_amd import interface
+
+    monkeypatch.setattr(interface, "SPLIT_WORKSPACE_MIB", mib)
+    assert interface._split_bytes() == expected
