@@ -116,6 +116,20 @@ int64_t ds_limit(const Problem& p, double limit, double factor) {
   return (int64_t)std::min(limit, factor * own);
 }
 
+// Is backward to hand dS over in a workspace with a place for every pair?  It takes a constant off a step, two launches, a pinned
+// copy and a wait (17-33 us), and costs memory that grows with all pairs instead of the selected ones.  So the line is drawn
+// where the constant no longer counts.  Steps with pairs numbered / dense, 10 % and 40 % kept, 128-token blocks: H4 S4096 (128
+// MiB) 110 / 84 and 136 / 114 us; H24 S3072 (432 MiB) 165 / 145 and 279 / 261; H24 S4096 (768 MiB) 187 / 170 and 369 / 352;
+// H24 S5120 (1.2 GiB) 252 / 235 and 570 / 550; H24 S6784 (2.1 GiB) 378 / 362 and 927 / 910.
+// Steps recorded into a graph use it as far as the limit allows: the wait for the pair count cannot be captured.
+constexpr int64_t kDenseMost = 1LL << 30;
+bool dense_fits(int64_t bytes, int64_t limit) {
+  if (bytes > limit) return false;
+  if (bytes <= kDenseMost) return true;
+  pybind11::gil_scoped_acquire gil;
+  return pybind11::module_::import("torch").attr("cuda").attr("is_current_stream_capturing")().cast<bool>();
+}
+
 using Chunk = std::tuple<int64_t, int64_t, int64_t>;  // first unit, end unit, pairs
 
 // Cuts the (batch, kv head) units into consecutive chunks of equal length whose dS fits `limit` bytes: as few chunks as the
@@ -444,7 +458,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
     return s->padded() ? o.narrow(2, 0, q_len) : o;
   }
   s->limit = ds_limit(p, limit, factor);
-  s->dense = p.dense_bytes() <= s->limit;
+  s->dense = dense_fits(p.dense_bytes(), s->limit);
   const bool cut = q_len != p.Sq;
   const at::Tensor o = Attention::apply(q, k, v, mask, std::move(s));
   return cut ? o.narrow(2, 0, q_len) : o;
@@ -494,6 +508,7 @@ std::vector<at::Tensor> backward_on_lists(const at::Tensor& q, const at::Tensor&
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bind", &bind);
   m.def("plan_head_chunks", &plan_head_chunks);
+  m.def("dense_fits", &dense_fits);
   m.def("attention", &attention, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("forward", &forward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("backward", &backward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());

@@ -45,3 +45,30 @@ def test_dense_numbering_changes_no_bit(gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims
             assert torch.equal(got[2], lists.k_cnt) and torch.equal(got[3], lists.k_idx)
         else:
             assert (got[2] == -7).all() and (got[3] == -7).all()
+
+
+@pytest.mark.parametrize("H,S,keep,dense", [
+    (24, 6912, 5, False),  # 54 key blocks: places for all pairs would be 2.3 GB, the selected ones are 0.2 GB
+    (24, 2048, 2, True),   # 0.2 GB, all pairs
+])
+def test_backward_memory_of_a_sparse_call(gpu, H, S, keep, dense):
+    """Outside small problems the dS workspace follows the selected pairs."""
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd import interface, masks
+
+    n = S // 128
+    q, k, v = (torch.randn((1, H, S, 128), device=gpu, dtype=torch.bfloat16).requires_grad_(True) for _ in range(3))
+    mask = masks.random_block_mask(1, H, n, n, keep, 0).to(gpu)
+    assert interface.dense_ds_fits(q, k) is dense
+    print(f"memory of backward H{H} S{S} keep {keep}", flush=True)
+    o = fba.flex_block_attn_func(q, k, v, 128, 128, mask)
+    do = torch.randn_like(o)
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    torch.autograd.grad(o, (q, k, v), do)
+    torch.cuda.synchronize()
+    ds = interface.dense_ds_bytes(q, k) if dense else int(mask.sum()) * 128 * 128 * 2
+    # the three gradients, statistics (two floats a row), the tail-splitting workspace, rounding by the allocator
+    rest = 3 * q.numel() * 2 + 2 * H * S * 4 + interface._split_bytes() + 2 ** 22
+    assert torch.cuda.max_memory_allocated() - before <= ds + rest
