@@ -1,4 +1,5 @@
 // Tail splitting: which items of a launch are cut into parts (see SplitPlan in fba_kernels.h).
+#include <algorithm>
 #include <cstdlib>
 #include <mutex>
 
@@ -61,7 +62,8 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, double step_c
 namespace {
 
 constexpr int kQueueBytes = 256;
-constexpr int kRankBlock = 256;
+constexpr int kRankItems = 64;      // items a block of the ordering launch places
+constexpr int kMostOrdered = 2048;  // items of a launch that is ordered at all: eight rounds
 
 __global__ void queue_reset_kernel(int* queue) { queue[threadIdx.x] = 0; }
 
@@ -74,12 +76,14 @@ __global__ void queue_reset_kernel(int* queue) { queue[threadIdx.x] = 0; }
 // every run is cut into segments of `segment` items counted from its end, and each segment is sorted by counting, for every
 // item, the items of the segment in front of it (longer, or as long with a lower number): no atomics, one result.  Segments
 // keep the heads of a large launch one after the other, so that work-groups that run together still share Q and dO in L2.
-// Grid: spans * ceil(longest run / 256) blocks.
-__global__ __attribute__((amdgpu_flat_work_group_size(kRankBlock, kRankBlock))) void order_items_kernel(const BwdParams p, int spans, int segment, int32_t* order) {
-  __shared__ int lens[kRankBlock];
+// Lists of one length keep index order, so for them the launch is all cost: it has to be short.  Four lanes share the counting of
+// an item, with eight LDS reads in flight each; with one lane per item and a read at a time the chain of reads set the time.
+// Grid: spans * ceil(longest run / 64) blocks.
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void order_items_kernel(const BwdParams p, int spans, int segment, int32_t* order) {
+  __shared__ int lens[kMostOrdered];
   const int tid = threadIdx.x;
   if (p.queue != nullptr && blockIdx.x == 0 && tid < kQueueBytes / 4) p.queue[tid] = 0;
-  const int span = blockIdx.x % spans, i0 = blockIdx.x / spans * kRankBlock;
+  const int span = blockIdx.x % spans, i0 = blockIdx.x / spans * kRankItems;
   const int start = span * (p.num_items / spans) + min(span, p.num_items % spans);
   const int count = p.num_items / spans + (span < p.num_items % spans);
   if (i0 >= count) return;
@@ -94,21 +98,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(kRankBlock, kRankBlock))) 
     return n;
   };
   auto segment_end = [&](int i) { return count - (count - 1 - i) / segment * segment; };
-  const int i = min(i0 + tid, count - 1);
-  const int own = length(i), hi = segment_end(i), lo = max(0, hi - segment);
-  const int from = max(0, segment_end(i0) - segment), to = segment_end(min(i0 + kRankBlock, count) - 1);  // of all items of the block
-  int rank = lo;
-  for (int j0 = from; j0 < to; j0 += kRankBlock) {
-    __syncthreads();
-    lens[tid] = length(min(j0 + tid, count - 1));
-    __syncthreads();
-    const int first = max(lo, j0), last = min(hi, j0 + kRankBlock);
-    for (int j = first; j < last; ++j) {
-      const int other = lens[j - j0];
-      rank += other > own || (other == own && j < i);
-    }
+  const int from = max(0, segment_end(i0) - segment), to = segment_end(min(i0 + kRankItems, count) - 1);  // of all items of the block
+  for (int j = from + tid; j < to; j += 256) lens[j - from] = length(j);
+  __syncthreads();
+  const int i = min(i0 + (tid >> 2), count - 1);
+  const int own = lens[i - from], hi = segment_end(i), lo = max(0, hi - segment);
+  int before = 0;
+#pragma unroll 8
+  for (int j = lo + (tid & 3); j < hi; j += 4) {
+    const int other = lens[j - from];
+    before += other > own || (other == own && j < i);
   }
-  if (i0 + tid < count) order[(int64_t)rank * spans + span] = start + i;
+  before += __shfl_xor(before, 1);
+  before += __shfl_xor(before, 2);
+  if ((tid & 3) == 0 && i0 + (tid >> 2) < count) order[(int64_t)(lo + before) * spans + span] = start + i;
 }
 
 }  // namespace
@@ -129,13 +132,20 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
   const int64_t bottom = parts * slot_bytes;
   int* const queue = ws != nullptr && top >= bottom ? reinterpret_cast<int*>(ws + top) : nullptr;
   top = (top - (int64_t)p.num_items * 4) & ~(int64_t)15;
-  // Items are ordered where they start in more than one round and in at most eight, and the longest possible list has at
-  // least 128 slabs.  One round starts everything at once; over many rounds the spread of the last one no longer counts, while
-  // tiles in index order share more of their lists in L2 (structured masks): measured, steps with items in index order /
-  // ordered, B2 H16/4 S8192 (2 rounds) 1113 / 1062 us, B1 H24 S30720 random (7.5 rounds per chunk) 16.53 / 16.04 ms, H24
-  // S69120 top-k (17 rounds) 25.3 / 25.2 ms, H24 S115200 sliding window (28 rounds) 52.1 / 52.9 ms.  With shorter lists the
-  // spread is worth less than the launch (21 us for 640 items, rocprofv3).
-  const bool ordered = !p.tiled && queue != nullptr && top >= bottom && p.num_items > slots && p.num_items <= 8 * slots && p.Hq / p.Hkv * (p.Sq / 32) >= 128;
+  // Items are ordered where they start in more than one round and in at most eight.  One round starts everything at once; over
+  // many rounds the spread of the last one no longer counts, while tiles in index order share more of their lists in L2
+  // (structured masks).  Steps, items in index order / ordered: masks that choose per head, a quarter kept, H8 S8192 (2 rounds)
+  // 344 / 314 us, H24 S6144 (4.5) 599 / 585, B2 H16/4 S8192 (2) 1088 / 1065, 40 % kept, H24 S30720 (7.5 per chunk) 16.53 / 16.04
+  // ms; causal H8 S15360 (3.75) 2341 / 2116 us; H24 S69120 top-k (17) 25.3 / 25.2 ms, H24 S115200 sliding window (28) 52.1 / 52.9
+  // ms.  Where all lists are equally long it gains nothing and costs the launch (6.6 us for 1920 items, rocprofv3), or next to
+  // nothing where a launch has to clear the claim counters anyway: all blocks, H8 S9216 1371 / 1376 us, H24 S6144 1740 / 1734.  So
+  // without claims the longest possible list has to have 192 slabs, with them 128: bands of a quarter, H12 S4096 (128 slabs, 1.5
+  // rounds) 174 / 179 us, which the 179 / 176 us of a random mask of that size do not make up for, H32 S4096 (4 rounds) 365 / 367
+  // against 377 / 359 us; a random mask at H8 S6144 (192 slabs, 1.5 rounds) 302 / 297 us, 308 / 289 where all
+  // heads share it.
+  const int longest = p.Hq / p.Hkv * (p.Sq / 32);
+  const bool ordered = !p.tiled && queue != nullptr && top >= bottom && p.num_items > slots && p.num_items <= std::min(8 * slots, kMostOrdered) &&
+                       longest >= (p.split.first + parts >= 4 * slots ? 128 : 192);
   if (ordered) p.split.main_wgs = p.split.first;
 
   // Launches of four rounds and more let the work-groups claim their grid indices, with some more work-groups than indices,
@@ -152,9 +162,9 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
     const int spans = heads >= 8 ? 8 : 1;
     const int tiles_per_head = p.Skv / tile_rows, two_rounds = 2 * slots / spans;
     const int segment = (two_rounds + tiles_per_head - 1) / tiles_per_head * tiles_per_head;
-    const int blocks = spans * (((p.num_items + spans - 1) / spans + kRankBlock - 1) / kRankBlock);
+    const int blocks = spans * (((p.num_items + spans - 1) / spans + kRankItems - 1) / kRankItems);
     int32_t* const order = reinterpret_cast<int32_t*>(ws + top);
-    hipLaunchKernelGGL(order_items_kernel, dim3(blocks), dim3(kRankBlock), 0, stream, p, spans, segment, order);
+    hipLaunchKernelGGL(order_items_kernel, dim3(blocks), dim3(256), 0, stream, p, spans, segment, order);
     p.order = order;
   } else if (p.queue != nullptr) {
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(kQueueBytes / 4), 0, stream, p.queue);

@@ -16,6 +16,12 @@ MAX_ABS, REL_L2 = 2e-2, 1e-2
     (2, 3, 3, 4096, 12288, 128, 384, 4, 0.3),   # 576 items in one run, 64 of them split, key blocks of three tiles
     (1, 8, 8, 4096, 16384, 128, 128, 4, 0.05),  # 1024 items, one head per XCD, two segments
     (1, 4, 4, 4096, 8320, 128, 128, 4, 1.0),    # 260 lists of one length
+    # the same where lists of up to 192 slabs make launches without claim counters ordered as well
+    (1, 18, 9, 3072, 3968, 128, 128, 4, 0.3),
+    (1, 1, 1, 6144, 32896, 128, 128, 2, 0.2),
+    (2, 3, 3, 6144, 12288, 128, 384, 4, 0.3),
+    (1, 4, 4, 6144, 8320, 128, 128, 4, 1.0),
+    (1, 8, 8, 6144, 32640, 128, 128, 4, 0.05),  # 2040 items, 255 on each run: segments that are no multiple of 64
 ])
 def test_ordered_key_tiles(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, density):
     import flex_block_attn_amd as fba
