@@ -130,6 +130,15 @@ bool dense_fits(int64_t bytes, int64_t limit) {
   return pybind11::module_::import("torch").attr("cuda").attr("is_current_stream_capturing")().cast<bool>();
 }
 
+// Listed pairs of every (batch, kv head) unit, from the pair numbers at the head boundaries of the mask: the heads of a GQA group
+// share their kv head's launch.
+std::vector<int64_t> unit_pairs(const std::vector<int64_t>& bounds, int64_t units, int64_t group) {
+  std::vector<int64_t> pairs(units);
+  const bool shared = bounds.size() == 2;  // one mask for all heads
+  for (int64_t u = 0; u < units; ++u) pairs[u] = shared ? bounds[1] * group : bounds[(u + 1) * group] - bounds[u * group];
+  return pairs;
+}
+
 using Chunk = std::tuple<int64_t, int64_t, int64_t>;  // first unit, end unit, pairs
 
 // Cuts the (batch, kv head) units into consecutive chunks of equal length whose dS fits `limit` bytes: as few chunks as the
@@ -211,15 +220,11 @@ std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, cons
   if (dense) {
     ds = workspace(p.dense_bytes());
   } else if (mode != HandOver::kNever && !bounds.empty()) {
-    std::vector<int64_t> unit_pairs(units);
-    int64_t total = 0, most = 0;
-    for (int64_t u = 0; u < units; ++u) {  // the heads of a GQA group share their kv head's launch
-      unit_pairs[u] = p.mask_bh == 1 ? bounds.back() * group : bounds[(u + 1) * group] - bounds[u * group];
-      total += unit_pairs[u];
-    }
+    const std::vector<int64_t> pairs = unit_pairs(bounds, units, group);
+    int64_t total = std::accumulate(pairs.begin(), pairs.end(), int64_t{0}), most = 0;
     if (total > 0) {
       if (mode == HandOver::kWhole) chunks = std::vector<Chunk>{{0, units, total}};
-      else chunks = plan_head_chunks(unit_pairs, p.pair_bytes(), limit);
+      else chunks = plan_head_chunks(pairs, p.pair_bytes(), limit);
     }
     if (chunks) {
       for (const Chunk& c : *chunks) most = std::max(most, std::get<2>(c));
@@ -507,6 +512,7 @@ std::vector<at::Tensor> backward_on_lists(const at::Tensor& q, const at::Tensor&
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bind", &bind);
+  m.def("unit_pairs", &unit_pairs);
   m.def("plan_head_chunks", &plan_head_chunks);
   m.def("dense_fits", &dense_fits);
   m.def("attention", &attention, pybind11::call_guard<pybind11::gil_scoped_release>());

@@ -296,12 +296,9 @@ def ds_workspace_limit(q, k):
 
 
 def _unit_pairs(lists, B, Hq, Hkv):
-    """Listed pairs of every (batch, kv head): the heads of a GQA group share their kv head's launch."""
+    """(listed pairs of every (batch, kv head), pair numbers at the head boundaries), as backward counts them."""
     bounds = number_pairs(lists).pair_bounds()
-    group = Hq // Hkv
-    if lists.mask_bh == 1:
-        return [bounds[-1] * group] * (B * Hkv), bounds
-    return [bounds[(u + 1) * group] - bounds[u * group] for u in range(B * Hkv)], bounds
+    return _lib.host().unit_pairs(bounds, B * Hkv, Hq // Hkv), bounds
 
 
 def ds_workspace_bytes(lists, B, Hq, q_block_size, kv_block_size):

@@ -72,3 +72,10 @@ def test_backward_memory_of_a_sparse_call(gpu, H, S, keep, dense):
     # the three gradients, statistics (two floats a row), the tail-splitting workspace, rounding by the allocator
     rest = 3 * q.numel() * 2 + 2 * H * S * 4 + interface._split_bytes() + 2 ** 22
     assert torch.cuda.max_memory_allocated() - before <= ds + rest
+
+
+@pytest.mark.parametrize("cfg", [(2, 4, 2, 1024, 768, 128, 256, 4), (1, 3, 3, 1536, 1536, 384, 384, 2)])
+def test_dense_numbering_with_32_keys_per_wave(gpu, monkeypatch, cfg):
+    """The same in the dK/dV kernel kept for measurement."""
+    monkeypatch.setenv("FBA_DKDV_KEYS_PER_WAVE", "32")
+    test_dense_numbering_changes_no_bit(gpu, *cfg)

@@ -379,3 +379,11 @@ def test_split_workspace_setting(monkeypatch, mib, expected):
 
     monkeypatch.setattr(interface, "SPLIT_WORKSPACE_MIB", mib)
     assert interface._split_bytes() == expected
+
+
+def test_pairs_of_every_kv_head(lib):
+    """What backward plans its chunks from: pair numbers at the head boundaries of the mask, summed over the heads of a group."""
+    assert lib.host().unit_pairs([0, 1, 3, 6, 10], 2, 2) == [3, 7]
+    assert lib.host().unit_pairs([0, 4, 4, 9], 3, 1) == [4, 0, 5]
+    assert lib.host().unit_pairs([0, 5], 3, 2) == [10, 10, 10]  # one mask for all heads
+    assert lib.host().unit_pairs([0, 5], 1, 1) == [5]
