@@ -203,8 +203,8 @@ def main():
     ap.add_argument("--fwd-tile-rows", choices=["128", "384"], default=None,
                     help="query rows per forward work-group where both kernels apply (measurement of the two forward variants)")
     ap.add_argument("--dkdv-keys-per-wave", choices=["32", "64"], default=None,
-                    help="keys per wave of the dK/dV kernel on block lists: 32 (two waves per SIMD, the default) or 64 (one wave per "
-                         "SIMD, accumulators in accumulation registers); measurement of the two variants")
+                    help="keys per wave of the dK/dV kernel on block lists: 32 (two waves per SIMD) or 64 (one wave per "
+                         "SIMD, accumulators in accumulation registers, the default); measurement of the two variants")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="also run a plain 256 MiB device copy three times, as the known-size yardstick for rocprofv3's FETCH_SIZE / WRITE_SIZE counters")
     ap.add_argument("--probe-atomics", action="store_true",

@@ -2,7 +2,7 @@
 //
 //   dQ = dS K                                   (reference: flex_block_attn_h100.cu:750-753)
 // The reference forms dS and dQ in one key-major kernel and adds dQ into an fp32 buffer with reducing stores
-// (:707-708).  Here the key-major kernel (dkdv_kernel with kHandOver) stores the bf16 dS of every selected block pair
+// (:707-708).  Here the key-major kernel (dkdv64_kernel; dkdv_slab_kernel on tile lists) stores the bf16 dS of every selected block pair
 // once, and this query-major kernel reads it back: two products per pair instead of the six of dq_kernel, which
 // recomputes S and dP.  Every dQ element is still written exactly once, by the work-group that owns its row.
 //

@@ -37,7 +37,13 @@ int device_compute_units() { return compute_units(); }
 // max_steps steps each the round takes about  max_steps step_cost / parts + m parts  in units of what one part's results
 // cost, least at parts = sqrt(max_steps step_cost / m).  The lists are on the device: step_cost assumes that 40 % of the
 // longest possible list is there.  One part's 64 KiB cost 27 ns at what the stores and the merge sustain (2.4 TB/s) and a
-// forward step of such a round 0.65 us, so forward has step_cost 9.  Measured, forward / backward in us (always as many
+// forward step of such a round 0.65 us, so forward has step_cost 9, and 18 on tile lists, whose parts store half as much.  dK/dV
+// has 6 with 128 keys (0.9 us a slab, 128 KiB a part) and 9 with 64 keys (0.6 us, 64 KiB); dQ has forward's 9 where it recomputes
+// S and dP and 4 from dS, whose step is two products instead of six.  Times with a quarter / half / once / twice / four times each
+// value: forward (9) H8 S768 60 % kept 14.8 / 14.6 / 14.4 / 18.9 / 19.5 us, H4 S4096 20 % kept 21.2 / 20.7 / 28.6 / 29.4 / 29.3, 60 %
+// kept 45.6 / 45.1 / 42.2 / 41.1 / 40.9; (18) H4 S4096 60 % kept 36.3 / 35.1 / 34.7 / 40.3 / 39.6; steps, (6) H4 S4096 60 % kept 157 /
+// 156 / 144 / 144 / 144; (4) 145 / 144 / 144 / 143 / 154; (9, 64 keys) H2 S4096 60 % kept 132 / 130 / 127 / 128 / 128.  No value is
+// ahead at every density: short lists want fewer parts, long ones more.  Measured, forward / backward in us (always as many
 // parts as slots allow, against this rule): B1 H8 S768, 128-token blocks, half kept 22.0 / 54.9 -> 15.8 / 43.0; H4 S1536
 // 23.9 / 58.5 -> 19.8 / 54.7; H8 S4096, a quarter kept 43.2 / 104.8 -> 37.0 / 92.9.
 SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, double step_cost, int64_t slot_bytes, void* ws, int64_t ws_bytes) {

@@ -412,8 +412,8 @@ def flex_block_attn_func(q, k, v, q_block_size, kv_block_size, block_mask):
         o = _lib.host().attention(q, k, v, q_block_size, kv_block_size, block_mask, DS_WORKSPACE_LIMIT_GIB * 2 ** 30, DS_WORKSPACE_FACTOR, split)
         if o is not None:
             return o
-    # arguments that need preparation (lengths that are no whole tiles, a mask that is not contiguous), and everything that
-    # is going to be reported
+    # arguments that need preparation (a mask that is not contiguous, strided tensors whose lengths are no whole tiles), calls
+    # that are traced, and everything that is going to be reported
     pad_q = _pad_rows(q.shape[2], q_block_size, kv_block_size)
     pad_k = _pad_rows(k.shape[2], kv_block_size, q_block_size)
     if pad_q == 0 and pad_k == 0:

@@ -66,9 +66,11 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  *   split_ws_bytes  its size; fba_split_workspace_bytes() is what the planner can use at most (a smaller buffer limits
  *                   the number of ranges, never correctness)
  * On tile lists forward (64-row tiles) and the dK/dV kernel split; the dQ kernels do not.
- * The same workspace lends its last 256 bytes (when they lie behind the partial results) to the dK/dV kernels of launches of
- * four rounds and more: eight counters, zeroed by a one-wave launch in front, from which the work-groups claim the tile they
- * work on, with an eighth more work-groups launched than there are tiles.  The hardware deals work-groups to the eight
+ * The same workspace lends what lies behind the partial results to the dK/dV kernels, from its end: 256 bytes for eight counters
+ * in launches of four rounds and more, zeroed by a small launch in front, from which the work-groups claim the tile they work
+ * on, with an eighth more work-groups launched than there are tiles; and, on block lists in launches of one to eight rounds, four
+ * bytes a tile for the order in which tiles are taken (long lists first), written by the same launch in front.  What does not
+ * fit is done without.  The hardware deals work-groups to the eight
  * XCDs in equal numbers; with claims an XCD that is through with its share takes over tiles of the others instead of
  * idling.  Which work-group computes a tile does not enter the result.
  */
