@@ -117,12 +117,13 @@ int64_t ds_limit(const Problem& p, double limit, double factor) {
 }
 
 // Is backward to hand dS over in a workspace with a place for every pair?  It takes a constant off a step, two launches, a pinned
-// copy and a wait (17-33 us), and costs memory that grows with all pairs instead of the selected ones.  So the line is drawn
-// where the constant no longer counts.  Steps with pairs numbered / dense, 10 % and 40 % kept, 128-token blocks: H4 S4096 (128
-// MiB) 110 / 84 and 136 / 114 us; H24 S3072 (432 MiB) 165 / 145 and 279 / 261; H24 S4096 (768 MiB) 187 / 170 and 369 / 352;
-// H24 S5120 (1.2 GiB) 252 / 235 and 570 / 550; H24 S6784 (2.1 GiB) 378 / 362 and 927 / 910.
+// copy and a wait (17-36 us), and costs memory that grows with all pairs instead of the selected ones.  So the line is drawn
+// where the constant is 2 to 5 % of a step, and the memory stays under 1 % of the card's.  Steps with pairs numbered / dense,
+// 10 % and 40 % kept, 128-token blocks: H4 S4096 (128 MiB) 110 / 84 and 136 / 114 us; H24 S3072 (432 MiB) 165 / 145 and 279 / 261;
+// H24 S4096 (768 MiB) 187 / 170 and 369 / 352; H24 S5120 (1.2 GiB) 252 / 235 and 570 / 550; H24 S6784 (2.1 GiB) 378 / 362 and
+// 927 / 910; B2 H22 S3584, 64 x 128 blocks, 57 % kept (1.05 GiB) 830 / 794.
 // Steps recorded into a graph use it as far as the limit allows: the wait for the pair count cannot be captured.
-constexpr int64_t kDenseMost = 1LL << 30;
+constexpr int64_t kDenseMost = 2LL << 30;
 bool dense_fits(int64_t bytes, int64_t limit) {
   if (bytes > limit) return false;
   if (bytes <= kDenseMost) return true;

@@ -315,7 +315,7 @@ def dense_ds_bytes(q, k):
 
 def dense_ds_fits(q, k):
     """Whether backward hands dS over without numbering the selected pairs: true for small problems, where the numbering
-    launches and the wait for the pair count would be a good part of the time (all pairs of all heads in at most 1 GiB and
+    launches and the wait for the pair count would be a good part of the time (all pairs of all heads in at most 2 GiB and
     within the limit above), and within the limit alone while the current stream is captured."""
     with torch.cuda.device_of(q):
         return _lib.host().dense_fits(dense_ds_bytes(q, k), ds_workspace_limit(q, k))
