@@ -348,6 +348,9 @@ constexpr int kChunkBytes = 2 * kSlabBytes;  // 64 keys
 constexpr int kHalfRows = 64;
 constexpr int kHalfSlotBytes = (kHalfRows * kHeadDim + 2 * kHalfRows) * 4;  // partial result of one part of a split item
 constexpr int kHalfSmem = 5 * kChunkBytes;
+// Softmax reference of a row that has met no score yet.  Finite and below every finite score of use, so that exp2 never sees inf -
+// inf where all keys of a slab are masked out or have scores of -inf, also when only one of a row group's two waves meets others.
+constexpr float kNoReference = -3e38f;
 
 // The entries of a tile list that name one 64-row half, in order.  All lanes of a wave call everything together.
 struct HalfList {
@@ -448,7 +451,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     st.tr.rd[mb][1] += par * kSlabBytes;
   }
   st.c = p.scale_log2e;
-  st.m_run = kRows ? -1e30f : -INFINITY;  // finite where whole slabs can be masked out, so that exp2 never sees inf - inf
+  st.m_run = kNoReference;
   st.l_run = 0.f;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
@@ -581,8 +584,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const float* stat = reinterpret_cast<const float*>(smem + 4 * kSlabBytes) + other * 128;
   const float m_other = stat[lane];
   const float m = fmaxf(st.m_run, m_other);
-  const float w_own = st.m_run == -INFINITY ? 0.f : fast_exp2((st.m_run - m) * st.c);
-  const float w_other = m_other == -INFINITY ? 0.f : fast_exp2((m_other - m) * st.c);
+  const float w_own = fast_exp2((st.m_run - m) * st.c);
+  const float w_other = fast_exp2((m_other - m) * st.c);
   const float l = sum_halves(w_own * st.l_run + w_other * stat[64 + lane]);
   f32x4 out[2][4];
   {

@@ -61,3 +61,28 @@ def test_fwd_halves(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kind):
     assert torch.equal(torch.isinf(lse), empty) and bool((o[empty[..., 0]] == 0).all())
     assert float((lse - lse_want)[~empty].abs().max()) <= 2e-2  # the denominator sums bf16-rounded P
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
+
+
+@pytest.mark.parametrize("qbs,kbs,Skv", [(64, 64, 384), (64, 128, 384), (16, 64, 384), (192, 64, 384), (64, 64, 16384)])
+def test_fwd_scores_of_minus_infinity(gpu, qbs, kbs, Skv):
+    """Keys whose scores are -inf count for nothing, also where they fill the first slabs a wave meets, all of one wave's slabs, or
+    (last case) a whole part of a split list."""
+    import flex_block_attn_amd as fba
+
+    Sq = 384
+    g = torch.Generator().manual_seed(Skv + qbs)
+    q, k, v = (torch.randn((1, 1, s, 128), generator=g).to(torch.bfloat16) for s in (Sq, Skv, Skv))
+    q[..., 0] = q[..., 0].abs() + 0.125
+    out = torch.rand((Skv,), generator=g) < 0.3
+    out[:96] = True                        # the first chunk and the first half of the second
+    out[torch.arange(Skv) % 64 >= 32] = True  # everything of one of the two waves of a row group
+    out[Skv // 2: Skv // 2 + Skv // 4] = True
+    k[0, 0, out, 0] = -float("inf")
+    mask = torch.ones((Sq // qbs, Skv // kbs), dtype=torch.bool)
+    print(f"-inf scores Skv{Skv} q{qbs} k{kbs}", flush=True)
+    o, lse = fba.forward_with_lists(q.to(gpu), k.to(gpu), v.to(gpu), qbs, kbs, fba.lists_for(mask.to(gpu), qbs, kbs))
+    s = (q[0, 0].double() @ k[0, 0].double().T) / 128 ** 0.5
+    want = s.softmax(-1) @ v[0, 0].double()
+    got = o[0, 0].double().cpu()
+    assert float((got - want).abs().max()) <= MAX_ABS and float((got - want).norm() / want.norm()) <= REL_L2
+    assert float((lse.reshape(-1).double().cpu() - s.logsumexp(-1)).abs().max()) <= 2e-2
