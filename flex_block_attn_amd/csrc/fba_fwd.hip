@@ -348,9 +348,10 @@ constexpr int kChunkBytes = 2 * kSlabBytes;  // 64 keys
 constexpr int kHalfRows = 64;
 constexpr int kHalfSlotBytes = (kHalfRows * kHeadDim + 2 * kHalfRows) * 4;  // partial result of one part of a split item
 constexpr int kHalfSmem = 5 * kChunkBytes;
-// Softmax reference of a row that has met no score yet.  Finite and below every finite score of use, so that exp2 never sees inf -
-// inf where all keys of a slab are masked out or have scores of -inf, also when only one of a row group's two waves meets others.
-constexpr float kNoReference = -3e38f;
+// Softmax reference of a row that has met no score yet.  Finite and below every score of use, so that exp2 never sees inf - inf
+// where all keys of a slab are masked out or have scores of -inf, also when only one of a row group's two waves meets others.
+// (Scores below it count for nothing; fp32 cannot tell such scores from their neighbours in any case.)
+constexpr float kNoReference = -1e30f;
 
 // The entries of a tile list that name one 64-row half, in order.  All lanes of a wave call everything together.
 struct HalfList {
