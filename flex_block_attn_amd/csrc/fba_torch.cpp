@@ -18,6 +18,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/custom_class.h>
 #include <torch/extension.h>
@@ -470,6 +471,25 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   return cut ? o.narrow(2, 0, q_len) : o;
 }
 
+// The same for whatever a Python caller passes: nothing for objects that are no tensors, for tensor subclasses (their results are
+// of their type, which Python sees to) and for block sizes that are no ints of 32 bits.
+c10::optional<at::Tensor> attention_of(pybind11::handle q, pybind11::handle k, pybind11::handle v, pybind11::handle q_block, pybind11::handle k_block,
+                                       pybind11::handle mask, double limit, double factor, int64_t split_bytes) {
+  for (pybind11::handle t : {q, k, v, mask})
+    if (!THPVariable_CheckTypeExact(Py_TYPE(t.ptr()))) return c10::nullopt;
+  int64_t blocks[2];
+  for (int i = 0; i < 2; ++i) {
+    PyObject* const size = (i ? k_block : q_block).ptr();
+    int overflow = 0;
+    if (!PyLong_CheckExact(size)) return c10::nullopt;
+    blocks[i] = PyLong_AsLongLongAndOverflow(size, &overflow);
+    if (overflow != 0 || blocks[i] > 0x7fffffffLL) return c10::nullopt;
+  }
+  const at::Tensor qt = THPVariable_Unpack(q.ptr()), kt = THPVariable_Unpack(k.ptr()), vt = THPVariable_Unpack(v.ptr()), mt = THPVariable_Unpack(mask.ptr());
+  pybind11::gil_scoped_release no_gil;
+  return attention(qt, kt, vt, blocks[0], blocks[1], mt, limit, factor, split_bytes);
+}
+
 // ---------------------------------------------------------------------------------------------------------------------
 // entry points on lists (checked by the caller)
 // ---------------------------------------------------------------------------------------------------------------------
@@ -516,7 +536,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("unit_pairs", &unit_pairs);
   m.def("plan_head_chunks", &plan_head_chunks);
   m.def("dense_fits", &dense_fits);
-  m.def("attention", &attention, pybind11::call_guard<pybind11::gil_scoped_release>());
+  m.def("attention", &attention_of);
   m.def("forward", &forward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("backward", &backward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
 }

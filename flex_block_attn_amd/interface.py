@@ -239,11 +239,21 @@ def _split_workspace(device):
     return ws, _ptr(ws), n
 
 
+# Types that torch.empty_like turns into a plain tensor.  Results for any other tensor type have the type empty_like gives them, so
+# that a subclass goes through the operator as through torch's own.
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _typed_like(result, t):
+    return result if type(t) in _PLAIN else torch.empty_like(t).copy_(result)
+
+
 def forward_with_lists(q, k, v, q_block_size, kv_block_size, lists):
     """Forward on compacted lists -> (o [B,H,Sq,128] bf16, lse [B,H,Sq,1] fp32)."""
     B, Hq, Hkv, Sq, Skv = _check_qkv(q, k, v)
     _check_lists(lists, q, B, Hq, Sq, Skv, q_block_size, kv_block_size)
-    return _lib.host().forward(q, k, v, q_block_size, kv_block_size, lists.mask_bh, lists.q_cnt, lists.q_idx, _split_bytes())
+    o, lse = _lib.host().forward(q, k, v, q_block_size, kv_block_size, lists.mask_bh, lists.q_cnt, lists.q_idx, _split_bytes())
+    return _typed_like(o, q), lse
 
 
 def number_pairs(lists):
@@ -350,8 +360,9 @@ def backward_with_lists(q, k, v, o, lse, do, q_block_size, kv_block_size, lists,
     lse = lse.contiguous()
     dense = hand_over is None and lists.pair_base is None and dense_ds_fits(q, k)
     bounds = [] if dense or hand_over is False else number_pairs(lists).pair_bounds()
-    return tuple(_lib.host().backward(q, k, v, o, lse, do, q_block_size, kv_block_size, lists.mask_bh, lists.q_cnt, lists.q_idx, lists.k_cnt, lists.k_idx,
-                                      lists.pair_base, lists.q_slot, lists.k_slot, bounds, hand_over, dense, ds_workspace_limit(q, k), _split_bytes()))
+    grads = _lib.host().backward(q, k, v, o, lse, do, q_block_size, kv_block_size, lists.mask_bh, lists.q_cnt, lists.q_idx, lists.k_cnt, lists.k_idx,
+                                 lists.pair_base, lists.q_slot, lists.k_slot, bounds, hand_over, dense, ds_workspace_limit(q, k), _split_bytes())
+    return tuple(_typed_like(g, t) for g, t in zip(grads, (q, k, v)))
 
 
 def _flex_block_attn_forward(q, k, v, q_block_size, kv_block_size, block_mask, small_block_mask, use_small_block_mode):
@@ -407,13 +418,12 @@ def flex_block_attn_func(q, k, v, q_block_size, kv_block_size, block_mask):
     q: (batch, heads, q_seq_len, 128) bf16; k, v: (batch, kv_heads, kv_seq_len, 128) bf16; block_mask: bool
     [q_seq_len / q_block_size, kv_seq_len / kv_block_size] or [batch, heads, ...]. Returns o shaped like q.
     """
-    if type(q_block_size) is int and type(kv_block_size) is int:
-        split = -1 if SPLIT_WORKSPACE_MIB is None else _split_bytes()
-        o = _lib.host().attention(q, k, v, q_block_size, kv_block_size, block_mask, DS_WORKSPACE_LIMIT_GIB * 2 ** 30, DS_WORKSPACE_FACTOR, split)
-        if o is not None:
-            return o
+    split = -1 if SPLIT_WORKSPACE_MIB is None else _split_bytes()
+    o = _lib.host().attention(q, k, v, q_block_size, kv_block_size, block_mask, DS_WORKSPACE_LIMIT_GIB * 2 ** 30, DS_WORKSPACE_FACTOR, split)
+    if o is not None:
+        return o
     # arguments that need preparation (a mask that is not contiguous, strided tensors whose lengths are no whole tiles), calls
-    # that are traced, and everything that is going to be reported
+    # that are traced, tensor subclasses, and everything that is going to be reported
     pad_q = _pad_rows(q.shape[2], q_block_size, kv_block_size)
     pad_k = _pad_rows(k.shape[2], kv_block_size, q_block_size)
     if pad_q == 0 and pad_k == 0:

@@ -106,3 +106,30 @@ def test_unpacked_output_may_be_strided(gpu):
     got = torch.autograd.grad(o, (q, k, v), torch.ones_like(o))
     want = torch.autograd.grad(fba.flex_block_attn_func(q, k, v, 128, 128, mask), (q, k, v), torch.ones_like(o))
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+class Marked(torch.Tensor):
+    """A tensor subclass without semantics of its own."""
+
+
+@pytest.mark.parametrize("S,bs", [(256, 128), (256, 64), (192, 64)])
+def test_tensor_subclasses_keep_their_type(gpu, S, bs):
+    """Results have the type that torch's own functions would give them: o that of q, gradients those of their tensors."""
+    import flex_block_attn_amd as fba
+
+    g = torch.Generator().manual_seed(S)
+    plain = [torch.randn((1, 1, S, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(4)]
+    mask = torch.ones((S // bs, S // bs), dtype=torch.bool, device=gpu)
+    leaves = [t.clone().requires_grad_() for t in plain[:3]]
+    want_o = fba.flex_block_attn_func(*leaves, bs, bs, mask)
+    want = torch.autograd.grad(want_o, leaves, plain[3])
+    assert type(want_o) is torch.Tensor
+    for which in ((0, 1, 2), (0,)):
+        leaves = [t.clone().as_subclass(Marked).requires_grad_() if i in which else t.clone().requires_grad_() for i, t in enumerate(plain[:3])]
+        o = fba.flex_block_attn_func(*leaves, bs, bs, mask)
+        got = torch.autograd.grad(o, leaves, plain[3])
+        assert type(o) is Marked and torch.equal(o.as_subclass(torch.Tensor), want_o)
+        assert all(torch.equal(a.as_subclass(torch.Tensor), b) for a, b in zip(got, want))
+        with torch.no_grad():
+            assert type(fba.flex_block_attn_func(*leaves, bs, bs, mask)) is Marked
+    assert type(fba.flex_block_attn_func(torch.nn.Parameter(plain[0].clone()), plain[1], plain[2], bs, bs, mask)) is torch.Tensor

@@ -387,3 +387,20 @@ def test_pairs_of_every_kv_head(lib):
     assert lib.host().unit_pairs([0, 4, 4, 9], 3, 1) == [4, 0, 5]
     assert lib.host().unit_pairs([0, 5], 3, 2) == [10, 10, 10]  # one mask for all heads
     assert lib.host().unit_pairs([0, 5], 1, 1) == [5]
+
+
+def test_arguments_that_are_no_tensors_or_sizes():
+    """What the native call does not take reaches the checks in Python."""
+    import flex_block_attn_amd as fba
+
+    q = torch.zeros((1, 1, 128, 128), dtype=torch.bfloat16)
+    mask = torch.ones((1, 1), dtype=torch.bool)
+    for bad in (None, [[True]], mask.numpy()):
+        with pytest.raises(AttributeError):
+            fba.flex_block_attn_func(q, q, q, 128, 128, bad)
+    with pytest.raises(AttributeError):
+        fba.flex_block_attn_func(None, q, q, 128, 128, mask)
+    with pytest.raises(AssertionError, match="must be divisible by"):
+        fba.flex_block_attn_func(q, q, q, 2 ** 70, 128, mask)
+    with pytest.raises(ValueError, match="GPU tensor"):
+        fba.flex_block_attn_func(q, q, q, 128, 128, mask)
