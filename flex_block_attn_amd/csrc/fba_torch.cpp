@@ -426,9 +426,10 @@ struct Attention : torch::autograd::Function<Attention> {
 // shapes, strided tensors), which Python then reports or prepares.
 c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t q_block, int64_t k_block, const at::Tensor& mask,
                                     double limit, double factor, int64_t split_bytes) {
-  // a traced call has to appear in the trace, and forward-mode differentiation has to be refused: both go through the Python
-  // autograd function, which does that
+  // a traced call has to appear in the trace, forward-mode differentiation and function transforms have to be refused: all go
+  // through the Python autograd function, which does that
   if (torch::jit::tracer::isTracing()) return c10::nullopt;
+  if (c10::impl::tls_local_dispatch_key_set().included_.has(c10::DispatchKey::FuncTorchDynamicLayerFrontMode)) return c10::nullopt;
   for (const at::Tensor* t : {&q, &k, &v})
     if (t->_fw_grad(0).defined()) return c10::nullopt;
   for (const at::Tensor* t : {&q, &k, &v})

@@ -133,3 +133,19 @@ def test_tensor_subclasses_keep_their_type(gpu, S, bs):
         with torch.no_grad():
             assert type(fba.flex_block_attn_func(*leaves, bs, bs, mask)) is Marked
     assert type(fba.flex_block_attn_func(torch.nn.Parameter(plain[0].clone()), plain[1], plain[2], bs, bs, mask)) is torch.Tensor
+
+
+@pytest.mark.parametrize("transform", ["grad", "vjp", "vmap"])
+def test_function_transforms_are_refused_with_the_reason(gpu, transform):
+    import flex_block_attn_amd as fba
+
+    q, k, v = _inputs(gpu, 7)
+    mask = torch.ones((2, 2), dtype=torch.bool, device=gpu)
+    call = lambda x: fba.flex_block_attn_func(x, k, v, 128, 128, mask)
+    with pytest.raises(RuntimeError, match="functorch transforms"):
+        if transform == "grad":
+            torch.func.grad(lambda x: call(x).float().sum())(q)
+        elif transform == "vjp":
+            torch.func.vjp(call, q)
+        else:
+            torch.vmap(call)(q[None])
