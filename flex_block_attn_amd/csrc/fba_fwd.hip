@@ -625,6 +625,200 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
           pack4(out[mb][g][0] * inv, out[mb][g][1] * inv, out[mb][g][2] * inv, out[mb][g][3] * inv);
 }
 
+// Forward straight from the block mask, for problems too small to fill the GPU: no lists, no parts, one launch.
+//
+// Work-group = 32 query rows, eight waves, one work-group per CU.  Every wave reads the mask row of these rows itself (64 key
+// blocks to a ballot) and takes every eighth of the selected 32-key slabs; it brings in its K and V slab on its own (16 KiB of LDS
+// per wave, no barrier in the loop), with softmax statistics and O of its own, and the eight meet in LDS at the end.  Rows
+// past the end of a sequence that is no whole number of 32 are loaded as copies of the last row and not stored.
+//
+// Such a call is bound by latency: a chain of launches (lists, attention, merge of the parts) that each wait for the one in
+// front, and inside a kernel of loads that wait for loads.  Calls without gradients, lists and parts / from the mask: H1 S768,
+// 128-token blocks, 40 % kept 15.6 / 7.0 us, H2 S1536 384-token blocks 18.6 / 9.6, H1 S6144 30.3 / 17.5, H3 S2048 against 3840 keys
+// 24.3 / 16.8 us.  In longer lists a step of all eight waves takes 1.3 us, what the copies of 128 KiB take (a slab feeds 16 matrix
+// instructions here and 64 with 128 rows), so the line is drawn where that begins to count (fwd_takes_mask).  K rows straight to
+// registers, two slabs ahead, take 3 us a step: every load touches 32 rows.
+constexpr int kMaskWaves = 8;
+constexpr int kMaskRows = 32;
+constexpr int kMaskStatBase = kMaskWaves * 2 * kSlabBytes;                  // softmax references, then denominators [wave][row]
+constexpr int kMaskSmem = kMaskStatBase + 2 * kMaskWaves * kMaskRows * 4;
+
+// The 32-key slabs that some row of the work-group selects, in order.  All lanes of a wave call everything together.
+template <bool kTwo>
+struct MaskCursor {
+  const uint8_t *row0, *row1;  // mask rows of the first and the last 16 query rows (the same unless kTwo)
+  int nK, nsub, lane;
+  int base, sub;               // first of the 64 key blocks at hand, slab inside the current block
+  int ahead0, ahead1;          // this lane's mask bytes of the 64 blocks that follow
+  unsigned long long m0, m1, left;  // ballots of the 64 blocks; those not passed yet, the current one lowest
+
+  FBA_DEVICE int load(const uint8_t* row, int at) const { return at + lane < nK ? row[at + lane] : 0; }
+  FBA_DEVICE void take() {
+    m0 = __builtin_amdgcn_ballot_w64(ahead0 != 0);
+    m1 = kTwo ? __builtin_amdgcn_ballot_w64(ahead1 != 0) : m0;
+    left = m0 | m1;
+    ahead0 = load(row0, base + 64);
+    if constexpr (kTwo) ahead1 = load(row1, base + 64);
+  }
+  FBA_DEVICE void start() {
+    base = sub = 0;
+    ahead0 = load(row0, 0);
+    ahead1 = kTwo ? load(row1, 0) : 0;
+    take();
+  }
+  // n slabs on; false past the last one
+  FBA_DEVICE bool skip(int n) {
+    sub += n;
+    for (;;) {
+      while (left == 0) {
+        base += 64;
+        if (base >= nK) return false;
+        take();
+      }
+      if (sub < nsub) return true;
+      sub -= nsub;
+      left &= left - 1;
+    }
+  }
+  FBA_DEVICE int slab() const { return (base + __builtin_ctzll(left)) * nsub + sub; }
+  FBA_DEVICE int halves() const {  // which 16-row halves select the current block
+    const int b = __builtin_ctzll(left);
+    return (int)((m0 >> b) & 1) | (int)((m1 >> b) & 1) << 1;
+  }
+};
+
+template <bool kTwo>  // q_block is an odd multiple of 16: the two 16-row halves have mask rows of their own
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * kMaskWaves, 64 * kMaskWaves), amdgpu_waves_per_eu(2, 2))) void fwd_mask_kernel(const FwdMaskParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // [wave](K slab | V slab), statistics
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int item = xcd_remap(blockIdx.x, p.items_per_xcd);
+  if (item >= p.num_items) return;
+  const int tiles_per_head = (p.Sq + kMaskRows - 1) / kMaskRows;
+  const int bh = item / tiles_per_head;
+  const int row0 = (item - bh * tiles_per_head) * kMaskRows;
+  const int b = bh / p.Hq, hq = bh - b * p.Hq;
+  const int64_t kv_row0 = (int64_t)(b * p.Hkv + hq / (p.Hq / p.Hkv)) * p.Skv;
+  const char* kp = reinterpret_cast<const char*>(p.k + kv_row0 * kHeadDim);
+  const char* vp = reinterpret_cast<const char*>(p.v + kv_row0 * kHeadDim);
+
+  MaskCursor<kTwo> cursor;
+  const uint8_t* mask = p.mask + (p.mask_bh == 1 ? 0 : (int64_t)bh * p.nQ * p.nK);
+  cursor.row0 = mask + (int64_t)(row0 / p.q_block) * p.nK;
+  cursor.row1 = kTwo ? mask + (int64_t)(min(row0 + 16, p.Sq - 1) / p.q_block) * p.nK : cursor.row0;
+  cursor.nK = p.nK;
+  cursor.nsub = p.k_block / kSlab;
+  cursor.lane = lane;
+  cursor.start();
+
+  FwdState st;
+  {
+    const __bf16* qp = p.q + ((int64_t)bh * p.Sq + min(row0 + l32, p.Sq - 1)) * kHeadDim;
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) st.qreg[ks] = *reinterpret_cast<const bf16x8*>(qp + 16 * ks + 8 * h);
+  }
+  st.rm.init(lane);
+  st.tr.init(lane);
+  st.c = p.scale_log2e;
+  st.m_run = kNoReference;
+  st.l_run = 0.f;
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) st.acc_o[mb][r] = 0.f;
+
+  // copy i (0..7) of a slab fills its rows 4 i .. 4 i + 3; the swizzle repeats after 16 rows
+  uint32_t dma_off[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 4 * i + (lane >> 4);
+    dma_off[i] = (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4));
+  }
+  const char* const k_lds = smem + wave * 2 * kSlabBytes;
+  const char* const v_lds = k_lds + kSlabBytes;
+  const uint32_t k_dst = lds_addr(k_lds), v_dst = lds_addr(v_lds);
+  auto copy_slab = [&](uint32_t dst, const char* src) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) dma16(dst + 4 * i * kRowBytes, src + (i >> 2) * 16 * kRowBytes, dma_off[i & 3]);
+  };
+  // The compiler knows of no order between the copies and its LDS reads: no read moves up across a fence, and reads of a buffer
+  // have returned before it is filled again.
+  auto fence = [] { asm volatile("" ::: "memory"); };
+  auto reads_done = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+
+  bool more = cursor.skip(wave);
+  if (more) {
+    const int64_t off = (int64_t)cursor.slab() * kSlabBytes;
+    copy_slab(k_dst, kp + off);
+    copy_slab(v_dst, vp + off);
+  }
+  while (more) {
+    const int halves = cursor.halves();
+    more = cursor.skip(kMaskWaves);
+    const int64_t off = more ? (int64_t)cursor.slab() * kSlabBytes : 0;
+    const bool active = !kTwo || ((halves >> (l32 >> 4)) & 1) != 0;
+    wait_vmem<8>();  // K has landed; the eight copies of V, requested last, may still fly
+    fence();
+    f32x16 s = qk_half(st, k_lds);
+    pin(s);
+    reads_done();
+    if (more) copy_slab(k_dst, kp + off);
+    bf16x8 pk[2];
+    softmax_reference(st, s, active);
+    softmax_exp<kTwo>(st, s, pk, active);
+    if (more) wait_vmem<8>(); else wait_vmem<0>();
+    fence();
+    pv_half(st, v_lds, pk);
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb) pin(st.acc_o[mb]);
+    reads_done();
+    if (more) copy_slab(v_dst, vp + off);
+  }
+
+  // Every wave hands in its O^T (16 KiB in place of its slabs, chunk c of row r at slot c ^ r, so that neither side meets bank
+  // conflicts) and its statistics; thread t forms columns 8 (t % 16) .. +7 of row t / 16.
+  {
+    f32x4* dst = reinterpret_cast<f32x4*>(smem + wave * 2 * kSlabBytes) + l32 * 32;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        dst[(8 * mb + 2 * g + h) ^ l32] = (f32x4){st.acc_o[mb][4 * g + 0], st.acc_o[mb][4 * g + 1], st.acc_o[mb][4 * g + 2], st.acc_o[mb][4 * g + 3]};
+    float* stat = reinterpret_cast<float*>(smem + kMaskStatBase);
+    const float l = sum_halves(st.l_run);
+    if (h == 0) {
+      stat[wave * kMaskRows + l32] = st.m_run;
+      stat[(kMaskWaves + wave) * kMaskRows + l32] = l;
+    }
+  }
+  __syncthreads();
+  const int r = tid >> 4, c8 = 2 * (tid & 15);
+  const float* stat = reinterpret_cast<const float*>(smem + kMaskStatBase) + r;
+  float m = stat[0];
+#pragma unroll
+  for (int w = 1; w < kMaskWaves; ++w) m = fmaxf(m, stat[w * kMaskRows]);
+  float l = 0.f;
+  f32x4 out[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+  for (int w = 0; w < kMaskWaves; ++w) {
+    const float weight = fast_exp2((stat[w * kMaskRows] - m) * st.c);
+    l += weight * stat[(kMaskWaves + w) * kMaskRows];
+    const f32x4* src = reinterpret_cast<const f32x4*>(smem + w * 2 * kSlabBytes) + r * 32;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const f32x4 o = src[(c8 + j) ^ r];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[j][e] += weight * o[e];
+    }
+  }
+  if (row0 + r >= p.Sq) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int64_t orow = (int64_t)bh * p.Sq + row0 + r;
+  *reinterpret_cast<bf16x8*>(p.o + orow * kHeadDim + 4 * c8) =
+      pack8(out[0][0] * inv, out[0][1] * inv, out[0][2] * inv, out[0][3] * inv, out[1][0] * inv, out[1][1] * inv, out[1][2] * inv, out[1][3] * inv);
+  if (c8 == 0) p.lse[orow] = l > 0.f ? (m * st.c + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
+}
+
 // Combines the parts of the split items: O = sum_p 2^(m_p - m) O_p / sum_p 2^(m_p - m) l_p with m = max_p m_p, in part
 // order.  One thread per (query row, four head-dim columns).
 template <int kTileRows>
@@ -671,6 +865,31 @@ hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Is a problem small enough for fwd_mask_kernel?  Calls without gradients, lists / mask, at 10, 40 and 90 % kept (cross lengths: 10, 50
+// and 90 %), 128-token blocks unless noted.  One round of work-groups: n = 192 of 32 rows against 192 slabs (H1 S6144) 24.1 / 9.1,
+// 30.3 / 17.5, 41.0 / 30.7 us, n = 12 against 120 slabs (H3, 128 rows, 3840 keys) 16.3 / 7.4, 19.3 / 13.6, 21.6 / 19.7; n = 12 against 480
+// 18.3 / 12.6, 29.6 / 42.7, 40.6 / 72.1: the fewer rows, the more parts the kernels on lists make of them.  Two rounds: n = 384 against 96
+// slabs (H4 S3072) 23.7 / 13.3, 30.4 / 24.1, 40.8 / 38.0, but 64-token blocks, whose 64-row work-groups fill the GPU without parts,
+// 13.8 / 14.5, 24.9 / 23.0, 36.9 / 38.3, and n = 384 against 192 (H2 S6144) 25.7 / 17.9, 36.0 / 33.7, 54.7 / 60.7.  More: n = 576 against 24
+// (H24 S768) 11.5 / 15.1, 13.4 / 18.1, 18.9 / 23.7.
+bool fwd_takes_mask(int64_t rows, int64_t kv_len, int q_block, int k_block) {
+  const int64_t n = rows / kMaskRows, slabs = kv_len / kSlab;  // of whole work-groups; at most that many slabs to a row
+  const int cus = device_compute_units();
+  if (n <= cus) return 5 * slabs <= 600 + 2 * n;
+  return n <= 2 * cus && slabs <= 96 && (q_block % 64 != 0 || (q_block % 128 == 0 && k_block % 128 == 0));
+}
+
+hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream) {
+  void (*fn)(const FwdMaskParams) = p.q_block % 32 != 0 ? &fwd_mask_kernel<true> : &fwd_mask_kernel<false>;
+  p.num_items = p.B * p.Hq * ((p.Sq + kMaskRows - 1) / kMaskRows);
+  int grid;
+  plan_xcd_mapping(p.B * p.Hq, p.num_items, p.items_per_xcd, grid);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kMaskSmem);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(grid), dim3(64 * kMaskWaves), kMaskSmem, stream, p);
+  return hipGetLastError();
+}
 
 hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   if (p.tiled) return launch_fwd_halves(p, stream);

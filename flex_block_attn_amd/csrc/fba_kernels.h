@@ -66,6 +66,21 @@ struct FwdParams {
   SplitPlan split;
 };
 
+// Forward straight from the block mask (fwd_mask_kernel): mask [mask_bh, nQ, nK], one byte per entry, any block sizes and lengths
+// the operator takes.
+struct FwdMaskParams {
+  const __bf16* q;
+  const __bf16* k;
+  const __bf16* v;
+  __bf16* o;
+  float* lse;
+  const uint8_t* mask;
+  int64_t mask_bh;
+  int B, Hq, Hkv, Sq, Skv, nQ, nK, q_block, k_block;
+  float scale_log2e;
+  int num_items, items_per_xcd;
+};
+
 struct BwdParams {
   const __bf16* q;
   const __bf16* k;
@@ -135,6 +150,8 @@ hipError_t launch_resize_rows(int n, const void* const* src, void* const* dst, c
                               hipStream_t stream);
 hipError_t launch_resize_mask(const uint8_t* src, uint8_t* dst, int64_t M, int src_q, int src_k, int dst_q, int dst_k, hipStream_t stream);
 hipError_t launch_fwd(FwdParams p, hipStream_t stream);
+hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream);
+bool fwd_takes_mask(int64_t rows, int64_t kv_len, int q_block, int k_block);
 hipError_t launch_bwd_stats(const __bf16* o, const __bf16* d_o, const float* lse, float* stats, int64_t rows, hipStream_t stream);
 hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);

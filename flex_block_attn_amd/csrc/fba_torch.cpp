@@ -39,7 +39,7 @@ constexpr int64_t kXcds = 8;
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                \
   X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots) X(fba_tile_slots)        \
-  X(fba_fwd) X(fba_fwd_tiled) X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) \
+  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask) X(fba_fwd_takes_mask) X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) \
   X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
@@ -196,6 +196,18 @@ std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor
   check((p.tiled() ? lib.fba_fwd_tiled : lib.fba_fwd)(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), l.q_cnt, l.q_idx,
                                                       p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(),
                                                       split.bytes, current_stream(q)));
+  return {o, lse};
+}
+
+// Does forward read the block mask itself?  (Decided on the padded lengths, whether or not the call pads.)
+bool takes_mask(const Problem& p) { return lib.fba_fwd_takes_mask(p.B * p.Hq * p.Sq, p.Skv, p.q_block, p.k_block) != 0; }
+
+// Forward from the mask; q, k, v as the caller has them (lengths need not be whole tiles).
+std::pair<at::Tensor, at::Tensor> run_forward_on_mask(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask) {
+  at::Tensor o = at::empty_like(q);
+  at::Tensor lse = at::empty({p.B, p.Hq, q.size(2), 1}, q.options().dtype(at::kFloat));
+  check(lib.fba_fwd_mask(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), static_cast<const uint8_t*>(mask.data_ptr()),
+                         p.mask_bh, p.B, p.Hq, p.Hkv, q.size(2), k.size(2), kHeadDim, p.q_block, p.k_block, current_stream(q)));
   return {o, lse};
 }
 
@@ -394,7 +406,7 @@ struct Attention : torch::autograd::Function<Attention> {
                             c10::intrusive_ptr<Saved> s) {
     const Inputs in(q, k, v, mask, *s);
     build_lists(*s, in.mask, /*backward=*/true, /*numbered=*/!s->dense);
-    auto [o, lse] = run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
+    auto [o, lse] = takes_mask(s->p) ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask) : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
     ctx->save_for_backward({in.q, in.k, in.v, o, lse});
     ctx->saved_data["s"] = c10::IValue::make_capsule(std::move(s));
     return o;
@@ -460,6 +472,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   s->kv_len = kv_len;
   const bool backward = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
   if (!backward) {
+    if (takes_mask(p)) return run_forward_on_mask(p, q, k, v, mask).first;
     const Inputs in(q, k, v, mask, *s);
     build_lists(*s, in.mask, false, false);
     const at::Tensor o = run_forward(p, in.q, in.k, in.v, s->lists, split_bytes).first;
@@ -510,6 +523,15 @@ std::pair<at::Tensor, at::Tensor> forward_on_lists(const at::Tensor& q, const at
   return run_forward(p, q, k, v, l, split_bytes);
 }
 
+// Nothing where forward takes lists.  `mask` is a contiguous bool tensor.
+c10::optional<std::pair<at::Tensor, at::Tensor>> forward_on_mask(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, int64_t q_block, int64_t k_block,
+                                                                 const at::Tensor& mask) {
+  const c10::DeviceGuard guard(q.device());
+  const Problem p = problem_of(q, k, q_block, k_block, mask.dim() == 2 ? 1 : q.size(0) * q.size(1));
+  if (!takes_mask(p)) return c10::nullopt;
+  return run_forward_on_mask(p, q, k, v, mask);
+}
+
 std::vector<at::Tensor> backward_on_lists(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& lse,
                                           const at::Tensor& d_o, int64_t q_block, int64_t k_block, int64_t mask_bh, const at::Tensor& q_cnt,
                                           const at::Tensor& q_idx, const at::Tensor& k_cnt, const at::Tensor& k_idx,
@@ -539,5 +561,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("dense_fits", &dense_fits);
   m.def("attention", &attention_of);
   m.def("forward", &forward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
+  m.def("forward_on_mask", &forward_on_mask, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("backward", &backward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
 }

@@ -256,6 +256,14 @@ def forward_with_lists(q, k, v, q_block_size, kv_block_size, lists):
     return _typed_like(o, q), lse
 
 
+def _forward(q, k, v, q_block_size, kv_block_size, block_mask, lists):
+    """Forward with the kernel the native call takes: problems too small to fill the GPU read the mask itself."""
+    B, Hq, Hkv, Sq, Skv = _check_qkv(q, k, v)
+    _check_lists(lists, q, B, Hq, Sq, Skv, q_block_size, kv_block_size)
+    got = _lib.host().forward_on_mask(q, k, v, q_block_size, kv_block_size, block_mask.contiguous())
+    return forward_with_lists(q, k, v, q_block_size, kv_block_size, lists) if got is None else (_typed_like(got[0], q), got[1])
+
+
 def number_pairs(lists):
     """Pair numbering for the dS hand-over, kept on `lists`: block pairs of block lists (fba_pair_slots), pairs of
     128-row tiles of tile lists (fba_tile_slots).  The number of listed pairs, which sizes the workspace, is copied to
@@ -396,7 +404,7 @@ class FlexBlockAttnFunc(torch.autograd.Function):
         _check_blocks(q, k, q_block_size, kv_block_size, block_mask)
         is_grad = is_grad_enabled and any(x.requires_grad for x in [q, k, v])
         lists = lists_for(block_mask, q_block_size, kv_block_size, with_pair_numbers=is_grad and not dense_ds_fits(q, k))
-        o, lse = forward_with_lists(q, k, v, q_block_size, kv_block_size, lists)
+        o, lse = _forward(q, k, v, q_block_size, kv_block_size, block_mask, lists)
         if is_grad:
             ctx.save_for_backward(q, k, v, o, lse)
             ctx.q_block_size = q_block_size

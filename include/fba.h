@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2004
+#define FBA_VERSION 2005
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -86,6 +86,17 @@ int32_t fba_fwd(const void* q, const void* k, const void* v, void* o, float* lse
                 const int32_t* q_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv,
                 int32_t head_dim, int32_t q_block, int32_t k_block,
                 void* split_ws, int64_t split_ws_bytes, void* hip_stream);
+
+/*
+ * Forward straight from the block mask, in one launch and without a workspace: for problems too small to fill the GPU, where lists
+ * and parts cost more than they give.  mask [mask_bh, nQ, nK], one byte per entry, nonzero = selected.  Any block sizes and lengths
+ * the operator takes (Sq and Skv need not be whole tiles); o and lse as fba_fwd writes them, up to the order of fp32 sums.
+ */
+int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int64_t mask_bh, int32_t B,
+                     int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block,
+                     void* hip_stream);
+/* 1 where it is the faster one for rows = B * Hq * Sq query rows on the current device (both work for every size). */
+int32_t fba_fwd_takes_mask(int64_t rows, int32_t Skv, int32_t q_block, int32_t k_block);
 
 /*
  * Backward, three stream-ordered launches.  Replaces attn_backward (attn.cpp:30,
