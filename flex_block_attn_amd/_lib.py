@@ -33,7 +33,7 @@ SIGNATURES = {
     "fba_split_workspace_bytes": (_c_i64, []),
     "fba_fwd": (_c_i32, [_c_ptr] * 7 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_fwd_mask": (_c_i32, [_c_ptr] * 6 + [_c_i64] + [_c_i32] * 8 + [_c_ptr]),
-    "fba_fwd_takes_mask": (_c_i32, [_c_i64] + [_c_i32] * 3),
+    "fba_fwd_takes_mask": (_c_i32, [_c_i64, _c_i32]),
     "fba_bwd": (_c_i32, [_c_ptr] * 14 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_probe_mfma": (_c_i32, [_c_ptr, _c_ptr, _c_i32, _c_i32, _c_ptr]),
     "fba_probe_read": (_c_i32, [_c_ptr, _c_i64, _c_ptr, _c_i32, _c_ptr]),

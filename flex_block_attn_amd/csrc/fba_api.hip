@@ -181,7 +181,7 @@ int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float
   return e == hipSuccess ? FBA_OK : hip_fail(e, "forward (from the mask) launch");
 }
 
-int32_t fba_fwd_takes_mask(int64_t rows, int32_t Skv, int32_t q_block, int32_t k_block) { return fba::fwd_takes_mask(rows, Skv, q_block, k_block) ? 1 : 0; }
+int32_t fba_fwd_takes_mask(int64_t rows, int32_t Skv) { return fba::fwd_takes_mask(rows, Skv) ? 1 : 0; }
 
 int32_t fba_block_mean(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, int32_t head_dim, void* hip_stream) {
   if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);

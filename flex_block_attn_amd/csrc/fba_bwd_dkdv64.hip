@@ -71,12 +71,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   if (slot < 0) {
     item = p.order != nullptr ? grid_index : xcd_remap(grid_index, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else {
-    parts = p.split.parts;
-    item = p.split.first + slot / parts;
-    part = slot % parts;
+    if (p.order != nullptr) item = const_idx(p.order)[item];
+  } else if (!split_position(p.split, p.order, slot, item, part, parts)) {
+    return;
   }
-  if (p.order != nullptr) item = const_idx(p.order)[item];
   const int tiles_per_head = p.Skv / TK;
   const int bhk = item / tiles_per_head;
   const int kt = item - bhk * tiles_per_head;
@@ -610,12 +608,12 @@ hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
   if (e != hipSuccess) return e;
   int grid;
-  if ((e = plan_key_tiles(p, 128, 6, 2 * 128 * kHeadDim * 4, grid, stream)) != hipSuccess) return e;
+  if ((e = plan_key_tiles(p, 128, 14, 2 * 128 * kHeadDim * 4, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(256), kSmemBytes + 16, stream, p);
   const int split_items = p.num_items - p.split.first;
   if (split_items > 0) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
-    e = launch_partial_sum(p.split.ws, p.split.parts, 2 * 128 * kHeadDim, 128, outs, 2, p.split.first, split_items, p.order, stream);
+    e = launch_partial_sum(p.split, 2 * 128 * kHeadDim, 128, outs, 2, p.order, stream);
     if (e != hipSuccess) return e;
   }
   return hipGetLastError();

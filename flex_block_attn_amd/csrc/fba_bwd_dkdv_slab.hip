@@ -68,14 +68,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   }
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
   int item, part = 0, parts = 1;
-  if (grid_index < p.split.main_wgs) {
+  const int slot = grid_index - p.split.main_wgs;  // where a part's results go
+  if (slot < 0) {
     item = xcd_remap(grid_index, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else {
-    const int s = grid_index - p.split.main_wgs;
-    item = p.split.first + s / p.split.parts;
-    part = s - (item - p.split.first) * p.split.parts;
-    parts = p.split.parts;
+  } else if (!split_position(p.split, nullptr, slot, item, part, parts)) {
+    return;
   }
   const int tiles_per_head = p.Skv / kTK;
   const int bhk = item / tiles_per_head;
@@ -369,7 +367,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   if constexpr (kHandOver) poison = poison_unless_fit(p);
   if (parts > 1) {
     // part of a split item: unscaled fp32 partial sums go to the workspace, dV rows (position 0), then dK rows (position 1)
-    float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * kSlotFloats + par * (kTK * kHeadDim) + (kg * 32 + l32) * kHeadDim;
+    float* prow = p.split.ws + (int64_t)slot * kSlotFloats + par * (kTK * kHeadDim) + (kg * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -400,12 +398,12 @@ hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes);
   if (e != hipSuccess) return e;
   int grid;
-  if ((e = plan_key_tiles(p, kTK, 9, kSlotFloats * 4, grid, stream)) != hipSuccess) return e;
+  if ((e = plan_key_tiles(p, kTK, 22, kSlotFloats * 4, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes, stream, p);
   const int split_items = p.num_items - p.split.first;
   if (split_items > 0) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, kTK * kHeadDim}};
-    return launch_partial_sum(p.split.ws, p.split.parts, kSlotFloats, kTK, outs, 2, p.split.first, split_items, p.order, stream);
+    return launch_partial_sum(p.split, kSlotFloats, kTK, outs, 2, p.order, stream);
   }
   return hipGetLastError();
 }

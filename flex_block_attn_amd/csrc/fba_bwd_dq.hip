@@ -45,11 +45,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else {
-    const int s = blockIdx.x - p.split.main_wgs;
-    item = p.split.first + s / p.split.parts;
-    part = s - (item - p.split.first) * p.split.parts;
-    parts = p.split.parts;
+  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+    return;
   }
   const int tiles_per_head = p.Sq / TQ;
   const int bh = item / tiles_per_head;
@@ -222,7 +219,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   }
 
   if (parts > 1) {  // part of a split item: unscaled fp32 partial sums go to the workspace
-    float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
+    float* prow = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -245,7 +242,8 @@ hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {
   constexpr int kSmem = kRing * kPairBytes;
   p.num_items = p.B * p.Hq * (p.Sq / 128);
   // tail splitting on block lists (two work-groups per compute unit); a part stores a 128 x 128 fp32 tile
-  p.split = plan_split(p.num_items, 2, p.Skv / 32, 9, 128 * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes);
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / 128, 128, p.q_block, p.nQ, 1, p.k_block / 32};
+  p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, 128 * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   void (*fn)(const BwdParams) = p.tiled ? &dq_kernel<true> : &dq_kernel<false>;
@@ -254,7 +252,7 @@ hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kSmem, stream, p);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0};
-    return launch_partial_sum(p.split.ws, p.split.parts, 128 * kHeadDim, 128, &out, 1, p.split.first, split_items, nullptr, stream);
+    return launch_partial_sum(p.split, 128 * kHeadDim, 128, &out, 1, nullptr, stream);
   }
   return hipGetLastError();
 }

@@ -53,11 +53,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else {
-    const int s = blockIdx.x - p.split.main_wgs;
-    item = p.split.first + s / p.split.parts;
-    part = s - (item - p.split.first) * p.split.parts;
-    parts = p.split.parts;
+  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+    return;
   }
   const int tiles_per_head = p.Sq / TQ;
   const int bh = item / tiles_per_head;
@@ -230,7 +227,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
 
   const float poison = dense ? 1.f : poison_unless_fit(p);
   if (parts > 1) {  // part of a split item: unscaled fp32 partial sums go to the workspace
-    float* prow = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
+    float* prow = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -283,24 +280,28 @@ hipError_t zero_unit_address(const char** out) {
 struct PartialOuts {
   PartialOut out[2];
 };
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_sum_kernel(const float* ws, int parts, int64_t slot_floats,
-                                                                                          int rows, PartialOuts outs, int first, const int32_t* order) {
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_sum_kernel(const SplitPlan split, int64_t slot_floats, int rows, PartialOuts outs,
+                                                                                          const int32_t* order) {
   const int tid = threadIdx.x;
   const PartialOut& o = outs.out[blockIdx.y];
-  const int row = blockIdx.x * 8 + (tid >> 5);  // among the rows of all split items
   const int c4 = (tid & 31) * 4;
+  const int parts = parts_made(split);
+  if (parts == 1) return;  // done whole
+  for (int block = blockIdx.x; block < split.items * (rows / 8); block += gridDim.x) {
+  const int row = block * 8 + (tid >> 5);  // among the rows of all split items
   const int it = row / rows, r = row - it * rows;
-  const int64_t item = order != nullptr ? order[first + it] : first + it;
-  const float* src = ws + (int64_t)it * parts * slot_floats + o.offset + r * kHeadDim + c4;
+  const int64_t item = order != nullptr ? order[split.first + it] : split.first + it;
+  const float* src = split.ws + (int64_t)it * parts * slot_floats + o.offset + r * kHeadDim + c4;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int q = 0; q < parts; ++q) acc += *reinterpret_cast<const f32x4*>(src + q * slot_floats);
   *reinterpret_cast<bf16x4*>(o.out + (item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
+  }
 }
 
-hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int first, int n_items,
-                              const int32_t* order, hipStream_t stream) {
+hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order,
+                              hipStream_t stream) {
   PartialOuts o{{outs[0], outs[n_outs - 1]}};
-  hipLaunchKernelGGL(partial_sum_kernel, dim3(n_items * (rows / 8), n_outs), dim3(256), 0, stream, ws, parts, slot_floats, rows, o, first, order);
+  hipLaunchKernelGGL(partial_sum_kernel, dim3(merge_grid(split.items * (rows / 8)), n_outs), dim3(256), 0, stream, split, slot_floats, rows, o, order);
   return hipGetLastError();
 }
 
@@ -311,7 +312,8 @@ hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
   constexpr int kRows = 32 * kWaves, kSmem = kRing * stage_bytes(kWaves);
   p.num_items = p.B * p.Hq * (p.Sq / kRows);
   // tail splitting on block lists (two work-groups of four waves per compute unit, one of more); a part stores a tile of fp32 sums
-  p.split = plan_split(p.num_items, kWaves == 4 ? 2 : 1, p.Skv / 32, 4, kRows * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes);
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / kRows, kRows, p.q_block, p.nQ, 1, p.k_block / kSlab};
+  p.split = plan_split(p.num_items, kWaves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18}, kRows * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   const bool dense = p.pair_base == nullptr;
@@ -328,7 +330,7 @@ hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(64 * kWaves), kSmem, stream, p);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0};
-    e = launch_partial_sum(p.split.ws, p.split.parts, kRows * kHeadDim, kRows, &out, 1, p.split.first, split_items, nullptr, stream);
+    e = launch_partial_sum(p.split, kRows * kHeadDim, kRows, &out, 1, nullptr, stream);
     if (e != hipSuccess) return e;
   }
   return hipGetLastError();

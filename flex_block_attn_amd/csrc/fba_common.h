@@ -120,6 +120,52 @@ FBA_DEVICE float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 // measured 13-17 % slower).
 FBA_DEVICE int xcd_remap(int bid, int per_xcd) { return per_xcd > 0 ? (bid % kNumXcd) * per_xcd + bid / kNumXcd : bid; }
 
+// Sum over the 64 lanes, by register moves inside rows of 16 lanes, then from row to row (no LDS round trips).
+FBA_DEVICE int wave_sum(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8: lane 15 of a row has the row's sum
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  return __builtin_amdgcn_readlane(x, 15) + __builtin_amdgcn_readlane(x, 31) + __builtin_amdgcn_readlane(x, 47) + __builtin_amdgcn_readlane(x, 63);
+}
+
+// How many parts every split item of a launch is cut into (see SplitPlan in fba_kernels.h): by the mean length of the lists of 64 of
+// them, which every wave finds alike.  All lanes of a wave call this together.
+template <typename Plan>
+FBA_DEVICE int split_parts(const Plan& plan) {
+  const auto& l = plan.lengths;
+  if (l.cnt == nullptr) return plan.parts;
+  const int item = plan.first + (int)((threadIdx.x & 63) * (int64_t)plan.items / 64);
+  const int head = item / l.tiles, row = (item - head * l.tiles) * l.tile_rows / l.list_rows;
+  int n[4];  // of up to four heads of the group, in flight together
+#pragma unroll
+  for (int j = 0; j < 4; ++j) n[j] = l.cnt[(l.shared ? 0 : (int64_t)(head * l.group + j * l.group / 4) * l.rows_per_head) + row];
+  const int sum = wave_sum(n[0] + n[1] + n[2] + n[3]);
+  const int64_t steps = (int64_t)sum * l.steps * l.group;  // of 4 * 64 lists
+  int parts = 1;
+#pragma unroll
+  for (int j = 0; j < 7; ++j) parts += steps >= 256LL * plan.least[j];
+  return parts;
+}
+// Work-group s of those that do the parts.  The parts of an item follow each other, so that with 2, 4 or 8 of them an XCD (work-groups
+// are dealt to the eight round-robin) does the same range of all lists and has it in its L2.  (Part by part instead, so that an XCD
+// does all ranges: forward, H3 2304 rows against 61440 keys 120 -> 140 us.)  False: the launch has more work-groups than parts.
+template <typename Plan>
+FBA_DEVICE bool split_position(const Plan& plan, const int32_t* order, int s, int& item, int& part, int& parts) {
+  parts = split_parts(plan);
+  if (s == 0 && threadIdx.x == 0 && plan.lengths.cnt != nullptr) *plan.note = parts;
+  const int i = s / parts;
+  if (i >= plan.items) return false;
+  part = s - i * parts;
+  item = plan.first + i;
+  if (order != nullptr) item = __builtin_amdgcn_readfirstlane(order[item]);
+  return true;
+}
+
+// For the merge: how many parts the kernel in front made.
+template <typename Plan>
+FBA_DEVICE int parts_made(const Plan& plan) { return plan.lengths.cnt == nullptr ? plan.parts : *plan.note; }
+
 // Work claimed instead of given.  The hardware deals work-groups to the eight XCDs round-robin, as many to a fast XCD as to
 // a slow one, and an XCD that is through with its share idles until the kernel ends.  A launch with a claim counter per XCD
 // (zeroed beforehand) has some work-groups more than grid indices to do; every work-group claims an index of its own XCD

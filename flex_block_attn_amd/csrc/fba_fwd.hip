@@ -135,11 +135,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else {
-    const int s = blockIdx.x - p.split.main_wgs;
-    item = p.split.first + s / p.split.parts;
-    part = s - (item - p.split.first) * p.split.parts;
-    parts = p.split.parts;
+  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+    return;
   }
   const int tiles_per_head = p.Sq / TQ;
   const int bh = item / tiles_per_head;
@@ -298,7 +295,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const float l = sum_halves(st.l_run);
   if (parts > 1) {
     // part of a split item: unnormalised O^T, the softmax reference in log2 units and the denominator go to the workspace
-    float* slot = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (kFwdSlotBytes / 4);
+    float* slot = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (kFwdSlotBytes / 4);
     float* prow = slot + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
@@ -410,11 +407,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else {
-    const int s = blockIdx.x - p.split.main_wgs;
-    item = p.split.first + s / p.split.parts;
-    part = s - (item - p.split.first) * p.split.parts;
-    parts = p.split.parts;
+  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+    return;
   }
   const int tiles_per_head = p.Sq / kHalfRows;
   const int bh = item / tiles_per_head;
@@ -602,7 +596,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       }
   }
   if (parts > 1) {  // as in fwd_kernel
-    float* slot = p.split.ws + ((int64_t)(item - p.split.first) * parts + part) * (kHalfSlotBytes / 4);
+    float* slot = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (kHalfSlotBytes / 4);
     float* prow = slot + (rg * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
@@ -825,10 +819,12 @@ template <int kTileRows>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge_kernel(const FwdParams p) {
   const int tid = threadIdx.x;
   constexpr int kSlotFloats = kTileRows * kHeadDim + 2 * kTileRows;
-  const int row = blockIdx.x * 8 + (tid >> 5), c4 = (tid & 31) * 4;  // row among the kTileRows * (split items) rows
+  const int parts = parts_made(p.split);
+  if (parts == 1) return;  // done whole
+  for (int block = blockIdx.x; block < p.split.items * (kTileRows / 8); block += gridDim.x) {
+  const int row = block * 8 + (tid >> 5), c4 = (tid & 31) * 4;  // row among the kTileRows * (split items) rows
   const int it = row / kTileRows, r = row % kTileRows;
   const int item = p.split.first + it;
-  const int parts = p.split.parts;
   const float* slot0 = p.split.ws + (int64_t)it * parts * kSlotFloats;
   float m = -INFINITY;
   for (int q = 0; q < parts; ++q) m = fmaxf(m, slot0[(int64_t)q * kSlotFloats + kTileRows * kHeadDim + r]);
@@ -846,6 +842,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge
   const int64_t orow = (int64_t)item * kTileRows + r;  // items are consecutive tiles of [B, Hq, Sq]
   *reinterpret_cast<bf16x4*>(p.o + orow * kHeadDim + c4) = pack4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
   if (c4 == 0) p.lse[orow] = l > 0.f ? (m + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
+  }
 }
 
 namespace {
@@ -854,13 +851,14 @@ hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
   void (*fn)(const FwdParams) = p.q_block % 64 != 0 ? &fwd_half_kernel<true> : &fwd_half_kernel<false>;
   p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
   // two work-groups per compute unit; a step is as long as one of fwd_kernel, a part's results are half as large
-  p.split = plan_split(p.num_items, 2, p.Skv / 64, 18, kHalfSlotBytes, p.split.ws, p.split_ws_bytes);
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / kHalfRows, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
+  p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kHalfSmem);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kHalfSmem, stream, p);
-  if (split_items > 0) hipLaunchKernelGGL(fwd_merge_kernel<kHalfRows>, dim3(split_items * kHalfRows / 8), dim3(256), 0, stream, p);
+  if (split_items > 0) hipLaunchKernelGGL(fwd_merge_kernel<kHalfRows>, dim3(merge_grid(split_items * kHalfRows / 8)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -869,15 +867,11 @@ hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
 // Is a problem small enough for fwd_mask_kernel?  Calls without gradients, lists / mask, at 10, 40 and 90 % kept (cross lengths: 10, 50
 // and 90 %), 128-token blocks unless noted.  One round of work-groups: n = 192 of 32 rows against 192 slabs (H1 S6144) 24.1 / 9.1,
 // 30.3 / 17.5, 41.0 / 30.7 us, n = 12 against 120 slabs (H3, 128 rows, 3840 keys) 16.3 / 7.4, 19.3 / 13.6, 21.6 / 19.7; n = 12 against 480
-// 18.3 / 12.6, 29.6 / 42.7, 40.6 / 72.1: the fewer rows, the more parts the kernels on lists make of them.  Two rounds: n = 384 against 96
-// slabs (H4 S3072) 23.7 / 13.3, 30.4 / 24.1, 40.8 / 38.0, but 64-token blocks, whose 64-row work-groups fill the GPU without parts,
-// 13.8 / 14.5, 24.9 / 23.0, 36.9 / 38.3, and n = 384 against 192 (H2 S6144) 25.7 / 17.9, 36.0 / 33.7, 54.7 / 60.7.  More: n = 576 against 24
-// (H24 S768) 11.5 / 15.1, 13.4 / 18.1, 18.9 / 23.7.
-bool fwd_takes_mask(int64_t rows, int64_t kv_len, int q_block, int k_block) {
+// 18.3 / 12.6, 29.6 / 42.7, 40.6 / 72.1: the fewer rows, the more parts the kernels on lists make of them.  Two rounds: n = 288 against 72
+// (H4 S2304, all blocks) 30.9 / 33.1, n = 576 against 24 (H24 S768) 11.5 / 15.1, 13.4 / 18.1, 18.9 / 23.7.
+bool fwd_takes_mask(int64_t rows, int64_t kv_len) {
   const int64_t n = rows / kMaskRows, slabs = kv_len / kSlab;  // of whole work-groups; at most that many slabs to a row
-  const int cus = device_compute_units();
-  if (n <= cus) return 5 * slabs <= 600 + 2 * n;
-  return n <= 2 * cus && slabs <= 96 && (q_block % 64 != 0 || (q_block % 128 == 0 && k_block % 128 == 0));
+  return n <= device_compute_units() && 5 * slabs <= 600 + 2 * n;
 }
 
 hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream) {
@@ -899,13 +893,14 @@ hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   const int rows = wide ? 384 : 128;
   p.num_items = p.B * p.Hq * (p.Sq / rows);
   // tail splitting for the 128-row kernels (two work-groups per compute unit)
-  p.split = plan_split(p.num_items, 2, p.Skv / 32, 9, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes);
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / rows, rows, p.q_block, p.nQ, 1, p.k_block / kSlab};
+  p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_wgs = (p.num_items - p.split.first) * p.split.parts;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs), dim3(rows * 2), kSmem, stream, p);
-  if (split_wgs > 0) hipLaunchKernelGGL(fwd_merge_kernel<128>, dim3((p.num_items - p.split.first) * 16), dim3(256), 0, stream, p);
+  if (split_wgs > 0) hipLaunchKernelGGL(fwd_merge_kernel<128>, dim3(merge_grid((p.num_items - p.split.first) * 16)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -15,18 +15,47 @@ namespace fba {
 // would run as a partial round with most compute units idle.  With a workspace, those items are cut into `parts` ranges of
 // their lists, each run by its own work-group at the end of the grid; the work-groups store fp32 partial results into the
 // workspace and a small merge kernel combines them in a fixed order.  Items [0, first) run whole.
+//
+// How many parts pay depends on how long the lists are, which only the device knows.  The host plans for the longest possible ones and
+// says from which length on which number pays; the kernel looks at the lists (split_parts in fba_common.h) and leaves a note for the
+// merge.  Work-groups that are not needed exit at once; with one part the items are done whole and nothing is merged.
+
+// Length of an item's list in steps of the kernel: entries of its list row(s) times the steps of an entry.
+struct ListLengths {
+  const int32_t* cnt;  // [1 or heads * group, rows_per_head]; null: the plan's number of parts stands
+  int shared;          // one row set for all heads
+  int tiles, tile_rows, list_rows, rows_per_head;  // items per head, rows of an item, rows that share a list row, list rows per head
+  int group;           // rows of `group` consecutive heads add up (dK/dV: query heads of a kv head)
+  int steps;           // of an entry
+};
+
+constexpr int kMostParts = 8;
 struct SplitPlan {
   float* ws;      // null: nothing is split
   int first;      // first item that is split
-  int parts;      // work-groups per split item (>= 2 when ws is set)
+  int parts;      // work-groups per split item, at most (>= 2 when ws is set)
   int main_wgs;   // work-groups in front of the split ones (a multiple of the XCD count)
+  int items;      // that are split
+  int least[kMostParts - 1];  // steps of a list from which on 2, 3, ... parts pay
+  ListLengths lengths;
+  int32_t* note;  // behind the parts' results: how many parts the kernel made, for the merge
+};
+
+// What a step of a list takes, in units of what one part's results cost (see fba_split.hip): in a work-group alone on its compute unit,
+// in a launch where few share one and where all do.
+struct StepCost {
+  double alone, few, full;
 };
 
 // Items and work-group slots of a launch -> plan (first = num_items, parts = 1 when nothing is split).  `slot_bytes` is
 // what one part stores; the workspace must hold (num_items - first) * parts of them.  `max_steps` is the longest possible list
-// of an item in steps, `step_cost` what a step takes in units of what one part's results cost (see fba_split.hip).  main_wgs
-// is left to the launcher.
-SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, double step_cost, int64_t slot_bytes, void* ws, int64_t ws_bytes);
+// of an item.  main_wgs is left to the launcher.
+SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
+                     const ListLengths& lengths);
+
+// Work-groups of a launch that merges parts: each does every so many of the blocks of eight rows, so that little is launched where
+// the lists turn out too short for parts.
+inline int merge_grid(int blocks) { return blocks < 2048 ? blocks : 2048; }
 
 // How the whole items of a launch are dealt to the XCDs (see xcd_remap): contiguous spans when the launch has at least
 // one (batch, head) per XCD, work-group order otherwise.  Sets items_per_xcd and the number of work-groups that come
@@ -44,7 +73,7 @@ inline void plan_xcd_mapping(int heads, int whole_items, int& items_per_xcd, int
 
 constexpr int kSplitMaxSlots = 512;                           // two work-groups on each of 256 compute units
 constexpr int64_t kSplitSlotBytes = 128 * 128 * 4 * 2;        // dK and dV partials of a key tile; forward: O^T + (m, l)
-constexpr int64_t kSplitWsBytes = (kSplitMaxSlots / 2) * kSplitSlotBytes + (1 << 20);
+constexpr int64_t kSplitWsBytes = kSplitMaxSlots * kSplitSlotBytes + (1 << 20);
 
 struct FwdParams {
   const __bf16* q;
@@ -151,7 +180,7 @@ hipError_t launch_resize_rows(int n, const void* const* src, void* const* dst, c
 hipError_t launch_resize_mask(const uint8_t* src, uint8_t* dst, int64_t M, int src_q, int src_k, int dst_q, int dst_k, hipStream_t stream);
 hipError_t launch_fwd(FwdParams p, hipStream_t stream);
 hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream);
-bool fwd_takes_mask(int64_t rows, int64_t kv_len, int q_block, int k_block);
+bool fwd_takes_mask(int64_t rows, int64_t kv_len);
 hipError_t launch_bwd_stats(const __bf16* o, const __bf16* d_o, const float* lse, float* stats, int64_t rows, hipStream_t stream);
 hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);
@@ -168,9 +197,9 @@ struct PartialOut {
   float scale;
   int64_t offset;
 };
-// Items [first, first + n_items) were split; order: null, or the item of every grid index.
-hipError_t launch_partial_sum(const float* ws, int parts, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, int first, int n_items,
-                              const int32_t* order, hipStream_t stream);
+// order: null, or the item of every grid index.
+hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order,
+                              hipStream_t stream);
 hipError_t launch_probe_mfma(const float* src, float* sink, int work_groups, int iters, hipStream_t stream);
 hipError_t launch_probe_read(const void* src, int64_t bytes, uint32_t* sink, int work_groups, hipStream_t stream);
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,

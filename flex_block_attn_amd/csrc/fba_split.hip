@@ -29,39 +29,76 @@ int compute_units() {
 int device_compute_units() { return compute_units(); }
 
 // The hardware hands work-groups to free slots in index order.  With n items on s slots the last n % s items form a
-// partial round; when that round would fill at most half of the slots, each of its items is cut into up to floor(s / (n % s))
-// parts (at most 8), so that the parts fill the slots once and take 1 / parts of a round.  Launches smaller than the
+// partial round; the lists of these items are cut into parts (at most 8) where parts fill the slots better.  Launches smaller than the
 // machine (n < s) are split the same way.
 //
-// How many parts pay: every part writes its partial results, and the merge reads them back, so with m items of at most
-// max_steps steps each the round takes about  max_steps step_cost / parts + m parts  in units of what one part's results
-// cost, least at parts = sqrt(max_steps step_cost / m).  The lists are on the device: step_cost assumes that 40 % of the
-// longest possible list is there.  One part's 64 KiB cost 27 ns at what the stores and the merge sustain (2.4 TB/s) and a
-// forward step of such a round 0.65 us, so forward has step_cost 9, and 18 on tile lists, whose parts store half as much.  dK/dV
-// has 6 with 128 keys (0.9 us a slab, 128 KiB a part) and 9 with 64 keys (0.6 us, 64 KiB); dQ has forward's 9 where it recomputes
-// S and dP and 4 from dS, whose step is two products instead of six.  Times with a quarter / half / once / twice / four times each
-// value: forward (9) H8 S768 60 % kept 14.8 / 14.6 / 14.4 / 18.9 / 19.5 us, H4 S4096 20 % kept 21.2 / 20.7 / 28.6 / 29.4 / 29.3, 60 %
-// kept 45.6 / 45.1 / 42.2 / 41.1 / 40.9; (18) H4 S4096 60 % kept 36.3 / 35.1 / 34.7 / 40.3 / 39.6; steps, (6) H4 S4096 60 % kept 157 /
-// 156 / 144 / 144 / 144; (4) 145 / 144 / 144 / 143 / 154; (9, 64 keys) H2 S4096 60 % kept 132 / 130 / 127 / 128 / 128.  No value is
-// ahead at every density: short lists want fewer parts, long ones more.  Measured, forward / backward in us (always as many
-// parts as slots allow, against this rule): B1 H8 S768, 128-token blocks, half kept 22.0 / 54.9 -> 15.8 / 43.0; H4 S1536
-// 23.9 / 58.5 -> 19.8 / 54.7; H8 S4096, a quarter kept 43.2 / 104.8 -> 37.0 / 92.9.
-SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, double step_cost, int64_t slot_bytes, void* ws, int64_t ws_bytes) {
-  SplitPlan plan{nullptr, num_items, 1, 0};
+// How many parts pay: every part writes its partial results and the merge reads them back, so with m items of L steps a round
+// takes  L slope(parts) + m parts  in units of what one part's results cost, 27 ns for 64 KiB at what the stores and the merge
+// sustain (2.4 TB/s; taken a quarter dearer, since the parts of a launch end together).  slope is what a step takes times the rounds
+// the parts make, over their number.  A forward step takes 0.50 us in a work-group alone on its compute unit, 0.73 us where the
+// first share one and 0.95 us where all do (16, 22.5 and 30 units), so 72 items are better off in 3 parts than in 7: H24 384 rows
+// against 15360 keys, half kept, 63.6 -> 55.2 us.  On tile lists parts store half as much and a step is as long; dQ that recomputes S
+// and dP is like forward, dQ from dS two products instead of six; a dK/dV slab takes 0.9 us with 128 keys (128 KiB a part) and
+// 0.6 us with 64 (64 KiB).
+//
+// L is on the device: the host says from which lengths on which numbers of parts pay, up to the longest possible lists, and the kernel
+// looks at the lists.  Forward / backward, parts for lists that hold 40 % -> for the lists there are, 10 % kept: H3 S6400 27.8 / 73.9
+// -> 20.6 / 66.6 us, H5 S5120 26.8 / 62.1 -> 15.5 / 62.0, H1 S30720 62.2 / 206.9 -> 59.6 / 185.9.  Looking costs a load that
+// nothing covers, 0.5 to 1 us a launch and as much for the merge, so few items, whose parts cost little, take the number that suits
+// lists which hold 60 %.
+//
+// More than half a round is cut as well, in launches of less than two rounds, where work-groups end together: dK/dV of 136 tiles (H1
+// S17408), 40 and 90 % kept, backward 272 -> 255 and 540 -> 492 us, of 420 tiles (H3 S17920) 90 % kept 1612 -> 1424.  With items in falling
+// order of length the later rounds end at different times in any case: 680 tiles (H8 S10880) 40 % kept 579 -> 599.
+constexpr double kMergeCost = 60;   // the launch
+constexpr int64_t kNoteBytes = 16;  // behind the parts' results
+constexpr int kFewItems = 100;
+SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
+                     const ListLengths& lengths) {
+  SplitPlan plan{};
+  plan.first = num_items;
+  plan.parts = 1;
   if (ws == nullptr || num_items <= 0) return plan;
   int slots = compute_units() * wgs_per_cu;
   if (slots > kSplitMaxSlots) slots = kSplitMaxSlots;
   const int rest = num_items % slots;
-  if (rest == 0 || 2 * rest > slots) return plan;
-  int parts = slots / rest;
-  if (parts > 8) parts = 8;
-  const double whole = max_steps * step_cost;
-  while (parts >= 2 && (double)parts * parts * rest > whole) --parts;
-  while (parts >= 2 && (int64_t)rest * parts * slot_bytes > ws_bytes) --parts;
-  if (parts < 2 || whole / parts + (double)rest * parts > 0.9 * whole) return plan;
+  if (rest == 0 || (num_items >= 2 * slots && 2 * rest > slots)) return plan;
+  // cost(n) = slope(n) steps + parts and, where there are any, the launch that merges them.  From how long a list on is a number of
+  // parts the cheapest: the slope falls from one candidate to the next, and one that is never the cheapest gives way.
+  auto slope = [&](int n) {
+    const int wgs = rest * n, alone = slots / wgs_per_cu;
+    if (num_items > slots) return step.full * ((wgs + slots - 1) / slots) / n;  // those of the whole rounds are still there
+    if (wgs <= alone) return step.alone / n;
+    if (wgs <= slots) return (step.few + (step.full - step.few) * (wgs - alone) / (slots - alone)) / n;
+    return step.full * ((wgs + slots - 1) / slots) / n;
+  };
+  struct Candidate { int parts; double slope, fixed, least; } hull[kMostParts] = {{1, slope(1), 0., 0.}};
+  int n_hull = 1;
+  for (int n = 2; n <= kMostParts && (int64_t)rest * n * slot_bytes + kNoteBytes <= ws_bytes; ++n) {
+    if (num_items > slots && rest * n > slots && 2 * rest <= slots) break;  // a last round that fills up while others end gains nothing from another
+    Candidate next{n, slope(n), (double)rest * n + kMergeCost, 0.};
+    while (n_hull > 0 && next.slope < hull[n_hull - 1].slope) {
+      next.least = (next.fixed - hull[n_hull - 1].fixed) / (hull[n_hull - 1].slope - next.slope);
+      if (n_hull == 1 || next.least > hull[n_hull - 1].least) {
+        hull[n_hull++] = next;
+        break;
+      }
+      --n_hull;
+    }
+  }
+  if (n_hull == 1 || hull[1].least > 0.5 * max_steps) return plan;  // lists of usual density stay whole
+  const double longest = rest <= kFewItems ? 0.6 * max_steps : max_steps;
+  while (hull[n_hull - 1].least > longest) --n_hull;
+  for (int j = 0; j < kMostParts - 1; ++j) plan.least[j] = 0x7fffffff;
+  for (int i = 1; i < n_hull; ++i)
+    for (int n = hull[i - 1].parts + 1; n <= hull[i].parts; ++n) plan.least[n - 2] = (int)hull[i].least + 1;
+  plan.parts = hull[n_hull - 1].parts;
+  plan.items = rest;
+  plan.lengths = lengths;
+  if (rest <= kFewItems) plan.lengths.cnt = nullptr;
+  plan.note = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + (int64_t)rest * plan.parts * slot_bytes);
   plan.ws = static_cast<float*>(ws);
   plan.first = num_items - rest;
-  plan.parts = parts;
   return plan;
 }
 
@@ -127,7 +164,10 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
   const int heads = p.B * p.Hkv;
   char* const ws = reinterpret_cast<char*>(p.split.ws);  // whether or not anything is split
   p.num_items = heads * (p.Skv / tile_rows);
-  p.split = plan_split(p.num_items, 1, p.Hq / p.Hkv * (p.Sq / 32), step_cost, slot_bytes, ws, p.split_ws_bytes);
+  const int group = p.Hq / p.Hkv;
+  const ListLengths lengths = p.tiled ? ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tile_rows, tile_rows, 128, p.Skv / 128, group, 1}
+                                      : ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tile_rows, tile_rows, p.k_block, p.nK, group, p.q_block / 32};
+  p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{step_cost, step_cost, step_cost}, slot_bytes, ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(heads, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int parts = (p.num_items - p.split.first) * p.split.parts;
   p.queue = nullptr;
@@ -135,7 +175,7 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
 
   // What else lives in the workspace, from its end: the claim counters, then the order of the items.
   int64_t top = ws == nullptr ? 0 : (p.split_ws_bytes - kQueueBytes) & ~(int64_t)15;
-  const int64_t bottom = parts * slot_bytes;
+  const int64_t bottom = parts * slot_bytes + kNoteBytes;
   int* const queue = ws != nullptr && top >= bottom ? reinterpret_cast<int*>(ws + top) : nullptr;
   top = (top - (int64_t)p.num_items * 4) & ~(int64_t)15;
   // Items are ordered where they start in more than one round and in at most eight.  One round starts everything at once; over

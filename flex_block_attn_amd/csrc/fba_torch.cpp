@@ -200,7 +200,7 @@ std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor
 }
 
 // Does forward read the block mask itself?  (Decided on the padded lengths, whether or not the call pads.)
-bool takes_mask(const Problem& p) { return lib.fba_fwd_takes_mask(p.B * p.Hq * p.Sq, p.Skv, p.q_block, p.k_block) != 0; }
+bool takes_mask(const Problem& p) { return lib.fba_fwd_takes_mask(p.B * p.Hq * p.Sq, p.Skv) != 0; }
 
 // Forward from the mask; q, k, v as the caller has them (lengths need not be whole tiles).
 std::pair<at::Tensor, at::Tensor> run_forward_on_mask(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask) {

@@ -59,7 +59,7 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  * Tail splitting (no counterpart in the reference).  Work-groups are handed to free compute-unit slots in index order,
  * so the last (items % slots) 128-row tiles of a launch would run as a partial round with most of the GPU idle; the same
  * holds for a whole launch with fewer tiles than slots.  Entry points that take `split_ws` cut the lists of those tiles
- * into up to eight ranges, run each range in a work-group of its own at the end of the grid, store fp32 partial results
+ * into up to eight ranges (how many is decided by the lengths of the lists, on the device), run each range in a work-group of its own at the end of the grid, store fp32 partial results
  * into split_ws and combine them in a small second launch, in a fixed order (results stay bit-reproducible).
  *   split_ws        null (nothing is split), or 16-byte aligned device memory owned by the caller for the duration of
  *                   the call's work on the stream; its contents before and after are meaningless
@@ -96,7 +96,7 @@ int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float
                      int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block,
                      void* hip_stream);
 /* 1 where it is the faster one for rows = B * Hq * Sq query rows on the current device (both work for every size). */
-int32_t fba_fwd_takes_mask(int64_t rows, int32_t Skv, int32_t q_block, int32_t k_block);
+int32_t fba_fwd_takes_mask(int64_t rows, int32_t Skv);
 
 /*
  * Backward, three stream-ordered launches.  Replaces attn_backward (attn.cpp:30,

@@ -69,7 +69,7 @@ def test_fwd_from_the_mask(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kin
     assert torch.equal(torch.isinf(lse), empty) and bool((o[empty[..., 0]] == 0).all())
     assert (lse - lse_want)[~empty].abs().max().item() <= 1e-3 if bool((~empty).any()) else True
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
-    takes = _lib.load().fba_fwd_takes_mask(B * Hq * Sq, Skv, qbs, kbs)
+    takes = _lib.load().fba_fwd_takes_mask(B * Hq * Sq, Skv)
     assert takes == (Skv <= 1152)  # few rows: at most 120 slabs and a little more
     if takes:
         assert torch.equal(fba.flex_block_attn_func(q, k, v, qbs, kbs, m), o)
