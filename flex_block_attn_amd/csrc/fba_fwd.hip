@@ -852,7 +852,7 @@ hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
   p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
   // two work-groups per compute unit; a step is as long as one of fwd_kernel, a part's results are half as large
   const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / kHalfRows, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
-  p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
+  p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60, false}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kHalfSmem);

@@ -45,6 +45,7 @@ struct SplitPlan {
 // in a launch where few share one and where all do.
 struct StepCost {
   double alone, few, full;
+  bool most = true;  // may more than half a round be cut?
 };
 
 // Items and work-group slots of a launch -> plan (first = num_items, parts = 1 when nothing is split).  `slot_bytes` is

@@ -37,7 +37,8 @@ int device_compute_units() { return compute_units(); }
 // sustain (2.4 TB/s; taken a quarter dearer, since the parts of a launch end together).  slope is what a step takes times the rounds
 // the parts make, over their number.  A forward step takes 0.50 us in a work-group alone on its compute unit, 0.73 us where the
 // first share one and 0.95 us where all do (16, 22.5 and 30 units), so 72 items are better off in 3 parts than in 7: H24 384 rows
-// against 15360 keys, half kept, 63.6 -> 55.2 us.  On tile lists parts store half as much and a step is as long; dQ that recomputes S
+// against 15360 keys, half kept, 63.6 -> 55.2 us; whole items that fill every unit take up to 0.59 us a step (H2 S15360 all blocks, 240 items: 284 us whole,
+// 236 and a merge in two parts).  On tile lists parts store half as much and a step is as long; dQ that recomputes S
 // and dP is like forward, dQ from dS two products instead of six; a dK/dV slab takes 0.9 us with 128 keys (128 KiB a part) and
 // 0.6 us with 64 (64 KiB).
 //
@@ -49,10 +50,11 @@ int device_compute_units() { return compute_units(); }
 //
 // More than half a round is cut as well, in launches of less than two rounds, where work-groups end together: dK/dV of 136 tiles (H1
 // S17408), 40 and 90 % kept, backward 272 -> 255 and 540 -> 492 us, of 420 tiles (H3 S17920) 90 % kept 1612 -> 1424.  With items in falling
-// order of length the later rounds end at different times in any case: 680 tiles (H8 S10880) 40 % kept 579 -> 599.
+// order of length the later rounds end at different times in any case: 680 tiles (H8 S10880) 40 % kept 579 -> 599.  Nor on tile lists, where
+// a part scans its lists twice: H8/4 S13824, 64 x 384 blocks, 44 % kept, dK/dV 401 -> 456 us.
 constexpr double kMergeCost = 60;   // the launch
 constexpr int64_t kNoteBytes = 16;  // behind the parts' results
-constexpr int kFewItems = 100;
+constexpr int kFewItems = 128;
 SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
                      const ListLengths& lengths) {
   SplitPlan plan{};
@@ -62,12 +64,13 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   int slots = compute_units() * wgs_per_cu;
   if (slots > kSplitMaxSlots) slots = kSplitMaxSlots;
   const int rest = num_items % slots;
-  if (rest == 0 || (num_items >= 2 * slots && 2 * rest > slots)) return plan;
+  if (rest == 0 || (2 * rest > slots && (num_items >= 2 * slots || !step.most))) return plan;
   // cost(n) = slope(n) steps + parts and, where there are any, the launch that merges them.  From how long a list on is a number of
   // parts the cheapest: the slope falls from one candidate to the next, and one that is never the cheapest gives way.
   auto slope = [&](int n) {
     const int wgs = rest * n, alone = slots / wgs_per_cu;
-    if (num_items > slots) return step.full * ((wgs + slots - 1) / slots) / n;  // those of the whole rounds are still there
+    if (n == 1 && wgs <= alone && num_items >= 2 * slots) return step.few;  // items of the round before are still there
+    if (n == 1 && wgs <= alone) return step.alone * (1 + 0.15 * std::max(0, 2 * wgs - alone) / alone);  // a full chip runs at a lower clock
     if (wgs <= alone) return step.alone / n;
     if (wgs <= slots) return (step.few + (step.full - step.few) * (wgs - alone) / (slots - alone)) / n;
     return step.full * ((wgs + slots - 1) / slots) / n;
@@ -77,6 +80,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   for (int n = 2; n <= kMostParts && (int64_t)rest * n * slot_bytes + kNoteBytes <= ws_bytes; ++n) {
     if (num_items > slots && rest * n > slots && 2 * rest <= slots) break;  // a last round that fills up while others end gains nothing from another
     Candidate next{n, slope(n), (double)rest * n + kMergeCost, 0.};
+    if (wgs_per_cu == 1 && 2 * rest > slots && next.slope > 0.75 * slope(1)) continue;  // 0.8 of a round in five parts: H2 S29440 1055 -> 1095 us
     while (n_hull > 0 && next.slope < hull[n_hull - 1].slope) {
       next.least = (next.fixed - hull[n_hull - 1].fixed) / (hull[n_hull - 1].slope - next.slope);
       if (n_hull == 1 || next.least > hull[n_hull - 1].least) {
@@ -167,7 +171,7 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
   const int group = p.Hq / p.Hkv;
   const ListLengths lengths = p.tiled ? ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tile_rows, tile_rows, 128, p.Skv / 128, group, 1}
                                       : ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tile_rows, tile_rows, p.k_block, p.nK, group, p.q_block / 32};
-  p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{step_cost, step_cost, step_cost}, slot_bytes, ws, p.split_ws_bytes, lengths);
+  p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{step_cost, step_cost, step_cost, !p.tiled}, slot_bytes, ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(heads, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int parts = (p.num_items - p.split.first) * p.split.parts;
   p.queue = nullptr;
