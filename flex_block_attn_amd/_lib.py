@@ -52,6 +52,8 @@ SIGNATURES = {
     "fba_block_mean": (_c_i32, [_c_ptr, _c_ptr, _c_i64, _c_i32, _c_i32, _c_i32, _c_ptr]),
     "fba_ssta_mask": (_c_i32, [_c_ptr, _c_ptr, _c_ptr, _c_ptr] + [_c_i32] * 10 + [_c_ptr]),
     "fba_tile_permute": (_c_i32, [_c_ptr, _c_ptr, _c_i64] + [_c_i32] * 8 + [_c_ptr]),
+    "fba_tile_gather": (_c_i32, [_c_i32] + [_c_ptr] * 4 + [_c_i32] * 8 + [_c_ptr]),
+    "fba_ssta_mask_3d": (_c_i32, [_c_ptr] * 3 + [_c_i32] * 11 + [_c_ptr]),
     "fba_fwd_tiled": (_c_i32, [_c_ptr] * 7 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_bwd_tiled": (_c_i32, [_c_ptr] * 14 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_bwd_stats": (_c_i32, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_i32, _c_ptr]),

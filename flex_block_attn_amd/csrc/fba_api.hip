@@ -206,8 +206,28 @@ int32_t fba_ssta_mask(const float* q_mean, const float* k_mean, const uint8_t* b
   if (nK > 4096) return fail(FBA_ERR_UNSUPPORTED, "at most 4096 key blocks are ranked per query block (got %d)", nK);
   if ((int64_t)B * Hq > 65535) return fail(FBA_ERR_UNSUPPORTED, "B*Hq (%lld) must be at most 65535", (long long)B * Hq);
   hipError_t e = fba::launch_ssta_mask(q_mean, k_mean, base, mask, (int64_t)B * Hq, Hq, Hkv, nQ, nK, q_block, k_block, topk, band,
-                                       sink, (hipStream_t)hip_stream);
+                                       sink, fba::TileWindow{}, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "ssta_mask launch");
+}
+
+int32_t fba_ssta_mask_3d(const float* q_mean, const float* k_mean, uint8_t* mask, int32_t B, int32_t Hq, int32_t Hkv, int32_t nT, int32_t nH,
+                         int32_t nW, int32_t half_t, int32_t half_h, int32_t half_w, int32_t topk, int32_t sink, void* hip_stream) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || nT <= 0 || nH <= 0 || nW <= 0)
+    return fail(FBA_ERR_INVALID, "B, Hq, Hkv and the grid of tiles must be positive (got %d %d %d, %d x %d x %d)", B, Hq, Hkv, nT, nH, nW);
+  if (Hq % Hkv != 0) return fail(FBA_ERR_INVALID, "Hq (%d) must be a multiple of Hkv (%d)", Hq, Hkv);
+  if (topk < 0 || sink < 0) return fail(FBA_ERR_INVALID, "topk, sink must be >= 0 (got %d %d)", topk, sink);
+  if (!q_mean || !k_mean || !mask) return fail(FBA_ERR_INVALID, "null pointer argument");
+  const int64_t tiles = (int64_t)nT * nH * nW;
+  if (tiles > 4096) return fail(FBA_ERR_UNSUPPORTED, "at most 4096 key blocks are ranked per query block (got %lld)", (long long)tiles);
+  if ((int64_t)B * Hq > 65535) return fail(FBA_ERR_UNSUPPORTED, "B*Hq (%lld) must be at most 65535", (long long)B * Hq);
+  fba::TileWindow w{{nT, nH, nW}, {half_t, half_h, half_w}, {}, {}};
+  for (int x = 0; x < 3; ++x) {  // the window of a border tile is shifted inwards
+    w.low[x] = w.half[x] < w.n[x] - 1 ? w.half[x] : w.n[x] - 1;
+    w.high[x] = w.n[x] - 1 - w.half[x] > 0 ? w.n[x] - 1 - w.half[x] : 0;
+  }
+  hipError_t e = fba::launch_ssta_mask(q_mean, k_mean, nullptr, mask, (int64_t)B * Hq, Hq, Hkv, (int)tiles, (int)tiles, 1, 1, topk, -1, sink, w,
+                                       (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "ssta_mask (3-D) launch");
 }
 
 int32_t fba_tile_permute(const void* x, void* out, int64_t n_seq, int32_t T, int32_t H, int32_t W, int32_t tile_t,
@@ -222,6 +242,26 @@ int32_t fba_tile_permute(const void* x, void* out, int64_t n_seq, int32_t T, int
   if (int rc = check_ptrs({{"x", x}, {"out", out}})) return rc;
   hipError_t e = fba::launch_tile_permute(x, out, n_seq, T, H, W, tile_t, tile_h, tile_w, to_tiles ? 1 : 0, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "tile_permute launch");
+}
+
+int32_t fba_tile_gather(int32_t n, const void* const* x, void* const* out, float* const* mean, const int64_t* n_seq, int32_t T, int32_t H, int32_t W,
+                        int32_t tile_t, int32_t tile_h, int32_t tile_w, int32_t head_dim, int32_t to_tiles, void* hip_stream) {
+  if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);
+  if (n < 1 || n > 3) return fail(FBA_ERR_INVALID, "tile_gather takes one to three tensors (got %d)", n);
+  if (!x || !out || !mean || !n_seq) return fail(FBA_ERR_INVALID, "null pointer argument");
+  if (T <= 0 || H <= 0 || W <= 0 || tile_t <= 0 || tile_h <= 0 || tile_w <= 0) return fail(FBA_ERR_INVALID, "grid and tile extents must be positive");
+  if (T % tile_t != 0 || H % tile_h != 0 || W % tile_w != 0)
+    return fail(FBA_ERR_INVALID, "tile (%d, %d, %d) must divide the grid (%d, %d, %d)", tile_t, tile_h, tile_w, T, H, W);
+  if ((int64_t)T * H * W > 0x7fffffffLL) return fail(FBA_ERR_INVALID, "grid too large");
+  const int64_t tile_rows = (int64_t)tile_t * tile_h * tile_w;
+  for (int j = 0; j < n; ++j) {
+    if (int rc = check_ptrs({{"x", x[j]}, {"out", out[j]}})) return rc;
+    if (x[j] == out[j]) return fail(FBA_ERR_INVALID, "x and out must not alias");
+    if (n_seq[j] <= 0) return fail(FBA_ERR_INVALID, "n_seq must be positive");
+    if (to_tiles && mean[j] && tile_rows % 16 != 0) return fail(FBA_ERR_INVALID, "means need tiles of a multiple of 16 tokens (got %lld)", (long long)tile_rows);
+  }
+  hipError_t e = fba::launch_tile_gather(n, x, out, mean, n_seq, T, H, W, tile_t, tile_h, tile_w, to_tiles ? 1 : 0, (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "tile_gather launch");
 }
 
 int32_t fba_tile_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block,

@@ -171,9 +171,29 @@ hipError_t launch_mask_compact(const uint8_t* mask, int64_t mask_bh, int nQ, int
 hipError_t launch_tile_lists(const uint8_t* mask, int64_t mask_bh, int nQ, int nK, int q_block, int k_block, int n_qt,
                              int n_kt, int n_qs, int32_t* qt_cnt, int32_t* qt_ent, int32_t* kt_cnt, int32_t* kt_ent,
                              hipStream_t stream);
+// Sliding window over blocks that are the tiles of a (t, h, w) grid of `n` tiles, T-major: tile j is in the window of tile i when on every
+// axis it is at most `half` away from i's coordinate, which is first moved into [low, high] (shifted in at the borders).
+// n[0] = 0: no window.
+struct TileWindow {
+  int n[3], half[3], low[3], high[3];
+  __host__ __device__ bool holds(int i, int j) const {
+    const int a[3] = {i / (n[1] * n[2]), i / n[2] % n[1], i % n[2]}, b[3] = {j / (n[1] * n[2]), j / n[2] % n[1], j % n[2]};
+    bool in = true;
+    for (int x = 0; x < 3; ++x) {
+      int c = a[x] < low[x] ? low[x] : a[x];
+      c = c > high[x] ? high[x] : c;
+      const int d = c > b[x] ? c - b[x] : b[x] - c;
+      in = in && d <= half[x];
+    }
+    return in;
+  }
+};
+
 hipError_t launch_block_mean(const __bf16* x, float* out, int64_t n_blocks, int block, hipStream_t stream);
 hipError_t launch_ssta_mask(const float* q_mean, const float* k_mean, const uint8_t* base, uint8_t* mask, int64_t BH, int Hq, int Hkv, int nQ,
-                            int nK, int q_block, int k_block, int topk, int band, int sink, hipStream_t stream);
+                            int nK, int q_block, int k_block, int topk, int band, int sink, const TileWindow& window, hipStream_t stream);
+hipError_t launch_tile_gather(int n, const void* const* x, void* const* out, float* const* mean, const int64_t* n_seq, int T, int H, int W, int tT,
+                              int tH, int tW, int to_tiles, hipStream_t stream);
 hipError_t launch_tile_permute(const void* x, void* out, int64_t n_seq, int T, int H, int W, int tT, int tH, int tW,
                                int to_tiles, hipStream_t stream);
 hipError_t launch_resize_rows(int n, const void* const* src, void* const* dst, const int64_t* n_seq, const int32_t* src_len, const int32_t* dst_len,

@@ -57,12 +57,13 @@ constexpr int kChunksSmall = 16;   // nK <= 1024: 32 score registers per lane
 constexpr int kChunksLarge = 64;   // nK <= 4096: 128 score registers per lane
 
 // mask[bh, i, j] = (j among the topk largest <q_mean[bh,i], k_mean[kv(bh),j]>, ties to the lower j)
-//                  || |j - (i*q_block)/k_block| <= band || j < sink || base[i, j]   (base: optional [nQ, nK] mask).
+//                  || |j - (i*q_block)/k_block| <= band || j < sink || base[i, j]   (base: optional [nQ, nK] mask)
+//                  || j in the sliding window of i (window: optional, blocks as tiles of a 3-D grid, see TileWindow).
 // A wave ranks two query blocks; lane l holds the scores of key blocks l, l+64, ... (kMaxChunks of them) in registers.
 template <int kMaxChunks>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void ssta_mask_kernel(
     const float* __restrict__ q_mean, const float* __restrict__ k_mean, const uint8_t* __restrict__ base,
-    uint8_t* __restrict__ mask, int Hq, int Hkv, int nQ, int nK, int q_block, int k_block, int topk, int band, int sink) {
+    uint8_t* __restrict__ mask, int Hq, int Hkv, int nQ, int nK, int q_block, int k_block, int topk, int band, int sink, const TileWindow window) {
   __shared__ float k_lds[kChunk * kRowStride];
   __shared__ float q_lds[kQPerGroup * kD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -136,10 +137,78 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void ssta_mask
       const int j = t * kChunk + lane;
       if (j < nK) {
         const int dist = j > diag ? j - diag : diag - j;
-        const uint32_t keep = base ? (base[(size_t)i * nK + j] != 0) : 0u;
+        const uint32_t keep = base ? (base[(size_t)i * nK + j] != 0) : window.n[0] > 0 ? window.holds(i, j) : 0u;
         row[j] = (uint8_t)((uint32_t)((sel >> t) & 1u) | (dist <= band) | (j < sink) | keep);
       }
     }
+  }
+}
+
+// Token rows of up to three tensors between raster and tile order (see tile_permute_kernel), a work-group per tile, and on the way to
+// tiles the mean of every tile's rows, in the order in which block_mean_kernel adds them up.  Where a row lies in the grid is worked
+// out once per row of a tile and kept in LDS.  Bound by memory like the single steps, which read q and k a second time for their
+// means and are a launch each: q, k, v and two means, H24 S69120 3 x 163 + 2 x 89 -> 488 us (5.2 TB/s).  With the window worked out in
+// ssta_mask_kernel instead of on the host, H1 S1536 162 -> 64 us a call, H3 S15360 340 -> 287, H24 S69120 13.38 -> 13.15 ms.
+constexpr int kMostTileRows = 2048;
+struct GatherJobs {
+  const uint4* src[3];
+  uint4* dst[3];
+  float* mean[3];      // null: not wanted
+  unsigned first[3];   // first block of each tensor
+};
+template <bool kToTiles>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void tile_gather_kernel(const GatherJobs jobs, int T, int H, int W, int tT, int tH, int tW,
+                                                                                          float inv_rows) {
+  __shared__ int offs[kMostTileRows];  // of a tile's rows from its first one, in raster order
+  __shared__ float red[16][kD + 4];
+  const int tid = threadIdx.x, c = tid & 15, r0 = tid >> 4;
+  const int j = blockIdx.x >= jobs.first[2] ? 2 : blockIdx.x >= jobs.first[1] ? 1 : 0;
+  const int tile_sz = tT * tH * tW, nH = H / tH, nW = W / tW;
+  const int64_t block = blockIdx.x - jobs.first[j];  // tiles of all sequences in tile order
+  const int tiles = T / tT * nH * nW;
+  const int64_t seq = block / tiles;
+  const int tile = (int)(block - seq * tiles);
+  const int bt = tile / (nH * nW), bh = (tile / nW) % nH, bw = tile % nW;
+  for (int in = tid; in < tile_sz; in += 256) {
+    const int it = in / (tH * tW), rest = in - it * (tH * tW), ih = rest / tW;
+    offs[in] = (it * H + ih) * W + rest - ih * tW;
+  }
+  __syncthreads();
+  const int64_t raster0 = (seq * T * H * W + ((int64_t)bt * tT * H + bh * tH) * W + bw * tW) * 16 + c, tile0 = block * tile_sz * 16 + c;
+  const uint4* const src = jobs.src[j] + (kToTiles ? raster0 : tile0);
+  uint4* const dst = jobs.dst[j] + (kToTiles ? tile0 : raster0);
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  auto add = [&](const uint4& u) {
+    acc[0] += bf16_lo(u.x); acc[1] += bf16_hi(u.x); acc[2] += bf16_lo(u.y); acc[3] += bf16_hi(u.y);
+    acc[4] += bf16_lo(u.z); acc[5] += bf16_hi(u.z); acc[6] += bf16_lo(u.w); acc[7] += bf16_hi(u.w);
+  };
+  auto at = [&](int r, bool raster) { return (int64_t)(raster ? offs[r] : r) * 16; };
+  int r = r0;
+  for (; r + 48 < tile_sz; r += 64) {
+    uint4 u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = src[at(r + 16 * i, kToTiles)];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dst[at(r + 16 * i, !kToTiles)] = u[i];
+    if constexpr (kToTiles) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) add(u[i]);
+    }
+  }
+  for (; r < tile_sz; r += 16) {
+    const uint4 u = src[at(r, kToTiles)];
+    dst[at(r, !kToTiles)] = u;
+    if constexpr (kToTiles) add(u);
+  }
+  if (!kToTiles || jobs.mean[j] == nullptr) return;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) red[r0][c * 8 + e] = acc[e];
+  __syncthreads();
+  if (tid < kD) {
+    float s = 0.f;
+#pragma unroll
+    for (int g = 0; g < 16; ++g) s += red[g][tid];
+    jobs.mean[j][block * kD + tid] = s * inv_rows;
   }
 }
 
@@ -239,12 +308,41 @@ hipError_t launch_block_mean(const __bf16* x, float* out, int64_t n_blocks, int 
 }
 
 hipError_t launch_ssta_mask(const float* q_mean, const float* k_mean, const uint8_t* base, uint8_t* mask, int64_t BH, int Hq, int Hkv, int nQ,
-                            int nK, int q_block, int k_block, int topk, int band, int sink, hipStream_t stream) {
+                            int nK, int q_block, int k_block, int topk, int band, int sink, const TileWindow& window, hipStream_t stream) {
   if (BH <= 0 || BH > 65535 || nK > kChunk * kChunksLarge) return hipErrorInvalidValue;
-  void (*fn)(const float*, const float*, const uint8_t*, uint8_t*, int, int, int, int, int, int, int, int, int) =
+  void (*fn)(const float*, const float*, const uint8_t*, uint8_t*, int, int, int, int, int, int, int, int, int, const TileWindow) =
       nK <= kChunk * kChunksSmall ? &ssta_mask_kernel<kChunksSmall> : &ssta_mask_kernel<kChunksLarge>;
   hipLaunchKernelGGL(fn, dim3((unsigned)((nQ + kQPerGroup - 1) / kQPerGroup), (unsigned)BH), dim3(256), 0,
-                     stream, q_mean, k_mean, base, mask, Hq, Hkv, nQ, nK, q_block, k_block, topk, band, sink);
+                     stream, q_mean, k_mean, base, mask, Hq, Hkv, nQ, nK, q_block, k_block, topk, band, sink, window);
+  return hipGetLastError();
+}
+
+hipError_t launch_tile_gather(int n, const void* const* x, void* const* out, float* const* mean, const int64_t* n_seq, int T, int H, int W, int tT,
+                              int tH, int tW, int to_tiles, hipStream_t stream) {
+  const int64_t tile_sz = (int64_t)tT * tH * tW, tiles = (int64_t)(T / tT) * (H / tH) * (W / tW);
+  // tiles of a few rows would leave most of a work-group idle, large ones do not fit the table
+  if (tile_sz < 64 || tile_sz > kMostTileRows) {
+    for (int j = 0; j < n; ++j) {
+      hipError_t e = launch_tile_permute(x[j], out[j], n_seq[j], T, H, W, tT, tH, tW, to_tiles, stream);
+      if (e == hipSuccess && to_tiles && mean[j] != nullptr) e = launch_block_mean((const __bf16*)out[j], mean[j], n_seq[j] * tiles, (int)tile_sz, stream);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  GatherJobs jobs{};
+  int64_t blocks = 0;
+  for (int j = 0; j < 3; ++j) {
+    jobs.first[j] = (unsigned)blocks;  // a tensor that is not there starts behind the grid's last block
+    if (j >= n) continue;
+    jobs.src[j] = static_cast<const uint4*>(x[j]);
+    jobs.dst[j] = static_cast<uint4*>(out[j]);
+    jobs.mean[j] = to_tiles ? mean[j] : nullptr;
+    blocks += n_seq[j] * tiles;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+  }
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(to_tiles ? tile_gather_kernel<true> : tile_gather_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, jobs, T, H, W, tT, tH, tW,
+                     1.0f / (float)tile_sz);
   return hipGetLastError();
 }
 

@@ -5,6 +5,8 @@ The reference names these (create_sta_3d_mask, create_ssta_3d_mask, create_moba_
 not released them (flex_block_attn/__init__.py:7-12, README.md:54-55); the definitions below are this package's own and
 are stated in include/fba.h.  The static sliding-tile mask is `masks.sta_3d_block_mask`.
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -93,6 +95,46 @@ class _TilePermute(torch.autograd.Function):
         return _permute(g.to(torch.bfloat16), grid, tile, not to_tiles), None, None, None
 
 
+def _gather(xs, grid, tile, to_tiles, means=()):
+    """`_permute` of up to three tensors on one device in one launch -> (permuted tensors, means of the tiles of those numbered
+    in `means`, (B, H, tiles, 128) fp32)."""
+    xs = [_check_seq(x, "x") for x in xs]
+    T, Hh, W = grid
+    for x in xs:
+        if T * Hh * W != x.shape[2]:
+            raise ValueError(f"grid {tuple(grid)} does not have seq_len ({x.shape[2]}) tokens")
+    outs = [torch.empty_like(x) for x in xs]
+    tiles = T * Hh * W // (tile[0] * tile[1] * tile[2])
+    mean = {j: torch.empty((*xs[j].shape[:2], tiles, HEAD_DIM), dtype=torch.float32, device=xs[j].device) for j in means}
+    n = len(xs)
+    pointers = ctypes.c_void_p * n
+    with torch.cuda.device(xs[0].device):
+        _lib.call("fba_tile_gather", n, pointers(*(x.data_ptr() for x in xs)), pointers(*(o.data_ptr() for o in outs)),
+                  pointers(*(mean[j].data_ptr() if j in mean else None for j in range(n))), (ctypes.c_int64 * n)(*(x.shape[0] * x.shape[1] for x in xs)),
+                  T, Hh, W, tile[0], tile[1], tile[2], HEAD_DIM, int(to_tiles), _stream())
+    return outs, [mean[j] for j in means]
+
+
+class _TilePermuteAll(torch.autograd.Function):
+    """q, k, v from raster to tile order in one launch, with the tile means of q and k (constants of the backward pass)."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, grid, tile):
+        ctx.args = (tuple(grid), tuple(tile))
+        outs, means = _gather((q, k, v), grid, tile, True, means=(0, 1))
+        ctx.mark_non_differentiable(*means)
+        return (*outs, *means)
+
+    @staticmethod
+    def backward(ctx, gq, gk, gv, *_):
+        wanted = [j for j in range(3) if ctx.needs_input_grad[j]]
+        outs, _ = _gather([(gq, gk, gv)[j].to(torch.bfloat16) for j in wanted], *ctx.args, False)
+        grads = [None] * 5
+        for j, g in zip(wanted, outs):
+            grads[j] = g
+        return tuple(grads)
+
+
 def tile_tokens(x, grid, tile=(6, 8, 8)):
     """(B, H, T*Hh*W, 128) in raster order of the latent grid -> tile order: the tokens of each `tile` become one
     contiguous block (384 tokens for 6x8x8), tiles in raster order of the tile grid."""
@@ -115,10 +157,23 @@ def create_sta_3d_mask(tiles, window, device=None, clamp=True):
 def create_ssta_3d_mask(q, k, grid, tile=(6, 8, 8), window=(3, 3, 3), topk=16, sink_blocks=1):
     """Sliding-tile window united with score-selected tiles, for q, k already in tile order: bool (B, H, n, n) with
     n = number of tiles."""
-    tiles = tuple(g // t for g, t in zip(grid, tile))
     block = tile[0] * tile[1] * tile[2]
-    base = create_sta_3d_mask(tiles, window, device=q.device)
-    return create_ssta_mask(q, k, block, block, topk=topk, band=-1, sink_blocks=sink_blocks, base_mask=base)
+    return _ssta_3d_mask_from_means(block_mean(q, block), block_mean(k, block), grid, tile, window, topk, sink_blocks)
+
+
+def _ssta_3d_mask_from_means(q_mean, k_mean, grid, tile, window, topk, sink_blocks):
+    """`ssta_mask_from_means` with the sliding window over the grid of tiles, which the kernel works out by itself."""
+    nT, nH, nW = (g // t for g, t in zip(grid, tile))
+    half = [w // 2 for w in window]
+    B, Hq, nQ, _ = q_mean.shape
+    Hkv, nK = k_mean.shape[1], k_mean.shape[2]
+    if nT * nH * nW != nQ or nQ != nK or q_mean.shape[0] != k_mean.shape[0] or q_mean.device != k_mean.device or min(half) < 0:
+        base = create_sta_3d_mask((nT, nH, nW), window, device=q_mean.device)  # reported there
+        return ssta_mask_from_means(q_mean, k_mean, 1, 1, topk, -1, sink_blocks, base)
+    mask = torch.empty((B, Hq, nQ, nK), dtype=torch.bool, device=q_mean.device)
+    with torch.cuda.device(q_mean.device):
+        _lib.call("fba_ssta_mask_3d", _ptr(q_mean), _ptr(k_mean), _ptr(mask), B, Hq, Hkv, nT, nH, nW, *half, topk, sink_blocks, _stream())
+    return mask
 
 
 def create_moba_3d_mask(q, k, grid, tile=(6, 8, 8), topk=16):
@@ -134,7 +189,12 @@ def ssta_3d_attention(q, k, v, grid, tile=(6, 8, 8), window=(3, 3, 3), topk=16, 
     from .interface import flex_block_attn_func
 
     block = tile[0] * tile[1] * tile[2]
-    qt, kt, vt = (tile_tokens(x, grid, tile) for x in (q, k, v))
-    with torch.no_grad():
-        mask = create_ssta_3d_mask(qt.detach(), kt.detach(), grid, tile, window, topk, sink_blocks)
+    if block > 0 and block % 16 == 0 and q.device == k.device == v.device:
+        qt, kt, vt, q_mean, k_mean = _TilePermuteAll.apply(q, k, v, grid, tile)
+        with torch.no_grad():
+            mask = _ssta_3d_mask_from_means(q_mean, k_mean, grid, tile, window, topk, sink_blocks)
+    else:
+        qt, kt, vt = (tile_tokens(x, grid, tile) for x in (q, k, v))
+        with torch.no_grad():
+            mask = create_ssta_3d_mask(qt.detach(), kt.detach(), grid, tile, window, topk, sink_blocks)
     return untile_tokens(flex_block_attn_func(qt, kt, vt, block, block, mask), grid, tile)

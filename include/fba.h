@@ -271,11 +271,20 @@ int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, cons
  * fba_tile_permute: moves 256-byte token rows of x [n_seq, T*H*W, 128] bf16 between raster order of the (T, H, W) grid
  *   and tile order (tiles of tile_t x tile_h x tile_w tokens, tiles in raster order of the tile grid, tokens in raster
  *   order inside a tile), so that one tile is one contiguous block of the attention; to_tiles = 0 is the inverse.
+ *
+ * fba_tile_gather: the same for up to three tensors x[j] [n_seq[j], T*H*W, 128] in one launch; with to_tiles also the means of the
+ *   tiles (what fba_block_mean gives for out[j], bit for bit) into mean[j] [n_seq[j], tiles, 128] fp32 where mean[j] is not null.
+ * fba_ssta_mask_3d: fba_ssta_mask for blocks that are the tiles of an nT x nH x nW grid, with the sliding window of half_* tiles to
+ *   either side (shifted inwards at the borders) in place of the band and of a base mask.
  */
 int32_t fba_block_mean(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, int32_t head_dim, void* hip_stream);
 int32_t fba_ssta_mask(const float* q_mean, const float* k_mean, const uint8_t* base, uint8_t* mask, int32_t B, int32_t Hq, int32_t Hkv, int32_t nQ,
                       int32_t nK, int32_t q_block, int32_t k_block, int32_t topk, int32_t band, int32_t sink,
                       void* hip_stream);
+int32_t fba_tile_gather(int32_t n, const void* const* x, void* const* out, float* const* mean, const int64_t* n_seq, int32_t T, int32_t H, int32_t W,
+                        int32_t tile_t, int32_t tile_h, int32_t tile_w, int32_t head_dim, int32_t to_tiles, void* hip_stream);
+int32_t fba_ssta_mask_3d(const float* q_mean, const float* k_mean, uint8_t* mask, int32_t B, int32_t Hq, int32_t Hkv, int32_t nT, int32_t nH,
+                         int32_t nW, int32_t half_t, int32_t half_h, int32_t half_w, int32_t topk, int32_t sink, void* hip_stream);
 int32_t fba_tile_permute(const void* x, void* out, int64_t n_seq, int32_t T, int32_t H, int32_t W, int32_t tile_t,
                          int32_t tile_h, int32_t tile_w, int32_t head_dim, int32_t to_tiles, void* hip_stream);
 
