@@ -408,8 +408,13 @@ struct Attention : torch::autograd::Function<Attention> {
     build_lists(*s, in.mask, /*backward=*/true, /*numbered=*/!s->dense);
     auto [o, lse] = takes_mask(s->p) ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask) : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
     ctx->save_for_backward({in.q, in.k, in.v, o, lse});
+    // The rows that were appended are cut off here and not behind this function, where autograd would give back gradients for them in
+    // two launches of its own, a fill and a copy (13 of 280 us at B2 H8/2 S3136).  What is handed out shares its version with
+    // the saved tensor, so that a change in place is noticed.
+    const bool cut = s->q_len != s->p.Sq;
+    const int64_t q_len = s->q_len;
     ctx->saved_data["s"] = c10::IValue::make_capsule(std::move(s));
-    return o;
+    return cut ? o.narrow(2, 0, q_len).detach() : o;
   }
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx, torch::autograd::variable_list grads) {
     const auto saved = ctx->get_saved_variables();
@@ -421,7 +426,11 @@ struct Attention : torch::autograd::Function<Attention> {
     const at::Tensor q = unpacked(s, "q", saved[0], q_shape, at::kBFloat16, false), k = unpacked(s, "k", saved[1], kv_shape, at::kBFloat16, false),
                      v = unpacked(s, "v", saved[2], kv_shape, at::kBFloat16, false), o = unpacked(s, "o", saved[3], q_shape, at::kBFloat16, true),
                      lse = unpacked(s, "lse", saved[4], lse_shape, at::kFloat, true);
-    const at::Tensor d_o = grads[0].to(at::kBFloat16).contiguous();
+    at::Tensor d_o = grads[0].to(at::kBFloat16).contiguous();
+    if (s.q_len != p.Sq) {
+      if ((reinterpret_cast<uintptr_t>(d_o.data_ptr()) & 15) != 0) d_o = d_o.clone();  // the copy moves 16 bytes at a time
+      d_o = resized({{d_o, p.Sq}})[0];
+    }
     std::vector<int64_t> bounds;
     if (!s.dense) {
       s.copied.synchronize();
@@ -480,9 +489,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   }
   s->limit = ds_limit(p, limit, factor);
   s->dense = dense_fits(p.dense_bytes(), s->limit);
-  const bool cut = q_len != p.Sq;
-  const at::Tensor o = Attention::apply(q, k, v, mask, std::move(s));
-  return cut ? o.narrow(2, 0, q_len) : o;
+  return Attention::apply(q, k, v, mask, std::move(s));
 }
 
 // The same for whatever a Python caller passes: nothing for objects that are no tensors, for tensor subclasses (their results are

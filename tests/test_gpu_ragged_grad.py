@@ -1,0 +1,34 @@
+"""Gradients of outputs whose rows were cut: whatever layout the incoming gradient has (strided, expanded, off the 16-byte grid, fp32 through
+a cast), the same bits as for a plain contiguous one; none at all for an output that enters nothing."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,qbs,kbs", [(1, 2, 1, 336, 448, 16, 64), (2, 1, 1, 192, 256, 64, 64)])
+def test_layouts_of_the_gradient(gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs):
+    import flex_block_attn_amd as fba
+
+    g = torch.Generator().manual_seed(Sq)
+    m = torch.ones((Sq // qbs, Skv // kbs), dtype=torch.bool, device=gpu)
+    q = torch.randn((B, Hq, Sq, 128), generator=g).to(torch.bfloat16).to(gpu).requires_grad_(True)
+    k, v = (torch.randn((B, Hkv, Skv, 128), generator=g).to(torch.bfloat16).to(gpu).requires_grad_(True) for _ in range(2))
+    do = torch.randn((B, Hq, Sq, 128), generator=g).to(torch.bfloat16).to(gpu)
+    print(f"ragged gradient B{B} Hq{Hq} Sq{Sq} q{qbs}", flush=True)
+
+    def grads(do):
+        return torch.autograd.grad(fba.flex_block_attn_func(q, k, v, qbs, kbs, m), (q, k, v), do)
+
+    want = grads(do)
+    off = torch.empty(do.numel() + 1, dtype=do.dtype, device=gpu)[1:].view(do.shape).copy_(do)
+    assert off.data_ptr() % 16 != 0
+    for other in (off, do.transpose(2, 3).contiguous().transpose(2, 3)):
+        assert all(torch.equal(a, b) for a, b in zip(grads(other), want))
+    ones = grads(torch.ones_like(do))
+    assert all(torch.equal(a, b) for a, b in zip(grads(torch.ones((), dtype=do.dtype, device=gpu).expand_as(do)), ones))
+    o = fba.flex_block_attn_func(q, k, v, qbs, kbs, m)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(o.float(), (q, k, v), do.float()), want))
+    other = torch.ones((), device=gpu, requires_grad=True)
+    o = fba.flex_block_attn_func(q, k, v, qbs, kbs, m)
+    assert torch.autograd.grad(other * 2, (q,), allow_unused=True)[0] is None and o.shape == q.shape
