@@ -52,7 +52,11 @@ int device_compute_units() { return compute_units(); }
 // S17408), 40 and 90 % kept, backward 272 -> 255 and 540 -> 492 us, of 420 tiles (H3 S17920) 90 % kept 1612 -> 1424.  With items in falling
 // order of length the later rounds end at different times in any case: 680 tiles (H8 S10880) 40 % kept 579 -> 599.  Nor on tile lists, where
 // a part scans its lists twice: H8/4 S13824, 64 x 384 blocks, 44 % kept, dK/dV 401 -> 456 us.
+//
+// A part on a tile list scans the whole list before it takes its own steps: H5 S1536, 16 x 64 blocks, a third kept, dK/dV of 120 half
+// tiles of 27 steps 25.4 us whole, 22.4 us and a merge of 5.0 in two parts.
 constexpr double kMergeCost = 60;   // the launch
+constexpr double kScanCost = 40;    // and, on tile lists, the scans
 constexpr int64_t kNoteBytes = 16;  // behind the parts' results
 constexpr int kFewItems = 128;
 SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
@@ -79,7 +83,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   int n_hull = 1;
   for (int n = 2; n <= kMostParts && (int64_t)rest * n * slot_bytes + kNoteBytes <= ws_bytes; ++n) {
     if (num_items > slots && rest * n > slots && 2 * rest <= slots) break;  // a last round that fills up while others end gains nothing from another
-    Candidate next{n, slope(n), (double)rest * n + kMergeCost, 0.};
+    Candidate next{n, slope(n), (double)rest * n + kMergeCost + (step.most ? 0 : kScanCost), 0.};
     if (wgs_per_cu == 1 && 2 * rest > slots && next.slope > 0.75 * slope(1)) continue;  // 0.8 of a round in five parts: H2 S29440 1055 -> 1095 us
     while (n_hull > 0 && next.slope < hull[n_hull - 1].slope) {
       next.least = (next.fixed - hull[n_hull - 1].fixed) / (hull[n_hull - 1].slope - next.slope);
@@ -90,7 +94,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
       --n_hull;
     }
   }
-  if (n_hull == 1 || hull[1].least > 0.5 * max_steps) return plan;  // lists of usual density stay whole
+  if (n_hull == 1 || hull[1].least > 0.6 * max_steps) return plan;  // lists of usual density stay whole
   const double longest = rest <= kFewItems ? 0.6 * max_steps : max_steps;
   while (hull[n_hull - 1].least > longest) --n_hull;
   for (int j = 0; j < kMostParts - 1; ++j) plan.least[j] = 0x7fffffff;
