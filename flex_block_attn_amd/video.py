@@ -6,6 +6,7 @@ not released them (flex_block_attn/__init__.py:7-12, README.md:54-55); the defin
 are stated in include/fba.h.  The static sliding-tile mask is `masks.sta_3d_block_mask`.
 """
 import ctypes
+import numbers
 
 import torch
 
@@ -164,12 +165,15 @@ def create_ssta_3d_mask(q, k, grid, tile=(6, 8, 8), window=(3, 3, 3), topk=16, s
 def _ssta_3d_mask_from_means(q_mean, k_mean, grid, tile, window, topk, sink_blocks):
     """`ssta_mask_from_means` with the sliding window over the grid of tiles, which the kernel works out by itself."""
     nT, nH, nW = (g // t for g, t in zip(grid, tile))
-    half = [w // 2 for w in window]
+    extents = tuple(window)
     B, Hq, nQ, _ = q_mean.shape
     Hkv, nK = k_mean.shape[1], k_mean.shape[2]
-    if nT * nH * nW != nQ or nQ != nK or q_mean.shape[0] != k_mean.shape[0] or q_mean.device != k_mean.device or min(half) < 0:
-        base = create_sta_3d_mask((nT, nH, nW), window, device=q_mean.device)  # reported there
+    # The kernel takes three extents that a 32-bit integer holds; anything else is worked out, or refused, where the mask is made of tensors.
+    plain = len(extents) == 3 and all(isinstance(w, numbers.Integral) and 0 <= w < 2**31 for w in extents)
+    if not plain or nT * nH * nW != nQ or nQ != nK or q_mean.shape[0] != k_mean.shape[0] or q_mean.device != k_mean.device:
+        base = create_sta_3d_mask((nT, nH, nW), extents, device=q_mean.device)
         return ssta_mask_from_means(q_mean, k_mean, 1, 1, topk, -1, sink_blocks, base)
+    half = [int(w) // 2 for w in extents]
     mask = torch.empty((B, Hq, nQ, nK), dtype=torch.bool, device=q_mean.device)
     with torch.cuda.device(q_mean.device):
         _lib.call("fba_ssta_mask_3d", _ptr(q_mean), _ptr(k_mean), _ptr(mask), B, Hq, Hkv, nT, nH, nW, *half, topk, sink_blocks, _stream())

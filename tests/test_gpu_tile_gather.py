@@ -53,3 +53,38 @@ def test_window_in_the_mask_kernel(gpu, tiles, window, topk, sink):
     assert torch.equal(got, want)
     if topk == 0 and sink == 0:
         assert torch.equal(got, base.expand_as(got))
+
+
+@pytest.mark.parametrize("window", [(3.0, 3.0, 3.0), (3.5, 1.2, 5.0), (2**33, 1, 2**33 + 4), (2**31, 3, 2**40), (2**31 - 1, 1, 1), (-1, 3, 3), (float("nan"), 3, 3),
+                                    torch.tensor([3, 1, 5]), torch.tensor([3.0, 1.0, 5.0])])
+def test_extents_that_are_no_small_whole_numbers(gpu, window):
+    """What the mask made of tensors takes, the operator takes, with the same result."""
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd import masks, video
+
+    tiles, tile = (2, 3, 4), (1, 4, 4)
+    grid = tuple(n * t for n, t in zip(tiles, tile))
+    S = grid[0] * grid[1] * grid[2]
+    g = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn((1, 2, S, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(3))
+    base = masks.sta_3d_block_mask(tiles, window).to(gpu)
+    want = fba.create_ssta_mask(q, k, 16, 16, topk=0, band=-1, sink_blocks=1, base_mask=base)
+    assert torch.equal(video.create_ssta_3d_mask(q, k, grid, tile, window, topk=0), want)
+    # the same through the whole operator (key blocks of 64 tokens and more)
+    tile = (1, 8, 8)
+    grid = tuple(n * t for n, t in zip(tiles, tile))
+    q, k, v = (torch.randn((1, 2, grid[0] * grid[1] * grid[2], 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(3))
+    qt, kt, vt = (fba.tile_tokens(x, grid, tile) for x in (q, k, v))
+    o = fba.flex_block_attn_func(qt, kt, vt, 64, 64, fba.create_ssta_mask(qt, kt, 64, 64, topk=1, band=-1, sink_blocks=0, base_mask=base))
+    assert torch.equal(video.ssta_3d_attention(q, k, v, grid, tile, window, topk=1, sink_blocks=0), fba.untile_tokens(o, grid, tile))
+
+
+@pytest.mark.parametrize("window", [(3, 3), (3, 3, 3, 3), None, ("3", "3", "3"), torch.tensor([3, 3, 3])])
+def test_refused_extents(gpu, window):
+    from flex_block_attn_amd import video
+
+    q = torch.randn((1, 1, 2 * 16 * 16, 128), device=gpu).to(torch.bfloat16)
+    if isinstance(window, torch.Tensor):
+        window = window.to(gpu)
+    with pytest.raises((ValueError, TypeError, RuntimeError)):
+        video.create_ssta_3d_mask(q, q, (2, 16, 16), (1, 8, 8), window)
