@@ -285,6 +285,50 @@ static int fill_bwd(fba::BwdParams& p, const Shape& s) {
   return FBA_OK;
 }
 
+int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
+                       int32_t k_block, int64_t split_ws_bytes, int64_t* plan) {
+  const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
+  if (int rc = check_shape(s)) return rc;
+  if (plan == nullptr || split_ws_bytes < 0) return fail(FBA_ERR_INVALID, "null plan or negative split_ws_bytes");
+  const bool tiled = q_block % 128 != 0 || k_block % 128 != 0;
+  if (int rc = check_lists(s, tiled, "split_plan")) return rc;
+  // addresses that are only compared with null and subtracted from each other
+  float* const ws = split_ws_bytes > 0 ? reinterpret_cast<float*>(16) : nullptr;
+  const int32_t* const cnt = reinterpret_cast<const int32_t*>(16);
+  fba::BwdParams b{};
+  fill_bwd(b, s);
+  b.tiled = tiled ? 1 : 0;
+  b.q_cnt = b.k_cnt = cnt;
+  b.split.ws = ws; b.split_ws_bytes = split_ws_bytes;
+  switch (launch) {
+    case 0: {
+      fba::FwdParams f{};
+      f.mask_bh = mask_bh;
+      f.B = B; f.Hq = Hq; f.Hkv = Hkv; f.Sq = Sq; f.Skv = Skv; f.nQ = b.nQ; f.nK = b.nK;
+      f.q_block = q_block; f.k_block = k_block;
+      f.q_cnt = cnt; f.tiled = b.tiled; f.variant = 1;
+      f.split = b.split; f.split_ws_bytes = split_ws_bytes;
+      fba::plan_fwd(f);
+      b.num_items = f.num_items;
+      b.split = f.split;
+      break;
+    }
+    case 1: fba::plan_bwd_dkdv(b, tiled ? fba::kKeyTiles64 : fba::kKeyTiles128); break;
+    case 2: fba::plan_bwd_dq(b); break;
+    case 3: fba::plan_bwd_dq_from_ds(b); break;
+    default: return fail(FBA_ERR_INVALID, "launch must be 0 to 3, got %d", launch);
+  }
+  const fba::SplitPlan& sp = b.split;
+  const bool split = sp.first < b.num_items;
+  plan[0] = b.num_items;
+  plan[1] = sp.first;
+  plan[2] = sp.parts;
+  plan[3] = split && sp.lengths.cnt != nullptr;
+  plan[4] = split ? reinterpret_cast<const char*>(sp.note) - reinterpret_cast<const char*>(ws) : 0;
+  for (int j = 0; j < fba::kMostParts - 1; ++j) plan[5 + j] = split ? sp.least[j] : 0x7fffffff;
+  return FBA_OK;
+}
+
 int32_t fba_bwd_stats(const void* o, const void* d_o, const float* lse, float* stats, int64_t rows, int32_t head_dim,
                       void* hip_stream) {
   if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);

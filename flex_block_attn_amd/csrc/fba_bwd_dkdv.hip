@@ -382,7 +382,7 @@ hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
   if (e != hipSuccess) return e;
   int grid;
-  if ((e = plan_key_tiles(p, 128, 14, 2 * 128 * kHeadDim * 4, grid, stream)) != hipSuccess) return e;
+  if ((e = plan_key_tiles(p, kKeyTiles128, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes + 16, stream, p);
   const int split_items = p.num_items - p.split.first;
   if (split_items > 0) {

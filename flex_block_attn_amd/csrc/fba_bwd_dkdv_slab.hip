@@ -43,6 +43,7 @@ constexpr int kCountBase = kListBase + kChapter * 8;  // two sets of eight count
 constexpr int kClaimBase = kCountBase + 64;
 constexpr int kSmemBytes = kClaimBase + 16;
 constexpr int kSlotFloats = 2 * kTK * kHeadDim;     // partial result of one part of a split item: dV rows, then dK rows
+static_assert(kKeyTiles64.rows == kTK && kKeyTiles64.slot_bytes == kSlotFloats * 4);
 
 template <int N>
 using IC = std::integral_constant<int, N>;
@@ -398,7 +399,7 @@ hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes);
   if (e != hipSuccess) return e;
   int grid;
-  if ((e = plan_key_tiles(p, kTK, 22, kSlotFloats * 4, grid, stream)) != hipSuccess) return e;
+  if ((e = plan_key_tiles(p, kKeyTiles64, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes, stream, p);
   const int split_items = p.num_items - p.split.first;
   if (split_items > 0) {

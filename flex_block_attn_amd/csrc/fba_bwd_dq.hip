@@ -238,12 +238,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     }
 }
 
-hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {
-  constexpr int kSmem = kRing * kPairBytes;
+// Tail splitting on block lists (two work-groups per compute unit); a part stores a 128 x 128 fp32 tile.
+void plan_bwd_dq(BwdParams& p) {
   p.num_items = p.B * p.Hq * (p.Sq / 128);
-  // tail splitting on block lists (two work-groups per compute unit); a part stores a 128 x 128 fp32 tile
   const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / 128, 128, p.q_block, p.nQ, 1, p.k_block / 32};
   p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, 128 * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
+}
+
+hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {
+  constexpr int kSmem = kRing * kPairBytes;
+  plan_bwd_dq(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   void (*fn)(const BwdParams) = p.tiled ? &dq_kernel<true> : &dq_kernel<false>;

@@ -305,15 +305,27 @@ hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int r
   return hipGetLastError();
 }
 
+// Tail splitting on block lists (two work-groups of four waves per compute unit, one of more); a part stores a tile of fp32 sums.
+//
+// Wide work-groups where the query blocks allow them and the launch has two rounds of them: smaller launches fill the chip
+// better with 128 rows.  Backward, 128 rows everywhere / wide, 40 % kept: H24 S30720, 384-token blocks 12.49 -> 12.31 ms (dQ
+// 3.36 -> 3.18 ms), 256-token blocks 12.49 -> 12.25 ms; H24 S115200 sliding window, step 51.5 -> 50.9 ms.
+int plan_bwd_dq_from_ds(BwdParams& p) {
+  const int64_t rows = (int64_t)p.B * p.Hq * p.Sq, enough = 2LL * device_compute_units();  // work-groups
+  const int waves = p.tiled ? 4 : p.q_block % 384 == 0 && rows / 384 >= enough ? 12 : p.q_block % 256 == 0 && rows / 256 >= enough ? 8 : 4;
+  const int tile = 32 * waves;
+  p.num_items = p.B * p.Hq * (p.Sq / tile);
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / tile, tile, p.q_block, p.nQ, 1, p.k_block / kSlab};
+  p.split = plan_split(p.num_items, waves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18}, (int64_t)tile * kHeadDim * 4, p.tiled ? nullptr : p.split.ws,
+                       p.split_ws_bytes, lengths);
+  return waves;
+}
+
 namespace {
 
 template <int kWaves>
 hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
   constexpr int kRows = 32 * kWaves, kSmem = kRing * stage_bytes(kWaves);
-  p.num_items = p.B * p.Hq * (p.Sq / kRows);
-  // tail splitting on block lists (two work-groups of four waves per compute unit, one of more); a part stores a tile of fp32 sums
-  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / kRows, kRows, p.q_block, p.nQ, 1, p.k_block / kSlab};
-  p.split = plan_split(p.num_items, kWaves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18}, kRows * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   const bool dense = p.pair_base == nullptr;
@@ -340,13 +352,8 @@ hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
 
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
   if (p.ds_ws == nullptr) return hipErrorInvalidValue;
-  // Wide work-groups where the query blocks allow them and the launch has two rounds of them: smaller launches fill the chip
-  // better with 128 rows.  Backward, 128 rows everywhere / wide, 40 % kept: H24 S30720, 384-token blocks 12.49 -> 12.31 ms (dQ
-  // 3.36 -> 3.18 ms), 256-token blocks 12.49 -> 12.25 ms; H24 S115200 sliding window, step 51.5 -> 50.9 ms.
-  const int64_t rows = (int64_t)p.B * p.Hq * p.Sq, enough = 2LL * device_compute_units();  // work-groups
-  if (!p.tiled && p.q_block % 384 == 0 && rows / 384 >= enough) return launch_dq_rows<12>(p, stream);
-  if (!p.tiled && p.q_block % 256 == 0 && rows / 256 >= enough) return launch_dq_rows<8>(p, stream);
-  return launch_dq_rows<4>(p, stream);
+  const int waves = plan_bwd_dq_from_ds(p);
+  return waves == 12 ? launch_dq_rows<12>(p, stream) : waves == 8 ? launch_dq_rows<8>(p, stream) : launch_dq_rows<4>(p, stream);
 }
 
 }  // namespace fba

@@ -130,12 +130,14 @@ FBA_DEVICE int wave_sum(int x) {
 }
 
 // How many parts every split item of a launch is cut into (see SplitPlan in fba_kernels.h): by the mean length of the lists of 64 of
-// them, which every wave finds alike.  All lanes of a wave call this together.
+// them, which every wave finds alike.  `order`: the item of every grid index (long lists first, so the split ones are the shortest of the
+// launch), null where they are the same.  All lanes of a wave call this together.
 template <typename Plan>
-FBA_DEVICE int split_parts(const Plan& plan) {
+FBA_DEVICE int split_parts(const Plan& plan, const int32_t* order) {
   const auto& l = plan.lengths;
   if (l.cnt == nullptr) return plan.parts;
-  const int item = plan.first + (int)((threadIdx.x & 63) * (int64_t)plan.items / 64);
+  const int index = plan.first + (int)((threadIdx.x & 63) * (int64_t)plan.items / 64);
+  const int item = order != nullptr ? order[index] : index;
   const int head = item / l.tiles, row = (item - head * l.tiles) * l.tile_rows / l.list_rows;
   int n[4];  // of up to four heads of the group, in flight together
 #pragma unroll
@@ -152,7 +154,7 @@ FBA_DEVICE int split_parts(const Plan& plan) {
 // does all ranges: forward, H3 2304 rows against 61440 keys 120 -> 140 us.)  False: the launch has more work-groups than parts.
 template <typename Plan>
 FBA_DEVICE bool split_position(const Plan& plan, const int32_t* order, int s, int& item, int& part, int& parts) {
-  parts = split_parts(plan);
+  parts = split_parts(plan, order);
   if (s == 0 && threadIdx.x == 0 && plan.lengths.cnt != nullptr) *plan.note = parts;
   const int i = s / parts;
   if (i >= plan.items) return false;

@@ -845,14 +845,26 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge
   }
 }
 
+// Tail splitting (two work-groups per compute unit); the 384-row kernel does without.
+void plan_fwd(FwdParams& p) {
+  if (p.tiled) {  // a step is as long as one of fwd_kernel, a part's results are half as large
+    p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
+    const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / kHalfRows, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
+    p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60, false}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
+    return;
+  }
+  const bool wide = p.q_block % 384 == 0 && p.variant != 1;
+  const int rows = wide ? 384 : 128;
+  p.num_items = p.B * p.Hq * (p.Sq / rows);
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / rows, rows, p.q_block, p.nQ, 1, p.k_block / kSlab};
+  p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
+}
+
 namespace {
 
 hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
   void (*fn)(const FwdParams) = p.q_block % 64 != 0 ? &fwd_half_kernel<true> : &fwd_half_kernel<false>;
-  p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
-  // two work-groups per compute unit; a step is as long as one of fwd_kernel, a part's results are half as large
-  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / kHalfRows, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
-  p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60, false}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
+  plan_fwd(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kHalfSmem);
@@ -891,10 +903,7 @@ hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   const bool wide = p.q_block % 384 == 0 && p.variant != 1;
   void (*fn)(const FwdParams) = wide ? &fwd_kernel<12> : &fwd_kernel<4>;
   const int rows = wide ? 384 : 128;
-  p.num_items = p.B * p.Hq * (p.Sq / rows);
-  // tail splitting for the 128-row kernels (two work-groups per compute unit)
-  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / rows, rows, p.q_block, p.nQ, 1, p.k_block / kSlab};
-  p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
+  plan_fwd(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_wgs = (p.num_items - p.split.first) * p.split.parts;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);

@@ -54,6 +54,22 @@ struct StepCost {
 SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
                      const ListLengths& lengths);
 
+// The plans of the launches below, from the sizes, q_cnt / k_cnt, split.ws and split_ws_bytes of their parameters: num_items and split are set.
+struct FwdParams;
+struct BwdParams;
+void plan_fwd(FwdParams& p);
+void plan_bwd_dq(BwdParams& p);
+int plan_bwd_dq_from_ds(BwdParams& p);  // waves of a work-group
+// dK/dV: key rows of an item, its step's cost (see StepCost), bytes that a part stores (dV, then dK)
+struct KeyTiles {
+  int rows;
+  double step;
+  int64_t slot_bytes;
+};
+constexpr KeyTiles kKeyTiles128{128, 14, 2 * 128 * 128 * 4};  // block lists: dkdv64_kernel, dkdv_kernel
+constexpr KeyTiles kKeyTiles64{64, 22, 2 * 64 * 128 * 4};     // tile lists: dkdv_slab_kernel
+void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles);
+
 // Work-groups of a launch that merges parts: each does every so many of the blocks of eight rows, so that little is launched where
 // the lists turn out too short for parts.
 inline int merge_grid(int blocks) { return blocks < 2048 ? blocks : 2048; }
@@ -210,7 +226,7 @@ hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream);  // tile lists
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream);
 // Shape of a dK/dV launch over key tiles of `tile_rows` rows, whose parts store `slot_bytes` each: sets p.num_items, split,
 // items_per_xcd, order, queue and total_work and the number of work-groups, and launches what has to run in front.
-hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t slot_bytes, int& grid, hipStream_t stream);
+hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream);
 int device_compute_units();
 // One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats).
 struct PartialOut {

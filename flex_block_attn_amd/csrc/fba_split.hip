@@ -167,15 +167,21 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void order_ite
 
 }  // namespace
 
-hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t slot_bytes, int& grid, hipStream_t stream) {
-  const int slots = compute_units();  // one work-group per compute unit
+// One work-group per compute unit.
+void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles) {
+  p.num_items = p.B * p.Hkv * (p.Skv / tiles.rows);
+  const int group = p.Hq / p.Hkv;
+  const ListLengths lengths = p.tiled ? ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tiles.rows, tiles.rows, 128, p.Skv / 128, group, 1}
+                                      : ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tiles.rows, tiles.rows, p.k_block, p.nK, group, p.q_block / 32};
+  p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{tiles.step, tiles.step, tiles.step, !p.tiled}, tiles.slot_bytes, p.split.ws, p.split_ws_bytes,
+                       lengths);
+}
+
+hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream) {
+  const int slots = compute_units();
   const int heads = p.B * p.Hkv;
   char* const ws = reinterpret_cast<char*>(p.split.ws);  // whether or not anything is split
-  p.num_items = heads * (p.Skv / tile_rows);
-  const int group = p.Hq / p.Hkv;
-  const ListLengths lengths = p.tiled ? ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tile_rows, tile_rows, 128, p.Skv / 128, group, 1}
-                                      : ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tile_rows, tile_rows, p.k_block, p.nK, group, p.q_block / 32};
-  p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{step_cost, step_cost, step_cost, !p.tiled}, slot_bytes, ws, p.split_ws_bytes, lengths);
+  plan_bwd_dkdv(p, tiles);
   plan_xcd_mapping(heads, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int parts = (p.num_items - p.split.first) * p.split.parts;
   p.queue = nullptr;
@@ -183,7 +189,7 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
 
   // What else lives in the workspace, from its end: the claim counters, then the order of the items.
   int64_t top = ws == nullptr ? 0 : (p.split_ws_bytes - kQueueBytes) & ~(int64_t)15;
-  const int64_t bottom = parts * slot_bytes + kNoteBytes;
+  const int64_t bottom = parts * tiles.slot_bytes + kNoteBytes;
   int* const queue = ws != nullptr && top >= bottom ? reinterpret_cast<int*>(ws + top) : nullptr;
   top = (top - (int64_t)p.num_items * 4) & ~(int64_t)15;
   // Items are ordered where they start in more than one round and in at most eight.  One round starts everything at once; over
@@ -214,7 +220,7 @@ hipError_t plan_key_tiles(BwdParams& p, int tile_rows, double step_cost, int64_t
   }
   if (ordered) {
     const int spans = heads >= 8 ? 8 : 1;
-    const int tiles_per_head = p.Skv / tile_rows, two_rounds = 2 * slots / spans;
+    const int tiles_per_head = p.Skv / tiles.rows, two_rounds = 2 * slots / spans;
     const int segment = (two_rounds + tiles_per_head - 1) / tiles_per_head * tiles_per_head;
     const int blocks = spans * (((p.num_items + spans - 1) / spans + kRankItems - 1) / kRankItems);
     int32_t* const order = reinterpret_cast<int32_t*>(ws + top);

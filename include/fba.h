@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2005
+#define FBA_VERSION 2006
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -59,8 +59,10 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  * Tail splitting (no counterpart in the reference).  Work-groups are handed to free compute-unit slots in index order,
  * so the last (items % slots) 128-row tiles of a launch would run as a partial round with most of the GPU idle; the same
  * holds for a whole launch with fewer tiles than slots.  Entry points that take `split_ws` cut the lists of those tiles
- * into up to eight ranges (how many is decided by the lengths of the lists, on the device), run each range in a work-group of its own at the end of the grid, store fp32 partial results
- * into split_ws and combine them in a small second launch, in a fixed order (results stay bit-reproducible).
+ * into up to eight ranges, run each range in a work-group of its own at the end of the grid, store fp32 partial results
+ * into split_ws and combine them in a small second launch, in a fixed order (results stay bit-reproducible).  How many ranges: the
+ * device decides by the lengths of the lists where more than 128 tiles are left over; up to 128 the host decides, for lists that hold
+ * 60 % of the longest possible ones.
  *   split_ws        null (nothing is split), or 16-byte aligned device memory owned by the caller for the duration of
  *                   the call's work on the stream; its contents before and after are meaningless
  *   split_ws_bytes  its size; fba_split_workspace_bytes() is what the planner can use at most (a smaller buffer limits
@@ -75,6 +77,16 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  * idling.  Which work-group computes a tile does not enter the result.
  */
 int64_t fba_split_workspace_bytes(void);
+/*
+ * What a launch on such sizes would cut, for tests and measurements (no GPU needed: 256 compute units are assumed then).  launch: 0 forward, 1 dK/dV,
+ * 2 dQ that recomputes S and dP, 3 dQ from dS; the lists are those the block sizes need.  plan [12]:
+ *   0 tiles of the launch   1 first tile that is cut (that many: none)   2 most ranges of a tile's list
+ *   3 1 where the device decides how many, up to that, by the mean length of the lists, 0 where it is that many whatever the lists
+ *   4 offset in split_ws of the int32 in which the device leaves its decision   5.. list steps from which on 2, 3, ... 8 ranges are made
+ * A step is 32 keys (forward, dQ; 64 in forward on tile lists) or 32 query rows of one query head (dK/dV).
+ */
+int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim,
+                       int32_t q_block, int32_t k_block, int64_t split_ws_bytes, int64_t* plan);
 
 /*
  * Forward.  Replaces attn_forward (attn.cpp:29, flex_block_attn_h100.cu:810-1007; kernel :52-318).

@@ -1,0 +1,128 @@
+"""How many parts the device makes, read from the note it leaves in the workspace: by the mean length of the lists that are really cut, which in
+launches with ordered tiles are the shortest.  Lists that differ along the sequence and from head to head, grouped heads, a shared mask, block and
+tile lists; lengths well off the lines of the plan, so that no choice of sample decides.  Launches cut in parts agree with whole ones to the
+rounding of bf16 results (fp32 sums in another order), bit for bit where one part is made."""
+import ctypes
+
+import pytest
+import torch
+
+FWD, DKDV, DQ = 0, 1, 2
+HEAD = 128
+
+
+def plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, ws_bytes=None):
+    from flex_block_attn_amd import _lib
+
+    out = (ctypes.c_int64 * 12)()
+    n = _lib.load().fba_split_workspace_bytes() if ws_bytes is None else ws_bytes
+    _lib.call("fba_split_plan", launch, 1 if dims == 2 else B * Hq, B, Hq, Hkv, Sq, Skv, HEAD, qbs, kbs, n, out)
+    return dict(zip(("items", "first", "parts", "device", "note"), out), least=list(out)[5:])
+
+
+def mask_of(kind, B, Hq, Sq, Skv, qbs, kbs, dims, g):
+    nQ, nK = Sq // qbs, Skv // kbs
+    m = torch.rand((B, Hq, nQ, nK) if dims == 4 else (nQ, nK), generator=g)
+    if kind == "causal":
+        at = torch.arange(nQ)[:, None] / nQ >= torch.arange(nK)[None, :] / nK
+        return at.expand(m.shape).contiguous()
+    if kind == "last head":  # dense in the last head, sparse in the others
+        return m < torch.where(torch.arange(Hq) == Hq - 1, 0.9, 0.05)[None, :, None, None]
+    return m < kind
+
+
+def steps(launch, m, B, Hq, Hkv, Sq, Skv, qbs, kbs):
+    """List length of every tile of the launch, in steps (fine masks: 128-row tiles list what some of their rows select)."""
+    m = m.expand(B, Hq, *m.shape[-2:])
+    tiled = qbs % 128 or kbs % 128
+    if launch == DKDV:
+        per_key = m.sum(2) * (qbs // 32)  # [B, Hq, nK]
+        per_key = per_key.view(B, Hkv, Hq // Hkv, -1).sum(2)
+        return per_key.repeat_interleave(kbs // 128, -1).flatten()
+    if tiled:
+        union = m.repeat_interleave(qbs, 2).view(B, Hq, Sq // 128, 128, -1).any(3).sum(-1) * (kbs // 64)
+        return union.repeat_interleave(2, -1).flatten()  # two 64-row halves read one list
+    return (m.sum(-1) * (kbs // 32)).repeat_interleave(qbs // 128, -1).flatten()
+
+
+CASES = [
+    # launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, mask, tiles taken in order of length
+    (DKDV, 1, 3, 3, 8192, 17920, 256, 128, 4, "causal", True),
+    (DKDV, 1, 3, 3, 8192, 17920, 256, 128, 4, "last head", True),
+    (DKDV, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.9, True),
+    (DKDV, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.2, True),
+    (DKDV, 1, 1, 1, 8192, 17408, 128, 128, 2, "causal", False),
+    (DKDV, 1, 1, 1, 8192, 17408, 128, 128, 2, 0.1, False),
+    (DKDV, 1, 8, 1, 2048, 17408, 128, 128, 4, 0.5, False),       # lists over eight heads
+    (DKDV, 1, 8, 1, 2048, 17408, 128, 128, 4, "last head", False),
+    (FWD, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.1, False),
+    (FWD, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.5, False),
+    (FWD, 1, 5, 5, 4352, 30720, 128, 384, 4, 0.5, False),        # 170 tiles
+    (FWD, 1, 2, 1, 8192, 16384, 64, 64, 4, 0.4, False),          # tile lists, half a round of 64-row halves
+    (FWD, 1, 1, 1, 12800, 16384, 64, 64, 4, 0.4, False),         # tile lists, 200 halves
+    (FWD, 1, 1, 1, 12800, 16384, 64, 64, 2, 0.03, False),
+    (DQ, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.1, False),
+    (DQ, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.5, False),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("launch,B,Hq,Hkv,Sq,Skv,qbs,kbs,dims,kind,ordered", CASES)
+def test_the_device_decides_by_the_lists_it_cuts(gpu, launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kind, ordered):
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd import _lib
+    from flex_block_attn_amd.interface import _ptr, _stream
+
+    g = torch.Generator().manual_seed(Sq + Skv)
+    m = mask_of(kind, B, Hq, Sq, Skv, qbs, kbs, dims, g)
+    pl = plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims)
+    length = steps(launch, m, B, Hq, Hkv, Sq, Skv, qbs, kbs)
+    assert length.numel() == pl["items"]
+    if ordered:
+        length = length.sort(descending=True).values
+    mean = float(length[pl["first"]:].double().mean()) if pl["first"] < pl["items"] else 0.0
+    want = 1 + sum(mean >= n for n in pl["least"])
+    print(f"parts launch {launch} B{B} Hq{Hq} Hkv{Hkv} Sq{Sq} Skv{Skv} q{qbs} k{kbs} {kind}: {pl} mean {mean:.0f} -> {want}", flush=True)
+    q, do = (torch.randn((B, Hq, Sq, HEAD), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    k, v = (torch.randn((B, Hkv, Skv, HEAD), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    lists = fba.lists_for(m.to(gpu), qbs, kbs)
+    stats = torch.stack([torch.full((B, Hq, Sq), 6.0), torch.zeros((B, Hq, Sq))]).to(gpu)  # finite and alike for both runs
+    shape = (lists.mask_bh, B, Hq, Hkv, Sq, Skv, HEAD, qbs, kbs)
+
+    def run(ws, n):
+        tail = (_ptr(ws) if ws is not None else None, n, _stream())
+        if launch == FWD:
+            outs = torch.empty_like(q), torch.empty((B, Hq, Sq, 1), device=gpu)
+            _lib.call("fba_fwd_tiled" if lists.tiled else "fba_fwd", *map(_ptr, (q, k, v, *outs, lists.q_cnt, lists.q_idx)), *shape, *tail)
+        elif launch == DQ:
+            outs = (torch.empty_like(q),)
+            _lib.call("fba_bwd_dq", *map(_ptr, (q, k, v, do, stats, *outs, lists.q_cnt, lists.q_idx)), *shape, *tail)
+        else:
+            outs = torch.empty_like(k), torch.empty_like(v)
+            _lib.call("fba_bwd_dkdv", *map(_ptr, (q, k, v, do, stats, *outs, lists.k_cnt, lists.k_idx)), *shape, *tail)
+        return outs
+
+    n = _lib.load().fba_split_workspace_bytes()
+    ws = torch.full((n,), 0x5A, dtype=torch.uint8, device=gpu)
+    cut, whole = run(ws, n), run(None, 0)
+    made = int(ws[pl["note"]:pl["note"] + 4].view(torch.int32)) if pl["device"] else pl["parts"]
+    assert made == want
+    for a, b in zip(cut, whole):
+        a, b = a.float(), b.float()
+        fin = torch.isfinite(b)
+        assert torch.equal(torch.isfinite(a), fin)
+        assert ((a - b)[fin].norm() <= 2.0 ** -8 * b[fin].norm()).item()  # each side rounds to bf16 once
+        assert torch.equal(a, b) == (want == 1)
+
+
+@pytest.mark.parametrize("launch,B,Hq,Hkv,Sq,Skv,qbs,kbs,dims,kind,ordered", CASES)
+def test_the_cases_say_what_they_claim(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kind, ordered):
+    """The device decides, and the mean length lies at least a fifth off every line."""
+    pl = plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims)
+    assert pl["device"] == 1 and pl["items"] - pl["first"] > 128 and pl["parts"] >= 2
+    m = mask_of(kind, B, Hq, Sq, Skv, qbs, kbs, dims, torch.Generator().manual_seed(Sq + Skv))
+    length = steps(launch, m, B, Hq, Hkv, Sq, Skv, qbs, kbs)
+    if ordered:
+        length = length.sort(descending=True).values
+    mean = float(length[pl["first"]:].double().mean())
+    assert all(not 0.8 * mean < n < 1.2 * mean for n in pl["least"]), (mean, pl)
