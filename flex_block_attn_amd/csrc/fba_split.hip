@@ -48,9 +48,11 @@ int device_compute_units() { return compute_units(); }
 // nothing covers, 0.5 to 1 us a launch and as much for the merge, so few items, whose parts cost little, take the number that suits
 // lists which hold 60 %.
 //
-// More than half a round is cut as well, in launches of less than two rounds, where work-groups end together: dK/dV of 136 tiles (H1
-// S17408), 40 and 90 % kept, backward 272 -> 255 and 540 -> 492 us, of 420 tiles (H3 S17920) 90 % kept 1612 -> 1424.  With items in falling
-// order of length the later rounds end at different times in any case: 680 tiles (H8 S10880) 40 % kept 579 -> 599.  Nor on tile lists, where
+// More than half a round is cut as well, in launches of less than one round, where work-groups end together: dK/dV of 136 tiles (H1
+// S17408), 30, 50 and 100 % kept, backward 227 -> 213, 350 -> 301 and 566 -> 496 us.  In a second round only of lists that are nearly full and so
+// nearly alike: with items in falling order of length the long ones make way for the short ones by themselves, and a chip that is not full
+// runs faster.  420 tiles (H3 S17920), 30, 70 and 100 % kept, whole / cut 474 / 503, 995 / 1001 and 1387 / 1340 us; 680 tiles (H8 S10880),
+// more than two rounds, 40 % kept 579 / 599.  Nor on tile lists, where
 // a part scans its lists twice: H8/4 S13824, 64 x 384 blocks, 44 % kept, dK/dV 401 -> 456 us.
 //
 // A part on a tile list scans the whole list before it takes its own steps: H5 S1536, 16 x 64 blocks, a third kept, dK/dV of 120 half
@@ -95,6 +97,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
     }
   }
   if (n_hull == 1 || hull[1].least > 0.6 * max_steps) return plan;  // lists of usual density stay whole
+  if (num_items > slots && 2 * rest > slots) hull[1].least = std::max(hull[1].least, 0.8 * max_steps);
   const double longest = rest <= kFewItems ? 0.6 * max_steps : max_steps;
   while (hull[n_hull - 1].least > longest) --n_hull;
   for (int j = 0; j < kMostParts - 1; ++j) plan.least[j] = 0x7fffffff;
