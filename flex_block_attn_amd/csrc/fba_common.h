@@ -139,9 +139,10 @@ FBA_DEVICE int split_parts(const Plan& plan, const int32_t* order) {
   const int index = plan.first + (int)((threadIdx.x & 63) * (int64_t)plan.items / 64);
   const int item = order != nullptr ? order[index] : index;
   const int head = item / l.tiles, row = (item - head * l.tiles) * l.tile_rows / l.list_rows;
-  int n[4];  // of up to four heads of the group, in flight together
+  int n[4];  // of up to four heads of the group, other ones from item to item, in flight together
 #pragma unroll
-  for (int j = 0; j < 4; ++j) n[j] = l.cnt[(l.shared ? 0 : (int64_t)(head * l.group + j * l.group / 4) * l.rows_per_head) + row];
+  for (int j = 0; j < 4; ++j)
+    n[j] = l.cnt[(l.shared ? 0 : (int64_t)(head * l.group + ((threadIdx.x & 63) + j * l.group / 4) % l.group) * l.rows_per_head) + row];
   const int sum = wave_sum(n[0] + n[1] + n[2] + n[3]);
   const int64_t steps = (int64_t)sum * l.steps * l.group;  // of 4 * 64 lists
   int parts = 1;
