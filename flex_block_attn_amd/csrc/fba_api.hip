@@ -323,9 +323,15 @@ int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, i
   plan[0] = b.num_items;
   plan[1] = sp.first;
   plan[2] = sp.parts;
-  plan[3] = split && sp.lengths.cnt != nullptr;
-  plan[4] = split ? reinterpret_cast<const char*>(sp.note) - reinterpret_cast<const char*>(ws) : 0;
-  for (int j = 0; j < fba::kMostParts - 1; ++j) plan[5 + j] = split ? sp.least[j] : 0x7fffffff;
+  const fba::ListLook& l = sp.look;
+  const bool looks = split && l.cnt != nullptr;
+  plan[3] = looks;
+  plan[4] = looks ? reinterpret_cast<const char*>(sp.note) - reinterpret_cast<const char*>(ws) : 0;
+  plan[5] = looks ? (int64_t)(1000 * l.longest / l.step) : 0;
+  plan[6] = looks ? (int64_t)(1000 * l.sum * 64 / l.step) : 0;
+  plan[7] = looks ? (int64_t)(1000 * l.least) : 0;
+  plan[8] = looks ? l.fewest : 0;
+  for (int j = 0; j < fba::kMostParts - 2; ++j) plan[9 + j] = looks && l.more[j] != 0x7fffffff ? (int64_t)(l.more[j] * l.step / 64) : 0x7fffffff;
   return FBA_OK;
 }
 

@@ -68,7 +68,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     item = p.order != nullptr ? grid_index : xcd_remap(grid_index, p.items_per_xcd);
     if (item >= p.split.first) return;
     if (p.order != nullptr) item = const_idx(p.order)[item];
-  } else if (!split_position(p.split, p.order, slot, item, part, parts)) {
+  } else if (!split_position<Look::kGroups>(p.split, p.order, slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Skv / TK;

@@ -73,7 +73,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   if (slot < 0) {
     item = xcd_remap(grid_index, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position(p.split, nullptr, slot, item, part, parts)) {
+  } else if (!split_position<Look::kNever>(p.split, nullptr, slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Skv / kTK;

@@ -45,7 +45,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / TQ;
@@ -241,7 +241,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 // Tail splitting on block lists (two work-groups per compute unit); a part stores a 128 x 128 fp32 tile.
 void plan_bwd_dq(BwdParams& p) {
   p.num_items = p.B * p.Hq * (p.Sq / 128);
-  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / 128, 128, p.q_block, p.nQ, 1, p.k_block / 32};
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, 128, p.q_block, p.nQ, 1, p.k_block / 32};
   p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, 128 * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
 }
 

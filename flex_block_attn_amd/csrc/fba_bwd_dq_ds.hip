@@ -53,7 +53,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<kWaves == 4 ? Look::kSingle : Look::kNever>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / TQ;
@@ -315,7 +315,7 @@ int plan_bwd_dq_from_ds(BwdParams& p) {
   const int waves = p.tiled ? 4 : p.q_block % 384 == 0 && rows / 384 >= enough ? 12 : p.q_block % 256 == 0 && rows / 256 >= enough ? 8 : 4;
   const int tile = 32 * waves;
   p.num_items = p.B * p.Hq * (p.Sq / tile);
-  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / tile, tile, p.q_block, p.nQ, 1, p.k_block / kSlab};
+  const ListLengths lengths{waves == 4 ? p.q_cnt : nullptr, p.mask_bh == 1, tile, p.q_block, p.nQ, 1, p.k_block / kSlab};
   p.split = plan_split(p.num_items, waves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18}, (int64_t)tile * kHeadDim * 4, p.tiled ? nullptr : p.split.ws,
                        p.split_ws_bytes, lengths);
   return waves;

@@ -129,34 +129,52 @@ FBA_DEVICE int wave_sum(int x) {
   return __builtin_amdgcn_readlane(x, 15) + __builtin_amdgcn_readlane(x, 31) + __builtin_amdgcn_readlane(x, 47) + __builtin_amdgcn_readlane(x, 63);
 }
 
-// How many parts every split item of a launch is cut into (see SplitPlan in fba_kernels.h): by the mean length of the lists of 64 of
-// them, which every wave finds alike.  `order`: the item of every grid index (long lists first, so the split ones are the shortest of the
-// launch), null where they are the same.  All lanes of a wave call this together.
-template <typename Plan>
-FBA_DEVICE int split_parts(const Plan& plan, const int32_t* order) {
-  const auto& l = plan.lengths;
-  if (l.cnt == nullptr) return plan.parts;
-  const int index = plan.first + (int)((threadIdx.x & 63) * (int64_t)plan.items / 64);
-  const int item = order != nullptr ? order[index] : index;
-  const int head = item / l.tiles, row = (item - head * l.tiles) * l.tile_rows / l.list_rows;
-  int n[4];  // of up to four heads of the group, other ones from item to item, in flight together
+// Largest value (>= 0) of the 64 lanes.
+FBA_DEVICE int wave_max(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
+  return max(max(__builtin_amdgcn_readlane(x, 15), __builtin_amdgcn_readlane(x, 31)), max(__builtin_amdgcn_readlane(x, 47), __builtin_amdgcn_readlane(x, 63)));
+}
+
+// How many parts every split item of a launch is cut into (see SplitPlan in fba_kernels.h): by 64 of the launch's lists, which every wave finds
+// alike.  All lanes of a wave call this together, with every wave of every part waiting for it, so it is short: one load, four neighbouring lists
+// to a cache line, and no division (64 lists far apart, each read four times, and four divisions: forward of H1 S10240, 64-token blocks, 40 % kept 38.6 us, of
+// H1 S16384, a quarter kept, 50.2; so 38.0 and 49.5).  kGroups: the lists of up to four query heads of a group add up, other heads from item to item.
+// kNever: for launches that the host always decides.
+enum class Look { kNever, kSingle, kGroups };
+template <Look kLook, typename Plan>
+FBA_DEVICE int split_parts(const Plan& plan) {
+  const auto& l = plan.look;
+  if (kLook == Look::kNever || l.cnt == nullptr) return plan.parts;
+  const int lane = threadIdx.x & 63;
+  const int row = min((lane >> 2) * l.stride + (lane & 3), l.last);
+  int n;
+  if (kLook == Look::kGroups && l.group > 1) {
+    const int r = (lane * 5 & 63) * l.group / 64;
+    const int32_t* const first = l.cnt + row + (int64_t)(row / l.rows_per_head) * (l.group - 1) * l.rows_per_head;  // of the group's first head
+    int of[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-    n[j] = l.cnt[(l.shared ? 0 : (int64_t)(head * l.group + ((threadIdx.x & 63) + j * l.group / 4) % l.group) * l.rows_per_head) + row];
-  const int sum = wave_sum(n[0] + n[1] + n[2] + n[3]);
-  const int64_t steps = (int64_t)sum * l.steps * l.group;  // of 4 * 64 lists
-  int parts = 1;
+    for (int j = 0; j < 4; ++j) of[j] = first[(int64_t)((j * l.group + r) / 4) * l.rows_per_head];
+    n = of[0] + of[1] + of[2] + of[3];
+  } else {
+    n = l.cnt[row];
+  }
+  const int sum = wave_sum(n);
+  if (l.longest * (float)wave_max(n) + l.sum * (float)sum < l.least) return 1;
+  int parts = l.fewest;
 #pragma unroll
-  for (int j = 0; j < 7; ++j) parts += steps >= 256LL * plan.least[j];
+  for (const int least : l.more) parts += sum >= least;
   return parts;
 }
 // Work-group s of those that do the parts.  The parts of an item follow each other, so that with 2, 4 or 8 of them an XCD (work-groups
 // are dealt to the eight round-robin) does the same range of all lists and has it in its L2.  (Part by part instead, so that an XCD
 // does all ranges: forward, H3 2304 rows against 61440 keys 120 -> 140 us.)  False: the launch has more work-groups than parts.
-template <typename Plan>
+template <Look kLook, typename Plan>
 FBA_DEVICE bool split_position(const Plan& plan, const int32_t* order, int s, int& item, int& part, int& parts) {
-  parts = split_parts(plan, order);
-  if (s == 0 && threadIdx.x == 0 && plan.lengths.cnt != nullptr) *plan.note = parts;
+  parts = split_parts<kLook>(plan);
+  if (kLook != Look::kNever && s == 0 && threadIdx.x == 0 && plan.look.cnt != nullptr) *plan.note = parts;
   const int i = s / parts;
   if (i >= plan.items) return false;
   part = s - i * parts;
@@ -167,7 +185,7 @@ FBA_DEVICE bool split_position(const Plan& plan, const int32_t* order, int s, in
 
 // For the merge: how many parts the kernel in front made.
 template <typename Plan>
-FBA_DEVICE int parts_made(const Plan& plan) { return plan.lengths.cnt == nullptr ? plan.parts : *plan.note; }
+FBA_DEVICE int parts_made(const Plan& plan) { return plan.look.cnt == nullptr ? plan.parts : *plan.note; }
 
 // Work claimed instead of given.  The hardware deals work-groups to the eight XCDs round-robin, as many to a fast XCD as to
 // a slow one, and an XCD that is through with its share idles until the kernel ends.  A launch with a claim counter per XCD

@@ -135,7 +135,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / TQ;
@@ -280,6 +280,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     };
     step(IC<0>{}, std::true_type{}, 0);
     step(IC<1>{}, std::false_type{}, 1);
+    // Where the loop lies in the 64-byte lines of the instruction cache counts where a wave has its SIMD to itself (launches of less than a
+    // round): H12 S2048, all blocks, 37.0 us with the loop 24 or 56 bytes into a line, 36.1 at 8, 40 or 60; it follows 24 bytes behind this point.
+    asm volatile(".p2align 6\n.fill 12, 4, 0xbf800000");
     for (int t = 2; t < nsteps; t += 4) {  // nsteps is even
       step(IC<2>{}, std::false_type{}, t);
       step(IC<3>{}, std::false_type{}, t + 1);
@@ -407,7 +410,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   if ((int)blockIdx.x < p.split.main_wgs) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / kHalfRows;
@@ -849,14 +852,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge
 void plan_fwd(FwdParams& p) {
   if (p.tiled) {  // a step is as long as one of fwd_kernel, a part's results are half as large
     p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
-    const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / kHalfRows, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
+    const ListLengths lengths{p.q_cnt, p.mask_bh == 1, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
     p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60, false}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
     return;
   }
   const bool wide = p.q_block % 384 == 0 && p.variant != 1;
   const int rows = wide ? 384 : 128;
   p.num_items = p.B * p.Hq * (p.Sq / rows);
-  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, p.Sq / rows, rows, p.q_block, p.nQ, 1, p.k_block / kSlab};
+  const ListLengths lengths{p.q_cnt, p.mask_bh == 1, rows, p.q_block, p.nQ, 1, p.k_block / kSlab};
   p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
 }
 

@@ -24,20 +24,31 @@ namespace fba {
 struct ListLengths {
   const int32_t* cnt;  // [1 or heads * group, rows_per_head]; null: the plan's number of parts stands
   int shared;          // one row set for all heads
-  int tiles, tile_rows, list_rows, rows_per_head;  // items per head, rows of an item, rows that share a list row, list rows per head
+  int tile_rows, list_rows, rows_per_head;  // rows of an item, rows that share a list row, list rows per head
   int group;           // rows of `group` consecutive heads add up (dK/dV: query heads of a kv head)
   int steps;           // of an entry
 };
 
-constexpr int kMostParts = 8;
+constexpr int kMostParts = 8;  // of a split item
+
+// Which lists the device looks at, and the line in units of what it finds: n entries in a lane, one list or four of a group.
+struct ListLook {
+  const int32_t* cnt;        // null: the plan's number of parts stands
+  int stride, last;          // rows 0..3, stride + 0..3, ... 15 stride + 0..3, none of them beyond the last one
+  int group, rows_per_head;  // see ListLengths; row numbers are those of one head of a group
+  float step;                // steps of an entry
+  float longest, sum, least; // parts are made where longest * (largest n) + sum * (sum of n) >= least,
+  int fewest;                // at least as many as this,
+  int more[kMostParts - 2];  // and one more for each of these that the sum of n reaches
+};
+
 struct SplitPlan {
   float* ws;      // null: nothing is split
   int first;      // first item that is split
   int parts;      // work-groups per split item, at most (>= 2 when ws is set)
   int main_wgs;   // work-groups in front of the split ones (a multiple of the XCD count)
   int items;      // that are split
-  int least[kMostParts - 1];  // steps of a list from which on 2, 3, ... parts pay
-  ListLengths lengths;
+  ListLook look;
   int32_t* note;  // behind the parts' results: how many parts the kernel made, for the merge
 };
 

@@ -1,5 +1,6 @@
 // Tail splitting: which items of a launch are cut into parts (see SplitPlan in fba_kernels.h).
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <mutex>
 
@@ -49,8 +50,8 @@ int device_compute_units() { return compute_units(); }
 // lists which hold 60 %.
 //
 // More than half a round is cut as well, in launches of less than one round, where work-groups end together: dK/dV of 136 tiles (H1
-// S17408), 30, 50 and 100 % kept, backward 227 -> 213, 350 -> 301 and 566 -> 496 us.  In a second round only of lists that are nearly full and so
-// nearly alike: with items in falling order of length the long ones make way for the short ones by themselves, and a chip that is not full
+// S17408), 30, 50 and 100 % kept, backward 227 -> 213, 350 -> 301 and 566 -> 496 us.  In a second round only where all the launch's lists are nearly
+// full and so nearly alike: with items in falling order of length the long ones make way for the short ones by themselves, and a chip that is not full
 // runs faster.  420 tiles (H3 S17920), 30, 70 and 100 % kept, whole / cut 474 / 503, 995 / 1001 and 1387 / 1340 us; 680 tiles (H8 S10880),
 // more than two rounds, 40 % kept 579 / 599.  Nor on tile lists, where
 // a part scans its lists twice: H8/4 S13824, 64 x 384 blocks, 44 % kept, dK/dV 401 -> 456 us.
@@ -97,19 +98,34 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
     }
   }
   if (n_hull == 1 || hull[1].least > 0.6 * max_steps) return plan;  // lists of usual density stay whole
-  if (num_items > slots && 2 * rest > slots) hull[1].least = std::max(hull[1].least, 0.8 * max_steps);
-  const double longest = rest <= kFewItems ? 0.6 * max_steps : max_steps;
+  const bool second = num_items > slots && 2 * rest > slots;
+  if (second) hull[1].least = std::max(hull[1].least, 0.9 * max_steps);
+  const double longest = rest <= kFewItems || lengths.cnt == nullptr ? 0.6 * max_steps : max_steps;
   while (hull[n_hull - 1].least > longest) --n_hull;
-  for (int j = 0; j < kMostParts - 1; ++j) plan.least[j] = 0x7fffffff;
-  for (int i = 1; i < n_hull; ++i)
-    for (int n = hull[i - 1].parts + 1; n <= hull[i].parts; ++n) plan.least[n - 2] = (int)hull[i].least + 1;
   plan.parts = hull[n_hull - 1].parts;
   plan.items = rest;
-  plan.lengths = lengths;
-  if (rest <= kFewItems) plan.lengths.cnt = nullptr;
+  plan.first = num_items - rest;
   plan.note = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + (int64_t)rest * plan.parts * slot_bytes);
   plan.ws = static_cast<float*>(ws);
-  plan.first = num_items - rest;
+  if (rest <= kFewItems || lengths.cnt == nullptr) return plan;
+
+  // The lists of the items that are split, or all of the launch's where these are taken in an order of their own (second rounds of dK/dV).
+  ListLook& look = plan.look;
+  const int64_t rows = (int64_t)num_items * lengths.tile_rows / lengths.list_rows, from = second ? 0 : (int64_t)plan.first * lengths.tile_rows / lengths.list_rows;
+  const int64_t span = lengths.shared ? std::min<int64_t>(rows - from, lengths.rows_per_head) : rows - from;
+  look.cnt = lengths.cnt + (lengths.shared ? lengths.rows_per_head - span : from);
+  look.group = lengths.shared ? 1 : lengths.group;
+  look.rows_per_head = lengths.rows_per_head;
+  look.stride = (int)(std::max<int64_t>(span - 4, 0) / 15);
+  look.last = (int)(span - 1);
+  look.step = (float)lengths.steps * lengths.group / (look.group > 1 ? 4 : 1);
+  look.longest = 0.f;
+  look.sum = (float)(hull[0].slope - hull[1].slope) * look.step / 64;
+  look.least = (float)(hull[1].least * (hull[0].slope - hull[1].slope));
+  look.fewest = hull[1].parts;
+  for (int& n : look.more) n = 0x7fffffff;
+  for (int i = 2; i < n_hull; ++i)
+    for (int n = hull[i - 1].parts + 1; n <= hull[i].parts; ++n) look.more[n - look.fewest - 1] = (int)std::ceil(hull[i].least * 64 / look.step);
   return plan;
 }
 
@@ -174,8 +190,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void order_ite
 void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles) {
   p.num_items = p.B * p.Hkv * (p.Skv / tiles.rows);
   const int group = p.Hq / p.Hkv;
-  const ListLengths lengths = p.tiled ? ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tiles.rows, tiles.rows, 128, p.Skv / 128, group, 1}
-                                      : ListLengths{p.k_cnt, p.mask_bh == 1, p.Skv / tiles.rows, tiles.rows, p.k_block, p.nK, group, p.q_block / 32};
+  const ListLengths lengths{p.tiled ? nullptr : p.k_cnt, p.mask_bh == 1, tiles.rows, p.k_block, p.nK, group, p.q_block / 32};  // tile lists: the host decides
   p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{tiles.step, tiles.step, tiles.step, !p.tiled}, tiles.slot_bytes, p.split.ws, p.split_ws_bytes,
                        lengths);
 }
