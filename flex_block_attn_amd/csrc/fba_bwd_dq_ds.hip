@@ -316,7 +316,7 @@ int plan_bwd_dq_from_ds(BwdParams& p) {
   const int tile = 32 * waves;
   p.num_items = p.B * p.Hq * (p.Sq / tile);
   const ListLengths lengths{waves == 4 ? p.q_cnt : nullptr, p.mask_bh == 1, tile, p.q_block, p.nQ, 1, p.k_block / kSlab};
-  p.split = plan_split(p.num_items, waves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18}, (int64_t)tile * kHeadDim * 4, p.tiled ? nullptr : p.split.ws,
+  p.split = plan_split(p.num_items, waves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18, /*scans=*/false, /*own_pace=*/false}, (int64_t)tile * kHeadDim * 4, p.tiled ? nullptr : p.split.ws,
                        p.split_ws_bytes, lengths);
   return waves;
 }

@@ -853,7 +853,7 @@ void plan_fwd(FwdParams& p) {
   if (p.tiled) {  // a step is as long as one of fwd_kernel, a part's results are half as large
     p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
     const ListLengths lengths{p.q_cnt, p.mask_bh == 1, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
-    p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60, false}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
+    p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60, /*scans=*/true}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
     return;
   }
   const bool wide = p.q_block % 384 == 0 && p.variant != 1;

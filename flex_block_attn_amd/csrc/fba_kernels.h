@@ -56,7 +56,8 @@ struct SplitPlan {
 // in a launch where few share one and where all do.
 struct StepCost {
   double alone, few, full;
-  bool most = true;  // may more than half a round be cut?
+  bool scans = false;     // a part reads its whole list before it takes its own steps (tile lists)
+  bool own_pace = true;   // a whole round ends with its longest list (false: bound by memory, which the short ones leave to the long ones)
 };
 
 // Items and work-group slots of a launch -> plan (first = num_items, parts = 1 when nothing is split).  `slot_bytes` is

@@ -49,6 +49,15 @@ int device_compute_units() { return compute_units(); }
 // nothing covers, 0.5 to 1 us a launch and as much for the merge, so few items, whose parts cost little, take the number that suits
 // lists which hold 60 %.
 //
+// Lists that differ: whole items of a single round take as long as the longest list, parts about as long as a list that is 0.6 of the mean and 0.4
+// of the longest.  So the line for one round is drawn where  slope(1) longest - slope(parts) (0.6 mean + 0.4 longest)  reaches what the
+// parts cost besides.  Forward, decided by the mean / so: H1 S20480, 128-token blocks, Bernoulli masks of 10 % 56.5 / 45.8 us, densities that
+// rise ninefold along the sequence 74.1 / 50.9, causal H5 S4352 68.2 / 50.6.  So that such masks can be cut, launches of up to half a round
+// are planned too where lists of one length would have to hold more than 60 %, if lists that fall to nothing gain well; lists of one
+// length there pay 2 us for the look and a merge with nothing to do (H5 S4352, a quarter kept 22.1 -> 24.3 us; always cut they took 30.8).
+// dQ from dS is not judged by the longest list: it is bound by memory, which the short lists leave to the long ones (H3 S10240, 30 % kept,
+// backward 182 -> 195 us).
+//
 // More than half a round is cut as well, in launches of less than one round, where work-groups end together: dK/dV of 136 tiles (H1
 // S17408), 30, 50 and 100 % kept, backward 227 -> 213, 350 -> 301 and 566 -> 496 us.  In a second round only where all the launch's lists are nearly
 // full and so nearly alike: with items in falling order of length the long ones make way for the short ones by themselves, and a chip that is not full
@@ -71,7 +80,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   int slots = compute_units() * wgs_per_cu;
   if (slots > kSplitMaxSlots) slots = kSplitMaxSlots;
   const int rest = num_items % slots;
-  if (rest == 0 || (2 * rest > slots && (num_items >= 2 * slots || !step.most))) return plan;
+  if (rest == 0 || (2 * rest > slots && (num_items >= 2 * slots || step.scans))) return plan;
   // cost(n) = slope(n) steps + parts and, where there are any, the launch that merges them.  From how long a list on is a number of
   // parts the cheapest: the slope falls from one candidate to the next, and one that is never the cheapest gives way.
   auto slope = [&](int n) {
@@ -86,7 +95,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   int n_hull = 1;
   for (int n = 2; n <= kMostParts && (int64_t)rest * n * slot_bytes + kNoteBytes <= ws_bytes; ++n) {
     if (num_items > slots && rest * n > slots && 2 * rest <= slots) break;  // a last round that fills up while others end gains nothing from another
-    Candidate next{n, slope(n), (double)rest * n + kMergeCost + (step.most ? 0 : kScanCost), 0.};
+    Candidate next{n, slope(n), (double)rest * n + kMergeCost + (step.scans ? kScanCost : 0), 0.};
     if (wgs_per_cu == 1 && 2 * rest > slots && next.slope > 0.75 * slope(1)) continue;  // 0.8 of a round in five parts: H2 S29440 1055 -> 1095 us
     while (n_hull > 0 && next.slope < hull[n_hull - 1].slope) {
       next.least = (next.fixed - hull[n_hull - 1].fixed) / (hull[n_hull - 1].slope - next.slope);
@@ -97,17 +106,21 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
       --n_hull;
     }
   }
-  if (n_hull == 1 || hull[1].least > 0.6 * max_steps) return plan;  // lists of usual density stay whole
+  if (n_hull == 1) return plan;
+  const bool device = rest > kFewItems && lengths.cnt != nullptr, one_round = device && num_items < slots && step.own_pace;
+  const double least = hull[1].least * (hull[0].slope - hull[1].slope);
+  const bool uneven = one_round && 2 * rest <= slots && max_steps * (hull[0].slope - 0.5 * hull[1].slope) >= 2.5 * least;
+  if (hull[1].least > 0.6 * max_steps && !uneven) return plan;  // lists of usual density stay whole
   const bool second = num_items > slots && 2 * rest > slots;
   if (second) hull[1].least = std::max(hull[1].least, 0.9 * max_steps);
-  const double longest = rest <= kFewItems || lengths.cnt == nullptr ? 0.6 * max_steps : max_steps;
-  while (hull[n_hull - 1].least > longest) --n_hull;
+  const double longest = device ? max_steps : 0.6 * max_steps;
+  while (n_hull > 2 && hull[n_hull - 1].least > longest) --n_hull;
   plan.parts = hull[n_hull - 1].parts;
   plan.items = rest;
   plan.first = num_items - rest;
   plan.note = reinterpret_cast<int32_t*>(static_cast<char*>(ws) + (int64_t)rest * plan.parts * slot_bytes);
   plan.ws = static_cast<float*>(ws);
-  if (rest <= kFewItems || lengths.cnt == nullptr) return plan;
+  if (!device) return plan;
 
   // The lists of the items that are split, or all of the launch's where these are taken in an order of their own (second rounds of dK/dV).
   ListLook& look = plan.look;
@@ -119,8 +132,9 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   look.stride = (int)(std::max<int64_t>(span - 4, 0) / 15);
   look.last = (int)(span - 1);
   look.step = (float)lengths.steps * lengths.group / (look.group > 1 ? 4 : 1);
-  look.longest = 0.f;
-  look.sum = (float)(hull[0].slope - hull[1].slope) * look.step / 64;
+  const double by_longest = one_round ? hull[0].slope - 0.4 * hull[1].slope : 0.;
+  look.longest = (float)(by_longest * look.step);
+  look.sum = (float)((hull[0].slope - hull[1].slope - by_longest) * look.step / 64);
   look.least = (float)(hull[1].least * (hull[0].slope - hull[1].slope));
   look.fewest = hull[1].parts;
   for (int& n : look.more) n = 0x7fffffff;
@@ -191,7 +205,7 @@ void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles) {
   p.num_items = p.B * p.Hkv * (p.Skv / tiles.rows);
   const int group = p.Hq / p.Hkv;
   const ListLengths lengths{p.tiled ? nullptr : p.k_cnt, p.mask_bh == 1, tiles.rows, p.k_block, p.nK, group, p.q_block / 32};  // tile lists: the host decides
-  p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{tiles.step, tiles.step, tiles.step, !p.tiled}, tiles.slot_bytes, p.split.ws, p.split_ws_bytes,
+  p.split = plan_split(p.num_items, 1, group * (p.Sq / 32), StepCost{tiles.step, tiles.step, tiles.step, p.tiled != 0}, tiles.slot_bytes, p.split.ws, p.split_ws_bytes,
                        lengths);
 }
 

@@ -76,6 +76,14 @@ CASES = [
     (FWD, 1, 3, 3, 8192, 17920, 8192, 128, 4, 0.6),              # three lists in all
     (FWD, 1, 3, 3, 8192, 17920, 4096, 128, 2, 0.6),              # two
     (DKDV, 1, 5, 1, 4096, 17408, 256, 17408, 4, 1.0),            # one list of five heads' each
+    # lists of one round that differ: cut for the longest where the mean would not be
+    (FWD, 1, 1, 1, 20480, 20480, 128, 128, 4, 0.1),
+    (FWD, 1, 5, 5, 4352, 4352, 128, 128, 4, "causal"),
+    (FWD, 1, 5, 5, 4352, 4352, 128, 128, 2, 0.05),
+    (FWD, 1, 1, 1, 16384, 8192, 64, 64, 4, "causal"),
+    (DKDV, 1, 1, 1, 6144, 17408, 128, 128, 4, "causal"),
+    (DKDV, 1, 8, 1, 2048, 17408, 128, 128, 2, "causal"),
+    (DQ, 1, 5, 5, 4352, 4352, 128, 128, 4, "causal"),
     (DQ, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.1),
     (DQ, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.5),
 ]
@@ -137,6 +145,18 @@ def test_the_cases_say_what_they_claim(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, di
     want, off, mean = decision(pl, looked_at(pl, length))
     assert abs(off) > 0.1, (off, mean, pl)
     assert want == 1 or all(not 0.85 * mean < n < 1.15 * mean for n in pl["more"]), (mean, pl)
+
+
+@pytest.mark.parametrize("launch,B,Hq,Hkv,Sq,Skv,qbs,kbs", [(FWD, 1, 5, 5, 4352, 4352, 128, 128), (FWD, 1, 1, 1, 16384, 8192, 64, 64), (DKDV, 1, 1, 1, 6144, 17408, 128, 128),
+                                                             (DKDV, 1, 8, 1, 2048, 17408, 128, 128), (DQ, 1, 5, 5, 4352, 4352, 128, 128)])
+def test_the_longest_list_of_a_round_decides(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs):
+    """Lists that fall to nothing are cut where lists of one length, as long as their mean, are not."""
+    pl = plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, 4)
+    most = Hq // Hkv * Sq // 32 if launch == DKDV else Skv // (64 if qbs < 128 else 32)
+    at = next(n for n in range(most) if (pl["longest"] + pl["mean"]) * n >= pl["least"])  # equal lists are cut from here on
+    falling = torch.linspace(0, min(most, 1.9 * at), 129)
+    assert float(falling.mean()) < at and decision(pl, falling)[0] > 1
+    assert decision(pl, falling * 0 + at - 1)[0] == 1 and decision(pl, falling * 0 + at)[0] > 1
 
 
 def test_second_rounds_are_cut_where_lists_are_nearly_full():
