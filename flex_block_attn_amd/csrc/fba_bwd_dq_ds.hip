@@ -276,7 +276,8 @@ hipError_t zero_unit_address(const char** out) {
 }  // namespace
 
 // Sums the fp32 partial rows of the split items in part order: out = scale * sum_p partial_p, as bf16.  One thread per four
-// columns; an item has `rows` rows of 128 columns; blockIdx.y picks the output (dK/dV: two per slot, one launch for both).
+// columns; an item has `rows` rows of 128 columns; blockIdx.y picks the output (dK/dV: two per slot, one launch for both).  All parts are
+// requested at once, as in fwd_merge_kernel.
 struct PartialOuts {
   PartialOut out[2];
 };
@@ -288,13 +289,22 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_s
   const int parts = parts_made(split);
   if (parts == 1) return;  // done whole
   for (int block = blockIdx.x; block < split.items * (rows / 8); block += gridDim.x) {
-  const int row = block * 8 + (tid >> 5);  // among the rows of all split items
-  const int it = row / rows, r = row - it * rows;
-  const int64_t item = order != nullptr ? order[split.first + it] : split.first + it;
-  const float* src = split.ws + (int64_t)it * parts * slot_floats + o.offset + r * kHeadDim + c4;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int q = 0; q < parts; ++q) acc += *reinterpret_cast<const f32x4*>(src + q * slot_floats);
-  *reinterpret_cast<bf16x4*>(o.out + (item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
+    const int row = block * 8 + (tid >> 5);  // among the rows of all split items
+    const int it = row / rows, r = row - it * rows;
+    const float* src = split.ws + (int64_t)it * parts * slot_floats + o.offset + r * kHeadDim + c4;
+    f32x4 of[kMostParts];
+#pragma unroll
+    for (int q = 0; q < kMostParts; ++q)
+      if (q < parts) {
+        of[q] = *reinterpret_cast<const f32x4*>(src);
+        src += slot_floats;
+      }
+    const int64_t item = order != nullptr ? order[split.first + it] : split.first + it;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < kMostParts; ++q)
+      if (q < parts) acc += of[q];
+    *reinterpret_cast<bf16x4*>(o.out + (item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
   }
 }
 

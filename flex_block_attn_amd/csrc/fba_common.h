@@ -183,10 +183,6 @@ FBA_DEVICE bool split_position(const Plan& plan, const int32_t* order, int s, in
   return true;
 }
 
-// For the merge: how many parts the kernel in front made.
-template <typename Plan>
-FBA_DEVICE int parts_made(const Plan& plan) { return plan.look.cnt == nullptr ? plan.parts : *plan.note; }
-
 // Work claimed instead of given.  The hardware deals work-groups to the eight XCDs round-robin, as many to a fast XCD as to
 // a slow one, and an XCD that is through with its share idles until the kernel ends.  A launch with a claim counter per XCD
 // (zeroed beforehand) has some work-groups more than grid indices to do; every work-group claims an index of its own XCD
@@ -242,6 +238,10 @@ struct TileCopy {
 // (s_load_dword) wherever they sit, also behind inline asm and barriers.
 typedef const FBA_CONST int32_t* ConstIdx;
 FBA_DEVICE ConstIdx const_idx(const int32_t* p) { return (ConstIdx)(uintptr_t)p; }
+
+// For the merge: how many parts the kernel in front made.  A scalar load: the merge's addresses wait for it.
+template <typename Plan>
+FBA_DEVICE int parts_made(const Plan& plan) { return plan.look.cnt == nullptr ? plan.parts : const_idx(plan.note)[0]; }
 
 // Address of a __shared__ object inside the work-group's LDS allocation.
 FBA_DEVICE uint32_t lds_addr(const void* p) { return (uint32_t)(uintptr_t)(FBA_LDS const char*)p; }

@@ -817,7 +817,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kMaskWaves, 64 * kMas
 }
 
 // Combines the parts of the split items: O = sum_p 2^(m_p - m) O_p / sum_p 2^(m_p - m) l_p with m = max_p m_p, in part
-// order.  One thread per (query row, four head-dim columns).
+// order.  One thread per (query row, four head-dim columns).  Bound by latency: whatever the parts hold is requested at once (part after
+// part, each waiting for the one in front: H7 384 rows against 46720 keys, eight parts, 7.1 us, so 4.6).
 template <int kTileRows>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge_kernel(const FwdParams p) {
   const int tid = threadIdx.x;
@@ -825,26 +826,37 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge
   const int parts = parts_made(p.split);
   if (parts == 1) return;  // done whole
   for (int block = blockIdx.x; block < p.split.items * (kTileRows / 8); block += gridDim.x) {
-  const int row = block * 8 + (tid >> 5), c4 = (tid & 31) * 4;  // row among the kTileRows * (split items) rows
-  const int it = row / kTileRows, r = row % kTileRows;
-  const int item = p.split.first + it;
-  const float* slot0 = p.split.ws + (int64_t)it * parts * kSlotFloats;
-  float m = -INFINITY;
-  for (int q = 0; q < parts; ++q) m = fmaxf(m, slot0[(int64_t)q * kSlotFloats + kTileRows * kHeadDim + r]);
-  float l = 0.f;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int q = 0; q < parts; ++q) {
-    const float* slot = slot0 + (int64_t)q * kSlotFloats;
-    const float mq = slot[kTileRows * kHeadDim + r];
-    const float w = mq == -INFINITY ? 0.f : fast_exp2(mq - m);
-    l += w * slot[kTileRows * kHeadDim + kTileRows + r];
-    const f32x4 o4 = *reinterpret_cast<const f32x4*>(slot + r * kHeadDim + c4);
-    acc += w * o4;
-  }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  const int64_t orow = (int64_t)item * kTileRows + r;  // items are consecutive tiles of [B, Hq, Sq]
-  *reinterpret_cast<bf16x4*>(p.o + orow * kHeadDim + c4) = pack4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-  if (c4 == 0) p.lse[orow] = l > 0.f ? (m + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
+    const int row = block * 8 + (tid >> 5), c4 = (tid & 31) * 4;  // row among the kTileRows * (split items) rows
+    const int it = row / kTileRows, r = row % kTileRows;
+    const int item = p.split.first + it;
+    const float* slot = p.split.ws + (int64_t)it * parts * kSlotFloats;
+    float mq[kMostParts], lq[kMostParts];
+    f32x4 oq[kMostParts];
+#pragma unroll
+    for (int q = 0; q < kMostParts; ++q)
+      if (q < parts) {
+        mq[q] = slot[kTileRows * kHeadDim + r];
+        lq[q] = slot[kTileRows * kHeadDim + kTileRows + r];
+        oq[q] = *reinterpret_cast<const f32x4*>(slot + r * kHeadDim + c4);
+        slot += kSlotFloats;
+      }
+    float m = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < kMostParts; ++q)
+      if (q < parts) m = fmaxf(m, mq[q]);
+    float l = 0.f;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < kMostParts; ++q)
+      if (q < parts) {
+        const float w = mq[q] == -INFINITY ? 0.f : fast_exp2(mq[q] - m);
+        l += w * lq[q];
+        acc += w * oq[q];
+      }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int64_t orow = (int64_t)item * kTileRows + r;  // items are consecutive tiles of [B, Hq, Sq]
+    *reinterpret_cast<bf16x4*>(p.o + orow * kHeadDim + c4) = pack4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+    if (c4 == 0) p.lse[orow] = l > 0.f ? (m + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
   }
 }
 

@@ -84,7 +84,7 @@ void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles);
 
 // Work-groups of a launch that merges parts: each does every so many of the blocks of eight rows, so that little is launched where
 // the lists turn out too short for parts.
-inline int merge_grid(int blocks) { return blocks < 2048 ? blocks : 2048; }
+inline int merge_grid(int blocks) { return blocks < 1024 ? blocks : 1024; }
 
 // How the whole items of a launch are dealt to the XCDs (see xcd_remap): contiguous spans when the launch has at least
 // one (batch, head) per XCD, work-group order otherwise.  Sets items_per_xcd and the number of work-groups that come
