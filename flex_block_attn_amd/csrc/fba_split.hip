@@ -55,7 +55,8 @@ int device_compute_units() { return compute_units(); }
 // rise ninefold along the sequence 74.1 / 50.9, causal H5 S4352 68.2 / 50.6.  So that such masks can be cut, launches of up to half a round
 // are planned too where lists of one length would have to hold more than 60 %, if lists that fall to nothing gain well; lists of one
 // length there pay 2 us for the look and a merge with nothing to do (H5 S4352, a quarter kept 22.1 -> 24.3 us; always cut they took 30.8).
-// dQ from dS is not judged by the longest list: it is bound by memory, which the short lists leave to the long ones (H3 S10240, 30 % kept,
+// Tile lists of 128 rows differ more than the halves that are worked on, so only half of what the longest is above the mean counts there (H2
+// S8192, 64-token blocks, 31 % kept, lists of 67 chunks and up to 74 for halves of 40 each).  dQ from dS is not judged by the longest list: it is bound by memory, which the short lists leave to the long ones (H3 S10240, 30 % kept,
 // backward 182 -> 195 us).
 //
 // More than half a round is cut as well, in launches of less than one round, where work-groups end together: dK/dV of 136 tiles (H1
@@ -132,7 +133,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   look.stride = (int)(std::max<int64_t>(span - 4, 0) / 15);
   look.last = (int)(span - 1);
   look.step = (float)lengths.steps * lengths.group / (look.group > 1 ? 4 : 1);
-  const double by_longest = one_round ? hull[0].slope - 0.4 * hull[1].slope : 0.;
+  const double by_longest = one_round ? (hull[0].slope - 0.4 * hull[1].slope) * (step.scans ? 0.5 : 1.) : 0.;
   look.longest = (float)(by_longest * look.step);
   look.sum = (float)((hull[0].slope - hull[1].slope - by_longest) * look.step / 64);
   look.least = (float)(hull[1].least * (hull[0].slope - hull[1].slope));
