@@ -56,7 +56,7 @@ int device_compute_units() { return compute_units(); }
 // are planned too where lists of one length would have to hold more than 60 %, if lists that fall to nothing gain well; lists of one
 // length there pay 2 us for the look and a merge with nothing to do (H5 S4352, a quarter kept 22.1 -> 24.3 us; always cut they took 30.8).
 // Tile lists of 128 rows differ more than the halves that are worked on, so only half of what the longest is above the mean counts there (H2
-// S8192, 64-token blocks, 31 % kept, lists of 67 chunks and up to 74 for halves of 40 each).  dQ from dS is not judged by the longest list: it is bound by memory, which the short lists leave to the long ones (H3 S10240, 30 % kept,
+// S8192, 64-token blocks, 31 % kept, lists of 67 chunks and up to 73 for halves of 40 each).  dQ from dS is not judged by the longest list: it is bound by memory, which the short lists leave to the long ones (H3 S10240, 30 % kept,
 // backward 182 -> 195 us).
 //
 // More than half a round is cut as well, in launches of less than one round, where work-groups end together: dK/dV of 136 tiles (H1

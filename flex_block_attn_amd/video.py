@@ -122,15 +122,19 @@ class _TilePermuteAll(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, grid, tile):
         ctx.args = (tuple(grid), tuple(tile))
+        ctx.set_materialize_grads(False)  # autograd would fill two tensors of zeros for the means
         outs, means = _gather((q, k, v), grid, tile, True, means=(0, 1))
         ctx.mark_non_differentiable(*means)
         return (*outs, *means)
 
     @staticmethod
     def backward(ctx, gq, gk, gv, *_):
-        wanted = [j for j in range(3) if ctx.needs_input_grad[j]]
-        outs, _ = _gather([(gq, gk, gv)[j].to(torch.bfloat16) for j in wanted], *ctx.args, False)
+        given = (gq, gk, gv)
+        wanted = [j for j in range(3) if ctx.needs_input_grad[j] and given[j] is not None]
         grads = [None] * 5
+        if not wanted:
+            return tuple(grads)
+        outs, _ = _gather([given[j].to(torch.bfloat16) for j in wanted], *ctx.args, False)
         for j, g in zip(wanted, outs):
             grads[j] = g
         return tuple(grads)

@@ -88,3 +88,35 @@ def test_refused_extents(gpu, window):
         window = window.to(gpu)
     with pytest.raises((ValueError, TypeError, RuntimeError)):
         video.create_ssta_3d_mask(q, q, (2, 16, 16), (1, 8, 8), window)
+
+
+def test_outputs_that_enter_nothing(gpu):
+    """Only what has a gradient is gathered back: nothing is filled for the means, and inputs whose output enters nothing get no gradient."""
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd import video
+
+    grid, tile = (2, 16, 16), (1, 8, 8)
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn((1, 2, 512, 128), generator=g).to(torch.bfloat16).to(gpu).requires_grad_(True) for _ in range(3))
+    got = []
+    inner = video._gather
+
+    def gather(xs, grid, tile, to_tiles, means=()):
+        if not to_tiles:
+            got.append(len(xs))
+        return inner(xs, grid, tile, to_tiles, means)
+
+    video._gather = gather
+    try:
+        for used, n in ((0,), 1), ((1, 2), 2), ((0, 1, 2), 3):
+            outs = video._TilePermuteAll.apply(q, k, v, grid, tile)
+            weights = torch.randn((1, 2, 512, 128), generator=g).to(torch.bfloat16).to(gpu)
+            grads = torch.autograd.grad([outs[j] for j in used], (q, k, v), [weights] * len(used), allow_unused=True)
+            for j in range(3):
+                assert (grads[j] is None) if j not in used else torch.equal(grads[j], fba.untile_tokens(weights, grid, tile))
+            assert got.pop() == n and not got
+        with torch.profiler.profile() as prof:
+            torch.autograd.grad(video._TilePermuteAll.apply(q, k, v, grid, tile)[:3], (q, k, v), [weights] * 3)
+        assert not [e.key for e in prof.key_averages() if "zero" in e.key or "fill" in e.key]
+    finally:
+        video._gather = inner
