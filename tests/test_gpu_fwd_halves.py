@@ -3,10 +3,10 @@ at a time.  List lengths around 64 and its multiples, halves that select
 nothing, the first or only the last entries, one chunk in all, key blocks of one and of several chunks, 16-row groups, grouped
 heads, shared and separate masks, split launches.  Against the oracle's explicit dense formula (fp32) with the operator's parity
 bar for N(0,1) inputs; O, LSE bit-equal on a repeat, and rows without keys exactly 0 and -inf."""
+import ctypes
+
 import pytest
 import torch
-
-pytestmark = pytest.mark.gpu
 
 MAX_ABS, REL_L2 = 2e-2, 1e-2
 
@@ -27,6 +27,16 @@ def _mask(kind, shape, g):
     return m
 
 
+@pytest.mark.parametrize("Skv,cut", [(768, False), (1280, True)])
+def test_last_round_of_the_split_case(Skv, cut):
+    from flex_block_attn_amd import _lib
+
+    plan = (ctypes.c_int64 * 15)()
+    _lib.call("fba_split_plan", 0, 30, 1, 30, 30, 1152, Skv, 128, 16, 64, _lib.load().fba_split_workspace_bytes(), plan)
+    assert plan[0] == 540 and plan[1] == (512 if cut else 540) and (plan[2] > 1) == cut
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,qbs,kbs,dims,kind", [
     (1, 1, 1, 128, 128, 64, 64, 2, "all"),
     (1, 1, 1, 128, 128, 16, 128, 2, "one"),
@@ -41,7 +51,8 @@ def _mask(kind, shape, g):
     (1, 3, 1, 384, 1152, 128, 64, 4, "random"),   # halves that agree
     (1, 2, 2, 768, 1152, 384, 192, 2, "ends"),
     (2, 24, 24, 1536, 1536, 64, 64, 4, "random"),  # more items than slots
-    (1, 30, 30, 1152, 768, 16, 64, 4, "random"),   # the last round of 28 items is split
+    (1, 30, 30, 1152, 768, 16, 64, 4, "random"),   # a round and 28 items, whole
+    (1, 30, 30, 1152, 1280, 16, 64, 4, "random"),  # the last round of 28 items is split
 ])
 def test_fwd_halves(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kind):
     import flex_block_attn_amd as fba
@@ -63,6 +74,7 @@ def test_fwd_halves(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kind):
     assert torch.equal(o, o2) and torch.equal(lse, lse2)
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("qbs,kbs,Skv", [(64, 64, 384), (64, 128, 384), (16, 64, 384), (192, 64, 384), (64, 64, 16384)])
 def test_fwd_scores_of_minus_infinity(gpu, qbs, kbs, Skv):
     """Keys whose scores are -inf count for nothing, also where they fill the first slabs a wave meets, all of one wave's slabs, or

@@ -39,6 +39,7 @@ def _reference_allclose(got, want):
 
 def _run_case(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, mask, seed=0, peaky=False, ref_allclose=False):
     import flex_block_attn_amd as fba
+    from flex_block_attn_amd import _lib
 
     q, k, v, do = oracle.seeded_qkv(B, Hq, Hkv, Sq, Skv, seed=seed, peaky=peaky)
     qb, kb, vb, dob = (t.to(torch.bfloat16) for t in (q, k, v, do))
@@ -53,6 +54,18 @@ def _run_case(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, mask, seed=0, peaky=Fa
     _check(oracle, o, o_ref, "o", res, peaky)
     if ref_allclose:
         _reference_allclose(o, o_ref)
+    if Sq % 128 == 0 and Skv % 128 == 0 and _lib.load().fba_fwd_takes_mask(B * Hq * Sq, Skv):
+        # the operator has read the mask itself: the same inputs through the kernels on lists
+        with torch.no_grad():
+            o_lists, lse = fba.forward_with_lists(qg, kg, vg, qbs, kbs, fba.lists_for(mask.to(gpu), qbs, kbs))
+        _check(oracle, o_lists, o_ref, "o on lists", res, peaky)
+        if ref_allclose:
+            _reference_allclose(o_lists, o_ref)
+        lse, want = lse.flatten().cpu(), lse_ref.flatten().float()
+        assert torch.equal(torch.isinf(lse), torch.isinf(want))
+        # the denominator sums P rounded to bf16 (2^-8 of it at most), the scores are fp32 sums of 128 products
+        fin = ~torch.isinf(want)
+        assert ((lse - want)[fin].abs() <= 2.0 ** -8 + 128 * 2.0 ** -24 * want[fin].abs()).all()
     _check(oracle, qg.grad, dq_ref, "dq", res, peaky)
     _check(oracle, kg.grad, dk_ref, "dk", res, peaky)
     _check(oracle, vg.grad, dv_ref, "dv", res, peaky)
@@ -834,7 +847,7 @@ def test_measurement_variants_give_the_same_bits(gpu, cfg, monkeypatch):
 
 def test_tile_list_forward_splits_its_tail(oracle, gpu, monkeypatch):
     """Forward on tile lists with and without the splitting workspace: a launch smaller than the GPU (every tile cut into
-    parts) against the oracle, and a launch of 2.25 rounds (the last quarter round cut into parts) against itself without
+    parts) against the oracle, and a launch of 4.5 rounds (the last half round cut into parts) against itself without
     splitting; entries switched off for some 16-row groups, an empty query block and a range that starts inside an entry's
     second slab are all in there."""
     import flex_block_attn_amd as fba
@@ -846,7 +859,23 @@ def test_tile_list_forward_splits_its_tail(oracle, gpu, monkeypatch):
     for split in (None, "0"):
         monkeypatch.setattr(interface, "SPLIT_WORKSPACE_MIB", split)
         _run_case(oracle, gpu, 1, 2, 2, 768, 384, 64, 64, m, seed=32)
-    B, H, S, bs = 1, 9, 16384, 64  # 1152 tiles of 128 rows on 512 slots
+    # 24 halves against lists of up to 64 chunks
+    m = torch.rand((1, 2, 12, 64), generator=g) < 0.5
+    m[..., 3, :] = False
+    q, k, v, _ = oracle.seeded_qkv(1, 2, 2, 768, 4096, seed=33)
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    o_ref, lse_ref = oracle.c_attention_forward(q, k, v, m, 64, 64)
+    lists = fba.lists_for(m.to(gpu), 64, 64)
+    outs, res = [], {}
+    for split in (None, "0"):
+        monkeypatch.setattr(interface, "SPLIT_WORKSPACE_MIB", split)
+        o, lse = fba.forward_with_lists(q.to(gpu), k.to(gpu), v.to(gpu), 64, 64, lists)
+        _check(oracle, o, o_ref, f"o split {split}", res)
+        assert torch.equal(torch.isinf(lse).flatten().cpu(), torch.isinf(lse_ref).flatten())
+        outs.append(o)
+    rows = (torch.arange(768) // 64 != 3).to(gpu)
+    assert not torch.equal(outs[0][:, :, rows], outs[1][:, :, rows])  # the parts did sum in another order
+    B, H, S, bs = 1, 9, 16384, 64  # 2304 halves of 128-row tiles on 512 slots
     nb = S // bs
     q, k, v = (torch.randn((B, H, S, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(3))
     mask = (torch.rand((B, H, nb, nb), generator=g) < 0.15).to(gpu)
