@@ -164,3 +164,29 @@ def test_second_rounds_are_cut_where_lists_are_nearly_full():
         pl = plan(DKDV, 1, 3, Hkv, Sq, 17920 * 3 // Hkv, 256, 128, 4)
         assert pl["items"] == 420 and pl["first"] == 256 and pl["parts"] == 3
         assert 0.89 <= pl["least"] / pl["mean"] / ((3 // Hkv) * Sq / 32) <= 0.91
+
+
+@pytest.mark.gpu
+def test_a_replayed_graph_decides_by_the_lists_of_that_replay(gpu):
+    import flex_block_attn_amd as fba
+
+    H, S = 1, 20480
+    assert plan(FWD, 1, H, H, S, S, 128, 128, 4)["device"] == 1
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn((1, H, S, HEAD), generator=g).to(torch.bfloat16).to(gpu) for _ in range(3))
+    masks = [(torch.rand((1, H, S // 128, S // 128), generator=g) < d).to(gpu) for d in (0.02, 0.5, 0.02)]
+    m = masks[0].clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        fba.flex_block_attn_func(q, k, v, 128, 128, m)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        o = fba.flex_block_attn_func(q, k, v, 128, 128, m)
+    for mask in masks:
+        m.copy_(mask)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = o.clone()
+        assert torch.equal(got, fba.flex_block_attn_func(q, k, v, 128, 128, mask))
