@@ -1,4 +1,5 @@
 // C ABI entry points: argument validation, variant selection, launches.  See include/fba.h for the contract.
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -327,11 +328,10 @@ int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, i
   const bool looks = split && l.cnt != nullptr;
   plan[3] = looks;
   plan[4] = looks ? reinterpret_cast<const char*>(sp.note) - reinterpret_cast<const char*>(ws) : 0;
-  plan[5] = looks ? (int64_t)(1000 * l.longest / l.step) : 0;
-  plan[6] = looks ? (int64_t)(1000 * l.sum * 64 / l.step) : 0;
-  plan[7] = looks ? (int64_t)(1000 * l.least) : 0;
-  plan[8] = looks ? l.fewest : 0;
-  for (int j = 0; j < fba::kMostParts - 2; ++j) plan[9 + j] = looks && l.more[j] != 0x7fffffff ? (int64_t)(l.more[j] * l.step / 64) : 0x7fffffff;
+  const float cost[4] = {l.spread, l.whole / l.step, l.cut / l.step, l.least};
+  for (int j = 0; j < 4; ++j) plan[5 + j] = looks ? (int64_t)(1000 * cost[j]) : 0;
+  plan[9] = looks ? l.fewest : 0;
+  for (int j = 0; j < fba::kMostParts - 2; ++j) plan[10 + j] = looks && l.more[j] < 1e9f ? (int64_t)std::ceil(l.more[j] * l.step) : 0x7fffffff;
   return FBA_OK;
 }
 

@@ -144,6 +144,7 @@ FBA_DEVICE int wave_max(int x) {
 // H1 S16384, a quarter kept, 50.2; so 38.0 and 49.5).  kGroups: the lists of up to four query heads of a group add up, other heads from item to item.
 // kNever: for launches that the host always decides.
 enum class Look { kNever, kSingle, kGroups };
+constexpr float kPartsSpread = 0.4f;  // how much of what the longest list is above the mean the parts of all lists take longer
 template <Look kLook, typename Plan>
 FBA_DEVICE int split_parts(const Plan& plan) {
   const auto& l = plan.look;
@@ -161,11 +162,12 @@ FBA_DEVICE int split_parts(const Plan& plan) {
   } else {
     n = l.cnt[row];
   }
-  const int sum = wave_sum(n);
-  if (l.longest * (float)wave_max(n) + l.sum * (float)sum < l.least) return 1;
+  const float mean = (float)wave_sum(n) * (1.f / 64.f);
+  const float longest = mean + l.spread * ((float)wave_max(n) - mean), cut = mean + kPartsSpread * (longest - mean);
+  if (l.whole * longest - l.cut * cut < l.least) return 1;
   int parts = l.fewest;
 #pragma unroll
-  for (const int least : l.more) parts += sum >= least;
+  for (const float more : l.more) parts += cut >= more;
   return parts;
 }
 // Work-group s of those that do the parts.  The parts of an item follow each other, so that with 2, 4 or 8 of them an XCD (work-groups

@@ -37,9 +37,10 @@ struct ListLook {
   int stride, last;          // rows 0..3, stride + 0..3, ... 15 stride + 0..3, none of them beyond the last one
   int group, rows_per_head;  // see ListLengths; row numbers are those of one head of a group
   float step;                // steps of an entry
-  float longest, sum, least; // parts are made where longest * (largest n) + sum * (sum of n) >= least,
-  int fewest;                // at least as many as this,
-  int more[kMostParts - 2];  // and one more for each of these that the sum of n reaches
+  // Whole items take as long as a list of  mean + spread (largest - mean)  entries, call it L, parts as long as one of  mean + 0.4 (L - mean).
+  float spread, whole, cut, least;  // parts are made where whole * (the first) - cut * (the second) >= least,
+  int fewest;                       // at least as many as this,
+  float more[kMostParts - 2];       // and one more for each of these that the second reaches
 };
 
 struct SplitPlan {

@@ -44,34 +44,34 @@ int device_compute_units() { return compute_units(); }
 // 0.6 us with 64 (64 KiB).
 //
 // L is on the device: the host says from which lengths on which numbers of parts pay, up to the longest possible lists, and the kernel
-// looks at the lists.  Forward / backward, parts for lists that hold 40 % -> for the lists there are, 10 % kept: H3 S6400 27.8 / 73.9
-// -> 20.6 / 66.6 us, H5 S5120 26.8 / 62.1 -> 15.5 / 62.0, H1 S30720 62.2 / 206.9 -> 59.6 / 185.9.  Looking costs a load that
-// nothing covers, 0.5 to 1 us a launch and as much for the merge, so few items, whose parts cost little, take the number that suits
-// lists which hold 60 %.
+// looks at the lists (a load of 16 cache lines, 0.3 to 0.5 us a launch).  Forward + backward, parts for lists that hold 60 % / for the
+// lists there are, 128-token blocks, 10 and 80 % kept: H1 S12800 138 / 98 and 327 / 328 us, H4 S1920 62.7 / 51.9 and 81.5 / 83.6, H2
+// S4096 74.2 / 65.5 and 110.0 / 108.8, H2 S1536 50.7 / 49.3 and 64.0 / 66.4.
 //
-// Lists that differ: whole items of a single round take as long as the longest list, parts about as long as a list that is 0.6 of the mean and 0.4
-// of the longest.  So the line for one round is drawn where  slope(1) longest - slope(parts) (0.6 mean + 0.4 longest)  reaches what the
-// parts cost besides.  Forward, decided by the mean / so: H1 S20480, 128-token blocks, Bernoulli masks of 10 % 56.5 / 45.8 us, densities that
-// rise ninefold along the sequence 74.1 / 50.9, causal H5 S4352 68.2 / 50.6.  So that such masks can be cut, launches of up to half a round
-// are planned too where lists of one length would have to hold more than 60 %, if lists that fall to nothing gain well; lists of one
-// length there pay 2 us for the look and a merge with nothing to do (H5 S4352, a quarter kept 22.1 -> 24.3 us; always cut they took 30.8).
-// Tile lists of 128 rows differ more than the halves that are worked on, so only half of what the longest is above the mean counts there (H2
-// S8192, 64-token blocks, 31 % kept, lists of 67 chunks and up to 73 for halves of 40 each).  dQ from dS is not judged by the longest list: it is bound by memory, which the short lists leave to the long ones (H3 S10240, 30 % kept,
+// Lists that differ: whole items of a single round take as long as the longest list, parts about as long as a list that is 0.6 of the mean
+// and 0.4 of the longest.  So the line for one round is drawn where  slope(1) longest - slope(parts) (0.6 mean + 0.4 longest)  reaches
+// what the parts cost besides.  Forward, decided by the mean / so: H1 S20480, 128-token blocks, Bernoulli masks of 10 % 56.5 / 45.8 us,
+// densities that rise ninefold along the sequence 74.1 / 50.9, causal H5 S4352 68.2 / 50.6.  So that such masks can be cut, launches of
+// up to half a round are planned too where lists of one length would have to hold more than 60 %, if lists that fall to nothing
+// gain well; lists of one length there pay 2 us for the look and a merge with nothing to do (H5 S4352, a quarter kept 22.1 -> 24.0 us;
+// always cut they took 30.8).  Tile lists of 128 rows differ more than the halves that are worked on, so only half of what the longest
+// is above the mean counts there (H2 S8192, 64-token blocks, 31 % kept, lists of 67 chunks and up to 73 for halves of 40 each).  dQ from
+// dS is not judged by the longest list: it is bound by memory, which the short lists leave to the long ones (H3 S10240, 30 % kept,
 // backward 182 -> 195 us).
 //
 // More than half a round is cut as well, in launches of less than one round, where work-groups end together: dK/dV of 136 tiles (H1
-// S17408), 30, 50 and 100 % kept, backward 227 -> 213, 350 -> 301 and 566 -> 496 us.  In a second round only where all the launch's lists are nearly
-// full and so nearly alike: with items in falling order of length the long ones make way for the short ones by themselves, and a chip that is not full
-// runs faster.  420 tiles (H3 S17920), 30, 70 and 100 % kept, whole / cut 474 / 503, 995 / 1001 and 1387 / 1340 us; 680 tiles (H8 S10880),
-// more than two rounds, 40 % kept 579 / 599.  Nor on tile lists, where
-// a part scans its lists twice: H8/4 S13824, 64 x 384 blocks, 44 % kept, dK/dV 401 -> 456 us.
+// S17408), 30, 50 and 100 % kept, backward 227 -> 213, 350 -> 301 and 566 -> 496 us.  In a second round only where all the launch's lists
+// are nearly full and so nearly alike: with items in falling order of length the long ones make way for the short ones by themselves,
+// and a chip that is not full runs faster.  420 tiles (H3 S17920), 30, 70 and 100 % kept, whole / cut 474 / 503, 995 / 1001 and 1387 /
+// 1340 us; 680 tiles (H8 S10880), more than two rounds, 40 % kept 579 / 599.  Nor on tile lists, where a part scans its lists twice: H8/4
+// S13824, 64 x 384 blocks, 44 % kept, dK/dV 401 -> 456 us.
 //
 // A part on a tile list scans the whole list before it takes its own steps: H5 S1536, 16 x 64 blocks, a third kept, dK/dV of 120 half
 // tiles of 27 steps 25.4 us whole, 22.4 us and a merge of 5.0 in two parts.
 constexpr double kMergeCost = 60;   // the launch
 constexpr double kScanCost = 40;    // and, on tile lists, the scans
 constexpr int64_t kNoteBytes = 16;  // behind the parts' results
-constexpr int kFewItems = 128;
+constexpr float kNever = 3e38f;     // entries
 SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
                      const ListLengths& lengths) {
   SplitPlan plan{};
@@ -108,7 +108,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
     }
   }
   if (n_hull == 1) return plan;
-  const bool device = rest > kFewItems && lengths.cnt != nullptr, one_round = device && num_items < slots && step.own_pace;
+  const bool device = lengths.cnt != nullptr, one_round = device && num_items < slots && step.own_pace;
   const double least = hull[1].least * (hull[0].slope - hull[1].slope);
   const bool uneven = one_round && 2 * rest <= slots && max_steps * (hull[0].slope - 0.5 * hull[1].slope) >= 2.5 * least;
   if (hull[1].least > 0.6 * max_steps && !uneven) return plan;  // lists of usual density stay whole
@@ -133,14 +133,14 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   look.stride = (int)(std::max<int64_t>(span - 4, 0) / 15);
   look.last = (int)(span - 1);
   look.step = (float)lengths.steps * lengths.group / (look.group > 1 ? 4 : 1);
-  const double by_longest = one_round ? (hull[0].slope - 0.4 * hull[1].slope) * (step.scans ? 0.5 : 1.) : 0.;
-  look.longest = (float)(by_longest * look.step);
-  look.sum = (float)((hull[0].slope - hull[1].slope - by_longest) * look.step / 64);
+  look.spread = !one_round ? 0.f : step.scans ? 0.5f : 1.f;
+  look.whole = (float)hull[0].slope * look.step;
+  look.cut = (float)hull[1].slope * look.step;
   look.least = (float)(hull[1].least * (hull[0].slope - hull[1].slope));
   look.fewest = hull[1].parts;
-  for (int& n : look.more) n = 0x7fffffff;
+  for (float& n : look.more) n = kNever;
   for (int i = 2; i < n_hull; ++i)
-    for (int n = hull[i - 1].parts + 1; n <= hull[i].parts; ++n) look.more[n - look.fewest - 1] = (int)std::ceil(hull[i].least * 64 / look.step);
+    for (int n = hull[i - 1].parts + 1; n <= hull[i].parts; ++n) look.more[n - look.fewest - 1] = (float)(hull[i].least / look.step);
   return plan;
 }
 

@@ -61,8 +61,8 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  * holds for a whole launch with fewer tiles than slots.  Entry points that take `split_ws` cut the lists of those tiles
  * into up to eight ranges, run each range in a work-group of its own at the end of the grid, store fp32 partial results
  * into split_ws and combine them in a small second launch, in a fixed order (results stay bit-reproducible).  How many ranges: the
- * device decides by the lengths of the lists where more than 128 tiles are left over; up to 128 the host decides, for lists that hold
- * 60 % of the longest possible ones.
+ * device decides by the lengths of the lists; dK/dV on tile lists and dQ in wide work-groups are planned by the host for lists that hold 60 % of
+ * the longest possible ones.
  *   split_ws        null (nothing is split), or 16-byte aligned device memory owned by the caller for the duration of
  *                   the call's work on the stream; its contents before and after are meaningless
  *   split_ws_bytes  its size; fba_split_workspace_bytes() is what the planner can use at most (a smaller buffer limits
@@ -79,12 +79,12 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
 int64_t fba_split_workspace_bytes(void);
 /*
  * What a launch on such sizes would cut, for tests and measurements (no GPU needed: 256 compute units are assumed then).  launch: 0 forward, 1 dK/dV,
- * 2 dQ that recomputes S and dP, 3 dQ from dS; the lists are those the block sizes need.  plan [15]:
+ * 2 dQ that recomputes S and dP, 3 dQ from dS; the lists are those the block sizes need.  plan [16]:
  *   0 tiles of the launch   1 first tile that is cut (that many: none)   2 most ranges of a tile's list
  *   3 1 where the device decides how many, up to that, by the lengths of the lists, 0 where it is that many whatever the lists; the rest only if 1
  *   4 offset in split_ws of the int32 in which the device leaves its decision
- *   5, 6, 7 lists are cut where plan[5] * (longest list) + plan[6] * (mean list) >= plan[7], lengths in steps
- *   8 into at least so many ranges   9.. and one more for each mean length among these that the mean reaches
+ *   5, 6, 7, 8 (thousandths) with L = mean + plan[5] (longest list - mean) and M = mean + 0.4 (L - mean), lengths in steps, lists are cut where
+ *   plan[6] L - plan[7] M >= plan[8]   9 into at least so many ranges   10.. and one more for each of these lengths that M reaches
  * A step is 32 keys (forward, dQ; 64 in forward on tile lists) or 32 query rows of one query head (dK/dV).
  */
 int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim,

@@ -31,7 +31,7 @@ def _mask(kind, shape, g):
 def test_last_round_of_the_split_case(Skv, cut):
     from flex_block_attn_amd import _lib
 
-    plan = (ctypes.c_int64 * 15)()
+    plan = (ctypes.c_int64 * 16)()
     _lib.call("fba_split_plan", 0, 30, 1, 30, 30, 1152, Skv, 128, 16, 64, _lib.load().fba_split_workspace_bytes(), plan)
     assert plan[0] == 540 and plan[1] == (512 if cut else 540) and (plan[2] > 1) == cut
 

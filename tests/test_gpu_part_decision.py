@@ -14,17 +14,19 @@ HEAD = 128
 def plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, ws_bytes=None):
     from flex_block_attn_amd import _lib
 
-    out = (ctypes.c_int64 * 15)()
+    out = (ctypes.c_int64 * 16)()
     n = _lib.load().fba_split_workspace_bytes() if ws_bytes is None else ws_bytes
     _lib.call("fba_split_plan", launch, 1 if dims == 2 else B * Hq, B, Hq, Hkv, Sq, Skv, HEAD, qbs, kbs, n, out)
-    return dict(zip(("items", "first", "parts", "device", "note", "longest", "mean", "least", "fewest"), out), more=list(out)[9:])
+    return dict(zip(("items", "first", "parts", "device", "note", "spread", "whole", "cut", "least", "fewest"), out), more=list(out)[10:])
 
 
 def decision(pl, length):
-    """(parts, how far off the line between one part and more, mean) for lists of these lengths."""
+    """(parts, how far off the line between one part and more, what the number of parts goes by) for lists of these lengths."""
     mean, longest = float(length.double().mean()), float(length.max())
-    gain = pl["longest"] * longest + pl["mean"] * mean
-    return pl["fewest"] + sum(mean >= n for n in pl["more"]) if gain >= pl["least"] else 1, gain / pl["least"] - 1, mean
+    whole = mean + pl["spread"] / 1000 * (longest - mean)
+    cut = mean + 0.4 * (whole - mean)
+    gain = pl["whole"] * whole - pl["cut"] * cut
+    return pl["fewest"] + sum(cut >= n for n in pl["more"]) if gain >= pl["least"] else 1, gain / pl["least"] - 1, cut
 
 
 def looked_at(pl, length):
@@ -76,6 +78,11 @@ CASES = [
     (FWD, 1, 3, 3, 8192, 17920, 8192, 128, 4, 0.6),              # three lists in all
     (FWD, 1, 3, 3, 8192, 17920, 4096, 128, 2, 0.6),              # two
     (DKDV, 1, 5, 1, 4096, 17408, 256, 17408, 4, 1.0),            # one list of five heads' each
+    (FWD, 1, 2, 2, 1536, 1536, 128, 128, 2, 0.2),                # 24 tiles
+    (FWD, 1, 6, 6, 384, 12288, 128, 128, 4, 0.9),
+    (DKDV, 1, 1, 1, 12800, 12800, 128, 128, 4, 0.05),            # 100 tiles
+    (DKDV, 1, 1, 1, 12800, 12800, 128, 128, 4, 0.7),
+    (DQ, 1, 1, 1, 12800, 12800, 128, 128, 2, "causal"),
     # lists of one round that differ: cut for the longest where the mean would not be
     (FWD, 1, 1, 1, 20480, 20480, 128, 128, 4, 0.1),
     (FWD, 1, 5, 5, 4352, 4352, 128, 128, 4, "causal"),
@@ -139,7 +146,7 @@ def test_the_device_decides_by_the_lists_it_cuts(gpu, launch, B, Hq, Hkv, Sq, Sk
 def test_the_cases_say_what_they_claim(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kind):
     """The device decides, and the mean length lies well off every line."""
     pl = plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims)
-    assert pl["device"] == 1 and pl["items"] - pl["first"] > 128 and pl["parts"] >= 2
+    assert pl["device"] == 1 and pl["parts"] >= 2
     m = mask_of(kind, B, Hq, Sq, Skv, qbs, kbs, dims, torch.Generator().manual_seed(Sq + Skv))
     length = steps(launch, m, B, Hq, Hkv, Sq, Skv, qbs, kbs)
     want, off, mean = decision(pl, looked_at(pl, length))
@@ -153,7 +160,7 @@ def test_the_longest_list_of_a_round_decides(launch, B, Hq, Hkv, Sq, Skv, qbs, k
     """Lists that fall to nothing are cut where lists of one length, as long as their mean, are not."""
     pl = plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, 4)
     most = Hq // Hkv * Sq // 32 if launch == DKDV else Skv // (64 if qbs < 128 else 32)
-    at = next(n for n in range(most) if (pl["longest"] + pl["mean"]) * n >= pl["least"])  # equal lists are cut from here on
+    at = next(n for n in range(most) if (pl["whole"] - pl["cut"]) * n >= pl["least"])  # equal lists are cut from here on
     falling = torch.linspace(0, min(most, 1.9 * at), 129)
     assert float(falling.mean()) < at and decision(pl, falling)[0] > 1
     assert decision(pl, falling * 0 + at - 1)[0] == 1 and decision(pl, falling * 0 + at)[0] > 1
@@ -163,7 +170,7 @@ def test_second_rounds_are_cut_where_lists_are_nearly_full():
     for Sq, Hkv in ((8192, 3), (17920, 3), (8192, 1)):
         pl = plan(DKDV, 1, 3, Hkv, Sq, 17920 * 3 // Hkv, 256, 128, 4)
         assert pl["items"] == 420 and pl["first"] == 256 and pl["parts"] == 3
-        assert 0.89 <= pl["least"] / pl["mean"] / ((3 // Hkv) * Sq / 32) <= 0.91
+        assert pl["spread"] == 0 and 0.89 <= pl["least"] / (pl["whole"] - pl["cut"]) / ((3 // Hkv) * Sq / 32) <= 0.91
 
 
 @pytest.mark.gpu

@@ -12,11 +12,11 @@ MAX_ABS, REL_L2 = 2e-2, 1e-2
 
 CASES = {
     # B, Hq, Hkv, Sq, Skv, qbs, kbs, dims: parts of forward, dK/dV, dQ, dQ from dS: "device" decides, the host, or nothing is cut
-    (1, 1, 1, 8192, 17408, 128, 128, 2): ("host", "device", "host", "host"),          # dK/dV 136 tiles: more than half a round
+    (1, 1, 1, 8192, 17408, 128, 128, 2): ("device", "device", "device", "device"),    # dK/dV 136 tiles: more than half a round
     (1, 5, 5, 4352, 4352, 128, 128, 4): ("device", None, "device", None),             # 170 items everywhere
     (1, 12, 3, 2304, 9216, 128, 384, 4): ("device", None, "device", None),            # 216 items everywhere
     (1, 3, 3, 8192, 17920, 256, 128, 4): ("device", "device", "device", "device"),    # dK/dV 420 tiles: a round and more than half
-    (1, 8, 1, 2048, 17408, 128, 128, 4): ("host", "device", "host", "host"),          # dK/dV 136 tiles, lists over eight heads
+    (1, 8, 1, 2048, 17408, 128, 128, 4): ("device", "device", "device", "device"),    # dK/dV 136 tiles, lists over eight heads
     (1, 3, 3, 2944, 2944, 64, 64, 4): (None, None, None, None),                       # tile lists, 138 items of 64 rows and of 64 keys
     (1, 5, 1, 6528, 8704, 16, 64, 4): (None, None, None, None),                       # 510 of 64 rows, 136 of 64 keys
     (1, 3, 3, 2944, 8192, 64, 64, 4): ("device", "host", None, None),                 # 138 of 64 rows, 384 of 64 keys
@@ -30,7 +30,7 @@ def test_what_is_cut(case):
 
     B, Hq, Hkv, Sq, Skv, qbs, kbs, dims = case
     for launch, want in enumerate(CASES[case]):
-        plan = (ctypes.c_int64 * 15)()
+        plan = (ctypes.c_int64 * 16)()
         _lib.call("fba_split_plan", launch, B * Hq if dims == 4 else 1, B, Hq, Hkv, Sq, Skv, 128, qbs, kbs, _lib.load().fba_split_workspace_bytes(), plan)
         cut = plan[1] < plan[0]
         assert cut == (plan[2] > 1) and (("device" if plan[3] else "host") if cut else None) == want, (launch, list(plan))
