@@ -141,8 +141,9 @@ FBA_DEVICE int wave_max(int x) {
 // How many parts every split item of a launch is cut into (see SplitPlan in fba_kernels.h): by 64 of the launch's lists, which every wave finds
 // alike.  All lanes of a wave call this together, with every wave of every part waiting for it, so it is short: one load, four neighbouring lists
 // to a cache line, and no division (64 lists far apart, each read four times, and four divisions: forward of H1 S10240, 64-token blocks, 40 % kept 38.6 us, of
-// H1 S16384, a quarter kept, 50.2; so 38.0 and 49.5).  kGroups: the lists of up to four query heads of a group add up, other heads from item to item.
-// kNever: for launches that the host always decides.
+// H1 S16384, a quarter kept, 50.2; so 38.0 and 49.5).  kGroups: the lists of up to four query heads of a group add up, other heads from item to item;
+// launches that take their items in falling order of length, which have more than a round, look at the lists of those they cut through that
+// order.  kNever: for launches that the host always decides.
 enum class Look { kNever, kSingle, kGroups };
 constexpr float kPartsSpread = 0.4f;  // how much of what the longest list is above the mean the parts of all lists take longer
 template <Look kLook, typename Plan>
@@ -150,8 +151,12 @@ FBA_DEVICE int split_parts(const Plan& plan) {
   const auto& l = plan.look;
   if (kLook == Look::kNever || l.cnt == nullptr) return plan.parts;
   const int lane = threadIdx.x & 63;
-  const int row = min((lane >> 2) * l.stride + (lane & 3), l.last);
+  int row = l.first + min((lane >> 2) * l.stride + (lane & 3), l.last);
   int n;
+  if (kLook == Look::kGroups && l.order != nullptr) {
+    row = l.order[plan.first + lane * plan.items / 64] / l.row_tiles;
+    if (l.shared) row %= l.rows_per_head;
+  }
   if (kLook == Look::kGroups && l.group > 1) {
     const int r = (lane * 5 & 63) * l.group / 64;
     const int32_t* const first = l.cnt + row + (int64_t)(row / l.rows_per_head) * (l.group - 1) * l.rows_per_head;  // of the group's first head

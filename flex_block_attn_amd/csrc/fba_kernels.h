@@ -34,8 +34,11 @@ constexpr int kMostParts = 8;  // of a split item
 // Which lists the device looks at, and the line in units of what it finds: n entries in a lane, one list or four of a group.
 struct ListLook {
   const int32_t* cnt;        // null: the plan's number of parts stands
-  int stride, last;          // rows 0..3, stride + 0..3, ... 15 stride + 0..3, none of them beyond the last one
-  int group, rows_per_head;  // see ListLengths; row numbers are those of one head of a group
+  int first, stride, last;   // rows first + 0..3, first + stride + 0..3, ... first + 15 stride + 0..3, none of them beyond first + last
+  int group, rows_per_head;  // see ListLengths; row numbers count one head of a group
+  // Where the split items are the last of an order of their own (dK/dV), their rows instead: item order[i] has row order[i] / row_tiles.  Else null.
+  const int32_t* order;
+  int row_tiles, shared;
   float step;                // steps of an entry
   // Whole items take as long as a list of  mean + spread (largest - mean)  entries, call it L, parts as long as one of  mean + 0.4 (L - mean).
   float spread, whole, cut, least;  // parts are made where whole * (the first) - cut * (the second) >= least,

@@ -123,11 +123,14 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   plan.ws = static_cast<float*>(ws);
   if (!device) return plan;
 
-  // The lists of the items that are split, or all of the launch's where these are taken in an order of their own (second rounds of dK/dV).
+  // The lists of the items that are split, or all of the launch's in second rounds more than half full (dK/dV), which have to be alike.
   ListLook& look = plan.look;
   const int64_t rows = (int64_t)num_items * lengths.tile_rows / lengths.list_rows, from = second ? 0 : (int64_t)plan.first * lengths.tile_rows / lengths.list_rows;
   const int64_t span = lengths.shared ? std::min<int64_t>(rows - from, lengths.rows_per_head) : rows - from;
-  look.cnt = lengths.cnt + (lengths.shared ? lengths.rows_per_head - span : from);
+  look.cnt = lengths.cnt;
+  look.first = (int)(lengths.shared ? lengths.rows_per_head - span : from);
+  look.row_tiles = std::max(lengths.list_rows / lengths.tile_rows, 1);
+  look.shared = lengths.shared;
   look.group = lengths.shared ? 1 : lengths.group;
   look.rows_per_head = lengths.rows_per_head;
   look.stride = (int)(std::max<int64_t>(span - 4, 0) / 15);
@@ -259,6 +262,7 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
     int32_t* const order = reinterpret_cast<int32_t*>(ws + top);
     hipLaunchKernelGGL(order_items_kernel, dim3(blocks), dim3(256), 0, stream, p, spans, segment, order);
     p.order = order;
+    if (2 * p.split.items <= slots) p.split.look.order = order;
   } else if (p.queue != nullptr) {
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(kQueueBytes / 4), 0, stream, p.queue);
   }

@@ -29,9 +29,15 @@ def decision(pl, length):
     return pl["fewest"] + sum(cut >= n for n in pl["more"]) if gain >= pl["least"] else 1, gain / pl["least"] - 1, cut
 
 
-def looked_at(pl, length):
-    """The lists that are cut; all of a launch with a second round, where those are the shortest."""
-    return length if pl["first"] and 2 * (pl["items"] - pl["first"]) > 256 and pl["items"] < 512 else length[pl["first"]:]
+def looked_at(pl, length, ordered):
+    """The lists that are cut, the shortest in dK/dV launches of more than a round with long lists; all lists of a second round more than half full."""
+    if pl["first"] and 2 * (pl["items"] - pl["first"]) > 256 and pl["items"] < 512:
+        return length
+    return (length.sort(descending=True).values if ordered else length)[pl["first"]:]
+
+
+def is_ordered(launch, pl, Hq, Hkv, Sq):
+    return launch == DKDV and 256 < pl["items"] <= 512 and Hq // Hkv * Sq // 32 >= 192
 
 
 def mask_of(kind, B, Hq, Sq, Skv, qbs, kbs, dims, g):
@@ -65,6 +71,11 @@ CASES = [
     (DKDV, 1, 3, 3, 8192, 17920, 256, 128, 4, "last head"),
     (DKDV, 1, 3, 3, 8192, 17920, 256, 128, 4, 1.0),
     (DKDV, 1, 3, 3, 8192, 17920, 256, 128, 4, 0.6),
+    (DKDV, 1, 5, 5, 8192, 7680, 256, 128, 4, "last head"),    # 44 beyond a round, in order of length: the shortest
+    (DKDV, 1, 2, 2, 8192, 18432, 256, 128, 4, "causal"),
+    (DKDV, 1, 2, 2, 8192, 18432, 256, 256, 2, "causal"),
+    (DKDV, 1, 9, 3, 2048, 12288, 128, 128, 4, "causal"),
+    (DKDV, 1, 16, 8, 1024, 8704, 128, 128, 4, "last head"),   # 32 beyond two rounds, in index order: the last kv head's
     (DKDV, 1, 1, 1, 8192, 17408, 128, 128, 2, "causal"),
     (DKDV, 1, 1, 1, 8192, 17408, 128, 128, 2, 0.04),
     (DKDV, 1, 8, 1, 2048, 17408, 128, 128, 4, 0.5),       # lists over eight heads
@@ -108,7 +119,7 @@ def test_the_device_decides_by_the_lists_it_cuts(gpu, launch, B, Hq, Hkv, Sq, Sk
     pl = plan(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims)
     length = steps(launch, m, B, Hq, Hkv, Sq, Skv, qbs, kbs)
     assert length.numel() == pl["items"]
-    want, _, mean = decision(pl, looked_at(pl, length))
+    want, _, mean = decision(pl, looked_at(pl, length, is_ordered(launch, pl, Hq, Hkv, Sq)))
     print(f"parts launch {launch} B{B} Hq{Hq} Hkv{Hkv} Sq{Sq} Skv{Skv} q{qbs} k{kbs} {kind}: {pl} mean {mean:.0f} -> {want}", flush=True)
     q, do = (torch.randn((B, Hq, Sq, HEAD), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
     k, v = (torch.randn((B, Hkv, Skv, HEAD), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
@@ -149,7 +160,7 @@ def test_the_cases_say_what_they_claim(launch, B, Hq, Hkv, Sq, Skv, qbs, kbs, di
     assert pl["device"] == 1 and pl["parts"] >= 2
     m = mask_of(kind, B, Hq, Sq, Skv, qbs, kbs, dims, torch.Generator().manual_seed(Sq + Skv))
     length = steps(launch, m, B, Hq, Hkv, Sq, Skv, qbs, kbs)
-    want, off, mean = decision(pl, looked_at(pl, length))
+    want, off, mean = decision(pl, looked_at(pl, length, is_ordered(launch, pl, Hq, Hkv, Sq)))
     assert abs(off) > 0.1, (off, mean, pl)
     assert want == 1 or all(not 0.85 * mean < n < 1.15 * mean for n in pl["more"]), (mean, pl)
 
