@@ -177,6 +177,14 @@ def test_the_longest_list_of_a_round_decides(launch, B, Hq, Hkv, Sq, Skv, qbs, k
     assert decision(pl, falling * 0 + at - 1)[0] == 1 and decision(pl, falling * 0 + at)[0] > 1
 
 
+@pytest.mark.parametrize("launch,H,S,parts", [(FWD, 24, 11520, 2), (FWD, 16, 8704, 4), (FWD, 24, 3072, 4), (DKDV, 8, 9216, 4)])
+def test_full_lists_behind_two_rounds_are_cut_like_usual_ones(launch, H, S, parts):
+    pl = plan(launch, 1, H, H, S, S, 128, 128, 4)
+    steps = torch.full((1,), S // 32)
+    assert decision(pl, steps)[0] == pl["parts"] == parts
+    assert pl["items"] < 1024 or decision(pl, (0.6 * steps).int())[0] == parts
+
+
 def test_second_rounds_are_cut_where_lists_are_nearly_full():
     for Sq, Hkv in ((8192, 3), (17920, 3), (8192, 1)):
         pl = plan(DKDV, 1, 3, Hkv, Sq, 17920 * 3 // Hkv, 256, 128, 4)
