@@ -87,7 +87,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   auto slope = [&](int n) {
     const int wgs = rest * n, alone = slots / wgs_per_cu;
     if (n == 1 && wgs <= alone && num_items >= 2 * slots) return step.few;  // items of the round before are still there
-    if (n == 1 && wgs <= alone) return step.alone * (1 + 0.15 * std::max(0, 2 * wgs - alone) / alone);  // a full chip runs at a lower clock
+    if (n == 1 && wgs <= alone) return step.alone * (1 + 0.15 * std::max(0, 2 * wgs - alone) / alone);  // a full chip runs at a lower clock: 240 items 0.59 us a step
     if (wgs <= alone) return step.alone / n;
     if (wgs <= slots) return (step.few + (step.full - step.few) * (wgs - alone) / (slots - alone)) / n;
     return step.full * ((wgs + slots - 1) / slots) / n;
