@@ -46,7 +46,8 @@ int device_compute_units() { return compute_units(); }
 // L is on the device: the host says from which lengths on which numbers of parts pay, up to the longest possible lists, and the kernel
 // looks at the lists (a load of 16 cache lines, 0.3 to 0.5 us a launch).  Forward + backward, parts for lists that hold 60 % / for the
 // lists there are, 128-token blocks, 10 and 80 % kept: H1 S12800 138 / 98 and 327 / 328 us, H4 S1920 62.7 / 51.9 and 81.5 / 83.6, H2
-// S4096 74.2 / 65.5 and 110.0 / 108.8, H2 S1536 50.7 / 49.3 and 64.0 / 66.4.
+// S4096 74.2 / 65.5 and 110.0 / 108.8, H2 S1536 50.7 / 49.3 and 64.0 / 66.4.  Behind a whole round: H24 S3072, 10 and 30 % kept, 160 / 140 and 240 / 230
+// us, H12 S3072 15 % 112.4 / 114.3 (lists just short of the line, of which the longest would have been worth cutting).
 //
 // Lists that differ: whole items of a single round take as long as the longest list, parts about as long as a list that is 0.6 of the mean
 // and 0.4 of the longest.  So the line for one round is drawn where  slope(1) longest - slope(parts) (0.6 mean + 0.4 longest)  reaches
