@@ -83,6 +83,36 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int kblk = (kt * TK) / p.k_block;
   const int64_t krow0 = (int64_t)bhk * p.Skv + (int64_t)kt * TK;
 
+  // What a work-group takes besides its slabs counts where lists are short: 23 us, of them 6.5 until the first slab's products, 10
+  // behind the last one until the halves are exchanged, 5 for the stores (timestamps in a copy of the kernel).  So the V and
+  // K rows are requested before the first look at the lists, which is a chain of scalar loads; what the walk over them reads first is
+  // requested together; and see `finish` below.  dK/dV, before / now: B2 H16 S8192, 128-token blocks, 8 and 16 of 64 kept 385 / 334
+  // and 617 / 577 us, B2 H16 S8448, 2 of 22 384-token blocks 356 / 302 us, H24 S30720, 32 of 80 8.78 / 8.58 ms.
+  //
+  // V tile into LDS: wave w brings in rows 32 w .. 32 w + 31 (two slabs' worth of copies)
+  {
+    const char* src = reinterpret_cast<const char*>(p.v) + (krow0 + 32 * wave) * kRowBytes;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const uint32_t dst = lds_addr(smem) + kTileBase + wave * kSlabBytes + j * 16 * kRowBytes;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int row = 4 * g + (lane >> 4);  // row inside the 16-row half; swz depends on row % 16 only
+        dma16(dst + g * 4 * kRowBytes, src + j * 16 * kRowBytes, (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4)));
+      }
+    }
+  }
+  // K rows of the wave's two key groups as B operands, in registers for the whole list: lane holds key l32 of the group,
+  // d = 16 ks + 8 h .. +7
+  bf16x8 kreg[2][8];
+  {
+    const __bf16* kp = p.k + (krow0 + 64 * kg + l32) * kHeadDim + 8 * h;
+#pragma unroll
+    for (int grp = 0; grp < 2; ++grp)
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks) kreg[grp][ks] = *reinterpret_cast<const bf16x8*>(kp + grp * 32 * kHeadDim + 16 * ks);
+  }
+
   const int nsub = p.q_block / kSlab;
   const int row_len = p.nQ;  // entries per list row
   auto list_row = [&](int g) -> int64_t {
@@ -90,8 +120,23 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     return (p.mask_bh == 1 ? 0 : bh) * p.nK + kblk;
   };
   const ConstIdx k_cnt = const_idx(p.k_cnt);
+  {  // what the walk over the lists will read first, requested together: it is then in the scalar cache
+    const int64_t lr = list_row(0);
+    int first = k_cnt[lr] ^ const_idx(p.k_idx + lr * row_len)[0];
+    if constexpr (kMode == kNumbered) {
+      const ConstIdx pb = const_idx(p.pair_base);
+      first ^= pb[lr] ^ pb[p.mask_bh * p.nK] ^ pb[p.nK] ^ pb[0];
+    }
+    asm volatile("" : : "s"(first));
+  }
   int slabs_all = 0;
-  for (int g = 0; g < group; ++g) slabs_all += k_cnt[list_row(g)];
+  for (int g = 0; g < group; g += 4) {  // four loads in flight
+    int n[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) n[i] = k_cnt[list_row(min(g + i, group - 1))];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) slabs_all += g + i < group ? n[i] : 0;
+  }
   slabs_all *= nsub;
   if constexpr (kMode == kNumbered) {
     // lists that number more pairs than the workspace holds: no slab is touched, nothing is stored into the workspace
@@ -149,30 +194,24 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 #pragma unroll
       for (int r = 0; r < 16; ++r) { acc_k[grp][mb][r] = 0.f; acc_v[grp][mb][r] = 0.f; }
 
-  if (nslabs > 0) {
-    // V tile into LDS: wave w brings in rows 32 w .. 32 w + 31 (two slabs' worth of copies)
-    {
-      const char* src = reinterpret_cast<const char*>(p.v) + (krow0 + 32 * wave) * kRowBytes;
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const uint32_t dst = lds0 + kTileBase + wave * kSlabBytes + j * 16 * kRowBytes;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int row = 4 * g + (lane >> 4);  // row inside the 16-row half; swz depends on row % 16 only
-          dma16(dst + g * 4 * kRowBytes, src + j * 16 * kRowBytes, (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4)));
-        }
-      }
+  if (nslabs == 0) {  // no query block selects this key tile, or the lists do not fit the workspace: zeros, or NaN
+    float value = 0.f;
+    wait_vmem<0>();  // no copy may still be writing LDS when the work-group gives it back
+    if constexpr (kMode == kNumbered) {
+      __syncthreads();
+      value *= *reinterpret_cast<volatile float*>(smem + kSmemBytes + 4);
     }
-    // K rows of the wave's two key groups as B operands, in registers for the whole list: lane holds key l32 of the group,
-    // d = 16 ks + 8 h .. +7
-    bf16x8 kreg[2][8];
-    {
-      const __bf16* kp = p.k + (krow0 + 64 * kg + l32) * kHeadDim + 8 * h;
-#pragma unroll
-      for (int grp = 0; grp < 2; ++grp)
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) kreg[grp][ks] = *reinterpret_cast<const bf16x8*>(kp + grp * 32 * kHeadDim + 16 * ks);
+    if (parts > 1) {
+      f32x4* out = reinterpret_cast<f32x4*>(p.split.ws + (int64_t)slot * (2 * TK * kHeadDim)) + tid;
+      for (int i = 0; i < 2 * TK * kHeadDim / 4 / 256; ++i) out[i * 256] = (f32x4){value, value, value, value};
+    } else {
+      const bf16x8 values = pack8(value, value, value, value, value, value, value, value);
+      bf16x8 *dk = reinterpret_cast<bf16x8*>(p.dk + krow0 * kHeadDim) + tid, *dv = reinterpret_cast<bf16x8*>(p.dv + krow0 * kHeadDim) + tid;
+      for (int i = 0; i < TK * kHeadDim / 8 / 256; ++i) dk[i * 256] = dv[i * 256] = values;
     }
+    return;
+  }
+  {
     // Cursor over (query head of the group, list entry, pair of slabs).  Slabs are numbered in list order; slabs 2i and 2i+1
     // form pair i, the first for the waves of parity 0, the second for those of parity 1.  A pair never straddles two query
     // blocks (q_block is a multiple of 128 and ranges start on multiples of four slabs), so the cursor moves a pair at a
@@ -276,6 +315,17 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     int64_t unit_nxt = unit_next + par * kDsUnitBytes;
     issue_copy(3 * par + 1, row_next + par * kSlab);
     advance();
+    // The compiler zeroes the accumulation registers where it likes, possibly right in front of the first matrix
+    // instruction that adds to them, and does not know that those instructions (inline asm) read them: every accumulator
+    // is pinned here, written, and a few wait states separate the writes from the first read.
+#pragma unroll
+    for (int grp = 0; grp < 2; ++grp)
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+        asm volatile("" : "+a"(acc_v[grp][mb]));
+        asm volatile("" : "+a"(acc_k[grp][mb]));
+      }
+    asm volatile("s_nop 7");
     wait_vmem<0>();
     __syncthreads();
     // a value of its own from here on: held in one register through the loop instead of being fetched back from the
@@ -405,7 +455,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     // slab (buffer at `po`, operands pk / dsk).  Eight groups of four
     // matrix instructions (one transposed dO operand and one transposed Q operand, each against both key groups) and four
     // accumulator elements of arithmetic; the operands and statistics of group n+1 are requested before group n starts.
-    auto softmax_and_accumulate = [&](auto in_c, int so, int po) {
+    auto softmax_and_accumulate = [&](auto in_c, auto arithmetic_c, int so, int po) {
+      constexpr bool kArithmetic = decltype(arithmetic_c)::value;  // false behind the last slab: only the accumulation is left
       constexpr int kIn = decltype(in_c)::value;  // set of the slab that is accumulated; the new P, dS go to the other
       bf16x2 pw[2][8], dw[2][8];  // new P and dS, packed: [key group][register pair]
       LdsPtr ts = t_base + po;
@@ -427,7 +478,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         if (n < 7) {
           adv_n = fetch_dv(n + 1);
           adk_n = fetch_dk(n + 1);
-          if (n >= 3) l4_n = lds_read_f32x4(st_ptr + so + 32 * ((n + 1) & 3));
+          if (kArithmetic && n >= 3) l4_n = lds_read_f32x4(st_ptr + so + 32 * ((n + 1) & 3));
         }
         __builtin_amdgcn_sched_barrier(0);
         const int j = n >> 2, mb = n & 3, grp = n >> 2, g = n & 3;
@@ -438,6 +489,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
           if (e == 1) mfma32_acc(acc_v[1][mb], adv, pk[kIn][1][j]);
           if (e == 2) mfma32_acc(acc_k[0][mb], adk, dsk[kIn][0][j]);
           if (e == 3) mfma32_acc(acc_k[1][mb], adk, dsk[kIn][1][j]);
+          if constexpr (!kArithmetic) continue;
           pv[e] = grp == 0 ? s[0][4 * g + e] : fast_exp2(__builtin_fmaf(s[1][4 * g + e], c, -l4[e]));
           dsv[e] = pv[e] * dp[grp][4 * g + e];
           if (e & 1) {
@@ -453,6 +505,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         __builtin_amdgcn_sched_barrier(0);
         adv = adv_n; adk = adk_n; l4 = l4_n;
       }
+      if constexpr (!kArithmetic) return;
 #pragma unroll
       for (int grp = 0; grp < 2; ++grp)
 #pragma unroll
@@ -486,7 +539,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     int cur = 0, prev = 0, nxt = kStageBytes;
     auto iteration = [&](auto in_c) {
       constexpr int kIn = decltype(in_c)::value;
-      softmax_and_accumulate(in_c, cur, prev);
+      softmax_and_accumulate(in_c, std::true_type{}, cur, prev);
       char* ds_unit = nullptr;  // where dS_t goes
       if constexpr (kHandOver) ds_unit = reinterpret_cast<char*>(p.ds_ws) + unit_cur;
       // slab t+2 will replace slab t-1 (past the end of the lists: a repeat of the last slab that nobody reads); its copies
@@ -508,24 +561,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       cur = nxt;
       nxt = freed;
     };
-    // The compiler zeroes the accumulation registers where it likes, possibly right in front of the first matrix
-    // instruction that adds to them, and does not know that those instructions (inline asm) read them: every accumulator
-    // is pinned here, written, and a few wait states separate the writes from the first read.
-#pragma unroll
-    for (int grp = 0; grp < 2; ++grp)
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        asm volatile("" : "+a"(acc_v[grp][mb]));
-        asm volatile("" : "+a"(acc_k[grp][mb]));
-      }
-    asm volatile("s_nop 7");
     iteration(IC<0>{});  // nlocal is even and at least 2: iterations 0 .. nlocal-2, an odd number of them
     for (int t = 1; t + 1 < nlocal; t += 2) {
       iteration(IC<1>{});
       iteration(IC<0>{});
     }
     // the wave's last slab (an odd one): no scores() follows that could carry its dS stores
-    softmax_and_accumulate(IC<1>{}, cur, prev);
+    softmax_and_accumulate(IC<1>{}, std::true_type{}, cur, prev);
     if constexpr (kHandOver) {
       char* ds_unit = reinterpret_cast<char*>(p.ds_ws) + unit_cur;
 #pragma unroll
@@ -534,73 +576,93 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         store16_stream_second(ds_unit + grp * 4 * kDsUnitBytes, ho_off0, dsk[0][grp][1]);
       }
     }
-    // ... and its share of dV, dK (the arithmetic of this call runs on stale registers and is dropped)
-    softmax_and_accumulate(IC<0>{}, nxt, cur);
-    wait_vmem<0>();
-    __syncthreads();  // no copy is writing LDS any more; V and the ring are free
+    // ... and its share of dV, dK
+    softmax_and_accumulate(IC<0>{}, std::false_type{}, nxt, cur);
+    wait_vmem<0>();  // no copy is writing LDS any more
 
     drain_matrix_pipe();
-    // The two waves of a key group swap halves: parity 1 hands its dV part to parity 0 through the first 64 KiB of LDS,
-    // parity 0 hands its dK part to parity 1 through the next 64 KiB (32 KiB per wave each).
-    f32x4* send = reinterpret_cast<f32x4*>(smem + (par ? 0 : 65536) + kg * 32768) + lane;
-    const f32x4* recv = reinterpret_cast<const f32x4*>(smem + (par ? 65536 : 0) + kg * 32768) + lane;
+    // read from here on only: what the compiler takes from an accumulator may not move in front of the idle cycles
 #pragma unroll
     for (int grp = 0; grp < 2; ++grp)
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x16& a = par ? acc_v[grp][mb] : acc_k[grp][mb];
-          send[((grp * 4 + mb) * 4 + g) * 64] = (f32x4){a[4 * g + 0], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
-        }
-    __syncthreads();
-#pragma unroll
-    for (int grp = 0; grp < 2; ++grp)
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x4 r = recv[((grp * 4 + mb) * 4 + g) * 64];
-          f32x16& a = par ? acc_k[grp][mb] : acc_v[grp][mb];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) a[4 * g + e] += r[e];
-        }
-  }
-
-  float poison = 1.f;
-  if constexpr (kMode == kNumbered) {
-    __syncthreads();
-    poison = *reinterpret_cast<volatile float*>(smem + kSmemBytes + 4);
-  }
-  if (parts > 1) {
-    // part of a split item: unscaled fp32 partial sums go to the workspace, dV tile (parity 0), then dK tile (parity 1)
-    float* prow = p.split.ws + (int64_t)slot * (2 * TK * kHeadDim) + par * (TK * kHeadDim) +
-                  (kg * 64 + l32) * kHeadDim;
-#pragma unroll
-    for (int grp = 0; grp < 2; ++grp)
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x16& a = par ? acc_k[grp][mb] : acc_v[grp][mb];
-          *reinterpret_cast<f32x4*>(prow + grp * 32 * kHeadDim + 32 * mb + 8 * g + 4 * h) =
-              (f32x4){a[4 * g + 0] * poison, a[4 * g + 1] * poison, a[4 * g + 2] * poison, a[4 * g + 3] * poison};
-        }
-    return;
-  }
-  // parity 0 writes dV, parity 1 writes dK (both zero when no query block selects this key tile)
-  __bf16* orow = (par ? p.dk : p.dv) + (krow0 + kg * 64 + l32) * kHeadDim;
-  const float oscale = (par ? p.scale : 1.f) * poison;
-#pragma unroll
-  for (int grp = 0; grp < 2; ++grp)
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& a = par ? acc_k[grp][mb] : acc_v[grp][mb];
-        *reinterpret_cast<bf16x4*>(orow + grp * 32 * kHeadDim + 32 * mb + 8 * g + 4 * h) =
-            pack4(a[4 * g + 0] * oscale, a[4 * g + 1] * oscale, a[4 * g + 2] * oscale, a[4 * g + 3] * oscale);
+      for (int mb = 0; mb < 4; ++mb) {
+        asm volatile("" : "+a"(acc_v[grp][mb]));
+        asm volatile("" : "+a"(acc_k[grp][mb]));
       }
+  }
+  __syncthreads();  // V and the ring are free
+
+  // The two waves of a key group swap halves: parity 1 hands its dV part to parity 0 through the first 64 KiB of LDS, parity 0
+  // hands its dK part to parity 1 through the next 64 KiB (32 KiB per wave each).  Then parity 0 writes dV and parity 1 dK, or, of a
+  // part of a split item, their fp32 partial sums.  Both go through the 32 KiB the wave has just read, so that a store fills whole
+  // lines: a lane holds pieces of one row, 8 bytes to each of 32 rows per store.  A branch
+  // for each parity, because an accumulator picked by value costs two reads and a select per element.
+  auto finish = [&](f32x16(&keep)[2][4], f32x16(&give)[2][4], __bf16* out, float oscale) {
+    // the lane's number, counted anew: whatever lives on from in front of the loop costs the loop a register
+    uint32_t zero;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero)), l32 = lane & 31, h = lane >> 5;
+    f32x4* const send = reinterpret_cast<f32x4*>(smem + (par ? 0 : 65536) + kg * 32768) + lane;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) {
+      const f32x16& a = give[i >> 4][(i >> 2) & 3];
+      const int g = i & 3;
+      send[i * 64] = (f32x4){a[4 * g + 0], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+      if (g == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    char* const own = smem + (par ? 65536 : 0) + kg * 32768;
+    float* const prow = p.split.ws + (int64_t)slot * (2 * TK * kHeadDim) + par * (TK * kHeadDim) + kg * 64 * kHeadDim;
+    __bf16* const orow = out + (krow0 + kg * 64) * kHeadDim;
+#pragma unroll
+    for (int grp = 0; grp < 2; ++grp) {  // 32 keys at a time, results in place of what was received
+      char* const half = own + grp * 16384;
+      const f32x4* recv = reinterpret_cast<const f32x4*>(half) + lane;
+#pragma unroll
+      for (int mb = 0; mb < 4; ++mb) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 r = recv[(mb * 4 + g) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) keep[grp][mb][4 * g + e] += r[e];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (parts > 1) {  // 32 rows of 512 bytes: 16-byte chunk c of row r at slot c ^ r
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) {
+          const f32x16& a = keep[grp][mb];
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<f32x4*>(half + l32 * 512 + (((8 * mb + 2 * g + h) ^ l32) << 4)) =
+                (f32x4){a[4 * g + 0] * oscale, a[4 * g + 1] * oscale, a[4 * g + 2] * oscale, a[4 * g + 3] * oscale};
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int row = 2 * i + h;
+          reinterpret_cast<f32x4*>(prow)[(grp * 16 + i) * 64 + lane] = *reinterpret_cast<const f32x4*>(half + row * 512 + ((l32 ^ row) << 4));
+        }
+      } else {
+#pragma unroll
+        for (int mb = 0; mb < 4; ++mb) {
+          const f32x16& a = keep[grp][mb];
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<bf16x4*>(half + tile_off(l32, 4 * mb + g) + 8 * h) =
+                pack4(a[4 * g + 0] * oscale, a[4 * g + 1] * oscale, a[4 * g + 2] * oscale, a[4 * g + 3] * oscale);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) reinterpret_cast<bf16x8*>(orow)[(grp * 8 + i) * 64 + lane] = lds_read_b128(half, tile_off(4 * i + (lane >> 4), lane & 15));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  float poison = 1.f;
+  if constexpr (kMode == kNumbered) poison = *reinterpret_cast<volatile float*>(smem + kSmemBytes + 4);
+  if (par) finish(acc_k, acc_v, p.dk, parts > 1 ? poison : p.scale * poison);
+  else finish(acc_v, acc_k, p.dv, poison);
 }
 
 hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
