@@ -40,6 +40,10 @@ using IC = std::integral_constant<int, N>;
 FBA_DEVICE void mfma32_acc(f32x16& acc, bf16x8 a, bf16x8 b) {
   asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
+// The same with nothing to add to: the accumulators need no zeroing (256 instructions of a wave alone on its SIMD).
+FBA_DEVICE void mfma32_acc_first(f32x16& acc, bf16x8 a, bf16x8 b) {
+  asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=a"(acc) : "v"(a), "v"(b));
+}
 // More idle cycles than any matrix instruction needs to retire its result.
 FBA_DEVICE void drain_matrix_pipe() { asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory"); }
 
@@ -78,8 +82,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int tiles_per_head = p.Skv / TK;
   const int bhk = item / tiles_per_head;
   const int kt = item - bhk * tiles_per_head;
-  const int b = bhk / p.Hkv, hkv = bhk - b * p.Hkv;
   const int group = p.Hq / p.Hkv;
+  const int64_t bh0 = (int64_t)bhk * group;  // first query head of the group, over all batches
   const int kblk = (kt * TK) / p.k_block;
   const int64_t krow0 = (int64_t)bhk * p.Skv + (int64_t)kt * TK;
 
@@ -116,18 +120,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int nsub = p.q_block / kSlab;
   const int row_len = p.nQ;  // entries per list row
   auto list_row = [&](int g) -> int64_t {
-    const int64_t bh = (int64_t)b * p.Hq + hkv * group + g;
-    return (p.mask_bh == 1 ? 0 : bh) * p.nK + kblk;
+    return (p.mask_bh == 1 ? 0 : bh0 + g) * p.nK + kblk;
   };
   const ConstIdx k_cnt = const_idx(p.k_cnt);
-  {  // what the walk over the lists will read first, requested together: it is then in the scalar cache
+  {
     const int64_t lr = list_row(0);
-    int first = k_cnt[lr] ^ const_idx(p.k_idx + lr * row_len)[0];
-    if constexpr (kMode == kNumbered) {
-      const ConstIdx pb = const_idx(p.pair_base);
-      first ^= pb[lr] ^ pb[p.mask_bh * p.nK] ^ pb[p.nK] ^ pb[0];
-    }
-    asm volatile("" : : "s"(first));
+    const ConstIdx pb = const_idx(kMode == kNumbered ? p.pair_base : p.k_cnt);
+    read_ahead(k_cnt[lr], const_idx(p.k_idx)[lr * row_len], pb[0], pb[kMode == kNumbered ? lr : 0], pb[kMode == kNumbered ? p.nK : 0],
+               pb[kMode == kNumbered ? p.mask_bh * p.nK : 0]);
   }
   int slabs_all = 0;
   for (int g = 0; g < group; g += 4) {  // four loads in flight
@@ -186,13 +186,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const uint32_t stat_off = (uint32_t)((lane >> 5) * rows_total * 4 + (lane & 31) * 4);
   const float c = p.scale_log2e;
 
-  f32x16 acc_k[2][4], acc_v[2][4];  // [32-key group][32 head-dim columns]
-#pragma unroll
-  for (int grp = 0; grp < 2; ++grp)
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) { acc_k[grp][mb][r] = 0.f; acc_v[grp][mb][r] = 0.f; }
+  f32x16 acc_k[2][4], acc_v[2][4];  // [32-key group][32 head-dim columns]; first written by the first slab's accumulation
 
   if (nslabs == 0) {  // no query block selects this key tile, or the lists do not fit the workspace: zeros, or NaN
     float value = 0.f;
@@ -238,7 +232,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       const int64_t lr = list_row(g);
       cnt_cur = k_cnt[lr];
       idx_cur = const_idx(p.k_idx + lr * row_len);
-      const int64_t bh = (int64_t)b * p.Hq + hkv * group + g;
+      const int64_t bh = bh0 + g;
       head_row0 = bh * p.Sq;
       if constexpr (kHandOver) {
         if constexpr (kMode == kDense) {
@@ -315,17 +309,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     int64_t unit_nxt = unit_next + par * kDsUnitBytes;
     issue_copy(3 * par + 1, row_next + par * kSlab);
     advance();
-    // The compiler zeroes the accumulation registers where it likes, possibly right in front of the first matrix
-    // instruction that adds to them, and does not know that those instructions (inline asm) read them: every accumulator
-    // is pinned here, written, and a few wait states separate the writes from the first read.
-#pragma unroll
-    for (int grp = 0; grp < 2; ++grp)
-#pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        asm volatile("" : "+a"(acc_v[grp][mb]));
-        asm volatile("" : "+a"(acc_k[grp][mb]));
-      }
-    asm volatile("s_nop 7");
     wait_vmem<0>();
     __syncthreads();
     // a value of its own from here on: held in one register through the loop instead of being fetched back from the
@@ -455,7 +438,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     // slab (buffer at `po`, operands pk / dsk).  Eight groups of four
     // matrix instructions (one transposed dO operand and one transposed Q operand, each against both key groups) and four
     // accumulator elements of arithmetic; the operands and statistics of group n+1 are requested before group n starts.
-    auto softmax_and_accumulate = [&](auto in_c, auto arithmetic_c, int so, int po) {
+    auto softmax_and_accumulate = [&](auto in_c, auto first_c, auto arithmetic_c, int so, int po) {
+      constexpr bool kFirst = decltype(first_c)::value;  // nothing has been accumulated yet
       constexpr bool kArithmetic = decltype(arithmetic_c)::value;  // false behind the last slab: only the accumulation is left
       constexpr int kIn = decltype(in_c)::value;  // set of the slab that is accumulated; the new P, dS go to the other
       bf16x2 pw[2][8], dw[2][8];  // new P and dS, packed: [key group][register pair]
@@ -483,12 +467,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         __builtin_amdgcn_sched_barrier(0);
         const int j = n >> 2, mb = n & 3, grp = n >> 2, g = n & 3;
         float pv[4], dsv[4];
+        auto accumulate = [&](f32x16& acc, bf16x8 a, bf16x8 b) {
+          if (kFirst && n < 4) mfma32_acc_first(acc, a, b);
+          else mfma32_acc(acc, a, b);
+        };
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          if (e == 0) mfma32_acc(acc_v[0][mb], adv, pk[kIn][0][j]);
-          if (e == 1) mfma32_acc(acc_v[1][mb], adv, pk[kIn][1][j]);
-          if (e == 2) mfma32_acc(acc_k[0][mb], adk, dsk[kIn][0][j]);
-          if (e == 3) mfma32_acc(acc_k[1][mb], adk, dsk[kIn][1][j]);
+          if (e == 0) accumulate(acc_v[0][mb], adv, pk[kIn][0][j]);
+          if (e == 1) accumulate(acc_v[1][mb], adv, pk[kIn][1][j]);
+          if (e == 2) accumulate(acc_k[0][mb], adk, dsk[kIn][0][j]);
+          if (e == 3) accumulate(acc_k[1][mb], adk, dsk[kIn][1][j]);
           if constexpr (!kArithmetic) continue;
           pv[e] = grp == 0 ? s[0][4 * g + e] : fast_exp2(__builtin_fmaf(s[1][4 * g + e], c, -l4[e]));
           dsv[e] = pv[e] * dp[grp][4 * g + e];
@@ -537,9 +525,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     // t % 2.  The first iteration adds nothing (P = dS = 0 against the finite rows of slab 0).  An iteration has no branch
     // but the cursor's change of block; the wave's last slab is handled behind the loop.
     int cur = 0, prev = 0, nxt = kStageBytes;
-    auto iteration = [&](auto in_c) {
+    auto iteration = [&](auto in_c, auto first_c) {
       constexpr int kIn = decltype(in_c)::value;
-      softmax_and_accumulate(in_c, std::true_type{}, cur, prev);
+      softmax_and_accumulate(in_c, first_c, std::true_type{}, cur, prev);
       char* ds_unit = nullptr;  // where dS_t goes
       if constexpr (kHandOver) ds_unit = reinterpret_cast<char*>(p.ds_ws) + unit_cur;
       // slab t+2 will replace slab t-1 (past the end of the lists: a repeat of the last slab that nobody reads); its copies
@@ -561,13 +549,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       cur = nxt;
       nxt = freed;
     };
-    iteration(IC<0>{});  // nlocal is even and at least 2: iterations 0 .. nlocal-2, an odd number of them
+    iteration(IC<0>{}, std::true_type{});  // nlocal is even and at least 2: iterations 0 .. nlocal-2, an odd number of them
     for (int t = 1; t + 1 < nlocal; t += 2) {
-      iteration(IC<1>{});
-      iteration(IC<0>{});
+      iteration(IC<1>{}, std::false_type{});
+      iteration(IC<0>{}, std::false_type{});
     }
     // the wave's last slab (an odd one): no scores() follows that could carry its dS stores
-    softmax_and_accumulate(IC<1>{}, std::true_type{}, cur, prev);
+    softmax_and_accumulate(IC<1>{}, std::false_type{}, std::true_type{}, cur, prev);
     if constexpr (kHandOver) {
       char* ds_unit = reinterpret_cast<char*>(p.ds_ws) + unit_cur;
 #pragma unroll
@@ -577,7 +565,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
       }
     }
     // ... and its share of dV, dK
-    softmax_and_accumulate(IC<0>{}, std::false_type{}, nxt, cur);
+    softmax_and_accumulate(IC<0>{}, std::false_type{}, std::false_type{}, nxt, cur);
     wait_vmem<0>();  // no copy is writing LDS any more
 
     drain_matrix_pipe();

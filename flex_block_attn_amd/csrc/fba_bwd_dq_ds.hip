@@ -71,8 +71,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const int n_kt = p.Skv / 128;
   const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (kTiled ? tiles_per_head : p.nQ) + (kTiled ? qt : qblk);
   constexpr bool dense = kMode == kDense;
+  {
+    const int32_t* const base = dense ? p.q_cnt : p.pair_base;
+    const int32_t* const slot_row = dense || kTiled ? p.q_cnt : p.q_slot + mrow * p.nK;
+    read_ahead(const_idx(p.q_cnt)[mrow], const_idx(p.q_idx)[mrow * p.nK], const_idx(slot_row)[0], const_idx(base)[0],
+               const_idx(base)[dense ? 0 : p.mask_bh * (kTiled ? n_kt : p.nK)]);
+  }
   // lists that number more pairs than the workspace holds: nothing is fetched, and the output becomes NaN
-  const int cnt = dense || workspace_holds_lists(p) ? p.q_cnt[mrow] : 0;
+  const int cnt = dense || workspace_holds_lists(p) ? const_idx(p.q_cnt)[mrow] : 0;
   const ConstIdx idx = const_idx(p.q_idx + mrow * p.nK);
   // block lists: pair number per list entry; tile lists: pair number per key tile, for this query tile
   const ConstIdx slots = const_idx(dense ? nullptr : p.q_slot + mrow * (kTiled ? n_kt : p.nK));
@@ -236,16 +242,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
             (f32x4){acc[mb][4 * g + 0] * poison, acc[mb][4 * g + 1] * poison, acc[mb][4 * g + 2] * poison, acc[mb][4 * g + 3] * poison};
     return;
   }
-  __bf16* orow = p.dq + (qrow0 + l32) * kHeadDim;
-  const float oscale = p.scale * poison;
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const bf16x4 ov = pack4(acc[mb][4 * g + 0] * oscale, acc[mb][4 * g + 1] * oscale, acc[mb][4 * g + 2] * oscale,
-                              acc[mb][4 * g + 3] * oscale);
-      *reinterpret_cast<bf16x4*>(orow + 32 * mb + 8 * g + 4 * h) = ov;
-    }
+  // (the ring is free: the last step ended with a barrier and requested nothing)
+  store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + qrow0 * kHeadDim, lane);
 }
 
 namespace {

@@ -150,8 +150,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const char* vp = reinterpret_cast<const char*>(p.v + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
 
   const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * p.nQ + (qt * TQ) / p.q_block;
-  const int cnt = p.q_cnt[mrow];
   const ConstIdx idx = const_idx(p.q_idx + mrow * p.nK);
+  const int cnt = const_idx(p.q_cnt)[mrow];
+  read_ahead(cnt, idx[0]);
   const int nsub = p.k_block / kSlab;
   // this work-group's range of 32-key steps of the list: all of it, or part `part` of `parts` (even boundaries)
   const int steps_all = cnt * nsub;
@@ -313,17 +314,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     return;
   }
   // epilogue: O = O^T / l, LSE = ln2 * (c m + log2 l)
-  __bf16* orow = p.o + (qrow0 + l32) * kHeadDim;
-  const float inv = l > 0.f ? 1.f / l : 0.f;
   if (h == 0) p.lse[qrow0 + l32] = l > 0.f ? (st.m_run * st.c + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const bf16x4 ov = pack4(st.acc_o[mb][4 * g + 0] * inv, st.acc_o[mb][4 * g + 1] * inv, st.acc_o[mb][4 * g + 2] * inv,
-                              st.acc_o[mb][4 * g + 3] * inv);
-      *reinterpret_cast<bf16x4*>(orow + 32 * mb + 8 * g + 4 * h) = ov;
-    }
+  __syncthreads();  // everybody is done with the rings, and no copy is on its way into them
+  store_tile_bf16(smem + wave * kSlabBytes, st.acc_o, l > 0.f ? 1.f / l : 0.f, p.o + qrow0 * kHeadDim, lane);
 }
 
 // Forward on tile lists (q_block or k_block no multiple of 128).
@@ -914,16 +907,16 @@ hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream) {
 
 hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   if (p.tiled) return launch_fwd_halves(p, stream);
-  constexpr int kSmem = 2 * kRing * kSlabBytes;
   const bool wide = p.q_block % 384 == 0 && p.variant != 1;
+  const int smem = (wide ? 12 : 2 * kRing) * kSlabBytes;  // the rings; the results of twelve waves
   void (*fn)(const FwdParams) = wide ? &fwd_kernel<12> : &fwd_kernel<4>;
   const int rows = wide ? 384 : 128;
   plan_fwd(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_wgs = (p.num_items - p.split.first) * p.split.parts;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs), dim3(rows * 2), kSmem, stream, p);
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs), dim3(rows * 2), smem, stream, p);
   if (split_wgs > 0) hipLaunchKernelGGL(fwd_merge_kernel<128>, dim3(merge_grid((p.num_items - p.split.first) * 16)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
