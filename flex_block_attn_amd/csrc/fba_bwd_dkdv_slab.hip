@@ -85,6 +85,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   const int64_t krow0 = (int64_t)bhk * p.Skv + (int64_t)kt * kTK;
   const int row_len = p.Sq / kSlab;  // entries per list row
   const int lists_per_head = p.Skv / 128;
+  {
+    const bool numbered = kHandOver && p.pair_base != nullptr;
+    const ConstIdx pb = const_idx(numbered ? p.pair_base : p.k_cnt);
+    read_ahead(const_idx(p.k_cnt)[(p.mask_bh == 1 ? 0 : (int64_t)b * p.Hq + hkv * group) * lists_per_head + (kt >> 1)], pb[0],
+               pb[numbered ? p.mask_bh * lists_per_head : 0]);
+  }
   // lists that number more pairs than the workspace holds: no slab is touched, and the outputs become NaN
   bool fits = true;
   if constexpr (kHandOver) fits = workspace_holds_lists(p);
@@ -125,16 +131,21 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
       const int64_t bh = (int64_t)b * p.Hq + hkv * group + scan_g;
       const int64_t lr = (p.mask_bh == 1 ? 0 : bh) * lists_per_head + (kt >> 1);
       const int cnt = const_idx(p.k_cnt)[lr];
+      // entries are asked for a round ahead, the first ones before the count is there
+      auto load = [&](const int32_t* x, int e) { return e < row_len ? x[lr * row_len + e] : 0; };
+      int ent_ahead = load(p.k_idx, scan_e + tid), pair_ahead = 0;
+      if constexpr (kHandOver) pair_ahead = p.pair_base != nullptr ? load(p.k_slot, scan_e + tid) : 0;
       while (scan_e < cnt) {
         if (n > kChapter - kRound || seen >= hi) return n;
         const int e = scan_e + tid;
-        const int ent = e < cnt ? p.k_idx[lr * row_len + e] : 0;
-        int pair = 0;
+        const int ent = e < cnt ? ent_ahead : 0;
+        int pair = pair_ahead;
+        ent_ahead = load(p.k_idx, e + kRound);
         if constexpr (kHandOver) {
           if (p.pair_base == nullptr) {  // dense numbering
             pair = (int)((bh * lists_per_head + (kt >> 1)) * (p.Sq / 128)) + (ent >> 10);
           } else {
-            pair = e < cnt ? p.k_slot[lr * row_len + e] : 0;
+            pair_ahead = load(p.k_slot, e + kRound);
             if (p.mask_bh == 1) pair += (int)(bh * const_idx(p.pair_base)[lists_per_head]);
           }
         }
@@ -326,70 +337,43 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   wait_vmem<0>();
   __syncthreads();
 
-  // The four waves of a key group add up their partial sums through LDS: positions 2 and 3 hand theirs to 0 and 1, then 1
-  // hands its dV part to 0 and 0 its dK part to 1 (32 KiB and 16 KiB per wave).
-  auto put = [&](const f32x16 (&a)[4], int base) {
-    f32x4* dst = reinterpret_cast<f32x4*>(smem + base) + lane;
+  // The four waves of a key group add up their partial sums through LDS, first of dV and then of dK: every wave puts its 32 x 128
+  // tile there (16 KiB, chunk c of row r at slot c ^ r, so that neither side meets bank conflicts) and thread t forms columns
+  // 8 (t % 16) .. +7 of rows t / 16 and t / 16 + 32, so that a store fills whole lines.  (Half of the waves adding what the others
+  // had put there, in three rounds, and stores of 8 bytes to 32 rows, before / now: B2 H16 S8192, 64-token blocks, 16 and 32 of 128
+  // kept 442 / 424 and 707 / 691 us.  What is left beside the slabs is 2 us for the claim, 6.2 to 6.7 until the first products, 4 here.)
+  const float poison = kHandOver ? poison_unless_fit(p) : 1.f;
+  auto finish = [&](const f32x16 (&a)[4], int which, __bf16* out, float oscale) {
+    f32x4* dst = reinterpret_cast<f32x4*>(smem + wave * 16384) + l32 * 32;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) dst[(mb * 4 + g) * 64] = (f32x4){a[mb][4 * g + 0], a[mb][4 * g + 1], a[mb][4 * g + 2], a[mb][4 * g + 3]};
-  };
-  auto take = [&](f32x16 (&a)[4], int base) {
-    const f32x4* src = reinterpret_cast<const f32x4*>(smem + base) + lane;
+      for (int g = 0; g < 4; ++g) dst[(8 * mb + 2 * g + h) ^ l32] = (f32x4){a[mb][4 * g + 0], a[mb][4 * g + 1], a[mb][4 * g + 2], a[mb][4 * g + 3]};
+    __syncthreads();
+    const int r = tid >> 4, c8 = 2 * (tid & 15);
+    float* const part_out = p.split.ws + (int64_t)slot * kSlotFloats + which * (kTK * kHeadDim);
 #pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
+    for (int k2 = 0; k2 < 2; ++k2) {  // the two key groups
+      f32x4 sum[2];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 r = src[(mb * 4 + g) * 64];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) a[mb][4 * g + e] += r[e];
+      for (int j = 0; j < 2; ++j) {
+        const f32x4* src = reinterpret_cast<const f32x4*>(smem + k2 * 16384) + r * 32 + ((c8 + j) ^ r);  // two waves to the next position
+        sum[j] = (src[0] + src[4 * 1024]) + (src[2 * 1024] + src[6 * 1024]);
+        sum[j] *= oscale;
       }
-  };
-  const int slot32 = ((par & 1) * 2 + kg) * 32768;
-  if (par >= 2) {
-    put(acc_v, slot32);
-    put(acc_k, slot32 + 16384);
-  }
-  __syncthreads();
-  if (par < 2) {
-    take(acc_v, slot32);
-    take(acc_k, slot32 + 16384);
-  }
-  __syncthreads();
-  if (par == 0) put(acc_k, kg * 16384);
-  if (par == 1) put(acc_v, 32768 + kg * 16384);
-  __syncthreads();
-  if (par >= 2) return;
-  if (par == 0) take(acc_v, 32768 + kg * 16384);
-  else take(acc_k, kg * 16384);
-
-  float poison = 1.f;
-  if constexpr (kHandOver) poison = poison_unless_fit(p);
-  if (parts > 1) {
-    // part of a split item: unscaled fp32 partial sums go to the workspace, dV rows (position 0), then dK rows (position 1)
-    float* prow = p.split.ws + (int64_t)slot * kSlotFloats + par * (kTK * kHeadDim) + (kg * 32 + l32) * kHeadDim;
-#pragma unroll
-    for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& a = par ? acc_k[mb] : acc_v[mb];
-        *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) =
-            (f32x4){a[4 * g + 0] * poison, a[4 * g + 1] * poison, a[4 * g + 2] * poison, a[4 * g + 3] * poison};
+      const int row = 32 * k2 + r;
+      if (parts > 1) {  // of a split item: fp32 partial sums, dV rows, then dK rows
+        *reinterpret_cast<f32x4*>(part_out + row * kHeadDim + 4 * c8) = sum[0];
+        *reinterpret_cast<f32x4*>(part_out + row * kHeadDim + 4 * c8 + 4) = sum[1];
+      } else {
+        *reinterpret_cast<bf16x8*>(out + (krow0 + row) * kHeadDim + 4 * c8) =
+            pack8(sum[0][0], sum[0][1], sum[0][2], sum[0][3], sum[1][0], sum[1][1], sum[1][2], sum[1][3]);
       }
-    return;
-  }
-  // position 0 writes dV, position 1 writes dK (both zero when no query block selects these keys)
-  __bf16* orow = (par ? p.dk : p.dv) + (krow0 + kg * 32 + l32) * kHeadDim;
-  const float oscale = (par ? p.scale : 1.f) * poison;
-#pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const f32x16& a = par ? acc_k[mb] : acc_v[mb];
-      *reinterpret_cast<bf16x4*>(orow + 32 * mb + 8 * g + 4 * h) =
-          pack4(a[4 * g + 0] * oscale, a[4 * g + 1] * oscale, a[4 * g + 2] * oscale, a[4 * g + 3] * oscale);
     }
+  };
+  finish(acc_v, 0, p.dv, poison);
+  __syncthreads();
+  finish(acc_k, 1, p.dk, parts > 1 ? poison : p.scale * poison);
 }
 
 hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
