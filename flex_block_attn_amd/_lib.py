@@ -34,7 +34,10 @@ SIGNATURES = {
     "fba_split_plan": (_c_i32, [_c_i32, _c_i64] + [_c_i32] * 8 + [_c_i64, _c_ptr]),
     "fba_fwd": (_c_i32, [_c_ptr] * 7 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_fwd_mask": (_c_i32, [_c_ptr] * 6 + [_c_i64] + [_c_i32] * 8 + [_c_ptr]),
+    "fba_fwd_mask_copy": (_c_i32, [_c_ptr] * 7 + [_c_i32, _c_i64] + [_c_i32] * 8 + [_c_ptr]),
     "fba_fwd_takes_mask": (_c_i32, [_c_i64, _c_i32]),
+    "fba_bwd_mask": (_c_i32, [_c_ptr] * 7 + [_c_i32, _c_i64] + [_c_ptr] * 3 + [_c_i32] * 8 + [_c_ptr]),
+    "fba_bwd_takes_mask": (_c_i32, [_c_i32] * 5),
     "fba_bwd": (_c_i32, [_c_ptr] * 14 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_probe_mfma": (_c_i32, [_c_ptr, _c_ptr, _c_i32, _c_i32, _c_ptr]),
     "fba_probe_read": (_c_i32, [_c_ptr, _c_i64, _c_ptr, _c_i32, _c_ptr]),
@@ -63,7 +66,7 @@ SIGNATURES = {
 }
 
 # fba_version() of the library these signatures describe (include/fba.h; bumped whenever an argument list changes)
-ABI_VERSION = 2006
+ABI_VERSION = 2007
 
 _lib = None
 _host = None

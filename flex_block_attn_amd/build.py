@@ -16,7 +16,7 @@ import sysconfig
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 LIB_NAME = "libfba_gfx950.so"
 LIB_PATH = os.path.join(CSRC, LIB_NAME)
-SOURCES = ["fba_api.hip", "fba_mask_compact.hip", "fba_ssta_mask.hip", "fba_fwd.hip", "fba_bwd_dq.hip", "fba_bwd_dq_ds.hip", "fba_bwd_dkdv.hip", "fba_bwd_dkdv64.hip", "fba_bwd_dkdv_slab.hip", "fba_probe.hip", "fba_split.hip"]
+SOURCES = ["fba_api.hip", "fba_mask_compact.hip", "fba_ssta_mask.hip", "fba_fwd.hip", "fba_bwd_dq.hip", "fba_bwd_dq_ds.hip", "fba_bwd_dkdv.hip", "fba_bwd_dkdv64.hip", "fba_bwd_dkdv_slab.hip", "fba_bwd_mask.hip", "fba_probe.hip", "fba_split.hip"]
 
 # Per-file extras.  --amdgpu-mfma-vgpr-form keeps MFMA accumulators in ordinary VGPRs, so the softmax arithmetic on
 # them needs no accumulator-register copies; it pays off where the whole working set fits 256 registers.
@@ -24,6 +24,7 @@ EXTRA_FLAGS = {
     "fba_fwd.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"],
     "fba_bwd_dq.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"],
     "fba_bwd_dq_ds.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"],
+    "fba_bwd_mask.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"],
     "fba_bwd_dkdv64.hip": ["-mllvm", "--amdgpu-mfma-vgpr-form"],
 }
 

@@ -165,8 +165,8 @@ int32_t fba_fwd_tiled(const void* q, const void* k, const void* v, void* o, floa
   return fwd_impl(q, k, v, o, lse, qt_cnt, qt_ent, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, true);
 }
 
-int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int64_t mask_bh, int32_t B, int32_t Hq,
-                     int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* hip_stream) {
+int32_t fba_fwd_mask_copy(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, uint8_t* mask_copy, int32_t o_rows,
+                          int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* hip_stream) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}})) return rc;
@@ -174,7 +174,8 @@ int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float
   if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
   fba::FwdMaskParams p{};
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.o = (__bf16*)o; p.lse = lse;
-  p.mask = mask; p.mask_bh = mask_bh;
+  if (o_rows < Sq || (int64_t)B * Hq * o_rows > 0x7fffffffLL) return fail(FBA_ERR_INVALID, "o_rows (%d) must be Sq (%d) or more, B*Hq*o_rows below 2^31", o_rows, Sq);
+  p.mask = mask; p.mask_copy = mask_copy; p.o_rows = o_rows; p.mask_bh = mask_bh;
   p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.Sq = Sq; p.Skv = Skv; p.nQ = Sq / q_block; p.nK = Skv / k_block;
   p.q_block = q_block; p.k_block = k_block;
   p.scale_log2e = 1.4426950408889634f / 11.313708498984761f;
@@ -182,7 +183,38 @@ int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float
   return e == hipSuccess ? FBA_OK : hip_fail(e, "forward (from the mask) launch");
 }
 
+int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int64_t mask_bh, int32_t B, int32_t Hq,
+                     int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* hip_stream) {
+  return fba_fwd_mask_copy(q, k, v, o, lse, mask, nullptr, Sq, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, hip_stream);
+}
+
 int32_t fba_fwd_takes_mask(int64_t rows, int32_t Skv) { return fba::fwd_takes_mask(rows, Skv) ? 1 : 0; }
+
+int32_t fba_bwd_mask(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, const uint8_t* mask, int32_t o_rows,
+                     int64_t mask_bh, void* dq, void* dk, void* dv, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
+                     int32_t k_block, void* hip_stream) {
+  const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
+  if (int rc = check_shape(s)) return rc;
+  if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}})) return rc;
+  if (!lse || !mask) return fail(FBA_ERR_INVALID, "null pointer argument");
+  if ((int64_t)B * Hq * Sq >= (1LL << 30) || (int64_t)B * Hkv * Skv >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq and B*Hkv*Skv must be below 2^30");
+  if (o_rows < Sq || (int64_t)B * Hq * o_rows > 0x7fffffffLL) return fail(FBA_ERR_INVALID, "o_rows (%d) must be Sq (%d) or more, B*Hq*o_rows below 2^31", o_rows, Sq);
+  fba::BwdMaskParams p{};
+  p.o_rows = o_rows;
+  p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.o = (const __bf16*)o; p.d_o = (const __bf16*)d_o; p.lse = lse;
+  p.dq = (__bf16*)dq; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv;
+  p.mask = mask; p.mask_bh = mask_bh;
+  p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.Sq = Sq; p.Skv = Skv; p.nQ = Sq / q_block; p.nK = Skv / k_block;
+  p.q_block = q_block; p.k_block = k_block;
+  p.scale = 1.f / 11.313708498984761f;
+  p.scale_log2e = 1.4426950408889634f / 11.313708498984761f;
+  hipError_t e = fba::launch_bwd_mask(p, (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "backward (from the mask) launch");
+}
+
+int32_t fba_bwd_takes_mask(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv) {
+  return fba::bwd_takes_mask((int64_t)B * Hq, (int64_t)B * Hkv, Sq, Skv) ? 1 : 0;
+}
 
 int32_t fba_block_mean(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, int32_t head_dim, void* hip_stream) {
   if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);

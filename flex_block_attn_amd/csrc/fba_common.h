@@ -448,6 +448,50 @@ FBA_DEVICE void store_tile_bf16(char* buf, const f32x16 (&acc)[4], float scale, 
     *reinterpret_cast<bf16x8*>(out + i * 4 * kHeadDim + lane * 8) = lds_read_b128(buf, tile_off(4 * i + (lane >> 4), lane & 15));
 }
 
+// The 32-key slabs that some row of the work-group selects, in order.  All lanes of a wave call everything together.
+template <bool kTwo>
+struct MaskCursor {
+  const uint8_t *row0, *row1;  // mask rows of the first and the last 16 query rows (the same unless kTwo)
+  int nK, nsub, lane;
+  int base, sub;               // first of the 64 key blocks at hand, slab inside the current block
+  int ahead0, ahead1;          // this lane's mask bytes of the 64 blocks that follow
+  unsigned long long m0, m1, left;  // ballots of the 64 blocks; those not passed yet, the current one lowest
+
+  FBA_DEVICE int load(const uint8_t* row, int at) const { return at + lane < nK ? row[at + lane] : 0; }
+  FBA_DEVICE void take() {
+    m0 = __builtin_amdgcn_ballot_w64(ahead0 != 0);
+    m1 = kTwo ? __builtin_amdgcn_ballot_w64(ahead1 != 0) : m0;
+    left = m0 | m1;
+    ahead0 = load(row0, base + 64);
+    if constexpr (kTwo) ahead1 = load(row1, base + 64);
+  }
+  FBA_DEVICE void start() {
+    base = sub = 0;
+    ahead0 = load(row0, 0);
+    ahead1 = kTwo ? load(row1, 0) : 0;
+    take();
+  }
+  // n slabs on; false past the last one
+  FBA_DEVICE bool skip(int n) {
+    sub += n;
+    for (;;) {
+      while (left == 0) {
+        base += 64;
+        if (base >= nK) return false;
+        take();
+      }
+      if (sub < nsub) return true;
+      sub -= nsub;
+      left &= left - 1;
+    }
+  }
+  FBA_DEVICE int slab() const { return (base + __builtin_ctzll(left)) * nsub + sub; }
+  FBA_DEVICE int halves() const {  // which 16-row halves select the current block
+    const int b = __builtin_ctzll(left);
+    return (int)((m0 >> b) & 1) | (int)((m1 >> b) & 1) << 1;
+  }
+};
+
 // dS hand-over between the key-major and the query-major backward kernel.  A "unit" is dS of one 32-query slab
 // against 32 keys, 2 KiB of bf16, cut into 256 slots of 8 bytes: slot (key, u) holds dS[4u .. 4u+3][key].  In the
 // key-major kernel lane (key = lane % 32, h = lane / 32) holds, as packed register chunk j, the slots u = 4j + h and

@@ -633,50 +633,6 @@ constexpr int kMaskRows = 32;
 constexpr int kMaskStatBase = kMaskWaves * 2 * kSlabBytes;                  // softmax references, then denominators [wave][row]
 constexpr int kMaskSmem = kMaskStatBase + 2 * kMaskWaves * kMaskRows * 4;
 
-// The 32-key slabs that some row of the work-group selects, in order.  All lanes of a wave call everything together.
-template <bool kTwo>
-struct MaskCursor {
-  const uint8_t *row0, *row1;  // mask rows of the first and the last 16 query rows (the same unless kTwo)
-  int nK, nsub, lane;
-  int base, sub;               // first of the 64 key blocks at hand, slab inside the current block
-  int ahead0, ahead1;          // this lane's mask bytes of the 64 blocks that follow
-  unsigned long long m0, m1, left;  // ballots of the 64 blocks; those not passed yet, the current one lowest
-
-  FBA_DEVICE int load(const uint8_t* row, int at) const { return at + lane < nK ? row[at + lane] : 0; }
-  FBA_DEVICE void take() {
-    m0 = __builtin_amdgcn_ballot_w64(ahead0 != 0);
-    m1 = kTwo ? __builtin_amdgcn_ballot_w64(ahead1 != 0) : m0;
-    left = m0 | m1;
-    ahead0 = load(row0, base + 64);
-    if constexpr (kTwo) ahead1 = load(row1, base + 64);
-  }
-  FBA_DEVICE void start() {
-    base = sub = 0;
-    ahead0 = load(row0, 0);
-    ahead1 = kTwo ? load(row1, 0) : 0;
-    take();
-  }
-  // n slabs on; false past the last one
-  FBA_DEVICE bool skip(int n) {
-    sub += n;
-    for (;;) {
-      while (left == 0) {
-        base += 64;
-        if (base >= nK) return false;
-        take();
-      }
-      if (sub < nsub) return true;
-      sub -= nsub;
-      left &= left - 1;
-    }
-  }
-  FBA_DEVICE int slab() const { return (base + __builtin_ctzll(left)) * nsub + sub; }
-  FBA_DEVICE int halves() const {  // which 16-row halves select the current block
-    const int b = __builtin_ctzll(left);
-    return (int)((m0 >> b) & 1) | (int)((m1 >> b) & 1) << 1;
-  }
-};
-
 template <bool kTwo>  // q_block is an odd multiple of 16: the two 16-row halves have mask rows of their own
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kMaskWaves, 64 * kMaskWaves), amdgpu_waves_per_eu(2, 2))) void fwd_mask_kernel(const FwdMaskParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // [wave](K slab | V slab), statistics
@@ -700,6 +656,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kMaskWaves, 64 * kMas
   cursor.nsub = p.k_block / kSlab;
   cursor.lane = lane;
   cursor.start();
+
+  if (p.mask_copy != nullptr && (p.mask_bh > 1 || bh == 0)) {  // the rows of the query blocks that begin here
+    const int64_t at = (p.mask_bh == 1 ? 0 : (int64_t)bh * p.nQ * p.nK);
+    for (int i = (row0 + p.q_block - 1) / p.q_block; i * p.q_block < min(row0 + kMaskRows, p.Sq); ++i)
+      for (int j = tid; j < p.nK; j += 64 * kMaskWaves) p.mask_copy[at + (int64_t)i * p.nK + j] = mask[(int64_t)i * p.nK + j];
+  }
 
   FwdState st;
   {
@@ -803,10 +765,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kMaskWaves, 64 * kMas
   }
   if (row0 + r >= p.Sq) return;
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  const int64_t orow = (int64_t)bh * p.Sq + row0 + r;
-  *reinterpret_cast<bf16x8*>(p.o + orow * kHeadDim + 4 * c8) =
+  *reinterpret_cast<bf16x8*>(p.o + ((int64_t)bh * p.o_rows + row0 + r) * kHeadDim + 4 * c8) =
       pack8(out[0][0] * inv, out[0][1] * inv, out[0][2] * inv, out[0][3] * inv, out[1][0] * inv, out[1][1] * inv, out[1][2] * inv, out[1][3] * inv);
-  if (c8 == 0) p.lse[orow] = l > 0.f ? (m * st.c + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
+  if (c8 == 0) p.lse[(int64_t)bh * p.Sq + row0 + r] = l > 0.f ? (m * st.c + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
 }
 
 // Combines the parts of the split items: O = sum_p 2^(m_p - m) O_p / sum_p 2^(m_p - m) l_p with m = max_p m_p, in part

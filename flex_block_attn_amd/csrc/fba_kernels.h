@@ -141,6 +141,27 @@ struct FwdMaskParams {
   int B, Hq, Hkv, Sq, Skv, nQ, nK, q_block, k_block;
   float scale_log2e;
   int num_items, items_per_xcd;
+  uint8_t* mask_copy;  // null, or where a copy of the mask goes
+  int o_rows;          // from a head of o to the next, Sq or more
+};
+
+// Backward straight from the block mask (bwd_mask_kernel).
+struct BwdMaskParams {
+  const __bf16* q;
+  const __bf16* k;
+  const __bf16* v;
+  const __bf16* o;
+  const __bf16* d_o;
+  const float* lse;
+  __bf16* dq;
+  __bf16* dk;
+  __bf16* dv;
+  const uint8_t* mask;
+  int64_t mask_bh;
+  int B, Hq, Hkv, Sq, Skv, nQ, nK, q_block, k_block;
+  int o_rows;  // from a head of o to the next
+  float scale, scale_log2e;
+  int key_items, key_wgs, key_per_xcd, query_items, query_per_xcd;  // key tiles, the work-groups for them, query tiles
 };
 
 struct BwdParams {
@@ -234,6 +255,8 @@ hipError_t launch_resize_mask(const uint8_t* src, uint8_t* dst, int64_t M, int s
 hipError_t launch_fwd(FwdParams p, hipStream_t stream);
 hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream);
 bool fwd_takes_mask(int64_t rows, int64_t kv_len);
+hipError_t launch_bwd_mask(BwdMaskParams p, hipStream_t stream);
+bool bwd_takes_mask(int64_t heads, int64_t kv_heads, int64_t q_len, int64_t kv_len);
 hipError_t launch_bwd_stats(const __bf16* o, const __bf16* d_o, const float* lse, float* stats, int64_t rows, hipStream_t stream);
 hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);

@@ -39,7 +39,7 @@ constexpr int64_t kXcds = 8;
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                \
   X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots) X(fba_tile_slots)        \
-  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask) X(fba_fwd_takes_mask) X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) \
+  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) \
   X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
@@ -202,13 +202,30 @@ std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor
 // Does forward read the block mask itself?  (Decided on the padded lengths, whether or not the call pads.)
 bool takes_mask(const Problem& p) { return lib.fba_fwd_takes_mask(p.B * p.Hq * p.Sq, p.Skv) != 0; }
 
-// Forward from the mask; q, k, v as the caller has them (lengths need not be whole tiles).
-std::pair<at::Tensor, at::Tensor> run_forward_on_mask(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask) {
-  at::Tensor o = at::empty_like(q);
+// Does backward, too?  Then neither pass builds lists, and nothing is padded.
+bool backward_takes_mask(const Problem& p) { return takes_mask(p) && lib.fba_bwd_takes_mask(p.B, p.Hq, p.Hkv, p.Sq, p.Skv) != 0; }
+
+// Forward from the mask; q, k, v as the caller has them (lengths need not be whole tiles).  mask_copy: null, or where a copy of the mask
+// goes.  o_rows: rows of a head of o, as many as q has or more.
+std::pair<at::Tensor, at::Tensor> run_forward_on_mask(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask,
+                                                      void* mask_copy = nullptr, int64_t o_rows = 0) {
+  o_rows = std::max(o_rows, q.size(2));
+  at::Tensor o = at::empty({p.B, p.Hq, o_rows, kHeadDim}, q.options());
   at::Tensor lse = at::empty({p.B, p.Hq, q.size(2), 1}, q.options().dtype(at::kFloat));
-  check(lib.fba_fwd_mask(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), static_cast<const uint8_t*>(mask.data_ptr()),
-                         p.mask_bh, p.B, p.Hq, p.Hkv, q.size(2), k.size(2), kHeadDim, p.q_block, p.k_block, current_stream(q)));
+  check(lib.fba_fwd_mask_copy(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), static_cast<const uint8_t*>(mask.data_ptr()),
+                              static_cast<uint8_t*>(mask_copy), o_rows, p.mask_bh, p.B, p.Hq, p.Hkv, q.size(2), k.size(2), kHeadDim, p.q_block, p.k_block,
+                              current_stream(q)));
   return {o, lse};
+}
+
+// Backward from the mask; p as forward had it.
+std::vector<at::Tensor> run_backward_on_mask(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o,
+                                             const at::Tensor& lse, const at::Tensor& d_o, const at::Tensor& mask) {
+  at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+  check(lib.fba_bwd_mask(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(),
+                         static_cast<const uint8_t*>(mask.data_ptr()), o.size(2), p.mask_bh, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), p.B, p.Hq, p.Hkv, q.size(2),
+                         k.size(2), kHeadDim, p.q_block, p.k_block, current_stream(q)));
+  return {dq, dk, dv};
 }
 
 enum class HandOver { kNever, kAuto, kWhole };  // dQ recomputes; as the limits allow; all heads at once whatever the size
@@ -299,9 +316,11 @@ struct Saved : torch::CustomClassHolder {
   Problem p;
   Lists lists;
   at::Tensor list_buffer, host_bounds;
+  bool from_mask = false;  // there are no lists: list_buffer holds a copy of the mask
+  int64_t o_rows = 0;      // and o has as many rows to a head as if there were
   c10::Event copied{c10::DeviceType::CUDA};
-  bool dense;
-  int64_t limit, split_bytes;
+  bool dense = false;
+  int64_t limit = 0, split_bytes;
   int64_t q_len, kv_len;  // of the caller's tensors; p describes the padded ones
   bool padded() const { return q_len != p.Sq || kv_len != p.Skv; }
   explicit Saved(const Problem& problem) : p(problem), lists(problem) {}
@@ -404,6 +423,16 @@ at::Tensor unpacked(const Saved& s, const char* name, const at::Tensor& t, at::I
 struct Attention : torch::autograd::Function<Attention> {
   static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask,
                             c10::intrusive_ptr<Saved> s) {
+    if (s->from_mask) {  // (the caller may write to the mask before backward comes)
+      s->list_buffer = at::empty({mask.numel()}, mask.options().dtype(at::kByte));
+      // Where lists would have padded the queries, o has the strides it has there.
+      const int64_t q_len = s->q_len;
+      auto [o, lse] = run_forward_on_mask(s->p, q, k, v, mask, s->list_buffer.data_ptr(), s->o_rows);
+      const bool cut = s->o_rows != q_len;
+      ctx->save_for_backward({q, k, v, o, lse});
+      ctx->saved_data["s"] = c10::IValue::make_capsule(std::move(s));
+      return cut ? o.narrow(2, 0, q_len).detach() : o;
+    }
     const Inputs in(q, k, v, mask, *s);
     build_lists(*s, in.mask, /*backward=*/true, /*numbered=*/!s->dense);
     auto [o, lse] = takes_mask(s->p) ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask) : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
@@ -422,11 +451,17 @@ struct Attention : torch::autograd::Function<Attention> {
     Saved& s = *static_cast<Saved*>(capsule.get());
     const c10::DeviceGuard guard(s.list_buffer.device());
     const Problem& p = s.p;
-    const int64_t q_shape[4] = {p.B, p.Hq, p.Sq, kHeadDim}, kv_shape[4] = {p.B, p.Hkv, p.Skv, kHeadDim}, lse_shape[4] = {p.B, p.Hq, p.Sq, 1};
+    const int64_t q_shape[4] = {p.B, p.Hq, p.Sq, kHeadDim}, o_shape[4] = {p.B, p.Hq, s.from_mask ? s.o_rows : p.Sq, kHeadDim},
+                  kv_shape[4] = {p.B, p.Hkv, p.Skv, kHeadDim}, lse_shape[4] = {p.B, p.Hq, p.Sq, 1};
     const at::Tensor q = unpacked(s, "q", saved[0], q_shape, at::kBFloat16, false), k = unpacked(s, "k", saved[1], kv_shape, at::kBFloat16, false),
-                     v = unpacked(s, "v", saved[2], kv_shape, at::kBFloat16, false), o = unpacked(s, "o", saved[3], q_shape, at::kBFloat16, true),
+                     v = unpacked(s, "v", saved[2], kv_shape, at::kBFloat16, false), o = unpacked(s, "o", saved[3], o_shape, at::kBFloat16, true),
                      lse = unpacked(s, "lse", saved[4], lse_shape, at::kFloat, true);
     at::Tensor d_o = grads[0].to(at::kBFloat16).contiguous();
+    if (s.from_mask) {
+      if (s.o_rows != p.Sq && (reinterpret_cast<uintptr_t>(d_o.data_ptr()) & 15) != 0) d_o = d_o.clone();  // as below
+      const auto g = run_backward_on_mask(p, q, k, v, o, lse, d_o, s.list_buffer);
+      return {g[0], g[1], g[2], at::Tensor(), at::Tensor()};
+    }
     if (s.q_len != p.Sq) {
       if ((reinterpret_cast<uintptr_t>(d_o.data_ptr()) & 15) != 0) d_o = d_o.clone();  // the copy moves 16 bytes at a time
       d_o = resized({{d_o, p.Sq}})[0];
@@ -487,8 +522,15 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
     const at::Tensor o = run_forward(p, in.q, in.k, in.v, s->lists, split_bytes).first;
     return s->padded() ? o.narrow(2, 0, q_len) : o;
   }
-  s->limit = ds_limit(p, limit, factor);
-  s->dense = dense_fits(p.dense_bytes(), s->limit);
+  if (backward_takes_mask(p)) {
+    s->from_mask = true;
+    s->o_rows = p.Sq;
+    s->p.Sq = q_len;
+    s->p.Skv = kv_len;
+  } else {
+    s->limit = ds_limit(p, limit, factor);
+    s->dense = dense_fits(p.dense_bytes(), s->limit);
+  }
   return Attention::apply(q, k, v, mask, std::move(s));
 }
 
@@ -539,6 +581,17 @@ c10::optional<std::pair<at::Tensor, at::Tensor>> forward_on_mask(const at::Tenso
   return run_forward_on_mask(p, q, k, v, mask);
 }
 
+// For the Python autograd function: is backward to take the mask, too?  If so, forward_on_mask comes before it.
+bool backward_takes_mask_of(const at::Tensor& q, const at::Tensor& k, int64_t q_block, int64_t k_block) {
+  const c10::DeviceGuard guard(q.device());
+  return backward_takes_mask(problem_of(q, k, q_block, k_block, 1));
+}
+std::vector<at::Tensor> backward_on_mask(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& lse,
+                                         const at::Tensor& d_o, int64_t q_block, int64_t k_block, const at::Tensor& mask) {
+  const c10::DeviceGuard guard(q.device());
+  return run_backward_on_mask(problem_of(q, k, q_block, k_block, mask.dim() == 2 ? 1 : q.size(0) * q.size(1)), q, k, v, o, lse, d_o, mask);
+}
+
 std::vector<at::Tensor> backward_on_lists(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o, const at::Tensor& lse,
                                           const at::Tensor& d_o, int64_t q_block, int64_t k_block, int64_t mask_bh, const at::Tensor& q_cnt,
                                           const at::Tensor& q_idx, const at::Tensor& k_cnt, const at::Tensor& k_idx,
@@ -569,5 +622,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attention", &attention_of);
   m.def("forward", &forward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("forward_on_mask", &forward_on_mask, pybind11::call_guard<pybind11::gil_scoped_release>());
+  m.def("backward_takes_mask", &backward_takes_mask_of);
+  m.def("backward_on_mask", &backward_on_mask, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("backward", &backward_on_lists, pybind11::call_guard<pybind11::gil_scoped_release>());
 }

@@ -264,6 +264,34 @@ def _forward(q, k, v, q_block_size, kv_block_size, block_mask, lists):
     return forward_with_lists(q, k, v, q_block_size, kv_block_size, lists) if got is None else (_typed_like(got[0], q), got[1])
 
 
+def _backward_takes_mask(q, k, v, q_block_size, kv_block_size, block_mask):
+    """Whether neither pass needs lists (small problems, as the native call decides).  A mask that lists could not be made of is left to them."""
+    if block_mask.dtype != torch.bool or not block_mask.is_cuda or block_mask.device != q.device or block_mask.numel() == 0:
+        return False
+    _check_qkv(q, k, v)
+    return q.numel() > 0 and k.numel() > 0 and _lib.host().backward_takes_mask(q, k, q_block_size, kv_block_size)
+
+
+def _backward_inputs(q, o, lse, do):
+    """o, lse and dO of a backward pass as the kernels take them."""
+    if do.dtype != torch.bfloat16:
+        do = do.to(torch.bfloat16)
+    do = do.contiguous()
+    o = o.contiguous()
+    if o.shape != q.shape or do.shape != q.shape:
+        raise ValueError("o and do must have the shape of q")
+    if lse.dtype != torch.float32 or lse.numel() != q.shape[0] * q.shape[1] * q.shape[2]:
+        raise ValueError("lse must be float32 with B*H*Sq elements")
+    return o, lse.contiguous(), do
+
+
+def _backward_on_mask(q, k, v, o, lse, do, q_block_size, kv_block_size, mask):
+    _check_qkv(q, k, v)
+    o, lse, do = _backward_inputs(q, o, lse, do)
+    grads = _lib.host().backward_on_mask(q, k, v, o, lse, do, q_block_size, kv_block_size, mask)
+    return tuple(_typed_like(g, t) for g, t in zip(grads, (q, k, v)))
+
+
 def number_pairs(lists):
     """Pair numbering for the dS hand-over, kept on `lists`: block pairs of block lists (fba_pair_slots), pairs of
     128-row tiles of tile lists (fba_tile_slots).  The number of listed pairs, which sizes the workspace, is copied to
@@ -357,15 +385,7 @@ def backward_with_lists(q, k, v, o, lse, do, q_block_size, kv_block_size, lists,
     fba_bwd_tiled_handover in one call).  False: dQ recomputes S and dP (fba_bwd or fba_bwd_tiled, no workspace)."""
     B, Hq, Hkv, Sq, Skv = _check_qkv(q, k, v)
     _check_lists(lists, q, B, Hq, Sq, Skv, q_block_size, kv_block_size)
-    if do.dtype != torch.bfloat16:
-        do = do.to(torch.bfloat16)
-    do = do.contiguous()
-    o = o.contiguous()
-    if o.shape != q.shape or do.shape != q.shape:
-        raise ValueError("o and do must have the shape of q")
-    if lse.dtype != torch.float32 or lse.numel() != B * Hq * Sq:
-        raise ValueError("lse must be float32 with B*H*Sq elements")
-    lse = lse.contiguous()
+    o, lse, do = _backward_inputs(q, o, lse, do)
     dense = hand_over is None and lists.pair_base is None and dense_ds_fits(q, k)
     bounds = [] if dense or hand_over is False else number_pairs(lists).pair_bounds()
     grads = _lib.host().backward(q, k, v, o, lse, do, q_block_size, kv_block_size, lists.mask_bh, lists.q_cnt, lists.q_idx, lists.k_cnt, lists.k_idx,
@@ -403,6 +423,15 @@ class FlexBlockAttnFunc(torch.autograd.Function):
     def forward(ctx, q, k, v, q_block_size, kv_block_size, block_mask, is_grad_enabled):
         _check_blocks(q, k, q_block_size, kv_block_size, block_mask)
         is_grad = is_grad_enabled and any(x.requires_grad for x in [q, k, v])
+        if is_grad and _backward_takes_mask(q, k, v, q_block_size, kv_block_size, block_mask):
+            mask = block_mask.contiguous().clone()  # the caller may write to theirs before backward comes
+            o, lse = _lib.host().forward_on_mask(q, k, v, q_block_size, kv_block_size, mask)
+            o = _typed_like(o, q)
+            ctx.save_for_backward(q, k, v, o, lse)
+            ctx.q_block_size = q_block_size
+            ctx.kv_block_size = kv_block_size
+            ctx.lists, ctx.mask = None, mask
+            return o
         lists = lists_for(block_mask, q_block_size, kv_block_size, with_pair_numbers=is_grad and not dense_ds_fits(q, k))
         o, lse = _forward(q, k, v, q_block_size, kv_block_size, block_mask, lists)
         if is_grad:
@@ -415,6 +444,8 @@ class FlexBlockAttnFunc(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout, *args):
         q, k, v, o, lse = ctx.saved_tensors
+        if ctx.lists is None:
+            return *_backward_on_mask(q, k, v, o, lse, dout, ctx.q_block_size, ctx.kv_block_size, ctx.mask), None, None, None, None
         dq, dk, dv = backward_with_lists(q, k, v, o, lse, dout, ctx.q_block_size, ctx.kv_block_size, ctx.lists)
         return dq, dk, dv, None, None, None, None
 

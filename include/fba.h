@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2006
+#define FBA_VERSION 2007
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -109,8 +109,24 @@ int32_t fba_fwd(const void* q, const void* k, const void* v, void* o, float* lse
 int32_t fba_fwd_mask(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int64_t mask_bh, int32_t B,
                      int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block,
                      void* hip_stream);
+/* The same, leaving a copy of the mask in mask_copy (as large as mask; null: none), for a backward pass that comes when the caller may have
+ * written to the mask.  o_rows: rows from a head of o to the next, Sq or more. */
+int32_t fba_fwd_mask_copy(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, uint8_t* mask_copy,
+                          int32_t o_rows, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
+                          int32_t k_block, void* hip_stream);
 /* 1 where it is the faster one for rows = B * Hq * Sq query rows on the current device (both work for every size). */
 int32_t fba_fwd_takes_mask(int64_t rows, int32_t Skv);
+
+/*
+ * Backward straight from the block mask, in one launch and without a workspace, for problems too small to fill the GPU.  mask as for
+ * fba_fwd_mask; o (o_rows rows from a head to the next) and lse as forward wrote them; any block sizes and lengths the operator takes.  dq, dk, dv as fba_bwd writes them, up to
+ * the order of fp32 sums.
+ */
+int32_t fba_bwd_mask(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, const uint8_t* mask,
+                     int32_t o_rows, int64_t mask_bh, void* dq, void* dk, void* dv, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv,
+                     int32_t head_dim, int32_t q_block, int32_t k_block, void* hip_stream);
+/* 1 where it is the faster one on the current device (both work for every size). */
+int32_t fba_bwd_takes_mask(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv);
 
 /*
  * Backward, three stream-ordered launches.  Replaces attn_backward (attn.cpp:30,
