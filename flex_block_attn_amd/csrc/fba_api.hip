@@ -373,7 +373,7 @@ int32_t fba_bwd_stats(const void* o, const void* d_o, const float* lse, float* s
   if (rows < 0 || rows >= (1LL << 30)) return fail(FBA_ERR_INVALID, "rows must be in [0, 2^30)");
   if (int rc = check_ptrs({{"o", o}, {"d_o", d_o}})) return rc;
   if (!lse || !stats) return fail(FBA_ERR_INVALID, "null pointer argument");
-  hipError_t e = fba::launch_bwd_stats((const __bf16*)o, (const __bf16*)d_o, lse, stats, rows, (hipStream_t)hip_stream);
+  hipError_t e = fba::launch_bwd_stats({(const __bf16*)o, (const __bf16*)d_o, lse, stats, rows}, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "stats launch");
 }
 
@@ -400,7 +400,7 @@ static int dq_impl(const void* q, const void* k, const void* v, const void* d_o,
 static int dkdv_impl(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dk, void* dv,
                      const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv,
                      int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
-                     void* hip_stream, bool tiled) {
+                     void* hip_stream, bool tiled, const fba::BwdStats& make) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"d_o", d_o}, {"dk", dk}, {"dv", dv}})) return rc;
@@ -412,7 +412,7 @@ static int dkdv_impl(const void* q, const void* k, const void* v, const void* d_
   fill_bwd(p, s);
   p.tiled = tiled ? 1 : 0;
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
-  p.stats = stats; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv; p.k_cnt = k_cnt; p.k_idx = k_idx;
+  p.stats = stats; p.make = make; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv; p.k_cnt = k_cnt; p.k_idx = k_idx;
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
   hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dkdv launch");
@@ -431,9 +431,8 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}})) return rc;
   if (!lse || !stats || !q_cnt || !q_idx || !k_cnt || !k_idx) return fail(FBA_ERR_INVALID, "null pointer argument");
   if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
-  if (int rc = fba_bwd_stats(o, d_o, lse, stats, (int64_t)B * Hq * Sq, head_dim, hip_stream)) return rc;
   if (int rc = dkdv_impl(q, k, v, d_o, stats, dk, dv, k_cnt, k_idx, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block,
-                         split_ws, split_ws_bytes, hip_stream, tiled))
+                         split_ws, split_ws_bytes, hip_stream, tiled, {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq}))
     return rc;
   return dq_impl(q, k, v, d_o, stats, dq, q_cnt, q_idx, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes,
                  hip_stream, tiled);
@@ -452,7 +451,7 @@ int32_t fba_bwd_dkdv(const void* q, const void* k, const void* v, const void* d_
                      int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
                      void* hip_stream) {
   return dkdv_impl(q, k, v, d_o, stats, dk, dv, k_cnt, k_idx, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws,
-                   split_ws_bytes, hip_stream, false);
+                   split_ws_bytes, hip_stream, false, {});
 }
 
 int32_t fba_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
@@ -503,11 +502,11 @@ static int check_handover(const Shape& s, const void* ds_ws, int64_t ds_ws_bytes
   return FBA_OK;
 }
 
-int32_t fba_bwd_dkdv_handover(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dk, void* dv,
+static int dkdv_handover_impl(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dk, void* dv,
                               void* ds_ws, int64_t ds_ws_bytes, const int32_t* k_cnt, const int32_t* k_idx, const int32_t* pair_base,
                               int64_t n_pairs, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv,
                               int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
-                              void* hip_stream) {
+                              void* hip_stream, const fba::BwdStats& make) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_handover(s, ds_ws, ds_ws_bytes, pair_base, n_pairs, "dkdv")) return rc;
@@ -518,12 +517,21 @@ int32_t fba_bwd_dkdv_handover(const void* q, const void* k, const void* v, const
   fba::BwdParams p{};
   fill_bwd(p, s);
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
-  p.stats = stats; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv; p.k_cnt = k_cnt; p.k_idx = k_idx;
+  p.stats = stats; p.make = make; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv; p.k_cnt = k_cnt; p.k_idx = k_idx;
   p.ds_ws = (__bf16*)ds_ws; p.pair_base = pair_base;
   p.ws_pairs = ds_ws_bytes / ((int64_t)q_block * k_block * 2);
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
   hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dkdv (hand-over) launch");
+}
+
+int32_t fba_bwd_dkdv_handover(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dk, void* dv,
+                              void* ds_ws, int64_t ds_ws_bytes, const int32_t* k_cnt, const int32_t* k_idx, const int32_t* pair_base,
+                              int64_t n_pairs, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv,
+                              int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
+                              void* hip_stream) {
+  return dkdv_handover_impl(q, k, v, d_o, stats, dk, dv, ds_ws, ds_ws_bytes, k_cnt, k_idx, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim,
+                            q_block, k_block, split_ws, split_ws_bytes, hip_stream, {});
 }
 
 int32_t fba_bwd_dq_from_ds(const void* k, const void* ds_ws, int64_t ds_ws_bytes, void* dq, const int32_t* q_cnt, const int32_t* q_idx,
@@ -559,9 +567,8 @@ int32_t fba_bwd_handover(const void* q, const void* k, const void* v, const void
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}})) return rc;
   if (!lse || !stats || !q_cnt || !q_idx || !k_cnt || !k_idx || !q_slot) return fail(FBA_ERR_INVALID, "null pointer argument");
   if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
-  if (int rc = fba_bwd_stats(o, d_o, lse, stats, (int64_t)B * Hq * Sq, head_dim, hip_stream)) return rc;
-  if (int rc = fba_bwd_dkdv_handover(q, k, v, d_o, stats, dk, dv, ds_ws, ds_ws_bytes, k_cnt, k_idx, pair_base, n_pairs, mask_bh, B, Hq,
-                                     Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream))
+  if (int rc = dkdv_handover_impl(q, k, v, d_o, stats, dk, dv, ds_ws, ds_ws_bytes, k_cnt, k_idx, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim,
+                                  q_block, k_block, split_ws, split_ws_bytes, hip_stream, {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq}))
     return rc;
   return fba_bwd_dq_from_ds(k, ds_ws, ds_ws_bytes, dq, q_cnt, q_idx, q_slot, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim,
                             q_block, k_block, split_ws, split_ws_bytes, hip_stream);
@@ -597,9 +604,9 @@ int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, cons
   if (ds_ws_bytes < need)
     return fail(FBA_ERR_INVALID, "backward: ds_ws holds %lld bytes, %lld tile pairs of 128 x 128 need %lld", (long long)ds_ws_bytes,
                 (long long)n_pairs, (long long)need);
-  if (int rc = fba_bwd_stats(o, d_o, lse, stats, (int64_t)B * Hq * Sq, head_dim, hip_stream)) return rc;
   fba::BwdParams p{};
   fill_bwd(p, s);
+  p.make = {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq};
   p.tiled = 1;
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
   p.stats = stats; p.dq = (__bf16*)dq; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv;
@@ -716,9 +723,9 @@ int32_t fba_bwd_dense(const void* q, const void* k, const void* v, const void* o
   if (ds_ws_bytes < need)
     return fail(FBA_ERR_INVALID, "backward: ds_ws holds %lld bytes, all pairs of %d heads, %d x %d, need %lld", (long long)ds_ws_bytes, B * Hq, Sq,
                 Skv, (long long)need);
-  if (int rc = fba_bwd_stats(o, d_o, lse, stats, (int64_t)B * Hq * Sq, head_dim, hip_stream)) return rc;
   fba::BwdParams p{};
   fill_bwd(p, s);
+  p.make = {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq};
   p.tiled = tiled ? 1 : 0;
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
   p.stats = stats; p.dq = (__bf16*)dq; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv;

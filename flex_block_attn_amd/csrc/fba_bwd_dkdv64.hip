@@ -71,8 +71,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   }
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
   int item, part = 0, parts = 1;
-  const int slot = grid_index - p.split.main_wgs;  // where a part's results go
-  if (slot < 0) {
+  int slot = grid_index - p.split.main_wgs;  // where a part's results go
+  int piece_begin = -1, piece_slabs = 0;      // of a launch in pieces
+  const int pieces = p.pieces.header != nullptr ? const_idx(p.pieces.header)[0] : 0;
+  if (pieces > 0) {
+    if (grid_index >= pieces) return;
+    const ConstIdx piece = const_idx(reinterpret_cast<const int32_t*>(p.pieces.list + grid_index));
+    item = piece[0];
+    piece_begin = piece[1];
+    piece_slabs = piece[2];
+    slot = piece[3];
+    parts = slot >= 0 ? 2 : 1;  // more than one, that is all that counts
+  } else if (slot < 0) {
     item = p.order != nullptr ? grid_index : xcd_remap(grid_index, p.items_per_xcd);
     if (item >= p.split.first) return;
     if (p.order != nullptr) item = const_idx(p.order)[item];
@@ -148,8 +158,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   }
   // this work-group's range of listed slabs: all of them, or part `part` of `parts` (boundaries on multiples of four slabs;
   // block lists only)
-  const int s_begin = parts == 1 ? 0 : 4 * (int)(((int64_t)(slabs_all / 4) * part) / parts);
-  const int nslabs = (parts == 1 ? slabs_all : 4 * (int)(((int64_t)(slabs_all / 4) * (part + 1)) / parts)) - s_begin;
+  const int s_begin = piece_begin >= 0 ? piece_begin : parts == 1 ? 0 : 4 * (int)(((int64_t)(slabs_all / 4) * part) / parts);
+  const int nslabs = piece_begin >= 0 ? min(piece_slabs, slabs_all) : (parts == 1 ? slabs_all : 4 * (int)(((int64_t)(slabs_all / 4) * (part + 1)) / parts)) - s_begin;
   // (query head of the group, list entry, slab inside the query block) of slab s_begin
   int g_begin = 0, e_begin = 0, sub_begin = 0;
   if (parts > 1) {
@@ -658,12 +668,12 @@ hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
   if (e != hipSuccess) return e;
   int grid;
-  if ((e = plan_key_tiles(p, kKeyTiles128, grid, stream)) != hipSuccess) return e;
+  if ((e = plan_key_tiles(p, kKeyTiles128, grid, stream, /*takes_pieces=*/true)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(256), kSmemBytes + 16, stream, p);
   const int split_items = p.num_items - p.split.first;
-  if (split_items > 0) {
+  if (split_items > 0 || p.pieces.header != nullptr) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
-    e = launch_partial_sum(p.split, 2 * 128 * kHeadDim, 128, outs, 2, p.order, stream);
+    e = launch_partial_sum(p.split, 2 * 128 * kHeadDim, 128, outs, 2, p.order, stream, p.pieces);
     if (e != hipSuccess) return e;
   }
   return hipGetLastError();

@@ -18,6 +18,7 @@
 // work-group's query tile names key blocks with a predicate per 16 rows.  A wave whose rows do not select a key block has
 // no unit there (the key-major kernel stored none): it copies 2 KiB of zeros instead, so that every wave issues the same
 // number of copies per stage, and leaves the matrix work of those steps out.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -280,10 +281,31 @@ struct PartialOuts {
   PartialOut out[2];
 };
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_sum_kernel(const SplitPlan split, int64_t slot_floats, int rows, PartialOuts outs,
-                                                                                          const int32_t* order) {
+                                                                                          const int32_t* order, const Pieces pieces) {
   const int tid = threadIdx.x;
   const PartialOut& o = outs.out[blockIdx.y];
   const int c4 = (tid & 31) * 4;
+  if (pieces.header != nullptr && const_idx(pieces.header)[0] > 0) {  // items cut each by its own length
+    const int n_rows = const_idx(pieces.header)[1] * rows;
+    for (int row = blockIdx.x * 8 + (tid >> 5); row < n_rows; row += gridDim.x * 8) {
+      const int it = row / rows, r = row - it * rows;
+      const CutItem cut = pieces.cut[it];
+      const float* src = split.ws + cut.slot * slot_floats + o.offset + r * kHeadDim + c4;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int q = 0; q < cut.pieces; q += kMostParts) {
+        f32x4 of[kMostParts];
+#pragma unroll
+        for (int i = 0; i < kMostParts; ++i)
+          if (q + i < cut.pieces) of[i] = *reinterpret_cast<const f32x4*>(src + (q + i) * slot_floats);
+#pragma unroll
+        for (int i = 0; i < kMostParts; ++i)
+          if (q + i < cut.pieces) acc += of[i];
+      }
+      *reinterpret_cast<bf16x4*>(o.out + ((int64_t)cut.item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
+    }
+    return;
+  }
+  if (split.items == 0) return;  // the host has planned no parts
   const int parts = parts_made(split);
   if (parts == 1) return;  // done whole
   for (int block = blockIdx.x; block < split.items * (rows / 8); block += gridDim.x) {
@@ -307,9 +329,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_s
 }
 
 hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order,
-                              hipStream_t stream) {
+                              hipStream_t stream, const Pieces& pieces) {
   PartialOuts o{{outs[0], outs[n_outs - 1]}};
-  hipLaunchKernelGGL(partial_sum_kernel, dim3(merge_grid(split.items * (rows / 8)), n_outs), dim3(256), 0, stream, split, slot_floats, rows, o, order);
+  const int grid = std::max(merge_grid(split.items * (rows / 8)), pieces.header != nullptr ? 128 : 0);
+  hipLaunchKernelGGL(partial_sum_kernel, dim3(grid, n_outs), dim3(256), 0, stream, split, slot_floats, rows, o, order, pieces);
   return hipGetLastError();
 }
 

@@ -164,6 +164,30 @@ struct BwdMaskParams {
   int key_items, key_wgs, key_per_xcd, query_items, query_per_xcd;  // key tiles, the work-groups for them, query tiles
 };
 
+// Backward statistics (see stats_rows in fba_split.hip); stats null: there are some already.
+struct BwdStats {
+  const __bf16* o;
+  const __bf16* d_o;
+  const float* lse;
+  float* stats;  // [2, rows]
+  int64_t rows;
+};
+
+// A dK/dV launch whose lists differ so much that the longest of them would set its time: all items as pieces, long ones first.  Made on the
+// device (plan_pieces in fba_split.hip), because only there the lists are known.
+struct Piece {
+  int32_t item, begin, slabs;  // slabs begin .. begin + slabs - 1 of the item's list
+  int32_t slot;                // where the partial results go, or -1: the item is whole
+};
+struct CutItem {
+  int32_t item, slot, pieces, unused;  // the item's pieces have consecutive slots
+};
+struct Pieces {  // in the caller's workspace
+  const int32_t* header;  // number of pieces (0: the launch runs as the host has planned it), of items that are cut; null: no launch of this kind
+  const Piece* list;
+  const CutItem* cut;
+};
+
 struct BwdParams {
   const __bf16* q;
   const __bf16* k;
@@ -210,9 +234,11 @@ struct BwdParams {
   int* queue;
   int total_work;
   // dkdv64_kernel, dkdv_kernel on block lists: the item of every grid index, long lists first (null: items in xcd_remap's
-  // order; see order_items_kernel)
+  // order; see order_items)
   const int32_t* order;
   int64_t split_ws_bytes;  // size of split.ws as handed in by the caller
+  Pieces pieces;           // dkdv64_kernel
+  BwdStats make;           // statistics that are to be formed in front of the dK/dV kernel
 };
 
 // How a backward call hands dS over: not at all (dQ recomputes), through pairs numbered in list order, or through a place
@@ -257,15 +283,16 @@ hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream);
 bool fwd_takes_mask(int64_t rows, int64_t kv_len);
 hipError_t launch_bwd_mask(BwdMaskParams p, hipStream_t stream);
 bool bwd_takes_mask(int64_t heads, int64_t kv_heads, int64_t q_len, int64_t kv_len);
-hipError_t launch_bwd_stats(const __bf16* o, const __bf16* d_o, const float* lse, float* stats, int64_t rows, hipStream_t stream);
+hipError_t launch_bwd_stats(const BwdStats& s, hipStream_t stream);
 hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);
 hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream);  // block lists only: 64 keys per wave, one wave per SIMD
 hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream);  // tile lists only: 64 keys per work-group
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream);
 // Shape of a dK/dV launch over key tiles of `tile_rows` rows, whose parts store `slot_bytes` each: sets p.num_items, split,
-// items_per_xcd, order, queue and total_work and the number of work-groups, and launches what has to run in front.
-hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream);
+// items_per_xcd, order, queue and total_work and the number of work-groups, and launches what has to run in front, p.make's statistics
+// among it.
+hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream, bool takes_pieces = false);
 int device_compute_units();
 // One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats).
 struct PartialOut {
@@ -275,7 +302,7 @@ struct PartialOut {
 };
 // order: null, or the item of every grid index.
 hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order,
-                              hipStream_t stream);
+                              hipStream_t stream, const Pieces& pieces = {});
 hipError_t launch_probe_mfma(const float* src, float* sink, int work_groups, int iters, hipStream_t stream);
 hipError_t launch_probe_read(const void* src, int64_t bytes, uint32_t* sink, int work_groups, hipStream_t stream);
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,

@@ -4,6 +4,7 @@
 #include <cstdlib>
 #include <mutex>
 
+#include "fba_common.h"
 #include "fba_kernels.h"
 
 namespace fba {
@@ -156,7 +157,33 @@ constexpr int kQueueBytes = 256;
 constexpr int kRankItems = 64;      // items a block of the ordering launch places
 constexpr int kMostOrdered = 2048;  // items of a launch that is ordered at all: eight rounds
 
-__global__ void queue_reset_kernel(int* queue) { queue[threadIdx.x] = 0; }
+// Backward statistics, one pass over O and dO: stats[r] = lse[r] * log2(e) and stats[rows + r] = -delta[r] =
+// -sum_c dO[r, c] * O[r, c] in fp32 (reference: bwd_attend_prep_ker, flex_block_attn_h100.cu:375-379).  The backward
+// kernels exponentiate in base 2, hence the pre-scaled LSE; they start the dP accumulators from the second plane, so that
+// the matrix instructions themselves form dP - delta (the reference preloads its accumulator the same way,
+// flex_block_attn_h100.cu:445-467), hence the sign.  16 lanes per row (16 bytes of each operand per lane); 256 threads to a block.
+constexpr int kStatsRows = 16;
+FBA_DEVICE void stats_rows(const BwdStats& s, int block, int blocks) {
+  const int sub = threadIdx.x & 15;
+  for (int64_t r = (int64_t)block * kStatsRows + (threadIdx.x >> 4); r < s.rows; r += (int64_t)blocks * kStatsRows) {
+    const bf16x8 a = *reinterpret_cast<const bf16x8*>(s.o + r * kHeadDim + sub * 8);
+    const bf16x8 b = *reinterpret_cast<const bf16x8*>(s.d_o + r * kHeadDim + sub * 8);
+    float acc = 0.f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc += (float)a[t] * (float)b[t];
+    acc += __shfl_xor(acc, 8);
+    acc += __shfl_xor(acc, 4);
+    acc += __shfl_xor(acc, 2);
+    acc += __shfl_xor(acc, 1);
+    if (sub == 0) {
+      s.stats[r] = s.lse[r] * 1.4426950408889634f;
+      s.stats[s.rows + r] = -acc;
+    }
+  }
+}
+int stats_blocks(const BwdStats& s) { return (int)std::min<int64_t>((s.rows + kStatsRows - 1) / kStatsRows, 65536); }
+
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void bwd_stats_kernel(const BwdStats s) { stats_rows(s, blockIdx.x, gridDim.x); }
 
 // Which item every grid index of a dK/dV launch works on: long lists first.  The lists of a random mask differ by 10-20 %
 // in length, so with items in index order the last round of work-groups ends with the longest list that happened to start
@@ -169,12 +196,14 @@ __global__ void queue_reset_kernel(int* queue) { queue[threadIdx.x] = 0; }
 // keep the heads of a large launch one after the other, so that work-groups that run together still share Q and dO in L2.
 // Lists of one length keep index order, so for them the launch is all cost: it has to be short.  Four lanes share the counting of
 // an item, with eight LDS reads in flight each; with one lane per item and a read at a time the chain of reads set the time.
-// Grid: spans * ceil(longest run / 64) blocks.
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void order_items_kernel(const BwdParams p, int spans, int segment, int32_t* order) {
-  __shared__ int lens[kMostOrdered];
-  const int tid = threadIdx.x;
-  if (p.queue != nullptr && blockIdx.x == 0 && tid < kQueueBytes / 4) p.queue[tid] = 0;
-  const int span = blockIdx.x % spans, i0 = blockIdx.x / spans * kRankItems;
+// spans * ceil(longest run / 64) blocks.
+struct ItemOrder {
+  int blocks, spans, segment;
+  int32_t* order;
+};
+FBA_DEVICE void order_items(const BwdParams& p, const ItemOrder& make, int block, int* lens) {
+  const int tid = threadIdx.x, spans = make.spans, segment = make.segment;
+  const int span = block % spans, i0 = block / spans * kRankItems;
   const int start = span * (p.num_items / spans) + min(span, p.num_items % spans);
   const int count = p.num_items / spans + (span < p.num_items % spans);
   if (i0 >= count) return;
@@ -202,10 +231,178 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void order_ite
   }
   before += __shfl_xor(before, 1);
   before += __shfl_xor(before, 2);
-  if ((tid & 3) == 0 && i0 + (tid >> 2) < count) order[(int64_t)(lo + before) * spans + span] = start + i;
+  if ((tid & 3) == 0 && i0 + (tid >> 2) < count) make.order[(int64_t)(lo + before) * spans + span] = start + i;
+}
+
+// Lists of very different length (a sink block that every query selects, windows shifted in at a border): while other compute units are done, the
+// longest list goes on.  Then the items are cut to about equal pieces instead, and the pieces start in falling order of length.
+//
+// What decides: with the whole chip at work a slab takes a work-group 1.0 us (two slabs in 2.0), with most of it idle 0.75, since the
+// clock rises; so lists up to 1.3 times what an even share would be lose nothing by it, and cutting costs the partial results and their
+// merge, about 20 us.  (H1 S30720, 60 % kept at random, lists of 37 to 59 blocks on 240 compute units: 45 an even share, dK/dV 552 us whole; as
+// much when the longest were cut.)
+// Steps, whole lists / pieces: score-driven masks with a sink block, top-12 of 63 blocks, H1 S24192 755 / 408 us, H2 947 / 667, H3 1093 / 930 (H4 and
+// more are left alone), H2 S69120 2895 / 1738; 3 x 3 x 3 windows over 3 x 4 x 5 tiles, H1 823 / 634, H2 1506 / 1098; video latents H4 S73728 11450 / 8583.
+// Launches of less than a round: the smallest piece with which there is one for every compute unit at most.  Others: an even share;
+// what is longer than 1.5 of them is cut.
+struct PieceMaker {
+  int32_t* header;
+  Piece* list;
+  CutItem* cut;
+  int slots, max_slots, most;  // compute units, partial results the workspace has room for, pieces the launch has work-groups for
+  int parts;                   // that the host has planned for all items alike
+};
+constexpr int kFrontThreads = 256, kFrontWaves = kFrontThreads / 64;
+constexpr int kBins = 256;
+constexpr float kSlabAlone = 0.75f, kSlabFull = 1.f, kPiecesCost = 20.f;  // us
+
+// Sum over (or largest of) the block's threads, the same in all of them.  `scratch`: kFrontWaves ints.
+template <bool kMax>
+FBA_DEVICE int over_block(int x, int* scratch) {
+  const int w = kMax ? wave_max(x) : wave_sum(x);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = w;
+  __syncthreads();
+  int all = scratch[0];
+#pragma unroll
+  for (int i = 1; i < kFrontWaves; ++i) all = kMax ? max(all, scratch[i]) : all + scratch[i];
+  return all;
+}
+// Sum over the threads in front of this one, and over all.
+FBA_DEVICE int before_thread(int x, int* scratch, int& all) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int sum = x;
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    const int y = __shfl_up(sum, d);
+    sum += lane >= d ? y : 0;
+  }
+  __syncthreads();
+  if (lane == 63) scratch[wave] = sum;
+  __syncthreads();
+  int before = sum - x;
+  all = 0;
+#pragma unroll
+  for (int i = 0; i < kFrontWaves; ++i) {
+    before += i < wave ? scratch[i] : 0;
+    all += scratch[i];
+  }
+  return before;
+}
+
+FBA_DEVICE int list_entries(const BwdParams& p, int item) {  // of a key tile of 128 rows, over the query heads of its group
+  const int tiles_per_head = p.Skv / 128, group = p.Hq / p.Hkv;
+  const int bhk = item / tiles_per_head, kblk = (item - bhk * tiles_per_head) * 128 / p.k_block;
+  if (p.mask_bh == 1) return p.k_cnt[kblk] * group;
+  const int64_t row = (int64_t)bhk * group * p.nK + kblk;  // query heads of a kv head are consecutive
+  int n = 0;
+  for (int g = 0; g < group; ++g) n += p.k_cnt[row + (int64_t)g * p.nK];
+  return n;
+}
+
+FBA_DEVICE void plan_pieces(const BwdParams& p, const PieceMaker& make, int* lens) {
+  __shared__ int scratch[kFrontWaves], bins[kBins];
+  const int tid = threadIdx.x, items = p.num_items;
+  const int each = (items + kFrontThreads - 1) / kFrontThreads, first = min(tid * each, items), last = min(first + each, items);  // this thread's
+  int longest = 0, sum = 0;
+  for (int j = tid; j < items; j += kFrontThreads) {
+    const int n = list_entries(p, j) * (p.q_block / 32);
+    lens[j] = n;
+    longest = max(longest, n);
+    sum += n;
+  }
+  longest = over_block<true>(longest, scratch);
+  const float share = (float)over_block<false>(sum, scratch) / (float)make.slots;  // (items times the longest possible list is below 2^31)
+  float whole = (float)longest;  // how long the longest list makes the launch, in slabs
+  int size = max(64, ((int)share + 4) & ~3), most = size + size / 2;  // of a piece; what is longer is cut
+  if (items <= make.slots) {
+    for (int n = 2; n <= make.parts; ++n)  // parts of all items alike, where the host has planned them
+      whole = fminf(whole, n * items <= make.slots ? (float)longest / n : fmaxf((float)longest / n, share + 0.5f * (float)longest / n));
+    int low = min(size, longest), high = max(longest, 4);  // the smallest size that makes no more pieces than there are compute units
+    while (high - low > max(4, high / 32)) {
+      const int middle = (low + high) / 2;
+      const float per = 1.f / (float)middle;
+      int n = 0;
+      for (int j = first; j < last; ++j) n += max(1, (int)__builtin_ceilf((float)lens[j] * per));
+      if (over_block<false>(n, scratch) <= make.slots) high = middle; else low = middle + 1;
+    }
+    size = most = (high + 7) & ~3;
+  }
+  const float per_size = 1.f / (float)size;
+  auto pieces_of = [&](int n) { return n <= most ? 1 : (int)__builtin_ceilf((float)n * per_size); };
+  const float cut_time = 1.05f * fmaxf(kSlabAlone * (float)most, kSlabFull * share) + kPiecesCost;
+  int n_cut = 0, n_slots = 0, cut_at = 0, slot_at = 0;
+  bool cuts = fmaxf(kSlabAlone * whole, kSlabFull * share) > 1.05f * cut_time;
+  if (cuts) {
+    int packed = 0;  // items that are cut << 16 | their pieces: an even share or more each, so some thousands at most
+    for (int j = first; j < last; ++j) {
+      const int n = pieces_of(lens[j]);
+      packed += n > 1 ? 1 << 16 | n : 0;
+    }
+    int all;
+    const int before = before_thread(packed, scratch, all);
+    n_cut = all >> 16;
+    n_slots = all & 0xffff;
+    cut_at = before >> 16;
+    slot_at = before & 0xffff;
+    cuts = n_cut > 0 && n_slots <= make.max_slots && items + n_slots - n_cut <= make.most;
+  }
+  if (tid == 0) {
+    make.header[0] = cuts ? items + n_slots - n_cut : 0;
+    make.header[1] = n_cut;
+  }
+  if (!cuts) return;
+
+  // long pieces first: counted by length, then dealt out (which of two as long as each other comes first makes no difference to any result)
+  bins[tid] = 0;
+  __syncthreads();
+  const float per_slab = (float)(kBins - 1) / (float)most;
+  auto bin_of = [&](int slabs) { return kBins - 1 - min((int)((float)slabs * per_slab), kBins - 1); };
+  for (int j = first; j < last; ++j) {
+    const int n = pieces_of(lens[j]);
+    atomicAdd(&bins[bin_of(lens[j] / n)], n);
+  }
+  __syncthreads();
+  int unused;
+  const int in_front = before_thread(bins[tid], scratch, unused);
+  bins[tid] = in_front;
+  __syncthreads();
+  for (int j = first; j < last; ++j) {
+    const int n = pieces_of(lens[j]), quads = lens[j] / 4;  // boundaries on multiples of four slabs
+    const int at = atomicAdd(&bins[bin_of(lens[j] / n)], n);
+    for (int q = 0; q < n; ++q) {
+      const int from = (int)((int64_t)quads * q / n), to = (int)((int64_t)quads * (q + 1) / n);
+      make.list[at + q] = {j, 4 * from, 4 * (to - from), n > 1 ? slot_at + q : -1};
+    }
+    if (n > 1) {
+      make.cut[cut_at++] = {j, slot_at, n, 0};
+      slot_at += n;
+    }
+  }
+}
+static_assert(kBins == kFrontThreads);
+
+// What runs in front of a dK/dV kernel, side by side in one launch: the plan of its pieces, the order of its items, its claim counters, the
+// statistics.  In launches of their own the order or the counters took 5 to 6 us and a gap beside 5 us of statistics at S24192; now all of it takes 6 to
+// 8.5 us (H4 S8192, 32 of 64 kept, step 309 -> 298 us; H8 S9216 1369 -> 1334).
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void bwd_front_kernel(const BwdParams p, const ItemOrder make,
+                                                                                        const PieceMaker pieces) {
+  __shared__ int lens[kMostOrdered];
+  const int planner = pieces.header != nullptr ? 1 : 0;  // the first block
+  const int block = (int)blockIdx.x - planner;
+  if (p.queue != nullptr && blockIdx.x == 0 && threadIdx.x < kQueueBytes / 4) p.queue[threadIdx.x] = 0;
+  if (block < 0) plan_pieces(p, pieces, lens);
+  else if (block < make.blocks) order_items(p, make, block, lens);
+  else if (p.make.stats != nullptr) stats_rows(p.make, block - make.blocks, gridDim.x - planner - make.blocks);
 }
 
 }  // namespace
+
+hipError_t launch_bwd_stats(const BwdStats& s, hipStream_t stream) {
+  if (s.rows <= 0) return hipSuccess;
+  hipLaunchKernelGGL(bwd_stats_kernel, dim3(stats_blocks(s)), dim3(256), 0, stream, s);
+  return hipGetLastError();
+}
 
 // One work-group per compute unit.
 void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles) {
@@ -216,7 +413,7 @@ void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles) {
                        lengths);
 }
 
-hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream) {
+hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream, bool takes_pieces) {
   const int slots = compute_units();
   const int heads = p.B * p.Hkv;
   char* const ws = reinterpret_cast<char*>(p.split.ws);  // whether or not anything is split
@@ -231,6 +428,7 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
   const int64_t bottom = parts * tiles.slot_bytes + kNoteBytes;
   int* const queue = ws != nullptr && top >= bottom ? reinterpret_cast<int*>(ws + top) : nullptr;
   top = (top - (int64_t)p.num_items * 4) & ~(int64_t)15;
+  const int64_t order_at = top;
   // Items are ordered where they start in more than one round and in at most eight.  One round starts everything at once; over
   // many rounds the spread of the last one no longer counts, while tiles in index order share more of their lists in L2
   // (structured masks).  Steps, items in index order / ordered: masks that choose per head, a quarter kept, H8 S8192 (2 rounds)
@@ -243,32 +441,50 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
   // against 377 / 359 us; a random mask at H8 S6144 (192 slabs, 1.5 rounds) 302 / 297 us, 308 / 289 where all
   // heads share it.
   const int longest = p.Hq / p.Hkv * (p.Sq / 32);
-  const bool ordered = !p.tiled && queue != nullptr && top >= bottom && p.num_items > slots && p.num_items <= std::min(8 * slots, kMostOrdered) &&
+  const bool ordered = !p.tiled && queue != nullptr && order_at >= bottom && p.num_items > slots && p.num_items <= std::min(8 * slots, kMostOrdered) &&
                        longest >= (p.split.first + parts >= 4 * slots ? 128 : 192);
   if (ordered) p.split.main_wgs = p.split.first;
+
+  // Room for pieces, where lists can be so long that cutting them pays (plan_pieces) and there are not so many that the longest cannot
+  // count.  A launch that needs none pays for work-groups that exit at once, one to a compute unit; the planning hides behind the statistics,
+  // so a dK/dV kernel called by itself goes without.
+  PieceMaker maker{};
+  const int most_pieces = p.num_items <= slots ? slots : p.num_items + slots;
+  const int64_t piece_bytes = 64 + most_pieces * (int64_t)sizeof(Piece) + slots * (int64_t)sizeof(CutItem);
+  top = (top - piece_bytes) & ~(int64_t)63;
+  p.pieces = {};
+  if (takes_pieces && p.make.stats != nullptr && !p.tiled && queue != nullptr && p.num_items <= kMostOrdered && longest >= (p.num_items > slots ? 256 : 512) && (int64_t)p.num_items * longest < 0x7fffffffLL &&
+      top >= std::max(bottom, 2 * slots * tiles.slot_bytes)) {
+    maker = {reinterpret_cast<int32_t*>(ws + top), reinterpret_cast<Piece*>(ws + top + 64), reinterpret_cast<CutItem*>(ws + top + 64) + most_pieces, slots,
+             2 * slots, most_pieces, p.split.items == p.num_items ? p.split.parts : 1};
+    p.pieces = {maker.header, maker.list, maker.cut};
+    p.split.ws = reinterpret_cast<float*>(ws);
+  }
 
   // Launches of four rounds and more let the work-groups claim their grid indices, with some more work-groups than indices,
   // so that an XCD that is through early takes over from the others (claim_work; either mapping deals grid index i to XCD
   // i % 8, which is all a claim relies on).  FBA_CLAIM_WORK=0 switches claiming off, for measurements.
   p.total_work = p.split.main_wgs + parts;
+  if (p.pieces.header != nullptr) p.total_work = std::max(p.total_work, most_pieces);
   grid = p.total_work;
   const char* claim = getenv("FBA_CLAIM_WORK");
-  if (queue != nullptr && !(claim != nullptr && claim[0] == '0') && p.total_work >= 4 * slots) {
+  if (queue != nullptr && !(claim != nullptr && claim[0] == '0') && p.split.main_wgs + parts >= 4 * slots) {
     p.queue = queue;
     grid += (p.total_work / 8 + 7) / 8 * 8;  // an eighth more work-groups, a whole number per XCD
   }
+  ItemOrder make{};
   if (ordered) {
-    const int spans = heads >= 8 ? 8 : 1;
-    const int tiles_per_head = p.Skv / tiles.rows, two_rounds = 2 * slots / spans;
-    const int segment = (two_rounds + tiles_per_head - 1) / tiles_per_head * tiles_per_head;
-    const int blocks = spans * (((p.num_items + spans - 1) / spans + kRankItems - 1) / kRankItems);
-    int32_t* const order = reinterpret_cast<int32_t*>(ws + top);
-    hipLaunchKernelGGL(order_items_kernel, dim3(blocks), dim3(256), 0, stream, p, spans, segment, order);
-    p.order = order;
-    if (2 * p.split.items <= slots) p.split.look.order = order;
-  } else if (p.queue != nullptr) {
-    hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(kQueueBytes / 4), 0, stream, p.queue);
+    const int tiles_per_head = p.Skv / tiles.rows;
+    make.spans = heads >= 8 ? 8 : 1;
+    const int two_rounds = 2 * slots / make.spans;
+    make.segment = (two_rounds + tiles_per_head - 1) / tiles_per_head * tiles_per_head;
+    make.blocks = make.spans * (((p.num_items + make.spans - 1) / make.spans + kRankItems - 1) / kRankItems);
+    make.order = reinterpret_cast<int32_t*>(ws + order_at);
+    p.order = make.order;
+    if (2 * p.split.items <= slots) p.split.look.order = p.order;
   }
+  const int front = (maker.header != nullptr) + make.blocks + (p.make.stats != nullptr ? stats_blocks(p.make) : p.queue != nullptr ? 1 : 0);
+  if (front > 0) hipLaunchKernelGGL(bwd_front_kernel, dim3(front), dim3(kFrontThreads), 0, stream, p, make, maker);
   return hipGetLastError();
 }
 
