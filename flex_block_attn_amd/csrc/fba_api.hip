@@ -216,14 +216,28 @@ int32_t fba_bwd_takes_mask(int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32
   return fba::bwd_takes_mask((int64_t)B * Hq, (int64_t)B * Hkv, Sq, Skv) ? 1 : 0;
 }
 
-int32_t fba_block_mean(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, int32_t head_dim, void* hip_stream) {
-  if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);
+static int check_means(const void* x, const float* out, int64_t n_seq, int32_t S, int32_t block) {
   if (n_seq <= 0 || S <= 0) return fail(FBA_ERR_INVALID, "n_seq and S must be positive (got %lld %d)", (long long)n_seq, S);
   if (block <= 0 || block % 16 != 0 || S % block != 0)
     return fail(FBA_ERR_INVALID, "block (%d) must be a positive multiple of 16 that divides S (%d)", block, S);
   if (!out) return fail(FBA_ERR_INVALID, "out is null");
-  if (int rc = check_ptrs({{"x", x}})) return rc;
-  hipError_t e = fba::launch_block_mean((const __bf16*)x, out, n_seq * (S / block), block, (hipStream_t)hip_stream);
+  return check_ptrs({{"x", x}});
+}
+
+int32_t fba_block_mean(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, int32_t head_dim, void* hip_stream) {
+  if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);
+  if (int rc = check_means(x, out, n_seq, S, block)) return rc;
+  hipError_t e = fba::launch_block_mean({{(const __bf16*)x, out, n_seq * (S / block), block}, {}}, (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "block_mean launch");
+}
+
+int32_t fba_block_mean_pair(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, const void* x2, float* out2, int64_t n_seq2, int32_t S2,
+                            int32_t block2, int32_t head_dim, void* hip_stream) {
+  if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);
+  if (int rc = check_means(x, out, n_seq, S, block)) return rc;
+  if (int rc = check_means(x2, out2, n_seq2, S2, block2)) return rc;
+  hipError_t e = fba::launch_block_mean({{(const __bf16*)x, out, n_seq * (S / block), block}, {(const __bf16*)x2, out2, n_seq2 * (S2 / block2), block2}},
+                                        (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "block_mean launch");
 }
 

@@ -268,7 +268,14 @@ struct TileWindow {
   }
 };
 
-hipError_t launch_block_mean(const __bf16* x, float* out, int64_t n_blocks, int block, hipStream_t stream);
+// Means of the blocks of one tensor, or of two in one launch (the second with n_blocks = 0: there is none).
+struct BlockMeans {
+  const __bf16* x;
+  float* out;
+  int64_t n_blocks;
+  int block;
+};
+hipError_t launch_block_mean(const BlockMeans (&of)[2], hipStream_t stream);
 hipError_t launch_ssta_mask(const float* q_mean, const float* k_mean, const uint8_t* base, uint8_t* mask, int64_t BH, int Hq, int Hkv, int nQ,
                             int nK, int q_block, int k_block, int topk, int band, int sink, const TileWindow& window, hipStream_t stream);
 hipError_t launch_tile_gather(int n, const void* const* x, void* const* out, float* const* mean, const int64_t* n_seq, int T, int H, int W, int tT,

@@ -13,14 +13,22 @@ constexpr int kD = 128;
 __device__ __forceinline__ float bf16_lo(uint32_t u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 
-// out[g, :] = mean over rows [g*block, (g+1)*block) of x, x [n_blocks*block, 128] bf16, out fp32.
-// One work-group per block: 16 lanes cover one 256-byte row, the 16 row groups of the work-group stride through the
+// out[g, :] = mean over rows [g*block, (g+1)*block) of x, x [n_blocks*block, 128] bf16, out fp32; of one tensor or two (q and k of a mask
+// in one launch).  One work-group per block: 16 lanes cover one 256-byte row, the 16 row groups of the work-group stride through the
 // block, then add up through LDS in a fixed order (the result does not depend on scheduling).
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void block_mean_kernel(
-    const __bf16* __restrict__ x, float* __restrict__ out, int block, float inv_block) {
+struct MeanJobs {
+  const __bf16* x[2];
+  float* out[2];
+  int block[2];
+  float inv_block[2];
+  unsigned second;  // first block of the second tensor (past the end: there is none)
+};
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void block_mean_kernel(const MeanJobs jobs) {
   __shared__ float red[16][kD + 4];
   const int tid = threadIdx.x, c = tid & 15, r0 = tid >> 4;
-  const uint4* src = reinterpret_cast<const uint4*>(x + (size_t)blockIdx.x * block * kD);
+  const int which = blockIdx.x >= jobs.second ? 1 : 0, block = jobs.block[which];
+  const unsigned g0 = blockIdx.x - (which ? jobs.second : 0);
+  const uint4* src = reinterpret_cast<const uint4*>(jobs.x[which] + (size_t)g0 * block * kD);
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   int r = r0;
   for (; r + 48 < block; r += 64) {
@@ -45,91 +53,130 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void block_mea
     float s = 0.f;
 #pragma unroll
     for (int g = 0; g < 16; ++g) s += red[g][tid];
-    out[(size_t)blockIdx.x * kD + tid] = s * inv_block;
+    jobs.out[which][(size_t)g0 * kD + tid] = s * jobs.inv_block[which];
   }
 }
 
 constexpr int kQPerWave = 2;
-constexpr int kQPerGroup = 8;      // query blocks per work-group (4 waves x 2)
-constexpr int kChunk = 64;         // key blocks per LDS chunk: one per lane
-constexpr int kRowStride = kD + 1; // floats; lane-per-row reads hit 64 different banks
-constexpr int kChunksSmall = 16;   // nK <= 1024: 32 score registers per lane
-constexpr int kChunksLarge = 64;   // nK <= 4096: 128 score registers per lane
+constexpr int kQPerGroup = 8;       // query blocks per work-group (4 waves x 2)
+constexpr int kChunk = 64;          // key blocks per LDS chunk: one per lane
+constexpr int kMostChunks = 64;     // nK <= 4096
+constexpr int kRowStride = kD + 4;  // floats; 16 lanes read 16 bytes of a row each from 64 different banks
+
+// A score as an unsigned number in the same order, -0 as +0; 0 for what is never picked (NaN, -inf, no key block).
+__device__ __forceinline__ uint32_t rank_key(float x) {
+  const uint32_t u = __float_as_uint(x + 0.f);
+  return x > -__builtin_inff() ? u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u) : 0u;
+}
 
 // mask[bh, i, j] = (j among the topk largest <q_mean[bh,i], k_mean[kv(bh),j]>, ties to the lower j)
 //                  || |j - (i*q_block)/k_block| <= band || j < sink || base[i, j]   (base: optional [nQ, nK] mask)
 //                  || j in the sliding window of i (window: optional, blocks as tiles of a 3-D grid, see TileWindow).
 // A wave ranks two query blocks; lane l holds the scores of key blocks l, l+64, ... (kMaxChunks of them) in registers.
+//
+// Bound by latency.  The k-th largest score is found bit by bit, from how many scores reach a candidate (a ballot and a population count per
+// 64 of them), both query blocks side by side; picking the largest topk times over, with a maximum over the wave each time, took
+// most of the time.  Key means come in as 16 bytes a lane, a chunk ahead.  Before / now, launch included: 189 x 63 blocks, top-12, 28.7 / 10.9 us;
+// 24 heads of 540 x 180, top-16, 110 / 47; 8 of 300 x 300 61 / 34; 50 x 1000, top-40, 154 / 59; 30 x 2000, top-5, 195 / 182.
 template <int kMaxChunks>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void ssta_mask_kernel(
     const float* __restrict__ q_mean, const float* __restrict__ k_mean, const uint8_t* __restrict__ base,
     uint8_t* __restrict__ mask, int Hq, int Hkv, int nQ, int nK, int q_block, int k_block, int topk, int band, int sink, const TileWindow window) {
-  __shared__ float k_lds[kChunk * kRowStride];
-  __shared__ float q_lds[kQPerGroup * kD];
+  __shared__ __attribute__((aligned(16))) float k_lds[kChunk * kRowStride];
+  __shared__ __attribute__((aligned(16))) float q_lds[kQPerGroup * kD];
+  constexpr int kLoads = kChunk * kD / 4 / 256;  // of 16 bytes, per thread and chunk
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t bh = blockIdx.y;
   const int64_t kv_seq = (bh / Hq) * Hkv + (bh % Hq) / (Hq / Hkv);
   const int i0 = blockIdx.x * kQPerGroup;
-  for (int idx = tid; idx < kQPerGroup * kD; idx += 256) {
-    const int i = i0 + (idx >> 7);
-    q_lds[idx] = i < nQ ? q_mean[((size_t)(bh * nQ + i) << 7) + (idx & 127)] : 0.f;
-  }
-  const float ninf = -__builtin_inff();
-  float sc[kQPerWave][kMaxChunks];
   const int n_chunks = (nK + kChunk - 1) / kChunk;
+  const float4* const k_rows = reinterpret_cast<const float4*>(k_mean) + kv_seq * nK * (kD / 4);
+  float4 ahead[kLoads];
+  auto load = [&](int chunk) {
+#pragma unroll
+    for (int x = 0; x < kLoads; ++x) {
+      const int j = chunk * kChunk + (tid >> 5) + 8 * x;
+      ahead[x] = j < nK ? k_rows[(size_t)j * (kD / 4) + (tid & 31)] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+  };
+  load(0);
+  {
+    const int i = i0 + (tid >> 5);
+    reinterpret_cast<float4*>(q_lds)[tid] =
+        i < nQ ? reinterpret_cast<const float4*>(q_mean)[((size_t)bh * nQ + i) * (kD / 4) + (tid & 31)] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  uint32_t key[kQPerWave][kMaxChunks];
 #pragma unroll
   for (int t = 0; t < kMaxChunks; ++t) {
-    sc[0][t] = ninf;
-    sc[1][t] = ninf;
+    key[0][t] = key[1][t] = 0;
     if (t < n_chunks) {  // uniform over the work-group
       __syncthreads();
-      for (int idx = tid; idx < kChunk * kD; idx += 256) {
-        const int r = idx >> 7, j = t * kChunk + r;
-        k_lds[r * kRowStride + (idx & 127)] = j < nK ? k_mean[((size_t)(kv_seq * nK + j) << 7) + (idx & 127)] : 0.f;
-      }
+#pragma unroll
+      for (int x = 0; x < kLoads; ++x) *reinterpret_cast<float4*>(k_lds + ((tid >> 5) + 8 * x) * kRowStride + 4 * (tid & 31)) = ahead[x];
       __syncthreads();
+      if (t + 1 < n_chunks) load(t + 1);
       float s0 = 0.f, s1 = 0.f;
-      const float* kr = k_lds + lane * kRowStride;
-      const float* q0 = q_lds + (wave * kQPerWave) * kD;
+      const float4* kr = reinterpret_cast<const float4*>(k_lds + lane * kRowStride);
+      const float4* q0 = reinterpret_cast<const float4*>(q_lds + (wave * kQPerWave) * kD);
 #pragma unroll 8
-      for (int d = 0; d < kD; ++d) {
-        const float kv = kr[d];
-        s0 += q0[d] * kv;
-        s1 += q0[kD + d] * kv;
+      for (int d = 0; d < kD / 4; ++d) {
+        const float4 kv = kr[d], a = q0[d], b = q0[kD / 4 + d];
+        s0 = __builtin_fmaf(a.x, kv.x, s0); s1 = __builtin_fmaf(b.x, kv.x, s1);
+        s0 = __builtin_fmaf(a.y, kv.y, s0); s1 = __builtin_fmaf(b.y, kv.y, s1);
+        s0 = __builtin_fmaf(a.z, kv.z, s0); s1 = __builtin_fmaf(b.z, kv.z, s1);
+        s0 = __builtin_fmaf(a.w, kv.w, s0); s1 = __builtin_fmaf(b.w, kv.w, s1);
       }
       if (t * kChunk + lane < nK) {
-        sc[0][t] = s0;
-        sc[1][t] = s1;
+        key[0][t] = rank_key(s0);
+        key[1][t] = rank_key(s1);
       }
     }
   }
+  // how many keys of a query block reach `least`, over the wave
+  auto reach = [&](int qq, uint32_t least) {
+    int n = 0;
+#pragma unroll
+    for (int t = 0; t < kMaxChunks; ++t)
+      if (t < n_chunks) n += __popcll(__builtin_amdgcn_ballot_w64(key[qq][t] >= least));
+    return n;
+  };
+  uint32_t line[kQPerWave];  // the topk-th largest key, or one that exactly topk keys reach
+  int above[kQPerWave];      // keys beyond it, where it is the topk-th largest and keys equal to it have to be picked from; -1: all that reach it
+  bool open[kQPerWave];
+#pragma unroll
+  for (int qq = 0; qq < kQPerWave; ++qq) {
+    open[qq] = topk > 0 && reach(qq, 1u) > topk;
+    line[qq] = topk <= 0 ? 0xffffffffu : open[qq] ? 0u : 1u;  // (no key is all ones: that would be a NaN)
+    above[qq] = -1;
+  }
+  for (int bit = 31; bit >= 0 && (open[0] || open[1]); --bit) {
+#pragma unroll
+    for (int qq = 0; qq < kQPerWave; ++qq) {
+      const uint32_t least = line[qq] | 1u << bit;
+      const int n = open[qq] ? reach(qq, least) : 0;
+      if (n >= topk) line[qq] = least;
+      if (n == topk) open[qq] = false;
+    }
+  }
+#pragma unroll
+  for (int qq = 0; qq < kQPerWave; ++qq)
+    if (open[qq]) above[qq] = reach(qq, line[qq] + 1);
+
 #pragma unroll
   for (int qq = 0; qq < kQPerWave; ++qq) {
     const int i = i0 + wave * kQPerWave + qq;
     if (i >= nQ) break;  // uniform over the wave
     uint64_t sel = 0;
-    for (int round = 0; round < topk; ++round) {
-      float best = ninf;
-      int bt = -1;
+    int room = above[qq] < 0 ? 0x7fffffff : topk - above[qq];  // for keys on the line, those of lower j first
 #pragma unroll
-      for (int t = 0; t < kMaxChunks; ++t)
-        if (!((sel >> t) & 1u) && sc[qq][t] > best) {
-          best = sc[qq][t];
-          bt = t;
-        }
-      int j = bt < 0 ? 0x7fffffff : bt * kChunk + lane;
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) {
-        const float ob = __shfl_xor(best, off, 64);
-        const int oj = __shfl_xor(j, off, 64);
-        if (ob > best || (ob == best && oj < j)) {
-          best = ob;
-          j = oj;
-        }
+    for (int t = 0; t < kMaxChunks; ++t)
+      if (t < n_chunks) {
+        const bool on = key[qq][t] == line[qq];
+        const unsigned long long tie = __builtin_amdgcn_ballot_w64(on);
+        const int rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(tie >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tie, 0));
+        if (key[qq][t] > line[qq] || (on && rank < room)) sel |= 1ull << t;
+        room -= above[qq] < 0 ? 0 : __popcll(tie);
       }
-      if (j == 0x7fffffff) break;  // nothing left to pick: every lane sees the same j
-      if ((j & 63) == lane) sel |= 1ull << (j >> 6);
-    }
     const int diag = (int)(((int64_t)i * q_block) / k_block);
     uint8_t* row = mask + (size_t)(bh * nQ + i) * nK;
 #pragma unroll
@@ -300,18 +347,28 @@ hipError_t launch_resize_mask(const uint8_t* src, uint8_t* dst, int64_t M, int s
   return hipGetLastError();
 }
 
-hipError_t launch_block_mean(const __bf16* x, float* out, int64_t n_blocks, int block, hipStream_t stream) {
-  if (n_blocks <= 0) return hipSuccess;
-  if (n_blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(block_mean_kernel, dim3((unsigned)n_blocks), dim3(256), 0, stream, x, out, block, 1.0f / (float)block);
+hipError_t launch_block_mean(const BlockMeans (&of)[2], hipStream_t stream) {
+  const int64_t n = of[0].n_blocks + of[1].n_blocks;
+  if (n <= 0) return hipSuccess;
+  if (n > 0x7fffffffLL) return hipErrorInvalidValue;
+  MeanJobs jobs{};
+  for (int i = 0; i < 2; ++i) {
+    jobs.x[i] = of[i].x;
+    jobs.out[i] = of[i].out;
+    jobs.block[i] = of[i].block;
+    jobs.inv_block[i] = 1.0f / (float)of[i].block;
+  }
+  jobs.second = (unsigned)of[0].n_blocks;
+  hipLaunchKernelGGL(block_mean_kernel, dim3((unsigned)n), dim3(256), 0, stream, jobs);
   return hipGetLastError();
 }
 
 hipError_t launch_ssta_mask(const float* q_mean, const float* k_mean, const uint8_t* base, uint8_t* mask, int64_t BH, int Hq, int Hkv, int nQ,
                             int nK, int q_block, int k_block, int topk, int band, int sink, const TileWindow& window, hipStream_t stream) {
-  if (BH <= 0 || BH > 65535 || nK > kChunk * kChunksLarge) return hipErrorInvalidValue;
+  if (BH <= 0 || BH > 65535 || nK > kChunk * kMostChunks) return hipErrorInvalidValue;
+  // score registers per lane and query block: 256, 1024 or 4096 key blocks
   void (*fn)(const float*, const float*, const uint8_t*, uint8_t*, int, int, int, int, int, int, int, int, int, const TileWindow) =
-      nK <= kChunk * kChunksSmall ? &ssta_mask_kernel<kChunksSmall> : &ssta_mask_kernel<kChunksLarge>;
+      nK <= kChunk * 4 ? &ssta_mask_kernel<4> : nK <= kChunk * 16 ? &ssta_mask_kernel<16> : &ssta_mask_kernel<kMostChunks>;
   hipLaunchKernelGGL(fn, dim3((unsigned)((nQ + kQPerGroup - 1) / kQPerGroup), (unsigned)BH), dim3(256), 0,
                      stream, q_mean, k_mean, base, mask, Hq, Hkv, nQ, nK, q_block, k_block, topk, band, sink, window);
   return hipGetLastError();
@@ -324,7 +381,7 @@ hipError_t launch_tile_gather(int n, const void* const* x, void* const* out, flo
   if (tile_sz < 64 || tile_sz > kMostTileRows) {
     for (int j = 0; j < n; ++j) {
       hipError_t e = launch_tile_permute(x[j], out[j], n_seq[j], T, H, W, tT, tH, tW, to_tiles, stream);
-      if (e == hipSuccess && to_tiles && mean[j] != nullptr) e = launch_block_mean((const __bf16*)out[j], mean[j], n_seq[j] * tiles, (int)tile_sz, stream);
+      if (e == hipSuccess && to_tiles && mean[j] != nullptr) e = launch_block_mean({{(const __bf16*)out[j], mean[j], n_seq[j] * tiles, (int)tile_sz}, {}}, stream);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;

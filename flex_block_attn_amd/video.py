@@ -21,16 +21,33 @@ def _check_seq(x, name):
     return x.contiguous()
 
 
-def block_mean(x, block_size):
-    """(B, H, S, 128) bf16 -> (B, H, S / block_size, 128) fp32: the mean of every block of `block_size` rows."""
+def _means_of(x, block_size):
+    """(x as the kernels take it, an empty tensor for the means of its blocks)"""
     x = _check_seq(x, "x")
     B, H, S, _ = x.shape
     if block_size <= 0 or S % block_size:
         raise ValueError(f"seq_len ({S}) must be divisible by block_size ({block_size})")
-    out = torch.empty((B, H, S // block_size, HEAD_DIM), dtype=torch.float32, device=x.device)
+    return x, torch.empty((B, H, S // block_size, HEAD_DIM), dtype=torch.float32, device=x.device)
+
+
+def block_mean(x, block_size):
+    """(B, H, S, 128) bf16 -> (B, H, S / block_size, 128) fp32: the mean of every block of `block_size` rows."""
+    x, out = _means_of(x, block_size)
+    B, H, S, _ = x.shape
     with torch.cuda.device(x.device):
         _lib.call("fba_block_mean", _ptr(x), _ptr(out), B * H, S, block_size, HEAD_DIM, _stream())
     return out
+
+
+def _block_means(q, k, q_block_size, kv_block_size):
+    """`block_mean` of both, in one launch where they are on one device."""
+    (q, q_mean), (k, k_mean) = _means_of(q, q_block_size), _means_of(k, kv_block_size)
+    if q.device != k.device or q.numel() == 0 or k.numel() == 0:
+        return block_mean(q, q_block_size), block_mean(k, kv_block_size)
+    with torch.cuda.device(q.device):
+        _lib.call("fba_block_mean_pair", _ptr(q), _ptr(q_mean), q.shape[0] * q.shape[1], q.shape[2], q_block_size, _ptr(k), _ptr(k_mean),
+                  k.shape[0] * k.shape[1], k.shape[2], kv_block_size, HEAD_DIM, _stream())
+    return q_mean, k_mean
 
 
 def ssta_mask_from_means(q_mean, k_mean, q_block_size, kv_block_size, topk=16, band=1, sink_blocks=1, base_mask=None):
@@ -61,8 +78,7 @@ def create_ssta_mask(q, k, q_block_size, kv_block_size, topk=16, band=1, sink_bl
     query block i keeps the key block that holds its first row and its `band` neighbours on either side, the first
     `sink_blocks` key blocks, the `topk` key blocks with the largest <mean(q block i), mean(k block j)>, and whatever
     the optional 2-D `base_mask` (nQ, nK) selects (band=-1 switches the band off)."""
-    return ssta_mask_from_means(block_mean(q, q_block_size), block_mean(k, kv_block_size), q_block_size, kv_block_size,
-                                topk, band, sink_blocks, base_mask)
+    return ssta_mask_from_means(*_block_means(q, k, q_block_size, kv_block_size), q_block_size, kv_block_size, topk, band, sink_blocks, base_mask)
 
 
 def create_moba_mask(q, k, q_block_size, kv_block_size, topk):
@@ -163,7 +179,7 @@ def create_ssta_3d_mask(q, k, grid, tile=(6, 8, 8), window=(3, 3, 3), topk=16, s
     """Sliding-tile window united with score-selected tiles, for q, k already in tile order: bool (B, H, n, n) with
     n = number of tiles."""
     block = tile[0] * tile[1] * tile[2]
-    return _ssta_3d_mask_from_means(block_mean(q, block), block_mean(k, block), grid, tile, window, topk, sink_blocks)
+    return _ssta_3d_mask_from_means(*_block_means(q, k, block, block), grid, tile, window, topk, sink_blocks)
 
 
 def _ssta_3d_mask_from_means(q_mean, k_mean, grid, tile, window, topk, sink_blocks):

@@ -308,6 +308,9 @@ int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, cons
  *   either side (shifted inwards at the borders) in place of the band and of a base mask.
  */
 int32_t fba_block_mean(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, int32_t head_dim, void* hip_stream);
+/* The same of two tensors (q and k of a mask) in one launch. */
+int32_t fba_block_mean_pair(const void* x, float* out, int64_t n_seq, int32_t S, int32_t block, const void* x2, float* out2, int64_t n_seq2,
+                            int32_t S2, int32_t block2, int32_t head_dim, void* hip_stream);
 int32_t fba_ssta_mask(const float* q_mean, const float* k_mean, const uint8_t* base, uint8_t* mask, int32_t B, int32_t Hq, int32_t Hkv, int32_t nQ,
                       int32_t nK, int32_t q_block, int32_t k_block, int32_t topk, int32_t band, int32_t sink,
                       void* hip_stream);

@@ -1,0 +1,32 @@
+"""Which key blocks a score-driven mask picks: the top-k of every query block, ties to the lower block, never a score that is NaN or -inf.
+Whole-number means, so that scores are exact and full of ties; key blocks around one, four and sixteen score registers per lane (64 blocks
+each), more to pick than there are, nothing to pick, a last work-group with one query block.  Exact against a stable sort."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,nQ,nK,topk", [
+    (1, 1, 1, 1, 1, 1), (1, 2, 1, 9, 63, 5), (1, 1, 1, 8, 64, 64), (2, 2, 2, 7, 65, 16), (1, 1, 1, 17, 256, 3), (1, 1, 1, 5, 257, 16),
+    (1, 3, 1, 3, 1024, 100), (1, 1, 1, 3, 1025, 16), (1, 1, 1, 2, 4096, 70), (1, 1, 1, 4, 30, 40), (1, 1, 1, 4, 30, 0),
+])
+@pytest.mark.parametrize("kind", ["ties", "alike", "special"])
+def test_top_blocks(gpu, B, Hq, Hkv, nQ, nK, topk, kind):
+    from flex_block_attn_amd.video import ssta_mask_from_means
+
+    g = torch.Generator().manual_seed(nK + topk)
+    q, k = (torch.randint(-1, 2, (B, h, n, 128), generator=g).float() for h, n in ((Hq, nQ), (Hkv, nK)))
+    if kind == "alike":
+        k[:] = k[:, :, :1]
+    if kind == "special":
+        k[:, :, ::3] = 0.0  # scores of 0, and with an odd number of signs of -0
+        k[:, :, 1::5, 0] = float("nan")
+        k[:, :, 2::7, 0], q[..., 0] = float("-inf"), 1.0
+        k[:, :, 4::11, 0] = float("inf")
+    score = (q[:, :, :, None] * k.repeat_interleave(Hq // Hkv, 1)[:, :, None]).sum(-1)
+    rank = torch.where(score > float("-inf"), score + 0.0, float("-inf")).nan_to_num(nan=float("-inf"), posinf=float("inf"), neginf=float("-inf"))
+    order = rank.sort(dim=-1, descending=True, stable=True).indices
+    want = torch.zeros(score.shape, dtype=torch.bool).scatter_(-1, order[..., :topk], True) & (rank > float("-inf"))
+    got = ssta_mask_from_means(q.to(gpu), k.to(gpu), 128, 128, topk=topk, band=-1, sink_blocks=0)
+    assert torch.equal(got.cpu(), want)
