@@ -492,14 +492,19 @@ int32_t fba_probe_read(const void* src, int64_t bytes, uint32_t* sink, int32_t w
   return e == hipSuccess ? FBA_OK : hip_fail(e, "probe launch");
 }
 
-int32_t fba_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
-                       int32_t nQ, int32_t nK, int32_t* pair_base, int32_t* q_slot, void* hip_stream) {
+int32_t fba_pair_slots_bounds(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
+                       int32_t nQ, int32_t nK, int32_t* pair_base, int32_t* q_slot, int32_t* bounds, void* hip_stream) {
   if (mask_bh <= 0 || nQ <= 0 || nK <= 0)
     return fail(FBA_ERR_INVALID, "mask_bh, nQ, nK must be positive (got %lld %d %d)", (long long)mask_bh, nQ, nK);
   if (mask_bh * (int64_t)nQ * nK > 0x7fffffffLL) return fail(FBA_ERR_INVALID, "more than 2^31 mask entries");
   if (!q_cnt || !q_idx || !k_cnt || !k_idx || !pair_base || !q_slot) return fail(FBA_ERR_INVALID, "null pointer argument");
-  hipError_t e = fba::launch_pair_slots(q_cnt, q_idx, k_cnt, k_idx, mask_bh, nQ, nK, pair_base, q_slot, (hipStream_t)hip_stream);
+  hipError_t e = fba::launch_pair_slots(q_cnt, q_idx, k_cnt, k_idx, mask_bh, nQ, nK, pair_base, q_slot, bounds, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "pair_slots launch");
+}
+
+int32_t fba_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
+                       int32_t nQ, int32_t nK, int32_t* pair_base, int32_t* q_slot, void* hip_stream) {
+  return fba_pair_slots_bounds(q_cnt, q_idx, k_cnt, k_idx, mask_bh, nQ, nK, pair_base, q_slot, nullptr, hip_stream);
 }
 
 // Arguments of the dS hand-over, checked once for all three entry points that take them.
@@ -588,14 +593,19 @@ int32_t fba_bwd_handover(const void* q, const void* k, const void* v, const void
                             q_block, k_block, split_ws, split_ws_bytes, hip_stream);
 }
 
-int32_t fba_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int32_t n_qt, int32_t n_kt, int32_t* pair_base,
-                       int32_t* kt_slot, int32_t* slot_table, void* hip_stream) {
+int32_t fba_tile_slots_bounds(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int32_t n_qt, int32_t n_kt, int32_t* pair_base,
+                       int32_t* kt_slot, int32_t* slot_table, int32_t* bounds, void* hip_stream) {
   if (mask_bh <= 0 || n_qt <= 0 || n_kt <= 0)
     return fail(FBA_ERR_INVALID, "mask_bh, n_qt, n_kt must be positive (got %lld %d %d)", (long long)mask_bh, n_qt, n_kt);
   if (mask_bh * (int64_t)n_kt * n_qt * 4 > 0x7fffffffLL) return fail(FBA_ERR_INVALID, "more than 2^31 tile-list entries");
   if (!kt_cnt || !kt_ent || !pair_base || !kt_slot || !slot_table) return fail(FBA_ERR_INVALID, "null pointer argument");
-  hipError_t e = fba::launch_tile_slots(kt_cnt, kt_ent, mask_bh, n_qt, n_kt, 4 * n_qt, pair_base, kt_slot, slot_table, (hipStream_t)hip_stream);
+  hipError_t e = fba::launch_tile_slots(kt_cnt, kt_ent, mask_bh, n_qt, n_kt, 4 * n_qt, pair_base, kt_slot, slot_table, bounds, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "tile_slots launch");
+}
+
+int32_t fba_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int32_t n_qt, int32_t n_kt, int32_t* pair_base,
+                       int32_t* kt_slot, int32_t* slot_table, void* hip_stream) {
+  return fba_tile_slots_bounds(kt_cnt, kt_ent, mask_bh, n_qt, n_kt, pair_base, kt_slot, slot_table, nullptr, hip_stream);
 }
 
 int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,

@@ -313,8 +313,8 @@ hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int r
 hipError_t launch_probe_mfma(const float* src, float* sink, int work_groups, int iters, hipStream_t stream);
 hipError_t launch_probe_read(const void* src, int64_t bytes, uint32_t* sink, int work_groups, hipStream_t stream);
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
-                             int nQ, int nK, int32_t* pair_base, int32_t* q_slot, hipStream_t stream);
+                             int nQ, int nK, int32_t* pair_base, int32_t* q_slot, int32_t* bounds, hipStream_t stream);
 hipError_t launch_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int n_qt, int n_kt, int n_qs,
-                             int32_t* pair_base, int32_t* kt_slot, int32_t* slot_table, hipStream_t stream);
+                             int32_t* pair_base, int32_t* kt_slot, int32_t* slot_table, int32_t* bounds, hipStream_t stream);
 
 }  // namespace fba

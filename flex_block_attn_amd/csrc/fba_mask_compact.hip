@@ -122,7 +122,8 @@ hipError_t launch_tile_lists(const uint8_t* mask, int64_t mask_bh, int nQ, int n
 // query-major kernel finds what the key-major kernel stored: for J = q_idx[m, I, e], q_slot[m, I, e] = pair_base[m, J] +
 // position of I in the ascending row k_idx[m, J, :] (binary search).  Integer work, independent of scheduling.
 __global__ __attribute__((amdgpu_flat_work_group_size(1024, 1024))) void pair_base_kernel(const int32_t* __restrict__ k_cnt, int64_t n,
-                                                                                          int32_t* __restrict__ pair_base) {
+                                                                                          int32_t* __restrict__ pair_base, int64_t head_rows,
+                                                                                          int32_t* __restrict__ bounds) {
   __shared__ int32_t wave_sum[16];
   __shared__ int32_t carry_s;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -142,11 +143,87 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1024, 1024))) void pair_ba
     int32_t before = carry_s;
     for (int w = 0; w < wv; ++w) before += wave_sum[w];
     if (t < n) pair_base[t] = before + incl - x;
+    if (bounds != nullptr && t < n && t % head_rows == 0) bounds[t / head_rows] = before + incl - x;
     __syncthreads();
     if (tid == 1023) carry_s = before + incl;
     __syncthreads();
   }
-  if (tid == 0) pair_base[n] = carry_s;
+  if (tid == 0) {
+    pair_base[n] = carry_s;
+    if (bounds != nullptr) bounds[n / head_rows] = carry_s;
+  }
+}
+
+// Both steps in one launch, where there are so few rows that every work-group can add up what lies in front of its head by itself.  Bound by
+// latency: each of two launches waited for a chain of loads (4.4 and 4.9 us and a gap; together 5.5 to 6.5).  A third of the list is left
+// after every step of the search, from three loads side by side.
+constexpr int kMostOwnRows = 16384;  // of k_cnt
+constexpr int kMostOwnBlocks = 2048;  // of a head
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void pair_slots_kernel(
+    const int32_t* __restrict__ q_cnt, const int32_t* __restrict__ q_idx, const int32_t* __restrict__ k_cnt, const int32_t* __restrict__ k_idx,
+    int64_t mask_bh, int nQ, int nK, int blocks_per_head, int32_t* __restrict__ pair_base, int32_t* __restrict__ q_slot, int32_t* __restrict__ bounds) {
+  __shared__ int32_t base[kMostOwnBlocks];  // of the head's key blocks, from its first pair on
+  __shared__ int32_t sums[4];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int m = (int)blockIdx.x / blocks_per_head, part = (int)blockIdx.x - m * blocks_per_head;
+  // this thread's entry: where query block I lies in the list of key block J
+  const int entry = part * 256 + tid;
+  const bool in = entry < nQ * nK;
+  const int I = in ? entry / nK : 0, e = entry - I * nK;
+  const int64_t row = (int64_t)m * nQ + I;
+  const bool listed = in && e < q_cnt[row];
+  const int J = listed ? q_idx[row * nK + e] : 0;
+  const int32_t* const list = k_idx + ((int64_t)m * nK + J) * nQ;
+  int lo = 0, hi = listed ? k_cnt[(int64_t)m * nK + J] - 1 : 0;
+
+  int before = 0;
+  const int rows = m * nK;
+  for (int t = tid; t < rows; t += 256) before += k_cnt[t];
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) before += __shfl_xor(before, d);
+  if (lane == 0) sums[wv] = before;
+  __syncthreads();
+  const int first = sums[0] + sums[1] + sums[2] + sums[3];
+  int carry = 0;
+  for (int t0 = 0; t0 < nK; t0 += 256) {
+    const int x = t0 + tid < nK ? k_cnt[rows + t0 + tid] : 0;
+    int incl = x;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(incl, d);
+      if (lane >= d) incl += y;
+    }
+    __syncthreads();
+    if (lane == 63) sums[wv] = incl;
+    __syncthreads();
+    int at = carry + incl - x;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      at += w < wv ? sums[w] : 0;
+      carry += sums[w];
+    }
+    if (t0 + tid < nK) base[t0 + tid] = at;
+  }
+  __syncthreads();
+  if (part == 0) {
+    for (int j = tid; j < nK; j += 256) pair_base[rows + j] = first + base[j];
+    if (tid == 0) {
+      if (bounds != nullptr) bounds[m] = first;
+      if (m + 1 == mask_bh) {
+        pair_base[rows + nK] = first + carry;
+        if (bounds != nullptr) bounds[m + 1] = first + carry;
+      }
+    }
+  }
+  while (lo < hi) {  // I is in the list: the two orientations describe one mask
+    const int step = (hi - lo + 4) / 4, a = lo + step, b = min(a + step, hi), c = min(b + step, hi);
+    const int at_a = list[min(a, hi)], at_b = list[b], at_c = list[c];
+    if (I < at_a) hi = min(a, hi) - 1;
+    else if (I < at_b) { lo = min(a, hi); hi = b - 1; }
+    else if (I < at_c) { lo = b; hi = c - 1; }
+    else lo = c;
+  }
+  if (in) q_slot[row * nK + e] = listed ? first + base[J] + lo : -1;
 }
 
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void q_slot_kernel(
@@ -175,12 +252,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void q_slot_ke
 }
 
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
-                             int nQ, int nK, int32_t* pair_base, int32_t* q_slot, hipStream_t stream) {
+                             int nQ, int nK, int32_t* pair_base, int32_t* q_slot, int32_t* bounds, hipStream_t stream) {
   const int64_t n = mask_bh * nK, entries = mask_bh * nQ * nK;
   if (n <= 0 || entries <= 0) return hipSuccess;
   const int64_t blocks = (entries + 255) / 256;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(pair_base_kernel, dim3(1), dim3(1024), 0, stream, k_cnt, n, pair_base);
+  const int64_t per_head = ((int64_t)nQ * nK + 255) / 256;
+  if (n <= kMostOwnRows && nK <= kMostOwnBlocks && mask_bh * per_head <= 0x7fffffffLL) {
+    hipLaunchKernelGGL(pair_slots_kernel, dim3((unsigned)(mask_bh * per_head)), dim3(256), 0, stream, q_cnt, q_idx, k_cnt, k_idx, mask_bh, nQ, nK, (int)per_head,
+                       pair_base, q_slot, bounds);
+    return hipGetLastError();
+  }
+  hipLaunchKernelGGL(pair_base_kernel, dim3(1), dim3(1024), 0, stream, k_cnt, n, pair_base, (int64_t)nK, bounds);
   hipLaunchKernelGGL(q_slot_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, q_cnt, q_idx, k_cnt, k_idx, pair_base, mask_bh, nQ, nK, q_slot);
   return hipGetLastError();
 }
@@ -237,7 +320,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void tile_slot
 }
 
 hipError_t launch_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int n_qt, int n_kt, int n_qs,
-                             int32_t* pair_base, int32_t* kt_slot, int32_t* slot_table, hipStream_t stream) {
+                             int32_t* pair_base, int32_t* kt_slot, int32_t* slot_table, int32_t* bounds, hipStream_t stream) {
   const int64_t rows = mask_bh * n_kt, table = mask_bh * n_qt * n_kt;
   if (rows <= 0 || table <= 0 || n_qs <= 0) return hipSuccess;
   const int64_t blocks = (rows + 3) / 4;
@@ -245,7 +328,7 @@ hipError_t launch_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64
   // the per-row counts rest in the first `rows` entries of kt_slot (which has rows * n_qs >= rows entries) until the
   // prefix sum has read them
   hipLaunchKernelGGL(tile_pair_count_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, kt_cnt, kt_ent, rows, n_qs, kt_slot);
-  hipLaunchKernelGGL(pair_base_kernel, dim3(1), dim3(1024), 0, stream, kt_slot, rows, pair_base);
+  hipLaunchKernelGGL(pair_base_kernel, dim3(1), dim3(1024), 0, stream, kt_slot, rows, pair_base, (int64_t)n_kt, bounds);
   const int64_t fill_blocks = (table + 255) / 256;
   hipLaunchKernelGGL(fill_i32_kernel, dim3((unsigned)(fill_blocks < 4096 ? fill_blocks : 4096)), dim3(256), 0, stream, slot_table, table, -1);
   hipLaunchKernelGGL(tile_slots_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, kt_cnt, kt_ent, pair_base, rows, n_qt, n_kt, n_qs,

@@ -12,6 +12,7 @@
 #include <numeric>
 
 #include <ATen/ATen.h>
+#include <ATen/core/CachingHostAllocator.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/Event.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
@@ -38,7 +39,7 @@ constexpr int64_t kXcds = 8;
 // the C ABI, bound at run time
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                \
-  X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots) X(fba_tile_slots)        \
+  X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots_bounds) X(fba_tile_slots_bounds)        \
   X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) \
   X(fba_resize_rows) X(fba_resize_mask)
 
@@ -361,16 +362,20 @@ void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered)
   if (!numbered) return;
   l.pair_base = b + base;
   l.q_slot = b + q_slot;
+  // The host's copy of the numbers at the head boundaries is written by the kernel that forms them.
+  s.host_bounds = at::empty({M + 1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  int32_t* const bounds = s.host_bounds.data_ptr<int32_t>();
   if (p.tiled()) {
     l.k_slot = b + k_slot;
-    check(lib.fba_tile_slots(l.k_cnt, l.k_idx, M, l.q_rows, l.k_rows, l.pair_base, l.k_slot, l.q_slot, stream));
+    check(lib.fba_tile_slots_bounds(l.k_cnt, l.k_idx, M, l.q_rows, l.k_rows, l.pair_base, l.k_slot, l.q_slot, bounds, stream));
   } else {
-    check(lib.fba_pair_slots(l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, M, p.nQ(), p.nK(), l.pair_base, l.q_slot, stream));
+    check(lib.fba_pair_slots_bounds(l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, M, p.nQ(), p.nK(), l.pair_base, l.q_slot, bounds, stream));
   }
-  // The copy is ordered before whatever the caller enqueues next: backward waits for it alone, not for the forward kernel.
-  s.host_bounds = at::empty({M + 1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-  s.host_bounds.copy_(s.list_buffer.narrow(0, base, M * l.k_rows + 1).slice(0, 0, c10::nullopt, l.k_rows), /*non_blocking=*/true);
-  s.copied.record(c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(mask.device()));
+  // This is ordered before whatever the caller enqueues next: backward waits for it alone, not for the forward kernel.  The memory is
+  // given back to others only when this stream is through with it, also where nobody ever asks for gradients.
+  const c10::Stream on = c10::impl::VirtualGuardImpl(c10::DeviceType::CUDA).getStream(mask.device());
+  at::getHostAllocator(at::kCUDA)->record_event(bounds, s.host_bounds.storage().data_ptr().get_context(), on);
+  s.copied.record(on);
 }
 
 // Sequences that are no whole number of 128-row tiles: copies cut or padded with zeros to `len` rows, all in one launch.  A

@@ -178,6 +178,10 @@ int32_t fba_bwd_dkdv(const void* q, const void* k, const void* v, const void* d_
  */
 int32_t fba_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
                        int32_t nQ, int32_t nK, int32_t* pair_base, int32_t* q_slot, void* hip_stream);
+/* The same, leaving the numbers at the head boundaries (mask_bh + 1 of them, the last one the number of pairs) in `bounds` as well, which may be
+ * pinned host memory: the host then waits for this call, and not for a copy behind it. */
+int32_t fba_pair_slots_bounds(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,
+                       int32_t nQ, int32_t nK, int32_t* pair_base, int32_t* q_slot, int32_t* bounds, void* hip_stream);
 int32_t fba_bwd_handover(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,
                          void* ds_ws, int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* q_cnt, const int32_t* q_idx,
                          const int32_t* k_cnt, const int32_t* k_idx, const int32_t* pair_base, const int32_t* q_slot, int64_t n_pairs,
@@ -280,6 +284,9 @@ int32_t fba_bwd_tiled(const void* q, const void* k, const void* v, const void* o
  */
 int32_t fba_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int32_t n_qt, int32_t n_kt, int32_t* pair_base,
                        int32_t* kt_slot, int32_t* slot_table, void* hip_stream);
+/* See fba_pair_slots_bounds. */
+int32_t fba_tile_slots_bounds(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int32_t n_qt, int32_t n_kt, int32_t* pair_base,
+                       int32_t* kt_slot, int32_t* slot_table, int32_t* bounds, void* hip_stream);
 int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,
                                void* ds_ws, int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt,
                                const int32_t* qt_ent, const int32_t* kt_cnt, const int32_t* kt_ent, const int32_t* pair_base,
