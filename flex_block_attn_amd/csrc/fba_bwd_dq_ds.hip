@@ -37,6 +37,53 @@ constexpr int kRing = 4;
 template <int N>
 using IC = std::integral_constant<int, N>;
 
+// Tile lists, in chunks of 64 keys (two stages of the ring), which always lie in one key block and one key tile.  Every wave keeps 64 chunks in
+// registers, one per lane: key chunk << 8 | predicate bits of its block, and the number of the tile pair it lies in; they are handed out
+// by lane, so that a stage waits for no scalar load (a block of 64 keys asked for three every two stages, and every wait for one waits for
+// the LDS reads in flight as well).  All lanes of a wave call everything together.
+template <bool kDensePairs>
+struct TileChunks {
+  const int32_t* list;
+  const int32_t* slots;  // numbered pairs: by key tile
+  int slot0, slot_step;  // dense ones: of key tile 0, to the next
+  int blocks, total, lane;  // chunks of a key block, of the list
+  int base, at;             // first of the 64 at hand, the next one among them
+  uint32_t chunk, chunk_ahead;
+  int pair, pair_ahead;
+
+  FBA_DEVICE void load(int from) {
+    const int c = from + lane;
+    chunk_ahead = 0;
+    pair_ahead = 0;
+    if (c < total) {
+      const int e = c / blocks, entry = list[e];
+      const int key = (entry >> 8) * blocks + c - e * blocks;
+      chunk_ahead = (uint32_t)key << 8 | (entry & 255);
+      pair_ahead = kDensePairs ? slot0 + (key >> 1) * slot_step : slots[key >> 1];
+    }
+  }
+  FBA_DEVICE void take() {
+    chunk = chunk_ahead;
+    pair = pair_ahead;
+    at = 0;
+    load(base + 64);
+  }
+  FBA_DEVICE void start() {
+    base = 0;
+    load(0);
+    take();
+  }
+  FBA_DEVICE void next(uint32_t& c, int& p) {
+    if (at == 64) {
+      base += 64;
+      take();
+    }
+    c = (uint32_t)__builtin_amdgcn_readlane((int)chunk, at);
+    p = __builtin_amdgcn_readlane(pair, at);
+    ++at;
+  }
+};
+
 }  // namespace
 
 template <bool kTiled, int kMode, int kWaves>  // kMode: kNumbered or kDense
@@ -81,11 +128,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   // lists that number more pairs than the workspace holds: nothing is fetched, and the output becomes NaN
   const int cnt = dense || workspace_holds_lists(p) ? const_idx(p.q_cnt)[mrow] : 0;
   const ConstIdx idx = const_idx(p.q_idx + mrow * p.nK);
-  // block lists: pair number per list entry; tile lists: pair number per key tile, for this query tile
-  const ConstIdx slots = const_idx(dense ? nullptr : p.q_slot + mrow * (kTiled ? n_kt : p.nK));
+  // block lists: pair number per list entry (tile lists: see TileChunks)
+  const ConstIdx slots = const_idx(dense || kTiled ? nullptr : p.q_slot + mrow * p.nK);
   auto slot = [&](int e) -> int64_t {
     if constexpr (!dense) return slots[e];
-    else return kTiled ? ((int64_t)bh * n_kt + e) * tiles_per_head + qt : ((int64_t)bh * p.nK + idx[e]) * p.nQ + qblk;
+    else return ((int64_t)bh * p.nK + idx[e]) * p.nQ + qblk;
   };
   const int nsub = p.k_block / kSlab;
   // this work-group's range of 32-key steps of the list: all of it, or part `part` of `parts` (boundaries on whole rings)
@@ -99,7 +146,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   // the key tile with tile lists)
   const int64_t head_pairs = p.mask_bh == 1 && !dense ? (int64_t)bh * const_idx(p.pair_base)[kTiled ? n_kt : p.nK] : 0;
   const char* ds_base = reinterpret_cast<const char*>(p.ds_ws) + head_pairs * pair_bytes + ((int64_t)tq * nsub * 4 + (wave & 3)) * kDsUnitBytes;
-  auto key_block = [&](int e) -> int { return kTiled ? idx[e] >> 8 : idx[e]; };
   const int wave_bits = 3 << (2 * wave);  // predicate bits of this wave's two 16-row groups in a tile-list entry
 
   TransposedOffsets tr;
@@ -142,18 +188,41 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   // sources of the next stage to request, in list order; the following list entry is read one block ahead
   const int64_t block_bytes = (int64_t)p.k_block * kRowBytes;
   int e_next = e_begin + 1, rem = nsub - sub_begin;
-  int64_t k_off = nsteps > 0 ? key_block(e_begin) * block_bytes + (int64_t)sub_begin * kSlabBytes : 0;
+  int64_t k_off = nsteps > 0 && !kTiled ? idx[e_begin] * block_bytes + (int64_t)sub_begin * kSlabBytes : 0;
   int64_t ds_off_g = nsteps > 0 && !kTiled ? slot(e_begin) * pair_bytes + (int64_t)sub_begin * (4 * kDsUnitBytes) : 0;
-  int blk_next = e_next < cnt ? key_block(e_next) : 0;
+  int blk_next = e_next < cnt && !kTiled ? idx[e_next] : 0;
   int64_t slot_next = e_next < cnt && !kTiled ? slot(e_next) : 0;
-  // tile lists: predicate bits of the entry being requested and of the next one; pair number of the key tile that the
-  // next stage's slab lies in, read one stage ahead
-  int bits_req = kTiled && cnt > 0 ? idx[0] & 255 : 0;
-  int bits_req_next = kTiled && cnt > 1 ? idx[1] & 255 : 0;
-  int64_t tile_slot = kTiled && cnt > 0 ? slot((int)(k_off >> 15)) : 0;  // 32 KiB of K rows per key tile
+  [[maybe_unused]] TileChunks<dense> chunks;
+  uint32_t chunk = 0;                      // tile lists: the chunk whose stages are being requested (see TileChunks)
+  const char *chunk_k = kp, *chunk_ds = ds_base;
+  if constexpr (kTiled) {
+    chunks.list = p.q_idx + mrow * p.nK;
+    chunks.slots = dense ? nullptr : p.q_slot + mrow * n_kt;
+    chunks.slot0 = dense ? (int)(bh * n_kt * tiles_per_head + qt) : 0;
+    chunks.slot_step = tiles_per_head;
+    chunks.blocks = p.k_block / 64;
+    chunks.total = cnt * chunks.blocks;
+    chunks.lane = lane;
+    chunks.start();
+  }
   const uint32_t lane16 = (uint32_t)lane * 16;
-  auto copy_next = [&](int ring) {
+  auto copy_next = [&](auto ring_c) {
+    constexpr int ring = decltype(ring_c)::value;
     const uint32_t dst = ring_dst + ring * kStageBytes;
+    if constexpr (kTiled) {
+      if constexpr (ring % 2 == 0) {
+        int pair;
+        chunks.next(chunk, pair);
+        chunk_k = kp + (int64_t)(chunk >> 8) * (2 * kSlabBytes);
+        chunk_ds = (chunk & wave_bits) != 0 ? ds_base + pair * pair_bytes + (chunk >> 8 & 1) * (8 * kDsUnitBytes) : nullptr;
+      }
+      const char* const src = chunk_ds != nullptr ? chunk_ds + ring % 2 * (4 * kDsUnitBytes) : p.zero_unit;
+      dma16(dst + k_dst_wave, chunk_k + ring % 2 * kSlabBytes, k_off_lane[0]);
+      dma16(dst + k_dst_wave + 4 * kRowBytes, chunk_k + ring % 2 * kSlabBytes, k_off_lane[1]);
+      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes, src, lane16);
+      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes + 1024, src, lane16 + 1024);
+      return;
+    }
     if constexpr (kWaves == 4) {
       dma16(dst + k_dst_wave, kp + k_off, k_off_lane[0]);
       dma16(dst + k_dst_wave + 4 * kRowBytes, kp + k_off, k_off_lane[1]);
@@ -161,45 +230,38 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
       if (copies_k) dma16(dst + k_dst_wave, kp + k_off, k_off_lane[0]);
     }
     const char* src = ds_base + ds_off_g;
-    if constexpr (kTiled) {
-      const int t = (int)(k_off >> 13) & 3;  // 32-key slab inside its key tile
-      src = (bits_req & wave_bits) != 0 ? ds_base + tile_slot * pair_bytes + t * (4 * kDsUnitBytes) : p.zero_unit;
-    }
     dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes, src, lane16);
     dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes + 1024, src, lane16 + 1024);
     if (--rem == 0) {
       rem = nsub;
       k_off = blk_next * block_bytes;
       ds_off_g = slot_next * pair_bytes;
-      bits_req = bits_req_next;
       ++e_next;
-      blk_next = e_next < cnt ? key_block(e_next) : 0;
-      if constexpr (kTiled) bits_req_next = e_next < cnt ? idx[e_next] & 255 : 0;
-      else slot_next = e_next < cnt ? slot(e_next) : 0;
+      blk_next = e_next < cnt ? idx[e_next] : 0;
+      slot_next = e_next < cnt ? slot(e_next) : 0;
     } else {
       k_off += kSlabBytes;
       ds_off_g += 4 * kDsUnitBytes;
     }
-    if constexpr (kTiled) tile_slot = slot((int)(k_off >> 15));  // past the last stage: some listed tile's number, unused
   };
 
   if (nsteps > 0) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (j < nsteps) copy_next(j);
+    // tile lists: predicate bits of the chunk whose two stages are worked on, for stages 0, 1 and 2, 3 of the ring; 0 past the end
+    uint32_t bits[2] = {255, 255}, bits_new = 0;
+    if (0 < nsteps) copy_next(IC<0>{});
+    if constexpr (kTiled) bits[0] = chunk;
+    if (1 < nsteps) copy_next(IC<1>{});
+    if (2 < nsteps) copy_next(IC<2>{});
+    if constexpr (kTiled) bits[1] = 2 < nsteps ? chunk : 0;
+    if (3 < nsteps) copy_next(IC<3>{});
     wait_vmem<0>();
     __syncthreads();
-
-    // tile lists: predicate bits of the entry whose slab is worked on (a second walk over the list)
-    int e_cmp = 0, rem_cmp = nsub;
-    int bits_cmp = kTiled ? idx[0] & 255 : 255;
-    int bits_ahead = kTiled && cnt > 1 ? idx[1] & 255 : 0;
 
     // step t (t % 4 == R): dQ += K_t^T dS_t
     auto step = [&](auto ring_c, int t) {
       constexpr int R = decltype(ring_c)::value;
       const char* stage = smem + R * kStageBytes;
-      if (!kTiled || (bits_cmp & wave_bits) != 0) {
+      if (!kTiled || (bits[R / 2] & wave_bits) != 0) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
           const bf16x8 dsk = cat(lds_read_tr(stage, ds_off[j][0]), lds_read_tr(stage, ds_off[j][1]));
@@ -211,18 +273,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
           }
         }
       }
-      if constexpr (kTiled) {
-        if (--rem_cmp == 0) {
-          rem_cmp = nsub;
-          ++e_cmp;
-          bits_cmp = bits_ahead;
-          bits_ahead = e_cmp + 1 < cnt ? idx[e_cmp + 1] & 255 : 0;
-        }
-      }
       // stage t+1 must have landed (first read in step t+1); the copies of stages t+2 and t+3 may still fly
       if (t + 3 < nsteps) wait_stages(IC<2>{}); else if (t + 2 < nsteps) wait_stages(IC<1>{}); else wait_stages(IC<0>{});
       __syncthreads();
-      if (t + 4 < nsteps) copy_next(R);
+      if (t + 4 < nsteps) copy_next(IC<R>{});
+      if constexpr (kTiled) {
+        if constexpr (R % 2 == 0) bits_new = t + 4 < nsteps ? chunk : 0;
+        else bits[R / 2] = bits_new;
+      }
     };
     for (int t = 0; t < nsteps; t += 4) {  // nsteps is a multiple of 4
       step(IC<0>{}, t);
