@@ -154,11 +154,27 @@ __global__ __attribute__((amdgpu_flat_work_group_size(1024, 1024))) void pair_ba
   }
 }
 
+// Where I, which is in it, lies in an ascending list (the two orientations describe one mask): a quarter is left after every step, from
+// three loads side by side.
+FBA_DEVICE int position_of(const int32_t* __restrict__ list, int count, int I) {
+  int lo = 0, hi = count - 1;
+  while (lo < hi) {
+    const int step = (hi - lo + 4) / 4, a = lo + step, b = min(a + step, hi), c = min(b + step, hi);
+    const int at_a = list[a], at_b = list[b], at_c = list[c];
+    if (I < at_a) hi = a - 1;
+    else if (I < at_b) { lo = a; hi = b - 1; }
+    else if (I < at_c) { lo = b; hi = c - 1; }
+    else lo = c;
+  }
+  return lo;
+}
+
 // Both steps in one launch, where there are so few rows that every work-group can add up what lies in front of its head by itself.  Bound by
-// latency: each of two launches waited for a chain of loads (4.4 and 4.9 us and a gap; together 5.5 to 6.5).  A third of the list is left
-// after every step of the search, from three loads side by side.
+// latency: each of two launches waited for a chain of loads (4.4 and 4.9 us and a gap; together 5.5 to 6.5).
 constexpr int kMostOwnRows = 16384;  // of k_cnt
 constexpr int kMostOwnBlocks = 2048;  // of a head
+// One round of work-groups: with more of them the sums are formed over and over (24 heads of 540 x 180 blocks 36 us, in two launches 9 + 19).
+constexpr int64_t kMostOwnGroups = 2048;
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void pair_slots_kernel(
     const int32_t* __restrict__ q_cnt, const int32_t* __restrict__ q_idx, const int32_t* __restrict__ k_cnt, const int32_t* __restrict__ k_idx,
     int64_t mask_bh, int nQ, int nK, int blocks_per_head, int32_t* __restrict__ pair_base, int32_t* __restrict__ q_slot, int32_t* __restrict__ bounds) {
@@ -174,7 +190,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void pair_slot
   const bool listed = in && e < q_cnt[row];
   const int J = listed ? q_idx[row * nK + e] : 0;
   const int32_t* const list = k_idx + ((int64_t)m * nK + J) * nQ;
-  int lo = 0, hi = listed ? k_cnt[(int64_t)m * nK + J] - 1 : 0;
+  const int count = listed ? k_cnt[(int64_t)m * nK + J] : 0;
 
   int before = 0;
   const int rows = m * nK;
@@ -215,15 +231,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void pair_slot
       }
     }
   }
-  while (lo < hi) {  // I is in the list: the two orientations describe one mask
-    const int step = (hi - lo + 4) / 4, a = lo + step, b = min(a + step, hi), c = min(b + step, hi);
-    const int at_a = list[min(a, hi)], at_b = list[b], at_c = list[c];
-    if (I < at_a) hi = min(a, hi) - 1;
-    else if (I < at_b) { lo = min(a, hi); hi = b - 1; }
-    else if (I < at_c) { lo = b; hi = c - 1; }
-    else lo = c;
-  }
-  if (in) q_slot[row * nK + e] = listed ? first + base[J] + lo : -1;
+  const int at = listed ? position_of(list, count, I) : 0;
+  if (in) q_slot[row * nK + e] = listed ? first + base[J] + at : -1;
 }
 
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void q_slot_kernel(
@@ -240,13 +249,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void q_slot_ke
   if (e < q_cnt[row]) {
     const int J = q_idx[t];
     const int64_t krow = m * nK + J;
-    const int32_t* list = k_idx + krow * nQ;
-    int lo = 0, hi = k_cnt[krow] - 1;
-    while (lo < hi) {  // I is in the list: the two orientations describe one mask
-      const int mid = (lo + hi) >> 1;
-      if (list[mid] < I) lo = mid + 1; else hi = mid;
-    }
-    out = pair_base[krow] + lo;
+    out = pair_base[krow] + position_of(k_idx + krow * nQ, k_cnt[krow], I);
   }
   q_slot[t] = out;
 }
@@ -258,7 +261,7 @@ hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const i
   const int64_t blocks = (entries + 255) / 256;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
   const int64_t per_head = ((int64_t)nQ * nK + 255) / 256;
-  if (n <= kMostOwnRows && nK <= kMostOwnBlocks && mask_bh * per_head <= 0x7fffffffLL) {
+  if (n <= kMostOwnRows && nK <= kMostOwnBlocks && mask_bh * per_head <= kMostOwnGroups) {
     hipLaunchKernelGGL(pair_slots_kernel, dim3((unsigned)(mask_bh * per_head)), dim3(256), 0, stream, q_cnt, q_idx, k_cnt, k_idx, mask_bh, nQ, nK, (int)per_head,
                        pair_base, q_slot, bounds);
     return hipGetLastError();

@@ -162,26 +162,51 @@ constexpr int kMostOrdered = 2048;  // items of a launch that is ordered at all:
 // kernels exponentiate in base 2, hence the pre-scaled LSE; they start the dP accumulators from the second plane, so that
 // the matrix instructions themselves form dP - delta (the reference preloads its accumulator the same way,
 // flex_block_attn_h100.cu:445-467), hence the sign.  16 lanes per row (16 bytes of each operand per lane); 256 threads to a block.
-constexpr int kStatsRows = 16;
-FBA_DEVICE void stats_rows(const BwdStats& s, int block, int blocks) {
+//
+// Bound by memory: 524 bytes of a row, each once.  With a row to 16 lanes the blocks ended as soon as their two loads had come back, so that
+// starting them set the pace; launches that fill the GPU with four rows to 16 lanes request all eight loads first (262144 rows 30.1 -> 22.1 us,
+// 6.2 TB/s; 552960 rows 64.2 -> 55.7 us, 5.2 TB/s).
+constexpr int kStatsRows = 16, kStatsDeep = 4;
+constexpr int64_t kStatsMany = 131072;  // rows: eight blocks of 64 rows for each of 256 compute units
+__host__ __device__ inline bool stats_deep(const BwdStats& s) { return s.rows >= kStatsMany; }
+template <int kDeep>
+FBA_DEVICE void stats_rows_of(const BwdStats& s, int block, int blocks) {
   const int sub = threadIdx.x & 15;
-  for (int64_t r = (int64_t)block * kStatsRows + (threadIdx.x >> 4); r < s.rows; r += (int64_t)blocks * kStatsRows) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(s.o + r * kHeadDim + sub * 8);
-    const bf16x8 b = *reinterpret_cast<const bf16x8*>(s.d_o + r * kHeadDim + sub * 8);
-    float acc = 0.f;
+  for (int64_t r0 = (int64_t)block * (kStatsRows * kDeep) + (threadIdx.x >> 4); r0 < s.rows; r0 += (int64_t)blocks * (kStatsRows * kDeep)) {
+    bf16x8 a[kDeep], b[kDeep];
+    float lse[kDeep];
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc += (float)a[t] * (float)b[t];
-    acc += __shfl_xor(acc, 8);
-    acc += __shfl_xor(acc, 4);
-    acc += __shfl_xor(acc, 2);
-    acc += __shfl_xor(acc, 1);
-    if (sub == 0) {
-      s.stats[r] = s.lse[r] * 1.4426950408889634f;
-      s.stats[s.rows + r] = -acc;
+    for (int d = 0; d < kDeep; ++d) {
+      const int64_t r = r0 + d * kStatsRows < s.rows ? r0 + d * kStatsRows : r0;
+      a[d] = *reinterpret_cast<const bf16x8*>(s.o + r * kHeadDim + sub * 8);
+      b[d] = *reinterpret_cast<const bf16x8*>(s.d_o + r * kHeadDim + sub * 8);
+      lse[d] = s.lse[r];
+    }
+#pragma unroll
+    for (int d = 0; d < kDeep; ++d) {
+      const int64_t r = r0 + d * kStatsRows;
+      float acc = 0.f;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) acc += (float)a[d][t] * (float)b[d][t];
+      acc += __shfl_xor(acc, 8);
+      acc += __shfl_xor(acc, 4);
+      acc += __shfl_xor(acc, 2);
+      acc += __shfl_xor(acc, 1);
+      if (sub == 0 && r < s.rows) {
+        s.stats[r] = lse[d] * 1.4426950408889634f;
+        s.stats[s.rows + r] = -acc;
+      }
     }
   }
 }
-int stats_blocks(const BwdStats& s) { return (int)std::min<int64_t>((s.rows + kStatsRows - 1) / kStatsRows, 65536); }
+FBA_DEVICE void stats_rows(const BwdStats& s, int block, int blocks) {
+  if (stats_deep(s)) stats_rows_of<kStatsDeep>(s, block, blocks);
+  else stats_rows_of<1>(s, block, blocks);
+}
+int stats_blocks(const BwdStats& s) {
+  const int rows = kStatsRows * (stats_deep(s) ? kStatsDeep : 1);
+  return (int)std::min<int64_t>((s.rows + rows - 1) / rows, 65536);
+}
 
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void bwd_stats_kernel(const BwdStats s) { stats_rows(s, blockIdx.x, gridDim.x); }
 

@@ -1,6 +1,6 @@
 """Numbers of the listed pairs and their values at the head boundaries (fba_pair_slots_bounds, fba_tile_slots_bounds): in one launch where
 few rows lie in front of a head, in two beyond that.  One entry, a work-group's worth and one more, the largest head and the most rows
-of the one launch and one more of each, one mask for all heads, empty heads; the boundaries in device and in pinned host memory.  Exact."""
+of the one launch and one more of each, as many work-groups as it may have and more, one mask for all heads, empty heads; the boundaries in device and in pinned host memory.  Exact."""
 import pytest
 import torch
 
@@ -23,7 +23,7 @@ def _call(name, *args):
 
 @pytest.mark.parametrize("M,nQ,nK,density", [
     (1, 1, 1, 1.0), (1, 1, 1, 0.0), (3, 16, 16, 0.4), (3, 257, 1, 0.5), (1, 7, 2048, 0.3), (1, 7, 2049, 0.3), (8, 5, 2048, 0.2), (129, 3, 127, 0.6), (2, 300, 63, 0.9),
-    (5, 540, 180, 0.1),
+    (5, 540, 180, 0.1), (6, 540, 180, 0.1),
 ])
 @pytest.mark.parametrize("pinned", [False, True])
 def test_pair_numbers(gpu, M, nQ, nK, density, pinned):
