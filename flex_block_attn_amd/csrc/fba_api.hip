@@ -318,7 +318,7 @@ int32_t fba_tile_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t
   if (int rc = check_tile_list_shape(nQ, nK, q_block, k_block)) return rc;
   const int64_t Sq = (int64_t)nQ * q_block, Skv = (int64_t)nK * k_block;
   if (!mask || !qt_cnt || !qt_ent || !kt_cnt || !kt_ent) return fail(FBA_ERR_INVALID, "null pointer argument");
-  hipError_t e = fba::launch_tile_lists(mask, mask_bh, nQ, nK, q_block, k_block, (int)(Sq / 128), (int)(Skv / 128), (int)(Sq / 32),
+  hipError_t e = fba::launch_tile_lists(mask, mask_bh, nQ, nK, nK, q_block, k_block, (int)(Sq / 128), (int)(Skv / 128), (int)(Sq / 32),
                                         qt_cnt, qt_ent, kt_cnt, kt_ent, (hipStream_t)hip_stream);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "tile_lists launch");
 }
@@ -327,6 +327,7 @@ static int fill_bwd(fba::BwdParams& p, const Shape& s) {
   p.mask_bh = s.mask_bh;
   p.B = s.B; p.Hq = s.Hq; p.Hkv = s.Hkv; p.Sq = s.Sq; p.Skv = s.Skv; p.nQ = s.Sq / s.q_block; p.nK = s.Skv / s.k_block;
   p.q_block = s.q_block; p.k_block = s.k_block;
+  p.out_q = s.Sq; p.out_kv = s.Skv;
   p.scale = 1.f / 11.313708498984761f;
   p.scale_log2e = 1.4426950408889634f / 11.313708498984761f;
   return FBA_OK;
@@ -608,40 +609,67 @@ int32_t fba_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mas
   return fba_tile_slots_bounds(kt_cnt, kt_ent, mask_bh, n_qt, n_kt, pair_base, kt_slot, slot_table, nullptr, hip_stream);
 }
 
+static int bwd_tiled_impl(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats, void* ds_ws,
+                          int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt, const int32_t* qt_ent, const int32_t* kt_cnt,
+                          const int32_t* kt_ent, const int32_t* pair_base, const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh,
+                          int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t out_q, int32_t out_kv, int32_t head_dim, int32_t q_block,
+                          int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream, bool numbered) {
+  const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
+  if (int rc = check_shape(s)) return rc;
+  if (int rc = check_lists(s, true, "backward")) return rc;
+  if (int rc = check_split_ws(split_ws, split_ws_bytes)) return rc;
+  // everything is validated before the first launch, so that a rejected call leaves nothing on the stream
+  if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}})) return rc;
+  if (numbered || ds_ws != nullptr)
+    if (int rc = check_ptrs({{"ds_ws", ds_ws}})) return rc;
+  if (!lse || !stats || !qt_cnt || !qt_ent || !kt_cnt || !kt_ent || (numbered && (!pair_base || !kt_slot || !slot_table))) return fail(FBA_ERR_INVALID, "null pointer argument");
+  if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
+  if (out_q <= 0 || out_q > Sq || out_kv <= 0 || out_kv > Skv)
+    return fail(FBA_ERR_INVALID, "out_q (%d) and out_kv (%d) must be positive and Sq, Skv (%d, %d) at most", out_q, out_kv, Sq, Skv);
+  if (ds_ws != nullptr) {
+    if (n_pairs < 0) return fail(FBA_ERR_INVALID, "n_pairs must not be negative");
+    const int64_t pairs = numbered ? n_pairs : (int64_t)B * Hq * (Sq / 128) * (Skv / 128), need = pairs * 128 * 128 * 2;
+    if (ds_ws_bytes < need)
+      return fail(FBA_ERR_INVALID, "backward: ds_ws holds %lld bytes, %lld tile pairs of 128 x 128 need %lld", (long long)ds_ws_bytes, (long long)pairs,
+                  (long long)need);
+  }
+  fba::BwdParams p{};
+  fill_bwd(p, s);
+  p.make = {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq};
+  p.tiled = 1;
+  p.out_q = out_q; p.out_kv = out_kv;
+  p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
+  p.stats = stats; p.dq = (__bf16*)dq; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv;
+  p.q_cnt = qt_cnt; p.q_idx = qt_ent; p.k_cnt = kt_cnt; p.k_idx = kt_ent;
+  p.ds_ws = (__bf16*)ds_ws;
+  if (numbered) {
+    p.pair_base = pair_base; p.k_slot = kt_slot; p.q_slot = slot_table;
+    p.ws_pairs = ds_ws_bytes / (128 * 128 * 2);
+  }
+  p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
+  hipError_t e = fba::launch_bwd_dkdv_slab(p, (hipStream_t)hip_stream);
+  if (e != hipSuccess) return hip_fail(e, "dkdv (tile lists) launch");
+  e = ds_ws != nullptr ? fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream) : fba::launch_bwd_dq(p, (hipStream_t)hip_stream);
+  return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (tile lists) launch");
+}
+
+int32_t fba_bwd_tiled_cut(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats, void* ds_ws,
+                          int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt, const int32_t* qt_ent, const int32_t* kt_cnt,
+                          const int32_t* kt_ent, const int32_t* pair_base, const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh,
+                          int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t out_q, int32_t out_kv, int32_t head_dim, int32_t q_block,
+                          int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream) {
+  return bwd_tiled_impl(q, k, v, o, d_o, lse, stats, ds_ws, ds_ws_bytes, dq, dk, dv, qt_cnt, qt_ent, kt_cnt, kt_ent, pair_base, kt_slot, slot_table, n_pairs,
+                        mask_bh, B, Hq, Hkv, Sq, Skv, out_q, out_kv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, ds_ws != nullptr && pair_base != nullptr);
+}
+
 int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,
                                void* ds_ws, int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt,
                                const int32_t* qt_ent, const int32_t* kt_cnt, const int32_t* kt_ent, const int32_t* pair_base,
                                const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh, int32_t B,
                                int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block,
                                void* split_ws, int64_t split_ws_bytes, void* hip_stream) {
-  const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
-  if (int rc = check_shape(s)) return rc;
-  if (int rc = check_lists(s, true, "backward")) return rc;
-  if (int rc = check_split_ws(split_ws, split_ws_bytes)) return rc;
-  // everything is validated before the first launch, so that a rejected call leaves nothing on the stream
-  if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}, {"ds_ws", ds_ws}})) return rc;
-  if (!lse || !stats || !qt_cnt || !qt_ent || !kt_cnt || !kt_ent || !pair_base || !kt_slot || !slot_table)
-    return fail(FBA_ERR_INVALID, "null pointer argument");
-  if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
-  if (n_pairs < 0) return fail(FBA_ERR_INVALID, "n_pairs must not be negative");
-  const int64_t need = n_pairs * 128 * 128 * 2;
-  if (ds_ws_bytes < need)
-    return fail(FBA_ERR_INVALID, "backward: ds_ws holds %lld bytes, %lld tile pairs of 128 x 128 need %lld", (long long)ds_ws_bytes,
-                (long long)n_pairs, (long long)need);
-  fba::BwdParams p{};
-  fill_bwd(p, s);
-  p.make = {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq};
-  p.tiled = 1;
-  p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
-  p.stats = stats; p.dq = (__bf16*)dq; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv;
-  p.q_cnt = qt_cnt; p.q_idx = qt_ent; p.k_cnt = kt_cnt; p.k_idx = kt_ent;
-  p.ds_ws = (__bf16*)ds_ws; p.pair_base = pair_base; p.k_slot = kt_slot; p.q_slot = slot_table;
-  p.ws_pairs = ds_ws_bytes / (128 * 128 * 2);
-  p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = fba::launch_bwd_dkdv_slab(p, (hipStream_t)hip_stream);
-  if (e != hipSuccess) return hip_fail(e, "dkdv (tile lists, hand-over) launch");
-  e = fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream);
-  return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (from dS, tile lists) launch");
+  return bwd_tiled_impl(q, k, v, o, d_o, lse, stats, ds_ws, ds_ws_bytes, dq, dk, dv, qt_cnt, qt_ent, kt_cnt, kt_ent, pair_base, kt_slot, slot_table, n_pairs,
+                        mask_bh, B, Hq, Hkv, Sq, Skv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, true);
 }
 
 }  // extern "C"
@@ -680,26 +708,31 @@ int scratch_address(float** out) {
 
 extern "C" {
 
-int32_t fba_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block, int32_t* q_cnt,
-                  int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream) {
+int32_t fba_lists_cut(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t mask_q, int32_t mask_k, int32_t q_block, int32_t k_block,
+                      int32_t* q_cnt, int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream) {
   const bool both = k_cnt != nullptr && k_idx != nullptr;
   if (!both && (k_cnt != nullptr || k_idx != nullptr)) return fail(FBA_ERR_INVALID, "k_cnt and k_idx must both be given or both be null");
-  if (both) {
-    return q_block % 128 == 0 && k_block % 128 == 0 ? fba_mask_compact(mask, mask_bh, nQ, nK, q_cnt, q_idx, k_cnt, k_idx, hip_stream)
-                                                    : fba_tile_lists(mask, mask_bh, nQ, nK, q_block, k_block, q_cnt, q_idx, k_cnt, k_idx, hip_stream);
-  }
   if (mask_bh <= 0 || nQ <= 0 || nK <= 0)
     return fail(FBA_ERR_INVALID, "mask_bh, nQ, nK must be positive (got %lld %d %d)", (long long)mask_bh, nQ, nK);
+  if (mask_q <= 0 || mask_q > nQ || mask_k <= 0 || mask_k > nK)
+    return fail(FBA_ERR_INVALID, "the mask's rows and columns (%d, %d) must be positive and nQ, nK (%d, %d) at most", mask_q, mask_k, nQ, nK);
   if (!mask || !q_cnt || !q_idx) return fail(FBA_ERR_INVALID, "null pointer argument");
   hipError_t e;
   if (q_block % 128 == 0 && k_block % 128 == 0) {
-    e = fba::launch_mask_compact(mask, mask_bh, nQ, nK, q_cnt, q_idx, nullptr, nullptr, (hipStream_t)hip_stream);
+    if (mask_q != nQ || mask_k != nK) return fail(FBA_ERR_INVALID, "block lists are of whole masks (got %d, %d of %d, %d)", mask_q, mask_k, nQ, nK);
+    e = fba::launch_mask_compact(mask, mask_bh, nQ, nK, q_cnt, q_idx, k_cnt, k_idx, (hipStream_t)hip_stream);
   } else {
     if (int rc = check_tile_list_shape(nQ, nK, q_block, k_block)) return rc;
-    e = fba::launch_tile_lists(mask, mask_bh, nQ, nK, q_block, k_block, (int)((int64_t)nQ * q_block / 128), 0, 0, q_cnt, q_idx, nullptr,
-                               nullptr, (hipStream_t)hip_stream);
+    const int64_t Sq = (int64_t)nQ * q_block, Skv = (int64_t)nK * k_block;
+    e = fba::launch_tile_lists(mask, mask_bh, mask_q, mask_k, nK, q_block, k_block, (int)(Sq / 128), both ? (int)(Skv / 128) : 0, (int)(Sq / 32), q_cnt, q_idx,
+                               k_cnt, k_idx, (hipStream_t)hip_stream);
   }
   return e == hipSuccess ? FBA_OK : hip_fail(e, "list launch");
+}
+
+int32_t fba_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block, int32_t* q_cnt,
+                  int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream) {
+  return fba_lists_cut(mask, mask_bh, nQ, nK, nQ, nK, q_block, k_block, q_cnt, q_idx, k_cnt, k_idx, hip_stream);
 }
 
 int32_t fba_resize_rows(int32_t n, const void* const* src, void* const* dst, const int64_t* n_seq, const int32_t* src_len, const int32_t* dst_len,

@@ -343,6 +343,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   // had put there, in three rounds, and stores of 8 bytes to 32 rows, before / now: B2 H16 S8192, 64-token blocks, 16 and 32 of 128
   // kept 442 / 424 and 707 / 691 us.  What is left beside the slabs is 2 us for the claim, 6.2 to 6.7 until the first products, 4 here.)
   const float poison = kHandOver ? poison_unless_fit(p) : 1.f;
+  const int64_t out_row0 = krow0 - (int64_t)bhk * (p.Skv - p.out_kv);
+  const int out_left = p.out_kv - kt * kTK;
   auto finish = [&](const f32x16 (&a)[4], int which, __bf16* out, float oscale) {
     f32x4* dst = reinterpret_cast<f32x4*>(smem + wave * 16384) + l32 * 32;
 #pragma unroll
@@ -366,8 +368,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         *reinterpret_cast<f32x4*>(part_out + row * kHeadDim + 4 * c8) = sum[0];
         *reinterpret_cast<f32x4*>(part_out + row * kHeadDim + 4 * c8 + 4) = sum[1];
       } else {
-        *reinterpret_cast<bf16x8*>(out + (krow0 + row) * kHeadDim + 4 * c8) =
-            pack8(sum[0][0], sum[0][1], sum[0][2], sum[0][3], sum[1][0], sum[1][1], sum[1][2], sum[1][3]);
+        if (row < out_left)
+          *reinterpret_cast<bf16x8*>(out + (out_row0 + row) * kHeadDim + 4 * c8) =
+              pack8(sum[0][0], sum[0][1], sum[0][2], sum[0][3], sum[1][0], sum[1][1], sum[1][2], sum[1][3]);
       }
     }
   };
@@ -387,7 +390,7 @@ hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes, stream, p);
   const int split_items = p.num_items - p.split.first;
   if (split_items > 0) {
-    const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, kTK * kHeadDim}};
+    const PartialOut outs[2] = {{p.dv, 1.f, 0, p.Skv, p.out_kv}, {p.dk, p.scale, kTK * kHeadDim, p.Skv, p.out_kv}};
     return launch_partial_sum(p.split, kSlotFloats, kTK, outs, 2, p.order, stream);
   }
   return hipGetLastError();

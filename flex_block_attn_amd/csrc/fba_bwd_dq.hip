@@ -227,7 +227,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) = (f32x4){acc[mb][4 * g + 0], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]};
     return;
   }
-  __bf16* orow = p.dq + (qrow0 + l32) * kHeadDim;
+  if (kTiled && wave * 32 + l32 >= p.out_q - qt * TQ) return;
+  __bf16* orow = p.dq + (qrow0 + l32 - (kTiled ? (int64_t)bh * (p.Sq - p.out_q) : 0)) * kHeadDim;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll

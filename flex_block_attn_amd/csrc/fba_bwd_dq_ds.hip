@@ -302,7 +302,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     return;
   }
   // (the ring is free: the last step ended with a barrier and requested nothing)
-  store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + qrow0 * kHeadDim, lane);
+  if constexpr (kTiled)
+    store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + (qrow0 - (int64_t)bh * (p.Sq - p.out_q)) * kHeadDim, lane, p.out_q - qt * TQ - wave * 32);
+  else
+    store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + qrow0 * kHeadDim, lane);
 }
 
 namespace {
@@ -378,11 +381,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_s
         src += slot_floats;
       }
     const int64_t item = order != nullptr ? order[split.first + it] : split.first + it;
+    int64_t out_row = item * rows + r;
+    if (o.head_rows != o.out_rows) {
+      const int64_t head = out_row / o.head_rows;
+      const int at = (int)(out_row - head * o.head_rows);
+      if (at >= o.out_rows) continue;
+      out_row = head * o.out_rows + at;
+    }
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int q = 0; q < kMostParts; ++q)
       if (q < parts) acc += of[q];
-    *reinterpret_cast<bf16x4*>(o.out + (item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
+    *reinterpret_cast<bf16x4*>(o.out + out_row * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
   }
 }
 

@@ -434,8 +434,8 @@ struct TransposedOffsets {
 // rows at `out`.  By way of 8 KiB of LDS that nobody else uses, so that a store fills four whole rows; straight from the
 // registers a store would put 8 bytes into each of 32 rows (2 to 2.7 us a work-group).  This and read_ahead, before / now: forward
 // of B2 H16/4 S8192, 128-token blocks, 4, 8 and 16 of 64 kept 97.6 / 88.3, 165 / 157 and 285 / 280 us, dQ from dS 79.8 / 71.2, 131 / 121
-// and 222 / 214.
-FBA_DEVICE void store_tile_bf16(char* buf, const f32x16 (&acc)[4], float scale, __bf16* out, int lane) {
+// and 222 / 214.  Rows from `rows` on are left out.
+FBA_DEVICE void store_tile_bf16(char* buf, const f32x16 (&acc)[4], float scale, __bf16* out, int lane, int rows = 32) {
   const int l32 = lane & 31, h = lane >> 5;
 #pragma unroll
   for (int mb = 0; mb < 4; ++mb)
@@ -445,7 +445,8 @@ FBA_DEVICE void store_tile_bf16(char* buf, const f32x16 (&acc)[4], float scale, 
           pack4(acc[mb][4 * g + 0] * scale, acc[mb][4 * g + 1] * scale, acc[mb][4 * g + 2] * scale, acc[mb][4 * g + 3] * scale);
 #pragma unroll
   for (int i = 0; i < 8; ++i)
-    *reinterpret_cast<bf16x8*>(out + i * 4 * kHeadDim + lane * 8) = lds_read_b128(buf, tile_off(4 * i + (lane >> 4), lane & 15));
+    if (4 * i + (lane >> 4) < rows)
+      *reinterpret_cast<bf16x8*>(out + i * 4 * kHeadDim + lane * 8) = lds_read_b128(buf, tile_off(4 * i + (lane >> 4), lane & 15));
 }
 
 // The 32-key slabs that some row of the work-group selects, in order.  All lanes of a wave call everything together.

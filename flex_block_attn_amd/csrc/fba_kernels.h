@@ -203,6 +203,7 @@ struct BwdParams {
   const int32_t* k_idx;
   int64_t mask_bh;
   int B, Hq, Hkv, Sq, Skv, nQ, nK, q_block, k_block;
+  int out_q, out_kv;  // rows of a head of dq and of dk, dv; with tile lists they may have fewer than q and k: none for what fills up the last tile
   float scale;        // 1 / sqrt(head_dim)
   float scale_log2e;  // log2(e) / sqrt(head_dim)
   int num_items, items_per_xcd;
@@ -247,7 +248,7 @@ constexpr int kRecompute = 0, kNumbered = 1, kDense = 2;
 
 hipError_t launch_mask_compact(const uint8_t* mask, int64_t mask_bh, int nQ, int nK, int32_t* q_cnt, int32_t* q_idx,
                                int32_t* k_cnt, int32_t* k_idx, hipStream_t stream);
-hipError_t launch_tile_lists(const uint8_t* mask, int64_t mask_bh, int nQ, int nK, int q_block, int k_block, int n_qt,
+hipError_t launch_tile_lists(const uint8_t* mask, int64_t mask_bh, int mask_q, int mask_k, int nK, int q_block, int k_block, int n_qt,
                              int n_kt, int n_qs, int32_t* qt_cnt, int32_t* qt_ent, int32_t* kt_cnt, int32_t* kt_ent,
                              hipStream_t stream);
 // Sliding window over blocks that are the tiles of a (t, h, w) grid of `n` tiles, T-major: tile j is in the window of tile i when on every
@@ -301,11 +302,13 @@ hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream);
 // among it.
 hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream, bool takes_pieces = false);
 int device_compute_units();
-// One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats).
+// One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats); rows of a head
+// that the items have and those of them that the output has (0: all).
 struct PartialOut {
   __bf16* out;
   float scale;
   int64_t offset;
+  int head_rows = 0, out_rows = 0;
 };
 // order: null, or the item of every grid index.
 hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order,

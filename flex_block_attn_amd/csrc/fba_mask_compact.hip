@@ -61,9 +61,15 @@ hipError_t launch_mask_compact(const uint8_t* mask, int64_t mask_bh, int nQ, int
 //       groups of query tile T; bit g is mask[m, (128 T + 16 g) / q_block, J].                       (forward, dQ)
 //   kt_ent[m, U, 0..kt_cnt) = (s << 8) | bits, ascending s: 32-row query slab s touches key tile U; bit 2w + f is
 //       mask[m, (32 s + 16 f) / q_block, (128 U + 32 w) / k_block], w = wave (32 keys), f = half of the slab.  (dK/dV)
-// One wave per output row, same ballot / prefix-popcount compaction as above; unused entries are -1.
+// One wave per output row, same ballot / prefix-popcount compaction as above; unused entries are -1.  The mask itself may have fewer rows
+// and columns (mask_q, mask_k): lengths that are no whole tiles, where blocks that nothing selects fill the last tile up.
+//
+// What bounds it are the key side's loads: bytes of a column, each in a line of its own.  A tile meets two columns at most (k_block is a multiple
+// of 64), a slab one mask row unless its halves have different ones, so one or two rows of two bytes are read and not all eight of the bits' places, and the
+// loads of four steps go out side by side: 24 masks of 480 x 480, 64-token blocks 71 -> 38 us.
+constexpr int kSideBySide = 4;
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void tile_lists_kernel(
-    const uint8_t* __restrict__ mask, int64_t mask_bh, int nQ, int nK, int q_block, int k_block, int n_qt, int n_kt,
+    const uint8_t* __restrict__ mask, int64_t mask_bh, int mask_q, int mask_k, int nK, int q_block, int k_block, int n_qt, int n_kt,
     int n_qs, int32_t* __restrict__ qt_cnt, int32_t* __restrict__ qt_ent, int32_t* __restrict__ kt_cnt,
     int32_t* __restrict__ kt_ent) {
   const int lane = threadIdx.x & 63;
@@ -75,43 +81,55 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void tile_list
   const int per = q_pass ? n_qt : n_kt;
   const int64_t m = r / per;
   const int tile = (int)(r - m * per);
-  const uint8_t* base = mask + m * (int64_t)nQ * nK;
+  const uint8_t* base = mask + m * (int64_t)mask_q * mask_k;
+  auto selects = [&](int i, int j) -> int {  // (no branch around the load)
+    const bool in = i < mask_q && j < mask_k;
+    return base[in ? (int64_t)i * mask_k + j : 0] != 0 && in ? 1 : 0;
+  };
+  const bool halves = q_block % 32 != 0;                                             // a slab's two have mask rows of their own
+  const int col0 = 128 * tile / k_block, col1 = (128 * tile + 64) / k_block;  // of the tile's halves
   const int len = q_pass ? nK : n_qs;
   int32_t* out = (q_pass ? qt_ent : kt_ent) + r * (int64_t)len;
 
   int cnt = 0;
-  for (int t0 = 0; t0 < len; t0 += 64) {
-    const int t = t0 + lane;
-    int bits = 0;
-    if (t < len) {
-      if (q_pass) {
+  for (int t0 = 0; t0 < len; t0 += 64 * kSideBySide) {
+    int bits[kSideBySide];
 #pragma unroll
-        for (int g = 0; g < 8; ++g) bits |= (base[(int64_t)((128 * tile + 16 * g) / q_block) * nK + t] != 0) << g;
-      } else {
+    for (int c = 0; c < kSideBySide; ++c) {
+      const int t = t0 + 64 * c + lane;
+      bits[c] = 0;
+      if (t < len) {
+        if (q_pass) {
 #pragma unroll
-        for (int wv = 0; wv < 4; ++wv)
-#pragma unroll
-          for (int f = 0; f < 2; ++f)
-            bits |= (base[(int64_t)((32 * t + 16 * f) / q_block) * nK + (128 * tile + 32 * wv) / k_block] != 0) << (2 * wv + f);
+          for (int g = 0; g < 8; ++g) bits[c] |= selects((128 * tile + 16 * g) / q_block, t) << g;
+        } else {
+          const int i0 = 32 * t / q_block, i1 = halves ? (32 * t + 16) / q_block : i0;
+          bits[c] = 0x05 * selects(i0, col0) | 0x50 * selects(i0, col1);
+          if (halves) bits[c] |= 0x0a * selects(i1, col0) | 0xa0 * selects(i1, col1);
+          else bits[c] |= bits[c] << 1;
+        }
       }
     }
-    const bool on = bits != 0;
-    const unsigned long long bal = __ballot(on);
-    if (on) out[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = (t << 8) | bits;
-    cnt += __popcll(bal);
+#pragma unroll
+    for (int c = 0; c < kSideBySide; ++c) {
+      const bool on = bits[c] != 0;
+      const unsigned long long bal = __ballot(on);
+      if (on) out[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = ((t0 + 64 * c + lane) << 8) | bits[c];
+      cnt += __popcll(bal);
+    }
   }
   for (int t = cnt + lane; t < len; t += 64) out[t] = -1;
   if (lane == 0) (q_pass ? qt_cnt : kt_cnt)[r] = cnt;
 }
 
-hipError_t launch_tile_lists(const uint8_t* mask, int64_t mask_bh, int nQ, int nK, int q_block, int k_block, int n_qt,
+hipError_t launch_tile_lists(const uint8_t* mask, int64_t mask_bh, int mask_q, int mask_k, int nK, int q_block, int k_block, int n_qt,
                              int n_kt, int n_qs, int32_t* qt_cnt, int32_t* qt_ent, int32_t* kt_cnt, int32_t* kt_ent,
                              hipStream_t stream) {
   const int64_t waves = mask_bh * ((int64_t)n_qt + n_kt);
   const int64_t blocks = (waves + 3) / 4;
   if (blocks <= 0) return hipSuccess;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(tile_lists_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, mask, mask_bh, nQ, nK, q_block, k_block,
+  hipLaunchKernelGGL(tile_lists_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, mask, mask_bh, mask_q, mask_k, nK, q_block, k_block,
                      n_qt, n_kt, n_qs, qt_cnt, qt_ent, kt_cnt, kt_ent);
   return hipGetLastError();
 }

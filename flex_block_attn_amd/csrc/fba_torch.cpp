@@ -39,8 +39,8 @@ constexpr int64_t kXcds = 8;
 // the C ABI, bound at run time
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                \
-  X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists) X(fba_pair_slots_bounds) X(fba_tile_slots_bounds)        \
-  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_tiled) X(fba_bwd_handover) X(fba_bwd_tiled_handover) X(fba_bwd_dense) \
+  X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists_cut) X(fba_pair_slots_bounds) X(fba_tile_slots_bounds)        \
+  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_handover) X(fba_bwd_tiled_cut) X(fba_bwd_dense) \
   X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
@@ -231,11 +231,14 @@ std::vector<at::Tensor> run_backward_on_mask(const Problem& p, const at::Tensor&
 
 enum class HandOver { kNever, kAuto, kWhole };  // dQ recomputes; as the limits allow; all heads at once whatever the size
 
-// bounds: pair numbers at the head boundaries of the mask (mask_bh + 1 of them); empty: pairs not numbered.
+// bounds: pair numbers at the head boundaries of the mask (mask_bh + 1 of them); empty: pairs not numbered.  out_q, out_kv: rows of a head of dq
+// and of dk, dv (0: as many as q and k have; fewer on tile lists only).
 std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o,
                                      const at::Tensor& lse, const at::Tensor& d_o, const Lists& l, const std::vector<int64_t>& bounds, HandOver mode,
-                                     bool dense, int64_t limit, int64_t split_bytes) {
-  at::Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+                                     bool dense, int64_t limit, int64_t split_bytes, int64_t out_q = 0, int64_t out_kv = 0) {
+  if (out_q == 0) out_q = p.Sq;
+  if (out_kv == 0) out_kv = p.Skv;
+  at::Tensor dq = at::empty({p.B, p.Hq, out_q, kHeadDim}, q.options()), dk = at::empty({p.B, p.Hkv, out_kv, kHeadDim}, k.options()), dv = at::empty_like(dk);
   void* const stream = current_stream(q);
   const int64_t group = p.Hq / p.Hkv, units = p.B * p.Hkv;
   auto workspace = [&](int64_t bytes) {
@@ -267,15 +270,19 @@ std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, cons
   const auto f32 = q.options().dtype(at::kFloat);
   if (!ds.defined() || dense) {
     at::Tensor stats = at::empty({2, p.B, p.Hq, p.Sq}, f32);
-    if (ds.defined())
+    if (p.tiled())
+      check(lib.fba_bwd_tiled_cut(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(), stats.data_ptr<float>(),
+                                  ds.defined() ? ds.data_ptr() : nullptr, ds.defined() ? ds.numel() : 0, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), l.q_cnt,
+                                  l.q_idx, l.k_cnt, l.k_idx, nullptr, nullptr, nullptr, 0, p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, out_q, out_kv, kHeadDim,
+                                  p.q_block, p.k_block, split.ptr(), split.bytes, stream));
+    else if (ds.defined())
       check(lib.fba_bwd_dense(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(), stats.data_ptr<float>(),
                               ds.data_ptr(), ds.numel(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, p.mask_bh,
                               p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes, stream));
     else
-      check((p.tiled() ? lib.fba_bwd_tiled : lib.fba_bwd)(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(),
-                                                          stats.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), l.q_cnt, l.q_idx,
-                                                          l.k_cnt, l.k_idx, p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block,
-                                                          p.k_block, split.ptr(), split.bytes, stream));
+      check(lib.fba_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(), stats.data_ptr<float>(), dq.data_ptr(),
+                        dk.data_ptr(), dv.data_ptr(), l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block,
+                        p.k_block, split.ptr(), split.bytes, stream));
     return {dq, dk, dv};
   }
   // One launch sequence per chunk of kv heads [u0, u1): every pointer moves to the chunk's first head, the chunk is described
@@ -296,10 +303,10 @@ std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, cons
     const int32_t *k_cnt = l.k_cnt + m0 * l.k_rows, *k_idx = l.k_idx + m0 * l.k_rows * l.k_len;
     const int32_t *base = l.pair_base + m0 * l.k_rows, *q_slot = l.q_slot + m0 * l.q_rows * l.slot_len;
     if (p.tiled())
-      check(lib.fba_bwd_tiled_handover(bf16_at(q, qo), bf16_at(k, ko), bf16_at(v, ko), bf16_at(o, qo), bf16_at(d_o, qo), lse0, stats.data_ptr<float>(), ws,
-                                       pairs * p.pair_bytes(), bf16_at(dq, qo), bf16_at(dk, ko), bf16_at(dv, ko), q_cnt, q_idx, k_cnt, k_idx, base,
-                                       l.k_slot + m0 * l.k_rows * l.k_len, q_slot, pairs, mask_bh, 1, nh, nu, p.Sq, p.Skv, kHeadDim, p.q_block,
-                                       p.k_block, split.ptr(), split.bytes, stream));
+      check(lib.fba_bwd_tiled_cut(bf16_at(q, qo), bf16_at(k, ko), bf16_at(v, ko), bf16_at(o, qo), bf16_at(d_o, qo), lse0, stats.data_ptr<float>(), ws,
+                                  pairs * p.pair_bytes(), bf16_at(dq, h0 * out_q * kHeadDim), bf16_at(dk, u0 * out_kv * kHeadDim),
+                                  bf16_at(dv, u0 * out_kv * kHeadDim), q_cnt, q_idx, k_cnt, k_idx, base, l.k_slot + m0 * l.k_rows * l.k_len, q_slot, pairs,
+                                  mask_bh, 1, nh, nu, p.Sq, p.Skv, out_q, out_kv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes, stream));
     else
       check(lib.fba_bwd_handover(bf16_at(q, qo), bf16_at(k, ko), bf16_at(v, ko), bf16_at(o, qo), bf16_at(d_o, qo), lse0, stats.data_ptr<float>(), ws,
                                  pairs * p.pair_bytes(), bf16_at(dq, qo), bf16_at(dk, ko), bf16_at(dv, ko), q_cnt, q_idx, k_cnt, k_idx, base, q_slot,
@@ -327,7 +334,8 @@ struct Saved : torch::CustomClassHolder {
   explicit Saved(const Problem& problem) : p(problem), lists(problem) {}
 };
 
-// The lists of `mask` in one buffer; key-major half and (numbered) pair numbers only where backward will read them.
+// The lists of `mask` in one buffer; key-major half and (numbered) pair numbers only where backward will read them.  The mask is the
+// caller's: blocks that fill up the last tiles are in the lists' extents only.
 void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered) {
   const Problem& p = s.p;
   Lists& l = s.lists;
@@ -358,7 +366,8 @@ void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered)
     l.k_cnt = b + k_cnt;
     l.k_idx = b + k_idx;
   }
-  check(lib.fba_lists(static_cast<const uint8_t*>(mask.data_ptr()), M, p.nQ(), p.nK(), p.q_block, p.k_block, l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, stream));
+  check(lib.fba_lists_cut(static_cast<const uint8_t*>(mask.data_ptr()), M, p.nQ(), p.nK(), s.q_len / p.q_block, s.kv_len / p.k_block, p.q_block, p.k_block,
+                          l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, stream));
   if (!numbered) return;
   l.pair_base = b + base;
   l.q_slot = b + q_slot;
@@ -399,7 +408,8 @@ std::vector<at::Tensor> resized(const std::vector<std::pair<at::Tensor, int64_t>
   return out;
 }
 
-// Inputs of a call as the kernels take them.  No block selects the rows that are appended.
+// Inputs of a call as the kernels take them.  No block selects the rows that are appended.  The mask is for a forward pass that reads
+// it itself; lists are made of the caller's, which saves a launch of 5 us (the fill of the last tiles) at B2 H8/2 S3136.
 struct Inputs {
   at::Tensor q, k, v, mask;
   Inputs(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_, const at::Tensor& mask_, const Saved& s) : q(q_), k(k_), v(v_), mask(mask_) {
@@ -409,6 +419,7 @@ struct Inputs {
     q = r[0];
     k = r[1];
     v = r[2];
+    if (!takes_mask(p)) return;
     mask = at::empty({p.mask_bh, p.nQ(), p.nK()}, mask_.options());
     check(lib.fba_resize_mask(static_cast<const uint8_t*>(mask_.data_ptr()), static_cast<uint8_t*>(mask.data_ptr()), p.mask_bh, s.q_len / p.q_block,
                               s.kv_len / p.k_block, p.nQ(), p.nK(), current_stream(q)));
@@ -439,7 +450,7 @@ struct Attention : torch::autograd::Function<Attention> {
       return cut ? o.narrow(2, 0, q_len).detach() : o;
     }
     const Inputs in(q, k, v, mask, *s);
-    build_lists(*s, in.mask, /*backward=*/true, /*numbered=*/!s->dense);
+    build_lists(*s, mask, /*backward=*/true, /*numbered=*/!s->dense);
     auto [o, lse] = takes_mask(s->p) ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask) : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
     ctx->save_for_backward({in.q, in.k, in.v, o, lse});
     // The rows that were appended are cut off here and not behind this function, where autograd would give back gradients for them in
@@ -477,8 +488,7 @@ struct Attention : torch::autograd::Function<Attention> {
       const int32_t* h = s.host_bounds.data_ptr<int32_t>();
       bounds.assign(h, h + p.mask_bh + 1);
     }
-    auto g = run_backward(p, q, k, v, o, lse, d_o, s.lists, bounds, HandOver::kAuto, s.dense, s.limit, s.split_bytes);
-    if (s.padded()) g = resized({{g[0], s.q_len}, {g[1], s.kv_len}, {g[2], s.kv_len}});
+    const auto g = run_backward(p, q, k, v, o, lse, d_o, s.lists, bounds, HandOver::kAuto, s.dense, s.limit, s.split_bytes, s.q_len, s.kv_len);
     return {g[0], g[1], g[2], at::Tensor(), at::Tensor()};
   }
 };
@@ -523,7 +533,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   if (!backward) {
     if (takes_mask(p)) return run_forward_on_mask(p, q, k, v, mask).first;
     const Inputs in(q, k, v, mask, *s);
-    build_lists(*s, in.mask, false, false);
+    build_lists(*s, mask, false, false);
     const at::Tensor o = run_forward(p, in.q, in.k, in.v, s->lists, split_bytes).first;
     return s->padded() ? o.narrow(2, 0, q_len) : o;
   }

@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2007
+#define FBA_VERSION 2008
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -205,6 +205,9 @@ int32_t fba_bwd_dq_from_ds(const void* k, const void* ds_ws, int64_t ds_ws_bytes
  */
 int32_t fba_lists(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t q_block, int32_t k_block, int32_t* q_cnt,
                   int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream);
+/* The same of a mask [mask_bh, mask_q, mask_k] as if fba_resize_mask had made it [mask_bh, nQ, nK] (tile lists only). */
+int32_t fba_lists_cut(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32_t nK, int32_t mask_q, int32_t mask_k, int32_t q_block, int32_t k_block,
+                      int32_t* q_cnt, int32_t* q_idx, int32_t* k_cnt, int32_t* k_idx, void* hip_stream);
 
 /*
  * Sequences that are no whole number of 128-row tiles (possible with tile lists only) are worked on in padded copies.
@@ -287,6 +290,16 @@ int32_t fba_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mas
 /* See fba_pair_slots_bounds. */
 int32_t fba_tile_slots_bounds(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int32_t n_qt, int32_t n_kt, int32_t* pair_base,
                        int32_t* kt_slot, int32_t* slot_table, int32_t* bounds, void* hip_stream);
+/*
+ * Backward on tile lists whose gradients have fewer rows than the padded inputs (lengths that are no whole tiles): dq [B, Hq, out_q, 128], dk
+ * and dv [B, Hkv, out_kv, 128]; the rows beyond are not written.  ds_ws null: as fba_bwd_tiled; pair_base null: as fba_bwd_dense, with a place
+ * for every tile pair; otherwise as fba_bwd_tiled_handover.  Bit for bit their results.
+ */
+int32_t fba_bwd_tiled_cut(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats, void* ds_ws,
+                          int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt, const int32_t* qt_ent, const int32_t* kt_cnt,
+                          const int32_t* kt_ent, const int32_t* pair_base, const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh,
+                          int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t out_q, int32_t out_kv, int32_t head_dim, int32_t q_block,
+                          int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream);
 int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,
                                void* ds_ws, int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt,
                                const int32_t* qt_ent, const int32_t* kt_cnt, const int32_t* kt_ent, const int32_t* pair_base,
