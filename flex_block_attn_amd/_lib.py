@@ -52,7 +52,7 @@ SIGNATURES = {
     "fba_lists": (_c_i32, [_c_ptr, _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr]),
     "fba_resize_rows": (_c_i32, [_c_i32] + [_c_ptr] * 6),
     "fba_resize_mask": (_c_i32, [_c_ptr, _c_ptr, _c_i64] + [_c_i32] * 4 + [_c_ptr]),
-    "fba_bwd_tiled_cut": (_c_i32, [_c_ptr] * 8 + [_c_i64] + [_c_ptr] * 10 + [_c_i64] * 2 + [_c_i32] * 10 + [_c_ptr, _c_i64, _c_ptr]),
+    "fba_bwd_tiled_cut": (_c_i32, [_c_ptr] * 9 + [_c_i64] + [_c_ptr] * 10 + [_c_i64] * 2 + [_c_i32] * 10 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_bwd_dense": (_c_i32, [_c_ptr] * 8 + [_c_i64] + [_c_ptr] * 7 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_bwd_noalloc": (_c_i32, [_c_ptr] * 13 + [_c_i64] + [_c_i32] * 8 + [_c_ptr]),
     "fba_lists_cut": (_c_i32, [_c_ptr, _c_i64] + [_c_i32] * 6 + [_c_ptr] * 5),

@@ -609,7 +609,7 @@ int32_t fba_tile_slots(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mas
   return fba_tile_slots_bounds(kt_cnt, kt_ent, mask_bh, n_qt, n_kt, pair_base, kt_slot, slot_table, nullptr, hip_stream);
 }
 
-static int bwd_tiled_impl(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats, void* ds_ws,
+static int bwd_tiled_impl(const void* q, const void* k, const void* v, const void* o, const void* d_o, void* d_o_ws, const float* lse, float* stats, void* ds_ws,
                           int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt, const int32_t* qt_ent, const int32_t* kt_cnt,
                           const int32_t* kt_ent, const int32_t* pair_base, const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh,
                           int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t out_q, int32_t out_kv, int32_t head_dim, int32_t q_block,
@@ -620,6 +620,8 @@ static int bwd_tiled_impl(const void* q, const void* k, const void* v, const voi
   if (int rc = check_split_ws(split_ws, split_ws_bytes)) return rc;
   // everything is validated before the first launch, so that a rejected call leaves nothing on the stream
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}})) return rc;
+  if (d_o_ws != nullptr)
+    if (int rc = check_ptrs({{"d_o_ws", d_o_ws}})) return rc;
   if (numbered || ds_ws != nullptr)
     if (int rc = check_ptrs({{"ds_ws", ds_ws}})) return rc;
   if (!lse || !stats || !qt_cnt || !qt_ent || !kt_cnt || !kt_ent || (numbered && (!pair_base || !kt_slot || !slot_table))) return fail(FBA_ERR_INVALID, "null pointer argument");
@@ -635,10 +637,10 @@ static int bwd_tiled_impl(const void* q, const void* k, const void* v, const voi
   }
   fba::BwdParams p{};
   fill_bwd(p, s);
-  p.make = {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq};
+  p.make = {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq, (__bf16*)d_o_ws, Sq, out_q};
   p.tiled = 1;
   p.out_q = out_q; p.out_kv = out_kv;
-  p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
+  p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)(d_o_ws != nullptr ? d_o_ws : d_o);
   p.stats = stats; p.dq = (__bf16*)dq; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv;
   p.q_cnt = qt_cnt; p.q_idx = qt_ent; p.k_cnt = kt_cnt; p.k_idx = kt_ent;
   p.ds_ws = (__bf16*)ds_ws;
@@ -653,12 +655,12 @@ static int bwd_tiled_impl(const void* q, const void* k, const void* v, const voi
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (tile lists) launch");
 }
 
-int32_t fba_bwd_tiled_cut(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats, void* ds_ws,
+int32_t fba_bwd_tiled_cut(const void* q, const void* k, const void* v, const void* o, const void* d_o, void* d_o_ws, const float* lse, float* stats, void* ds_ws,
                           int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt, const int32_t* qt_ent, const int32_t* kt_cnt,
                           const int32_t* kt_ent, const int32_t* pair_base, const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh,
                           int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t out_q, int32_t out_kv, int32_t head_dim, int32_t q_block,
                           int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream) {
-  return bwd_tiled_impl(q, k, v, o, d_o, lse, stats, ds_ws, ds_ws_bytes, dq, dk, dv, qt_cnt, qt_ent, kt_cnt, kt_ent, pair_base, kt_slot, slot_table, n_pairs,
+  return bwd_tiled_impl(q, k, v, o, d_o, d_o_ws, lse, stats, ds_ws, ds_ws_bytes, dq, dk, dv, qt_cnt, qt_ent, kt_cnt, kt_ent, pair_base, kt_slot, slot_table, n_pairs,
                         mask_bh, B, Hq, Hkv, Sq, Skv, out_q, out_kv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, ds_ws != nullptr && pair_base != nullptr);
 }
 
@@ -668,7 +670,7 @@ int32_t fba_bwd_tiled_handover(const void* q, const void* k, const void* v, cons
                                const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh, int32_t B,
                                int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block,
                                void* split_ws, int64_t split_ws_bytes, void* hip_stream) {
-  return bwd_tiled_impl(q, k, v, o, d_o, lse, stats, ds_ws, ds_ws_bytes, dq, dk, dv, qt_cnt, qt_ent, kt_cnt, kt_ent, pair_base, kt_slot, slot_table, n_pairs,
+  return bwd_tiled_impl(q, k, v, o, d_o, nullptr, lse, stats, ds_ws, ds_ws_bytes, dq, dk, dv, qt_cnt, qt_ent, kt_cnt, kt_ent, pair_base, kt_slot, slot_table, n_pairs,
                         mask_bh, B, Hq, Hkv, Sq, Skv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, true);
 }
 

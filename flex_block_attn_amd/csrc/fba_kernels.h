@@ -171,6 +171,9 @@ struct BwdStats {
   const float* lse;
   float* stats;  // [2, rows]
   int64_t rows;
+  // null, or where dO goes that has given_rows of the head_rows rows of a head, with rows of zeros for the rest
+  __bf16* filled = nullptr;
+  int head_rows = 0, given_rows = 0;
 };
 
 // A dK/dV launch whose lists differ so much that the longest of them would set its time: all items as pieces, long ones first.  Made on the

@@ -166,10 +166,13 @@ constexpr int kMostOrdered = 2048;  // items of a launch that is ordered at all:
 // Bound by memory: 524 bytes of a row, each once.  With a row to 16 lanes the blocks ended as soon as their two loads had come back, so that
 // starting them set the pace; launches that fill the GPU with four rows to 16 lanes request all eight loads first (262144 rows 30.1 -> 22.1 us,
 // 6.2 TB/s; 552960 rows 64.2 -> 55.7 us, 5.2 TB/s).
+//
+// kFill: dO has fewer rows to a head than O (lengths that are no whole tiles) and is copied on the way, with rows of zeros for what fills up the last
+// tile: a launch of 6.2 us less at B2 H8 S3136.
 constexpr int kStatsRows = 16, kStatsDeep = 4;
 constexpr int64_t kStatsMany = 131072;  // rows: eight blocks of 64 rows for each of 256 compute units
 __host__ __device__ inline bool stats_deep(const BwdStats& s) { return s.rows >= kStatsMany; }
-template <int kDeep>
+template <int kDeep, bool kFill>
 FBA_DEVICE void stats_rows_of(const BwdStats& s, int block, int blocks) {
   const int sub = threadIdx.x & 15;
   for (int64_t r0 = (int64_t)block * (kStatsRows * kDeep) + (threadIdx.x >> 4); r0 < s.rows; r0 += (int64_t)blocks * (kStatsRows * kDeep)) {
@@ -179,12 +182,22 @@ FBA_DEVICE void stats_rows_of(const BwdStats& s, int block, int blocks) {
     for (int d = 0; d < kDeep; ++d) {
       const int64_t r = r0 + d * kStatsRows < s.rows ? r0 + d * kStatsRows : r0;
       a[d] = *reinterpret_cast<const bf16x8*>(s.o + r * kHeadDim + sub * 8);
-      b[d] = *reinterpret_cast<const bf16x8*>(s.d_o + r * kHeadDim + sub * 8);
       lse[d] = s.lse[r];
+      if constexpr (kFill) {
+        const uint32_t head = (uint32_t)r / (uint32_t)s.head_rows;
+        const int at = (int)((uint32_t)r - head * (uint32_t)s.head_rows);
+        bf16x8 x = {};
+        if (at < s.given_rows) x = *reinterpret_cast<const bf16x8*>(s.d_o + ((int64_t)head * s.given_rows + at) * kHeadDim + sub * 8);
+        b[d] = x;
+      } else {
+        b[d] = *reinterpret_cast<const bf16x8*>(s.d_o + r * kHeadDim + sub * 8);
+      }
     }
 #pragma unroll
     for (int d = 0; d < kDeep; ++d) {
       const int64_t r = r0 + d * kStatsRows;
+      if constexpr (kFill)
+        if (r < s.rows) *reinterpret_cast<bf16x8*>(s.filled + r * kHeadDim + sub * 8) = b[d];
       float acc = 0.f;
 #pragma unroll
       for (int t = 0; t < 8; ++t) acc += (float)a[d][t] * (float)b[d][t];
@@ -200,8 +213,13 @@ FBA_DEVICE void stats_rows_of(const BwdStats& s, int block, int blocks) {
   }
 }
 FBA_DEVICE void stats_rows(const BwdStats& s, int block, int blocks) {
-  if (stats_deep(s)) stats_rows_of<kStatsDeep>(s, block, blocks);
-  else stats_rows_of<1>(s, block, blocks);
+  if (s.filled != nullptr) {
+    if (stats_deep(s)) stats_rows_of<kStatsDeep, true>(s, block, blocks);
+    else stats_rows_of<1, true>(s, block, blocks);
+  } else {
+    if (stats_deep(s)) stats_rows_of<kStatsDeep, false>(s, block, blocks);
+    else stats_rows_of<1, false>(s, block, blocks);
+  }
 }
 int stats_blocks(const BwdStats& s) {
   const int rows = kStatsRows * (stats_deep(s) ? kStatsDeep : 1);

@@ -232,13 +232,14 @@ std::vector<at::Tensor> run_backward_on_mask(const Problem& p, const at::Tensor&
 enum class HandOver { kNever, kAuto, kWhole };  // dQ recomputes; as the limits allow; all heads at once whatever the size
 
 // bounds: pair numbers at the head boundaries of the mask (mask_bh + 1 of them); empty: pairs not numbered.  out_q, out_kv: rows of a head of dq
-// and of dk, dv (0: as many as q and k have; fewer on tile lists only).
+// and of dk, dv (0: as many as q and k have; fewer on tile lists only); d_o has out_q as well.
 std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& o,
                                      const at::Tensor& lse, const at::Tensor& d_o, const Lists& l, const std::vector<int64_t>& bounds, HandOver mode,
                                      bool dense, int64_t limit, int64_t split_bytes, int64_t out_q = 0, int64_t out_kv = 0) {
   if (out_q == 0) out_q = p.Sq;
   if (out_kv == 0) out_kv = p.Skv;
   at::Tensor dq = at::empty({p.B, p.Hq, out_q, kHeadDim}, q.options()), dk = at::empty({p.B, p.Hkv, out_kv, kHeadDim}, k.options()), dv = at::empty_like(dk);
+  const at::Tensor d_o_ws = out_q != p.Sq ? at::empty_like(q) : at::Tensor();  // (dO filled up to whole tiles)
   void* const stream = current_stream(q);
   const int64_t group = p.Hq / p.Hkv, units = p.B * p.Hkv;
   auto workspace = [&](int64_t bytes) {
@@ -271,7 +272,8 @@ std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, cons
   if (!ds.defined() || dense) {
     at::Tensor stats = at::empty({2, p.B, p.Hq, p.Sq}, f32);
     if (p.tiled())
-      check(lib.fba_bwd_tiled_cut(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), lse.data_ptr<float>(), stats.data_ptr<float>(),
+      check(lib.fba_bwd_tiled_cut(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(), d_o_ws.defined() ? d_o_ws.data_ptr() : nullptr,
+                                  lse.data_ptr<float>(), stats.data_ptr<float>(),
                                   ds.defined() ? ds.data_ptr() : nullptr, ds.defined() ? ds.numel() : 0, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), l.q_cnt,
                                   l.q_idx, l.k_cnt, l.k_idx, nullptr, nullptr, nullptr, 0, p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, out_q, out_kv, kHeadDim,
                                   p.q_block, p.k_block, split.ptr(), split.bytes, stream));
@@ -303,7 +305,8 @@ std::vector<at::Tensor> run_backward(const Problem& p, const at::Tensor& q, cons
     const int32_t *k_cnt = l.k_cnt + m0 * l.k_rows, *k_idx = l.k_idx + m0 * l.k_rows * l.k_len;
     const int32_t *base = l.pair_base + m0 * l.k_rows, *q_slot = l.q_slot + m0 * l.q_rows * l.slot_len;
     if (p.tiled())
-      check(lib.fba_bwd_tiled_cut(bf16_at(q, qo), bf16_at(k, ko), bf16_at(v, ko), bf16_at(o, qo), bf16_at(d_o, qo), lse0, stats.data_ptr<float>(), ws,
+      check(lib.fba_bwd_tiled_cut(bf16_at(q, qo), bf16_at(k, ko), bf16_at(v, ko), bf16_at(o, qo), bf16_at(d_o, h0 * out_q * kHeadDim),
+                                  d_o_ws.defined() ? bf16_at(d_o_ws, qo) : nullptr, lse0, stats.data_ptr<float>(), ws,
                                   pairs * p.pair_bytes(), bf16_at(dq, h0 * out_q * kHeadDim), bf16_at(dk, u0 * out_kv * kHeadDim),
                                   bf16_at(dv, u0 * out_kv * kHeadDim), q_cnt, q_idx, k_cnt, k_idx, base, l.k_slot + m0 * l.k_rows * l.k_len, q_slot, pairs,
                                   mask_bh, 1, nh, nu, p.Sq, p.Skv, out_q, out_kv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes, stream));
@@ -478,10 +481,7 @@ struct Attention : torch::autograd::Function<Attention> {
       const auto g = run_backward_on_mask(p, q, k, v, o, lse, d_o, s.list_buffer);
       return {g[0], g[1], g[2], at::Tensor(), at::Tensor()};
     }
-    if (s.q_len != p.Sq) {
-      if ((reinterpret_cast<uintptr_t>(d_o.data_ptr()) & 15) != 0) d_o = d_o.clone();  // the copy moves 16 bytes at a time
-      d_o = resized({{d_o, p.Sq}})[0];
-    }
+    if (s.q_len != p.Sq && (reinterpret_cast<uintptr_t>(d_o.data_ptr()) & 15) != 0) d_o = d_o.clone();  // it is filled up 16 bytes at a time
     std::vector<int64_t> bounds;
     if (!s.dense) {
       s.copied.synchronize();

@@ -293,9 +293,10 @@ int32_t fba_tile_slots_bounds(const int32_t* kt_cnt, const int32_t* kt_ent, int6
 /*
  * Backward on tile lists whose gradients have fewer rows than the padded inputs (lengths that are no whole tiles): dq [B, Hq, out_q, 128], dk
  * and dv [B, Hkv, out_kv, 128]; the rows beyond are not written.  ds_ws null: as fba_bwd_tiled; pair_base null: as fba_bwd_dense, with a place
- * for every tile pair; otherwise as fba_bwd_tiled_handover.  Bit for bit their results.
+ * for every tile pair; otherwise as fba_bwd_tiled_handover.  d_o_ws null: d_o has Sq rows to a head; otherwise it has out_q and is filled up there
+ * (B * Hq * Sq rows, 16-byte aligned).  Bit for bit their results.
  */
-int32_t fba_bwd_tiled_cut(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats, void* ds_ws,
+int32_t fba_bwd_tiled_cut(const void* q, const void* k, const void* v, const void* o, const void* d_o, void* d_o_ws, const float* lse, float* stats, void* ds_ws,
                           int64_t ds_ws_bytes, void* dq, void* dk, void* dv, const int32_t* qt_cnt, const int32_t* qt_ent, const int32_t* kt_cnt,
                           const int32_t* kt_ent, const int32_t* pair_base, const int32_t* kt_slot, const int32_t* slot_table, int64_t n_pairs, int64_t mask_bh,
                           int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t out_q, int32_t out_kv, int32_t head_dim, int32_t q_block,

@@ -1,6 +1,6 @@
 """Lists of masks around the edges of a scan's step (both flavours; tile lists take four steps of 64 entries at a time), and tile lists of a
 mask that ends inside the last tile (fba_lists_cut) against those of the mask filled up with unselected blocks.  Exact.  Gradients that leave
-out the rows of the fill (fba_bwd_tiled_cut): the bits of the calls that write them."""
+out the rows of the fill (fba_bwd_tiled_cut), from dO with and without them: the bits of the calls that write them."""
 import ctypes
 
 import pytest
@@ -73,7 +73,8 @@ def test_lists_of_a_mask_that_ends_inside_a_tile(gpu, rows, cols, nQ, nK, qbs, k
     (1, 3, 1, 7, 3, 8, 4, 64, 192),         # key blocks that straddle tiles
     (1, 2, 1, 6, 4, 6, 4, 64, 64),          # nothing left out
 ])
-def test_gradients_without_the_fill(gpu, B, Hq, Hkv, rows, cols, nQ, nK, qbs, kbs):
+@pytest.mark.parametrize("fill", [True, False])
+def test_gradients_without_the_fill(gpu, fill, B, Hq, Hkv, rows, cols, nQ, nK, qbs, kbs):
     from flex_block_attn_amd import _lib
 
     g = torch.Generator().manual_seed(rows * cols + qbs)
@@ -115,8 +116,10 @@ def test_gradients_without_the_fill(gpu, B, Hq, Hkv, rows, cols, nQ, nK, qbs, kb
         else:
             _lib.call("fba_bwd_tiled_handover", *ins, _ptr(ds), ds.numel(), *map(_ptr, want), *l4, *map(_ptr, (base, slot, table)), pairs, *tail)
         numbers = (base, slot, table) if kind == "numbered" else (None,) * 3
-        _lib.call("fba_bwd_tiled_cut", *ins, _ptr(None if kind == "recompute" else ds), ds.numel(), *map(_ptr, got), *l4, *map(_ptr, numbers),
+        given, filled = do[:, :, :out_q].contiguous(), torch.full_like(do, 7)
+        _lib.call("fba_bwd_tiled_cut", *ins[:4], *map(_ptr, (given, filled) if fill else (do, None)), *ins[5:], _ptr(None if kind == "recompute" else ds), ds.numel(), *map(_ptr, got), *l4, *map(_ptr, numbers),
                   pairs if kind == "numbered" else 0, M, *shape, out_q, out_kv, 128, qbs, kbs, *ws)
         for a, b in zip(got, want):
             assert torch.equal(a, b[:, :, : a.shape[2]]), kind
             assert bool((b[:, :, a.shape[2] :] == 0).all()), kind
+        assert torch.equal(filled, do if fill else torch.full_like(do, 7)), kind
