@@ -350,15 +350,25 @@ constexpr float kNoReference = -1e30f;
 struct HalfList {
   const int32_t* list;
   int cnt, half_mask, lane;
+  int head[4];               // this lane's entries among the first 256
   int base;                  // position of `entries` in the list
   int entries, ahead;        // this lane's entry among the 64 at `base` and the 64 behind them
   unsigned long long left;   // lanes whose entry names the half and has not been taken
 
   FBA_DEVICE int load(int at) const { return at + lane < cnt ? list[at + lane] : 0; }
   FBA_DEVICE unsigned long long named(int e) const { return __builtin_amdgcn_ballot_w64((e & half_mask) != 0); }
+  // The head of the list, asked for before the count has come back (two round trips less in front of the first copy), and the count.
+  FBA_DEVICE void read_head(int row_len, const int32_t* count) {
+    const int at_count = const_idx(count)[0];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) head[i] = 64 * i + lane < row_len ? list[64 * i + lane] : 0;
+    cnt = at_count;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) head[i] = 64 * i + lane < cnt ? head[i] : 0;
+  }
   FBA_DEVICE int total() const {
-    int n = 0;
-    for (int at = 0; at < cnt; at += 256) {  // four loads in flight
+    int n = __popcll(named(head[0])) + __popcll(named(head[1])) + __popcll(named(head[2])) + __popcll(named(head[3]));
+    for (int at = 256; at < cnt; at += 256) {  // four loads in flight
       const int e0 = load(at), e1 = load(at + 64), e2 = load(at + 128), e3 = load(at + 192);
       n += __popcll(named(e0)) + __popcll(named(e1)) + __popcll(named(e2)) + __popcll(named(e3));
     }
@@ -367,8 +377,8 @@ struct HalfList {
   // next() gives entry number `skip` of those that name the half
   FBA_DEVICE void start(int skip) {
     base = 0;
-    entries = load(0);
-    ahead = load(64);
+    entries = head[0];
+    ahead = head[1];
     left = named(entries);
     while (__popcll(left) <= skip && base + 64 < cnt) {
       skip -= __popcll(left);
@@ -420,9 +430,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (p.Sq / 128) + (qt >> 1);
   HalfList cursor;
   cursor.list = p.q_idx + mrow * p.nK;
-  cursor.cnt = const_idx(p.q_cnt)[mrow];
   cursor.half_mask = 15 << (4 * half);
   cursor.lane = lane;
+  cursor.read_head(p.nK, p.q_cnt + mrow);
 
   FwdState st;
 #pragma unroll
@@ -591,28 +601,42 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         for (int e = 0; e < 4; ++e) out[mb][g][e] = w_own * a[4 * g + e] + w_other * o[e];
       }
   }
-  if (parts > 1) {  // as in fwd_kernel
+  // Results go through the LDS this wave has just read, 32 rows of 64 columns, so that a store fills whole lines: a lane holds pieces of one
+  // row, 8 bytes to each of 32 rows per store.  (With this and the head of the list read ahead: H24 S30720, 64-token blocks, 192 of 480 kept
+  // 4.85 -> 4.70 ms; B2 H8/2 S3136, 16 x 64 blocks, 12 of 49 kept 82.0 -> 79.5 us.)
+  char* const own = smem + other * kSlabBytes;
+  if (parts > 1) {  // as in fwd_kernel; rows of 256 bytes, 16-byte chunk c of row r at slot c ^ r % 16
     float* slot = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (kHalfSlotBytes / 4);
-    float* prow = slot + (rg * 32 + l32) * kHeadDim;
+    float* prow = slot + rg * 32 * kHeadDim + 32 * keep;
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(prow + 32 * (keep + mb) + 8 * g + 4 * h) = out[mb][g];
+      for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(own + l32 * 256 + (((8 * mb + 2 * g + h) ^ (l32 & 15)) << 4)) = out[mb][g];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = 4 * i + (lane >> 4);
+      *reinterpret_cast<f32x4*>(prow + row * kHeadDim + 4 * (lane & 15)) = *reinterpret_cast<const f32x4*>(own + row * 256 + (((lane ^ row) & 15) << 4));
+    }
     if (h == 0 && par == 0) {
       slot[kHalfRows * kHeadDim + rg * 32 + l32] = m * st.c;
       slot[kHalfRows * kHeadDim + kHalfRows + rg * 32 + l32] = l;
     }
     return;
   }
-  __bf16* orow = p.o + (qrow0 + l32) * kHeadDim;
   const float inv = l > 0.f ? 1.f / l : 0.f;
   if (h == 0 && par == 0) p.lse[qrow0 + l32] = l > 0.f ? (m * st.c + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
+  __bf16* orow = p.o + qrow0 * kHeadDim + 32 * keep;
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<bf16x4*>(orow + 32 * (keep + mb) + 8 * g + 4 * h) =
+    for (int g = 0; g < 4; ++g)  // rows of 128 bytes, 16-byte chunk c of row r at slot c ^ r % 8
+      *reinterpret_cast<bf16x4*>(own + l32 * 128 + (((4 * mb + g) ^ (l32 & 7)) << 4) + 8 * h) =
           pack4(out[mb][g][0] * inv, out[mb][g][1] * inv, out[mb][g][2] * inv, out[mb][g][3] * inv);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    *reinterpret_cast<bf16x8*>(orow + row * kHeadDim + 8 * (lane & 7)) = *reinterpret_cast<const bf16x8*>(own + row * 128 + (((lane ^ row) & 7) << 4));
+  }
 }
 
 // Forward straight from the block mask, for problems too small to fill the GPU: no lists, no parts, one launch.
