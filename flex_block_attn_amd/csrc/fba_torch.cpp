@@ -329,6 +329,7 @@ struct Saved : torch::CustomClassHolder {
   at::Tensor list_buffer, host_bounds;
   bool from_mask = false;  // there are no lists: list_buffer holds a copy of the mask
   int64_t o_rows = 0;      // and o has as many rows to a head as if there were
+  bool ragged_q = false, ragged_kv = false;  // lengths that lists would have been padded for
   c10::Event copied{c10::DeviceType::CUDA};
   bool dense = false;
   int64_t limit = 0, split_bytes;
@@ -391,16 +392,17 @@ void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered)
 }
 
 // Sequences that are no whole number of 128-row tiles: copies cut or padded with zeros to `len` rows, all in one launch.  A
-// tensor that has the length already is returned as it is.
-std::vector<at::Tensor> resized(const std::vector<std::pair<at::Tensor, int64_t>>& tensors) {
+// tensor that has the length already is returned as it is unless `always`.
+std::vector<at::Tensor> resized(const std::vector<std::pair<at::Tensor, int64_t>>& tensors, bool always = false) {
   std::vector<at::Tensor> out;
   const void* src[3];
   void* dst[3];
   int64_t n_seq[3];
   int32_t src_len[3], dst_len[3], n = 0;
   for (const auto& [t, len] : tensors) {
-    out.push_back(t.size(2) == len ? t : at::empty({t.size(0), t.size(1), len, kHeadDim}, t.options()));
-    if (t.size(2) == len) continue;
+    const bool as_is = t.size(2) == len && !always;
+    out.push_back(as_is ? t : at::empty({t.size(0), t.size(1), len, kHeadDim}, t.options()));
+    if (as_is) continue;
     src[n] = t.data_ptr();
     dst[n] = out.back().data_ptr();
     n_seq[n] = t.size(0) * t.size(1);
@@ -448,7 +450,14 @@ struct Attention : torch::autograd::Function<Attention> {
       const int64_t q_len = s->q_len;
       auto [o, lse] = run_forward_on_mask(s->p, q, k, v, mask, s->list_buffer.data_ptr(), s->o_rows);
       const bool cut = s->o_rows != q_len;
-      ctx->save_for_backward({q, k, v, o, lse});
+      // As with lists, inputs of lengths that are no whole tiles may be written to before backward comes: copies are saved (2.4 us of a
+      // replayed step of 77, B2 H2 S1984).
+      std::vector<std::pair<at::Tensor, int64_t>> copies;
+      if (s->ragged_q) copies.emplace_back(q, q_len);
+      if (s->ragged_kv) copies.insert(copies.end(), {{k, s->kv_len}, {v, s->kv_len}});
+      const std::vector<at::Tensor> own = resized(copies, /*always=*/true);
+      const at::Tensor* const own_kv = own.data() + (s->ragged_q ? 1 : 0);
+      ctx->save_for_backward({s->ragged_q ? own[0] : q, s->ragged_kv ? own_kv[0] : k, s->ragged_kv ? own_kv[1] : v, o, lse});
       ctx->saved_data["s"] = c10::IValue::make_capsule(std::move(s));
       return cut ? o.narrow(2, 0, q_len).detach() : o;
     }
@@ -540,6 +549,8 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   if (backward_takes_mask(p)) {
     s->from_mask = true;
     s->o_rows = p.Sq;
+    s->ragged_q = p.Sq != q_len;
+    s->ragged_kv = p.Skv != kv_len;
     s->p.Sq = q_len;
     s->p.Skv = kv_len;
   } else {

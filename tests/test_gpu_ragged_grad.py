@@ -32,3 +32,29 @@ def test_layouts_of_the_gradient(gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs):
     other = torch.ones((), device=gpu, requires_grad=True)
     o = fba.flex_block_attn_func(q, k, v, qbs, kbs, m)
     assert torch.autograd.grad(other * 2, (q,), allow_unused=True)[0] is None and o.shape == q.shape
+
+
+@pytest.mark.parametrize("H,Sq,Skv", [
+    (2, 1984, 1984),   # backward from the mask
+    (1, 176, 320),
+    (8, 3136, 3136),   # lists
+])
+def test_inputs_written_to_before_backward(gpu, H, Sq, Skv):
+    """Lengths that are no whole tiles: backward reads copies of q, k, v, so they may be written to after the call."""
+    import flex_block_attn_amd as fba
+
+    g = torch.Generator().manual_seed(Sq + Skv)
+    q, do = (torch.randn((1, H, Sq, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    k, v = (torch.randn((1, H, Skv, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(2))
+    m = (torch.rand((Sq // 16, Skv // 64), generator=g) < 0.4).to(gpu)
+    grads = []
+    for write in (False, True):
+        x = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        o = fba.flex_block_attn_func(*x, 16, 64, m)
+        if write:
+            with torch.no_grad():
+                for t in x:
+                    t.fill_(3.0)
+        grads.append(torch.autograd.grad(o, x, do))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
