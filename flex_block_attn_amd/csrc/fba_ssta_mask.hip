@@ -63,9 +63,10 @@ constexpr int kChunk = 64;          // key blocks per LDS chunk: one per lane
 constexpr int kMostChunks = 64;     // nK <= 4096
 constexpr int kRowStride = kD + 4;  // floats; 16 lanes read 16 bytes of a row each from 64 different banks
 
-// A score as an unsigned number in the same order, -0 as +0; 0 for what is never picked (NaN, -inf, no key block).
+// A score as an unsigned number in the same order; 0 for what is never picked (NaN, -inf, no key block).  -0 becomes +0 as an integer:
+// -ffast-math knows no signed zeros and would drop an addition of +0.
 __device__ __forceinline__ uint32_t rank_key(float x) {
-  const uint32_t u = __float_as_uint(x + 0.f);
+  const uint32_t bits = __float_as_uint(x), u = bits == 0x80000000u ? 0u : bits;
   return x > -__builtin_inff() ? u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u) : 0u;
 }
 

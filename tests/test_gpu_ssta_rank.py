@@ -20,7 +20,7 @@ def test_top_blocks(gpu, B, Hq, Hkv, nQ, nK, topk, kind):
     if kind == "alike":
         k[:] = k[:, :, :1]
     if kind == "special":
-        k[:, :, ::3] = 0.0  # scores of 0, and with an odd number of signs of -0
+        k[:, :, ::3] = 0.0  # scores of 0
         k[:, :, 1::5, 0] = float("nan")
         k[:, :, 2::7, 0], q[..., 0] = float("-inf"), 1.0
         k[:, :, 4::11, 0] = float("inf")
@@ -30,3 +30,16 @@ def test_top_blocks(gpu, B, Hq, Hkv, nQ, nK, topk, kind):
     want = torch.zeros(score.shape, dtype=torch.bool).scatter_(-1, order[..., :topk], True) & (rank > float("-inf"))
     got = ssta_mask_from_means(q.to(gpu), k.to(gpu), 128, 128, topk=topk, band=-1, sink_blocks=0)
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("nK", [5, 300, 1100])
+def test_a_score_of_minus_zero_ties_with_zero(gpu, nK):
+    """A negative product that underflows, added last to sums that are +0, leaves -0: as large as the +0 further on, so the lower block is picked."""
+    from flex_block_attn_amd.video import ssta_mask_from_means
+
+    q, k = torch.zeros((1, 1, 1, 128)), torch.zeros((1, 1, nK, 128))
+    q[..., 0], q[..., 127] = 1.0, 1e-30
+    k[..., 0] = -1.0
+    k[0, 0, 1, 0], k[0, 0, 1, 127], k[0, 0, nK - 1, 0] = 0.0, -1e-30, 0.0
+    got = ssta_mask_from_means(q.to(gpu), k.to(gpu), 128, 128, topk=1, band=-1, sink_blocks=0)
+    assert got.flatten().nonzero().flatten().tolist() == [1]
