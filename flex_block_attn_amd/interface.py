@@ -265,8 +265,11 @@ def _forward(q, k, v, q_block_size, kv_block_size, block_mask, lists):
 
 
 def _backward_takes_mask(q, k, v, q_block_size, kv_block_size, block_mask):
-    """Whether neither pass needs lists (small problems, as the native call decides).  A mask that lists could not be made of is left to them."""
+    """Whether neither pass needs lists (small problems, as the native call decides).  What lists could not be made of is left to them, so that it is
+    refused with gradients as without: other masks, and lengths that are no whole tiles (flex_block_attn_func pads them)."""
     if block_mask.dtype != torch.bool or not block_mask.is_cuda or block_mask.device != q.device or block_mask.numel() == 0:
+        return False
+    if q.shape[2] % 128 or k.shape[2] % 128:
         return False
     _check_qkv(q, k, v)
     return q.numel() > 0 and k.numel() > 0 and _lib.host().backward_takes_mask(q, k, q_block_size, kv_block_size)

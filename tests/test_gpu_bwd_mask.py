@@ -120,3 +120,17 @@ def test_the_rule_stays_within_one_buffer_of_the_forward_rule():
     lib = _lib.load()
     assert lib.fba_bwd_takes_mask(1, 2, 2, 1536, 1536) and not lib.fba_bwd_takes_mask(1, 24, 24, 30720, 30720)
     assert not lib.fba_bwd_takes_mask(1, 2, 2, 4096, 4096) and not lib.fba_bwd_takes_mask(1, 16, 1, 512, 512)
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_the_autograd_function_wants_whole_tiles(gpu, grad):
+    """Lengths that are no whole tiles are padded in front of it: handed to it directly they are refused, with gradients or without."""
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd._lib import FbaError
+    from flex_block_attn_amd.interface import FlexBlockAttnFunc
+
+    q, k, v = (torch.randn((1, 1, n, 128), device=gpu).to(torch.bfloat16).requires_grad_(grad) for n in (48, 192, 192))
+    m = torch.ones((3, 3), dtype=torch.bool, device=gpu)
+    with pytest.raises(FbaError, match="multiples of 128"):
+        FlexBlockAttnFunc.apply(q, k, v, 16, 64, m, True)
+    assert fba.flex_block_attn_func(q, k, v, 16, 64, m).shape == q.shape
