@@ -2,6 +2,7 @@
 // blocks of the sequence, and to the top-k key blocks ranked by <mean of the query block's rows, mean of the key block's
 // rows>.  Three HBM-bound kernels: block means of Q and K, then scores + top-k + union into the bool block mask the
 // compaction kernel consumes, and the (un)permutation of a video latent grid into contiguous tiles.
+#include "fba_common.h"
 #include "fba_kernels.h"
 
 namespace fba {
@@ -73,14 +74,17 @@ __device__ __forceinline__ uint32_t rank_key(float x) {
 // mask[bh, i, j] = (j among the topk largest <q_mean[bh,i], k_mean[kv(bh),j]>, ties to the lower j)
 //                  || |j - (i*q_block)/k_block| <= band || j < sink || base[i, j]   (base: optional [nQ, nK] mask)
 //                  || j in the sliding window of i (window: optional, blocks as tiles of a 3-D grid, see TileWindow).
-// A wave ranks two query blocks; lane l holds the scores of key blocks l, l+64, ... (kMaxChunks of them) in registers.
+// A wave ranks two query blocks; lane l holds the scores of key blocks l, l+64, ... (kMaxChunks of them) in registers: 128 of them with 64 chunks, and
+// no more than 256 registers altogether, so that two waves share a SIMD.  (In scratch, where HIP's float4 kept the compiler from unrolling the
+// chunks, and with one wave to a SIMD: see the last two figures.)
 //
 // Bound by latency.  The k-th largest score is found bit by bit, from how many scores reach a candidate (a ballot and a population count per
 // 64 of them), both query blocks side by side; picking the largest topk times over, with a maximum over the wave each time, took
-// most of the time.  Key means come in as 16 bytes a lane, a chunk ahead.  Before / now, launch included: 189 x 63 blocks, top-12, 28.7 / 10.9 us;
-// 24 heads of 540 x 180, top-16, 110 / 47; 8 of 300 x 300 61 / 34; 50 x 1000, top-40, 154 / 59; 30 x 2000, top-5, 195 / 182.
+// most of the time.  Key means come in as 16 bytes a lane, a chunk ahead.  Before / now, launch included: 189 x 63 blocks, top-12, 28.8 / 9.9 us;
+// 24 heads of 540 x 180, top-16, 106 / 39; 8 of 300 x 300 60 / 31; 50 x 1000, top-40, 154 / 58; 30 x 2000, top-5, 194 / 163 (182 in scratch, 160 with one
+// wave); 8 heads of 1000 x 4000, top-16, 1370 / 533 (605, 925).
 template <int kMaxChunks>
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void ssta_mask_kernel(
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(kMaxChunks > 16 ? 2 : 1))) void ssta_mask_kernel(
     const float* __restrict__ q_mean, const float* __restrict__ k_mean, const uint8_t* __restrict__ base,
     uint8_t* __restrict__ mask, int Hq, int Hkv, int nQ, int nK, int q_block, int k_block, int topk, int band, int sink, const TileWindow window) {
   __shared__ __attribute__((aligned(16))) float k_lds[kChunk * kRowStride];
@@ -91,20 +95,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void ssta_mask
   const int64_t kv_seq = (bh / Hq) * Hkv + (bh % Hq) / (Hq / Hkv);
   const int i0 = blockIdx.x * kQPerGroup;
   const int n_chunks = (nK + kChunk - 1) / kChunk;
-  const float4* const k_rows = reinterpret_cast<const float4*>(k_mean) + kv_seq * nK * (kD / 4);
-  float4 ahead[kLoads];
+  const f32x4* const k_rows = reinterpret_cast<const f32x4*>(k_mean) + kv_seq * nK * (kD / 4);
+  f32x4 ahead[kLoads];
   auto load = [&](int chunk) {
 #pragma unroll
     for (int x = 0; x < kLoads; ++x) {
       const int j = chunk * kChunk + (tid >> 5) + 8 * x;
-      ahead[x] = j < nK ? k_rows[(size_t)j * (kD / 4) + (tid & 31)] : make_float4(0.f, 0.f, 0.f, 0.f);
+      ahead[x] = j < nK ? k_rows[(size_t)j * (kD / 4) + (tid & 31)] : (f32x4){0.f, 0.f, 0.f, 0.f};
     }
   };
   load(0);
   {
     const int i = i0 + (tid >> 5);
-    reinterpret_cast<float4*>(q_lds)[tid] =
-        i < nQ ? reinterpret_cast<const float4*>(q_mean)[((size_t)bh * nQ + i) * (kD / 4) + (tid & 31)] : make_float4(0.f, 0.f, 0.f, 0.f);
+    reinterpret_cast<f32x4*>(q_lds)[tid] =
+        i < nQ ? reinterpret_cast<const f32x4*>(q_mean)[((size_t)bh * nQ + i) * (kD / 4) + (tid & 31)] : (f32x4){0.f, 0.f, 0.f, 0.f};
   }
   uint32_t key[kQPerWave][kMaxChunks];
 #pragma unroll
@@ -113,15 +117,15 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void ssta_mask
     if (t < n_chunks) {  // uniform over the work-group
       __syncthreads();
 #pragma unroll
-      for (int x = 0; x < kLoads; ++x) *reinterpret_cast<float4*>(k_lds + ((tid >> 5) + 8 * x) * kRowStride + 4 * (tid & 31)) = ahead[x];
+      for (int x = 0; x < kLoads; ++x) *reinterpret_cast<f32x4*>(k_lds + ((tid >> 5) + 8 * x) * kRowStride + 4 * (tid & 31)) = ahead[x];
       __syncthreads();
       if (t + 1 < n_chunks) load(t + 1);
       float s0 = 0.f, s1 = 0.f;
-      const float4* kr = reinterpret_cast<const float4*>(k_lds + lane * kRowStride);
-      const float4* q0 = reinterpret_cast<const float4*>(q_lds + (wave * kQPerWave) * kD);
+      const f32x4* kr = reinterpret_cast<const f32x4*>(k_lds + lane * kRowStride);
+      const f32x4* q0 = reinterpret_cast<const f32x4*>(q_lds + (wave * kQPerWave) * kD);
 #pragma unroll 8
       for (int d = 0; d < kD / 4; ++d) {
-        const float4 kv = kr[d], a = q0[d], b = q0[kD / 4 + d];
+        const f32x4 kv = kr[d], a = q0[d], b = q0[kD / 4 + d];
         s0 = __builtin_fmaf(a.x, kv.x, s0); s1 = __builtin_fmaf(b.x, kv.x, s1);
         s0 = __builtin_fmaf(a.y, kv.y, s0); s1 = __builtin_fmaf(b.y, kv.y, s1);
         s0 = __builtin_fmaf(a.z, kv.z, s0); s1 = __builtin_fmaf(b.z, kv.z, s1);
