@@ -64,6 +64,9 @@ constexpr int kChunk = 64;          // key blocks per LDS chunk: one per lane
 constexpr int kMostChunks = 64;     // nK <= 4096
 constexpr int kRowStride = kD + 4;  // floats; 16 lanes read 16 bytes of a row each from 64 different banks
 
+// Four floats of a mean.  Callers hand in means at the address of any float, and so much alignment is all that the loads may be told of.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));
+
 // A score as an unsigned number in the same order; 0 for what is never picked (NaN, -inf, no key block).  -0 becomes +0 as an integer:
 // -ffast-math knows no signed zeros and would drop an addition of +0.
 __device__ __forceinline__ uint32_t rank_key(float x) {
@@ -95,20 +98,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int64_t kv_seq = (bh / Hq) * Hkv + (bh % Hq) / (Hq / Hkv);
   const int i0 = blockIdx.x * kQPerGroup;
   const int n_chunks = (nK + kChunk - 1) / kChunk;
-  const f32x4* const k_rows = reinterpret_cast<const f32x4*>(k_mean) + kv_seq * nK * (kD / 4);
+  const f32x4_any* const k_rows = reinterpret_cast<const f32x4_any*>(k_mean) + kv_seq * nK * (kD / 4);
   f32x4 ahead[kLoads];
   auto load = [&](int chunk) {
 #pragma unroll
     for (int x = 0; x < kLoads; ++x) {
       const int j = chunk * kChunk + (tid >> 5) + 8 * x;
-      ahead[x] = j < nK ? k_rows[(size_t)j * (kD / 4) + (tid & 31)] : (f32x4){0.f, 0.f, 0.f, 0.f};
+      ahead[x] = j < nK ? (f32x4)k_rows[(size_t)j * (kD / 4) + (tid & 31)] : (f32x4){0.f, 0.f, 0.f, 0.f};
     }
   };
   load(0);
   {
     const int i = i0 + (tid >> 5);
     reinterpret_cast<f32x4*>(q_lds)[tid] =
-        i < nQ ? reinterpret_cast<const f32x4*>(q_mean)[((size_t)bh * nQ + i) * (kD / 4) + (tid & 31)] : (f32x4){0.f, 0.f, 0.f, 0.f};
+        i < nQ ? (f32x4)reinterpret_cast<const f32x4_any*>(q_mean)[((size_t)bh * nQ + i) * (kD / 4) + (tid & 31)] : (f32x4){0.f, 0.f, 0.f, 0.f};
   }
   uint32_t key[kQPerWave][kMaxChunks];
 #pragma unroll

@@ -43,3 +43,20 @@ def test_a_score_of_minus_zero_ties_with_zero(gpu, nK):
     k[0, 0, 1, 0], k[0, 0, 1, 127], k[0, 0, nK - 1, 0] = 0.0, -1e-30, 0.0
     got = ssta_mask_from_means(q.to(gpu), k.to(gpu), 128, 128, topk=1, band=-1, sink_blocks=0)
     assert got.flatten().nonzero().flatten().tolist() == [1]
+
+
+@pytest.mark.parametrize("nQ,nK", [(9, 63), (5, 300), (3, 1100)])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_means_at_any_float(gpu, nQ, nK, offset):
+    """Means that begin at a float that is no multiple of 16 bytes, as views of a longer buffer do."""
+    from flex_block_attn_amd.video import ssta_mask_from_means
+
+    g = torch.Generator().manual_seed(nK)
+    q, k = (torch.randn((1, 2, n, 128), generator=g).to(gpu) for n in (nQ, nK))
+    moved = []
+    for t in (q, k):
+        moved.append(torch.empty(t.numel() + 4, device=gpu)[offset:offset + t.numel()].view(t.shape).copy_(t))
+        assert moved[-1].data_ptr() % 16 == 4 * offset and moved[-1].is_contiguous()
+    want = ssta_mask_from_means(q, k, 128, 128, topk=7)
+    assert torch.equal(ssta_mask_from_means(*moved, 128, 128, topk=7), want)
+    assert torch.equal(ssta_mask_from_means(moved[0], k, 128, 128, topk=7), want)
