@@ -100,7 +100,8 @@ def test_bwd_from_the_mask(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, dims, kin
 
 
 def test_what_masked_rows_hold_is_discarded(gpu):
-    """Halves of a slab that a key tile is not selected by may hold anything: their products count for nothing."""
+    """Rows of a slab that do not select a key tile count for nothing, whatever comes of their products with it: dP overflows, P is infinite because they
+    select nothing at all.  What they hold themselves is finite (0 times an infinity of theirs would be NaN, as it is in the formula and on lists)."""
     g = torch.Generator().manual_seed(3)
     q, k, v, do = (torch.randn((1, 1, 64, 128), generator=g).to(torch.bfloat16).to(gpu) for _ in range(4))
     m = torch.tensor([[True], [False], [True], [True]], device=gpu)
@@ -110,7 +111,7 @@ def test_what_masked_rows_hold_is_discarded(gpu):
     do[0, 0, 16:32] = 3.0e38  # dP of these rows overflows
     got = _run(q, k, v, o, do, lse, 16, 64, m)
     assert torch.equal(got[0], want[0]) and bool((got[0][0, 0, 16:32] == 0).all())
-    assert torch.equal(got[1], want[1])
+    assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
 
 
 def test_the_rule_stays_within_one_buffer_of_the_forward_rule():
