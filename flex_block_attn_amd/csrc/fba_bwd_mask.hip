@@ -265,7 +265,7 @@ FBA_DEVICE void key_tile(const BwdMaskParams& p, int item, char* smem) {
       for (int e = 0; e < 4; ++e) {
         const float pv = fast_exp2(__builtin_fmaf(s[4 * g + e], p.scale_log2e, -l4[e]));
         const float ds = pv * dp[4 * g + e];
-        s[4 * g + e] = on ? pv : 0.f;  // selects: inf or NaN of a masked row is discarded
+        s[4 * g + e] = on ? pv : 0.f;  // selects: inf or NaN of a masked row's P and dS is discarded (not of its Q and dO, which meet these zeros)
         dp[4 * g + e] = on ? ds : 0.f;
       }
     }
@@ -383,7 +383,7 @@ FBA_DEVICE void query_tile(const BwdMaskParams& p, int item, char* smem) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const float ds = fast_exp2(__builtin_fmaf(s[r], p.scale_log2e, -lse2)) * dp[r];
-      dp[r] = active ? ds : 0.f;  // a select: inf or NaN of a masked row is discarded
+      dp[r] = active ? ds : 0.f;  // a select: inf or NaN of a masked row's P and dS is discarded (not of the keys it does not select)
     }
     bf16x8 dsk[2];
 #pragma unroll

@@ -40,7 +40,7 @@ constexpr int64_t kXcds = 8;
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                \
   X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists_cut) X(fba_pair_slots_bounds) X(fba_tile_slots_bounds)        \
-  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_handover) X(fba_bwd_tiled_cut) X(fba_bwd_dense) \
+  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_handover) X(fba_bwd_tiled_cut) X(fba_bwd_dense) \
   X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
