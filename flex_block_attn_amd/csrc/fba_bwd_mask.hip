@@ -13,7 +13,8 @@
 //
 // Like fwd_mask_kernel this is bound by latency: what it replaces is a chain of lists, statistics, dK/dV, merge, dQ, merge, each
 // waiting for the one in front, of which the host has to launch every one.  The slab loop has one buffer per operand, whose next
-// slab is asked for as soon as the matrix instructions that read it last have their operands.
+// slab is asked for as soon as the matrix instructions that read it last have their operands.  key_tile needs a few registers more than there are: 4 (14
+// with 16-row halves) go to scratch and come back between its two accumulations, behind copies that are on their way.
 #include <algorithm>
 #include <type_traits>
 

@@ -284,8 +284,9 @@ FBA_DEVICE void order_items(const BwdParams& p, const ItemOrder& make, int block
 // clock rises; so lists up to 1.3 times what an even share would be lose nothing by it, and cutting costs the partial results and their
 // merge, about 20 us.  (H1 S30720, 60 % kept at random, lists of 37 to 59 blocks on 240 compute units: 45 an even share, dK/dV 552 us whole; as
 // much when the longest were cut.)
-// Steps, whole lists / pieces: score-driven masks with a sink block, top-12 of 63 blocks, H1 S24192 755 / 408 us, H2 947 / 667, H3 1093 / 930 (H4 and
-// more are left alone), H2 S69120 2895 / 1738; 3 x 3 x 3 windows over 3 x 4 x 5 tiles, H1 823 / 634, H2 1506 / 1098; video latents H4 S73728 11450 / 8583.
+// Steps, whole lists / pieces (with the launches as they were before there were any; median of nine): score-driven masks with a sink block, 128-row query
+// and 384-row key blocks, top-12, H1 S24192 753 / 377 us, H2 947 / 636, top-16 H2 S69120 4196 / 2170; 3 x 3 x 3 windows over 3 x 4 x 5 tiles, H1 825 / 639, H2
+// 1495 / 1095; video latents H4 S73728 11906 / 9275.  What pieces alone are worth there: 714, 902, 4100, 822, 1473 and 11800 us without them.
 // Launches of less than a round: the smallest piece with which there is one for every compute unit at most.  Others: an even share;
 // what is longer than 1.5 of them is cut.
 struct PieceMaker {
@@ -489,8 +490,9 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
   if (ordered) p.split.main_wgs = p.split.first;
 
   // Room for pieces, where lists can be so long that cutting them pays (plan_pieces) and there are not so many that the longest cannot
-  // count.  A launch that needs none pays for work-groups that exit at once, one to a compute unit; the planning hides behind the statistics,
-  // so a dK/dV kernel called by itself goes without.
+  // count.  A launch that needs none pays for work-groups that exit at once, one to a compute unit, and for a merge that finds nothing to do (5 us in
+  // a trace): steps with / without pieces in the library, B2 H16/4 S8192 1033 / 1031 us, H8 S8192 290 / 288, H4 S16384 5 % kept 163 / 161, H1 S32768 10 % 268 / 267,
+  // H2 S32768 30 % 1276 / 1274.  The planning hides behind the statistics, so a dK/dV kernel called by itself goes without.
   PieceMaker maker{};
   const int most_pieces = p.num_items <= slots ? slots : p.num_items + slots;
   const int64_t piece_bytes = 64 + most_pieces * (int64_t)sizeof(Piece) + slots * (int64_t)sizeof(CutItem);
