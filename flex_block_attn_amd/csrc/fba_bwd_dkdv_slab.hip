@@ -51,7 +51,11 @@ using IC = std::integral_constant<int, N>;
 }  // namespace
 
 // kHandOver: every wave also stores the bf16 dS it forms to p.ds_ws (tile pairs of 16 units, see fba_common.h).
-// kHalves: q_block is an odd multiple of 16, so a 32-row slab may be selected by one of its 16-row halves only.
+// kHalves: q_block is an odd multiple of 16, so that 16-row groups select for themselves.  The list then holds the groups that select
+// these keys, and a slab is two neighbours of the list, wherever in the sequence their rows lie: the matrix instructions sum dV and dK
+// over 16 rows each, S and dP take the 32 rows as they come, and the two halves of a dS unit are stored apart.  With slabs of rows that follow
+// each other, half of such a slab was often masked (16-row blocks, a quarter kept: 42 % of the slabs worked on for 24 % of the
+// rows): B2 H8/2 S3136 q16 k64, 12 of 49 kept, step 241 -> 208 us; B1 H22/11 S14080 q16 k64, 131 of 220 kept 8.02 -> 6.99 ms.
 template <bool kHandOver, bool kHalves>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void dkdv_slab_kernel(const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -100,7 +104,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   uint32_t dma_off[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
-    const int row = 16 * kg + 4 * g + (lane >> 4);
+    const int row = 4 * g + (lane >> 4);  // of the 16
     dma_off[g] = (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4));
   }
   {  // V rows: wave w brings in rows 8 w .. 8 w + 7 (two copies)
@@ -119,11 +123,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     for (int ks = 0; ks < 8; ++ks) kreg[ks] = *reinterpret_cast<const bf16x8*>(kp + 16 * ks);
   }
 
-  // Compaction of the tile's lists (one per query head of the group) into LDS, a round of 512 entries at a time: every wave
+  // Compaction of the tile's lists (one per query head of the group) into LDS, a round of kRound entries at a time: every wave
   // tests 64 of them and the waves' counts give each its place.  The scan position is scalar state, the same in all waves.
-  // An LDS entry is {slab number over all heads << 2 | bits of its two 16-row halves, tile-pair number}.
+  // An LDS entry is {number over all heads, tile-pair number} of a slab, or of a 16-row group (kHalves: two threads to a list entry).
   int scan_g = fits ? 0 : group, scan_e = 0, seen = 0, flip_count = 0;
   int2* const list = reinterpret_cast<int2*>(smem + kListBase);
+  constexpr int kScan = kHalves ? kRound / 2 : kRound;  // list entries of a round
+  const int scan_at = kHalves ? tid >> 1 : tid, scan_half = kHalves ? tid & 1 : 0;
   // Places the entries of this half numbered [lo, hi) that follow the scan position, as many rounds as fit; returns how many.
   auto fill = [&](int lo, int hi) -> int {
     int n = 0;
@@ -133,23 +139,23 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
       const int cnt = const_idx(p.k_cnt)[lr];
       // entries are asked for a round ahead, the first ones before the count is there
       auto load = [&](const int32_t* x, int e) { return e < row_len ? x[lr * row_len + e] : 0; };
-      int ent_ahead = load(p.k_idx, scan_e + tid), pair_ahead = 0;
-      if constexpr (kHandOver) pair_ahead = p.pair_base != nullptr ? load(p.k_slot, scan_e + tid) : 0;
+      int ent_ahead = load(p.k_idx, scan_e + scan_at), pair_ahead = 0;
+      if constexpr (kHandOver) pair_ahead = p.pair_base != nullptr ? load(p.k_slot, scan_e + scan_at) : 0;
       while (scan_e < cnt) {
         if (n > kChapter - kRound || seen >= hi) return n;
-        const int e = scan_e + tid;
+        const int e = scan_e + scan_at;
         const int ent = e < cnt ? ent_ahead : 0;
         int pair = pair_ahead;
-        ent_ahead = load(p.k_idx, e + kRound);
+        ent_ahead = load(p.k_idx, e + kScan);
         if constexpr (kHandOver) {
           if (p.pair_base == nullptr) {  // dense numbering
             pair = (int)((bh * lists_per_head + (kt >> 1)) * (p.Sq / 128)) + (ent >> 10);
           } else {
-            pair_ahead = load(p.k_slot, e + kRound);
+            pair_ahead = load(p.k_slot, e + kScan);
             if (p.mask_bh == 1) pair += (int)(bh * const_idx(p.pair_base)[lists_per_head]);
           }
         }
-        const int bits = (ent >> (4 * half)) & 3;
+        const int bits = (ent >> (4 * half + scan_half)) & (kHalves ? 1 : 3);
         const unsigned long long on = __ballot(bits != 0);
         int* counts = reinterpret_cast<int*>(smem + kCountBase) + 8 * flip_count;
         flip_count ^= 1;
@@ -166,13 +172,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         const int at = seen + before + __popcll(on & ((1ull << lane) - 1ull));
         if (bits != 0 && at >= first && at < last) {
           int2 v;
-          v.x = (((int)(bh * row_len) + (ent >> 8)) << 2) | bits;
+          v.x = (int)(bh * row_len) + (ent >> 8);
+          if constexpr (kHalves) v.x = 2 * v.x + scan_half;
           v.y = pair;
           list[n + at - first] = v;
         }
         n += last > first ? last - first : 0;
         seen += all;
-        scan_e += kRound;
+        scan_e += kScan;
       }
       scan_e = 0;
       ++scan_g;
@@ -185,8 +192,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     const int total = seen;
     scan_g = fits ? 0 : group;
     scan_e = seen = 0;
-    lo = (int)((int64_t)total * part / parts);
-    hi = (int)((int64_t)total * (part + 1) / parts);
+    constexpr int kWhole = kHalves ? -2 : -1;  // pairs of 16-row groups stay together
+    lo = (int)((int64_t)total * part / parts) & kWhole;
+    hi = part + 1 == parts ? total : (int)((int64_t)total * (part + 1) / parts) & kWhole;
     __syncthreads();  // what the counting scan left in the list is not mixed with what follows
   }
 
@@ -205,8 +213,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   const char* const dobase = reinterpret_cast<const char*>(p.d_o);
   const char* const stbase = reinterpret_cast<const char*>(p.stats);
   const int64_t rows_total = (int64_t)p.B * p.Hq * p.Sq;
-  // statistics copy: lanes 0..31 fetch lse2[row0 + l], lanes 32..63 fetch -delta[row0 + l - 32]
-  const uint32_t stat_off = (uint32_t)((lane >> 5) * rows_total * 4 + (lane & 31) * 4);
+  // statistics copy: lanes 0..31 fetch lse2 of the slab's 32 rows, lanes 32..63 -delta
+  const uint32_t stat_off = (uint32_t)((lane >> 5) * rows_total * 4 + (lane & (kHalves ? 15 : 31)) * 4);
   const uint32_t ho_off0 = (uint32_t)ds_unit_store_off(0, lane);
   const float c = p.scale_log2e;
   // ring buffer of position `par`, step parity s: byte (2 par + s) * kStageBytes
@@ -226,17 +234,23 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   }
   const LdsPtr st_ptr = lds + 2 * par * kStageBytes + 2 * kSlabBytes + 16 * h;
 
+  // A slab of the list: first row / 16 and tile-pair number of its two 16-row groups, which follow each other unless kHalves; `both` is
+  // false where a list of an odd number of groups leaves the second place empty (the first group is copied there once more).
+  struct Slab {
+    int row[2], pair[2];
+    bool both;
+  };
   // Copy i (0..8) of the nine that a wave owes for its slab of a step: Q rows, dO rows, statistics.
-  auto copy_part = [&](int i, uint32_t dst, int slab) {
-    const int64_t row = (int64_t)slab * kSlab;
+  auto copy_part = [&](int i, uint32_t dst, const Slab& t) {
+    const int64_t row = (int64_t)(kg == 0 ? t.row[0] : t.row[1]) * 16;
     if (i < 4) dma16(dst + (16 * kg + 4 * i) * kRowBytes, qbase + row * kRowBytes, dma_off[i]);
     else if (i < 8) dma16(dst + kSlabBytes + (16 * kg + 4 * (i - 4)) * kRowBytes, dobase + row * kRowBytes, dma_off[i - 4]);
-    else dma4(dst + 2 * kSlabBytes, stbase + row * 4, stat_off);  // both waves copy the same 256 bytes
+    else dma4(dst + 2 * kSlabBytes, stbase + (int64_t)t.row[0] * 64, kHalves && (lane & 16) != 0 ? stat_off + (t.row[1] - t.row[0]) * 64 : stat_off);  // both waves copy the same 256 bytes
   };
 
   // One slab against this wave's 32 keys.  The copies of the next step's slab are issued in between the matrix
   // instructions of S and dP.
-  auto compute = [&](auto buf_c, int x, int y, int x_next) {
+  auto compute = [&](auto buf_c, const Slab& cur, const Slab& next) {
     constexpr int so = decltype(buf_c)::value * kStageBytes;
     constexpr int no = kStageBytes - so;
     f32x16 s, dp;
@@ -251,17 +265,15 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     for (int ks = 0; ks < 8; ++ks) {
       s = mfma32(lds_read_b128(q_ptr[ks] + so), kreg[ks], s);
       dp = mfma32(lds_read_b128(q_ptr[ks] + so + kSlabBytes), lds_read_b128(v_ptr[ks]), dp);
-      copy_part(ks, ring_dst + no, x_next >> 2);
+      copy_part(ks, ring_dst + no, next);
     }
-    copy_part(8, ring_dst + no, x_next >> 2);
-    const bool on0 = !kHalves || (x & 1) != 0, on1 = !kHalves || (x & 2) != 0;  // are the two 16-row halves selected?
+    copy_part(8, ring_dst + no, next);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const f32x4 l4 = lds_read_f32x4(st_ptr + so + 32 * g);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float pv = fast_exp2(__builtin_fmaf(s[4 * g + e], c, -l4[e]));
-        if constexpr (kHalves) pv = (g < 2 ? on0 : on1) ? pv : 0.f;  // a select: inf or NaN of a masked row is discarded
+        const float pv = fast_exp2(__builtin_fmaf(s[4 * g + e], c, -l4[e]));
         s[4 * g + e] = pv;
         dp[4 * g + e] = pv * dp[4 * g + e];
       }
@@ -274,9 +286,21 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     }
     if constexpr (kHandOver) {
       // 16 units per tile pair, ordered (32-key slab, 32-row slab); streaming stores: written once, read once much later
-      char* unit = reinterpret_cast<char*>(p.ds_ws) + (int64_t)y * (16 * kDsUnitBytes) + ((2 * half + kg) * 4 + ((x >> 2) & 3)) * kDsUnitBytes;
-      store16_stream(unit, ho_off0, dsk[0]);
-      store16_stream_second(unit, ho_off0, dsk[1]);
+      auto unit = [&](int f) {
+        return reinterpret_cast<char*>(p.ds_ws) + (int64_t)cur.pair[f] * (16 * kDsUnitBytes) + ((2 * half + kg) * 4 + ((cur.row[f] >> 1) & 3)) * kDsUnitBytes;
+      };
+      if constexpr (kHalves) {  // the halves of a unit are those of its rows: ds_unit_store_off(1, l) is ds_unit_store_off(0, l) ^ 128, and 1024 on
+        store16_stream(unit(0) + (cur.row[0] & 1) * 1024, ho_off0 ^ (uint32_t)((cur.row[0] & 1) << 7), dsk[0]);
+        if (cur.both) store16_stream(unit(1) + (cur.row[1] & 1) * 1024, ho_off0 ^ (uint32_t)((cur.row[1] & 1) << 7), dsk[1]);
+      } else {
+        store16_stream(unit(0), ho_off0, dsk[0]);
+        store16_stream_second(unit(0), ho_off0, dsk[1]);
+      }
+    }
+    if constexpr (kHalves) {  // (whole bits, so that inf and NaN go as well)
+      const u32x4 keep = cur.both ? ~0u : 0u;
+      pk[1] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, pk[1]) & keep);
+      dsk[1] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, dsk[1]) & keep);
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -294,31 +318,45 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   // buffer nobody reads, so that every wave has the same number of copies in flight at every wait).
   while (n > 0) {
     __syncthreads();  // the list is complete
-    const int nsteps = (n + kPar - 1) / kPar;
-    auto entry_of = [&](int step) -> int2 {
-      const int at = kPar * step + par;
-      return list[at < n ? at : n - 1];
+    const int slabs = kHalves ? (n + 1) / 2 : n;
+    const int nsteps = (slabs + kPar - 1) / kPar;
+    struct Entry {
+      int2 e[2];
+      bool both;
     };
-    auto uniform = [](int2 v) -> int2 { return make_int2(__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y)); };
-    int2 cur = uniform(entry_of(0)), nxt = uniform(entry_of(1));
+    auto entry_of = [&](int step) -> Entry {
+      const int at = kPar * step + par, s = at < slabs ? at : slabs - 1;
+      if constexpr (!kHalves) return {{list[s], {}}, true};
+      const bool both = 2 * s + 1 < n;
+      return {{list[2 * s], list[both ? 2 * s + 1 : 2 * s]}, both};
+    };
+    auto uniform = [](const Entry& e) -> Slab {
+      auto u = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+      if constexpr (!kHalves) {
+        const int r = 2 * u(e.e[0].x), y = u(e.e[0].y);
+        return {{r, r + 1}, {y, y}, true};
+      }
+      return {{u(e.e[0].x), u(e.e[1].x)}, {u(e.e[0].y), u(e.e[1].y)}, e.both};
+    };
+    Slab cur = uniform(entry_of(0)), nxt = uniform(entry_of(1));
 #pragma unroll
-    for (int i = 0; i < 9; ++i) copy_part(i, ring_dst, cur.x >> 2);
+    for (int i = 0; i < 9; ++i) copy_part(i, ring_dst, cur);
     wait_vmem<0>();
     __syncthreads();
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) pin(kreg[ks]);
     auto step = [&](auto buf_c, int i) {
-      const int2 after = entry_of(i + 2);  // read ahead, used behind the barrier
-      const bool worked = kPar * i + par < n;
+      const Entry after = entry_of(i + 2);  // read ahead, used behind the barrier
+      const bool worked = kPar * i + par < slabs;
       if (worked) {
-        compute(buf_c, cur.x, cur.y, nxt.x);
+        compute(buf_c, cur, nxt);
       } else {
 #pragma unroll
-        for (int j = 0; j < 9; ++j) copy_part(j, ring_dst + kStageBytes - decltype(buf_c)::value * kStageBytes, nxt.x >> 2);
+        for (int j = 0; j < 9; ++j) copy_part(j, ring_dst + kStageBytes - decltype(buf_c)::value * kStageBytes, nxt);
       }
       // the copies of the next step's slab must have landed; the two dS stores, if any, are younger and may still fly (the
       // counter covers loads and stores alike and runs down in issue order)
-      if (kHandOver && worked) wait_vmem<2>(); else wait_vmem<0>();
+      if (kHandOver && worked && cur.both) wait_vmem<2>(); else wait_vmem<0>();
       __syncthreads();  // everybody is done with this step's buffers and everybody's copies for the next have landed
       cur = nxt;
       nxt = uniform(after);

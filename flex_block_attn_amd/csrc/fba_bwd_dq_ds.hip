@@ -15,9 +15,9 @@
 // waves: half (256 rows) or a third (384) of the K bytes, and with 384 rows half as much dS again in flight per CU.
 //
 // kTiled: tile lists.  The workspace is divided into (128-row query tile, 128-key tile) pairs of 16 units; the list of the
-// work-group's query tile names key blocks with a predicate per 16 rows.  A wave whose rows do not select a key block has
-// no unit there (the key-major kernel stored none): it copies 2 KiB of zeros instead, so that every wave issues the same
-// number of copies per stage, and leaves the matrix work of those steps out.
+// work-group's query tile names key blocks with a predicate per 16 rows.  Where 16 rows do not select a key block that half of
+// their unit was never stored: zeros are copied instead, so that every wave issues the same number of copies per stage, and a wave
+// none of whose rows do leaves the matrix work of those steps out.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -214,13 +214,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
         int pair;
         chunks.next(chunk, pair);
         chunk_k = kp + (int64_t)(chunk >> 8) * (2 * kSlabBytes);
-        chunk_ds = (chunk & wave_bits) != 0 ? ds_base + pair * pair_bytes + (chunk >> 8 & 1) * (8 * kDsUnitBytes) : nullptr;
+        chunk_ds = ds_base + pair * pair_bytes + (chunk >> 8 & 1) * (8 * kDsUnitBytes);
       }
-      const char* const src = chunk_ds != nullptr ? chunk_ds + ring % 2 * (4 * kDsUnitBytes) : p.zero_unit;
+      // the halves of a unit are the dS of its two 16-row groups, each stored where the group selects the key block
+      auto src = [&](int f) { return (chunk >> (2 * wave + f) & 1) != 0 ? chunk_ds + ring % 2 * (4 * kDsUnitBytes) : p.zero_unit; };
       dma16(dst + k_dst_wave, chunk_k + ring % 2 * kSlabBytes, k_off_lane[0]);
       dma16(dst + k_dst_wave + 4 * kRowBytes, chunk_k + ring % 2 * kSlabBytes, k_off_lane[1]);
-      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes, src, lane16);
-      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes + 1024, src, lane16 + 1024);
+      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes, src(0), lane16);
+      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes + 1024, src(1), lane16 + 1024);
       return;
     }
     if constexpr (kWaves == 4) {
