@@ -12,6 +12,9 @@
 // MFMA 32x32x16 bf16 register layouts (lane = 32*h + i):
 //   A (32 x 16): row i,  k = 8h .. 8h+7          B (16 x 32): col i, k = 8h .. 8h+7
 //   C (32 x 32): col i,  acc[4g + e] is row 8g + 4h + e
+// MFMA 16x16x32 bf16 (lane = 16*g + i):
+//   A (16 x 32): row i,  k = 8g .. 8g+7          B (32 x 16): col i, k = 8g .. 8g+7
+//   C (16 x 16): col i,  acc[e] is row 4g + e
 // The A and B layouts are the same function of (lane, k), so an accumulator whose summed index sits in the
 // registers can be re-used, after bf16 packing, as either operand of the next product.
 #pragma once
@@ -44,6 +47,8 @@ FBA_DEVICE int swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 FBA_DEVICE int tile_off(int row, int chunk) { return row * kRowBytes + ((chunk ^ swz(row)) << 4); }
 
 FBA_DEVICE f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+
+FBA_DEVICE f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 FBA_DEVICE bf16x8 lds_read_b128(const char* base, int off) {
   return *reinterpret_cast<const bf16x8*>(base + off);

@@ -639,6 +639,261 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   }
 }
 
+// Forward on tile lists whose 16-row groups select for themselves, or their 32-row groups in large launches (see takes_rows).
+//
+// Work-group = the 128 query rows of a tile list, eight waves of 16 rows, two work-groups per CU, so four waves per SIMD.  The work-group
+// brings every chunk of 64 keys that some row selects into LDS, and the waves whose rows do work on it:
+//   S^T[key, q] = K[key, :] . Q[q, :], O^T[d, q] += V^T[d, key] . P^T[key, q]      16x16x32 matrix instructions, lane = query row
+// with the pipeline of fwd_kernel (P_{t-1} V_{t-1} | softmax of S_t | S_{t+1}).
+// Row r of a 16-key tile of S^T is key pi(r), bits 2 and 3 of r swapped: the accumulator of lane group g then holds keys
+// 0..3, 8..11, 4..7, 12..15 for g = 0..3, and the transposing fetch of V, which takes 4 rows for each of two groups at a time, meets 64
+// different banks.
+// Rings of three K chunks and two V chunks (80 KiB): step t requests V_t and K_{t+3}.
+//
+// Few rows of a chunk's 128 select it (with 16-row blocks, a quarter kept, 2.2 of 8 groups), so a launch of one round is bound by how
+// long a wave takes from barrier to barrier, and one of many by LDS: a 16-row wave fetches a chunk's 32 KiB for itself, 256 of its
+// cycles.  Copies alone would take a third of that (25 TB/s from L2).  Without gradients, fwd_half_kernel / this: B2 H8/2 S3136 q16 k64, 12 of 49
+// kept 83.0 / 66.3 us (18 of them in front); B1 H22/11 S14080 q16 k64, 131 of 220 kept 2.25 / 1.58 ms.  With the three parts of a step
+// one behind the other 79.6 us and 1.71 ms; with steps of 32 keys and rings of five 83.7 and 1.87.
+constexpr int kRowsWaves = 8;
+constexpr int kRowsOf = 16;  // rows of a wave
+constexpr int kRowsTile = kRowsWaves * kRowsOf;
+constexpr int kRowsSmem = 5 * kChunkBytes;
+
+// The chunks of 64 keys of a tile list, in order: key chunk << 8 | predicate bits of its key block.  Every wave keeps 64 of them in a
+// register, one per lane, and the 64 behind them; all lanes of a wave call everything together.
+struct ChunkList {
+  const int32_t* list;
+  int row_len, per_block, lane;
+  int base, now, ahead;
+
+  FBA_DEVICE int load(int from) const {  // (needs no count: what lies past the end is not asked for)
+    const int c = from + lane, e = c / per_block;
+    const int entry = e < row_len ? list[e] : 0;
+    return ((entry >> 8) * per_block + c - e * per_block) << 8 | (entry & 255);
+  }
+  FBA_DEVICE void start(int first) {
+    base = first;
+    now = load(first);
+    ahead = load(first + 64);
+  }
+  FBA_DEVICE int at(int t) {  // t rises by at most one from call to call
+    if (t == base + 64) {
+      base = t;
+      now = ahead;
+      ahead = load(t + 64);
+    }
+    return __builtin_amdgcn_readlane(now, t - base);
+  }
+};
+
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * kRowsWaves, 64 * kRowsWaves), amdgpu_waves_per_eu(4, 4))) void fwd_rows_kernel(const FwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // K ring [3][16 KiB] | V ring [2][16 KiB]
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int item, part = 0, parts = 1;
+  if ((int)blockIdx.x < p.split.main_wgs) {
+    item = xcd_remap(blockIdx.x, p.items_per_xcd);
+    if (item >= p.split.first) return;
+  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+    return;
+  }
+  const int tiles_per_head = p.Sq / kRowsTile;
+  const int bh = item / tiles_per_head;
+  const int qt = item - bh * tiles_per_head;
+  const int b = bh / p.Hq, hq = bh - b * p.Hq;
+  const int hkv = hq / (p.Hq / p.Hkv);
+  const int64_t qrow0 = (int64_t)bh * p.Sq + (int64_t)qt * kRowsTile + wave * kRowsOf;
+  const char* const kp = reinterpret_cast<const char*>(p.k + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
+  const char* const vp = reinterpret_cast<const char*>(p.v + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
+
+  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * tiles_per_head + qt;
+  const int per_block = p.k_block / 64;
+  ChunkList list{p.q_idx + mrow * p.nK, p.nK, per_block, lane};
+
+  const int chunks = const_idx(p.q_cnt)[mrow] * per_block;
+  bf16x8 qreg[4];  // Q as the B operand: lane holds row l16, d = 32 ks + 8 g .. +7
+  {
+    const __bf16* qp = p.q + (qrow0 + l16) * kHeadDim + 8 * g;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qreg[ks] = *reinterpret_cast<const bf16x8*>(qp + 32 * ks);
+  }
+  const int t_begin = (int)((int64_t)chunks * part / parts), t_end = (int)((int64_t)chunks * (part + 1) / parts);
+  const int nsteps = t_end - t_begin;
+
+  const float c = p.scale_log2e;
+  float m_run = kNoReference, l_run = 0.f;
+  f32x4 acc[8];  // O^T: lane holds row l16, columns 16 db + 4 g .. +3
+#pragma unroll
+  for (int db = 0; db < 8; ++db) acc[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
+
+  // wave w brings in rows 8 w .. 8 w + 7 of every chunk, two copies each of K and V
+  uint32_t dma_off[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 8 * wave + 4 * i + (lane >> 4);
+    dma_off[i] = (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4));
+  }
+  const uint32_t k_dst = lds_addr(smem) + 8 * wave * kRowBytes, v_dst = k_dst + 3 * kChunkBytes;
+  // fetches: K row pi(l16) of a 16-key tile, chunk 4 ks + g; V rows pi(4 g) .. +3 and 16 on, columns 16 db .. +15
+  // (the chunk number only flips bits of an address: one register each, with the rest formed where it is used)
+  uint32_t k_base, v_base;
+  {
+    const int row = (l16 & 3) | (l16 & 4) << 1 | (l16 & 8) >> 1, vrow = (l16 >> 2) | (g & 1) << 3 | (g & 2) << 1;
+    k_base = lds_addr(smem) + tile_off(row, g);
+    v_base = lds_addr(smem) + 3 * kChunkBytes + tile_off(vrow, (lane & 3) >> 1) + 8 * (lane & 1);
+  }
+  auto k_ptr = [&](int ks) { return (LdsPtr)(uintptr_t)(k_base ^ (uint32_t)(ks << 6)); };
+  auto v_ptr = [&](int db) { return (LdsPtr)(uintptr_t)(v_base ^ (uint32_t)(db << 5)); };
+
+  if (nsteps > 0) {
+    list.start(t_begin);
+    int t_ahead = t_begin;
+    auto next_chunk = [&]() -> int { return list.at(min(t_ahead++, t_end - 1)); };  // past the end: the last one again
+    auto piece = [&](int i, uint32_t dst, const char* base, int of) { dma16(dst + 4 * i * kRowBytes, base + (int64_t)(of >> 8) * kChunkBytes, dma_off[i]); };
+    // S^T of chunk `of`, where the wave's rows select it
+    auto scores = [&](f32x4 (&s)[4], int ko) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) s[t] = mfma16(lds_read_b128(k_ptr(ks) + ko + t * 16 * kRowBytes), qreg[ks], s[t]);
+    };
+    bf16x8 pk[2];
+    auto add_pv = [&](int vo, auto between) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int db = 0; db < 8; ++db) {
+          const int off = vo + 32 * u * kRowBytes;
+          acc[db] = mfma16(cat(lds_read_tr(v_ptr(db) + off), lds_read_tr(v_ptr(db) + off + 16 * kRowBytes)), pk[u], acc[db]);
+          between(8 * u + db);
+        }
+    };
+    int c0 = next_chunk(), c1 = next_chunk(), c2 = next_chunk();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) piece(i, k_dst, kp, c0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) piece(i, k_dst + kChunkBytes, kp, c1);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) piece(i, k_dst + 2 * kChunkBytes, kp, c2);
+    int c3 = next_chunk();
+    wait_vmem<2>();  // K_0 and K_1
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) pin(qreg[ks]);
+    f32x4 s_cur[4];
+    scores(s_cur, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) pin(s_cur[t]);
+    __syncthreads();  // K_3 goes where K_0 was
+
+    bool w_prev = false;  // did this wave form P for the previous chunk?
+    // step t, RK = t % 3, RV = t % 2
+    auto step = [&](auto rk_c, auto rv_c) {
+      constexpr int RK = decltype(rk_c)::value, RV = decltype(rv_c)::value;
+      const bool w_cur = (c0 >> wave & 1) != 0, w_nxt = (c1 >> wave & 1) != 0;
+      auto copies = [&](int i) {
+        if (i < 2) piece(i, v_dst + RV * kChunkBytes, vp, c0);
+        else piece(i - 2, k_dst + RK * kChunkBytes, kp, c3);
+      };
+      if (w_prev) {
+        add_pv((1 - RV) * kChunkBytes, [&](int i) { if (i % 3 == 1 && i < 12) copies(i / 3); });
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) copies(i);
+      }
+      if (w_cur) {
+        float mx = s_cur[0][0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s_cur[i >> 2][i & 3]);
+        // every lane tests the 16 keys it holds; the row's maximum is formed only when the reference rises (see softmax_reference)
+        if (__builtin_amdgcn_ballot_w64((mx - m_run) * c > kLazy) != 0) {
+          mx = fmaxf(mx, __shfl_xor(mx, 16));
+          const float m_new = fmaxf(m_run, max_halves(mx));
+          const float alpha = fast_exp2((m_run - m_new) * c);
+          m_run = m_new;
+          l_run *= alpha;
+#pragma unroll
+          for (int db = 0; db < 8; ++db) acc[db] *= alpha;
+        }
+      }
+      f32x4 s_nxt[4];
+      if (w_nxt) {
+        scores(s_nxt, (RK + 1) % 3 * kChunkBytes);  // past the last chunk: stale data, unused
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s_nxt[t] = s_cur[t];
+      }
+      if (w_cur) {
+        const float mc = m_run * c;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_cur[i >> 2][i & 3] = fast_exp2(__builtin_fmaf(s_cur[i >> 2][i & 3], c, -mc));
+        const bf16x2 one2 = {(__bf16)1.f, (__bf16)1.f};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const f32x4 lo = s_cur[2 * u], hi = s_cur[2 * u + 1];
+          pk[u] = pack8(lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) l_run = __builtin_amdgcn_fdot2_f32_bf16((bf16x2){pk[u][2 * t], pk[u][2 * t + 1]}, one2, l_run, false);
+        }
+      }
+      w_prev = w_cur;
+      pin(pk[0]);
+      pin(pk[1]);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) s_cur[t] = s_nxt[t];
+      c0 = c1;
+      c1 = c2;
+      c2 = c3;
+      c3 = next_chunk();
+      // V_t and K_{t+2} must have landed; the two copies of K_{t+3} may still fly.  (A list load among them only makes the wait stricter.)
+      wait_vmem<2>();
+      __syncthreads();
+    };
+    for (int t = 0; t < nsteps; t += 6) {
+      step(IC<0>{}, IC<0>{});
+      if (t + 1 >= nsteps) break;
+      step(IC<1>{}, IC<1>{});
+      if (t + 2 >= nsteps) break;
+      step(IC<2>{}, IC<0>{});
+      if (t + 3 >= nsteps) break;
+      step(IC<0>{}, IC<1>{});
+      if (t + 4 >= nsteps) break;
+      step(IC<1>{}, IC<0>{});
+      if (t + 5 >= nsteps) break;
+      step(IC<2>{}, IC<1>{});
+    }
+    if (w_prev) add_pv(((nsteps - 1) & 1) * kChunkBytes, [](int) {});
+  }
+  wait_vmem<0>();  // no copy is writing LDS any more
+  __syncthreads();
+
+  l_run += __shfl_xor(l_run, 16);
+  const float l = sum_halves(l_run);
+  if (parts > 1) {  // as in fwd_kernel
+    float* slot = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (kFwdSlotBytes / 4);
+    float* prow = slot + (wave * kRowsOf + l16) * kHeadDim + 4 * g;
+#pragma unroll
+    for (int db = 0; db < 8; ++db) *reinterpret_cast<f32x4*>(prow + 16 * db) = acc[db];
+    if (g == 0) {
+      slot[kRowsTile * kHeadDim + wave * kRowsOf + l16] = m_run * c;
+      slot[kRowsTile * kHeadDim + kRowsTile + wave * kRowsOf + l16] = l;
+    }
+    return;
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  if (g == 0) p.lse[qrow0 + l16] = l > 0.f ? (m_run * c + __builtin_log2f(l)) * 0.6931471805599453f : -INFINITY;
+  char* const own = smem + wave * kRowsOf * kRowBytes;  // so that a store fills four whole rows
+#pragma unroll
+  for (int db = 0; db < 8; ++db)
+    *reinterpret_cast<bf16x4*>(own + tile_off(l16, 2 * db + (g >> 1)) + 8 * (g & 1)) = pack4(acc[db][0] * inv, acc[db][1] * inv, acc[db][2] * inv, acc[db][3] * inv);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    *reinterpret_cast<bf16x8*>(p.o + (qrow0 + 4 * i) * kHeadDim + lane * 8) = lds_read_b128(own, tile_off(4 * i + (lane >> 4), lane & 15));
+}
+
 // Forward straight from the block mask, for problems too small to fill the GPU: no lists, no parts, one launch.
 //
 // Work-group = 32 query rows, eight waves, one work-group per CU.  Every wave reads the mask row of these rows itself (64 key
@@ -838,8 +1093,31 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void fwd_merge
   }
 }
 
+namespace {
+
+// Does a forward pass on tile lists go to fwd_rows_kernel?  Its 128-row work-groups leave out every 16 rows that do not select a chunk, and
+// bring in chunks that any of the 128 rows selects; fwd_half_kernel works on 32 rows and 64.  No gradients, fwd_half_kernel / fwd_rows_kernel, 64-token key
+// blocks, 12, 25 and 50 % kept (chunks of a compute unit alone in a launch of few work-groups come slowly, so those stay):
+//   16-row blocks: 256 tiles (H8 S4096) 35.4 / 43.5, 55.2 / 60.9, 78.1 / 78.1 us; 320 (H10 S4096) 50.4 / 50.5, 74.7 / 71.4, 102.2 / 93.3; 512 (H16
+//     S4096) 62.6 / 51.0, 101 / 72.5, 147 / 101; 704 (H22 S4096) 86.4 / 84.4, 141 / 119, 208 / 161; at 90 % 320 tiles 116 / 122, 704 240 / 214.
+//   32-row blocks: 320 tiles 39.3 / 39.5, 54.2 / 59.8, 78.8 / 88.8 us; 704 57.4 / 62.3, 92.0 / 97.4, 154 / 153; 1080 (H9 S15360) 245 / 237, 437 / 409, 772 / 682;
+//     2880 (H24 S15360) 652 / 634, 1147 / 1112, 2027 / 1894.
+//   64-row blocks: H24 S30720, 40 % kept 4.54 / 5.10 ms.
+bool takes_rows(const FwdParams& p) {
+  const int64_t tiles = (int64_t)p.B * p.Hq * (p.Sq / kRowsTile), units = device_compute_units();
+  return p.q_block % 32 != 0 ? 4 * tiles >= 5 * units : p.q_block % 64 != 0 && tiles >= 4 * units;
+}
+
+}  // namespace
+
 // Tail splitting (two work-groups per compute unit); the 384-row kernel does without.
 void plan_fwd(FwdParams& p) {
+  if (p.tiled && takes_rows(p)) {  // (steps of 64 keys against 128 rows; lines of 30 to 48 units cut the same launches)
+    p.num_items = p.B * p.Hq * (p.Sq / kRowsTile);
+    const ListLengths lengths{p.q_cnt, p.mask_bh == 1, kRowsTile, 128, p.Sq / 128, 1, p.k_block / 64};
+    p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{22, 30, 40}, kFwdSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
+    return;
+  }
   if (p.tiled) {  // a step is as long as one of fwd_kernel, a part's results are half as large
     p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
     const ListLengths lengths{p.q_cnt, p.mask_bh == 1, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
@@ -855,15 +1133,20 @@ void plan_fwd(FwdParams& p) {
 
 namespace {
 
-hipError_t launch_fwd_halves(FwdParams p, hipStream_t stream) {
-  void (*fn)(const FwdParams) = p.q_block % 64 != 0 ? &fwd_half_kernel<true> : &fwd_half_kernel<false>;
+hipError_t launch_fwd_tiled(FwdParams p, hipStream_t stream) {
+  const bool rows = takes_rows(p);
+  void (*fn)(const FwdParams) = rows ? &fwd_rows_kernel : p.q_block % 64 != 0 ? &fwd_half_kernel<true> : &fwd_half_kernel<false>;
+  const int smem = rows ? kRowsSmem : kHalfSmem, threads = rows ? 64 * kRowsWaves : 256;
   plan_fwd(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kHalfSmem);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kHalfSmem, stream, p);
-  if (split_items > 0) hipLaunchKernelGGL(fwd_merge_kernel<kHalfRows>, dim3(merge_grid(split_items * kHalfRows / 8)), dim3(256), 0, stream, p);
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(threads), smem, stream, p);
+  if (split_items > 0) {
+    if (rows) hipLaunchKernelGGL(fwd_merge_kernel<kRowsTile>, dim3(merge_grid(split_items * kRowsTile / 8)), dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL(fwd_merge_kernel<kHalfRows>, dim3(merge_grid(split_items * kHalfRows / 8)), dim3(256), 0, stream, p);
+  }
   return hipGetLastError();
 }
 
@@ -891,7 +1174,7 @@ hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream) {
 }
 
 hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
-  if (p.tiled) return launch_fwd_halves(p, stream);
+  if (p.tiled) return launch_fwd_tiled(p, stream);
   const bool wide = p.q_block % 384 == 0 && p.variant != 1;
   const int smem = (wide ? 12 : 2 * kRing) * kSlabBytes;  // the rings; the results of twelve waves
   void (*fn)(const FwdParams) = wide ? &fwd_kernel<12> : &fwd_kernel<4>;
