@@ -13,11 +13,6 @@
 // by the waves, mostly L2 hits) and dS units (2 KiB per wave, each read exactly once from HBM) travel global -> LDS directly
 // into a ring of four stages; stage t+4 is requested when stage t is dead.  More rows per work-group share a K slab among more
 // waves: half (256 rows) or a third (384) of the K bytes, and with 384 rows half as much dS again in flight per CU.
-//
-// kTiled: tile lists.  The workspace is divided into (128-row query tile, 128-key tile) pairs of 16 units; the list of the
-// work-group's query tile names key blocks with a predicate per 16 rows.  Where 16 rows do not select a key block that half of
-// their unit was never stored: zeros are copied instead, so that every wave issues the same number of copies per stage, and a wave
-// none of whose rows do leaves the matrix work of those steps out.
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -37,62 +32,14 @@ constexpr int kRing = 4;
 template <int N>
 using IC = std::integral_constant<int, N>;
 
-// Tile lists, in chunks of 64 keys (two stages of the ring), which always lie in one key block and one key tile.  Every wave keeps 64 chunks in
-// registers, one per lane: key chunk << 8 | predicate bits of its block, and the number of the tile pair it lies in; they are handed out
-// by lane, so that a stage waits for no scalar load (a block of 64 keys asked for three every two stages, and every wait for one waits for
-// the LDS reads in flight as well).  All lanes of a wave call everything together.
-template <bool kDensePairs>
-struct TileChunks {
-  const int32_t* list;
-  const int32_t* slots;  // numbered pairs: by key tile
-  int slot0, slot_step;  // dense ones: of key tile 0, to the next
-  int blocks, total, lane;  // chunks of a key block, of the list
-  int base, at;             // first of the 64 at hand, the next one among them
-  uint32_t chunk, chunk_ahead;
-  int pair, pair_ahead;
-
-  FBA_DEVICE void load(int from) {
-    const int c = from + lane;
-    chunk_ahead = 0;
-    pair_ahead = 0;
-    if (c < total) {
-      const int e = c / blocks, entry = list[e];
-      const int key = (entry >> 8) * blocks + c - e * blocks;
-      chunk_ahead = (uint32_t)key << 8 | (entry & 255);
-      pair_ahead = kDensePairs ? slot0 + (key >> 1) * slot_step : slots[key >> 1];
-    }
-  }
-  FBA_DEVICE void take() {
-    chunk = chunk_ahead;
-    pair = pair_ahead;
-    at = 0;
-    load(base + 64);
-  }
-  FBA_DEVICE void start() {
-    base = 0;
-    load(0);
-    take();
-  }
-  FBA_DEVICE void next(uint32_t& c, int& p) {
-    if (at == 64) {
-      base += 64;
-      take();
-    }
-    c = (uint32_t)__builtin_amdgcn_readlane((int)chunk, at);
-    p = __builtin_amdgcn_readlane(pair, at);
-    ++at;
-  }
-};
-
 }  // namespace
 
-template <bool kTiled, int kMode, int kWaves>  // kMode: kNumbered or kDense
+template <int kMode, int kWaves>  // kMode: kNumbered or kDense
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(kWaves == 12 ? 3 : 2, kWaves == 12 ? 3 : 2))) void dq_from_ds_kernel(
     const BwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // ring [4] of (K slab | dS units)
   constexpr int TQ = 32 * kWaves;
   constexpr int kStageBytes = stage_bytes(kWaves);
-  static_assert(!kTiled || kWaves == 4, "tile lists describe 128-row tiles");
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -115,21 +62,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
 
   const int qblk = (qt * TQ) / p.q_block;
   // the 128-row tile of the query block that this wave's rows lie in
-  const int tq = kTiled ? 0 : (qt * TQ - qblk * p.q_block) / 128 + (wave >> 2);
-  const int n_kt = p.Skv / 128;
-  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (kTiled ? tiles_per_head : p.nQ) + (kTiled ? qt : qblk);
+  const int tq = (qt * TQ - qblk * p.q_block) / 128 + (wave >> 2);
+  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * p.nQ + qblk;
   constexpr bool dense = kMode == kDense;
   {
     const int32_t* const base = dense ? p.q_cnt : p.pair_base;
-    const int32_t* const slot_row = dense || kTiled ? p.q_cnt : p.q_slot + mrow * p.nK;
+    const int32_t* const slot_row = dense ? p.q_cnt : p.q_slot + mrow * p.nK;
     read_ahead(const_idx(p.q_cnt)[mrow], const_idx(p.q_idx)[mrow * p.nK], const_idx(slot_row)[0], const_idx(base)[0],
-               const_idx(base)[dense ? 0 : p.mask_bh * (kTiled ? n_kt : p.nK)]);
+               const_idx(base)[dense ? 0 : p.mask_bh * p.nK]);
   }
   // lists that number more pairs than the workspace holds: nothing is fetched, and the output becomes NaN
   const int cnt = dense || workspace_holds_lists(p) ? const_idx(p.q_cnt)[mrow] : 0;
   const ConstIdx idx = const_idx(p.q_idx + mrow * p.nK);
-  // block lists: pair number per list entry (tile lists: see TileChunks)
-  const ConstIdx slots = const_idx(dense || kTiled ? nullptr : p.q_slot + mrow * p.nK);
+  // pair number per list entry
+  const ConstIdx slots = const_idx(dense ? nullptr : p.q_slot + mrow * p.nK);
   auto slot = [&](int e) -> int64_t {
     if constexpr (!dense) return slots[e];
     else return ((int64_t)bh * p.nK + idx[e]) * p.nQ + qblk;
@@ -141,12 +87,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const int t_end = parts == 1 ? steps_all : 4 * (int)(((int64_t)(steps_all / 4) * (part + 1)) / parts);
   const int nsteps = t_end - t_begin;
   const int e_begin = t_begin / nsub, sub_begin = t_begin - e_begin * nsub;
-  const int64_t pair_bytes = kTiled ? 16 * kDsUnitBytes : (int64_t)p.q_block * p.k_block * 2;
-  // dS of this wave's 32 rows: pair base + (tq * nsub + t) * 4 units + wave, t = 32-key slab inside the key block (inside
-  // the key tile with tile lists)
-  const int64_t head_pairs = p.mask_bh == 1 && !dense ? (int64_t)bh * const_idx(p.pair_base)[kTiled ? n_kt : p.nK] : 0;
+  const int64_t pair_bytes = (int64_t)p.q_block * p.k_block * 2;
+  // dS of this wave's 32 rows: pair base + (tq * nsub + t) * 4 units + wave, t = 32-key slab inside the key block
+  const int64_t head_pairs = p.mask_bh == 1 && !dense ? (int64_t)bh * const_idx(p.pair_base)[p.nK] : 0;
   const char* ds_base = reinterpret_cast<const char*>(p.ds_ws) + head_pairs * pair_bytes + ((int64_t)tq * nsub * 4 + (wave & 3)) * kDsUnitBytes;
-  const int wave_bits = 3 << (2 * wave);  // predicate bits of this wave's two 16-row groups in a tile-list entry
 
   TransposedOffsets tr;
   tr.init(lane);
@@ -188,42 +132,14 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   // sources of the next stage to request, in list order; the following list entry is read one block ahead
   const int64_t block_bytes = (int64_t)p.k_block * kRowBytes;
   int e_next = e_begin + 1, rem = nsub - sub_begin;
-  int64_t k_off = nsteps > 0 && !kTiled ? idx[e_begin] * block_bytes + (int64_t)sub_begin * kSlabBytes : 0;
-  int64_t ds_off_g = nsteps > 0 && !kTiled ? slot(e_begin) * pair_bytes + (int64_t)sub_begin * (4 * kDsUnitBytes) : 0;
-  int blk_next = e_next < cnt && !kTiled ? idx[e_next] : 0;
-  int64_t slot_next = e_next < cnt && !kTiled ? slot(e_next) : 0;
-  [[maybe_unused]] TileChunks<dense> chunks;
-  uint32_t chunk = 0;                      // tile lists: the chunk whose stages are being requested (see TileChunks)
-  const char *chunk_k = kp, *chunk_ds = ds_base;
-  if constexpr (kTiled) {
-    chunks.list = p.q_idx + mrow * p.nK;
-    chunks.slots = dense ? nullptr : p.q_slot + mrow * n_kt;
-    chunks.slot0 = dense ? (int)(bh * n_kt * tiles_per_head + qt) : 0;
-    chunks.slot_step = tiles_per_head;
-    chunks.blocks = p.k_block / 64;
-    chunks.total = cnt * chunks.blocks;
-    chunks.lane = lane;
-    chunks.start();
-  }
+  int64_t k_off = nsteps > 0 ? idx[e_begin] * block_bytes + (int64_t)sub_begin * kSlabBytes : 0;
+  int64_t ds_off_g = nsteps > 0 ? slot(e_begin) * pair_bytes + (int64_t)sub_begin * (4 * kDsUnitBytes) : 0;
+  int blk_next = e_next < cnt ? idx[e_next] : 0;
+  int64_t slot_next = e_next < cnt ? slot(e_next) : 0;
   const uint32_t lane16 = (uint32_t)lane * 16;
   auto copy_next = [&](auto ring_c) {
     constexpr int ring = decltype(ring_c)::value;
     const uint32_t dst = ring_dst + ring * kStageBytes;
-    if constexpr (kTiled) {
-      if constexpr (ring % 2 == 0) {
-        int pair;
-        chunks.next(chunk, pair);
-        chunk_k = kp + (int64_t)(chunk >> 8) * (2 * kSlabBytes);
-        chunk_ds = ds_base + pair * pair_bytes + (chunk >> 8 & 1) * (8 * kDsUnitBytes);
-      }
-      // the halves of a unit are the dS of its two 16-row groups, each stored where the group selects the key block
-      auto src = [&](int f) { return (chunk >> (2 * wave + f) & 1) != 0 ? chunk_ds + ring % 2 * (4 * kDsUnitBytes) : p.zero_unit; };
-      dma16(dst + k_dst_wave, chunk_k + ring % 2 * kSlabBytes, k_off_lane[0]);
-      dma16(dst + k_dst_wave + 4 * kRowBytes, chunk_k + ring % 2 * kSlabBytes, k_off_lane[1]);
-      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes, src(0), lane16);
-      dma16_stream(dst + kSlabBytes + wave * kDsUnitBytes + 1024, src(1), lane16 + 1024);
-      return;
-    }
     if constexpr (kWaves == 4) {
       dma16(dst + k_dst_wave, kp + k_off, k_off_lane[0]);
       dma16(dst + k_dst_wave + 4 * kRowBytes, kp + k_off, k_off_lane[1]);
@@ -247,15 +163,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   };
 
   if (nsteps > 0) {
-    // tile lists: predicate bits of the chunk whose two stages are worked on, for stages 0, 1 and 2, 3 of the ring; 0 past the end
-    uint32_t bits[2] = {255, 255}, bits_new = 0;
     if (0 < nsteps) copy_next(IC<0>{});
-    if constexpr (kTiled) bits[0] = chunk;
     if (1 < nsteps) copy_next(IC<1>{});
     if (2 < nsteps) copy_next(IC<2>{});
-    if constexpr (kTiled) bits[1] = 2 < nsteps ? chunk : 0;
     if (3 < nsteps) copy_next(IC<3>{});
-    // stage 0 (B2 H8/2 S3136, 16 x 64 blocks, one round of work-groups: 55.3 -> 53.4 us against waiting for all four)
+    // stage 0
     if (3 < nsteps) wait_stages(IC<3>{}); else wait_vmem<0>();
     __syncthreads();
 
@@ -263,26 +175,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     auto step = [&](auto ring_c, int t) {
       constexpr int R = decltype(ring_c)::value;
       const char* stage = smem + R * kStageBytes;
-      if (!kTiled || (bits[R / 2] & wave_bits) != 0) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const bf16x8 dsk = cat(lds_read_tr(stage, ds_off[j][0]), lds_read_tr(stage, ds_off[j][1]));
+      for (int j = 0; j < 2; ++j) {
+        const bf16x8 dsk = cat(lds_read_tr(stage, ds_off[j][0]), lds_read_tr(stage, ds_off[j][1]));
 #pragma unroll
-          for (int mb = 0; mb < 4; ++mb) {
-            const int roff = 16 * j * kRowBytes;
-            const bf16x8 a = cat(lds_read_tr(stage, tr.rd[mb][0] + roff), lds_read_tr(stage, tr.rd[mb][1] + roff));
-            acc[mb] = mfma32(a, dsk, acc[mb]);
-          }
+        for (int mb = 0; mb < 4; ++mb) {
+          const int roff = 16 * j * kRowBytes;
+          const bf16x8 a = cat(lds_read_tr(stage, tr.rd[mb][0] + roff), lds_read_tr(stage, tr.rd[mb][1] + roff));
+          acc[mb] = mfma32(a, dsk, acc[mb]);
         }
       }
       // stage t+1 must have landed (first read in step t+1); the copies of stages t+2 and t+3 may still fly
       if (t + 3 < nsteps) wait_stages(IC<2>{}); else if (t + 2 < nsteps) wait_stages(IC<1>{}); else wait_stages(IC<0>{});
       __syncthreads();
       if (t + 4 < nsteps) copy_next(IC<R>{});
-      if constexpr (kTiled) {
-        if constexpr (R % 2 == 0) bits_new = t + 4 < nsteps ? chunk : 0;
-        else bits[R / 2] = bits_new;
-      }
     };
     for (int t = 0; t < nsteps; t += 4) {  // nsteps is a multiple of 4
       step(IC<0>{}, t);
@@ -304,15 +210,235 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
     return;
   }
   // (the ring is free: the last step ended with a barrier and requested nothing)
-  if constexpr (kTiled)
-    store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + (qrow0 - (int64_t)bh * (p.Sq - p.out_q)) * kHeadDim, lane, p.out_q - qt * TQ - wave * 32);
-  else
-    store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + qrow0 * kHeadDim, lane);
+  store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + qrow0 * kHeadDim, lane);
+}
+
+// dQ from dS on tile lists.  The workspace is divided into (128-row query tile, 128-key tile) pairs of 16 units; the list of the work-group's
+// query tile names key blocks with a predicate per 16 rows.
+//
+// Work-group = the 128 rows of a list, four waves of 32, two work-groups per CU.  It steps through the key blocks that some row selects, 64 keys at a
+// time, with K in a ring of two chunks, and a wave none of whose rows select a block leaves its matrix work out.  dS is fetched by every wave for itself,
+// only where its rows select: room for three chunks of 64 keys by 32 rows, the next requested as soon as one is used up, so that a wave with work in
+// two steps of five has the dS of the next seven on its way.  Where only 16 of the rows select a chunk, the other half of its units was never
+// stored and zeros are copied instead.
+//
+// Every wave walks the list twice, for K and for its dS, each time with 64 chunks in registers, one per lane, so that no step waits for a scalar load
+// (a block of 64 keys asked for three every two steps, and every wait for one waits for the LDS reads in flight as well).
+//
+// Bound by what a step takes from barrier to barrier in launches of about a round (B2 H8/2 S3136 q16 k64: 36 of 46 us without any copy),
+// by memory in large ones.  In steps of 32 keys, with zeros for every wave that has no dS there, so that all waves have as many copies in flight, / so:
+// steps of H24 S30720, 64-token blocks, 192 of 480 kept 18.97 / 18.53 ms; B2 H8/2 S3136 q16 k64, 12 of 49 kept 188.7 / 180.6 us; B2 H8/4 S9472 q64 k128, 42 of
+// 74 1817 / 1759; H22 S4096, 64-token blocks, 16 of 64 308 / 301, but 40 of 64 549 / 558.  Steps of 32 keys with dS as here 592 / 571 us (B2 H3 S7168 q16 k128); the copies of
+// dS in between the next step's matrix instructions 18.97 / 19.39 ms for the first.
+namespace {
+
+constexpr int kAhead = 3;                         // chunks of dS that a wave has room for
+constexpr int kChunkUnits = 2 * kDsUnitBytes;     // 64 keys by 32 rows
+constexpr int kTilesRing = 2;                     // chunks of K
+constexpr int kTilesSmem = kTilesRing * 2 * kSlabBytes + 4 * kAhead * kChunkUnits;  // 80 KiB
+
+// The chunks of a tile list in order: key chunk << 8 | predicate bits of its block (0 past the end).
+struct TileChunks {
+  const int32_t* list;
+  int blocks, total, lane;  // chunks of a key block, chunks up to the end
+  FBA_DEVICE uint32_t load(int from) const {
+    const int c = from + lane;
+    if (c >= total) return 0;
+    const int e = c / blocks, entry = list[e];
+    return (uint32_t)((entry >> 8) * blocks + c - e * blocks) << 8 | (entry & 255);
+  }
+};
+
+}  // namespace
+
+template <int kMode>  // kNumbered or kDense
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void dq_tiles_kernel(const BwdParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // K chunks [2] | dS [wave][kAhead]
+  constexpr bool dense = kMode == kDense;
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int item, part = 0, parts = 1;
+  if ((int)blockIdx.x < p.split.main_wgs) {
+    item = xcd_remap(blockIdx.x, p.items_per_xcd);
+    if (item >= p.split.first) return;
+  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+    return;
+  }
+  const int tiles_per_head = p.Sq / 128, n_kt = p.Skv / 128;
+  const int bh = item / tiles_per_head;
+  const int qt = item - bh * tiles_per_head;
+  const int b = bh / p.Hq, hq = bh - b * p.Hq;
+  const int hkv = hq / (p.Hq / p.Hkv);
+  const int64_t qrow0 = (int64_t)bh * p.Sq + (int64_t)qt * 128 + wave * 32;
+  const char* const kp = reinterpret_cast<const char*>(p.k + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
+  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * tiles_per_head + qt;
+  {
+    const int32_t* const base = dense ? p.q_cnt : p.pair_base;
+    read_ahead(const_idx(p.q_cnt)[mrow], const_idx(base)[0], const_idx(base)[dense ? 0 : p.mask_bh * n_kt]);
+  }
+  // lists that number more pairs than the workspace holds: nothing is fetched, and the output becomes NaN
+  const int cnt = dense || workspace_holds_lists(p) ? const_idx(p.q_cnt)[mrow] : 0;
+  const int listed = cnt * (p.k_block / 64);
+  const int t_begin = (int)((int64_t)listed * part / parts), t_end = (int)((int64_t)listed * (part + 1) / parts);
+  const TileChunks chunks{p.q_idx + mrow * p.nK, p.k_block / 64, t_end, lane};
+  const int nsteps = t_end - t_begin;
+
+  // dS of this wave's rows: pair base + 32-key slab of the key tile * 4 units + wave
+  constexpr int64_t pair_bytes = 16 * kDsUnitBytes;
+  const int64_t head_pairs = p.mask_bh == 1 && !dense ? (int64_t)bh * const_idx(p.pair_base)[n_kt] : 0;
+  const char* const ds_base = reinterpret_cast<const char*>(p.ds_ws) + head_pairs * pair_bytes + wave * kDsUnitBytes;
+  const int32_t* const slots = dense ? nullptr : p.q_slot + mrow * n_kt;  // by key tile
+  const int slot0 = dense ? (int)(bh * n_kt * tiles_per_head + qt) : 0;   // dense pairs: of key tile 0
+  const uint32_t wave_bits = 3u << (2 * wave);  // predicate bits of this wave's two 16-row groups in a list entry
+
+  TransposedOffsets tr;
+  tr.init(lane);
+  uint32_t k_off_lane[4];  // K chunk: wave w brings in rows 16 w .. 16 w + 15
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int row = 4 * (4 * wave + g) + (lane >> 4);
+    k_off_lane[g] = (uint32_t)(row * kRowBytes + (((lane & 15) ^ swz(row)) << 4));
+  }
+  const uint32_t k_dst = lds_addr(smem) + 4 * wave * 4 * kRowBytes;
+  const int ds_lds = kTilesRing * 2 * kSlabBytes + wave * kAhead * kChunkUnits;
+  const uint32_t ds_dst = lds_addr(smem) + ds_lds;
+  // B operand from a unit: see dq_from_ds_kernel
+  int ds_off[2][2];
+#pragma unroll
+  for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+    for (int rr = 0; rr < 2; ++rr) {
+      const int G = lane >> 4, s = lane & 15;
+      ds_off[jj][rr] = ds_lds + ds_unit_slot_off(16 * jj + 8 * rr + 4 * (G >> 1) + (s >> 2), 4 * (G & 1) + (s & 3));
+    }
+
+  f32x16 acc[4];
+#pragma unroll
+  for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[mb][r] = 0.f;
+
+  if (nsteps > 0) {
+    // K: the chunk to be requested next
+    int k_base = t_begin, k_at = 0;
+    uint32_t k_now = chunks.load(k_base), k_ahead = chunks.load(k_base + 64);
+    auto request_k = [&](auto ring_c) -> uint32_t {  // past the end of the list chunk 0 once more, selected by nobody
+      constexpr int ring = decltype(ring_c)::value;
+      if (k_at == 64) {
+        k_base += 64;
+        k_at = 0;
+        k_now = k_ahead;
+        k_ahead = chunks.load(k_base + 64);
+      }
+      const uint32_t chunk = (uint32_t)__builtin_amdgcn_readlane((int)k_now, k_at++);
+      const char* const src = kp + (int64_t)(chunk >> 8) * (2 * kSlabBytes);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dma16(k_dst + ring * 2 * kSlabBytes + i * 4 * kRowBytes, src, k_off_lane[i]);
+      return chunk;
+    };
+    // dS: the chunks this wave selects and has not requested, among the 64 at ds_at
+    int ds_at = t_begin, pair_now, pair_ahead = 0;
+    uint32_t ds_now, ds_ahead = 0;
+    unsigned long long left;
+    auto ds_load = [&](int from) {
+      ds_ahead = chunks.load(from);
+      const int kt = (int)(ds_ahead >> 9);
+      if (from + lane < chunks.total) pair_ahead = dense ? slot0 + kt * tiles_per_head : slots[kt];
+    };
+    auto ds_take = [&] {
+      ds_now = ds_ahead;
+      pair_now = pair_ahead;
+      left = __builtin_amdgcn_ballot_w64((ds_now & wave_bits) != 0);
+      ds_load(ds_at + 64);
+    };
+    ds_load(ds_at);
+    ds_take();
+    const uint32_t lane16 = (uint32_t)lane * 16;
+    auto request_ds = [&](int place) -> bool {
+      while (left == 0) {
+        if (ds_at + 64 >= chunks.total) return false;
+        ds_at += 64;
+        ds_take();
+      }
+      const int i = __builtin_ctzll(left);
+      left &= left - 1;
+      const uint32_t of = (uint32_t)__builtin_amdgcn_readlane((int)ds_now, i);
+      const char* const src = ds_base + __builtin_amdgcn_readlane(pair_now, i) * pair_bytes + (of >> 8 & 1) * (8 * kDsUnitBytes);
+      const uint32_t dst = ds_dst + place * kChunkUnits;
+      // the halves of a unit are the dS of its two 16-row groups
+      const bool first = (of >> (2 * wave) & 1) != 0, second = (of >> (2 * wave) & 2) != 0;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        dma16_stream(dst + j * kDsUnitBytes, first ? src + j * (4 * kDsUnitBytes) : p.zero_unit, lane16);
+        dma16_stream(dst + j * kDsUnitBytes + 1024, second ? src + j * (4 * kDsUnitBytes) : p.zero_unit, lane16 + 1024);
+      }
+      return true;
+    };
+
+    uint32_t bits[2];  // of the chunks in the two places of K
+    bool all = request_ds(0);
+    bits[0] = request_k(IC<0>{});
+    all = all && request_ds(1);
+    bits[1] = request_k(IC<1>{});
+    all = all && request_ds(2);
+    if (all) wait_vmem<12>(); else wait_vmem<0>();  // the first chunk of dS and of K
+    __syncthreads();
+
+    int place = 0;     // of the next dS chunk to be used
+    bool req = false;  // was dS requested at the end of the last step?
+    // step t (t % 2 == R): dQ += K_t^T dS_t
+    auto step = [&](auto ring_c) {
+      constexpr int R = decltype(ring_c)::value;
+      const bool mine = (bits[R] & wave_bits) != 0;
+      if (mine) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const char* const k_stage = smem + (2 * R + u) * kSlabBytes;
+          const char* const ds_stage = smem + place * kChunkUnits + u * kDsUnitBytes;
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const bf16x8 dsk = cat(lds_read_tr(ds_stage, ds_off[j][0]), lds_read_tr(ds_stage, ds_off[j][1]));
+#pragma unroll
+            for (int mb = 0; mb < 4; ++mb) {
+              const int roff = 16 * j * kRowBytes;
+              const bf16x8 a = cat(lds_read_tr(k_stage, tr.rd[mb][0] + roff), lds_read_tr(k_stage, tr.rd[mb][1] + roff));
+              acc[mb] = mfma32(a, dsk, acc[mb]);
+            }
+          }
+        }
+      }
+      // K_{t+1} must have landed, requested at the end of step t - 1; the dS requested after it may still fly.  dS that step t + 1 reads is older: a chunk
+      // is requested where one is used up, with the two chunks between them still to come.
+      if (req) wait_vmem<4>(); else wait_vmem<0>();
+      __syncthreads();
+      bits[R] = request_k(IC<R>{});
+      req = mine && request_ds(place);
+      if (mine) place = place == kAhead - 1 ? 0 : place + 1;
+    };
+    for (int t = 0; t < nsteps; t += 2) {  // (an odd number of chunks: the last step has nothing to do)
+      step(IC<0>{});
+      step(IC<1>{});
+    }
+  }
+  wait_vmem<0>();  // no copy is writing LDS any more
+  __syncthreads();
+  const float poison = dense ? 1.f : poison_unless_fit(p);
+  if (parts > 1) {  // part of a split item: unscaled fp32 partial sums go to the workspace
+    float* prow = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (128 * kHeadDim) + (wave * 32 + l32) * kHeadDim;
+#pragma unroll
+    for (int mb = 0; mb < 4; ++mb)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<f32x4*>(prow + 32 * mb + 8 * g + 4 * h) =
+            (f32x4){acc[mb][4 * g + 0] * poison, acc[mb][4 * g + 1] * poison, acc[mb][4 * g + 2] * poison, acc[mb][4 * g + 3] * poison};
+    return;
+  }
+  store_tile_bf16(smem + wave * kSlabBytes, acc, p.scale * poison, p.dq + (qrow0 - (int64_t)bh * (p.Sq - p.out_q)) * kHeadDim, lane, p.out_q - qt * 128 - wave * 32);
 }
 
 namespace {
 
-// What a wave copies in place of a dS unit that nobody stored (tile lists).  Part of the library's device image and never
+// What a wave copies in place of half a dS unit that nobody stored (tile lists).  Part of the library's device image and never
 // written; host code reaches it only through the address hipGetSymbolAddress returns for the current device.
 __device__ __attribute__((aligned(256))) char g_zero_unit[kDsUnitBytes];
 
@@ -416,8 +542,13 @@ int plan_bwd_dq_from_ds(BwdParams& p) {
   const int waves = p.tiled ? 4 : p.q_block % 384 == 0 && rows / 384 >= enough ? 12 : p.q_block % 256 == 0 && rows / 256 >= enough ? 8 : 4;
   const int tile = 32 * waves;
   p.num_items = p.B * p.Hq * (p.Sq / tile);
+  if (p.tiled) {  // steps of 64 keys (B2 H3 S7168 q16 k128, two launches of 168 tiles, whole / in parts: step 586 / 570 us)
+    const ListLengths lengths{p.q_cnt, p.mask_bh == 1, tile, 128, p.Sq / 128, 1, p.k_block / 64};
+    p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{22, 28, 36, /*scans=*/false, /*own_pace=*/false}, (int64_t)tile * kHeadDim * 4, p.split.ws, p.split_ws_bytes, lengths);
+    return waves;
+  }
   const ListLengths lengths{waves == 4 ? p.q_cnt : nullptr, p.mask_bh == 1, tile, p.q_block, p.nQ, 1, p.k_block / kSlab};
-  p.split = plan_split(p.num_items, waves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18, /*scans=*/false, /*own_pace=*/false}, (int64_t)tile * kHeadDim * 4, p.tiled ? nullptr : p.split.ws,
+  p.split = plan_split(p.num_items, waves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18, /*scans=*/false, /*own_pace=*/false}, (int64_t)tile * kHeadDim * 4, p.split.ws,
                        p.split_ws_bytes, lengths);
   return waves;
 }
@@ -430,15 +561,8 @@ hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   const bool dense = p.pair_base == nullptr;
-  void (*fn)(const BwdParams) = dense ? &dq_from_ds_kernel<false, kDense, kWaves> : &dq_from_ds_kernel<false, kNumbered, kWaves>;
-  hipError_t e = hipSuccess;
-  if constexpr (kWaves == 4) {
-    if (p.tiled) {
-      fn = dense ? &dq_from_ds_kernel<true, kDense, kWaves> : &dq_from_ds_kernel<true, kNumbered, kWaves>;
-      if ((e = zero_unit_address(&p.zero_unit)) != hipSuccess) return e;
-    }
-  }
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
+  void (*fn)(const BwdParams) = dense ? &dq_from_ds_kernel<kDense, kWaves> : &dq_from_ds_kernel<kNumbered, kWaves>;
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(64 * kWaves), kSmem, stream, p);
   if (split_items > 0) {
@@ -449,11 +573,27 @@ hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+hipError_t launch_dq_tiles(BwdParams p, hipStream_t stream) {
+  plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
+  const int split_items = p.num_items - p.split.first;
+  hipError_t e = zero_unit_address(&p.zero_unit);
+  if (e != hipSuccess) return e;
+  void (*fn)(const BwdParams) = p.pair_base == nullptr ? &dq_tiles_kernel<kDense> : &dq_tiles_kernel<kNumbered>;
+  if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kTilesSmem)) != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kTilesSmem, stream, p);
+  if (split_items > 0) {
+    const PartialOut out{p.dq, p.scale, 0, p.Sq, p.out_q};
+    return launch_partial_sum(p.split, 128 * kHeadDim, 128, &out, 1, nullptr, stream);
+  }
+  return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
   if (p.ds_ws == nullptr) return hipErrorInvalidValue;
   const int waves = plan_bwd_dq_from_ds(p);
+  if (p.tiled) return launch_dq_tiles(p, stream);
   return waves == 12 ? launch_dq_rows<12>(p, stream) : waves == 8 ? launch_dq_rows<8>(p, stream) : launch_dq_rows<4>(p, stream);
 }
 

@@ -223,7 +223,7 @@ struct BwdParams {
   //   pair_base [mask_bh * Skv/128 + 1]:        exclusive prefix sum of the listed tile pairs per key tile
   //   k_slot    [mask_bh, Skv/128, Sq/32]:      pair number of every kt_ent entry
   //   q_slot    [mask_bh, Sq/128, Skv/128]:     pair number of (query tile, key tile), -1 where nothing is listed
-  //   zero_unit: 2 KiB of zeros in device memory, read in place of a dS unit that no wave stored
+  //   zero_unit: 2 KiB of zeros in device memory, read in place of half a dS unit that no wave stored
   // pair_base null: dense numbering, a place for every pair whether selected or not, (bh * nK + J) * nQ + I (tile lists:
   // (bh * Skv/128 + U) * Sq/128 + T) with bh over all heads; q_slot and k_slot are not read
   __bf16* ds_ws;
