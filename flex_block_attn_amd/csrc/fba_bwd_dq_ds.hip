@@ -542,9 +542,13 @@ int plan_bwd_dq_from_ds(BwdParams& p) {
   const int waves = p.tiled ? 4 : p.q_block % 384 == 0 && rows / 384 >= enough ? 12 : p.q_block % 256 == 0 && rows / 256 >= enough ? 8 : 4;
   const int tile = 32 * waves;
   p.num_items = p.B * p.Hq * (p.Sq / tile);
-  if (p.tiled) {  // steps of 64 keys (B2 H3 S7168 q16 k128, two launches of 168 tiles, whole / in parts: step 586 / 570 us)
+  if (p.tiled) {
+    // Steps of 64 keys.  Parts behind a whole round only: B2 H8/4 S9472 q64 k64, 60 of 148 kept, 1184 tiles, step whole / in parts 1372 / 1337 us; in launches of less
+    // than one they give nothing: B2 H3 S7168 q16 k128 358 / 359 us, H4 S6144 q32 k64 170.5 / 171.0, H8 S2944 q64 121.5 / 121.7, H2 S3072 q64 45.2 / 44.9.
+    const bool rounds = p.num_items > enough;
     const ListLengths lengths{p.q_cnt, p.mask_bh == 1, tile, 128, p.Sq / 128, 1, p.k_block / 64};
-    p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{22, 28, 36, /*scans=*/false, /*own_pace=*/false}, (int64_t)tile * kHeadDim * 4, p.split.ws, p.split_ws_bytes, lengths);
+    p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{22, 28, 36, /*scans=*/false, /*own_pace=*/false}, (int64_t)tile * kHeadDim * 4, rounds ? p.split.ws : nullptr,
+                         p.split_ws_bytes, lengths);
     return waves;
   }
   const ListLengths lengths{waves == 4 ? p.q_cnt : nullptr, p.mask_bh == 1, tile, p.q_block, p.nQ, 1, p.k_block / kSlab};

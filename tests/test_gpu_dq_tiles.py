@@ -1,8 +1,6 @@
 """dQ from handed-over dS on tile lists: waves that select nothing, one chunk, every chunk, chunks far apart; more than 64 chunks of either walk;
-odd numbers of chunks; 32-row groups of 64-row, 32-row and 16-row query blocks; key blocks of several chunks; lists cut into parts; dense and
-numbered pairs.  Against the oracle's explicit dense formula (fp32) with the operator's parity bar for N(0,1) inputs."""
-import ctypes
-
+odd numbers of chunks; 32-row groups of 64-row, 32-row and 16-row query blocks; key blocks of several chunks; tiles behind a whole round cut into
+parts; dense and numbered pairs.  Against the oracle's explicit dense formula (fp32) with the operator's parity bar for N(0,1) inputs."""
 import pytest
 import torch
 
@@ -30,23 +28,18 @@ def _mask(kind, shape, g, gpu):
     (1, 2, 2, 256, 128 * 65, 16, 64, "far"),
     (2, 2, 1, 384, 192 * 26, 32, 64, 0.1),
     (1, 3, 3, 768, 2688, 64, 192, 0.4),
-    (1, 1, 1, 512, 16384, 64, 128, "all"),   # parts
-    (1, 3, 1, 256, 16384, 16, 64, 0.3),      # parts that begin inside a key block's list
-    (1, 20, 20, 3456, 3456, 64, 64, 0.5),    # 540 tiles: 28 behind a whole round
+    (1, 1, 1, 512, 16384, 64, 128, "all"),
+    (1, 3, 1, 256, 16384, 16, 64, 0.3),
+    (1, 20, 20, 3456, 3456, 64, 64, 0.5),    # 540 tiles: 28 behind a whole round, in parts
 ])
 def test_dq_tiles(oracle, gpu, B, Hq, Hkv, Sq, Skv, qbs, kbs, kind):
     import flex_block_attn_amd as fba
-    from flex_block_attn_amd import _lib
 
     print(f"dq tiles B{B} Hq{Hq} Hkv{Hkv} Sq{Sq} Skv{Skv} q{qbs} k{kbs} {kind}", flush=True)
     g = torch.Generator(device=gpu).manual_seed(Sq + Skv + qbs)
     m = _mask(kind, (B, Hq, Sq // qbs, Skv // kbs), g, gpu)
     q, do = (torch.randn((B, Hq, Sq, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
     k, v = (torch.randn((B, Hkv, Skv, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
-    if Skv == 16384:
-        plan = (ctypes.c_int64 * 16)()
-        _lib.call("fba_split_plan", 3, B * Hq, B, Hq, Hkv, Sq, Skv, 128, qbs, kbs, _lib.load().fba_split_workspace_bytes(), plan)
-        assert plan[1] < plan[0] and plan[2] > 1
     lists = fba.lists_for(m, qbs, kbs)
     o, lse = fba.forward_with_lists(q, k, v, qbs, kbs, lists)
     dq = fba.backward_with_lists(q, k, v, o, lse, do, qbs, kbs, lists, hand_over=True)[0]
