@@ -42,10 +42,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
   int item, part = 0, parts = 1;
-  if ((int)blockIdx.x < p.split.main_wgs) {
+  int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
+  if (ws_slot < 0) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, ws_slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / TQ;
@@ -219,7 +220,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   }
 
   if (parts > 1) {  // part of a split item: unscaled fp32 partial sums go to the workspace
-    float* prow = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
+    float* prow = p.split.ws + (int64_t)ws_slot * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -244,6 +245,7 @@ void plan_bwd_dq(BwdParams& p) {
   p.num_items = p.B * p.Hq * (p.Sq / 128);
   const ListLengths lengths{p.q_cnt, p.mask_bh == 1, 128, p.q_block, p.nQ, 1, p.k_block / 32};
   p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, 128 * kHeadDim * 4, p.tiled ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
+  group_parts(p.split, p.Hq / p.Hkv * (p.Sq / 128), 2LL * p.Skv * kRowBytes);
 }
 
 hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {

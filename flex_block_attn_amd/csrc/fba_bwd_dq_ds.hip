@@ -45,10 +45,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
   int item, part = 0, parts = 1;
-  if ((int)blockIdx.x < p.split.main_wgs) {
+  int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
+  if (ws_slot < 0) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position<kWaves == 4 ? Look::kSingle : Look::kNever>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<kWaves == 4 ? Look::kSingle : Look::kNever>(p.split, ws_slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / TQ;
@@ -200,7 +201,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
 
   const float poison = dense ? 1.f : poison_unless_fit(p);
   if (parts > 1) {  // part of a split item: unscaled fp32 partial sums go to the workspace
-    float* prow = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
+    float* prow = p.split.ws + (int64_t)ws_slot * (TQ * kHeadDim) + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -258,10 +259,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int item, part = 0, parts = 1;
-  if ((int)blockIdx.x < p.split.main_wgs) {
+  int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
+  if (ws_slot < 0) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, ws_slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / 128, n_kt = p.Skv / 128;
@@ -424,7 +426,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   __syncthreads();
   const float poison = dense ? 1.f : poison_unless_fit(p);
   if (parts > 1) {  // part of a split item: unscaled fp32 partial sums go to the workspace
-    float* prow = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (128 * kHeadDim) + (wave * 32 + l32) * kHeadDim;
+    float* prow = p.split.ws + (int64_t)ws_slot * (128 * kHeadDim) + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
@@ -554,6 +556,7 @@ int plan_bwd_dq_from_ds(BwdParams& p) {
   const ListLengths lengths{waves == 4 ? p.q_cnt : nullptr, p.mask_bh == 1, tile, p.q_block, p.nQ, 1, p.k_block / kSlab};
   p.split = plan_split(p.num_items, waves == 4 ? 2 : 1, p.Skv / 32, StepCost{10, 14, 18, /*scans=*/false, /*own_pace=*/false}, (int64_t)tile * kHeadDim * 4, p.split.ws,
                        p.split_ws_bytes, lengths);
+  group_parts(p.split, p.Hq / p.Hkv * (p.Sq / tile), (int64_t)p.Skv * kRowBytes);
   return waves;
 }
 

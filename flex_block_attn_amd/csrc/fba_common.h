@@ -180,9 +180,30 @@ FBA_DEVICE int split_parts(const Plan& plan) {
   for (const float more : l.more) parts += cut >= more;
   return parts;
 }
-// Work-group s of those that do the parts.  The parts of an item follow each other, so that with 2, 4 or 8 of them an XCD (work-groups
-// are dealt to the eight round-robin) does the same range of all lists and has it in its L2.  (Part by part instead, so that an XCD
-// does all ranges: forward, H3 2304 rows against 61440 keys 120 -> 140 us.)  False: the launch has more work-groups than parts.
+// Work-group s of those that do the parts; s becomes the place of its results.  False: the launch has more work-groups than parts.
+//
+// Work-groups are dealt to the XCDs round-robin.  Where the parts of an item follow each other, an XCD does the same range of all lists if there are 2, 4 or
+// 8 parts and all ranges if not, of all heads either way.  Where that is more than its L2 holds (group_parts in fba_split.hip) an XCD gets an eighth of the
+// parts in the order (items that read the same keys, part, item), so that it does few ranges of few heads.
+template <Look kLook, typename Plan>
+FBA_DEVICE bool split_position(const Plan& plan, int& s, int& item, int& part, int& parts) {
+  parts = split_parts<kLook>(plan);
+  if (kLook != Look::kNever && s == 0 && threadIdx.x == 0 && plan.look.cnt != nullptr) *plan.note = parts;
+  int i = s / parts;
+  if (i >= plan.items) return false;
+  part = s - i * parts;
+  if ((plan.grouped >> parts & 1) != 0) {
+    const int n = plan.items * parts, xcd = s % kNumXcd, at = xcd * (n / kNumXcd) + min(xcd, n % kNumXcd) + s / kNumXcd;
+    const int group = at / (plan.share * parts), in_group = at - group * (plan.share * parts);
+    const int of = min(plan.share, plan.items - group * plan.share);  // items of the group
+    part = in_group / of;
+    i = group * plan.share + in_group - part * of;
+    s = i * parts + part;
+  }
+  item = plan.first + i;
+  return true;
+}
+// dK/dV: parts in turn, of items that may be taken in an order of their own.
 template <Look kLook, typename Plan>
 FBA_DEVICE bool split_position(const Plan& plan, const int32_t* order, int s, int& item, int& part, int& parts) {
   parts = split_parts<kLook>(plan);

@@ -132,10 +132,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
   int item, part = 0, parts = 1;
-  if ((int)blockIdx.x < p.split.main_wgs) {
+  int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
+  if (ws_slot < 0) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, ws_slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / TQ;
@@ -299,7 +300,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   const float l = sum_halves(st.l_run);
   if (parts > 1) {
     // part of a split item: unnormalised O^T, the softmax reference in log2 units and the denominator go to the workspace
-    float* slot = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (kFwdSlotBytes / 4);
+    float* slot = p.split.ws + (int64_t)ws_slot * (kFwdSlotBytes / 4);
     float* prow = slot + (wave * 32 + l32) * kHeadDim;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb)
@@ -410,10 +411,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = wave & 1, par = wave >> 1;  // row group, 32-key slab of a chunk
   int item, part = 0, parts = 1;
-  if ((int)blockIdx.x < p.split.main_wgs) {
+  int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
+  if (ws_slot < 0) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, ws_slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / kHalfRows;
@@ -606,7 +608,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   // 4.85 -> 4.70 ms; B2 H8/2 S3136, 16 x 64 blocks, 12 of 49 kept 82.0 -> 79.5 us.)
   char* const own = smem + other * kSlabBytes;
   if (parts > 1) {  // as in fwd_kernel; rows of 256 bytes, 16-byte chunk c of row r at slot c ^ r % 16
-    float* slot = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (kHalfSlotBytes / 4);
+    float* slot = p.split.ws + (int64_t)ws_slot * (kHalfSlotBytes / 4);
     float* prow = slot + rg * 32 * kHeadDim + 32 * keep;
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
@@ -692,10 +694,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kRowsWaves, 64 * kRow
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int item, part = 0, parts = 1;
-  if ((int)blockIdx.x < p.split.main_wgs) {
+  int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
+  if (ws_slot < 0) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position<Look::kSingle>(p.split, nullptr, blockIdx.x - p.split.main_wgs, item, part, parts)) {
+  } else if (!split_position<Look::kSingle>(p.split, ws_slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / kRowsTile;
@@ -873,7 +876,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kRowsWaves, 64 * kRow
   l_run += __shfl_xor(l_run, 16);
   const float l = sum_halves(l_run);
   if (parts > 1) {  // as in fwd_kernel
-    float* slot = p.split.ws + (int64_t)((int)blockIdx.x - p.split.main_wgs) * (kFwdSlotBytes / 4);
+    float* slot = p.split.ws + (int64_t)ws_slot * (kFwdSlotBytes / 4);
     float* prow = slot + (wave * kRowsOf + l16) * kHeadDim + 4 * g;
 #pragma unroll
     for (int db = 0; db < 8; ++db) *reinterpret_cast<f32x4*>(prow + 16 * db) = acc[db];
@@ -1116,12 +1119,14 @@ void plan_fwd(FwdParams& p) {
     p.num_items = p.B * p.Hq * (p.Sq / kRowsTile);
     const ListLengths lengths{p.q_cnt, p.mask_bh == 1, kRowsTile, 128, p.Sq / 128, 1, p.k_block / 64};
     p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{22, 30, 40}, kFwdSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
+    group_parts(p.split, p.Hq / p.Hkv * (p.Sq / kRowsTile), 2LL * p.Skv * kRowBytes);
     return;
   }
   if (p.tiled) {  // a step is as long as one of fwd_kernel, a part's results are half as large
     p.num_items = p.B * p.Hq * (p.Sq / kHalfRows);
     const ListLengths lengths{p.q_cnt, p.mask_bh == 1, kHalfRows, 128, p.Sq / 128, 1, p.k_block / 64};  // of the 128-row tile's list
     p.split = plan_split(p.num_items, 2, p.Skv / 64, StepCost{32, 45, 60, /*scans=*/true}, kHalfSlotBytes, p.split.ws, p.split_ws_bytes, lengths);
+    group_parts(p.split, p.Hq / p.Hkv * (p.Sq / kHalfRows), 2LL * p.Skv * kRowBytes);
     return;
   }
   const bool wide = p.q_block % 384 == 0 && p.variant != 1;
@@ -1129,6 +1134,7 @@ void plan_fwd(FwdParams& p) {
   p.num_items = p.B * p.Hq * (p.Sq / rows);
   const ListLengths lengths{p.q_cnt, p.mask_bh == 1, rows, p.q_block, p.nQ, 1, p.k_block / kSlab};
   p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
+  group_parts(p.split, p.Hq / p.Hkv * (p.Sq / rows), 2LL * p.Skv * kRowBytes);
 }
 
 namespace {

@@ -52,6 +52,8 @@ struct SplitPlan {
   int parts;      // work-groups per split item, at most (>= 2 when ws is set)
   int main_wgs;   // work-groups in front of the split ones (a multiple of the XCD count)
   int items;      // that are split
+  int share;      // consecutive items that read the same keys and values
+  uint32_t grouped;  // bit n: n parts are dealt to the XCDs by what they read (split_position)
   ListLook look;
   int32_t* note;  // behind the parts' results: how many parts the kernel made, for the merge
 };
@@ -69,6 +71,9 @@ struct StepCost {
 // of an item.  main_wgs is left to the launcher.
 SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
                      const ListLengths& lengths);
+
+// Sets share and grouped: `tiles` consecutive items read the same `bytes`.
+void group_parts(SplitPlan& plan, int tiles, int64_t bytes);
 
 // The plans of the launches below, from the sizes, q_cnt / k_cnt, split.ws and split_ws_bytes of their parameters: num_items and split are set.
 struct FwdParams;

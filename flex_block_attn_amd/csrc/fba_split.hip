@@ -151,6 +151,21 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   return plan;
 }
 
+// Forward and dQ launches of less than a round.  With parts that follow each other an XCD reads 1 / gcd(parts, 8) of what all items read; more than its L2
+// holds (4 MiB) comes from the memory-side cache as often as there are items that select it, which bounds such launches: 144 tiles of 24 heads on 6 kv heads of
+// 30720 keys in three parts copy 0.9 GB.  Parts in turn / grouped (keys and values of one kv head in MiB x kv heads, parts): forward H24/6, 768 rows against
+// 30720 keys (15 x 6, three) 144 / 129 us, H4 2304 against 46080 (22 x 4, three) 152 / 130, H24 1280 against 20480 (10 x 24, two) 147 / 139, H12 the same (10 x 12,
+// four) 100.6 / 96.3; steps H12 1536 against 15360 380 / 349, H8 768 against 7680 (3.75 x 8, three) 150 / 138.  Where an L2 holds it, the work-groups of an XCD
+// then all wait for the same few lines: steps H4 S3840 (1.9 x 4, four parts) 114.0 / 116.9, H2 S6144 140.6 / 143.4.  Behind a whole round: H12 S3456 155.4 / 156.8.
+void group_parts(SplitPlan& plan, int tiles, int64_t bytes) {
+  constexpr int64_t kL2Bytes = 4 << 20;
+  if (plan.ws == nullptr || plan.first > 0) return;
+  plan.share = tiles;
+  const int64_t all = (plan.items + tiles - 1) / tiles * bytes;
+  for (int n = 2; n <= plan.parts; ++n)
+    if (all > kL2Bytes * (n % 8 == 0 ? 8 : n % 4 == 0 ? 4 : n % 2 == 0 ? 2 : 1)) plan.grouped |= 1u << n;
+}
+
 namespace {
 
 constexpr int kQueueBytes = 256;
