@@ -59,12 +59,12 @@ int check_ptrs(std::initializer_list<std::pair<const char*, const void*>> ps) {
 // faster than the one with 32 keys per wave (two waves per SIMD) without the dS hand-over and about 7 % faster with it
 // (a wave alone on its SIMD pays for every cycle its dS stores take to issue).  Both do the same arithmetic in the same
 // order.  FBA_DKDV_KEYS_PER_WAVE = 32 or 64 overrides the choice (measurement of the two).
-hipError_t launch_dkdv_variant(fba::BwdParams& p, hipStream_t stream) {
+hipError_t launch_dkdv_variant(fba::BwdParams& p, hipStream_t stream, fba::Merge* later) {
   const char* env = getenv("FBA_DKDV_KEYS_PER_WAVE");
   const int keys = env ? atoi(env) : 64;
-  if (p.tiled) return fba::launch_bwd_dkdv_slab(p, stream);
-  if (keys == 64) return fba::launch_bwd_dkdv64(p, stream);
-  return fba::launch_bwd_dkdv(p, stream);
+  if (p.tiled) return fba::launch_bwd_dkdv_slab(p, stream, later);
+  if (keys == 64) return fba::launch_bwd_dkdv64(p, stream, later);
+  return fba::launch_bwd_dkdv(p, stream, later);
 }
 
 int hip_fail(hipError_t e, const char* what) { return fail(FBA_ERR_HIP, "%s: %s", what, hipGetErrorString(e)); }
@@ -395,7 +395,7 @@ int32_t fba_bwd_stats(const void* o, const void* d_o, const float* lse, float* s
 static int dq_impl(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dq,
                    const int32_t* q_cnt, const int32_t* q_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv,
                    int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
-                   void* hip_stream, bool tiled) {
+                   void* hip_stream, bool tiled, const fba::Merge& before) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"d_o", d_o}, {"dq", dq}})) return rc;
@@ -408,14 +408,14 @@ static int dq_impl(const void* q, const void* k, const void* v, const void* d_o,
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
   p.stats = stats; p.dq = (__bf16*)dq; p.q_cnt = q_cnt; p.q_idx = q_idx;
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = fba::launch_bwd_dq(p, (hipStream_t)hip_stream);
+  hipError_t e = fba::launch_bwd_dq(p, (hipStream_t)hip_stream, before);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dq launch");
 }
 
 static int dkdv_impl(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dk, void* dv,
                      const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv,
                      int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
-                     void* hip_stream, bool tiled, const fba::BwdStats& make) {
+                     void* hip_stream, bool tiled, const fba::BwdStats& make, fba::Merge* later) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"d_o", d_o}, {"dk", dk}, {"dv", dv}})) return rc;
@@ -429,7 +429,7 @@ static int dkdv_impl(const void* q, const void* k, const void* v, const void* d_
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.d_o = (const __bf16*)d_o;
   p.stats = stats; p.make = make; p.dk = (__bf16*)dk; p.dv = (__bf16*)dv; p.k_cnt = k_cnt; p.k_idx = k_idx;
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream);
+  hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream, later);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dkdv launch");
 }
 
@@ -446,11 +446,12 @@ static int bwd_impl(const void* q, const void* k, const void* v, const void* o, 
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}})) return rc;
   if (!lse || !stats || !q_cnt || !q_idx || !k_cnt || !k_idx) return fail(FBA_ERR_INVALID, "null pointer argument");
   if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
+  fba::Merge merge;
   if (int rc = dkdv_impl(q, k, v, d_o, stats, dk, dv, k_cnt, k_idx, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block,
-                         split_ws, split_ws_bytes, hip_stream, tiled, {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq}))
+                         split_ws, split_ws_bytes, hip_stream, tiled, {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq}, &merge))
     return rc;
   return dq_impl(q, k, v, d_o, stats, dq, q_cnt, q_idx, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes,
-                 hip_stream, tiled);
+                 hip_stream, tiled, merge);
 }
 
 int32_t fba_bwd_dq(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dq,
@@ -458,7 +459,7 @@ int32_t fba_bwd_dq(const void* q, const void* k, const void* v, const void* d_o,
                    int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
                    void* hip_stream) {
   return dq_impl(q, k, v, d_o, stats, dq, q_cnt, q_idx, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes,
-                 hip_stream, false);
+                 hip_stream, false, {});
 }
 
 int32_t fba_bwd_dkdv(const void* q, const void* k, const void* v, const void* d_o, const float* stats, void* dk, void* dv,
@@ -466,7 +467,7 @@ int32_t fba_bwd_dkdv(const void* q, const void* k, const void* v, const void* d_
                      int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
                      void* hip_stream) {
   return dkdv_impl(q, k, v, d_o, stats, dk, dv, k_cnt, k_idx, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws,
-                   split_ws_bytes, hip_stream, false, {});
+                   split_ws_bytes, hip_stream, false, {}, nullptr);
 }
 
 int32_t fba_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
@@ -526,7 +527,7 @@ static int dkdv_handover_impl(const void* q, const void* k, const void* v, const
                               void* ds_ws, int64_t ds_ws_bytes, const int32_t* k_cnt, const int32_t* k_idx, const int32_t* pair_base,
                               int64_t n_pairs, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv,
                               int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
-                              void* hip_stream, const fba::BwdStats& make) {
+                              void* hip_stream, const fba::BwdStats& make, fba::Merge* later) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_handover(s, ds_ws, ds_ws_bytes, pair_base, n_pairs, "dkdv")) return rc;
@@ -541,7 +542,7 @@ static int dkdv_handover_impl(const void* q, const void* k, const void* v, const
   p.ds_ws = (__bf16*)ds_ws; p.pair_base = pair_base;
   p.ws_pairs = ds_ws_bytes / ((int64_t)q_block * k_block * 2);
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream);
+  hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream, later);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dkdv (hand-over) launch");
 }
 
@@ -551,13 +552,13 @@ int32_t fba_bwd_dkdv_handover(const void* q, const void* k, const void* v, const
                               int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
                               void* hip_stream) {
   return dkdv_handover_impl(q, k, v, d_o, stats, dk, dv, ds_ws, ds_ws_bytes, k_cnt, k_idx, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim,
-                            q_block, k_block, split_ws, split_ws_bytes, hip_stream, {});
+                            q_block, k_block, split_ws, split_ws_bytes, hip_stream, {}, nullptr);
 }
 
-int32_t fba_bwd_dq_from_ds(const void* k, const void* ds_ws, int64_t ds_ws_bytes, void* dq, const int32_t* q_cnt, const int32_t* q_idx,
+static int dq_from_ds_impl(const void* k, const void* ds_ws, int64_t ds_ws_bytes, void* dq, const int32_t* q_cnt, const int32_t* q_idx,
                            const int32_t* q_slot, const int32_t* pair_base, int64_t n_pairs, int64_t mask_bh, int32_t B, int32_t Hq,
                            int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws,
-                           int64_t split_ws_bytes, void* hip_stream) {
+                           int64_t split_ws_bytes, void* hip_stream, const fba::Merge& before) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_handover(s, ds_ws, ds_ws_bytes, pair_base, n_pairs, "dq")) return rc;
@@ -570,8 +571,16 @@ int32_t fba_bwd_dq_from_ds(const void* k, const void* ds_ws, int64_t ds_ws_bytes
   p.ds_ws = (__bf16*)const_cast<void*>(ds_ws); p.pair_base = pair_base; p.q_slot = q_slot;
   p.ws_pairs = ds_ws_bytes / ((int64_t)q_block * k_block * 2);
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream);
+  hipError_t e = fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream, before);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (from dS) launch");
+}
+
+int32_t fba_bwd_dq_from_ds(const void* k, const void* ds_ws, int64_t ds_ws_bytes, void* dq, const int32_t* q_cnt, const int32_t* q_idx,
+                           const int32_t* q_slot, const int32_t* pair_base, int64_t n_pairs, int64_t mask_bh, int32_t B, int32_t Hq,
+                           int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws,
+                           int64_t split_ws_bytes, void* hip_stream) {
+  return dq_from_ds_impl(k, ds_ws, ds_ws_bytes, dq, q_cnt, q_idx, q_slot, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws,
+                         split_ws_bytes, hip_stream, {});
 }
 
 int32_t fba_bwd_handover(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse, float* stats,
@@ -587,11 +596,12 @@ int32_t fba_bwd_handover(const void* q, const void* k, const void* v, const void
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}, {"d_o", d_o}, {"dq", dq}, {"dk", dk}, {"dv", dv}})) return rc;
   if (!lse || !stats || !q_cnt || !q_idx || !k_cnt || !k_idx || !q_slot) return fail(FBA_ERR_INVALID, "null pointer argument");
   if ((int64_t)B * Hq * Sq >= (1LL << 30)) return fail(FBA_ERR_INVALID, "B*Hq*Sq must be below 2^30");
+  fba::Merge merge;
   if (int rc = dkdv_handover_impl(q, k, v, d_o, stats, dk, dv, ds_ws, ds_ws_bytes, k_cnt, k_idx, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim,
-                                  q_block, k_block, split_ws, split_ws_bytes, hip_stream, {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq}))
+                                  q_block, k_block, split_ws, split_ws_bytes, hip_stream, {(const __bf16*)o, (const __bf16*)d_o, lse, stats, (int64_t)B * Hq * Sq}, &merge))
     return rc;
-  return fba_bwd_dq_from_ds(k, ds_ws, ds_ws_bytes, dq, q_cnt, q_idx, q_slot, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim,
-                            q_block, k_block, split_ws, split_ws_bytes, hip_stream);
+  return dq_from_ds_impl(k, ds_ws, ds_ws_bytes, dq, q_cnt, q_idx, q_slot, pair_base, n_pairs, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim,
+                         q_block, k_block, split_ws, split_ws_bytes, hip_stream, merge);
 }
 
 int32_t fba_tile_slots_bounds(const int32_t* kt_cnt, const int32_t* kt_ent, int64_t mask_bh, int32_t n_qt, int32_t n_kt, int32_t* pair_base,
@@ -649,9 +659,10 @@ static int bwd_tiled_impl(const void* q, const void* k, const void* v, const voi
     p.ws_pairs = ds_ws_bytes / (128 * 128 * 2);
   }
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = fba::launch_bwd_dkdv_slab(p, (hipStream_t)hip_stream);
+  fba::Merge merge;
+  hipError_t e = fba::launch_bwd_dkdv_slab(p, (hipStream_t)hip_stream, &merge);
   if (e != hipSuccess) return hip_fail(e, "dkdv (tile lists) launch");
-  e = ds_ws != nullptr ? fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream) : fba::launch_bwd_dq(p, (hipStream_t)hip_stream);
+  e = ds_ws != nullptr ? fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream, merge) : fba::launch_bwd_dq(p, (hipStream_t)hip_stream, merge);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (tile lists) launch");
 }
 
@@ -791,9 +802,10 @@ int32_t fba_bwd_dense(const void* q, const void* k, const void* v, const void* o
   p.q_cnt = q_cnt; p.q_idx = q_idx; p.k_cnt = k_cnt; p.k_idx = k_idx;
   p.ds_ws = (__bf16*)ds_ws;  // pair_base stays null: dense numbering
   p.split.ws = (float*)split_ws; p.split_ws_bytes = split_ws_bytes;
-  hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream);
+  fba::Merge merge;
+  hipError_t e = launch_dkdv_variant(p, (hipStream_t)hip_stream, &merge);
   if (e != hipSuccess) return hip_fail(e, "dkdv (dense hand-over) launch");
-  e = fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream);
+  e = fba::launch_bwd_dq_from_ds(p, (hipStream_t)hip_stream, merge);
   return e == hipSuccess ? FBA_OK : hip_fail(e, "dq (from dS, dense) launch");
 }
 

@@ -376,7 +376,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     }
 }
 
-hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream) {
+hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream, Merge* later) {
   const bool hand_over = p.ds_ws != nullptr;
   void (*fn)(const BwdParams) = hand_over ? &dkdv_kernel<true> : &dkdv_kernel<false>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
@@ -384,11 +384,13 @@ hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream) {
   int grid;
   if ((e = plan_key_tiles(p, kKeyTiles128, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes + 16, stream, p);
-  const int split_items = p.num_items - p.split.first;
-  if (split_items > 0) {
+  if (p.num_items > p.split.first || p.pieces.header != nullptr) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
-    e = launch_partial_sum(p.split, 2 * 128 * kHeadDim, 128, outs, 2, p.order, stream);
-    if (e != hipSuccess) return e;
+    Merge m = merge_of(p.split, 2 * 128 * kHeadDim, 128, outs, 2, p.order, p.pieces);
+    m.results_end = p.results_end;
+    m.kept_from = p.kept_from;
+    if (later == nullptr) return launch_merge(m, stream);
+    *later = m;
   }
   return hipGetLastError();
 }

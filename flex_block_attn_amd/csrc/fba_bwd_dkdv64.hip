@@ -663,18 +663,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   else finish(acc_v, acc_k, p.dv, poison);
 }
 
-hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream) {
+hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream, Merge* later) {
   void (*fn)(const BwdParams) = p.ds_ws == nullptr ? &dkdv64_kernel<kRecompute> : p.pair_base == nullptr ? &dkdv64_kernel<kDense> : &dkdv64_kernel<kNumbered>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmemBytes + 16);
   if (e != hipSuccess) return e;
   int grid;
   if ((e = plan_key_tiles(p, kKeyTiles128, grid, stream, /*takes_pieces=*/true)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(256), kSmemBytes + 16, stream, p);
-  const int split_items = p.num_items - p.split.first;
-  if (split_items > 0 || p.pieces.header != nullptr) {
+  if (p.num_items > p.split.first || p.pieces.header != nullptr) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0}, {p.dk, p.scale, 128 * kHeadDim}};
-    e = launch_partial_sum(p.split, 2 * 128 * kHeadDim, 128, outs, 2, p.order, stream, p.pieces);
-    if (e != hipSuccess) return e;
+    Merge m = merge_of(p.split, 2 * 128 * kHeadDim, 128, outs, 2, p.order, p.pieces);
+    m.results_end = p.results_end;
+    m.kept_from = p.kept_from;
+    if (later == nullptr) return launch_merge(m, stream);
+    *later = m;
   }
   return hipGetLastError();
 }

@@ -417,7 +417,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   finish(acc_k, 1, p.dk, parts > 1 ? poison : p.scale * poison);
 }
 
-hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
+hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream, Merge* later) {
   const bool hand_over = p.ds_ws != nullptr, halves = p.q_block % 32 != 0;
   void (*fn)(const BwdParams) = hand_over ? (halves ? &dkdv_slab_kernel<true, true> : &dkdv_slab_kernel<true, false>)
                                           : (halves ? &dkdv_slab_kernel<false, true> : &dkdv_slab_kernel<false, false>);
@@ -426,10 +426,13 @@ hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream) {
   int grid;
   if ((e = plan_key_tiles(p, kKeyTiles64, grid, stream)) != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(grid), dim3(512), kSmemBytes, stream, p);
-  const int split_items = p.num_items - p.split.first;
-  if (split_items > 0) {
+  if (p.num_items > p.split.first || p.pieces.header != nullptr) {
     const PartialOut outs[2] = {{p.dv, 1.f, 0, p.Skv, p.out_kv}, {p.dk, p.scale, kTK * kHeadDim, p.Skv, p.out_kv}};
-    return launch_partial_sum(p.split, kSlotFloats, kTK, outs, 2, p.order, stream);
+    Merge m = merge_of(p.split, kSlotFloats, kTK, outs, 2, p.order, p.pieces);
+    m.results_end = p.results_end;
+    m.kept_from = p.kept_from;
+    if (later == nullptr) return launch_merge(m, stream);
+    *later = m;
   }
   return hipGetLastError();
 }

@@ -34,9 +34,11 @@ using IC = std::integral_constant<int, N>;
 
 // kTiled: see the forward kernel (tile lists with a predicate per 16-row group instead of block lists).
 template <bool kTiled>
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void dq_kernel(const BwdParams p) {
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void dq_kernel(const BwdParams p, const Merge before) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // ring [4] of (K slab | V slab)
   constexpr int TQ = 128;
+  const int own_wgs = (int)gridDim.x - before.wgs;
+  if ((int)blockIdx.x >= own_wgs) return merge_parts<256>(before, (int)blockIdx.x - own_wgs, before.wgs);
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -248,18 +250,18 @@ void plan_bwd_dq(BwdParams& p) {
   group_parts(p.split, p.Hq / p.Hkv * (p.Sq / 128), 2LL * p.Skv * kRowBytes);
 }
 
-hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream) {
+hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream, Merge before) {
   constexpr int kSmem = kRing * kPairBytes;
   plan_bwd_dq(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
-  void (*fn)(const BwdParams) = p.tiled ? &dq_kernel<true> : &dq_kernel<false>;
+  void (*fn)(const BwdParams, const Merge) = p.tiled ? &dq_kernel<true> : &dq_kernel<false>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kSmem, stream, p);
+  if (e != hipSuccess || (e = take_along(p.split, 128 * kHeadDim * 4, before, stream)) != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts + before.wgs), dim3(256), kSmem, stream, p, before);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0};
-    return launch_partial_sum(p.split, 128 * kHeadDim, 128, &out, 1, nullptr, stream);
+    return launch_merge(merge_of(p.split, 128 * kHeadDim, 128, &out, 1, nullptr, {}), stream);
   }
   return hipGetLastError();
 }

@@ -36,10 +36,12 @@ using IC = std::integral_constant<int, N>;
 
 template <int kMode, int kWaves>  // kMode: kNumbered or kDense
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(kWaves == 12 ? 3 : 2, kWaves == 12 ? 3 : 2))) void dq_from_ds_kernel(
-    const BwdParams p) {
+    const BwdParams p, const Merge before) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // ring [4] of (K slab | dS units)
   constexpr int TQ = 32 * kWaves;
   constexpr int kStageBytes = stage_bytes(kWaves);
+  const int own_wgs = (int)gridDim.x - before.wgs;
+  if ((int)blockIdx.x >= own_wgs) return merge_parts<64 * kWaves>(before, (int)blockIdx.x - own_wgs, before.wgs);
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -253,8 +255,10 @@ struct TileChunks {
 }  // namespace
 
 template <int kMode>  // kNumbered or kDense
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void dq_tiles_kernel(const BwdParams p) {
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void dq_tiles_kernel(const BwdParams p, const Merge before) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // K chunks [2] | dS [wave][kAhead]
+  const int own_wgs = (int)gridDim.x - before.wgs;
+  if ((int)blockIdx.x >= own_wgs) return merge_parts<256>(before, (int)blockIdx.x - own_wgs, before.wgs);
   constexpr bool dense = kMode == kDense;
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -465,73 +469,40 @@ hipError_t zero_unit_address(const char** out) {
 
 }  // namespace
 
-// Sums the fp32 partial rows of the split items in part order: out = scale * sum_p partial_p, as bf16.  One thread per four
-// columns; an item has `rows` rows of 128 columns; blockIdx.y picks the output (dK/dV: two per slot, one launch for both).  All parts are
-// requested at once, as in fwd_merge_kernel.
-struct PartialOuts {
-  PartialOut out[2];
-};
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void partial_sum_kernel(const SplitPlan split, int64_t slot_floats, int rows, PartialOuts outs,
-                                                                                          const int32_t* order, const Pieces pieces) {
-  const int tid = threadIdx.x;
-  const PartialOut& o = outs.out[blockIdx.y];
-  const int c4 = (tid & 31) * 4;
-  if (pieces.header != nullptr && const_idx(pieces.header)[0] > 0) {  // items cut each by its own length
-    const int n_rows = const_idx(pieces.header)[1] * rows;
-    for (int row = blockIdx.x * 8 + (tid >> 5); row < n_rows; row += gridDim.x * 8) {
-      const int it = row / rows, r = row - it * rows;
-      const CutItem cut = pieces.cut[it];
-      const float* src = split.ws + cut.slot * slot_floats + o.offset + r * kHeadDim + c4;
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      for (int q = 0; q < cut.pieces; q += kMostParts) {
-        f32x4 of[kMostParts];
-#pragma unroll
-        for (int i = 0; i < kMostParts; ++i)
-          if (q + i < cut.pieces) of[i] = *reinterpret_cast<const f32x4*>(src + (q + i) * slot_floats);
-#pragma unroll
-        for (int i = 0; i < kMostParts; ++i)
-          if (q + i < cut.pieces) acc += of[i];
-      }
-      *reinterpret_cast<bf16x4*>(o.out + ((int64_t)cut.item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
-    }
-    return;
-  }
-  if (split.items == 0) return;  // the host has planned no parts
-  const int parts = parts_made(split);
-  if (parts == 1) return;  // done whole
-  for (int block = blockIdx.x; block < split.items * (rows / 8); block += gridDim.x) {
-    const int row = block * 8 + (tid >> 5);  // among the rows of all split items
-    const int it = row / rows, r = row - it * rows;
-    const float* src = split.ws + (int64_t)it * parts * slot_floats + o.offset + r * kHeadDim + c4;
-    f32x4 of[kMostParts];
-#pragma unroll
-    for (int q = 0; q < kMostParts; ++q)
-      if (q < parts) {
-        of[q] = *reinterpret_cast<const f32x4*>(src);
-        src += slot_floats;
-      }
-    const int64_t item = order != nullptr ? order[split.first + it] : split.first + it;
-    int64_t out_row = item * rows + r;
-    if (o.head_rows != o.out_rows) {
-      const int64_t head = out_row / o.head_rows;
-      const int at = (int)(out_row - head * o.head_rows);
-      if (at >= o.out_rows) continue;
-      out_row = head * o.out_rows + at;
-    }
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int q = 0; q < kMostParts; ++q)
-      if (q < parts) acc += of[q];
-    *reinterpret_cast<bf16x4*>(o.out + out_row * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
-  }
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void merge_kernel(const Merge m) { merge_parts<256>(m, blockIdx.x, gridDim.x); }
+
+Merge merge_of(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order, const Pieces& pieces) {
+  Merge m;
+  m.ws = split.ws;
+  m.note = split.look.cnt == nullptr ? nullptr : split.note;
+  m.first = split.first; m.items = split.items; m.parts = split.parts;
+  m.rows = rows; m.slot_floats = slot_floats;
+  m.n_outs = n_outs;
+  for (int i = 0; i < n_outs; ++i) m.out[i] = outs[i];
+  m.order = order; m.pieces = pieces;
+  m.wgs = std::max(merge_grid(split.items * (rows / 8)), pieces.header != nullptr ? 128 : 0) * n_outs;
+  return m;
 }
 
-hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order,
-                              hipStream_t stream, const Pieces& pieces) {
-  PartialOuts o{{outs[0], outs[n_outs - 1]}};
-  const int grid = std::max(merge_grid(split.items * (rows / 8)), pieces.header != nullptr ? 128 : 0);
-  hipLaunchKernelGGL(partial_sum_kernel, dim3(grid, n_outs), dim3(256), 0, stream, split, slot_floats, rows, o, order, pieces);
+hipError_t launch_merge(const Merge& m, hipStream_t stream) {
+  if (m.wgs > 0) hipLaunchKernelGGL(merge_kernel, dim3(m.wgs), dim3(256), 0, stream, m);
   return hipGetLastError();
+}
+
+hipError_t take_along(SplitPlan& split, int64_t slot_bytes, Merge& before, hipStream_t stream) {
+  if (before.wgs == 0) return hipSuccess;
+  if (split.items > 0) {
+    const int64_t end = before.results_end + split.items * split.parts * slot_bytes + (int64_t)sizeof(int32_t);
+    if (end > before.kept_from) {
+      const hipError_t e = launch_merge(before, stream);
+      before = {};
+      return e;
+    }
+    split.ws += before.results_end / 4;
+    split.note += before.results_end / 4;
+  }
+  before.wgs = std::min(before.wgs, 128 * before.n_outs);  // a work-group or so to a compute unit, while others work on dQ
+  return hipSuccess;
 }
 
 // Tail splitting on block lists (two work-groups of four waves per compute unit, one of more); a part stores a tile of fp32 sums.
@@ -563,45 +534,45 @@ int plan_bwd_dq_from_ds(BwdParams& p) {
 namespace {
 
 template <int kWaves>
-hipError_t launch_dq_rows(BwdParams p, hipStream_t stream) {
+hipError_t launch_dq_rows(BwdParams p, hipStream_t stream, Merge before) {
   constexpr int kRows = 32 * kWaves, kSmem = kRing * stage_bytes(kWaves);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   const bool dense = p.pair_base == nullptr;
-  void (*fn)(const BwdParams) = dense ? &dq_from_ds_kernel<kDense, kWaves> : &dq_from_ds_kernel<kNumbered, kWaves>;
+  void (*fn)(const BwdParams, const Merge) = dense ? &dq_from_ds_kernel<kDense, kWaves> : &dq_from_ds_kernel<kNumbered, kWaves>;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kSmem);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(64 * kWaves), kSmem, stream, p);
+  if (e != hipSuccess || (e = take_along(p.split, kRows * kHeadDim * 4, before, stream)) != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts + before.wgs), dim3(64 * kWaves), kSmem, stream, p, before);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0};
-    e = launch_partial_sum(p.split, kRows * kHeadDim, kRows, &out, 1, nullptr, stream);
-    if (e != hipSuccess) return e;
+    return launch_merge(merge_of(p.split, kRows * kHeadDim, kRows, &out, 1, nullptr, {}), stream);
   }
   return hipGetLastError();
 }
 
-hipError_t launch_dq_tiles(BwdParams p, hipStream_t stream) {
+hipError_t launch_dq_tiles(BwdParams p, hipStream_t stream, Merge before) {
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_items = p.num_items - p.split.first;
   hipError_t e = zero_unit_address(&p.zero_unit);
   if (e != hipSuccess) return e;
-  void (*fn)(const BwdParams) = p.pair_base == nullptr ? &dq_tiles_kernel<kDense> : &dq_tiles_kernel<kNumbered>;
+  void (*fn)(const BwdParams, const Merge) = p.pair_base == nullptr ? &dq_tiles_kernel<kDense> : &dq_tiles_kernel<kNumbered>;
   if ((e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, kTilesSmem)) != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts), dim3(256), kTilesSmem, stream, p);
+  if ((e = take_along(p.split, 128 * kHeadDim * 4, before, stream)) != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_items * p.split.parts + before.wgs), dim3(256), kTilesSmem, stream, p, before);
   if (split_items > 0) {
     const PartialOut out{p.dq, p.scale, 0, p.Sq, p.out_q};
-    return launch_partial_sum(p.split, 128 * kHeadDim, 128, &out, 1, nullptr, stream);
+    return launch_merge(merge_of(p.split, 128 * kHeadDim, 128, &out, 1, nullptr, {}), stream);
   }
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream) {
+hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream, Merge before) {
   if (p.ds_ws == nullptr) return hipErrorInvalidValue;
   const int waves = plan_bwd_dq_from_ds(p);
-  if (p.tiled) return launch_dq_tiles(p, stream);
-  return waves == 12 ? launch_dq_rows<12>(p, stream) : waves == 8 ? launch_dq_rows<8>(p, stream) : launch_dq_rows<4>(p, stream);
+  if (p.tiled) return launch_dq_tiles(p, stream, before);
+  return waves == 12 ? launch_dq_rows<12>(p, stream, before) : waves == 8 ? launch_dq_rows<8>(p, stream, before) : launch_dq_rows<4>(p, stream, before);
 }
 
 }  // namespace fba

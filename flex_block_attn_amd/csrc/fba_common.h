@@ -272,9 +272,69 @@ struct TileCopy {
 typedef const FBA_CONST int32_t* ConstIdx;
 FBA_DEVICE ConstIdx const_idx(const int32_t* p) { return (ConstIdx)(uintptr_t)p; }
 
-// For the merge: how many parts the kernel in front made.  A scalar load: the merge's addresses wait for it.
+// For the merge of forward: how many parts the kernel in front made.  A scalar load: the merge's addresses wait for it.
 template <typename Plan>
 FBA_DEVICE int parts_made(const Plan& plan) { return plan.look.cnt == nullptr ? plan.parts : const_idx(plan.note)[0]; }
+
+// Sums the fp32 partial rows of split items in part order: out = scale * sum_p partial_p, as bf16.  One thread per four columns; work-group `wg` of
+// `wgs` with kThreads threads each, every n_outs-th for one of the outputs (dK/dV: two per slot).  All parts are requested at once, as in
+// fwd_merge_kernel.  M is Merge.
+constexpr int kMergeParts = 8;  // at a time
+template <int kThreads, typename M>
+FBA_DEVICE void merge_parts(const M& m, int wg, int wgs) {
+  const int tid = threadIdx.x;
+  const auto& o = m.out[wg % m.n_outs];
+  const int c4 = (tid & 31) * 4, rows = m.rows;
+  constexpr int kPer = kThreads / 32;  // rows at a time
+  const int row0 = wg / m.n_outs * kPer + (tid >> 5), row_step = wgs / m.n_outs * kPer;
+  if (m.pieces.header != nullptr && const_idx(m.pieces.header)[0] > 0) {  // items cut each by its own length
+    const int n_rows = const_idx(m.pieces.header)[1] * rows;
+    for (int row = row0; row < n_rows; row += row_step) {
+      const int it = row / rows, r = row - it * rows;
+      const auto cut = m.pieces.cut[it];
+      const float* src = m.ws + cut.slot * m.slot_floats + o.offset + r * kHeadDim + c4;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int q = 0; q < cut.pieces; q += kMergeParts) {
+        f32x4 of[kMergeParts];
+#pragma unroll
+        for (int i = 0; i < kMergeParts; ++i)
+          if (q + i < cut.pieces) of[i] = *reinterpret_cast<const f32x4*>(src + (q + i) * m.slot_floats);
+#pragma unroll
+        for (int i = 0; i < kMergeParts; ++i)
+          if (q + i < cut.pieces) acc += of[i];
+      }
+      *reinterpret_cast<bf16x4*>(o.out + ((int64_t)cut.item * rows + r) * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
+    }
+    return;
+  }
+  if (m.items == 0) return;  // the host has planned no parts
+  const int parts = m.note == nullptr ? m.parts : const_idx(m.note)[0];
+  if (parts == 1) return;  // done whole
+  for (int row = row0; row < m.items * rows; row += row_step) {  // among the rows of all split items
+    const int it = row / rows, r = row - it * rows;
+    const float* src = m.ws + (int64_t)it * parts * m.slot_floats + o.offset + r * kHeadDim + c4;
+    f32x4 of[kMergeParts];
+#pragma unroll
+    for (int q = 0; q < kMergeParts; ++q)
+      if (q < parts) {
+        of[q] = *reinterpret_cast<const f32x4*>(src);
+        src += m.slot_floats;
+      }
+    const int64_t item = m.order != nullptr ? m.order[m.first + it] : m.first + it;
+    int64_t out_row = item * rows + r;
+    if (o.head_rows != o.out_rows) {
+      const int64_t head = out_row / o.head_rows;
+      const int at = (int)(out_row - head * o.head_rows);
+      if (at >= o.out_rows) continue;
+      out_row = head * o.out_rows + at;
+    }
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < kMergeParts; ++q)
+      if (q < parts) acc += of[q];
+    *reinterpret_cast<bf16x4*>(o.out + out_row * kHeadDim + c4) = pack4(acc[0] * o.scale, acc[1] * o.scale, acc[2] * o.scale, acc[3] * o.scale);
+  }
+}
 
 // Scalar loads of what a work-group is about to read from its lists, one after the other as it finds its way: asked for together up
 // front they all are in the scalar cache by then, instead of 0.5 to 1 us for each link of the chain.

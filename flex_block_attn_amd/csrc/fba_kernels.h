@@ -72,6 +72,12 @@ struct StepCost {
 SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step, int64_t slot_bytes, void* ws, int64_t ws_bytes,
                      const ListLengths& lengths);
 
+// What a launch with the plan `split` leaves to be merged.
+struct Merge;
+struct PartialOut;
+struct Pieces;
+Merge merge_of(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order, const Pieces& pieces);
+
 // Sets share and grouped: `tiles` consecutive items read the same `bytes`.
 void group_parts(SplitPlan& plan, int tiles, int64_t bytes);
 
@@ -91,7 +97,7 @@ constexpr KeyTiles kKeyTiles128{128, 14, 2 * 128 * 128 * 4};  // block lists: dk
 constexpr KeyTiles kKeyTiles64{64, 22, 2 * 64 * 128 * 4};     // tile lists: dkdv_slab_kernel
 void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles);
 
-// Work-groups of a launch that merges parts: each does every so many of the blocks of eight rows, so that little is launched where
+// Work-groups of a launch that merges parts: each does every so many blocks of eight rows, so that little is launched where
 // the lists turn out too short for parts.
 inline int merge_grid(int blocks) { return blocks < 1024 ? blocks : 1024; }
 
@@ -196,6 +202,33 @@ struct Pieces {  // in the caller's workspace
   const CutItem* cut;
 };
 
+// One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats); rows of a head
+// that the items have and those of them that the output has (0: all).
+struct PartialOut {
+  __bf16* out;
+  float scale;
+  int64_t offset;
+  int head_rows = 0, out_rows = 0;
+};
+
+// The parts of a launch that are to be summed (merge_parts in fba_common.h).  dQ does not need dK and dV, so their merge rides in the dQ launch, as
+// work-groups behind its own: by itself it took 5 to 7 us, also where the device had made no parts.  Steps, a launch of its own / along: H12 S3072,
+// 128-token blocks, a third kept 131.1 / 126.6 us; H12 S3456 153.1 / 147.5; H2 S6144, 384-token blocks, half kept 140.4 / 138.6; H2 S7680 190.3 / 186.4; B2 H16/4
+// S8192 1020.5 / 1018.2.  (In front of dQ's work-groups instead, in launches of two rounds and more: the same.)
+struct Merge {
+  const float* ws = nullptr;
+  const int32_t* note = nullptr;  // how many parts there are; null: `parts`
+  int first = 0, items = 0, parts = 1;
+  int rows = 0;  // of an item
+  int64_t slot_floats = 0;
+  int n_outs = 0;
+  PartialOut out[2] = {};
+  const int32_t* order = nullptr;  // or the item of every grid index
+  Pieces pieces = {};
+  int wgs = 0;  // work-groups for it, a multiple of n_outs; 0: there is nothing to merge
+  int64_t results_end = 0, kept_from = 0;  // bytes of the workspace that the parts' results take, from where on it holds what the merge reads besides
+};
+
 struct BwdParams {
   const __bf16* q;
   const __bf16* k;
@@ -247,6 +280,7 @@ struct BwdParams {
   const int32_t* order;
   int64_t split_ws_bytes;  // size of split.ws as handed in by the caller
   Pieces pieces;           // dkdv64_kernel
+  int64_t results_end, kept_from;  // see Merge
   BwdStats make;           // statistics that are to be formed in front of the dK/dV kernel
 };
 
@@ -300,27 +334,22 @@ bool fwd_takes_mask(int64_t rows, int64_t kv_len);
 hipError_t launch_bwd_mask(BwdMaskParams p, hipStream_t stream);
 bool bwd_takes_mask(int64_t heads, int64_t kv_heads, int64_t q_len, int64_t kv_len);
 hipError_t launch_bwd_stats(const BwdStats& s, hipStream_t stream);
-hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream);
-hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream);
-hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream);  // block lists only: 64 keys per wave, one wave per SIMD
-hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream);  // tile lists only: 64 keys per work-group
-hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream);
+// dK/dV launches leave their merge, if any, in *later (null: they launch it); dQ launches take one along.
+hipError_t launch_bwd_dq(BwdParams p, hipStream_t stream, Merge before = {});
+hipError_t launch_bwd_dkdv(BwdParams p, hipStream_t stream, Merge* later = nullptr);
+hipError_t launch_bwd_dkdv64(BwdParams p, hipStream_t stream, Merge* later = nullptr);  // block lists only: 64 keys per wave, one wave per SIMD
+hipError_t launch_bwd_dkdv_slab(BwdParams p, hipStream_t stream, Merge* later = nullptr);  // tile lists only: 64 keys per work-group
+hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream, Merge before = {});
 // Shape of a dK/dV launch over key tiles of `tile_rows` rows, whose parts store `slot_bytes` each: sets p.num_items, split,
 // items_per_xcd, order, queue and total_work and the number of work-groups, and launches what has to run in front, p.make's statistics
 // among it.
 hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream, bool takes_pieces = false);
 int device_compute_units();
-// One output of the split items: where the sums go, what they are multiplied by, where in a part's slot they lie (floats); rows of a head
-// that the items have and those of them that the output has (0: all).
-struct PartialOut {
-  __bf16* out;
-  float scale;
-  int64_t offset;
-  int head_rows = 0, out_rows = 0;
-};
-// order: null, or the item of every grid index.
-hipError_t launch_partial_sum(const SplitPlan& split, int64_t slot_floats, int rows, const PartialOut* outs, int n_outs, const int32_t* order,
-                              hipStream_t stream, const Pieces& pieces = {});
+// Merges parts in a launch of its own, or of dK/dV with `later` set leaves that to the dQ launch (see Merge).
+hipError_t launch_merge(const Merge& m, hipStream_t stream);
+// For a dQ launch with the plan `split`, whose parts store `slot_bytes` each: it takes `before` along, with the results of its own parts behind
+// those that are still to be merged, or where they do not fit there `before` is launched now and cleared.
+hipError_t take_along(SplitPlan& split, int64_t slot_bytes, Merge& before, hipStream_t stream);
 hipError_t launch_probe_mfma(const float* src, float* sink, int work_groups, int iters, hipStream_t stream);
 hipError_t launch_probe_read(const void* src, int64_t bytes, uint32_t* sink, int work_groups, hipStream_t stream);
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,

@@ -485,6 +485,7 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
   // What else lives in the workspace, from its end: the claim counters, then the order of the items.
   int64_t top = ws == nullptr ? 0 : (p.split_ws_bytes - kQueueBytes) & ~(int64_t)15;
   const int64_t bottom = parts * tiles.slot_bytes + kNoteBytes;
+  p.results_end = (bottom + 15) & ~(int64_t)15;
   int* const queue = ws != nullptr && top >= bottom ? reinterpret_cast<int*>(ws + top) : nullptr;
   top = (top - (int64_t)p.num_items * 4) & ~(int64_t)15;
   const int64_t order_at = top;
@@ -519,7 +520,9 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
              2 * slots, most_pieces, p.split.items == p.num_items ? p.split.parts : 1};
     p.pieces = {maker.header, maker.list, maker.cut};
     p.split.ws = reinterpret_cast<float*>(ws);
+    p.results_end = 2 * slots * tiles.slot_bytes;
   }
+  p.kept_from = maker.header != nullptr ? top : ordered ? order_at : queue != nullptr ? reinterpret_cast<char*>(queue) - ws : p.split_ws_bytes;
 
   // Launches of four rounds and more let the work-groups claim their grid indices, with some more work-groups than indices,
   // so that an XCD that is through early takes over from the others (claim_work; either mapping deals grid index i to XCD
