@@ -149,12 +149,38 @@ FBA_DEVICE int wave_max(int x) {
 // H1 S16384, a quarter kept, 50.2; so 38.0 and 49.5).  kGroups: the lists of up to four query heads of a group add up, other heads from item to item;
 // launches that take their items in falling order of length, which have more than a round, look at the lists of those they cut through that
 // order.  kNever: for launches that the host always decides.
-enum class Look { kNever, kSingle, kGroups };
+enum class Look { kNever, kSingle, kGroups, kMasks };
 constexpr float kPartsSpread = 0.4f;  // how much of what the longest list is above the mean the parts of all lists take longer
+// kMasks: 16 rows of a block mask, four lanes to a row.
+FBA_DEVICE int blocks_selected(const uint8_t* row, int blocks, int lane4) {  // by all four lanes alike
+  int n = 0;
+  if (blocks < 16) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * i + lane4 < blocks) n += row[4 * i + lane4] != 0;
+  } else {
+    for (int at = 16 * lane4; at < blocks; at += 64) {  // the row's last 16 bytes once more where fewer are left, without those counted already
+      const int from = min(at, blocks - 16), again = at - from;
+      u32x4 bytes;
+      __builtin_memcpy(&bytes, row + from, 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t on = ((bytes[i] & 0x7f7f7f7fu) + 0x7f7f7f7fu | bytes[i]) & 0x80808080u;  // bit 7 of every byte that is not zero
+        const int drop = again - 4 * i;  // bytes of this word
+        if (drop > 0) on = drop >= 4 ? 0 : on >> 8 * drop;
+        n += __builtin_popcount(on);
+      }
+    }
+  }
+  n += __builtin_amdgcn_update_dpp(0, n, 0xb1, 0xf, 0xf, false);  // quad_perm 1, 0, 3, 2
+  return n + __builtin_amdgcn_update_dpp(0, n, 0x4e, 0xf, 0xf, false);  // 2, 3, 0, 1
+}
+template <Look kLook, typename Plan>
+FBA_DEVICE bool looks(const Plan& plan) { return kLook != Look::kNever && (kLook == Look::kMasks ? plan.look.mask != nullptr : plan.look.cnt != nullptr); }
 template <Look kLook, typename Plan>
 FBA_DEVICE int split_parts(const Plan& plan) {
   const auto& l = plan.look;
-  if (kLook == Look::kNever || l.cnt == nullptr) return plan.parts;
+  if (!looks<kLook>(plan)) return plan.parts;
   const int lane = threadIdx.x & 63;
   int row = l.first + min((lane >> 2) * l.stride + (lane & 3), l.last);
   int n;
@@ -162,7 +188,9 @@ FBA_DEVICE int split_parts(const Plan& plan) {
     row = l.order[plan.first + lane * plan.items / 64] / l.row_tiles;
     if (l.shared) row %= l.rows_per_head;
   }
-  if (kLook == Look::kGroups && l.group > 1) {
+  if (kLook == Look::kMasks) {
+    n = blocks_selected(l.mask + (int64_t)(l.first + min((lane >> 2) * l.stride, l.last)) * l.blocks, l.blocks, lane & 3);
+  } else if (kLook == Look::kGroups && l.group > 1) {
     const int r = (lane * 5 & 63) * l.group / 64;
     const int32_t* const first = l.cnt + row + (int64_t)(row / l.rows_per_head) * (l.group - 1) * l.rows_per_head;  // of the group's first head
     int of[4];
@@ -188,7 +216,7 @@ FBA_DEVICE int split_parts(const Plan& plan) {
 template <Look kLook, typename Plan>
 FBA_DEVICE bool split_position(const Plan& plan, int& s, int& item, int& part, int& parts) {
   parts = split_parts<kLook>(plan);
-  if (kLook != Look::kNever && s == 0 && threadIdx.x == 0 && plan.look.cnt != nullptr) *plan.note = parts;
+  if (kLook != Look::kNever && s == 0 && threadIdx.x == 0 && looks<kLook>(plan)) *plan.note = parts;
   int i = s / parts;
   if (i >= plan.items) return false;
   part = s - i * parts;
@@ -274,7 +302,7 @@ FBA_DEVICE ConstIdx const_idx(const int32_t* p) { return (ConstIdx)(uintptr_t)p;
 
 // For the merge of forward: how many parts the kernel in front made.  A scalar load: the merge's addresses wait for it.
 template <typename Plan>
-FBA_DEVICE int parts_made(const Plan& plan) { return plan.look.cnt == nullptr ? plan.parts : const_idx(plan.note)[0]; }
+FBA_DEVICE int parts_made(const Plan& plan) { return plan.look.cnt == nullptr && plan.look.mask == nullptr ? plan.parts : const_idx(plan.note)[0]; }
 
 // Sums the fp32 partial rows of split items in part order: out = scale * sum_p partial_p, as bf16.  One thread per four columns; work-group `wg` of
 // `wgs` with kThreads threads each, every n_outs-th for one of the outputs (dK/dV: two per slot).  All parts are requested at once, as in
@@ -576,6 +604,43 @@ struct MaskCursor {
   FBA_DEVICE int halves() const {  // which 16-row halves select the current block
     const int b = __builtin_ctzll(left);
     return (int)((m0 >> b) & 1) | (int)((m1 >> b) & 1) << 1;
+  }
+};
+
+// A mask row of up to 256 blocks as a list: those that are selected, in order.  All lanes of a wave call everything together; what is kept is in
+// scalar registers, so that the next entry costs no load and no wait.
+struct MaskList {
+  unsigned long long left, next[3];  // of the 64 blocks at hand, and of those that follow
+  int base;
+  FBA_DEVICE void load(const uint8_t* row, int blocks, int lane) {
+    int on[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) on[i] = 64 * i + lane < blocks ? row[64 * i + lane] : 0;
+    left = __builtin_amdgcn_ballot_w64(on[0] != 0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) next[i] = __builtin_amdgcn_ballot_w64(on[i + 1] != 0);
+    base = 0;
+  }
+  FBA_DEVICE int count() const { return __builtin_popcountll(left) + __builtin_popcountll(next[0]) + __builtin_popcountll(next[1]) + __builtin_popcountll(next[2]); }
+  FBA_DEVICE void word() {
+    left = next[0];
+    next[0] = next[1];
+    next[1] = next[2];
+    next[2] = 0;
+    base += 64;
+  }
+  FBA_DEVICE void skip(int n) {  // n entries, no more than there are
+    for (int here; n >= (here = __builtin_popcountll(left)) && base < 192; n -= here) word();
+    for (; n > 0; --n) left &= left - 1;
+  }
+  FBA_DEVICE int take() {  // 0 past the end
+    while (left == 0) {
+      if (base >= 192) return 0;
+      word();
+    }
+    const int block = base + __builtin_ctzll(left);
+    left &= left - 1;
+    return block;
   }
 };
 

@@ -27,13 +27,17 @@ struct ListLengths {
   int tile_rows, list_rows, rows_per_head;  // rows of an item, rows that share a list row, list rows per head
   int group;           // rows of `group` consecutive heads add up (dK/dV: query heads of a kv head)
   int steps;           // of an entry
+  const uint8_t* mask = nullptr;  // instead of cnt: the rows' masks, of `blocks` bytes each
+  int blocks = 0;
 };
 
 constexpr int kMostParts = 8;  // of a split item
 
 // Which lists the device looks at, and the line in units of what it finds: n entries in a lane, one list or four of a group.
 struct ListLook {
-  const int32_t* cnt;        // null: the plan's number of parts stands
+  const int32_t* cnt;        // null: the plan's number of parts stands, unless there are masks
+  const uint8_t* mask;       // null, or rows of `blocks` bytes, one of them for a block that is listed
+  int blocks;
   int first, stride, last;   // rows first + 0..3, first + stride + 0..3, ... first + 15 stride + 0..3, none of them beyond first + last
   int group, rows_per_head;  // see ListLengths; row numbers count one head of a group
   // Where the split items are the last of an order of their own (dK/dV), their rows instead: item order[i] has row order[i] / row_tiles.  Else null.
@@ -134,6 +138,8 @@ struct FwdParams {
   // tiled = 1: q_cnt / q_idx are tile lists (qt_cnt [mask_bh, Sq/128], qt_ent [mask_bh, Sq/128, nK], see
   // tile_lists_kernel) instead of block lists
   int tiled;
+  // null, or the block mask [mask_bh, nQ, nK] to be read in place of q_cnt / q_idx (block lists, up to kMaskBlocks key blocks)
+  const uint8_t* mask;
   int64_t split_ws_bytes;  // size of split.ws as handed in by the caller
   int variant;  // 0: 384-row work-groups where q_block allows (measurement of that variant); 1: 128-row work-groups
   SplitPlan split;
@@ -328,6 +334,7 @@ hipError_t launch_tile_permute(const void* x, void* out, int64_t n_seq, int T, i
 hipError_t launch_resize_rows(int n, const void* const* src, void* const* dst, const int64_t* n_seq, const int32_t* src_len, const int32_t* dst_len,
                               hipStream_t stream);
 hipError_t launch_resize_mask(const uint8_t* src, uint8_t* dst, int64_t M, int src_q, int src_k, int dst_q, int dst_k, hipStream_t stream);
+constexpr int kMaskBlocks = 256;
 hipError_t launch_fwd(FwdParams p, hipStream_t stream);
 hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream);
 bool fwd_takes_mask(int64_t rows, int64_t kv_len);

@@ -110,7 +110,7 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
     }
   }
   if (n_hull == 1) return plan;
-  const bool device = lengths.cnt != nullptr, one_round = device && num_items < slots && step.own_pace;
+  const bool device = lengths.cnt != nullptr || lengths.mask != nullptr, one_round = device && num_items < slots && step.own_pace;
   const double least = hull[1].least * (hull[0].slope - hull[1].slope);
   const bool uneven = one_round && 2 * rest <= slots && max_steps * (hull[0].slope - 0.5 * hull[1].slope) >= 2.5 * least;
   if (hull[1].least > 0.6 * max_steps && !uneven) return plan;  // lists of usual density stay whole
@@ -132,6 +132,8 @@ SplitPlan plan_split(int num_items, int wgs_per_cu, int max_steps, StepCost step
   const int64_t rows = (int64_t)num_items * lengths.tile_rows / lengths.list_rows, from = second ? 0 : (int64_t)plan.first * lengths.tile_rows / lengths.list_rows;
   const int64_t span = lengths.shared ? std::min<int64_t>(rows - from, lengths.rows_per_head) : rows - from;
   look.cnt = lengths.cnt;
+  look.mask = lengths.mask;
+  look.blocks = lengths.blocks;
   look.first = (int)(lengths.shared ? lengths.rows_per_head - span : from);
   look.row_tiles = std::max(lengths.list_rows / lengths.tile_rows, 1);
   look.shared = lengths.shared;

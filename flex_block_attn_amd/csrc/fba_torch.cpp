@@ -40,7 +40,7 @@ constexpr int64_t kXcds = 8;
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                \
   X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists_cut) X(fba_pair_slots_bounds) X(fba_tile_slots_bounds)        \
-  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_handover) X(fba_bwd_tiled_cut) X(fba_bwd_dense) \
+  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_blocks) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_handover) X(fba_bwd_tiled_cut) X(fba_bwd_dense) \
   X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
@@ -198,6 +198,17 @@ std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor
                                                       p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(),
                                                       split.bytes, current_stream(q)));
   return {o, lse};
+}
+
+// The same on the block mask, where fba_fwd_blocks takes it.
+bool takes_blocks(const Problem& p) { return !p.tiled() && p.nK() <= 256; }
+at::Tensor run_forward_on_blocks(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask, int64_t split_bytes) {
+  at::Tensor o = at::empty_like(q);
+  const at::Tensor lse = at::empty({p.B, p.Hq, p.Sq, 1}, q.options().dtype(at::kFloat));
+  SplitWorkspace split(q, split_bytes);
+  check(lib.fba_fwd_blocks(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), static_cast<const uint8_t*>(mask.data_ptr()), p.mask_bh, p.B, p.Hq,
+                           p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes, current_stream(q)));
+  return o;
 }
 
 // Does forward read the block mask itself?  (Decided on the padded lengths, whether or not the call pads.)
@@ -541,6 +552,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   const bool backward = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
   if (!backward) {
     if (takes_mask(p)) return run_forward_on_mask(p, q, k, v, mask).first;
+    if (takes_blocks(p)) return run_forward_on_blocks(p, q, k, v, mask, split_bytes);
     const Inputs in(q, k, v, mask, *s);
     build_lists(*s, mask, false, false);
     const at::Tensor o = run_forward(p, in.q, in.k, in.v, s->lists, split_bytes).first;

@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2008
+#define FBA_VERSION 2009
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -67,7 +67,7 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  *                   the call's work on the stream; its contents before and after are meaningless
  *   split_ws_bytes  its size; fba_split_workspace_bytes() is what the planner can use at most (a smaller buffer limits
  *                   the number of ranges, never correctness)
- * On tile lists forward (64-row tiles) and the dK/dV kernel split; the dQ kernels do not.
+ * On tile lists forward and the dK/dV kernel split, and dQ from dS behind a whole round; the recomputing dQ kernel does not.
  * The same workspace lends what lies behind the partial results to the dK/dV kernels, from its end: 256 bytes for eight counters
  * in launches of four rounds and more, zeroed by a small launch in front, from which the work-groups claim the tile they work
  * on, with an eighth more work-groups launched than there are tiles; and, on block lists in launches of one to eight rounds, four
@@ -100,6 +100,14 @@ int32_t fba_fwd(const void* q, const void* k, const void* v, void* o, float* lse
                 const int32_t* q_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv,
                 int32_t head_dim, int32_t q_block, int32_t k_block,
                 void* split_ws, int64_t split_ws_bytes, void* hip_stream);
+
+/*
+ * fba_fwd on the lists of this block mask [mask_bh, nQ, nK], one byte per entry, nonzero = selected, without the lists: for calls that need
+ * them for nothing else.  At most 256 key blocks (otherwise FBA_ERR_UNSUPPORTED).  How many ranges: by the lengths of 16 of its rows.
+ */
+int32_t fba_fwd_blocks(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int64_t mask_bh, int32_t B, int32_t Hq,
+                       int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
+                       void* hip_stream);
 
 /*
  * Forward straight from the block mask, in one launch and without a workspace: for problems too small to fill the GPU, where lists

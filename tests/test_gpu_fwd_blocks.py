@@ -1,0 +1,79 @@
+"""Calls without gradients on whole 128-row blocks read the block mask where lists had at most 256 key blocks: rows of one block to 256, whole words of 64 and around, fewer
+than 16; the first and the last block, none, all; parts, and as many as by the lists; a shared mask, grouped heads; mask bytes other than one; 257 blocks, which go through
+lists.  Against forward on lists, bit for bit: rows of equal length, so that both decide alike on the parts."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _masks(kind, shape, g, gpu):
+    nQ, nK = shape[-2:]
+    if kind == "all":
+        return torch.ones(shape, dtype=torch.bool, device=gpu)
+    if kind == "none":
+        return torch.zeros(shape, dtype=torch.bool, device=gpu)
+    keep = 1 if kind == "one" else max(1, round(kind * nK))
+    score = torch.rand(shape, generator=g, device=gpu)
+    if kind == "one":  # the first, the last, one in between
+        score[..., 0::3, 0] = score[..., 1::3, -1] = 2.0
+    return torch.zeros(shape, dtype=torch.bool, device=gpu).scatter_(-1, score.topk(keep, -1).indices, True)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,nK,qbs,kbs,dims", [
+    (1, 70, 70, 128, 1, 128, 128, 4),
+    (1, 70, 70, 128, 15, 128, 128, 4),
+    (1, 9, 3, 1024, 16, 128, 128, 4),
+    (1, 9, 3, 1024, 17, 128, 128, 4),
+    (2, 10, 5, 512, 63, 256, 128, 4),
+    (1, 24, 6, 768, 64, 128, 128, 4),
+    (1, 24, 24, 1280, 65, 128, 128, 2),
+    (1, 3, 3, 4992, 30, 384, 384, 4),
+    (1, 4, 4, 2304, 129, 128, 128, 4),
+    (1, 8, 8, 1152, 192, 384, 128, 4),
+    (1, 66, 66, 1024, 24, 128, 128, 4),   # behind a whole round
+    (1, 4, 2, 2304, 255, 128, 128, 2),
+    (1, 2, 2, 4608, 256, 128, 128, 4),
+    (1, 2, 2, 4608, 257, 128, 128, 4),
+])
+@pytest.mark.parametrize("kind", [0.4, "one", "none", "all"])
+def test_as_on_lists(gpu, B, Hq, Hkv, Sq, nK, qbs, kbs, dims, kind):
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd import _lib
+
+    print(f"blocks B{B} Hq{Hq} Hkv{Hkv} Sq{Sq} {nK} x {kbs} q{qbs} {kind}", flush=True)
+    g = torch.Generator(device=gpu).manual_seed(Sq + nK)
+    m = _masks(kind, ((B, Hq) if dims == 4 else ()) + (Sq // qbs, nK), g, gpu)
+    q = torch.randn((B, Hq, Sq, 128), generator=g, device=gpu).to(torch.bfloat16)
+    k, v = (torch.randn((B, Hkv, nK * kbs, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    assert not _lib.load().fba_fwd_takes_mask(B * Hq * Sq, nK * kbs)
+    want = fba.forward_with_lists(q, k, v, qbs, kbs, fba.lists_for(m, qbs, kbs))[0]
+    got = fba.flex_block_attn_func(q, k, v, qbs, kbs, m)
+    assert torch.equal(got, want)
+    if kind == "none":
+        assert not bool(got.any())
+
+
+def test_mask_bytes_and_limits(gpu):
+    """Any byte but zero selects; more key blocks than the kernel keeps, and blocks that are no whole tiles, are refused."""
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd import _lib
+    from flex_block_attn_amd.interface import _ptr, _stream
+
+    g = torch.Generator(device=gpu).manual_seed(5)
+    B, H, Sq, nK = 1, 12, 1536, 37
+    q = torch.randn((B, H, Sq, 128), generator=g, device=gpu).to(torch.bfloat16)
+    k, v = (torch.randn((B, H, nK * 128, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    m = torch.zeros((B, H, Sq // 128, nK), dtype=torch.uint8, device=gpu)
+    at = torch.rand(m.shape, generator=g, device=gpu).topk(20, -1).indices
+    m.scatter_(-1, at, torch.randint(1, 256, at.shape, generator=g, device=gpu).to(torch.uint8))
+    want, want_lse = fba.forward_with_lists(q, k, v, 128, 128, fba.lists_for(m != 0, 128, 128))
+    o, lse = torch.empty_like(q), torch.empty((B, H, Sq, 1), device=gpu)
+    ws = torch.empty(_lib.load().fba_split_workspace_bytes(), dtype=torch.uint8, device=gpu)
+    args = (*map(_ptr, (q, k, v, o, lse, m)), B * H, B, H, H, Sq, nK * 128, 128)
+    _lib.call("fba_fwd_blocks", *args, 128, 128, _ptr(ws), ws.numel(), _stream())
+    assert torch.equal(o, want) and torch.equal(lse.flatten(), want_lse.flatten())
+    with pytest.raises(_lib.FbaError):
+        _lib.call("fba_fwd_blocks", *args, 64, 64, _ptr(ws), ws.numel(), _stream())
+    with pytest.raises(_lib.FbaError, match="257 key blocks"):
+        _lib.call("fba_fwd_blocks", *args[:-2], 257 * 128, 128, 128, 128, _ptr(ws), ws.numel(), _stream())
