@@ -33,7 +33,7 @@ SIGNATURES = {
     "fba_split_workspace_bytes": (_c_i64, []),
     "fba_split_plan": (_c_i32, [_c_i32, _c_i64] + [_c_i32] * 8 + [_c_i64, _c_ptr]),
     "fba_fwd": (_c_i32, [_c_ptr] * 7 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
-    "fba_fwd_blocks": (_c_i32, [_c_ptr] * 6 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
+    "fba_fwd_blocks": (_c_i32, [_c_ptr] * 10 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_fwd_mask": (_c_i32, [_c_ptr] * 6 + [_c_i64] + [_c_i32] * 8 + [_c_ptr]),
     "fba_fwd_mask_copy": (_c_i32, [_c_ptr] * 7 + [_c_i32, _c_i64] + [_c_i32] * 8 + [_c_ptr]),
     "fba_fwd_takes_mask": (_c_i32, [_c_i64, _c_i32]),

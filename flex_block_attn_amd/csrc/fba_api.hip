@@ -124,7 +124,7 @@ int check_tile_list_shape(int32_t nQ, int32_t nK, int32_t q_block, int32_t k_blo
 
 int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, const int32_t* q_cnt, const int32_t* q_idx, const uint8_t* mask,
              int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
-             int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream, bool tiled) {
+             int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream, bool tiled, decltype(fba::FwdParams::make) make = {}) {
   const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
   if (int rc = check_shape(s)) return rc;
   if (int rc = check_ptrs({{"q", q}, {"k", k}, {"v", v}, {"o", o}})) return rc;
@@ -133,7 +133,7 @@ int fwd_impl(const void* q, const void* k, const void* v, void* o, float* lse, c
   if (int rc = check_split_ws(split_ws, split_ws_bytes)) return rc;
   fba::FwdParams p{};
   p.q = (const __bf16*)q; p.k = (const __bf16*)k; p.v = (const __bf16*)v; p.o = (__bf16*)o; p.lse = lse;
-  p.q_cnt = q_cnt; p.q_idx = q_idx; p.mask = mask; p.mask_bh = mask_bh;
+  p.q_cnt = q_cnt; p.q_idx = q_idx; p.mask = mask; p.make = make; p.mask_bh = mask_bh;
   p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.Sq = Sq; p.Skv = Skv; p.nQ = Sq / q_block; p.nK = Skv / k_block;
   p.q_block = q_block; p.k_block = k_block;
   p.scale_log2e = 1.4426950408889634f / 11.313708498984761f;
@@ -165,13 +165,18 @@ int32_t fba_fwd_tiled(const void* q, const void* k, const void* v, void* o, floa
   return fwd_impl(q, k, v, o, lse, qt_cnt, qt_ent, nullptr, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, true);
 }
 
-int32_t fba_fwd_blocks(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int64_t mask_bh, int32_t B, int32_t Hq,
-                       int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
-                       void* hip_stream) {
+int32_t fba_fwd_blocks(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int32_t* q_cnt, int32_t* q_idx, int32_t* k_cnt,
+                       int32_t* k_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
+                       int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream) {
   if (!mask) return fail(FBA_ERR_INVALID, "null pointer argument");
+  const bool make = q_cnt || q_idx || k_cnt || k_idx;
+  if (make && (!q_cnt || !q_idx || !k_cnt || !k_idx)) return fail(FBA_ERR_INVALID, "forward: all four lists, or none");
+  if (make && q_block > 0 && k_block > 0 && mask_bh * (Sq / q_block + Skv / k_block) > fba::kMakeRows)
+    return fail(FBA_ERR_UNSUPPORTED, "forward: more than %d rows of lists; build them with fba_mask_compact", fba::kMakeRows);
   if (k_block > 0 && Skv / k_block > fba::kMaskBlocks)
     return fail(FBA_ERR_UNSUPPORTED, "forward: %d key blocks are more than %d; build lists with fba_mask_compact and call fba_fwd", Skv / k_block, fba::kMaskBlocks);
-  return fwd_impl(q, k, v, o, lse, nullptr, nullptr, mask, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, false);
+  return fwd_impl(q, k, v, o, lse, nullptr, nullptr, mask, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, false,
+                  {q_cnt, q_idx, k_cnt, k_idx, 0});
 }
 
 int32_t fba_fwd_mask_copy(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, uint8_t* mask_copy, int32_t o_rows,

@@ -607,6 +607,38 @@ struct MaskCursor {
   }
 };
 
+// Row w of the lists that a block mask [mask_bh, nQ, nK] comes to: the query blocks' first, then, unless k_cnt is null, the key blocks'.  A wave's
+// work: 64 mask bytes per step, ballot + prefix popcount gives each active lane its slot, so the output order is the index order and the
+// result is independent of scheduling (bit-exact, no atomics).
+FBA_DEVICE void compact_row(const uint8_t* __restrict__ mask, int64_t mask_bh, int nQ, int nK, int32_t* __restrict__ q_cnt, int32_t* __restrict__ q_idx,
+                            int32_t* __restrict__ k_cnt, int32_t* __restrict__ k_idx, int64_t w) {
+  const int lane = threadIdx.x & 63;
+  const int64_t n_qrows = mask_bh * nQ, n_krows = k_cnt != nullptr ? mask_bh * nK : 0;  // forward alone needs no key-major lists
+  if (w >= n_qrows + n_krows) return;
+
+  const bool row_pass = w < n_qrows;
+  const int64_t r = row_pass ? w : w - n_qrows;
+  const int len = row_pass ? nK : nQ;           // entries per output row
+  const int64_t m = r / (row_pass ? nQ : nK);   // which (batch, head) mask
+  const int self = (int)(r - m * (row_pass ? nQ : nK));
+  const uint8_t* base = mask + m * (int64_t)nQ * nK;
+  // element t of this output row's source: row pass mask[self, t]; column pass mask[t, self]
+  const int64_t stride = row_pass ? 1 : nK;
+  const uint8_t* src = base + (row_pass ? (int64_t)self * nK : (int64_t)self);
+  int32_t* out = (row_pass ? q_idx : k_idx) + r * (int64_t)len;
+
+  int cnt = 0;
+  for (int t0 = 0; t0 < len; t0 += 64) {
+    const int t = t0 + lane;
+    const bool on = t < len && src[(int64_t)t * stride] != 0;
+    const unsigned long long bal = __builtin_amdgcn_ballot_w64(on);
+    if (on) out[cnt + __builtin_popcountll(bal & ((1ull << lane) - 1ull))] = t;
+    cnt += __builtin_popcountll(bal);
+  }
+  for (int t = cnt + lane; t < len; t += 64) out[t] = -1;
+  if (lane == 0) (row_pass ? q_cnt : k_cnt)[r] = cnt;
+}
+
 // A mask row of up to 256 blocks as a list: those that are selected, in order.  All lanes of a wave call everything together; what is kept is in
 // scalar registers, so that the next entry costs no load and no wait.
 struct MaskList {

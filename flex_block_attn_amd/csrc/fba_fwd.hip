@@ -126,7 +126,8 @@ FBA_DEVICE void softmax_exp(FwdState& st, f32x16& s, bf16x8 (&pk)[2], bool activ
 //
 // kMask: the list is read from the block mask, so that a call without gradients needs no launch that makes
 // lists: H8 S4096, 128-token blocks, 12 of 32 kept 32.7 -> 30.4 us, H12 S3072 32.8 -> 30.6, H2 S10240 68.5 -> 67.2, H24/6 768 rows against 30720 keys 128.0 ->
-// 126.4, H24 S11520, all blocks, 1396.5 -> 1393.3.
+// 126.4, H24 S11520, all blocks, 1396.5 -> 1393.3.  Steps that number no pairs have it make their lists on the way, a wave to a row in work-groups behind the others:
+// H4 S3840 115.1 -> 112.3 us, H2 S6144 139.5 -> 137.0, H12 S3456 146.6 -> 144.4.
 template <int kWaves, bool kMask>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(kWaves == 12 ? 3 : 2, kWaves == 12 ? 3 : 2))) void fwd_kernel(const FwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // K ring [4][8 KiB] | V ring [4][8 KiB]
@@ -134,6 +135,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if constexpr (kMask) {
+    const int own_wgs = (int)gridDim.x - p.make.wgs;
+    if ((int)blockIdx.x >= own_wgs)
+      return compact_row(p.mask, p.mask_bh, p.nQ, p.nK, p.make.q_cnt, p.make.q_idx, p.make.k_cnt, p.make.k_idx, ((int)blockIdx.x - own_wgs) * 4 + wave);
+  }
   // whole items first (dealt to the XCDs in contiguous spans), then the parts of the split items
   int item, part = 0, parts = 1;
   int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
@@ -1207,7 +1213,8 @@ hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   const int split_wgs = (p.num_items - p.split.first) * p.split.parts;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs), dim3(rows * 2), smem, stream, p);
+  p.make.wgs = p.make.q_cnt != nullptr ? (int)((p.mask_bh * (p.nQ + p.nK) + 3) / 4) : 0;
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs + p.make.wgs), dim3(rows * 2), smem, stream, p);
   if (split_wgs > 0) hipLaunchKernelGGL(fwd_merge_kernel<128>, dim3(merge_grid((p.num_items - p.split.first) * 16)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }

@@ -140,6 +140,11 @@ struct FwdParams {
   int tiled;
   // null, or the block mask [mask_bh, nQ, nK] to be read in place of q_cnt / q_idx (block lists, up to kMaskBlocks key blocks)
   const uint8_t* mask;
+  // lists that are to be made from it on the way, for a backward pass (q_cnt null: none), by so many work-groups
+  struct {
+    int32_t *q_cnt, *q_idx, *k_cnt, *k_idx;
+    int wgs;
+  } make;
   int64_t split_ws_bytes;  // size of split.ws as handed in by the caller
   int variant;  // 0: 384-row work-groups where q_block allows (measurement of that variant); 1: 128-row work-groups
   SplitPlan split;
@@ -334,7 +339,7 @@ hipError_t launch_tile_permute(const void* x, void* out, int64_t n_seq, int T, i
 hipError_t launch_resize_rows(int n, const void* const* src, void* const* dst, const int64_t* n_seq, const int32_t* src_len, const int32_t* dst_len,
                               hipStream_t stream);
 hipError_t launch_resize_mask(const uint8_t* src, uint8_t* dst, int64_t M, int src_q, int src_k, int dst_q, int dst_k, hipStream_t stream);
-constexpr int kMaskBlocks = 256;
+constexpr int kMaskBlocks = 256, kMakeRows = 1024;  // of lists that forward makes on the way, at most
 hipError_t launch_fwd(FwdParams p, hipStream_t stream);
 hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream);
 bool fwd_takes_mask(int64_t rows, int64_t kv_len);

@@ -5,8 +5,7 @@
 // (flex_block_attn_interface.py:85-86; scan at flex_block_attn_h100.cu:672, :738).  Here one launch emits
 //   q_cnt[m, i], q_idx[m, i, 0..q_cnt) = { j : mask[m, i, j] }   ascending, padded with -1 to nK entries
 //   k_cnt[m, j], k_idx[m, j, 0..k_cnt) = { i : mask[m, i, j] }   ascending, padded with -1 to nQ entries
-// One wave per output row: 64 mask bytes per step, ballot + prefix popcount gives each active lane its slot, so the
-// output order is the index order and the result is independent of scheduling (bit-exact, no atomics).
+// One wave per output row (compact_row in fba_common.h).
 #include "fba_common.h"
 #include "fba_kernels.h"
 
@@ -15,32 +14,7 @@ namespace fba {
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256))) void mask_compact_kernel(
     const uint8_t* __restrict__ mask, int64_t mask_bh, int nQ, int nK, int32_t* __restrict__ q_cnt,
     int32_t* __restrict__ q_idx, int32_t* __restrict__ k_cnt, int32_t* __restrict__ k_idx) {
-  const int lane = threadIdx.x & 63;
-  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int64_t n_qrows = mask_bh * nQ, n_krows = k_cnt != nullptr ? mask_bh * nK : 0;  // forward alone needs no key-major lists
-  if (w >= n_qrows + n_krows) return;
-
-  const bool row_pass = w < n_qrows;
-  const int64_t r = row_pass ? w : w - n_qrows;
-  const int len = row_pass ? nK : nQ;           // entries per output row
-  const int64_t m = r / (row_pass ? nQ : nK);   // which (batch, head) mask
-  const int self = (int)(r - m * (row_pass ? nQ : nK));
-  const uint8_t* base = mask + m * (int64_t)nQ * nK;
-  // element t of this output row's source: row pass mask[self, t]; column pass mask[t, self]
-  const int64_t stride = row_pass ? 1 : nK;
-  const uint8_t* src = base + (row_pass ? (int64_t)self * nK : (int64_t)self);
-  int32_t* out = (row_pass ? q_idx : k_idx) + r * (int64_t)len;
-
-  int cnt = 0;
-  for (int t0 = 0; t0 < len; t0 += 64) {
-    const int t = t0 + lane;
-    const bool on = t < len && src[(int64_t)t * stride] != 0;
-    const unsigned long long bal = __ballot(on);
-    if (on) out[cnt + __popcll(bal & ((1ull << lane) - 1ull))] = t;
-    cnt += __popcll(bal);
-  }
-  for (int t = cnt + lane; t < len; t += 64) out[t] = -1;
-  if (lane == 0) (row_pass ? q_cnt : k_cnt)[r] = cnt;
+  compact_row(mask, mask_bh, nQ, nK, q_cnt, q_idx, k_cnt, k_idx, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6));
 }
 
 hipError_t launch_mask_compact(const uint8_t* mask, int64_t mask_bh, int nQ, int nK, int32_t* q_cnt, int32_t* q_idx,

@@ -202,13 +202,18 @@ std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor
 
 // The same on the block mask, where fba_fwd_blocks takes it.
 bool takes_blocks(const Problem& p) { return !p.tiled() && p.nK() <= 256; }
-at::Tensor run_forward_on_blocks(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask, int64_t split_bytes) {
+// Is it to make the lists of a step on the way?  Steps that number their pairs need them before forward is through (the host waits for the count);
+// with more rows than that the lists would hold up the launch, whose last work-groups make them.
+bool makes_lists(const Problem& p, bool dense) { return dense && takes_blocks(p) && p.mask_bh * (p.nQ() + p.nK()) <= 1024; }
+std::pair<at::Tensor, at::Tensor> run_forward_on_blocks(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask,
+                                                        const Lists& make, int64_t split_bytes) {
   at::Tensor o = at::empty_like(q);
-  const at::Tensor lse = at::empty({p.B, p.Hq, p.Sq, 1}, q.options().dtype(at::kFloat));
+  at::Tensor lse = at::empty({p.B, p.Hq, p.Sq, 1}, q.options().dtype(at::kFloat));
   SplitWorkspace split(q, split_bytes);
-  check(lib.fba_fwd_blocks(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), static_cast<const uint8_t*>(mask.data_ptr()), p.mask_bh, p.B, p.Hq,
-                           p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes, current_stream(q)));
-  return o;
+  check(lib.fba_fwd_blocks(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr<float>(), static_cast<const uint8_t*>(mask.data_ptr()), make.q_cnt, make.q_idx,
+                           make.k_cnt, make.k_idx, p.mask_bh, p.B, p.Hq, p.Hkv, p.Sq, p.Skv, kHeadDim, p.q_block, p.k_block, split.ptr(), split.bytes,
+                           current_stream(q)));
+  return {o, lse};
 }
 
 // Does forward read the block mask itself?  (Decided on the padded lengths, whether or not the call pads.)
@@ -351,7 +356,7 @@ struct Saved : torch::CustomClassHolder {
 
 // The lists of `mask` in one buffer; key-major half and (numbered) pair numbers only where backward will read them.  The mask is the
 // caller's: blocks that fill up the last tiles are in the lists' extents only.
-void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered) {
+void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered, bool launch = true) {
   const Problem& p = s.p;
   Lists& l = s.lists;
   const int64_t M = p.mask_bh;
@@ -381,6 +386,7 @@ void build_lists(Saved& s, const at::Tensor& mask, bool backward, bool numbered)
     l.k_cnt = b + k_cnt;
     l.k_idx = b + k_idx;
   }
+  if (!launch) return;  // room for them only: forward makes them
   check(lib.fba_lists_cut(static_cast<const uint8_t*>(mask.data_ptr()), M, p.nQ(), p.nK(), s.q_len / p.q_block, s.kv_len / p.k_block, p.q_block, p.k_block,
                           l.q_cnt, l.q_idx, l.k_cnt, l.k_idx, stream));
   if (!numbered) return;
@@ -473,8 +479,11 @@ struct Attention : torch::autograd::Function<Attention> {
       return cut ? o.narrow(2, 0, q_len).detach() : o;
     }
     const Inputs in(q, k, v, mask, *s);
-    build_lists(*s, mask, /*backward=*/true, /*numbered=*/!s->dense);
-    auto [o, lse] = takes_mask(s->p) ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask) : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
+    const bool on_mask = takes_mask(s->p), with_lists = !on_mask && makes_lists(s->p, s->dense);
+    build_lists(*s, mask, /*backward=*/true, /*numbered=*/!s->dense, /*launch=*/!with_lists);
+    auto [o, lse] = on_mask      ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask)
+                    : with_lists ? run_forward_on_blocks(s->p, in.q, in.k, in.v, in.mask, s->lists, s->split_bytes)
+                                 : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
     ctx->save_for_backward({in.q, in.k, in.v, o, lse});
     // The rows that were appended are cut off here and not behind this function, where autograd would give back gradients for them in
     // two launches of its own, a fill and a copy (13 of 280 us at B2 H8/2 S3136).  What is handed out shares its version with
@@ -552,7 +561,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   const bool backward = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
   if (!backward) {
     if (takes_mask(p)) return run_forward_on_mask(p, q, k, v, mask).first;
-    if (takes_blocks(p)) return run_forward_on_blocks(p, q, k, v, mask, split_bytes);
+    if (takes_blocks(p)) return run_forward_on_blocks(p, q, k, v, mask, Lists(p), split_bytes).first;
     const Inputs in(q, k, v, mask, *s);
     build_lists(*s, mask, false, false);
     const at::Tensor o = run_forward(p, in.q, in.k, in.v, s->lists, split_bytes).first;

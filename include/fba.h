@@ -102,12 +102,14 @@ int32_t fba_fwd(const void* q, const void* k, const void* v, void* o, float* lse
                 void* split_ws, int64_t split_ws_bytes, void* hip_stream);
 
 /*
- * fba_fwd on the lists of this block mask [mask_bh, nQ, nK], one byte per entry, nonzero = selected, without the lists: for calls that need
- * them for nothing else.  At most 256 key blocks (otherwise FBA_ERR_UNSUPPORTED).  How many ranges: by the lengths of 16 of its rows.
+ * fba_fwd on the lists of this block mask [mask_bh, nQ, nK], one byte per entry, nonzero = selected, without the lists.  At most 256 key blocks (otherwise
+ * FBA_ERR_UNSUPPORTED).  How many ranges: by the lengths of 16 of its rows.
+ *   q_cnt, q_idx, k_cnt, k_idx   null, or where the lists go that fba_mask_compact makes of the mask, for a backward pass: made in the same launch, of
+ *                                mask_bh * (nQ + nK) <= 1024 rows
  */
-int32_t fba_fwd_blocks(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int64_t mask_bh, int32_t B, int32_t Hq,
-                       int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block, int32_t k_block, void* split_ws, int64_t split_ws_bytes,
-                       void* hip_stream);
+int32_t fba_fwd_blocks(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int32_t* q_cnt, int32_t* q_idx, int32_t* k_cnt,
+                       int32_t* k_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
+                       int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream);
 
 /*
  * Forward straight from the block mask, in one launch and without a workspace: for problems too small to fill the GPU, where lists

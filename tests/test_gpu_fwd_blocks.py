@@ -1,6 +1,7 @@
 """Calls without gradients on whole 128-row blocks read the block mask where lists had at most 256 key blocks: rows of one block to 256, whole words of 64 and around, fewer
 than 16; the first and the last block, none, all; parts, and as many as by the lists; a shared mask, grouped heads; mask bytes other than one; 257 blocks, which go through
-lists.  Against forward on lists, bit for bit: rows of equal length, so that both decide alike on the parts."""
+lists.  Against forward on lists, bit for bit: rows of equal length, so that both decide alike on the parts.  And the
+lists that a step has it make in the same launch."""
 import pytest
 import torch
 
@@ -54,6 +55,46 @@ def test_as_on_lists(gpu, B, Hq, Hkv, Sq, nK, qbs, kbs, dims, kind):
         assert not bool(got.any())
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,nK,qbs,kbs,dims", [
+    (1, 66, 66, 128, 1, 128, 128, 4),     # a row and a column of one block
+    (1, 12, 4, 1536, 37, 128, 128, 4),
+    (2, 3, 3, 4608, 12, 384, 384, 4),
+    (1, 8, 8, 8192, 192, 128, 128, 2),    # 256 rows, one mask for all heads
+    (1, 4, 4, 8192, 192, 128, 128, 4),    # 1024
+    (1, 16, 16, 8192, 1, 8192, 8192, 4),
+])
+def test_lists_on_the_way(gpu, B, Hq, Hkv, Sq, nK, qbs, kbs, dims):
+    """Forward and the lists of one launch: those of fba_mask_compact, padding and all; a step through the operator has the gradients of the lists."""
+    import flex_block_attn_amd as fba
+    from flex_block_attn_amd import _lib
+    from flex_block_attn_amd.interface import _ptr, _stream
+
+    g = torch.Generator(device=gpu).manual_seed(Sq + nK)
+    m = torch.rand(((B, Hq) if dims == 4 else ()) + (Sq // qbs, nK), generator=g, device=gpu) < 0.4
+    q, do = (torch.randn((B, Hq, Sq, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    k, v = (torch.randn((B, Hkv, nK * kbs, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(2))
+    want = fba.lists_for(m, qbs, kbs)
+    made = [torch.full_like(t, 77) for t in (want.q_cnt, want.q_idx, want.k_cnt, want.k_idx)]
+    o, lse = torch.empty_like(q), torch.empty((B, Hq, Sq, 1), device=gpu)
+    ws = torch.empty(_lib.load().fba_split_workspace_bytes(), dtype=torch.uint8, device=gpu)
+    tail = (want.mask_bh, B, Hq, Hkv, Sq, nK * kbs, 128, qbs, kbs, _ptr(ws), ws.numel(), _stream())
+    _lib.call("fba_fwd_blocks", *map(_ptr, (q, k, v, o, lse, m, *made)), *tail)
+    for a, b in zip(made, (want.q_cnt, want.q_idx, want.k_cnt, want.k_idx)):
+        assert torch.equal(a, b)
+    none = o.clone(), lse.clone()
+    _lib.call("fba_fwd_blocks", *map(_ptr, (q, k, v, o, lse, m)), None, None, None, None, *tail)
+    assert torch.equal(o, none[0]) and torch.equal(lse, none[1])
+    with pytest.raises(_lib.FbaError, match="all four"):
+        _lib.call("fba_fwd_blocks", *map(_ptr, (q, k, v, o, lse, m, *made[:2])), None, None, *tail)
+    ins = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    out = fba.flex_block_attn_func(*ins, qbs, kbs, m)
+    grads = torch.autograd.grad(out, ins, do)
+    if not _lib.load().fba_fwd_takes_mask(B * Hq * Sq, nK * kbs):
+        assert torch.equal(out, o)
+    for name, a, b in zip(("dq", "dk", "dv"), grads, fba.backward_with_lists(q, k, v, o, lse, do, qbs, kbs, want)):
+        assert float((a.float() - b.float()).norm()) <= 1e-2 * float(b.float().norm()), name  # bf16 sums of another order, where the operator takes other kernels
+
+
 def test_mask_bytes_and_limits(gpu):
     """Any byte but zero selects; more key blocks than the kernel keeps, and blocks that are no whole tiles, are refused."""
     import flex_block_attn_amd as fba
@@ -70,10 +111,13 @@ def test_mask_bytes_and_limits(gpu):
     want, want_lse = fba.forward_with_lists(q, k, v, 128, 128, fba.lists_for(m != 0, 128, 128))
     o, lse = torch.empty_like(q), torch.empty((B, H, Sq, 1), device=gpu)
     ws = torch.empty(_lib.load().fba_split_workspace_bytes(), dtype=torch.uint8, device=gpu)
-    args = (*map(_ptr, (q, k, v, o, lse, m)), B * H, B, H, H, Sq, nK * 128, 128)
+    args = (*map(_ptr, (q, k, v, o, lse, m)), None, None, None, None, B * H, B, H, H, Sq, nK * 128, 128)
     _lib.call("fba_fwd_blocks", *args, 128, 128, _ptr(ws), ws.numel(), _stream())
     assert torch.equal(o, want) and torch.equal(lse.flatten(), want_lse.flatten())
     with pytest.raises(_lib.FbaError):
         _lib.call("fba_fwd_blocks", *args, 64, 64, _ptr(ws), ws.numel(), _stream())
     with pytest.raises(_lib.FbaError, match="257 key blocks"):
         _lib.call("fba_fwd_blocks", *args[:-2], 257 * 128, 128, 128, 128, _ptr(ws), ws.numel(), _stream())
+    lists = [torch.empty(1, dtype=torch.int32, device=gpu) for _ in range(4)]  # (refused before anything is written)
+    with pytest.raises(_lib.FbaError, match="1024 rows"):
+        _lib.call("fba_fwd_blocks", *map(_ptr, (q, k, v, o, lse, m, *lists)), 22 * B * H, 22 * B, H, H, Sq, nK * 128, 128, 128, 128, _ptr(ws), ws.numel(), _stream())
