@@ -343,7 +343,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
   store_tile_bf16(smem + wave * kSlabBytes, st.acc_o, l > 0.f ? 1.f / l : 0.f, p.o + qrow0 * kHeadDim, lane);
 }
 
-// Forward on tile lists (q_block or k_block no multiple of 128).
+// Forward on tile lists (q_block or k_block no multiple of 128), and on block masks in small launches.
 //
 // Work-group = 64 query rows, four waves, two work-groups per CU.  The unit of work is a chunk of 64 keys; wave w owns rows
 // 32 (w % 2) .. +31 against keys 32 (w / 2) .. +31 of every chunk, with the same pipeline as fwd_kernel (P_{t-1} V_{t-1} |
@@ -359,33 +359,41 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
 // well, of a 128-row kernel that reads its tile list entry by entry: forward, 128-row query blocks and 64-key blocks, H24 S30720
 // 5.18 -> 4.83 ms, H8 S4096 48 -> 37 us.
 //
+// kFrom: tile lists, or block masks in small launches (takes_halves).
 // kRows: q_block is no multiple of 64, so the four 16-row groups of a half differ as well: a wave leaves out the matrix work
 // of chunks that neither of its groups selects, rows switched off inside an active wave are dealt with by selects.
 constexpr int kChunkBytes = 2 * kSlabBytes;  // 64 keys
 constexpr int kHalfRows = 64;
 constexpr int kHalfSlotBytes = (kHalfRows * kHeadDim + 2 * kHalfRows) * 4;  // partial result of one part of a split item
 constexpr int kHalfSmem = 5 * kChunkBytes;
-// Softmax reference of a row that has met no score yet.  Finite and below every score of use, so that exp2 never sees inf - inf
-// where all keys of a slab are masked out or have scores of -inf, also when only one of a row group's two waves meets others.
-// (Scores below it count for nothing; fp32 cannot tell such scores from their neighbours in any case.)
-constexpr float kNoReference = -1e30f;
+// Softmax reference of a row that has met no score yet.  Finite, so that exp2 never sees inf - inf where all keys of a slab are masked out or have scores of
+// -inf, also when only one of a row group's two waves meets others, and below every finite score that counts (a difference to it may be infinite: its exp2 is 0).
+constexpr float kNoReference = -3e38f;
 
-// The entries of a tile list that name one 64-row half, in order.  All lanes of a wave call everything together.
+// The entries of a tile list that name one 64-row half, in order; or the selected blocks of a mask row, which all name it.
+// All lanes of a wave call everything together.
+enum class From { kTiles, kMask };
+template <From kFrom>
 struct HalfList {
   const int32_t* list;
-  int cnt, half_mask, lane;
+  const uint8_t* row;
+  int cnt, half_mask, lane;  // cnt: entries; blocks of a mask row
   int head[4];               // this lane's entries among the first 256
   int base;                  // position of `entries` in the list
   int entries, ahead;        // this lane's entry among the 64 at `base` and the 64 behind them
   unsigned long long left;   // lanes whose entry names the half and has not been taken
 
-  FBA_DEVICE int load(int at) const { return at + lane < cnt ? list[at + lane] : 0; }
+  FBA_DEVICE int entry_at(int i) const {  // (within the row)
+    if constexpr (kFrom == From::kMask) return row[i] != 0 ? i << 8 | 255 : 0;
+    else return list[i];
+  }
+  FBA_DEVICE int load(int at) const { return at + lane < cnt ? entry_at(at + lane) : 0; }
   FBA_DEVICE unsigned long long named(int e) const { return __builtin_amdgcn_ballot_w64((e & half_mask) != 0); }
   // The head of the list, asked for before the count has come back (two round trips less in front of the first copy), and the count.
   FBA_DEVICE void read_head(int row_len, const int32_t* count) {
-    const int at_count = const_idx(count)[0];
+    const int at_count = kFrom == From::kMask ? row_len : const_idx(count)[0];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) head[i] = 64 * i + lane < row_len ? list[64 * i + lane] : 0;
+    for (int i = 0; i < 4; ++i) head[i] = 64 * i + lane < row_len ? entry_at(64 * i + lane) : 0;
     cnt = at_count;
 #pragma unroll
     for (int i = 0; i < 4; ++i) head[i] = 64 * i + lane < cnt ? head[i] : 0;
@@ -427,18 +435,23 @@ struct HalfList {
   }
 };
 
-template <bool kRows>
+template <bool kRows, From kFrom>
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2, 2))) void fwd_half_kernel(const FwdParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];  // K ring [3][16 KiB] | V ring [2][16 KiB]
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rg = wave & 1, par = wave >> 1;  // row group, 32-key slab of a chunk
+  if constexpr (kFrom == From::kMask) {
+    const int own_wgs = (int)gridDim.x - p.make.wgs;
+    if ((int)blockIdx.x >= own_wgs)
+      return compact_row(p.mask, p.mask_bh, p.nQ, p.nK, p.make.q_cnt, p.make.q_idx, p.make.k_cnt, p.make.k_idx, ((int)blockIdx.x - own_wgs) * 4 + wave);
+  }
   int item, part = 0, parts = 1;
   int ws_slot = (int)blockIdx.x - p.split.main_wgs;  // of a part's results
   if (ws_slot < 0) {
     item = xcd_remap(blockIdx.x, p.items_per_xcd);
     if (item >= p.split.first) return;
-  } else if (!split_position<Look::kSingle>(p.split, ws_slot, item, part, parts)) {
+  } else if (kFrom != From::kTiles || !split_position<Look::kSingle>(p.split, ws_slot, item, part, parts)) {
     return;
   }
   const int tiles_per_head = p.Sq / kHalfRows;
@@ -452,9 +465,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   const char* kp = reinterpret_cast<const char*>(p.k + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
   const char* vp = reinterpret_cast<const char*>(p.v + ((int64_t)(b * p.Hkv + hkv) * p.Skv) * kHeadDim);
 
-  const int64_t mrow = (p.mask_bh == 1 ? 0 : (int64_t)bh) * (p.Sq / 128) + (qt >> 1);
-  HalfList cursor;
+  const int64_t mrow = kFrom == From::kTiles ? (p.mask_bh == 1 ? 0 : (int64_t)bh) * (p.Sq / 128) + (qt >> 1) : (p.mask_bh == 1 ? 0 : (int64_t)bh) * p.nQ + qt * kHalfRows / p.q_block;
+  HalfList<kFrom> cursor;
   cursor.list = p.q_idx + mrow * p.nK;
+  cursor.row = p.mask + mrow * p.nK;
   cursor.half_mask = 15 << (4 * half);
   cursor.lane = lane;
   cursor.read_head(p.nK, p.q_cnt + mrow);
@@ -1134,6 +1148,18 @@ bool takes_rows(const FwdParams& p) {
   return p.q_block % 32 != 0 ? 4 * tiles >= 5 * units : p.q_block % 64 != 0 && tiles >= 4 * units;
 }
 
+// Does a block mask go to fwd_half_kernel, whole?  Where 128-row work-groups would leave half of the compute units without one, and parts, which fill them, pay
+// for their results and the merge: 64 rows at 64 keys a step take as long for a step as 128 rows at 32 keys, a work-group alone on its compute unit.  Long lists are
+// better off in more than two parts.  No gradients, 128-token blocks, 128 rows and parts / 64 rows, at 12, 35, 60 and 90 % kept: H6 S1408 (66 tiles) 9.4 / 6.6, 15.1 / 10.2,
+// 22.3 / 13.4 and 23.8 / 16.3 us; H3 S3456 (81) 13.1 / 8.9, 23.8 / 15.5, 27.9 / 22.5, 33.2 / 30.6; H3 S4736 (111) 15.9 / 10.8, 27.8 / 20.9, 35.3 / 29.6, 45.1 / 40.8; H6 S2688
+// (126) 13.8 / 12.4, 21.2 / 15.0, 28.8 / 20.8, 34.0 / 27.2.  Longer: H1 S8448 (66) 21.8 / 14.6, 30.6 / 30.0, 41.1 / 47.2, 49.1 / 66.7.  More tiles: H3 S5504 (129) 18.0 / 15.8,
+// 36.0 / 31.5, 45.9 / 47.2, 58.6 / 67.6, H6 S3072 (144) 11.6 / 15.2, 20.7 / 21.7, 32.0 / 30.5, 45.8 / 42.8.  Steps: H6 S1408 58.7 / 52.6, H5 S3200 96.3 / 87.5.
+bool takes_halves(const FwdParams& p) {
+  if (p.mask == nullptr) return false;
+  const int64_t tiles = (int64_t)p.B * p.Hq * (p.Sq / 128), units = device_compute_units();
+  return 2 * tiles <= units && p.Skv / kSlab <= (8 * tiles >= 3 * units ? 148 : 112);
+}
+
 }  // namespace
 
 // Tail splitting (two work-groups per compute unit); the 384-row kernel does without.
@@ -1152,11 +1178,11 @@ void plan_fwd(FwdParams& p) {
     group_parts(p.split, p.Hq / p.Hkv * (p.Sq / kHalfRows), 2LL * p.Skv * kRowBytes);
     return;
   }
-  const bool wide = p.q_block % 384 == 0 && p.variant != 1 && p.mask == nullptr;
-  const int rows = wide ? 384 : 128;
+  const bool wide = p.q_block % 384 == 0 && p.variant != 1 && p.mask == nullptr, halves = takes_halves(p);
+  const int rows = wide ? 384 : halves ? kHalfRows : 128;
   p.num_items = p.B * p.Hq * (p.Sq / rows);
   const ListLengths lengths{p.q_cnt, p.mask_bh == 1, rows, p.q_block, p.nQ, 1, p.k_block / kSlab, p.mask, p.nK};
-  p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, kFwdSlotBytes, wide ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
+  p.split = plan_split(p.num_items, 2, p.Skv / 32, StepCost{16, 22.5, 30}, kFwdSlotBytes, wide || halves ? nullptr : p.split.ws, p.split_ws_bytes, lengths);
   group_parts(p.split, p.Hq / p.Hkv * (p.Sq / rows), 2LL * p.Skv * kRowBytes);
 }
 
@@ -1164,7 +1190,7 @@ namespace {
 
 hipError_t launch_fwd_tiled(FwdParams p, hipStream_t stream) {
   const bool rows = takes_rows(p);
-  void (*fn)(const FwdParams) = rows ? &fwd_rows_kernel : p.q_block % 64 != 0 ? &fwd_half_kernel<true> : &fwd_half_kernel<false>;
+  void (*fn)(const FwdParams) = rows ? &fwd_rows_kernel : p.q_block % 64 != 0 ? &fwd_half_kernel<true, From::kTiles> : &fwd_half_kernel<false, From::kTiles>;
   const int smem = rows ? kRowsSmem : kHalfSmem, threads = rows ? 64 * kRowsWaves : 256;
   plan_fwd(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
@@ -1204,17 +1230,18 @@ hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream) {
 
 hipError_t launch_fwd(FwdParams p, hipStream_t stream) {
   if (p.tiled) return launch_fwd_tiled(p, stream);
-  const bool wide = p.q_block % 384 == 0 && p.variant != 1 && p.mask == nullptr;
-  const int smem = (wide ? 12 : 2 * kRing) * kSlabBytes;  // the rings; the results of twelve waves
-  void (*fn)(const FwdParams) = wide ? &fwd_kernel<12, false> : p.mask != nullptr ? &fwd_kernel<4, true> : &fwd_kernel<4, false>;
-  const int rows = wide ? 384 : 128;
+  const bool wide = p.q_block % 384 == 0 && p.variant != 1 && p.mask == nullptr, halves = takes_halves(p);
+  const int smem = halves ? kHalfSmem : (wide ? 12 : 2 * kRing) * kSlabBytes;  // the rings; the results of twelve waves
+  void (*fn)(const FwdParams) = halves ? &fwd_half_kernel<false, From::kMask>
+                                : wide ? &fwd_kernel<12, false> : p.mask != nullptr ? &fwd_kernel<4, true> : &fwd_kernel<4, false>;
+  const int threads = wide ? 768 : 256;
   plan_fwd(p);
   plan_xcd_mapping(p.B * p.Hq, p.split.first, p.items_per_xcd, p.split.main_wgs);
   const int split_wgs = (p.num_items - p.split.first) * p.split.parts;
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   if (e != hipSuccess) return e;
   p.make.wgs = p.make.q_cnt != nullptr ? (int)((p.mask_bh * (p.nQ + p.nK) + 3) / 4) : 0;
-  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs + p.make.wgs), dim3(rows * 2), smem, stream, p);
+  hipLaunchKernelGGL(fn, dim3(p.split.main_wgs + split_wgs + p.make.wgs), dim3(threads), smem, stream, p);
   if (split_wgs > 0) hipLaunchKernelGGL(fwd_merge_kernel<128>, dim3(merge_grid((p.num_items - p.split.first) * 16)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }

@@ -480,10 +480,11 @@ struct Attention : torch::autograd::Function<Attention> {
     }
     const Inputs in(q, k, v, mask, *s);
     const bool on_mask = takes_mask(s->p), with_lists = !on_mask && makes_lists(s->p, s->dense);
+    const bool on_blocks = with_lists || (takes_blocks(s->p) && s->p.B * s->p.Hq * s->p.Sq <= 128 * 128);  // where it may take 64-row work-groups
     build_lists(*s, mask, /*backward=*/true, /*numbered=*/!s->dense, /*launch=*/!with_lists);
-    auto [o, lse] = on_mask      ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask)
-                    : with_lists ? run_forward_on_blocks(s->p, in.q, in.k, in.v, in.mask, s->lists, s->split_bytes)
-                                 : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
+    auto [o, lse] = on_mask     ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask)
+                    : on_blocks ? run_forward_on_blocks(s->p, in.q, in.k, in.v, in.mask, with_lists ? s->lists : Lists(s->p), s->split_bytes)
+                                : run_forward(s->p, in.q, in.k, in.v, s->lists, s->split_bytes);
     ctx->save_for_backward({in.q, in.k, in.v, o, lse});
     // The rows that were appended are cut off here and not behind this function, where autograd would give back gradients for them in
     // two launches of its own, a fill and a copy (13 of 280 us at B2 H8/2 S3136).  What is handed out shares its version with

@@ -103,7 +103,8 @@ int32_t fba_fwd(const void* q, const void* k, const void* v, void* o, float* lse
 
 /*
  * fba_fwd on the lists of this block mask [mask_bh, nQ, nK], one byte per entry, nonzero = selected, without the lists.  At most 256 key blocks (otherwise
- * FBA_ERR_UNSUPPORTED).  How many ranges: by the lengths of 16 of its rows.
+ * FBA_ERR_UNSUPPORTED).  How many ranges: by the lengths of 16 of its rows; launches that leave half of the GPU without a 128-row tile work on 64
+ * rows, with the keys in two streams that meet at the end (fp32 sums in another order).
  *   q_cnt, q_idx, k_cnt, k_idx   null, or where the lists go that fba_mask_compact makes of the mask, for a backward pass: made in the same launch, of
  *                                mask_bh * (nQ + nK) <= 1024 rows
  */

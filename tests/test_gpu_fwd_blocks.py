@@ -1,6 +1,7 @@
 """Calls without gradients on whole 128-row blocks read the block mask where lists had at most 256 key blocks: rows of one block to 256, whole words of 64 and around, fewer
 than 16; the first and the last block, none, all; parts, and as many as by the lists; a shared mask, grouped heads; mask bytes other than one; 257 blocks, which go through
-lists.  Against forward on lists, bit for bit: rows of equal length, so that both decide alike on the parts.  And the
+lists.  Against forward on lists, bit for bit: rows of equal length, so that both decide alike on the parts; in
+small launches, which take 64-row work-groups, to what bf16 roundings come to.  And the
 lists that a step has it make in the same launch."""
 import pytest
 import torch
@@ -21,7 +22,20 @@ def _masks(kind, shape, g, gpu):
     return torch.zeros(shape, dtype=torch.bool, device=gpu).scatter_(-1, score.topk(keep, -1).indices, True)
 
 
+def halves(rows, kv_len):
+    """Does forward on a mask take 64-row work-groups?"""
+    return rows <= 128 * 128 and kv_len // 32 <= (148 if rows >= 96 * 128 else 112)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,nK,qbs,kbs,dims", [
+    (1, 65, 65, 128, 28, 128, 128, 4),    # 65 to 128 tiles: 64-row work-groups
+    (1, 6, 3, 1408, 11, 128, 128, 4),
+    (1, 3, 3, 4224, 11, 384, 384, 4),
+    (2, 8, 4, 1024, 1, 512, 512, 4),
+    (1, 4, 4, 3072, 37, 128, 128, 2),
+    (1, 2, 2, 8192, 8, 8192, 512, 4),
+    (1, 1, 1, 16384, 36, 128, 128, 4),
+    (1, 43, 43, 384, 3, 384, 1536, 4),    # 129
     (1, 70, 70, 128, 1, 128, 128, 4),
     (1, 70, 70, 128, 15, 128, 128, 4),
     (1, 9, 3, 1024, 16, 128, 128, 4),
@@ -50,7 +64,12 @@ def test_as_on_lists(gpu, B, Hq, Hkv, Sq, nK, qbs, kbs, dims, kind):
     assert not _lib.load().fba_fwd_takes_mask(B * Hq * Sq, nK * kbs)
     want = fba.forward_with_lists(q, k, v, qbs, kbs, fba.lists_for(m, qbs, kbs))[0]
     got = fba.flex_block_attn_func(q, k, v, qbs, kbs, m)
-    assert torch.equal(got, want)
+    if halves(B * Hq * Sq, nK * kbs):
+        # another kernel: either result is within 2.4e-3 (2-norm) of the exact one (P and O in bf16), and a block that is missed changes 64 rows by far more
+        a, b = (t.float().reshape(-1, 64 * 128) for t in (got, want))
+        assert bool(((a - b).norm(dim=1) <= 5e-3 * b.norm(dim=1)).all())
+    else:
+        assert torch.equal(got, want)
     if kind == "none":
         assert not bool(got.any())
 
@@ -90,7 +109,7 @@ def test_lists_on_the_way(gpu, B, Hq, Hkv, Sq, nK, qbs, kbs, dims):
     out = fba.flex_block_attn_func(*ins, qbs, kbs, m)
     grads = torch.autograd.grad(out, ins, do)
     if not _lib.load().fba_fwd_takes_mask(B * Hq * Sq, nK * kbs):
-        assert torch.equal(out, o)
+        assert torch.equal(out, o)  # the operator makes this very call
     for name, a, b in zip(("dq", "dk", "dv"), grads, fba.backward_with_lists(q, k, v, o, lse, do, qbs, kbs, want)):
         assert float((a.float() - b.float()).norm()) <= 1e-2 * float(b.float().norm()), name  # bf16 sums of another order, where the operator takes other kernels
 
@@ -113,7 +132,7 @@ def test_mask_bytes_and_limits(gpu):
     ws = torch.empty(_lib.load().fba_split_workspace_bytes(), dtype=torch.uint8, device=gpu)
     args = (*map(_ptr, (q, k, v, o, lse, m)), None, None, None, None, B * H, B, H, H, Sq, nK * 128, 128)
     _lib.call("fba_fwd_blocks", *args, 128, 128, _ptr(ws), ws.numel(), _stream())
-    assert torch.equal(o, want) and torch.equal(lse.flatten(), want_lse.flatten())
+    assert not halves(B * H * Sq, nK * 128) and torch.equal(o, want) and torch.equal(lse.flatten(), want_lse.flatten())
     with pytest.raises(_lib.FbaError):
         _lib.call("fba_fwd_blocks", *args, 64, 64, _ptr(ws), ws.numel(), _stream())
     with pytest.raises(_lib.FbaError, match="257 key blocks"):
