@@ -9,6 +9,7 @@
 // The library is not linked but bound by path (bind), so that FBA_LIBRARY can name another build of it.
 #include <dlfcn.h>
 
+#include <cstdlib>
 #include <numeric>
 
 #include <ATen/ATen.h>
@@ -200,8 +201,12 @@ std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor
   return {o, lse};
 }
 
-// The same on the block mask, where fba_fwd_blocks takes it.
-bool takes_blocks(const Problem& p) { return !p.tiled() && p.nK() <= 256; }
+// The same on the block mask, where fba_fwd_blocks takes it.  The 384-row work-groups that FBA_FWD_TILE_ROWS asks for read lists.
+bool takes_blocks(const Problem& p) {
+  if (p.tiled() || p.nK() > 256) return false;
+  const char* const rows = p.q_block % 384 == 0 ? std::getenv("FBA_FWD_TILE_ROWS") : nullptr;
+  return rows == nullptr || std::atoi(rows) != 384;
+}
 // Is it to make the lists of a step on the way?  Steps that number their pairs need them before forward is through (the host waits for the count);
 // with more rows than that the lists would hold up the launch, whose last work-groups make them.
 bool makes_lists(const Problem& p, bool dense) { return dense && takes_blocks(p) && p.mask_bh * (p.nQ() + p.nK()) <= 1024; }

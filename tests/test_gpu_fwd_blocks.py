@@ -140,3 +140,18 @@ def test_mask_bytes_and_limits(gpu):
     lists = [torch.empty(1, dtype=torch.int32, device=gpu) for _ in range(4)]  # (refused before anything is written)
     with pytest.raises(_lib.FbaError, match="1024 rows"):
         _lib.call("fba_fwd_blocks", *map(_ptr, (q, k, v, o, lse, m, *lists)), 22 * B * H, 22 * B, H, H, Sq, nK * 128, 128, 128, 128, _ptr(ws), ws.numel(), _stream())
+
+
+@pytest.mark.parametrize("step", [False, True])
+def test_with_384_row_work_groups_asked_for(gpu, monkeypatch, step):
+    """FBA_FWD_TILE_ROWS=384 is for 384-row work-groups, which read lists: the same bits as on lists, in a launch that would take 64-row work-groups (others)."""
+    import flex_block_attn_amd as fba
+
+    g = torch.Generator(device=gpu).manual_seed(384)
+    q, k, v = (torch.randn((1, 6, 1536, 128), generator=g, device=gpu).to(torch.bfloat16) for _ in range(3))
+    m = _masks(0.6, (1, 6, 4, 4), g, gpu)
+    assert halves(6 * 1536, 1536)
+    monkeypatch.setenv("FBA_FWD_TILE_ROWS", "384")
+    want, _ = fba.forward_with_lists(q, k, v, 384, 384, fba.lists_for(m, 384, 384))
+    got = fba.flex_block_attn_func(q.requires_grad_(step), k, v, 384, 384, m)
+    assert torch.equal(got, want)
