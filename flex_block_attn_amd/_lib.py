@@ -32,6 +32,7 @@ SIGNATURES = {
     "fba_mask_compact": (_c_i32, [_c_ptr, _c_i64, _c_i32, _c_i32, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr]),
     "fba_split_workspace_bytes": (_c_i64, []),
     "fba_split_plan": (_c_i32, [_c_i32, _c_i64] + [_c_i32] * 8 + [_c_i64, _c_ptr]),
+    "fba_split_regions": (_c_i32, [_c_i32, _c_i32, _c_i64] + [_c_i32] * 8 + [_c_i64, _c_ptr]),
     "fba_fwd": (_c_i32, [_c_ptr] * 7 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_fwd_blocks": (_c_i32, [_c_ptr] * 10 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_fwd_mask": (_c_i32, [_c_ptr] * 6 + [_c_i64] + [_c_i32] * 8 + [_c_ptr]),
@@ -72,7 +73,7 @@ SIGNATURES = {
 }
 
 # fba_version() of the library these signatures describe (include/fba.h; bumped whenever an argument list changes)
-ABI_VERSION = 2009
+ABI_VERSION = 2010
 
 _lib = None
 _host = None

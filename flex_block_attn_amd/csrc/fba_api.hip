@@ -396,6 +396,25 @@ int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, i
   return FBA_OK;
 }
 
+int32_t fba_split_regions(int32_t units, int32_t from_ds, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim,
+                          int32_t q_block, int32_t k_block, int64_t split_ws_bytes, int64_t* regions) {
+  const Shape s{mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block};
+  if (int rc = check_shape(s)) return rc;
+  if (regions == nullptr || split_ws_bytes <= 0 || units < 0) return fail(FBA_ERR_INVALID, "null regions, no workspace or negative units");
+  const bool tiled = q_block % 128 != 0 || k_block % 128 != 0;
+  if (int rc = check_lists(s, tiled, "split_regions")) return rc;
+  const fba::AssumedUnits assumed(units);
+  fba::BwdParams b{};
+  fill_bwd(b, s);
+  b.tiled = tiled ? 1 : 0;
+  b.q_cnt = b.k_cnt = reinterpret_cast<const int32_t*>(16);  // addresses that are only compared with null and subtracted from each other
+  b.split.ws = reinterpret_cast<float*>(16); b.split_ws_bytes = split_ws_bytes;
+  b.make.stats = reinterpret_cast<float*>(16);
+  const fba::SplitRegions r = fba::plan_split_regions(b, from_ds != 0);
+  regions[0] = r.parts_end; regions[1] = r.pieces_end; regions[2] = r.dq_from; regions[3] = r.dq_end; regions[4] = r.kept_from;
+  return FBA_OK;
+}
+
 int32_t fba_bwd_stats(const void* o, const void* d_o, const float* lse, float* stats, int64_t rows, int32_t head_dim,
                       void* hip_stream) {
   if (head_dim != 128) return fail(FBA_ERR_INVALID, "head_dim must be 128, got %d", head_dim);

@@ -491,15 +491,10 @@ hipError_t launch_merge(const Merge& m, hipStream_t stream) {
 
 hipError_t take_along(SplitPlan& split, int64_t slot_bytes, Merge& before, hipStream_t stream) {
   if (before.wgs == 0) return hipSuccess;
-  if (split.items > 0) {
-    const int64_t end = before.results_end + split.items * split.parts * slot_bytes + (int64_t)sizeof(int32_t);
-    if (end > before.kept_from) {
-      const hipError_t e = launch_merge(before, stream);
-      before = {};
-      return e;
-    }
-    split.ws += before.results_end / 4;
-    split.note += before.results_end / 4;
+  if (!put_behind(split, slot_bytes, before)) {
+    const hipError_t e = launch_merge(before, stream);
+    before = {};
+    return e;
   }
   before.wgs = std::min(before.wgs, 128 * before.n_outs);  // a work-group or so to a compute unit, while others work on dQ
   return hipSuccess;

@@ -357,11 +357,24 @@ hipError_t launch_bwd_dq_from_ds(BwdParams p, hipStream_t stream, Merge before =
 // among it.
 hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream, bool takes_pieces = false);
 int device_compute_units();
+// For plans without a device: as long as it lives, this thread plans for so many compute units (0: those there are).
+struct AssumedUnits {
+  explicit AssumedUnits(int units);
+  ~AssumedUnits();
+  AssumedUnits(const AssumedUnits&) = delete;
+  const int before;
+};
 // Merges parts in a launch of its own, or of dK/dV with `later` set leaves that to the dQ launch (see Merge).
 hipError_t launch_merge(const Merge& m, hipStream_t stream);
 // For a dQ launch with the plan `split`, whose parts store `slot_bytes` each: it takes `before` along, with the results of its own parts behind
 // those that are still to be merged, or where they do not fit there `before` is launched now and cleared.
 hipError_t take_along(SplitPlan& split, int64_t slot_bytes, Merge& before, hipStream_t stream);
+bool put_behind(SplitPlan& split, int64_t slot_bytes, const Merge& before);  // false where they do not fit
+// Where a whole backward pass with p.split.ws keeps what (fba_split_regions in include/fba.h).
+struct SplitRegions {
+  int64_t parts_end, pieces_end, dq_from, dq_end, kept_from;
+};
+SplitRegions plan_split_regions(BwdParams p, bool from_ds);
 hipError_t launch_probe_mfma(const float* src, float* sink, int work_groups, int iters, hipStream_t stream);
 hipError_t launch_probe_read(const void* src, int64_t bytes, uint32_t* sink, int work_groups, hipStream_t stream);
 hipError_t launch_pair_slots(const int32_t* q_cnt, const int32_t* q_idx, const int32_t* k_cnt, const int32_t* k_idx, int64_t mask_bh,

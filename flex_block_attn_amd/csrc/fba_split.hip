@@ -11,8 +11,11 @@ namespace fba {
 
 namespace {
 
+thread_local int assumed_units = 0;  // see AssumedUnits
+
 // Compute units of the current device (looked up once per device).
 int compute_units() {
+  if (assumed_units > 0) return assumed_units;
   constexpr int kMaxDevices = 64;
   static std::mutex mu;
   static int cache[kMaxDevices] = {};
@@ -29,6 +32,9 @@ int compute_units() {
 }  // namespace
 
 int device_compute_units() { return compute_units(); }
+
+AssumedUnits::AssumedUnits(int units) : before(assumed_units) { assumed_units = units; }
+AssumedUnits::~AssumedUnits() { assumed_units = before; }
 
 // The hardware hands work-groups to free slots in index order.  With n items on s slots the last n % s items form a
 // partial round; the lists of these items are cut into parts (at most 8) where parts fill the slots better.  Launches smaller than the
@@ -474,7 +480,18 @@ void plan_bwd_dkdv(BwdParams& p, const KeyTiles& tiles) {
                        lengths);
 }
 
-hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream, bool takes_pieces) {
+namespace {
+
+// A dK/dV launch as it is planned: work-groups, and what has to run in front of it.
+struct KeyTileLaunch {
+  int grid = 0;
+  ItemOrder make{};
+  PieceMaker maker{};
+};
+
+KeyTileLaunch place_key_tiles(BwdParams& p, const KeyTiles& tiles, bool takes_pieces) {
+  KeyTileLaunch launch;
+  auto& [grid, make, maker] = launch;
   const int slots = compute_units();
   const int heads = p.B * p.Hkv;
   char* const ws = reinterpret_cast<char*>(p.split.ws);  // whether or not anything is split
@@ -511,7 +528,6 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
   // count.  A launch that needs none pays for work-groups that exit at once, one to a compute unit, and for a merge that finds nothing to do (5 us in
   // a trace): steps with / without pieces in the library, B2 H16/4 S8192 1033 / 1031 us, H8 S8192 290 / 288, H4 S16384 5 % kept 163 / 161, H1 S32768 10 % 268 / 267,
   // H2 S32768 30 % 1276 / 1274.  The planning hides behind the statistics, so a dK/dV kernel called by itself goes without.
-  PieceMaker maker{};
   const int most_pieces = p.num_items <= slots ? slots : p.num_items + slots;
   const int64_t piece_bytes = 64 + most_pieces * (int64_t)sizeof(Piece) + slots * (int64_t)sizeof(CutItem);
   top = (top - piece_bytes) & ~(int64_t)63;
@@ -522,7 +538,8 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
              2 * slots, most_pieces, p.split.items == p.num_items ? p.split.parts : 1};
     p.pieces = {maker.header, maker.list, maker.cut};
     p.split.ws = reinterpret_cast<float*>(ws);
-    p.results_end = 2 * slots * tiles.slot_bytes;
+    // The device may decide against pieces, and then makes the parts that the host has planned: whichever end later.
+    p.results_end = std::max(p.results_end, 2 * slots * tiles.slot_bytes);
   }
   p.kept_from = maker.header != nullptr ? top : ordered ? order_at : queue != nullptr ? reinterpret_cast<char*>(queue) - ws : p.split_ws_bytes;
 
@@ -537,7 +554,6 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
     p.queue = queue;
     grid += (p.total_work / 8 + 7) / 8 * 8;  // an eighth more work-groups, a whole number per XCD
   }
-  ItemOrder make{};
   if (ordered) {
     const int tiles_per_head = p.Skv / tiles.rows;
     make.spans = heads >= 8 ? 8 : 1;
@@ -548,9 +564,51 @@ hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStr
     p.order = make.order;
     if (2 * p.split.items <= slots) p.split.look.order = p.order;
   }
+  return launch;
+}
+
+}  // namespace
+
+hipError_t plan_key_tiles(BwdParams& p, const KeyTiles& tiles, int& grid, hipStream_t stream, bool takes_pieces) {
+  const auto [work_groups, make, maker] = place_key_tiles(p, tiles, takes_pieces);
+  grid = work_groups;
   const int front = (maker.header != nullptr) + make.blocks + (p.make.stats != nullptr ? stats_blocks(p.make) : p.queue != nullptr ? 1 : 0);
   if (front > 0) hipLaunchKernelGGL(bwd_front_kernel, dim3(front), dim3(kFrontThreads), 0, stream, p, make, maker);
   return hipGetLastError();
+}
+
+bool put_behind(SplitPlan& split, int64_t slot_bytes, const Merge& before) {
+  if (split.items == 0) return true;
+  const int64_t end = before.results_end + split.items * split.parts * slot_bytes + (int64_t)sizeof(int32_t);
+  if (end > before.kept_from) return false;
+  split.ws += before.results_end / 4;
+  split.note += before.results_end / 4;
+  return true;
+}
+
+SplitRegions plan_split_regions(BwdParams p, bool from_ds) {
+  SplitRegions r{0, 0, -1, -1, p.split_ws_bytes};
+  float* const ws = p.split.ws;
+  BwdParams dq = p;
+  const KeyTiles& tiles = p.tiled ? kKeyTiles64 : kKeyTiles128;
+  place_key_tiles(p, tiles, /*takes_pieces=*/!p.tiled);
+  Merge before;
+  if (p.split.items > 0) r.parts_end = p.split.items * p.split.parts * tiles.slot_bytes + (int64_t)sizeof(int32_t);
+  if (p.pieces.header != nullptr) r.pieces_end = 2 * compute_units() * tiles.slot_bytes;
+  if (r.parts_end > 0 || r.pieces_end > 0) {
+    before.wgs = 1;
+    before.results_end = p.results_end;
+    r.kept_from = before.kept_from = p.kept_from;
+  }
+  int rows = 128;
+  if (from_ds) rows = 32 * plan_bwd_dq_from_ds(dq);
+  else plan_bwd_dq(dq);
+  const int64_t slot_bytes = rows * kHeadDim * 4;
+  if (dq.split.items > 0 && before.wgs > 0 && put_behind(dq.split, slot_bytes, before)) {
+    r.dq_from = reinterpret_cast<char*>(dq.split.ws) - reinterpret_cast<char*>(ws);
+    r.dq_end = std::max(r.dq_from + dq.split.items * dq.split.parts * slot_bytes, reinterpret_cast<char*>(dq.split.note + 1) - reinterpret_cast<char*>(ws));
+  }
+  return r;
 }
 
 }  // namespace fba

@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2009
+#define FBA_VERSION 2010
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -89,6 +89,15 @@ int64_t fba_split_workspace_bytes(void);
  */
 int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim,
                        int32_t q_block, int32_t k_block, int64_t split_ws_bytes, int64_t* plan);
+/*
+ * Where a whole backward pass on such sizes keeps what in split_ws, for tests (no GPU needed).  units: compute units (0: those of the device, or 256);
+ * from_ds: dQ from dS, or 0 for dQ that recomputes S and dP.  regions [5], bytes:
+ *   0 end of dK/dV's ranges and of the int32 behind them (0: none)   1 end of its pieces, which the device may make instead (0: none)
+ *   2, 3 dQ's ranges and the int32 behind them, while those of dK/dV are still to be summed (-1: it has none, or those of dK/dV are summed first)
+ *   4 what lies from here on stays as it is until those of dK/dV are summed
+ */
+int32_t fba_split_regions(int32_t units, int32_t from_ds, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim,
+                          int32_t q_block, int32_t k_block, int64_t split_ws_bytes, int64_t* regions);
 
 /*
  * Forward.  Replaces attn_forward (attn.cpp:29, flex_block_attn_h100.cu:810-1007; kernel :52-318).
