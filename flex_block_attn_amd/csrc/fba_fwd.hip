@@ -17,6 +17,7 @@
 // buffers of K_{t+1} and V_{t-1} are dead and receive K_{t+5} and V_{t+3}, i.e. every slab is requested four steps
 // before its first use.  One barrier per step orders all LDS traffic; before it each wave waits until its own copies
 // of the slabs needed next have landed (all but the two youngest batches of four).
+#include <algorithm>
 #include <type_traits>
 
 #include "fba_common.h"
@@ -1139,13 +1140,19 @@ namespace {
 // bring in chunks that any of the 128 rows selects; fwd_half_kernel works on 32 rows and 64.  No gradients, fwd_half_kernel / fwd_rows_kernel, 64-token key
 // blocks, 12, 25 and 50 % kept (chunks of a compute unit alone in a launch of few work-groups come slowly, so those stay):
 //   16-row blocks: 256 tiles (H8 S4096) 35.4 / 43.5, 55.2 / 60.9, 78.1 / 78.1 us; 320 (H10 S4096) 50.4 / 50.5, 74.7 / 71.4, 102.2 / 93.3; 512 (H16
-//     S4096) 62.6 / 51.0, 101 / 72.5, 147 / 101; 704 (H22 S4096) 86.4 / 84.4, 141 / 119, 208 / 161; at 90 % 320 tiles 116 / 122, 704 240 / 214.
+//     S4096) 62.6 / 51.0, 101 / 72.5, 147 / 101; 704 (H22 S4096) 86.4 / 84.4, 141 / 119, 208 / 161; at 90 % 704 240 / 214.  Launches of 64-row work-groups that
+//     are little more than a round cut long lists into parts, so the line rises with the keys.  15 (320 tiles: 12), 60 and 90 % kept: 320 tiles, 2048 keys 35.4 / 33.0,
+//     67.7 / 57.1, 72.0 / 67.6, 4096 keys 50.6 / 51.4, 104.9 / 100.8, 112.2 / 122.8, 8192 keys 77.8 / 84.6, 193 / 190, 207 / 233; 336 tiles, 4096 keys 62.0 / 57.7,
+//     123 / 102, 132 / 124, 5120 keys 76.6 / 67.9, 137 / 125, 146 / 151; 344 tiles, 8192 keys 105 / 100, 221 / 191, 236 / 234, 30720 keys 378 / 380, 799 / 693, 877 / 852.
 //   32-row blocks: 320 tiles 39.3 / 39.5, 54.2 / 59.8, 78.8 / 88.8 us; 704 57.4 / 62.3, 92.0 / 97.4, 154 / 153; 1080 (H9 S15360) 245 / 237, 437 / 409, 772 / 682;
-//     2880 (H24 S15360) 652 / 634, 1147 / 1112, 2027 / 1894.
+//     2880 (H24 S15360) 652 / 634, 1147 / 1112, 2027 / 1894.  Two and a half rounds of long lists with little kept are the worst case: H10 S16384, 6, 12 and 18 %
+//     159 / 167, 283 / 289, 391 / 391.
 //   64-row blocks: H24 S30720, 40 % kept 4.54 / 5.10 ms.
 bool takes_rows(const FwdParams& p) {
   const int64_t tiles = (int64_t)p.B * p.Hq * (p.Sq / kRowsTile), units = device_compute_units();
-  return p.q_block % 32 != 0 ? 4 * tiles >= 5 * units : p.q_block % 64 != 0 && tiles >= 4 * units;
+  if (p.q_block % 32 == 0) return p.q_block % 64 != 0 && tiles >= 4 * units;
+  const int thousands = std::min(std::max((p.Skv + 1023) / 1024, 2), 5);  // of keys
+  return 32 * tiles >= (38 + thousands) * units;  // 320, 328, 336 and 344 tiles where there are 256 compute units
 }
 
 // Does a block mask go to fwd_half_kernel, whole?  Where 128-row work-groups would leave half of the compute units without one, and parts, which fill them, pay
