@@ -35,6 +35,7 @@ SIGNATURES = {
     "fba_split_regions": (_c_i32, [_c_i32, _c_i32, _c_i64] + [_c_i32] * 8 + [_c_i64, _c_ptr]),
     "fba_fwd": (_c_i32, [_c_ptr] * 7 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
     "fba_fwd_blocks": (_c_i32, [_c_ptr] * 10 + [_c_i64] + [_c_i32] * 8 + [_c_ptr, _c_i64, _c_ptr]),
+    "fba_fwd_blocks_use": (_c_i32, [_c_i64] + [_c_i32] * 6),
     "fba_fwd_mask": (_c_i32, [_c_ptr] * 6 + [_c_i64] + [_c_i32] * 8 + [_c_ptr]),
     "fba_fwd_mask_copy": (_c_i32, [_c_ptr] * 7 + [_c_i32, _c_i64] + [_c_i32] * 8 + [_c_ptr]),
     "fba_fwd_takes_mask": (_c_i32, [_c_i64, _c_i32]),
@@ -73,7 +74,7 @@ SIGNATURES = {
 }
 
 # fba_version() of the library these signatures describe (include/fba.h; bumped whenever an argument list changes)
-ABI_VERSION = 2010
+ABI_VERSION = 2011
 
 _lib = None
 _host = None

@@ -171,12 +171,19 @@ int32_t fba_fwd_blocks(const void* q, const void* k, const void* v, void* o, flo
   if (!mask) return fail(FBA_ERR_INVALID, "null pointer argument");
   const bool make = q_cnt || q_idx || k_cnt || k_idx;
   if (make && (!q_cnt || !q_idx || !k_cnt || !k_idx)) return fail(FBA_ERR_INVALID, "forward: all four lists, or none");
-  if (make && q_block > 0 && k_block > 0 && mask_bh * (Sq / q_block + Skv / k_block) > fba::kMakeRows)
+  if (make && q_block > 0 && k_block > 0 && mask_bh * ((int64_t)Sq / q_block + Skv / k_block) > fba::kMakeRows)
     return fail(FBA_ERR_UNSUPPORTED, "forward: more than %d rows of lists; build them with fba_mask_compact", fba::kMakeRows);
   if (k_block > 0 && Skv / k_block > fba::kMaskBlocks)
     return fail(FBA_ERR_UNSUPPORTED, "forward: %d key blocks are more than %d; build lists with fba_mask_compact and call fba_fwd", Skv / k_block, fba::kMaskBlocks);
   return fwd_impl(q, k, v, o, lse, nullptr, nullptr, mask, mask_bh, B, Hq, Hkv, Sq, Skv, head_dim, q_block, k_block, split_ws, split_ws_bytes, hip_stream, false,
                   {q_cnt, q_idx, k_cnt, k_idx, 0});
+}
+
+int32_t fba_fwd_blocks_use(int64_t mask_bh, int32_t B, int32_t Hq, int32_t Sq, int32_t Skv, int32_t q_block, int32_t k_block) {
+  if (mask_bh <= 0 || B <= 0 || Hq <= 0 || Sq <= 0 || Skv <= 0 || q_block <= 0 || k_block <= 0) return 0;
+  if (q_block % 128 != 0 || k_block % 128 != 0 || Skv / k_block > fba::kMaskBlocks) return 0;
+  const bool lists = mask_bh * ((int64_t)Sq / q_block + Skv / k_block) <= fba::kMakeRows;
+  return FBA_BLOCKS_TAKEN | (lists ? FBA_BLOCKS_LISTS : 0) | (fba::fwd_takes_halves((int64_t)B * Hq * Sq, Skv) ? FBA_BLOCKS_HALVES : 0);
 }
 
 int32_t fba_fwd_mask_copy(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, uint8_t* mask_copy, int32_t o_rows,

@@ -1161,13 +1161,14 @@ bool takes_rows(const FwdParams& p) {
 // 22.3 / 13.4 and 23.8 / 16.3 us; H3 S3456 (81) 13.1 / 8.9, 23.8 / 15.5, 27.9 / 22.5, 33.2 / 30.6; H3 S4736 (111) 15.9 / 10.8, 27.8 / 20.9, 35.3 / 29.6, 45.1 / 40.8; H6 S2688
 // (126) 13.8 / 12.4, 21.2 / 15.0, 28.8 / 20.8, 34.0 / 27.2.  Longer: H1 S8448 (66) 21.8 / 14.6, 30.6 / 30.0, 41.1 / 47.2, 49.1 / 66.7.  More tiles: H3 S5504 (129) 18.0 / 15.8,
 // 36.0 / 31.5, 45.9 / 47.2, 58.6 / 67.6, H6 S3072 (144) 11.6 / 15.2, 20.7 / 21.7, 32.0 / 30.5, 45.8 / 42.8.  Steps: H6 S1408 58.7 / 52.6, H5 S3200 96.3 / 87.5.
-bool takes_halves(const FwdParams& p) {
-  if (p.mask == nullptr) return false;
-  const int64_t tiles = (int64_t)p.B * p.Hq * (p.Sq / 128), units = device_compute_units();
-  return 2 * tiles <= units && p.Skv / kSlab <= (8 * tiles >= 3 * units ? 148 : 112);
-}
+bool takes_halves(const FwdParams& p) { return p.mask != nullptr && fwd_takes_halves((int64_t)p.B * p.Hq * p.Sq, p.Skv); }
 
 }  // namespace
+
+bool fwd_takes_halves(int64_t rows, int64_t kv_len) {
+  const int64_t tiles = rows / 128, units = device_compute_units();
+  return 2 * tiles <= units && kv_len / kSlab <= (8 * tiles >= 3 * units ? 148 : 112);
+}
 
 // Tail splitting (two work-groups per compute unit); the 384-row kernel does without.
 void plan_fwd(FwdParams& p) {

@@ -343,6 +343,7 @@ constexpr int kMaskBlocks = 256, kMakeRows = 1024;  // of lists that forward mak
 hipError_t launch_fwd(FwdParams p, hipStream_t stream);
 hipError_t launch_fwd_mask(FwdMaskParams p, hipStream_t stream);
 bool fwd_takes_mask(int64_t rows, int64_t kv_len);
+bool fwd_takes_halves(int64_t rows, int64_t kv_len);  // of block masks in fwd_half_kernel; rows: of 128-row tiles
 hipError_t launch_bwd_mask(BwdMaskParams p, hipStream_t stream);
 bool bwd_takes_mask(int64_t heads, int64_t kv_heads, int64_t q_len, int64_t kv_len);
 hipError_t launch_bwd_stats(const BwdStats& s, hipStream_t stream);

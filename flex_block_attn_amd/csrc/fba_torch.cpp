@@ -41,7 +41,7 @@ constexpr int64_t kXcds = 8;
 // ---------------------------------------------------------------------------------------------------------------------
 #define FBA_FUNCTIONS(X)                                                                                                \
   X(fba_version) X(fba_last_error) X(fba_split_workspace_bytes) X(fba_lists_cut) X(fba_pair_slots_bounds) X(fba_tile_slots_bounds)        \
-  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_blocks) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_handover) X(fba_bwd_tiled_cut) X(fba_bwd_dense) \
+  X(fba_fwd) X(fba_fwd_tiled) X(fba_fwd_blocks) X(fba_fwd_blocks_use) X(fba_fwd_mask_copy) X(fba_fwd_takes_mask) X(fba_bwd_mask) X(fba_bwd_takes_mask) X(fba_bwd) X(fba_bwd_handover) X(fba_bwd_tiled_cut) X(fba_bwd_dense) \
   X(fba_resize_rows) X(fba_resize_mask)
 
 struct Library {
@@ -202,14 +202,11 @@ std::pair<at::Tensor, at::Tensor> run_forward(const Problem& p, const at::Tensor
 }
 
 // The same on the block mask, where fba_fwd_blocks takes it.  The 384-row work-groups that FBA_FWD_TILE_ROWS asks for read lists.
-bool takes_blocks(const Problem& p) {
-  if (p.tiled() || p.nK() > 256) return false;
-  const char* const rows = p.q_block % 384 == 0 ? std::getenv("FBA_FWD_TILE_ROWS") : nullptr;
-  return rows == nullptr || std::atoi(rows) != 384;
+int blocks_use(const Problem& p) {
+  const int use = lib.fba_fwd_blocks_use(p.mask_bh, p.B, p.Hq, p.Sq, p.Skv, p.q_block, p.k_block);
+  const char* const rows = use != 0 && p.q_block % 384 == 0 ? std::getenv("FBA_FWD_TILE_ROWS") : nullptr;
+  return rows == nullptr || std::atoi(rows) != 384 ? use : 0;
 }
-// Is it to make the lists of a step on the way?  Steps that number their pairs need them before forward is through (the host waits for the count);
-// with more rows than that the lists would hold up the launch, whose last work-groups make them.
-bool makes_lists(const Problem& p, bool dense) { return dense && takes_blocks(p) && p.mask_bh * (p.nQ() + p.nK()) <= 1024; }
 std::pair<at::Tensor, at::Tensor> run_forward_on_blocks(const Problem& p, const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, const at::Tensor& mask,
                                                         const Lists& make, int64_t split_bytes) {
   at::Tensor o = at::empty_like(q);
@@ -484,10 +481,13 @@ struct Attention : torch::autograd::Function<Attention> {
       return cut ? o.narrow(2, 0, q_len).detach() : o;
     }
     const Inputs in(q, k, v, mask, *s);
-    const bool on_mask = takes_mask(s->p), with_lists = !on_mask && makes_lists(s->p, s->dense);
-    // Lists that are there anyway: from the mask only where forward may take 64-row work-groups, few rows and short lists.  With longer ones it has nothing
+    // Forward makes the lists of a step on the way where it can.  Steps that number their pairs need them before forward is through (the host waits for the
+    // count); with many rows the lists would hold up the launch, whose last work-groups make them.
+    // Lists that are there anyway: from the mask only where forward takes 64-row work-groups on it.  Otherwise it has nothing
     // to gain from the mask (B1 H8/2 128 x 17920, 128-token blocks, 102 of 140 kept: forward 33.8 us on lists, 34.9 on the mask).
-    const bool on_blocks = with_lists || (takes_blocks(s->p) && s->p.B * s->p.Hq * s->p.Sq <= 128 * 128 && s->p.Skv <= 148 * 32);
+    const bool on_mask = takes_mask(s->p);
+    const int use = on_mask ? 0 : blocks_use(s->p);
+    const bool with_lists = s->dense && (use & FBA_BLOCKS_LISTS) != 0, on_blocks = with_lists || (use & FBA_BLOCKS_HALVES) != 0;
     build_lists(*s, mask, /*backward=*/true, /*numbered=*/!s->dense, /*launch=*/!with_lists);
     auto [o, lse] = on_mask     ? run_forward_on_mask(s->p, in.q, in.k, in.v, in.mask)
                     : on_blocks ? run_forward_on_blocks(s->p, in.q, in.k, in.v, in.mask, with_lists ? s->lists : Lists(s->p), s->split_bytes)
@@ -569,7 +569,7 @@ c10::optional<at::Tensor> attention(const at::Tensor& q, const at::Tensor& k, co
   const bool backward = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
   if (!backward) {
     if (takes_mask(p)) return run_forward_on_mask(p, q, k, v, mask).first;
-    if (takes_blocks(p)) return run_forward_on_blocks(p, q, k, v, mask, Lists(p), split_bytes).first;
+    if (blocks_use(p) != 0) return run_forward_on_blocks(p, q, k, v, mask, Lists(p), split_bytes).first;
     const Inputs in(q, k, v, mask, *s);
     build_lists(*s, mask, false, false);
     const at::Tensor o = run_forward(p, in.q, in.k, in.v, s->lists, split_bytes).first;

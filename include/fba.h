@@ -36,7 +36,7 @@ extern "C" {
 
 /* Library version: major * 1000 + minor; the minor number goes up whenever an argument list in this header changes, so a
  * binding can refuse a library built from another header (flex_block_attn_amd/_lib.py does). */
-#define FBA_VERSION 2010
+#define FBA_VERSION 2011
 int32_t fba_version(void);
 
 /* Message for the last non-OK return on the calling thread ("" if none). The pointer stays valid until the next
@@ -120,6 +120,12 @@ int32_t fba_fwd(const void* q, const void* k, const void* v, void* o, float* lse
 int32_t fba_fwd_blocks(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* mask, int32_t* q_cnt, int32_t* q_idx, int32_t* k_cnt,
                        int32_t* k_idx, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim, int32_t q_block,
                        int32_t k_block, void* split_ws, int64_t split_ws_bytes, void* hip_stream);
+/* What it does for these sizes on the current device (256 compute units are assumed without one): 0 where it does not take them, else TAKEN, and LISTS where it also makes
+ * the lists, HALVES where it works on 64 rows. */
+#define FBA_BLOCKS_TAKEN 1
+#define FBA_BLOCKS_LISTS 2
+#define FBA_BLOCKS_HALVES 4
+int32_t fba_fwd_blocks_use(int64_t mask_bh, int32_t B, int32_t Hq, int32_t Sq, int32_t Skv, int32_t q_block, int32_t k_block);
 
 /*
  * Forward straight from the block mask, in one launch and without a workspace: for problems too small to fill the GPU, where lists
