@@ -370,12 +370,17 @@ int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, i
   b.q_cnt = b.k_cnt = cnt;
   b.split.ws = ws; b.split_ws_bytes = split_ws_bytes;
   switch (launch) {
+    case 4:
+      if (fba_fwd_blocks_use(mask_bh, B, Hq, Sq, Skv, q_block, k_block) == 0) return fail(FBA_ERR_UNSUPPORTED, "split_plan: fba_fwd_blocks does not take such sizes");
+      [[fallthrough]];
     case 0: {
       fba::FwdParams f{};
       f.mask_bh = mask_bh;
       f.B = B; f.Hq = Hq; f.Hkv = Hkv; f.Sq = Sq; f.Skv = Skv; f.nQ = b.nQ; f.nK = b.nK;
       f.q_block = q_block; f.k_block = k_block;
-      f.q_cnt = cnt; f.tiled = b.tiled; f.variant = 1;
+      if (launch == 0) f.q_cnt = cnt;
+      else f.mask = reinterpret_cast<const uint8_t*>(cnt);
+      f.tiled = b.tiled; f.variant = 1;
       f.split = b.split; f.split_ws_bytes = split_ws_bytes;
       fba::plan_fwd(f);
       b.num_items = f.num_items;
@@ -385,7 +390,7 @@ int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, i
     case 1: fba::plan_bwd_dkdv(b, tiled ? fba::kKeyTiles64 : fba::kKeyTiles128); break;
     case 2: fba::plan_bwd_dq(b); break;
     case 3: fba::plan_bwd_dq_from_ds(b); break;
-    default: return fail(FBA_ERR_INVALID, "launch must be 0 to 3, got %d", launch);
+    default: return fail(FBA_ERR_INVALID, "launch must be 0 to 4, got %d", launch);
   }
   const fba::SplitPlan& sp = b.split;
   const bool split = sp.first < b.num_items;
@@ -393,7 +398,7 @@ int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, i
   plan[1] = sp.first;
   plan[2] = sp.parts;
   const fba::ListLook& l = sp.look;
-  const bool looks = split && l.cnt != nullptr;
+  const bool looks = split && (l.cnt != nullptr || l.mask != nullptr);
   plan[3] = looks;
   plan[4] = looks ? reinterpret_cast<const char*>(sp.note) - reinterpret_cast<const char*>(ws) : 0;
   const float cost[4] = {l.spread, l.whole / l.step, l.cut / l.step, l.least};

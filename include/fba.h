@@ -78,14 +78,15 @@ int32_t fba_mask_compact(const uint8_t* mask, int64_t mask_bh, int32_t nQ, int32
  */
 int64_t fba_split_workspace_bytes(void);
 /*
- * What a launch on such sizes would cut, for tests and measurements (no GPU needed: 256 compute units are assumed then).  launch: 0 forward, 1 dK/dV,
- * 2 dQ that recomputes S and dP, 3 dQ from dS; the lists are those the block sizes need.  plan [16]:
+ * What a launch on such sizes would cut, for tests and measurements (no GPU needed: 256 compute units are assumed then).  launch: 0 forward on lists, 1 dK/dV,
+ * 2 dQ that recomputes S and dP, 3 dQ from dS, 4 forward on the block mask (fba_fwd_blocks, which the operator calls without gradients and in some steps where that takes the
+ * sizes); the lists are those the block sizes need.  plan [16]:
  *   0 tiles of the launch   1 first tile that is cut (that many: none)   2 most ranges of a tile's list
  *   3 1 where the device decides how many, up to that, by the lengths of the lists, 0 where it is that many whatever the lists; the rest only if 1
  *   4 offset in split_ws of the int32 in which the device leaves its decision
  *   5, 6, 7, 8 (thousandths) with L = mean + plan[5] (longest list - mean) and M = mean + 0.4 (L - mean), lengths in steps, lists are cut where
  *   plan[6] L - plan[7] M >= plan[8]   9 into at least so many ranges   10.. and one more for each of these lengths that M reaches
- * A step is 32 keys (forward, dQ; 64 in forward on tile lists) or 32 query rows of one query head (dK/dV).
+ * A step is 32 keys (forward, dQ; 64 on tile lists, in forward and in dQ from dS) or 32 query rows of one query head (dK/dV).
  */
 int32_t fba_split_plan(int32_t launch, int64_t mask_bh, int32_t B, int32_t Hq, int32_t Hkv, int32_t Sq, int32_t Skv, int32_t head_dim,
                        int32_t q_block, int32_t k_block, int64_t split_ws_bytes, int64_t* plan);
