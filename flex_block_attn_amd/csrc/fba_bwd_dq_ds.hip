@@ -231,7 +231,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves),
 // Bound by what a step takes from barrier to barrier in launches of about a round (B2 H8/2 S3136 q16 k64: 36 of 46 us without any copy),
 // by memory in large ones.  In steps of 32 keys, with zeros for every wave that has no dS there, so that all waves have as many copies in flight, / so:
 // steps of H24 S30720, 64-token blocks, 192 of 480 kept 18.97 / 18.53 ms; B2 H8/2 S3136 q16 k64, 12 of 49 kept 188.7 / 180.6 us; B2 H8/4 S9472 q64 k128, 42 of
-// 74 1817 / 1759; H22 S4096, 64-token blocks, 16 of 64 308 / 301, but 40 of 64 549 / 558.  Steps of 32 keys with dS as here 592 / 571 us (B2 H3 S7168 q16 k128); the copies of
+// 74 1817 / 1759; H22 S4096, 64-token blocks, 16 of 64 308 / 301, but 40 of 64 549 / 558 (with
+// parts behind the round and dK/dV's merge in the launch 549 / 545).  Steps of 32 keys with dS as here 592 / 571 us (B2 H3 S7168 q16 k128); the copies of
 // dS in between the next step's matrix instructions 18.97 / 19.39 ms for the first.
 namespace {
 

@@ -127,7 +127,7 @@ FBA_DEVICE void softmax_exp(FwdState& st, f32x16& s, bf16x8 (&pk)[2], bool activ
 //
 // kMask: the list is read from the block mask, so that a call without gradients needs no launch that makes
 // lists: H8 S4096, 128-token blocks, 12 of 32 kept 32.7 -> 30.4 us, H12 S3072 32.8 -> 30.6, H2 S10240 68.5 -> 67.2, H24/6 768 rows against 30720 keys 128.0 ->
-// 126.4, H24 S11520, all blocks, 1396.5 -> 1393.3.  Steps that number no pairs have it make their lists on the way, a wave to a row in work-groups behind the others:
+// 126.4 (launches of a millisecond: nothing beyond noise, H24 S11520, all blocks, 1381.6 / 1381.8).  Steps that number no pairs have it make their lists on the way, a wave to a row in work-groups behind the others:
 // H4 S3840 115.1 -> 112.3 us, H2 S6144 139.5 -> 137.0, H12 S3456 146.6 -> 144.4.
 template <int kWaves, bool kMask>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * kWaves, 64 * kWaves), amdgpu_waves_per_eu(kWaves == 12 ? 3 : 2, kWaves == 12 ? 3 : 2))) void fwd_kernel(const FwdParams p) {

@@ -224,8 +224,8 @@ struct PartialOut {
 
 // The parts of a launch that are to be summed (merge_parts in fba_common.h).  dQ does not need dK and dV, so their merge rides in the dQ launch, as
 // work-groups behind its own: by itself it took 5 to 7 us, also where the device had made no parts.  Steps, a launch of its own / along: H12 S3072,
-// 128-token blocks, a third kept 131.1 / 126.6 us; H12 S3456 153.1 / 147.5; H2 S6144, 384-token blocks, half kept 140.4 / 138.6; H2 S7680 190.3 / 186.4; B2 H16/4
-// S8192 1020.5 / 1018.2.  (In front of dQ's work-groups instead, in launches of two rounds and more: the same.)
+// 128-token blocks, a third kept 131.1 / 126.6 us; H12 S3456 153.1 / 147.5; H2 S6144, 384-token blocks, half kept 140.4 / 138.6; H2 S7680 190.3 / 186.4; nothing
+// beyond noise in steps of a millisecond (B2 H16/4 S8192 1013.9 / 1013.2).  (In front of dQ's work-groups instead, in launches of two rounds and more: the same.)
 struct Merge {
   const float* ws = nullptr;
   const int32_t* note = nullptr;  // how many parts there are; null: `parts`
